@@ -49,26 +49,26 @@ SINK, LOCAL, CTX_SINK, CTX_LOCAL, BUDGET = 128, 256, 128, 8192, 4096      # LSer
 def listed():
     return [
         # one user's chat: a single short sequence, where a step is a chain of short launches
-        dict(name="decode, 1 sequence", kind="decode", size="8b", group=-1, batch=1, context=300),
+        dict(name="decode 1 sequence", kind="decode", size="8b", group=-1, batch=1, context=300),
         # the framework's headline: 16 sequences of 1024 tokens
-        dict(name="decode, 16 sequences", kind="decode", size="8b", group=-1, batch=16, context=1024),
+        dict(name="decode 16 sequences", kind="decode", size="8b", group=-1, batch=16, context=1024),
         # a server at ordinary load, weights with groups of 128, lengths and batch as they come
-        dict(name="decode, 61 sequences, g128", kind="decode", size="8b", group=128, batch=61, context=1100),
+        dict(name="decode 61 sequences g128", kind="decode", size="8b", group=128, batch=61, context=1100),
         # the large model at high load
-        dict(name="decode, 120 sequences, 70b", kind="decode", size="70b", group=-1, batch=120, context=900),
+        dict(name="decode 120 sequences 70b", kind="decode", size="70b", group=-1, batch=120, context=900),
         # one prompt of ordinary length
-        dict(name="prefill, 1 x 1501", kind="prefill", size="8b", group=-1, batch=1, prompt=1501),
+        dict(name="prefill 1 x 1501", kind="prefill", size="8b", group=-1, batch=1, prompt=1501),
         # several short prompts at once, weights with groups
-        dict(name="prefill, 7 x 333, g128", kind="prefill", size="8b", group=128, batch=7, prompt=333),
+        dict(name="prefill 7 x 333 g128", kind="prefill", size="8b", group=128, batch=7, prompt=333),
         # long-context serving: the context stage and a token behind 100 000
-        dict(name="LServe prefill, 1 x 12001", kind="lserve_prefill", kv="kv8", batch=1, prompt=12001),
-        dict(name="LServe decode, 100000", kind="lserve_decode", kv="kv8", batch=1, context=100000),
+        dict(name="LServe prefill 1 x 12001", kind="lserve_prefill", kv="kv8", batch=1, prompt=12001),
+        dict(name="LServe decode 100000", kind="lserve_decode", kv="kv8", batch=1, context=100000),
         # chat turns on the engine: prompts of some hundred tokens and answers behind them
-        dict(name="Bobavik turn, 16 x 500", kind="engine", arch="Bobavik", size="2048", seqs=16, prompt=500, steps=24),
-        dict(name="Bagedra turn, 48 x 150", kind="engine", arch="Bagedra", size="4096", seqs=48, prompt=150, steps=24),
+        dict(name="Bobavik turn 16 x 500", kind="engine", arch="Bobavik", size="2048", seqs=16, prompt=500, steps=24),
+        dict(name="Bagedra turn 48 x 150", kind="engine", arch="Bagedra", size="4096", seqs=48, prompt=150, steps=24),
         # a long document read in one step
-        dict(name="Bobavik prompt, 1 x 7999", kind="engine", arch="Bobavik", size="4096", seqs=1, prompt=7999, steps=0),
-        dict(name="Bagedra prompts, 2 x 8000", kind="engine", arch="Bagedra", size="2048", seqs=2, prompt=8000, steps=0),
+        dict(name="Bobavik prompt 1 x 7999", kind="engine", arch="Bobavik", size="4096", seqs=1, prompt=7999, steps=0),
+        dict(name="Bagedra prompts 2 x 8000", kind="engine", arch="Bagedra", size="2048", seqs=2, prompt=8000, steps=0),
     ]
 
 
