@@ -1,5 +1,5 @@
-// Prefill GEMM for EXACT shapes: M % 128 == 0, N % 256 == 0, K % 256 == 0 -- what the models' projections are at prefill.
-// (included by qgemm_kernel.h; the generic w4a8_gemm_kernel keeps ragged shapes)
+// Prefill GEMM for M >= 128 rows of any number, N % 256 == 0, K % 256 == 0 -- what the models' projections are at prefill.
+// (included by qgemm_kernel.h; the generic w4a8_gemm_kernel keeps ragged N and K)
 //
 // Same tile as the generic prefill kernel (128 rows x 256 channels per 256-thread workgroup, a wave = 64 channels x 128
 // rows = 32 accumulator tiles, K in 256-k chunks, two workgroups per CU, XCD-aware tile order) and the same arithmetic
@@ -110,7 +110,10 @@ __global__ __launch_bounds__(256, 2) void w4a8_gemm_exact_kernel(GemmArgs p) {
     }
   }
   const int ng = tile_n * WAVES + wave;  // 64-channel group of this wave
-  const int m0 = tile_m * MT;
+  // M need not be whole tiles: the last row tile starts at M - 128 and computes the rows it shares with the one before a second
+  // time (integer sums and the same epilogue: both store the same bits).  No predicate anywhere, and no more work than a padded
+  // tile would do.
+  const int m0 = min(tile_m * MT, p.M - MT);
   const int k0 = TO_SLAB ? (int)blockIdx.y * p.kslice : 0;      // first k of this workgroup's K slice
   const int nchunks = (TO_SLAB ? p.kslice : p.K) / KCHUNK;
   // (Two workgroups share a CU, one wave of each per SIMD, and the arbiter strictly favours the OLDER wave: per-workgroup

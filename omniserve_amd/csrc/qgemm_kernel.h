@@ -1218,7 +1218,7 @@ static void launch_variant(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
   // (the exact kernel decodes the 1-D XCD tile order and stores 16 B per lane: rows of the output must start 16-B aligned)
   static_assert(OMNI_GEMM_XCD_ORDER == 1, "w4a8_gemm_exact_kernel reads tiles_m / tiles_n of the 1-D XCD-ordered grid");
   const bool out16 = (a.out_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
-  if (MB == 8 && WAVES == 4 && exact_mode != 0 && a.M % 128 == 0 && a.N % 256 == 0 && a.K % KCHUNK == 0 && b.kslice >= a.K &&
+  if (MB == 8 && WAVES == 4 && exact_mode != 0 && a.M >= 128 && a.N % 256 == 0 && a.K % KCHUNK == 0 && b.kslice >= a.K &&
       (size_t)a.M * a.K < ((size_t)1 << 32) && out16) {
     // (the form that stages activations through registers -- OMNI_GEMM_EXACT=2, A/B -- exists in tuning builds only: the release
     //  library launches the LDS-DMA form alone, and the register form's g128 / W8A8 instantiations spill)
@@ -1233,7 +1233,7 @@ static void launch_variant(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
   }
   if (pl.sk > 1) {      // few tiles (decode at batch 129..512): K slices over grid.y -> int32 slabs -> the slab epilogue
     grid.y = pl.sk;
-    if (MB == 8 && WAVES == 4 && exact_mode != 0 && OMNI_GEMM_EXACT_DMA && a.M % 128 == 0 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 &&
+    if (MB == 8 && WAVES == 4 && exact_mode != 0 && OMNI_GEMM_EXACT_DMA && a.M >= 128 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 &&
         (size_t)a.M * a.K < ((size_t)1 << 32))
       hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, true, true>), grid, dim3(256), 0, st, b);
     else
@@ -1447,7 +1447,7 @@ static int launch_gemm_partial(GemmArgs a, void* slab, size_t slab_bytes, int* s
     b.tiles_n = (a.N / 64 + 3) / 4;
     b.tiles_m = (a.M + 127) / 128;
     b.tile_linear = 1;
-    if (OMNI_GEMM_EXACT_DMA && a.M % 128 == 0 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 && (size_t)a.M * a.K < ((size_t)1 << 32))
+    if (OMNI_GEMM_EXACT_DMA && a.M >= 128 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 && (size_t)a.M * a.K < ((size_t)1 << 32))
       hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, true, true>), dim3(b.tiles_m * b.tiles_n, pl.sk, 1), dim3(256), 0, st, b);
     else
       hipLaunchKernelGGL((w4a8_gemm_kernel<8, MODE, 4, true, false>), dim3(b.tiles_m * b.tiles_n, pl.sk, 1), dim3(256), 0, st, b);

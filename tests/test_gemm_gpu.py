@@ -362,3 +362,17 @@ def test_midm_planner_takes_the_big_matrices():
         assert waves(M, N, K) == 1, (M, N, K)
     _run_chn(128, 28672, 4096, seed=5)
     _run_chn(64, 28672, 4096, seed=6)
+
+
+# The straight-line prefill kernel at row counts that are not whole tiles: its last row tile starts at M - 128 and shares rows with the
+# tile before it (127 shared rows at M = 129, one at 255), on both tile orders (fewer than 8 row tiles, and super-blocks), one K chunk
+# and several, and a destination of which the rows around the output stay untouched.
+@pytest.mark.parametrize("M,N,K", [(129, 256, 256), (255, 512, 768), (257, 256, 512), (1101, 512, 256), (1501, 1024, 1024)])
+@pytest.mark.parametrize("mode", ["chn", "grp", "w8"])
+def test_prefill_rows_not_whole_tiles(mode, M, N, K):
+    if mode == "chn":
+        _run_chn(M, N, K, seed=M, out_view=True)
+    elif mode == "grp":
+        _run_grp(M, N, K, True)
+    else:
+        _run_w8(M, N, K)
