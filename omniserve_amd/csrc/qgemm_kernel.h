@@ -47,6 +47,7 @@ struct GemmArgs {
   int kslice;             // k per split (multiple of 64)
   int tiles_m, tiles_n;   // > 0: 1-D grid with the XCD-aware tile order of w4a8_gemm_kernel
   int tile_linear;        // 1 (with tiles_n > 0): workgroup w = tile (w % tiles_m, w / tiles_m) -- few row tiles
+  int band;               // w4a8_gemm_exact_kernel: row tiles per band of its tile order
   // ---- row-kernel-free decode forms (fused extension; see w4a8_gemv_kernel EPI / A16) ----
   const half_t* A16;      // [M,K] fp16 activations quantised on the fly (A16 kernels; `A` unused)
   uint32_t* amax;         // [AMAX_WORDS] row-maximum candidates (common.h): EPI = 1 raises them, A16 reads them
@@ -1196,12 +1197,60 @@ extern "C" void omni_gemm_set_midm_override(int mode, int sk);
 extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, int* sk);
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool w8 = false);
 
-template <int MODE, int MB, int WAVES>
-static void launch_variant(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
-  // prefill regime: chunked LDS staging, weights through L2, XCD-aware tile order
+// w4a8_gemm_exact_kernel's tile height (16-row blocks), K parts inside a workgroup, K slices over the grid (1: no slabs)
+struct PrefillPlan {
+  int mb, kw, sk;
+};
+// sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs
+PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only);
+
+// shapes the straight-line kernel takes: whole channel tiles and K chunks (also of a K slice: a.kslice); it stores 16 B
+// per lane, so rows of an fp16 output must start 16-B aligned
+static inline bool exact_shape(const GemmArgs& a, bool to_slab) {
+  const bool out16 = to_slab || ((a.out_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0);
+  return a.M > 128 && a.N % 256 == 0 && a.K % KCHUNK == 0 && a.kslice % KCHUNK == 0 && (size_t)a.M * a.K < ((size_t)1 << 32) && out16;
+}
+
+template <int MODE, int MB, int KW, bool TO_SLAB>
+static void launch_exact_tile(GemmArgs b, int sk, hipStream_t st) {
+  b.tiles_n = b.N / 256;
+  b.tiles_m = (b.M + MB * 16 - 1) / (MB * 16);
+  const int bands = (b.tiles_m + 7) / 8;
+  b.band = (b.tiles_m + bands - 1) / bands;
+  const int tiles = b.tiles_m * b.tiles_n;
+  hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, MB, KW, TO_SLAB>), dim3((tiles + 7) / 8 * 8, sk, 1), dim3(256 * KW), 0, st, b);
+}
+
+template <int MODE, int KW, bool TO_SLAB>
+static void launch_exact_rows(const GemmArgs& a, int mb, int sk, hipStream_t st) {
+  switch (mb) {
+    case 4: launch_exact_tile<MODE, 4, KW, TO_SLAB>(a, sk, st); break;
+    case 5: launch_exact_tile<MODE, 5, KW, TO_SLAB>(a, sk, st); break;
+    case 6: launch_exact_tile<MODE, 6, KW, TO_SLAB>(a, sk, st); break;
+    case 7: launch_exact_tile<MODE, 7, KW, TO_SLAB>(a, sk, st); break;
+    default: launch_exact_tile<MODE, 8, KW, TO_SLAB>(a, sk, st); break;
+  }
+}
+
+// prefill regime (M > 128): chunked LDS staging, weights through L2
+template <int MODE>
+static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
+  if (exact_shape(a, false)) {
+    const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false);
+    if (pp.sk > 1) {
+      launch_exact_rows<MODE, 1, true>(a, pp.mb, pp.sk, st);
+      const size_t total = (size_t)a.M * (a.N / 4);
+      hipLaunchKernelGGL((splitk_epilogue_kernel<MODE>), dim3((total + 63) / 64), dim3(64), 0, st, a, pp.sk);
+    } else if (pp.kw == 2) {
+      launch_exact_rows<MODE, 2, false>(a, pp.mb, 1, st);
+    } else {
+      launch_exact_rows<MODE, 1, false>(a, pp.mb, 1, st);
+    }
+    return;
+  }
   GemmArgs b = a;
-  b.tiles_n = (a.N / 64 + WAVES - 1) / WAVES;
-  b.tiles_m = (a.M + MB * 16 - 1) / (MB * 16);
+  b.tiles_n = (a.N / 64 + 3) / 4;
+  b.tiles_m = (a.M + 127) / 128;
 #if OMNI_GEMM_XCD_ORDER
   const int sbs = ((b.tiles_m + 7) / 8) * ((b.tiles_n + 7) / 8);
   dim3 grid(sbs * 64, 1, 1);
@@ -1213,36 +1262,14 @@ static void launch_variant(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
   dim3 grid(b.tiles_n, 1, b.tiles_m);
   b.tiles_n = b.tiles_m = 0;
 #endif
-  // exact shapes (the models' projections at prefill): the straight-line kernel of qgemm_exact.h
-  static const int exact_mode = omni_knob("OMNI_GEMM_EXACT", 1);   // 0: off (A/B, tuning builds)
-  // (the exact kernel decodes the 1-D XCD tile order and stores 16 B per lane: rows of the output must start 16-B aligned)
-  static_assert(OMNI_GEMM_XCD_ORDER == 1, "w4a8_gemm_exact_kernel reads tiles_m / tiles_n of the 1-D XCD-ordered grid");
-  const bool out16 = (a.out_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
-  if (MB == 8 && WAVES == 4 && exact_mode != 0 && a.M >= 128 && a.N % 256 == 0 && a.K % KCHUNK == 0 && b.kslice >= a.K &&
-      (size_t)a.M * a.K < ((size_t)1 << 32) && out16) {
-    // (the form that stages activations through registers -- OMNI_GEMM_EXACT=2, A/B -- exists in tuning builds only: the release
-    //  library launches the LDS-DMA form alone, and the register form's g128 / W8A8 instantiations spill)
-#if defined(OMNI_TUNING) || !OMNI_GEMM_EXACT_DMA
-    if (!(OMNI_GEMM_EXACT_DMA && exact_mode != 2)) {
-      hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, false>), grid, dim3(256), 0, st, b);
-      return;
-    }
-#endif
-    hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, true>), grid, dim3(256), 0, st, b);
-    return;
-  }
   if (pl.sk > 1) {      // few tiles (decode at batch 129..512): K slices over grid.y -> int32 slabs -> the slab epilogue
     grid.y = pl.sk;
-    if (MB == 8 && WAVES == 4 && exact_mode != 0 && OMNI_GEMM_EXACT_DMA && a.M >= 128 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 &&
-        (size_t)a.M * a.K < ((size_t)1 << 32))
-      hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, true, true>), grid, dim3(256), 0, st, b);
-    else
-      hipLaunchKernelGGL((w4a8_gemm_kernel<MB, MODE, WAVES, true, false>), grid, dim3(64 * WAVES), 0, st, b);
+    hipLaunchKernelGGL((w4a8_gemm_kernel<8, MODE, 4, true, false>), grid, dim3(256), 0, st, b);
     const size_t total = (size_t)a.M * (a.N / 4);
     hipLaunchKernelGGL((splitk_epilogue_kernel<MODE>), dim3((total + 63) / 64), dim3(64), 0, st, a, pl.sk);
     return;
   }
-  hipLaunchKernelGGL((w4a8_gemm_kernel<MB, MODE, WAVES, false, false>), grid, dim3(64 * WAVES), 0, st, b);
+  hipLaunchKernelGGL((w4a8_gemm_kernel<8, MODE, 4, false, false>), grid, dim3(256), 0, st, b);
 }
 
 // Load policy of a decode-shape GEMV's weight stream, decided PER CALL: plain loads when the call's weight tensor is the
@@ -1355,11 +1382,7 @@ static int launch_gemm(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
     return omni_launch_status();
   }
   if (a.M > 128) {
-#ifdef OMNI_GEMM_TILE_M64
-    launch_variant<MODE, 4, 4>(a, pl, st);
-#else
-    launch_variant<MODE, 8, 4>(a, pl, st);
-#endif
+    launch_prefill<MODE>(a, pl, st);
   } else {
     switch (pl.mb) {
       case 1: launch_gemv<MODE, 1>(a, pl, st); break;
@@ -1443,14 +1466,15 @@ static int launch_gemm_partial(GemmArgs a, void* slab, size_t slab_bytes, int* s
     return omni_launch_status();
   }
   if (a.M > 128) {      // decode batches of 129 .. 512 rows: the 128 x 256 tile with K slices over grid.y, slabs only
-    GemmArgs b = a;
-    b.tiles_n = (a.N / 64 + 3) / 4;
-    b.tiles_m = (a.M + 127) / 128;
-    b.tile_linear = 1;
-    if (OMNI_GEMM_EXACT_DMA && a.M >= 128 && a.N % 256 == 0 && b.kslice % KCHUNK == 0 && (size_t)a.M * a.K < ((size_t)1 << 32))
-      hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, true, true>), dim3(b.tiles_m * b.tiles_n, pl.sk, 1), dim3(256), 0, st, b);
-    else
+    if (exact_shape(a, true)) {
+      launch_exact_rows<MODE, 1, true>(a, plan_prefill(a.M, a.N, a.K, MODE, pl.sk, true).mb, pl.sk, st);
+    } else {
+      GemmArgs b = a;
+      b.tiles_n = (a.N / 64 + 3) / 4;
+      b.tiles_m = (a.M + 127) / 128;
+      b.tile_linear = 1;
       hipLaunchKernelGGL((w4a8_gemm_kernel<8, MODE, 4, true, false>), dim3(b.tiles_m * b.tiles_n, pl.sk, 1), dim3(256), 0, st, b);
+    }
     *sk_out = pl.sk;
     return omni_launch_status();
   }

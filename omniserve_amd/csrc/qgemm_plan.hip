@@ -186,6 +186,57 @@ GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred, bool w8) {
   return pl;
 }
 
+// Tile height, K parts inside a workgroup and use of the slab form for w4a8_gemm_exact_kernel: the smallest modelled time.
+//
+// The model's numbers are measured times of the kernel on an MI355X (us; 150 - 4096 rows at N x K = 6144 x 4096, 4096 x 4096, 28672 x 4096
+// and 4096 x 14336): one four-wave workgroup on a CU, two of them, and one eight-wave workgroup (KW = 2), each as fixed + per 256-k chunk
+// and 16-row blocks.  A grid of n workgroups per CU is whole pairs and a rest that runs alone or in pairs.  What the choice is about is
+// the last round: 1501 rows of the 4096 x 14336 projection were 192 tiles of 128 rows on 256 CUs (86.6 us per-channel, 171 per-group,
+// 129 W8A8); 256 tiles of 96 rows with two K parts each take 70.5 / 116 / 95.  2331 rows: 304 tiles, i.e. two rounds (141 / 226 / 197 us);
+// 480 tiles of 80 rows 111 / 184 / 160.  Few rows: 333 rows of 4096 x 4096 24.6 us with K slices over the grid, slabs and their epilogue
+// launch, 18.6 with 64-row tiles and KW = 2.
+struct TileCost {
+  float fix[3], chunk[3][5];      // [alone, pair, KW = 2][mb - 4]
+};
+static const TileCost kTileCost[3] = {
+    {{3.8f, 7.5f, 5.5f}, {{1.12f, 1.20f, 1.36f, 1.21f, 1.44f}, {1.50f, 1.80f, 2.10f, 2.14f, 2.40f}, {0.82f, 0.92f, 1.06f, 1.08f, 1.16f}}},
+    {{1.5f, 5.0f, 5.0f}, {{2.18f, 2.52f, 2.74f, 2.65f, 3.00f}, {2.92f, 3.18f, 3.46f, 3.54f, 3.94f}, {1.52f, 1.72f, 1.95f, 2.00f, 2.20f}}},
+    {{3.5f, 6.5f, 4.7f}, {{1.63f, 1.80f, 1.88f, 2.12f, 2.24f}, {2.18f, 2.65f, 3.00f, 3.08f, 3.36f}, {1.22f, 1.36f, 1.48f, 1.62f, 1.78f}}},
+};
+
+static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, int chunks) {
+  auto t = [&](int kind) { return c.fix[kind] + c.chunk[kind][mb - 4] * (float)chunks; };
+  if (kw == 2) {      // (nothing runs beside the next one's start: 4 us more per further round)
+    const long long rounds = (workgroups + 255) / 256;
+    return (float)rounds * (t(2) + 4.f) - 4.f;
+  }
+  const long long pairs = workgroups / 512, rest = workgroups - pairs * 512;
+  return (float)pairs * t(1) + (rest == 0 ? 0.f : rest <= 256 ? t(0) : t(1));
+}
+
+PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) {
+  const TileCost& c = kTileCost[mode];
+  PrefillPlan best{8, 1, slab_only ? sk : 1};
+  float time = 1e30f;
+  auto offer = [&](int mb, int kw, int split) {
+    const long long tiles = (long long)((M + 16 * mb - 1) / (16 * mb)) * (N / 256) * split;
+    float t = grid_time(c, mb, kw, tiles, K / (split * KCHUNK));
+    // the slabs written, read and reduced by a launch of their own
+    if (split > 1 && !slab_only) t += 4.5f + (float)split * M * N * 8.f / 4.5e6f;
+    if (t < time) { time = t; best = PrefillPlan{mb, kw, split}; }
+  };
+  for (int mb = 8; mb >= 4; --mb) {
+    if (slab_only) {
+      offer(mb, 1, sk);
+      continue;
+    }
+    offer(mb, 1, 1);
+    if (K % (2 * KCHUNK) == 0) offer(mb, 2, 1);
+    if (sk > 1) offer(mb, 1, sk);
+  }
+  return best;
+}
+
 }  // namespace omni
 
 extern "C" void omni_gemm_set_plan_override(int waves, int sk) {

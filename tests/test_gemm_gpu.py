@@ -376,3 +376,12 @@ def test_prefill_rows_not_whole_tiles(mode, M, N, K):
         _run_grp(M, N, K, True)
     else:
         _run_w8(M, N, K)
+
+
+# Its tile heights (4 .. 8 blocks of 16 rows) and its two forms (K whole, K in two parts that meet in LDS): the sizes at which
+# plan_prefill's model picks each of them.
+@pytest.mark.parametrize("M,N,K", [(129, 256, 256), (513, 8192, 256), (700, 16384, 256), (333, 16384, 256), (449, 16384, 256), (129, 256, 2048),
+                                   (513, 8192, 2048), (333, 16384, 2048), (385, 16384, 2048), (449, 16384, 2048), (225, 28672, 4096), (161, 28672, 4096), (385, 16384, 4096)])
+@pytest.mark.parametrize("mode", ["chn", "grp", "w8"])
+def test_prefill_tile_heights(mode, M, N, K):
+    {"chn": lambda: _run_chn(M, N, K, seed=M), "grp": lambda: _run_grp(M, N, K, False), "w8": lambda: _run_w8(M, N, K)}[mode]()
