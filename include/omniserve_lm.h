@@ -11,7 +11,7 @@
 extern "C" {
 #endif
 
-#define LM_ABI_VERSION 3
+#define LM_ABI_VERSION 4
 #define LM_NORM_LAYER 0
 #define LM_NORM_RMS 1
 #define LM_EPI_ELEM 0
@@ -147,8 +147,11 @@ typedef struct {
   const void* gate;
   int64_t ldg;
 } LmGemmPart;
+/* lm_gemm_rows, part (or null): lm_gemm_rows_scratch() f32 of scratch for one matrix over at most 64 rows, whose K may then be cut into
+ * slices (0: it is not). */
+int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi);
 int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, int rows_a, int rows_b,
-                 int x_div, int max_rows, float scale, int epi, int act, void* stream);
+                 int x_div, int max_rows, float scale, int epi, int act, float* part, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,
                   int max_tiles, int rows_a, int rows_b, int x_div, float scale, int epi, int act, void* stream);
 

@@ -19,7 +19,7 @@ ELEM = {torch.bfloat16: "bf16", torch.float32: "f32"}
 NORM = {"layer": 0, "rms": 1}
 ACT = {None: 0, "silu": 1, "gelu_tanh": 2, "sigmoid": 3}
 EPI_ELEM, EPI_F32, EPI_GLU, EPI_GATE = 0, 1, 2, 3
-ABI = 3
+ABI = 4
 ATTN_ROWS = 128          # query rows of one prefill tile
 PAGE = 64                # tokens per cache page
 ROWS_MAX = 64            # up to here a step's products stream the weights
@@ -60,7 +60,8 @@ PROTOTYPES = {
     "lm_route_scratch_words": (_i64, [_i, _i, _i]),
     "lm_route_max_tiles": (_i, [_i, _i, _i]),
     "lm_route": (_i, [_vp, _i64, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
-    "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp]),
+    "lm_gemm_rows_scratch": (_i64, [_i, _i, _i, _i]),
+    "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp]),
     "lm_gemm_tiles": (_i, [_PP, _PP, _i, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp]),
     "lm_argmax": (_i, [_vp, _vp, _i64, _i, _i, _vp]),
 }
@@ -181,6 +182,11 @@ class LmOps:
         return out
 
     # ---- products ------------------------------------------------------------------------------------------------
+    def _slices(self, x, w, epi):
+        """room for the sums of w's K slices"""
+        n = self._h.lm_gemm_rows_scratch(w.shape[0], w.shape[1], x.shape[0], epi)
+        return torch.empty((n,), dtype=torch.float32, device=x.device) if n else None
+
     def matmul(self, x, w, out=None, out_f32=False, scale=1.0):
         """x [T, k] w[n, k]^T.  Few rows: the weight-streaming kernel; many: the MFMA tiles for f32 results (the router, the
         output head), the vendor product for plain ones."""
@@ -192,7 +198,7 @@ class LmOps:
         part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), n, w.shape[1])
         epi = EPI_F32 if out_f32 else EPI_ELEM
         if T <= ROWS_MAX or n <= NARROW:
-            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, scale, epi, 0)
+            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, scale, epi, 0, _p(self._slices(x, w, epi)))
         else:
             self._call("lm_gemm_tiles", _c.byref(part), None, 1, None, None, None, 0, T, 0, 1, scale, epi, 0)
         return out
@@ -204,7 +210,7 @@ class LmOps:
         out = torch.empty((T, n), dtype=self.dtype, device=x.device)
         if T <= ROWS_MAX:
             part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), 2 * n, w.shape[1], bias=_p(bias))
-            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, 1.0, EPI_GLU, ACT[act])
+            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, 1.0, EPI_GLU, ACT[act], _p(self._slices(x, w, EPI_GLU)))
         else:
             y = self.matmul(x, w)
             self._call("lm_glu", _p(out), _ld(out), _p(y), _ld(y), _p(bias), T, n, ACT[act])
@@ -216,7 +222,7 @@ class LmOps:
         H, n, k = w.shape
         part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), n, k, gx=x_step, gy=out_step, gate=_p(gate), ldg=_ld(gate))
         T = x.shape[0]
-        self._call("lm_gemm_rows", _c.byref(part), None, H, None, None, T, 0, 1, T, 1.0, EPI_ELEM if gate is None else EPI_GATE, 0)
+        self._call("lm_gemm_rows", _c.byref(part), None, H, None, None, T, 0, 1, T, 1.0, EPI_ELEM if gate is None else EPI_GATE, 0, None)
         return out
 
     def route(self, z, bias, experts, top):
@@ -244,7 +250,7 @@ class LmOps:
         pb = None if b is None else _c.byref(b)
         epi, div, rb = (EPI_GLU if glu else EPI_ELEM), (1 if x_is_pairs else top), (tokens if b is not None else 0)
         if tiles is None:
-            self._call("lm_gemm_rows", _c.byref(a), pb, w.shape[0], _p(perm), _p(off), 0, rb, div, tokens, 1.0, epi, ACT["silu"])
+            self._call("lm_gemm_rows", _c.byref(a), pb, w.shape[0], _p(perm), _p(off), 0, rb, div, tokens, 1.0, epi, ACT["silu"], None)
         else:
             self._call("lm_gemm_tiles", _c.byref(a), pb, w.shape[0], _p(perm), _p(off), _p(tiles), max_tiles, 0, rb, div, 1.0, epi, ACT["silu"])
 

@@ -202,6 +202,15 @@ __device__ __forceinline__ void dma16_uncounted(const void* src, uint32_t lds_ds
                : "v"(src), "s"(lds_dst)
                : "memory");
 }
+// ... for what is read once: not kept in the caches
+__device__ __forceinline__ void dma16_stream(const void* src, uint32_t lds_dst) {
+  uint32_t keep;
+  lds_dst = __builtin_amdgcn_readfirstlane(lds_dst);
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(src), "s"(lds_dst)
+               : "memory");
+}
 template <int N>
 __device__ __forceinline__ void wait_pieces() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

@@ -1,8 +1,8 @@
 // Matrix products y = x W^T, one launch for a set of weight matrices ("groups"): a dense projection is one group, a mixture of
 // experts is one group per expert over the tokens routed to it, plus one for the shared expert over all tokens.
 //
-//   lm_gemm_rows   few rows (decode): HBM bound.  A workgroup owns 16 or 32 channels of a group and streams their weights
-//                  once; its waves split K and meet in LDS.  Weights are the A operand straight from global memory.
+//   lm_gemm_rows   few rows (decode): HBM bound.  A workgroup streams the weights of 16 - 80 channels of a group once, through an LDS
+//                  ring filled by DMA; the rows of x come the same way, shared by its waves.
 //   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 128 tiles, both operands by LDS-DMA, two stages ahead.
 //
 // Epilogues: element type, f32 times a factor, the gated unit act(gate + bias) * (up + bias) of a matrix whose rows alternate in
@@ -11,6 +11,13 @@
 #include "omniserve_lm.h"
 
 namespace lm {
+
+template <int N> struct Int { static constexpr int value = N; };
+template <int J, typename F>
+__device__ __forceinline__ void countdown(F&& f) {      // f(J), f(J - 1), ..., f(0)
+  f(Int<J>{});
+  if constexpr (J > 0) countdown<J - 1>(f);
+}
 
 struct Part {        // a family of equally shaped groups
   const elem_t* w;   // [groups][n][k]
@@ -191,6 +198,187 @@ __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(GemmArgs p) {
   }
 }
 
+// ---- few rows: the weights' stream --------------------------------------------------------------------------------------------
+// Both operands arrive by LDS-DMA in pieces of 8 rows x 128 bytes: 8 neighbouring lanes read 128 consecutive bytes.  An operand fragment
+// loaded straight into registers reads 64 bytes of each of 16 rows, which the address path takes at 15 B per clock and CU; with x read that way
+// once per 16 channels (4 bytes of x per byte of weights at 64 rows) that path and not HBM bounded the products: 4096 x 14336 at 48 rows 59 us
+// -> 26 (117 MB: 4.5 TB/s), 28672 x 4096 75 -> 49, 32 experts at 60 tokens (998 MB) 278 -> 172 us (5.8 TB/s).  A stage is consumed behind one
+// barrier; R - 1 more are on their way.
+constexpr int RB = 128;                // bytes of k of a stage's rows
+template <int NW, int KW> constexpr int ring_bytes = KW > 1 ? (144 << 10) / KW : NW <= 4 ? 64 << 10 : 80 << 10;      // of one K part
+
+// at most N pieces of this wave still fly, and its LDS reads have been answered
+template <int N>
+__device__ __forceinline__ void wait_stage() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// rows (at most 16 MB) of x times 16 NW channels of w, stages s0 .. s1 - 1 of k, into red [KW][16 MB][16 NW + 4]: part h of the
+// workgroup's waves takes every KW-th stage through a ring of its own
+template <int MB, int NW, int KW>
+__device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int n, int64_t k, int n0, const elem_t* x, int64_t ldx,
+                                              const int* perm, int div, int rows, int s0, int s1) {
+  constexpr int WST = 16 * NW * RB, XST = 16 * MB * RB, ST = WST + XST, R0 = ring_bytes<NW, KW> / ST;
+  constexpr int XP = (2 * MB + NW - 1) / NW;                   // pieces (8 rows) of x a wave carries (some twice: the same bytes)
+  constexpr int P = 2 + XP, RMAX = 63 / P + 2 < 10 ? 63 / P + 2 : 10, R = R0 < RMAX ? R0 : RMAX;      // (vmcnt counts to 63)
+  typedef Tile<RB> T;
+  const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, l4 = lane >> 4;
+  const int all = __builtin_amdgcn_readfirstlane(tid >> 6), h = KW == 1 ? 0 : all / NW, wave = all - h * NW;
+  lds += h * ring_bytes<NW, KW>;
+  const int pr = lane >> 3, ps = lane & 7;                 // a piece: lane -> (row, physical slot)
+  const uint8_t *wsrc[2], *xsrc[XP];
+  int xp[XP];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 8 * i + pr, c = min(n0 + 16 * wave + r, n - 1);
+    wsrc[i] = (const uint8_t*)(w + c * k) + (int64_t)(s0 + h) * RB + ((ps ^ T::swizzle(r)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < XP; ++i) {
+    xp[i] = (NW * i + wave) % (2 * MB);
+    const int r = 8 * xp[i] + pr, rc = min(r, rows - 1);
+    const int64_t row = perm ? perm[rc] / div : rc;
+    xsrc[i] = (const uint8_t*)(x + row * ldx) + (int64_t)(s0 + h) * RB + ((ps ^ T::swizzle(r)) << 4);
+  }
+  const uint32_t base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  auto stage = [&](int t) {                                // stage t of this part
+    const uint32_t dst = base + (uint32_t)(t % R) * ST;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16_stream(wsrc[i] + t * (KW * RB), dst + 2048 * wave + 1024 * i);
+#pragma unroll
+    for (int i = 0; i < XP; ++i) dma16_uncounted(xsrc[i] + t * (KW * RB), dst + WST + 1024 * xp[i]);
+  };
+  // sums of 4 stages and the sum of those: shorter chains of f32 additions than K / 32
+  f32x4 acc[MB], total[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) acc[m] = total[m] = zero4();
+  auto multiply = [&](int t) {
+    const uint8_t* wt = lds + (t % R) * ST + wave * (16 * RB);
+    const uint8_t* xt = lds + (t % R) * ST + WST;
+    frag_t a[2], b[2][MB];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      a[v] = T::frag(wt, l15, 4 * v + l4);
+#pragma unroll
+      for (int m = 0; m < MB; ++m) b[v][m] = *(const frag_t*)(xt + 16 * m * RB + T::slot(l15, 4 * v + l4));
+    }
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) acc[m] = mma(a[v], b[v][m], acc[m]);
+    if ((t & 3) == 3) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        total[m] += acc[m];
+        acc[m] = zero4();
+      }
+    }
+  };
+  const int nst = (s1 - s0 - h + KW - 1) / KW;
+  wait_pieces<0>();                                        // the compiler's own loads
+#pragma unroll
+  for (int t = 0; t < R - 1; ++t)
+    if (t < nst) stage(t);
+  int t = 0;
+  for (; t + R - 1 < nst; ++t) {                           // R - 2 stages fly behind stage t
+    wait_stage<(R - 2) * P>();
+    __builtin_amdgcn_s_barrier();                          // stage t is there for every wave, everyone has left stage t - 1
+    asm volatile("" ::: "memory");
+    stage(t + R - 1);
+    multiply(t);
+  }
+  // the last R - 1 stages: j fly behind this one
+  auto last = [&](auto jt) {
+    constexpr int J = decltype(jt)::value;
+    if (nst - 1 - J < 0) return;
+    wait_stage<J * P>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    multiply(nst - 1 - J);
+  };
+  countdown<R - 2>(last);
+  if (KW > 1 && nst < (s1 - s0 + KW - 1) / KW) __builtin_amdgcn_s_barrier();      // (other parts have a stage more)
+  __syncthreads();                                         // the rings are free
+  float* red = (float*)(lds - h * ring_bytes<NW, KW>) + h * (16 * MB * (16 * NW + 4));
+#pragma unroll
+  for (int m = 0; m < MB; ++m) *(f32x4*)&red[(16 * m + l15) * (16 * NW + 4) + 16 * wave + 4 * l4] = total[m] + acc[m];
+  __syncthreads();
+}
+
+// A workgroup: 16 NW channels of a group, rows 0 .. 16 MB - 1 of it, K slice blockIdx.z.  With several slices (one group) the f32 sums of a
+// slice go to part [slice][rows][n] and gemm_reduce_kernel finishes them.
+template <int EPI, int NW, int KW>
+__global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, float* part) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[KW * ring_bytes<NW, KW>];
+  constexpr int RC = 16 * NW, NT = 64 * NW * KW;
+  const int g = blockIdx.y, tid = threadIdx.x;
+  const bool is_b = g >= p.groups;
+  const Part& pt = is_b ? p.b : p.a;
+  const int n0 = blockIdx.x * RC;
+  if (n0 >= pt.n) return;
+  int first = 0, rows = is_b ? p.rows_b : p.rows_a;
+  const int* perm = is_b ? nullptr : p.perm;
+  if (perm) { first = p.off[g]; rows = p.off[g + 1] - first; perm += first; }
+  if (rows <= 0) return;
+  const elem_t* w = pt.w + (is_b ? 0 : (int64_t)g * pt.n * pt.k);
+  const int64_t x0 = is_b || perm ? 0 : g * pt.gx, y0 = is_b || perm ? 0 : g * pt.gy;
+  const int stages = pt.k * (int)sizeof(elem_t) / RB, slice = blockIdx.z, slices = gridDim.z;
+  const int s0 = stages * slice / slices, s1 = stages * (slice + 1) / slices;
+  const int div = is_b ? 1 : p.x_div;
+  for (int m0 = 0; m0 < rows; m0 += 64) {
+    const int here = min(64, rows - m0), mb = (here + 15) >> 4;
+    const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
+    const int* pm = perm ? perm + m0 : nullptr;
+    if (mb == 1) stream_stages<1, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 2) stream_stages<2, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 3) stream_stages<3, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else stream_stages<4, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    const float* red = (const float*)lds;
+    auto sum = [&](int m, int c) {
+      f32x4 v = *(const f32x4*)&red[m * (RC + 4) + c];
+#pragma unroll
+      for (int h = 1; h < KW; ++h) v += *(const f32x4*)&red[(16 * mb * h + m) * (RC + 4) + c];
+      return v;
+    };
+    if (slices > 1) {
+      for (int i = tid; i < here * (RC / 4); i += NT) {
+        const int m = i / (RC / 4), c = 4 * (i % (RC / 4));
+        if (n0 + c < pt.n) *(f32x4*)(part + ((int64_t)slice * rows + m0 + m) * pt.n + n0 + c) = sum(m, c);
+      }
+    } else {
+      constexpr int OC = EPI == LM_EPI_GLU ? RC / 2 : RC;
+      for (int i = tid; i < here * (OC / 4); i += NT) {
+        const int m = i / (OC / 4), c = 4 * (i % (OC / 4));
+        const int sc = EPI == LM_EPI_GLU ? 32 * (c >> 4) + (c & 15) : c;      // the gate's (or the only) channel inside the tile
+        if (n0 + sc >= pt.n) continue;
+        f32x4 v = sum(m, sc);
+        if constexpr (EPI == LM_EPI_GLU) v = glu(pt, p.act, n0 + sc, v, sum(m, sc + 16));
+        store4<EPI>(pt, pm ? pm[m] : m0 + m, (EPI == LM_EPI_GLU ? n0 / 2 : n0) + c, y0, v, p.scale);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// sums of the K slices in their order, then the epilogue
+template <int EPI>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs p, const float* part, int slices) {
+  const Part& pt = p.a;
+  const int oq = (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n) / 4;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)p.rows_a * oq) return;
+  const int m = (int)(i / oq), c = 4 * (int)(i % oq);
+  const int sc = EPI == LM_EPI_GLU ? 32 * (c >> 4) + (c & 15) : c;
+  f32x4 v = zero4(), up = zero4();
+  for (int k = 0; k < slices; ++k) {
+    const float* r = part + ((int64_t)k * p.rows_a + m) * pt.n + sc;
+    v += *(const f32x4*)r;
+    if constexpr (EPI == LM_EPI_GLU) up += *(const f32x4*)(r + 16);
+  }
+  if constexpr (EPI == LM_EPI_GLU) v = glu(pt, p.act, sc, v, up);
+  store4<EPI>(pt, m, c, 0, v, p.scale);
+}
+
 constexpr int TM = LM_TILE_ROWS, TN = 128;                  // rows, channels of a tile
 constexpr int SROWB = 64, SK = SROWB / (int)sizeof(elem_t);  // a stage: 64 bytes of k of every row
 constexpr int STAGE = (TM + TN) * SROWB, STAGES = 3;
@@ -358,31 +546,84 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   return LM_OK;
 }
 
-template <int NR, int KW, int EPI>
+template <int EPI>
 static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s) {
+  constexpr int NR = 2, MB = 4, KW = 8;
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
-  const int mb = max_rows <= 16 || (n <= 256 && !a.perm && max_rows <= 64) ? 1 : max_rows <= 32 ? 2 : 4;
-  const dim3 grid((n + 16 * NR - 1) / (16 * NR), a.groups + has_b, a.perm ? 1 : (max_rows + 16 * mb - 1) / (16 * mb));
-  const dim3 block(64 * KW);
-  if (mb == 1) hipLaunchKernelGGL((gemm_rows_kernel<NR, 1, KW, EPI>), grid, block, 0, s, a);
-  else if (mb == 2) hipLaunchKernelGGL((gemm_rows_kernel<NR, 2, KW, EPI>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((gemm_rows_kernel<NR, 4, KW, EPI>), grid, block, 0, s, a);
+  const dim3 grid((n + 16 * NR - 1) / (16 * NR), a.groups + has_b, a.perm ? 1 : (max_rows + 16 * MB - 1) / (16 * MB));
+  hipLaunchKernelGGL((gemm_rows_kernel<NR, MB, KW, EPI>), grid, dim3(64 * KW), 0, s, a);
   return launch_status();
 }
 
-// Channels per workgroup: the more the fewer reads of x, as long as every CU has work.  A product of few channels over many rows
-// (the router of a prompt) has its workgroups along the rows instead.
-template <int EPI>
-static int plan_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s) {
-  const int64_t n = (int64_t)a.groups * a.a.n;
-  if constexpr (EPI == LM_EPI_GLU) {
-    return n >= 64 * 256 ? launch_rows<4, 4, EPI>(a, max_rows, has_b, s) : launch_rows<2, 8, EPI>(a, max_rows, has_b, s);
-  } else {
-    if (max_rows > 64) return launch_rows<2, 8, EPI>(a, max_rows, has_b, s);
-    if (n >= 64 * 512 || (n >= 64 * 150 && max_rows > 16)) return launch_rows<4, 4, EPI>(a, max_rows, has_b, s);
-    if (n >= 64 * 150) return launch_rows<2, 4, EPI>(a, max_rows, has_b, s);
-    return launch_rows<1, 8, EPI>(a, max_rows, has_b, s);
+// How the products of few rows are dealt: workgroups of 16 nw channels, K slices over the grid (of one matrix, `sliced`).
+//
+// The least time of a model fitted to the kernel (MI355X, bf16, 1 - 64 rows, 8 - 260 MB of weights): a workgroup takes 0.07 nw + 0.02 per
+// 16 rows + 0.02 us per stage, workgroups beyond one per CU add up (a CU takes in about 22 GB/s times 1000, so a 257th tile costs as much as
+// 256 more: 16448 channels at 48 rows take 42 us as 257 tiles of 64, 30 as 206 of 80), and slices cost the launch that adds them.  By what
+// was measured the channels per workgroup matter most where n / 64 is far from a multiple of 256 (10816 x 4096, 48 rows: 26.5 us at 64,
+// 20.8 at 48; 4096 x 4096, 16 rows: 11.8 us at 64 and 4 slices, 9.8 at 16), slices where K is long (4096 x 14336, 48 rows: 40 us, 26
+// with 4).
+struct StreamPlan {
+  int nw, slices;
+};
+static StreamPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool sliced) {
+  StreamPlan best{4, 1};
+  float time = 1e30f;
+  const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
+  for (int nw = 5; nw >= 1; --nw) {
+    if (glu && nw != 4) continue;                          // (a gate block and its up block share a workgroup)
+    const int64_t tiles = (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw));
+    for (int s = 1; s <= (sliced ? 8 : 1) && stages >= 4 * s; s *= 2) {
+      float t = (float)((tiles * s + 255) / 256) * (float)((stages + s - 1) / s) * (0.07f * nw + 0.02f * mb + 0.02f);
+      if (s > 1) t += 4.5f + (float)s * rows * n * 8.f / 5e6f;
+      if (t < time) { time = t; best = StreamPlan{nw, s}; }
+    }
   }
+  return best;
+}
+
+// K parts inside a workgroup where there is no second one to run beside it on its CU
+template <int EPI, int NW>
+static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+  const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
+  constexpr int KW = NW <= 2 ? 4 : 2;
+  if ((int64_t)grid.x * grid.y * grid.z <= 256)
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW>), grid, dim3(64 * NW * KW), 0, s, a, part);
+  else
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1>), grid, dim3(64 * NW), 0, s, a, part);
+}
+
+template <int EPI>
+static int launch_stream(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
+  const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
+  // experts: how many have rows is not known here; 64 channels measured best from 60 to 1000 MB
+  const StreamPlan pl = a.perm || has_b ? StreamPlan{4, 1} : plan_stream(a.groups, n, a.a.k, max_rows, EPI == LM_EPI_GLU, part != nullptr);
+  if constexpr (EPI == LM_EPI_GLU) {
+    launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s);
+  } else {
+    switch (pl.nw) {
+      case 1: launch_stream_tiles<EPI, 1>(a, n, has_b, pl.slices, part, s); break;
+      case 2: launch_stream_tiles<EPI, 2>(a, n, has_b, pl.slices, part, s); break;
+      case 3: launch_stream_tiles<EPI, 3>(a, n, has_b, pl.slices, part, s); break;
+      case 4: launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s); break;
+      default: launch_stream_tiles<EPI, 5>(a, n, has_b, pl.slices, part, s); break;
+    }
+  }
+  if (pl.slices > 1) {
+    const int64_t q = (int64_t)a.rows_a * ((EPI == LM_EPI_GLU ? n / 2 : n) / 4);
+    hipLaunchKernelGGL((gemm_reduce_kernel<EPI>), dim3((unsigned)((q + 255) / 256)), dim3(256), 0, s, a, part, pl.slices);
+  }
+  return launch_status();
+}
+
+// More than 64 rows come here with few channels (the router of a prompt) or one matrix per head: workgroups along the rows.
+template <int EPI>
+static int plan_rows(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
+  if constexpr (EPI != LM_EPI_GLU) {
+    if (max_rows > 64) return launch_rows<EPI>(a, max_rows, has_b, s);
+  }
+  const bool one = a.groups == 1 && !a.perm && !has_b && max_rows <= 64 && max_rows == a.rows_a;
+  return launch_stream<EPI>(a, max_rows, has_b, one ? part : nullptr, s);
 }
 
 }  // namespace lm
@@ -390,14 +631,20 @@ static int plan_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s) 
 using namespace lm;
 
 extern "C" int lm_gemm_rows(const LmGemmPart* pa, const LmGemmPart* pb, int groups, const int* perm, const int* off, int rows_a,
-                            int rows_b, int x_div, int max_rows, float scale, int epi, int act, void* stream) {
+                            int rows_b, int x_div, int max_rows, float scale, int epi, int act, float* part, void* stream) {
   GemmArgs a;
   if (fill(a, pa, pb, groups, perm, off, rows_a, rows_b, x_div, scale, epi, act) || max_rows <= 0) return LM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   const int has_b = pb && rows_b > 0;
-  if (epi == LM_EPI_GLU) return plan_rows<LM_EPI_GLU>(a, max_rows, has_b, s);
-  if (epi == LM_EPI_GATE) return plan_rows<LM_EPI_GATE>(a, max_rows, has_b, s);
-  return epi == LM_EPI_F32 ? plan_rows<LM_EPI_F32>(a, max_rows, has_b, s) : plan_rows<LM_EPI_ELEM>(a, max_rows, has_b, s);
+  if (epi == LM_EPI_GLU) return plan_rows<LM_EPI_GLU>(a, max_rows, has_b, part, s);
+  if (epi == LM_EPI_GATE) return plan_rows<LM_EPI_GATE>(a, max_rows, has_b, part, s);
+  return epi == LM_EPI_F32 ? plan_rows<LM_EPI_F32>(a, max_rows, has_b, part, s) : plan_rows<LM_EPI_ELEM>(a, max_rows, has_b, part, s);
+}
+
+extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {
+  if (n <= 0 || k <= 0 || rows <= 0 || rows > 64) return 0;
+  const int s = plan_stream(1, n, k, rows, epi == LM_EPI_GLU, true).slices;
+  return s > 1 ? (int64_t)s * rows * n : 0;
 }
 
 extern "C" int lm_gemm_tiles(const LmGemmPart* pa, const LmGemmPart* pb, int groups, const int* perm, const int* off,

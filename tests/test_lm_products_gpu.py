@@ -1,0 +1,86 @@
+"""The engine's products of few rows (csrc/lm/lm_gemm.hip): every width of a workgroup, K in parts and in slices, fewer stages than parts,
+row counts at the edges of 16, views with a row stride, the gated unit, one matrix per head, experts with many rows.  Against float64."""
+import numpy as np
+import pytest
+import torch
+
+from tests.hybrid_util import errors
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DTYPES = [torch.bfloat16, torch.float32]
+TOL = {torch.bfloat16: 4e-3, torch.float32: 2e-6}      # the output's rounding (2^-9 of a value); f32 sums
+
+
+def _ops(dtype):
+    from omniserve_amd.backend.lm import lm_ops
+    return lm_ops(dtype)
+
+
+def _randn(seed, dtype, *shape):
+    return torch.randn(shape, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV).to(dtype)
+
+
+def _close(got, want, dtype):
+    assert errors(got.float().cpu().numpy(), want.cpu().numpy()).max() < TOL[dtype]
+
+
+# one stage for four K parts; 16 .. 80 channels per workgroup; more than 256 of them; slices of K with an uneven rest
+SHAPES = [(1, 16, 64), (2, 48, 192), (15, 4096, 320), (16, 64, 4096), (17, 4112, 256), (31, 6208, 128), (32, 10816, 64), (33, 16448, 192),
+          (47, 12352, 64), (48, 1024, 8256), (49, 32016, 64), (64, 2048, 6144), (64, 528, 3136)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_products(m, n, k, dtype):
+    ops = _ops(dtype)
+    x, w = _randn(1, dtype, m, k + 64)[:, 64:], _randn(2, dtype, n, k) * k ** -0.5
+    want = x.double() @ w.double().t()
+    guard = torch.full((m + 2, n), 7.0, dtype=dtype, device=DEV)
+    _close(ops.matmul(x, w, out=guard[1:-1]), want, dtype)
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+    assert errors(ops.matmul(x, w, out_f32=True, scale=0.5).cpu().numpy(), 0.5 * want.cpu().numpy()).max() < 2e-6
+    assert torch.equal(ops.matmul(x, w), ops.matmul(x, w))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (16, 1040, 128), (33, 2064, 192), (64, 512, 4160), (48, 9216, 64)])
+def test_gated_unit(m, n, k, dtype):
+    ops = _ops(dtype)
+    x, w, b = _randn(3, dtype, m, k), _randn(4, dtype, 2 * n, k) * k ** -0.5, _randn(5, torch.float32, 2 * n) * 0.1
+    y = (x.double() @ w.double().t() + b.double()).view(m, n // 16, 2, 16)
+    want = (torch.nn.functional.gelu(y[:, :, 0], approximate="tanh") * y[:, :, 1]).reshape(m, n)
+    got = ops.glu(x, w, b, "gelu_tanh")
+    assert errors(got.float().cpu().numpy(), want.cpu().numpy()).max() < max(TOL[dtype], 5e-6)      # (the exponential's few ulp)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m", [1, 16, 50, 65, 130])
+@pytest.mark.parametrize("heads,n,k", [(32, 128, 512), (16, 256, 128), (3, 64, 64)])
+def test_one_matrix_per_head(heads, n, k, m, dtype):
+    ops = _ops(dtype)
+    x, w = _randn(6, dtype, m, heads * k), _randn(7, dtype, heads, n, k) * k ** -0.5
+    gate, out = _randn(8, dtype, m, heads * n), torch.empty((m, heads * n), dtype=dtype, device=DEV)
+    want = torch.cat([x[:, h * k:(h + 1) * k].double() @ w[h].double().t() for h in range(heads)], dim=1)
+    _close(ops.head_products(x, w, out, k, n), want, dtype)
+    got = ops.head_products(x, w, out, k, n, gate=gate)
+    assert errors(got.float().cpu().numpy(), (want * torch.sigmoid(gate.double())).cpu().numpy()).max() < max(TOL[dtype], 5e-6)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("tokens,skew", [(1, False), (16, False), (64, False), (64, True)])
+def test_experts(tokens, skew, dtype):
+    """skew: every token chooses the same experts, 64 rows each"""
+    ops = _ops(dtype)
+    E, top, ff, W = 6, 3, 192, 256
+    z, bias = _randn(9, torch.float32, tokens, E), torch.zeros((E,), device=DEV)
+    if skew:
+        z = z * 0 + torch.arange(E, device=DEV)
+    wts, order = ops.route(z.contiguous(), bias, E, top)
+    h, w, ws = _randn(10, dtype, tokens, W), _randn(11, dtype, E, ff, W) * W ** -0.5, _randn(12, dtype, 2 * ff, W) * W ** -0.5
+    y, ys = (torch.empty((r, c), dtype=dtype, device=DEV) for r, c in ((tokens * top, ff), (tokens, 2 * ff)))
+    ops.grouped(order, tokens, h, w, y, False, False, (h, ws, ys))
+    ids = torch.argsort(-z, dim=1, stable=True)[:, :top]
+    want = torch.einsum("tw,tcfw->tcf", h.double(), w.double()[ids]).reshape(tokens * top, ff)
+    _close(y, want, dtype)
+    _close(ys, h.double() @ ws.double().t(), dtype)
