@@ -3,7 +3,7 @@
 //
 //   lm_gemm_rows   few rows (decode): HBM bound.  A workgroup streams the weights of 16 - 80 channels of a group once, through an LDS
 //                  ring filled by DMA; the rows of x come the same way, shared by its waves.
-//   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 128 tiles, both operands by LDS-DMA, two stages ahead.
+//   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 256 tiles, both operands by LDS-DMA, a workgroup per CU that takes tile after tile.
 //
 // Epilogues: element type, f32 times a factor, the gated unit act(gate + bias) * (up + bias) of a matrix whose rows alternate in
 // blocks of 16 between gate and up channels (both halves of a pair then sit in the same lane), or the product with sigmoid(gate).
@@ -379,147 +379,305 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs p, const floa
   store4<EPI>(pt, m, c, 0, v, p.scale);
 }
 
-constexpr int TM = LM_TILE_ROWS, TN = 128;                  // rows, channels of a tile
-constexpr int SROWB = 64, SK = SROWB / (int)sizeof(elem_t);  // a stage: 64 bytes of k of every row
-constexpr int STAGE = (TM + TN) * SROWB, STAGES = 3;
+constexpr int TM = LM_TILE_ROWS, TN = 256;                  // rows, channels of a tile
+constexpr int SROWB = 128, SK = SROWB / (int)sizeof(elem_t); // a stage: 128 bytes of k of every row (whole lines of the L2)
+constexpr int STAGE = (TM + TN) * SROWB;
 static_assert(TM == 256, "the wave layout");
 
-// LDS rows of 64 bytes, four 16-byte slots and four rows to a 256-byte line: slot s of row r at s ^ (0, 2, 3, 1)[r / 4 % 4], with
-// the property Tile::swizzle has for fragment reads
-__device__ __forceinline__ int stage_swizzle(int row) {
-  const int q = (row >> 2) & 3;
-  return (((q ^ (q >> 1)) & 1) << 1) | (q >> 1);
+// c += a b with c pinned to its accumulation registers: left to the compiler, 64 tiles of a lone wave move between register files inside the
+// loop (100 moves per 64 products).  The compiler does not see a matrix instruction: mma_drain() stands between the last of them and a read of c.
+__device__ __forceinline__ void mma_in_place(f32x4& c, frag_t a, frag_t b) {
+#if LM_ELEM == 0
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+#else
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a[i]), "v"(b[i]));
+#endif
+}
+// three of them with one LDS-DMA request in their shadow: a lone wave issues an instruction every four cycles and a product takes sixteen, so
+// at most three others fit between two products.  SADDR: src is a 32-bit offset from base.
+template <bool SADDR, typename S>
+__device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag_t a0, frag_t a1, frag_t a2, frag_t b, S src, const void* base,
+                                           uint32_t lds_dst) {
+#if LM_ELEM == 0
+  uint32_t keep;
+  if constexpr (SADDR)
+    asm volatile(
+        "v_mfma_f32_16x16x32_bf16 %1, %4, %7, %1\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %9\n\tv_mfma_f32_16x16x32_bf16 %2, %5, %7, %2\n\t"
+        "global_load_lds_dwordx4 %8, %10\n\tv_mfma_f32_16x16x32_bf16 %3, %6, %7, %3\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep), "+a"(c0), "+a"(c1), "+a"(c2)
+        : "v"(a0), "v"(a1), "v"(a2), "v"(b), "v"(src), "s"(lds_dst), "s"(base)
+        : "memory");
+  else
+    asm volatile(
+        "v_mfma_f32_16x16x32_bf16 %1, %4, %7, %1\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %9\n\tv_mfma_f32_16x16x32_bf16 %2, %5, %7, %2\n\t"
+        "global_load_lds_dwordx4 %8, off\n\tv_mfma_f32_16x16x32_bf16 %3, %6, %7, %3\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep), "+a"(c0), "+a"(c1), "+a"(c2)
+        : "v"(a0), "v"(a1), "v"(a2), "v"(b), "v"(src), "s"(lds_dst)
+        : "memory");
+#else
+  mma_in_place(c0, a0, b);
+  mma_in_place(c1, a1, b);
+  if constexpr (SADDR) dma16_uncounted((const uint8_t*)base + src, lds_dst);
+  else dma16_uncounted(src, lds_dst);
+  mma_in_place(c2, a2, b);
+#endif
+}
+// a value the optimiser knows nothing about: what is computed from it is computed where it stands, not kept across a loop
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// the lane, computed where it stands: no register holds it, or what is computed from it, across a loop
+__device__ __forceinline__ int lane_here() {
+  int v;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
+  return v;
+}
+template <int N, int M>
+__device__ __forceinline__ void mma_drain(f32x4 (&c)[N][M]) {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(c[i][j]));      // (a later value: no read of it moves up)
 }
 
-// 4 waves, 128 rows x 64 channels each; three stages: while one multiplies, two are on their way
+// 4 waves, 128 rows x 128 channels each.  A wave's operands are 16 fragments for 64 MFMAs (256 accumulator registers, one wave per SIMD):
+// with 64 x 128 per wave and two workgroups per CU the LDS had 72 KB to move per 512 MFMA cycles and SIMD, more than its 128 B per clock.
+// Nothing overlaps with a lone wave but what it issues itself: the fragments of a half stage are read while the half before it
+// multiplies, a stage ahead of it is requested.
+//
+// A workgroup takes tile after tile: the first two stages of the next one are on their way while it stores this one (16 us passed between
+// the products of a tile and those of the next where every tile had a workgroup; a stage takes 1 us and K = 640 has 10 of them).
+//
+// MI355X, bf16, before: 256 x 128 tiles of 64-byte stages, a workgroup per tile, two of them on a CU.  7999
+// tokens, 6 of 32 experts of 1792, width 4096: 2407 -> 1883 us up (998 TFLOP/s with the rows of the half empty tiles not counted), 1084 ->
+// 938 down; 6733 tokens, 8 of 64 experts of 640, width 2048: 410 -> 382 up, 256 -> 259 down; 8192 x 7168 x 4096 to f32: 569 -> 469.
 template <int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[STAGES * STAGE];
-  __shared__ int y_row[TM];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l15 = lane & 15, l4 = lane >> 4;
-  // linear order: bands of row tiles, all channel tiles of a band before the next one; of both parts a contiguous range per XCD
+__global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
+  constexpr bool DIRECT = EPI == LM_EPI_F32 || sizeof(elem_t) == 4;      // accumulators straight to memory
+  constexpr int OC = EPI == LM_EPI_GLU ? 64 : 128, PITCH = OC * (int)sizeof(elem_t) + 16, OUT = DIRECT ? 0 : 4 * 16 * PITCH;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE + OUT];
+  __shared__ int y_rows[2][TM];
+  typedef Tile<SROWB> T;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // linear order of a part: bands of row tiles, all channel tiles of a band before the next one; an XCD has a contiguous range of both
+  // parts, its workgroups take the tiles of it in turn
   const int nt_a = (p.a.n + TN - 1) / TN, nt_b = mt_b ? (p.b.n + TN - 1) / TN : 0;
-  const int wgs_b = 8 * ((mt_b * nt_b + 7) >> 3);
-  const bool is_b = (int)blockIdx.x < wgs_b;
-  const Part& pt = is_b ? p.b : p.a;
-  const int nt = is_b ? nt_b : nt_a, mts = is_b ? mt_b : mt_a;
-  const int id = xcd_contiguous(is_b ? blockIdx.x : blockIdx.x - wgs_b, mts * nt);
-  if (id < 0) return;
-  constexpr int GM = 4;
-  const int band = id / (GM * nt), in = id - band * GM * nt, bm = min(GM, mts - band * GM);
-  const int mi = band * GM + in % bm, ni = in / bm;
-  const int* perm = is_b ? nullptr : p.perm;
-  int first = mi * TM, rows, g = 0;
-  if (perm) {
-    const i32x4 t = *(const i32x4*)(p.tiles + 4 * mi);       // group, first place, rows
-    if (t[2] <= 0) return;
-    g = t[0];
-    first = t[1];
-    rows = t[2];
-  } else {
-    rows = min(TM, (is_b ? p.rows_b : p.rows_a) - first);
-  }
-  const int n0 = ni * TN;
-  const elem_t* w = pt.w + (int64_t)g * pt.n * pt.k;
-  // pieces of 16 rows: lane -> (row lane / 4, physical slot lane % 4); a wave carries 2 of the weights' and 4 of x's
-  const elem_t *wsrc[2], *xsrc[4];
-  const int pr = lane >> 2, ps = (lane & 3) ^ stage_swizzle(pr);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = min(16 * (4 * wave + i) + pr, rows - 1);
-    const int xr = perm ? perm[first + r] / p.x_div : first + r;
-    xsrc[i] = pt.x + (int64_t)xr * pt.ldx + ps * FR;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = w + (int64_t)min(n0 + 16 * (2 * wave + i) + pr, pt.n - 1) * pt.k + ps * FR;
-  y_row[tid] = tid < rows ? (perm ? perm[first + tid] : first + tid) : -1;
+  const int per_a = (mt_a * nt_a + 7) >> 3, per_b = (mt_b * nt_b + 7) >> 3, xcd = blockIdx.x & 7;
+  const int own_b = max(0, min(per_b, mt_b * nt_b - xcd * per_b)), own = own_b + max(0, min(per_a, mt_a * nt_a - xcd * per_a));
+  int at = blockIdx.x >> 3;                                 // in the XCD's range
+
+  // pieces of 8 rows: lane -> (row lane / 8, physical slot lane % 8); a wave carries 8 of the weights' and 8 of x's.  (A row of the tile past
+  // the matrix: its last one again; none of it is stored.)
+  const uint8_t* xsrc[8];
+  uint32_t woff[8];                                         // from the tile's first channel
+  const uint8_t* wbase = nullptr;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
-  const int uw = __builtin_amdgcn_readfirstlane(wave);
-  auto stage = [&](int st, int k0) {
-    const uint32_t dst = lds0 + st * STAGE;
+  const uint32_t dst0 = __builtin_amdgcn_readfirstlane(lds0 + 64 * SROWB * wave);
+  auto dst = [&](int t, int i) { return dst0 + (t & 1) * STAGE + 1024 * (i & 7) + (i < 8 ? 0 : TN * SROWB); };      // of piece i
+  auto stage = [&](int t) {                                 // requests the next stage of k
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_uncounted(wsrc[i] + k0, dst + 1024 * (2 * uw + i));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dma16_uncounted(xsrc[i] + k0, dst + TN * SROWB + 1024 * (4 * uw + i));
+    for (int i = 0; i < 16; ++i) {
+      if (i < 8) dma16_uncounted(wbase + woff[i], dst(t, i));
+      else {
+        dma16_uncounted(xsrc[i & 7], dst(t, i));
+        xsrc[i & 7] += SROWB;
+      }
+    }
+    wbase += SROWB;
   };
-  const int wn = 64 * (wave & 1), wm = 128 * (wave >> 1);
-  f32x4 acc[4][8];
+  bool is_b = false;
+  int n0 = 0, ns = 0;
+  // the next tile with rows from place `at` on: its rows of y, its first two stages requested; false: there is none
+  auto open_tile = [&](int (&y_row)[TM]) {
+    for (; at < own; at += (int)gridDim.x >> 3) {
+      is_b = at < own_b;
+      const Part& pt = is_b ? p.b : p.a;
+      const int nt = is_b ? nt_b : nt_a, mts = is_b ? mt_b : mt_a;
+      const int id = is_b ? xcd * per_b + at : xcd * per_a + at - own_b;
+      constexpr int GM = 4;
+      const int band = id / (GM * nt), in = id - band * GM * nt, bm = min(GM, mts - band * GM);
+      const int mi = band * GM + in % bm;
+      const int* perm = is_b ? nullptr : p.perm;
+      int first = mi * TM, rows, g = 0;
+      if (perm) {
+        const i32x4 t = *(const i32x4*)(p.tiles + 4 * mi);     // group, first place, rows
+        if (t[2] <= 0) continue;
+        g = t[0];
+        first = t[1];
+        rows = t[2];
+      } else {
+        rows = min(TM, (is_b ? p.rows_b : p.rows_a) - first);
+      }
+      const int ol = lane_here(), pr = ol >> 3, ps = ol & 7, otid = 64 * wave + ol, x_div = opaque(p.x_div);
+      n0 = in / bm * TN;
+      ns = pt.k / SK;
+      wbase = (const uint8_t*)(pt.w + ((int64_t)g * pt.n + n0) * pt.k);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 8; ++i) {
+        const int r = 64 * wave + 8 * i + pr, rc = min(r, rows - 1);
+        woff[i] = (uint32_t)min(r, pt.n - 1 - n0) * (uint32_t)(pt.k * (int)sizeof(elem_t)) + ((ps ^ T::swizzle(r)) << 4);
+        const int xr = perm ? perm[first + rc] / x_div : first + rc;
+        xsrc[i] = (const uint8_t*)(pt.x + (int64_t)xr * pt.ldx) + ((ps ^ T::swizzle(r)) << 4);
+      }
+      y_row[otid] = otid < rows ? (perm ? perm[first + otid] : first + otid) : -1;
+      wait_pieces<0>();                                     // the compiler's own loads
+      stage(0);
+      if (ns > 1) stage(1);
+      at += (int)gridDim.x >> 3;
+      return true;
+    }
+    return false;
+  };
+
+  const int wn = 128 * (wave & 1), wm = 128 * (wave >> 1);
+  int off[2];                                               // of a fragment of half u inside 16 rows
+  frag_t a[2][8], b[2][8];
+  auto fetch_b = [&](int t, auto half, int i) {
+    constexpr int U = decltype(half)::value;
+    b[U][i] = *(const frag_t*)(lds + (t & 1) * STAGE + 16 * SROWB * i + off[U] + (TN + wm) * SROWB);
+  };
+  auto fetch_a = [&](int t, auto half, int i) {
+    constexpr int U = decltype(half)::value;
+    a[U][i] = *(const frag_t*)(lds + (t & 1) * STAGE + 16 * SROWB * i + off[U] + wn * SROWB);
+  };
+  f32x4 acc[8][8];
+  // Stage t: MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products: a burst of
+  // them fills the queues of the address path and the LDS, and the lone wave, which issues in order, waits there with its matrix
+  // unit idle.  No condition inside: reads and products have to share a basic block.
+  auto step = [&](int t, auto more, auto dma) {
+    constexpr bool MORE = decltype(more)::value, DMA = decltype(dma)::value;
+    auto four = [&](auto half, int i0, int j) {
+      constexpr int U = decltype(half)::value;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = zero4();
-  const int nk = pt.k / SK;                                 // (>= 2: k is a multiple of 64)
-  const int lane_off = l15 * SROWB + ((l4 ^ stage_swizzle(l15)) << 4);
-  wait_pieces<0>();                                         // the compiler's own loads
-  stage(0, 0);
-  stage(1, SK);
-  int st = 0;
-  for (int t = 0; t < nk; ++t) {
-    if (t + 1 < nk) wait_pieces<6>();                       // stage t is there, the 6 pieces of t + 1 may still fly
-    else wait_pieces<0>();
-    __builtin_amdgcn_s_barrier();                           // ... for every wave, and everyone has left stage t - 1
-    asm volatile("" ::: "memory");
-    if (t + 2 < nk) stage(st == 0 ? 2 : st - 1, (t + 2) * SK);
-    const uint8_t* wt = lds + st * STAGE + wn * SROWB + lane_off;
-    const uint8_t* xt = lds + st * STAGE + (TN + wm) * SROWB + lane_off;
-    frag_t a[4], b[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = *(const frag_t*)(wt + 16 * SROWB * i);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b[j] = *(const frag_t*)(xt + 16 * SROWB * j);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][j] = mma(a[i], b[j], acc[i][j]);
-    __builtin_amdgcn_s_setprio(0);
-    st = st == 2 ? 0 : st + 1;
-  }
-  __syncthreads();                                          // the stages are free
-  if constexpr (EPI == LM_EPI_F32) {
+      for (int i = i0; i < i0 + 4; ++i) mma_in_place(acc[i][j], a[U][i], b[U][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int row = y_row[wm + 16 * j + l15];
-      if (row < 0) continue;
+      fetch_b(t, Int<1>{}, j);
+      __builtin_amdgcn_sched_barrier(0);
+      four(Int<0>{}, 0, j);
+      fetch_a(t, Int<1>{}, j);
+      __builtin_amdgcn_sched_barrier(0);
+      four(Int<0>{}, 4, j);
+    }
+    // stage t + 1 is there for every wave, and everyone has stage t in registers
+    if constexpr (MORE) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = n0 + wn + 16 * i + 4 * l4;
-        if (c < pt.n) store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (MORE) fetch_b(t + 1, Int<0>{}, j);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (DMA) {
+        mma3_dma16<true>(acc[0][j], acc[1][j], acc[2][j], a[1][0], a[1][1], a[1][2], b[1][j], woff[j], wbase, dst(t, j));
+        mma_in_place(acc[3][j], a[1][3], b[1][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        four(Int<1>{}, 0, j);
+      }
+      if constexpr (MORE) fetch_a(t + 1, Int<0>{}, j);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (DMA) {
+        mma3_dma16<false>(acc[4][j], acc[5][j], acc[6][j], a[1][4], a[1][5], a[1][6], b[1][j], xsrc[j], nullptr, dst(t, 8 + j));
+        xsrc[j] += SROWB;
+        mma_in_place(acc[7][j], a[1][7], b[1][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        four(Int<1>{}, 4, j);
       }
     }
-  } else {
-    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 32 rows of the wave's at a time
-    constexpr int OC = EPI == LM_EPI_GLU ? 32 : 64, PITCH = OC * (int)sizeof(elem_t) + 16, PPR = OC / FR;
-    static_assert(4 * 32 * PITCH <= STAGES * STAGE, "the waves' buffers");
-    uint8_t* buf = lds + wave * 32 * PITCH;
+    if constexpr (DMA) wbase += SROWB;
+  };
+
+  int parity = 0;
+  bool open = open_tile(y_rows[0]);
+  while (open) {
+    const float z = __builtin_bit_cast(float, opaque(0));   // (no register of zeros across the tiles)
 #pragma unroll
-    for (int part = 0; part < 4; ++part) {
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const int j = 2 * part + jj;
+      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{z, z, z, z};
+    // stage 0 is there: of what was requested last -- stage 1, or stores of the tile before -- 16 may still fly
+    if (ns > 1) wait_pieces<16>();
+    else wait_pieces<0>();
+    __syncthreads();
+    const int fl = lane_here();
 #pragma unroll
-        for (int i = 0; i < 4; i += EPI == LM_EPI_GLU ? 2 : 1) {
-          f32x4 v = acc[i][j];
-          int c = 16 * i;
-          if constexpr (EPI == LM_EPI_GLU) {
-            c = 8 * i;
-            if (n0 + wn + 16 * i < pt.n) v = glu(pt, p.act, n0 + wn + 16 * i + 4 * l4, v, acc[i + 1][j]);
-          }
-          *(quad_t*)(buf + (16 * jj + l15) * PITCH + (c + 4 * l4) * (int)sizeof(elem_t)) = to_quad(v);
+    for (int u = 0; u < 2; ++u) off[u] = T::slot(fl & 15, 4 * u + (fl >> 4));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      fetch_b(0, Int<0>{}, i);
+      fetch_a(0, Int<0>{}, i);
+    }
+    int t = 0;
+    for (; t + 2 < ns; ++t) step(t, Int<1>{}, Int<1>{});
+    if (t + 1 < ns) {
+      step(t, Int<1>{}, Int<0>{});
+      ++t;
+    }
+    step(t, Int<0>{}, Int<0>{});                            // (behind its barrier both stages are free)
+    mma_drain(acc);
+
+    const Part& pt = is_b ? p.b : p.a;
+    const int el = lane_here(), e15 = el & 15, e4 = el >> 4;
+    const int c0 = n0 + wn;                                 // the wave's first channel
+    const int* y_row = y_rows[parity];
+    // the results, packed; then the next tile
+    constexpr int NI = EPI == LM_EPI_GLU ? 4 : 8;
+    quad_t out[DIRECT ? 1 : 8][NI];
+    if constexpr (!DIRECT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          if constexpr (EPI == LM_EPI_GLU) out[j][i] = to_quad(glu(pt, p.act, min(c0 + 32 * i, pt.n - 32) + 4 * e4, acc[2 * i][j], acc[2 * i + 1][j]));
+          else out[j][i] = to_quad(acc[i][j]);
         }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int i = 0; i < 32 * PPR / 64; ++i) {
-        const int pc = 64 * i + lane, r = pc / PPR, q = pc % PPR;
-        const int row = y_row[wm + 32 * part + r], c = (EPI == LM_EPI_GLU ? (n0 + wn) / 2 : n0 + wn) + q * FR;
-        if (row >= 0 && c < (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n))
-          *(frag_t*)((elem_t*)pt.y + (int64_t)row * pt.ldy + c) = *(const frag_t*)(buf + r * PITCH + q * 16);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      open = open_tile(y_rows[parity ^ 1]);
     }
+    if constexpr (DIRECT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int row = y_row[wm + 16 * j + e15];
+        if (row < 0) continue;
+#pragma unroll
+        for (int i = 0; i < 8; i += EPI == LM_EPI_GLU ? 2 : 1) {
+          const int c = c0 + 16 * i + 4 * e4;
+          if (c >= pt.n) continue;
+          if constexpr (EPI == LM_EPI_GLU) store4<EPI>(pt, row, (c0 + 16 * i) / 2 + 4 * e4, 0, glu(pt, p.act, c, acc[i][j], acc[i + 1][j]), p.scale);
+          else store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
+        }
+        __builtin_amdgcn_sched_barrier(0);                  // (no addresses of later rows kept beside the accumulators)
+      }
+      open = open_tile(y_rows[parity ^ 1]);
+    } else {
+      // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
+      constexpr int PPR = OC / FR;
+      uint8_t* buf = lds + 2 * STAGE + wave * 16 * PITCH;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) *(quad_t*)(buf + e15 * PITCH + (16 * i + 4 * e4) * (int)sizeof(elem_t)) = out[j][i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 16 * PPR / 64; ++i) {
+          const int pc = 64 * i + el, r = pc / PPR, q = pc % PPR;
+          const int row = y_row[wm + 16 * j + r], c = (EPI == LM_EPI_GLU ? c0 / 2 : c0) + q * FR;
+          if (row >= 0 && c < (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n))
+            *(frag_t*)((elem_t*)pt.y + (int64_t)row * pt.ldy + c) = *(const frag_t*)(buf + r * PITCH + q * 16);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    parity ^= 1;
   }
 }
 
@@ -658,7 +816,8 @@ extern "C" int lm_gemm_tiles(const LmGemmPart* pa, const LmGemmPart* pb, int gro
   const int mt_a = perm ? max_tiles : (rows_a + TM - 1) / TM, mt_b = pb && rows_b > 0 ? (rows_b + TM - 1) / TM : 0;
   const int64_t tiles_a = (int64_t)mt_a * ((a.a.n + TN - 1) / TN), tiles_b = mt_b ? (int64_t)mt_b * ((a.b.n + TN - 1) / TN) : 0;
   if (tiles_a <= 0 || tiles_a + tiles_b > (1 << 30)) return LM_EINVAL;
-  const dim3 grid((unsigned)(8 * ((tiles_a + 7) / 8) + 8 * ((tiles_b + 7) / 8)));
+  // a workgroup per CU
+  const dim3 grid((unsigned)min((int64_t)256, 8 * ((tiles_a + 7) / 8 + (tiles_b + 7) / 8)));
   hipStream_t s = (hipStream_t)stream;
   if (epi == LM_EPI_ELEM) hipLaunchKernelGGL((gemm_tiles_kernel<LM_EPI_ELEM>), grid, dim3(256), 0, s, a, mt_a, mt_b);
   else if (epi == LM_EPI_F32) hipLaunchKernelGGL((gemm_tiles_kernel<LM_EPI_F32>), grid, dim3(256), 0, s, a, mt_a, mt_b);

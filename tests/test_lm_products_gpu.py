@@ -9,7 +9,7 @@ from tests.hybrid_util import errors
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 DTYPES = [torch.bfloat16, torch.float32]
-TOL = {torch.bfloat16: 4e-3, torch.float32: 2e-6}      # the output's rounding (2^-9 of a value); f32 sums
+TOL = {torch.bfloat16: 4e-3, torch.float32: 2e-6}      # the output's rounding (up to 2^-8 of a value); f32 sums
 
 
 def _ops(dtype):
@@ -23,6 +23,13 @@ def _randn(seed, dtype, *shape):
 
 def _close(got, want, dtype):
     assert errors(got.float().cpu().numpy(), want.cpu().numpy()).max() < TOL[dtype]
+
+
+def _rows_close(got, want, dtype):
+    """Rounding a value to bf16 moves it by at most 2^-8 of itself (7 fraction bits), so a row's error is at most 2^-8 of the row's own norm (5 % for the f32
+    sums in front of it); in f32 the exponential's few ulp."""
+    d = (got.double().cpu() - want.cpu()).norm(dim=1) / want.cpu().norm(dim=1)
+    assert d.max() < (1.05 * 2.0 ** -8 if dtype == torch.bfloat16 else 5e-6)
 
 
 # one stage for four K parts; 16 .. 80 channels per workgroup; more than 256 of them; slices of K with an uneven rest
@@ -84,3 +91,53 @@ def test_experts(tokens, skew, dtype):
     want = torch.einsum("tw,tcfw->tcf", h.double(), w.double()[ids]).reshape(tokens * top, ff)
     _close(y, want, dtype)
     _close(ys, h.double() @ ws.double().t(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k", [(65, 144, 64), (256, 256, 128), (257, 272, 192), (700, 1040, 320), (1300, 528, 1792)])
+def test_tiles(m, n, k, dtype):
+    """many rows: two stages of k and more, one tile and parts of tiles in both directions"""
+    ops = _ops(dtype)
+    x, w = _randn(13, dtype, m, k + 64)[:, 64:], _randn(14, dtype, n, k) * k ** -0.5
+    guard = torch.full((m + 2, n), 7.0, device=DEV)
+    ops.matmul(x, w, out=guard[1:-1], out_f32=True)
+    assert errors(guard[1:-1].cpu().numpy(), (x.double() @ w.double().t()).cpu().numpy()).max() < 2e-6
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("tokens,E,top,ff,W,skew", [(66, 6, 3, 192, 256, False), (300, 4, 2, 272, 320, True), (1000, 8, 2, 64, 128, False)])
+def test_experts_of_a_prompt(tokens, E, top, ff, W, skew, dtype):
+    """experts without rows, with whole tiles and parts of them; the gated unit and the plain product, a shared expert beside them"""
+    ops = _ops(dtype)
+    z, bias = _randn(15, torch.float32, tokens, E), torch.zeros((E,), device=DEV)
+    if skew:
+        z = z * 0 + torch.arange(E, device=DEV)
+    wts, order = ops.route(z.contiguous(), bias, E, top)
+    h = _randn(16, dtype, tokens, W)
+    wi, ws = _randn(17, dtype, E, 2 * ff, W) * W ** -0.5, _randn(18, dtype, 96, W) * W ** -0.5
+    wo, wd = _randn(19, dtype, E, W, (ff + 63) // 64 * 64) * ff ** -0.5, _randn(20, dtype, W, 64) * 0.1
+    act = torch.zeros((tokens * top, wo.shape[2]), dtype=dtype, device=DEV)
+    acts, y = torch.zeros((tokens, 64), dtype=dtype, device=DEV), torch.empty((tokens * (top + 1), W), dtype=dtype, device=DEV)
+    ops.grouped(order, tokens, h, wi, act, False, True, (h, ws, acts))
+    ids = torch.argsort(-z, dim=1, stable=True)[:, :top].cpu()
+
+    def glu(x, w):
+        v = (x @ w.t()).view(x.shape[0], w.shape[0] // 32, 2, 16)
+        return (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(x.shape[0], w.shape[0] // 2)
+
+    hd = h.double().cpu()
+    want, wid, wod = torch.empty((tokens * top, ff), dtype=torch.float64), wi.double().cpu(), wo.double().cpu()
+    for e in range(E):
+        t, c = torch.nonzero(ids == e, as_tuple=True)
+        want[t * top + c] = glu(hd[t], wid[e])
+    _rows_close(act[:, :ff], want, dtype)
+    _rows_close(acts[:, :48], glu(hd, ws.double().cpu()), dtype)
+    ops.grouped(order, tokens, act, wo, y, True, False, (acts, wd, y[tokens * top:]))
+    down = torch.empty((tokens * top, W), dtype=torch.float64)
+    a = act.double().cpu()
+    for e in range(E):
+        t, c = torch.nonzero(ids == e, as_tuple=True)
+        down[t * top + c] = a[t * top + c] @ wod[e].t()
+    _rows_close(y[:tokens * top], down, dtype)
+    _rows_close(y[tokens * top:], acts.double() @ wd.double().t(), dtype)
