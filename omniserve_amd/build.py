@@ -54,7 +54,7 @@ def _hipcc() -> str:
 
 def _deps_mtime(*roots) -> float:
     m = 0.0
-    for root in roots or (CSRC, INCLUDE):
+    for root in roots or (CSRC, LM_CSRC, INCLUDE):      # (qgemm_tiles.h takes a header of the engine's)
         for f in os.listdir(root):
             if f.endswith((".hip", ".h", ".cpp")):
                 m = max(m, os.path.getmtime(os.path.join(root, f)))

@@ -8,6 +8,7 @@
 // Epilogues: element type, f32 times a factor, the gated unit act(gate + bias) * (up + bias) of a matrix whose rows alternate in
 // blocks of 16 between gate and up channels (both halves of a pair then sit in the same lane), or the product with sigmoid(gate).
 #include "lm_common.h"
+#include "mfma_pinned.h"
 #include "omniserve_lm.h"
 
 namespace lm {
@@ -384,37 +385,22 @@ constexpr int SROWB = 128, SK = SROWB / (int)sizeof(elem_t); // a stage: 128 byt
 constexpr int STAGE = (TM + TN) * SROWB;
 static_assert(TM == 256, "the wave layout");
 
-// c += a b with c pinned to its accumulation registers: left to the compiler, 64 tiles of a lone wave move between register files inside the
-// loop (100 moves per 64 products).  The compiler does not see a matrix instruction: mma_drain() stands between the last of them and a read of c.
+// c += a b, c pinned (mfma_pinned.h)
 __device__ __forceinline__ void mma_in_place(f32x4& c, frag_t a, frag_t b) {
 #if LM_ELEM == 0
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  OMNI_MFMA_PINNED("v_mfma_f32_16x16x32_bf16", c, a, b);
 #else
 #pragma unroll
-  for (int i = 0; i < 4; ++i) asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a[i]), "v"(b[i]));
+  for (int i = 0; i < 4; ++i) OMNI_MFMA_PINNED("v_mfma_f32_16x16x4_f32", c, a[i], b[i]);
 #endif
 }
-// three of them with one LDS-DMA request in their shadow: a lone wave issues an instruction every four cycles and a product takes sixteen, so
-// at most three others fit between two products.  SADDR: src is a 32-bit offset from base.
+// three of them and an LDS-DMA request.  SADDR: src is a 32-bit offset from base.
 template <bool SADDR, typename S>
 __device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag_t a0, frag_t a1, frag_t a2, frag_t b, S src, const void* base,
                                            uint32_t lds_dst) {
 #if LM_ELEM == 0
-  uint32_t keep;
-  if constexpr (SADDR)
-    asm volatile(
-        "v_mfma_f32_16x16x32_bf16 %1, %4, %7, %1\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %9\n\tv_mfma_f32_16x16x32_bf16 %2, %5, %7, %2\n\t"
-        "global_load_lds_dwordx4 %8, %10\n\tv_mfma_f32_16x16x32_bf16 %3, %6, %7, %3\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep), "+a"(c0), "+a"(c1), "+a"(c2)
-        : "v"(a0), "v"(a1), "v"(a2), "v"(b), "v"(src), "s"(lds_dst), "s"(base)
-        : "memory");
-  else
-    asm volatile(
-        "v_mfma_f32_16x16x32_bf16 %1, %4, %7, %1\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %9\n\tv_mfma_f32_16x16x32_bf16 %2, %5, %7, %2\n\t"
-        "global_load_lds_dwordx4 %8, off\n\tv_mfma_f32_16x16x32_bf16 %3, %6, %7, %3\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep), "+a"(c0), "+a"(c1), "+a"(c2)
-        : "v"(a0), "v"(a1), "v"(a2), "v"(b), "v"(src), "s"(lds_dst)
-        : "memory");
+  if constexpr (SADDR) OMNI_MFMA3_DMA16("v_mfma_f32_16x16x32_bf16", "%10", c0, c1, c2, a0, a1, a2, b, src, base, lds_dst);
+  else OMNI_MFMA3_DMA16("v_mfma_f32_16x16x32_bf16", "off", c0, c1, c2, a0, a1, a2, b, src, 0, lds_dst);
 #else
   mma_in_place(c0, a0, b);
   mma_in_place(c1, a1, b);
@@ -422,25 +408,6 @@ __device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag
   else dma16_uncounted(src, lds_dst);
   mma_in_place(c2, a2, b);
 #endif
-}
-// a value the optimiser knows nothing about: what is computed from it is computed where it stands, not kept across a loop
-__device__ __forceinline__ int opaque(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-// the lane, computed where it stands: no register holds it, or what is computed from it, across a loop
-__device__ __forceinline__ int lane_here() {
-  int v;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
-  return v;
-}
-template <int N, int M>
-__device__ __forceinline__ void mma_drain(f32x4 (&c)[N][M]) {
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(c[i][j]));      // (a later value: no read of it moves up)
 }
 
 // 4 waves, 128 rows x 128 channels each.  A wave's operands are 16 fragments for 64 MFMAs (256 accumulator registers, one wave per SIMD):
@@ -621,7 +588,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       ++t;
     }
     step(t, Int<0>{}, Int<0>{});                            // (behind its barrier both stages are free)
-    mma_drain(acc);
+    accumulators_settle(acc);
 
     const Part& pt = is_b ? p.b : p.a;
     const int el = lane_here(), e15 = el & 15, e4 = el >> 4;

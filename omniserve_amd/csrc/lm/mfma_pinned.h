@@ -1,0 +1,44 @@
+// Matrix instructions of a wave that has its SIMD to itself and 256 accumulator registers.
+//
+//  * The accumulators are pinned to accumulation registers ("+a"): left to the compiler, 64 tiles of a lone wave move between the register
+//    files inside the loop (100 moves per 64 products).
+//  * A lone wave issues an instruction every four cycles and a product takes sixteen: at most three others fit between two products.
+//    OMNI_MFMA3_DMA16 is three products with one LDS-DMA request in their shadow.
+//  * The compiler does not see a matrix instruction here: accumulators_settle() stands between the last of them and a read of the results.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#define OMNI_MFMA_PINNED(OP, c, a, b) asm volatile(OP " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b))
+
+// ADDR: "%10" with a scalar base and src a 32-bit offset from it, "off" with src an address (base is then ignored).  M0 is the compiler's:
+// saved and restored.
+#define OMNI_MFMA3_DMA16(OP, ADDR, c0, c1, c2, a0, a1, a2, b, src, base, lds_dst)                                            \
+  do {                                                                                                                      \
+    uint32_t keep_m0;                                                                                                       \
+    asm volatile(OP " %1, %4, %7, %1\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %9\n\t" OP " %2, %5, %7, %2\n\t"                   \
+                 "global_load_lds_dwordx4 %8, " ADDR "\n\t" OP " %3, %6, %7, %3\n\ts_mov_b32 m0, %0"                         \
+                 : "=&s"(keep_m0), "+a"(c0), "+a"(c1), "+a"(c2)                                                             \
+                 : "v"(a0), "v"(a1), "v"(a2), "v"(b), "v"(src), "s"(lds_dst), "s"(base)                                      \
+                 : "memory");                                                                                               \
+  } while (0)
+
+// a value the optimiser knows nothing about: what is computed from it is computed where it stands, not kept across a loop
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// the lane, computed where it stands: no register holds it, or what is computed from it, across a loop
+__device__ __forceinline__ int lane_here() {
+  int v;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
+  return v;
+}
+template <typename V, int N, int M>
+__device__ __forceinline__ void accumulators_settle(V (&c)[N][M]) {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(c[i][j]));      // (a later value: no read of it moves up)
+}

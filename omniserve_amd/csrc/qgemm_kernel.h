@@ -560,6 +560,7 @@ __global__ __launch_bounds__(64 * WAVES, OMNI_GEMM_MIN_BLOCKS) void w4a8_gemm_ke
 
 }  // namespace omni
 #include "qgemm_exact.h"
+#include "qgemm_tiles.h"
 #include "qgemm_midm.h"
 namespace omni {
 
@@ -1197,7 +1198,8 @@ extern "C" void omni_gemm_set_midm_override(int mode, int sk);
 extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, int* sk);
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool w8 = false);
 
-// w4a8_gemm_exact_kernel's tile height (16-row blocks), K parts inside a workgroup, K slices over the grid (1: no slabs)
+// w4a8_gemm_exact_kernel's tile height (16-row blocks; 16: w8a8_tiles_kernel), K parts inside a workgroup, K slices over the grid (1: no
+// slabs)
 struct PrefillPlan {
   int mb, kw, sk;
 };
@@ -1232,11 +1234,27 @@ static void launch_exact_rows(const GemmArgs& a, int mb, int sk, hipStream_t st)
   }
 }
 
+// a workgroup per CU
+template <int MODE>
+static void launch_tiles(GemmArgs b, hipStream_t st) {
+  b.tiles_n = b.N / TILES_N;
+  b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
+  const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
+  b.band = (b.tiles_m + bands - 1) / bands;
+  hipLaunchKernelGGL((w8a8_tiles_kernel<MODE>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+}
+
 // prefill regime (M > 128): chunked LDS staging, weights through L2
 template <int MODE>
 static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
   if (exact_shape(a, false)) {
     const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false);
+    if constexpr (MODE == MODE_W8) {
+      if (pp.mb == 16) {
+        launch_tiles<MODE>(a, st);
+        return;
+      }
+    }
     if (pp.sk > 1) {
       launch_exact_rows<MODE, 1, true>(a, pp.mb, pp.sk, st);
       const size_t total = (size_t)a.M * (a.N / 4);

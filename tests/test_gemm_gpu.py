@@ -385,3 +385,11 @@ def test_prefill_rows_not_whole_tiles(mode, M, N, K):
 @pytest.mark.parametrize("mode", ["chn", "grp", "w8"])
 def test_prefill_tile_heights(mode, M, N, K):
     {"chn": lambda: _run_chn(M, N, K, seed=M), "grp": lambda: _run_grp(M, N, K, False), "w8": lambda: _run_w8(M, N, K)}[mode]()
+
+
+# W8A8 in 256 x 256 tiles (sizes at which plan_prefill's model picks them): one tile per workgroup and more, 8 .. 32 stages of K, last row
+# tiles of 1 row to all of them.
+@pytest.mark.parametrize("M,N,K", [(512, 18944, 1536), (768, 13312, 1536), (1281, 7936, 2048), (1537, 6656, 2048), (1024, 10240, 2048), (2017, 13824, 1024),
+                                   (333, 28672, 4096)])
+def test_w8a8_whole_tiles(M, N, K):
+    _run_w8(M, N, K)
