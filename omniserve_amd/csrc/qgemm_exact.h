@@ -196,6 +196,7 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
     __syncthreads();          // chunk c is visible in lds[c & 1]; everybody is done reading lds[(c + 1) & 1]
     const uint8_t* abuf = smem + (c & 1) * (MT * KCHUNK);
 
+    const bool small = MODE == MODE_GRP && MB < 8 && grp_scales_small(gs[0], gs[1]);      // (MB = 8 has no registers for both forms)
     // unpack (+ lane transpose / per-group dequant) of k-step s into MFMA A operands
     auto unpack = [&](int s, v4i (&wa)[4]) {
       if constexpr (W8C) {
@@ -223,6 +224,13 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
             const auto s01 = __builtin_amdgcn_permlane16_swap((uint32_t)s02[0], (uint32_t)s13[0], false, false);
             const auto s23 = __builtin_amdgcn_permlane16_swap((uint32_t)s02[1], (uint32_t)s13[1], false, false);
             d[b][0] = (uint32_t)s01[0]; d[b][1] = (uint32_t)s01[1]; d[b][2] = (uint32_t)s23[0]; d[b][3] = (uint32_t)s23[1];
+          }
+        }
+        if constexpr (MODE == MODE_GRP) {
+          if (small) {
+#pragma unroll
+            for (int ab = 0; ab < 4; ++ab) wa[ab] = grp_unpack_small(d[ab & 1], gs[s >> 1], gz[s >> 1], ab >> 1, ab & 1);
+            return;
           }
         }
 #pragma unroll

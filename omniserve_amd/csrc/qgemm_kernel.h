@@ -121,6 +121,34 @@ __device__ __forceinline__ void vadd4_zbyte_x4(uint32_t (&u)[4], uint32_t zw, in
   }
 }
 
+// Second level of per-group weights, u * scale + zero per byte, without the quarter-rate multiply and the four byte adds per word: the bytes
+// of a word are multiplied and added in 16-bit lanes, even and odd ones apart, and joined (5.5 full-rate operations per word, 9.5
+// equivalents before).  The general form multiplies whole words: a product above 255 spills into the neighbouring byte.  The lanes
+// would not; so this form is for scales up to 17 (15 * 17 = 255; a level that covers an int8 range with 16 steps needs no more), and
+// a wave with a larger one among its channels takes the general one.  The straight-line prefill kernel has both, up to 112-row tiles (MI355X:
+// 1501 rows of 4096 x 14336 116 -> 100 us, 2331 rows 182 -> 173, 768 rows of 6144 x 4096 36.1 -> 33.9); in the decode kernels the
+// branch costs more than the operations it saves (61 rows of 28672 x 4096 18.3 -> 19.5 us).
+// d: words of 8 weights; lower (a = 0) or upper (a = 1) nibbles, byte 2 a + b of the scale and zero dwords.
+__device__ __forceinline__ v4i grp_unpack_small(const uint32_t (&d)[4], uint32_t sc4, uint32_t z4, int a, int b) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  const uint32_t byte_twice = 0x0c000c00u + 0x00010001u * (uint32_t)(2 * a + b);      // {byte, 0, byte, 0}
+  const u16x2 sc = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, sc4, byte_twice));
+  const u16x2 ze = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, z4, byte_twice)), zo = ze << 8;
+  v4i w;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t x = d[q] >> (4 * a);
+    const u16x2 e = __builtin_bit_cast(u16x2, x & 0x000F000Fu) * sc + ze, o = __builtin_bit_cast(u16x2, x & 0x0F000F00u) * sc + zo;
+    w[q] = (int)((__builtin_bit_cast(uint32_t, e) & 0x00FF00FFu) | (__builtin_bit_cast(uint32_t, o) & 0xFF00FF00u));
+  }
+  return w;
+}
+// is none of the wave's scales (bytes of both words) above 17?
+__device__ __forceinline__ bool grp_scales_small(uint32_t s, uint32_t t) {
+  const uint32_t over = (((s & 0x7F7F7F7Fu) + 0x6E6E6E6Eu) | s | ((t & 0x7F7F7F7Fu) + 0x6E6E6E6Eu) | t) & 0x80808080u;
+  return __builtin_amdgcn_ballot_w64(over != 0) == 0;
+}
+
 // (the f32 result is made opaque before the fp16 conversion: hipcc otherwise may fold `(half)(f32 * f32)` into
 //  v_fma_mixlo_f16 -- ONE rounding where the reference rounds to f32 first; one output in ~10^4 then differs by an ulp,
 //  depending on the code around the call: seen in w4a8_gemm_exact_kernel (round 3) and in w4a8_midm_kernel's store forms)

@@ -393,3 +393,24 @@ def test_prefill_tile_heights(mode, M, N, K):
                                    (333, 28672, 4096)])
 def test_w8a8_whole_tiles(M, N, K):
     _run_w8(M, N, K)
+
+
+# Per-group weights whose second level is unpacked in 16-bit lanes (scales up to 17) in some chunks and in whole words (a scale above 17) in
+# others: the edge between the two forms, in the prefill kernel's tile heights and both of its K splits.
+@pytest.mark.parametrize("M,N,K", [(140, 512, 1024), (333, 512, 2048), (300, 512, 768), (449, 16384, 256), (700, 16384, 256)])
+def test_per_group_scales_around_the_lane_limit(M, N, K):
+    import omniserve_backend.qgemm_w4a8_per_group as mod
+    u, z, s2, s1 = w4a8.synth_per_group(N, K, seed=M)
+    rng = np.random.default_rng(M)
+    s2[:] = rng.integers(14, 18, size=s2.shape)            # products up to 255, to within one of the limit
+    big = rng.random(s2.shape) < 0.004                     # ... and a few beyond it
+    big[N // 2, 1] = big[N - 1, -1] = True
+    s2[big] = rng.integers(18, 41, size=int(big.sum()))
+    u[:, 0] = 15
+    qw, s1h, s2s, s2z = w4a8.pack_per_group(u, z, s2, s1)
+    a, sa, _ = _acts(M, K, M + 2)
+    want = w4a8.gemm_per_group(a, qw, s2z, s2s, s1h, sa)
+    out = torch.empty((M, N), dtype=torch.float16, device=dev())
+    mod.gemm_forward_cuda(to_dev(a), to_dev(qw), to_dev(s2z), to_dev(s2s), to_dev(s1h), to_dev(sa), out)
+    torch.cuda.synchronize()
+    assert_f16_equal(out, want, "per_group M=%d N=%d K=%d" % (M, N, K))
