@@ -539,7 +539,7 @@ struct DeltaDecodeArgs {
   int H, G;
 };
 
-template <int DK, int DV>
+template <int DK, int DV, bool STREAM>
 __global__ __launch_bounds__(4 * DV) void delta_decode_kernel(DeltaDecodeArgs p) {
   constexpr int TH = 4 * DV, COLS = DV / 4, ROWS = DK / STATE_GROUPS;
   __shared__ __attribute__((aligned(16))) float qkv[2 * DK + DV];
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(4 * DV) void delta_decode_kernel(DeltaDecodeArgs p)
   float* S = p.state + ((int64_t)slot * p.H + h) * DK * DV + 4 * col + (int64_t)grp * ROWS * DV;
   f32x4 s[ROWS];                         // requested before anything waits
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) s[i] = ps > 0 ? *(const f32x4*)(S + (int64_t)i * DV) : zero4();
+  for (int i = 0; i < ROWS; ++i) s[i] = ps > 0 ? load_state<STREAM>((const f32x4*)(S + (int64_t)i * DV)) : zero4();
   // convolution of this head's channels.  The ring has a row more than the inputs it is asked for: the new input (stored by every
   // head that uses it, equal bytes) replaces none that another workgroup still reads.
   float* ring = p.ring + (int64_t)slot * p.taps * channels;
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(4 * DV) void delta_decode_kernel(DeltaDecodeArgs p)
   for (int i = 0; i < ROWS; ++i) {
     s[i] += (rk * qkv[DK + grp * ROWS + i]) * u;
     acc += qkv[grp * ROWS + i] * s[i];
-    *(f32x4*)(S + (int64_t)i * DV) = s[i];
+    store_state<STREAM>((f32x4*)(S + (int64_t)i * DV), s[i]);
   }
   const f32x4 y = rq * over_groups<DV>(acc, red[1], grp, col);
   if (tid < COLS) {
@@ -661,7 +661,10 @@ extern "C" int lm_delta_decode(const void* x, int64_t ld, void* o, int64_t ldo, 
   hipStream_t s = (hipStream_t)stream;
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
-    hipLaunchKernelGGL((delta_decode_kernel<K, V>), dim3(B, H), dim3(4 * V), 0, s, a);                       \
+    if (streams_state(B, H, K, V))                                                                           \
+      hipLaunchKernelGGL((delta_decode_kernel<K, V, true>), dim3(B, H), dim3(4 * V), 0, s, a);               \
+    else                                                                                                     \
+      hipLaunchKernelGGL((delta_decode_kernel<K, V, false>), dim3(B, H), dim3(4 * V), 0, s, a);              \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)

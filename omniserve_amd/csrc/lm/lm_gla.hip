@@ -370,7 +370,7 @@ struct GlaDecodeArgs {
   int H;
 };
 
-template <int DK, int DV>
+template <int DK, int DV, bool STREAM>
 __global__ __launch_bounds__(4 * DV) void gla_decode_kernel(GlaDecodeArgs p) {
   constexpr int TH = 4 * DV, COLS = DV / 4, ROWS = DK / STATE_GROUPS;
   static_assert(TH == COLS * STATE_GROUPS, "layout");
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(4 * DV) void gla_decode_kernel(GlaDecodeArgs p) {
   float* S = p.state + ((int64_t)p.slot[b] * p.H + h) * DK * DV + 4 * col + (int64_t)grp * ROWS * DV;
   f32x4 s[ROWS];                         // requested before anything waits
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) s[i] = ps > 0 ? *(const f32x4*)(S + (int64_t)i * DV) : zero4();
+  for (int i = 0; i < ROWS; ++i) s[i] = ps > 0 ? load_state<STREAM>((const f32x4*)(S + (int64_t)i * DV)) : zero4();
   const f32x4 v = from_quad(*(const quad_t*)(row + (int64_t)2 * p.H * DK + (int64_t)h * DV + 4 * col));
   for (int d = tid; d < DK; d += TH) {
     const elem_t *a = p.a2 + (int64_t)(h * DK + d) * p.rp, *t = row + p.low_col;
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(4 * DV) void gla_decode_kernel(GlaDecodeArgs p) {
     const int d = grp * ROWS + i;
     s[i] = as[d] * s[i] + ks[d] * v;
     acc += qs[d] * s[i];
-    *(f32x4*)(S + (int64_t)i * DV) = s[i];
+    store_state<STREAM>((f32x4*)(S + (int64_t)i * DV), s[i]);
   }
   const f32x4 y = over_groups<DV>(acc, red, grp, col);
   if (tid < COLS) {
@@ -465,7 +465,10 @@ extern "C" int lm_gla_decode(const void* x, int64_t ld, void* o, int64_t ldo, fl
   hipStream_t s = (hipStream_t)stream;
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
-    hipLaunchKernelGGL((gla_decode_kernel<K, V>), dim3(B, H), dim3(4 * V), 0, s, a);                         \
+    if (streams_state(B, H, K, V))                                                                           \
+      hipLaunchKernelGGL((gla_decode_kernel<K, V, true>), dim3(B, H), dim3(4 * V), 0, s, a);                 \
+    else                                                                                                     \
+      hipLaunchKernelGGL((gla_decode_kernel<K, V, false>), dim3(B, H), dim3(4 * V), 0, s, a);                \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)
