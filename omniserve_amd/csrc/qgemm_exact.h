@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
   // one batch of scalar loads for the prologue's kernel arguments (hipcc otherwise fetches them in three dependent groups --
   // tile order, K slice, pointers -- in front of the first tile request)
   asm volatile("" ::"s"(p.A), "s"(p.W), "s"(p.wscales), "s"(p.ascales), "s"(p.wsz), "s"(p.asum), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.kslice),
-               "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.band), "s"((int)gridDim.x), "s"((int)gridDim.y));
+               "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.tile_linear), "s"((int)gridDim.x), "s"((int)gridDim.y));
 
 #ifdef OMNI_DEBUG_CLOCKS
   const unsigned long long tl0 = wall_clock64();
@@ -85,10 +85,10 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
     const int per = tiles >> 3, more = tiles & 7;
     if (i >= per + (xcd < more)) return;
     const int t = xcd * per + min(xcd, more) + i;
-    const int band = t / (p.band * p.tiles_n), in = t - band * p.band * p.tiles_n;
-    const int rows = min(p.band, p.tiles_m - band * p.band);
+    const int band = t / (p.tile_linear * p.tiles_n), in = t - band * p.tile_linear * p.tiles_n;
+    const int rows = min(p.tile_linear, p.tiles_m - band * p.tile_linear);
     tile_n = in / rows;
-    tile_m = band * p.band + in - tile_n * rows;
+    tile_m = band * p.tile_linear + in - tile_n * rows;
   }
   const int ng = tile_n * WAVES + wave;  // 64-channel group of this wave
   // M need not be whole tiles: the last row tile starts at M - MT and computes the rows it shares with the one before a second time

@@ -46,8 +46,8 @@ struct GemmArgs {
   int64_t out_stride;
   int kslice;             // k per split (multiple of 64)
   int tiles_m, tiles_n;   // > 0: 1-D grid with the XCD-aware tile order of w4a8_gemm_kernel
-  int tile_linear;        // 1 (with tiles_n > 0): workgroup w = tile (w % tiles_m, w / tiles_m) -- few row tiles
-  int band;               // w4a8_gemm_exact_kernel: row tiles per band of its tile order
+  int tile_linear;        // 1 (with tiles_n > 0): workgroup w = tile (w % tiles_m, w / tiles_m) -- few row tiles; w4a8_gemm_exact_kernel and
+                          // w8a8_tiles_kernel: row tiles per band of their order (a field of its own would move the decode kernels' arguments)
   // ---- row-kernel-free decode forms (fused extension; see w4a8_gemv_kernel EPI / A16) ----
   const half_t* A16;      // [M,K] fp16 activations quantised on the fly (A16 kernels; `A` unused)
   uint32_t* amax;         // [AMAX_WORDS] row-maximum candidates (common.h): EPI = 1 raises them, A16 reads them
@@ -1246,7 +1246,7 @@ static void launch_exact_tile(GemmArgs b, int sk, hipStream_t st) {
   b.tiles_n = b.N / 256;
   b.tiles_m = (b.M + MB * 16 - 1) / (MB * 16);
   const int bands = (b.tiles_m + 7) / 8;
-  b.band = (b.tiles_m + bands - 1) / bands;
+  b.tile_linear = (b.tiles_m + bands - 1) / bands;
   const int tiles = b.tiles_m * b.tiles_n;
   hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, MB, KW, TO_SLAB>), dim3((tiles + 7) / 8 * 8, sk, 1), dim3(256 * KW), 0, st, b);
 }
@@ -1268,7 +1268,7 @@ static void launch_tiles(GemmArgs b, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;
   b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
   const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
-  b.band = (b.tiles_m + bands - 1) / bands;
+  b.tile_linear = (b.tiles_m + bands - 1) / bands;
   hipLaunchKernelGGL((w8a8_tiles_kernel<MODE>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
 }
 

@@ -75,11 +75,11 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
   // one before are computed twice, to the same bits.
   auto open_tile = [&]() {
     if (at >= own) return false;
-    const int id = first + at, band = id / (p.band * p.tiles_n), in = id - band * p.band * p.tiles_n;
-    const int rows = min(p.band, p.tiles_m - band * p.band), tn = in / rows;
+    const int id = first + at, band = id / (p.tile_linear * p.tiles_n), in = id - band * p.tile_linear * p.tiles_n;
+    const int rows = min(p.tile_linear, p.tiles_m - band * p.tile_linear), tn = in / rows;
     at += (int)gridDim.x >> 3;
     n0 = tn * TILES_N;
-    m0 = min((band * p.band + in - tn * rows) * TILES_M, p.M - TILES_M);
+    m0 = min((band * p.tile_linear + in - tn * rows) * TILES_M, p.M - TILES_M);
     wbase = p.W + (size_t)n0 * p.K;
     abase = (const uint8_t*)p.A + (size_t)m0 * p.K;
     const int tid = 64 * wave + lane_here();
