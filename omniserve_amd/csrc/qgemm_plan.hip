@@ -216,7 +216,7 @@ static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, 
 
 // w8a8_tiles_kernel: rounds of a tile per CU.  A stage takes 0.95 us where few CUs have a tile and 1.4 where all have one; 8 us a tile for its
 // ends, which is what short K loses here.  (MI355X, this kernel against the best tile height of the other: 12001 rows of 28672 x 4096 1193 us /
-// 1403, of 4096 x 14336 555 / 720, of 16640 x 1024 237 / 252, of 16384 x 256 116 / 111; 2331 rows of 6144 x 4096 51 / 62; 1501 rows of 4096 x
+// 1403, of 4096 x 14336 561 / 656, of 16640 x 1024 237 / 252, of 16384 x 256 116 / 111; 2331 rows of 6144 x 4096 51 / 62; 1501 rows of 4096 x
 // 14336, 96 tiles, 128 / 95.)
 static float tiles_time(long long tiles, int stages) {
   const long long rounds = tiles / 256;

@@ -11,7 +11,7 @@
 //
 // Integer sums and the general kernel's epilogue: the same bits.
 //
-// MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 720 -> 555 (2540 TOPS); what
+// MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 656 -> 561 (2510 TOPS); what
 // is left of the 5 POPS nominal: the clock under this load and, at 28672 channels, 690 MB of results.
 #pragma once
 #include "lm/mfma_pinned.h"
