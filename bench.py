@@ -101,10 +101,9 @@ def _time_projection(runner, name):
             fn(i)
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
+    from omniserve_amd.persistent import record
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
-        for i in range(nl):
-            fn(i)
+    record(g, lambda: [fn(i) for i in range(nl)])
     g.replay()
     torch.cuda.synchronize()
     reps = 6
@@ -128,10 +127,9 @@ def _graph_time_ms(fn, nl, reps=6):
             fn(i)
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
+    from omniserve_amd.persistent import record
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
-        for i in range(nl):
-            fn(i)
+    record(g, lambda: [fn(i) for i in range(nl)])
     g.replay()
     torch.cuda.synchronize()
     s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

@@ -102,9 +102,10 @@ class Engine:
         key = (places, width)
         if key not in self._graphs:
             slots, out = DecodeSlots(self.builder, places, width), {}
+            model, cache = self.model, self.cache   # (not self: an engine and its graphs go with the last reference to it)
 
             def step():
-                out["logits"] = self.model.forward(slots.batch, self.cache)
+                out["logits"] = model.forward(slots.batch, cache)
 
             graph = GraphedStep(step, self.device)
             graph.capture()                         # every place is empty: neither the cache nor the state is touched

@@ -24,6 +24,7 @@ from .backend import (activation_ops, fused_attention_ctx_pool, fused_attention_
                       fused_attention_fine_grained_sparse, fused_attention_per_tensor_dense,
                       fused_attention_per_tensor_sparse, fused_attention_selector, fused_ext, fused_kernels, layernorm_ops,
                       prefill_attn, qgemm_w8a8)
+from .persistent import record
 from .rope import rope_table
 from .runtime import LlamaConfig
 from . import _lib
@@ -474,8 +475,7 @@ class LServeDecodeRunner:
                     p.copy_(q)
             torch.cuda.current_stream().wait_stream(s)
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                self._eager_step(hist, select)
+            record(g, lambda: self._eager_step(hist, select))
             self.graphs[key] = g
             # the capture itself did not execute: replay below does
         g.replay()

@@ -20,6 +20,9 @@ reference's call sequence and checks it against the eager run, with no allocatio
 """
 from __future__ import annotations
 
+import contextlib
+import gc
+import threading
 import types
 from typing import Callable, Optional
 
@@ -71,6 +74,36 @@ class PersistentActivationBuffer:
         return v
 
 
+_recording_lock = threading.Lock()
+_recordings, _collector_was_on = 0, False
+
+
+@contextlib.contextmanager
+def _collector_held():
+    """Python's cyclic collector off, in every thread, until the last of the recordings under way has ended."""
+    global _recordings, _collector_was_on
+    with _recording_lock:
+        if _recordings == 0:
+            _collector_was_on = gc.isenabled()
+            gc.disable()
+        _recordings += 1
+    try:
+        yield
+    finally:
+        with _recording_lock:
+            _recordings -= 1
+            if _recordings == 0 and _collector_was_on:
+                gc.enable()
+
+
+def record(graph: "torch.cuda.CUDAGraph", fn: Callable[[], None]) -> None:
+    """Records fn into graph.  A CUDAGraph's destructor waits for the device, which nothing may do while a stream records: the error
+    leaves a destructor and the process ends.  A graph in a reference cycle dies wherever the collector happens to run, so it does
+    not run here; what it would have taken goes in its next run behind the recording."""
+    with _collector_held(), torch.cuda.graph(graph):
+        fn()
+
+
 class GraphedStep:
     """One HIP graph around a step function whose inputs and outputs live in persistent device tensors."""
 
@@ -93,8 +126,7 @@ class GraphedStep:
                 restore()
         torch.cuda.current_stream(self.device).wait_stream(side)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            self.fn()
+        record(graph, self.fn)
         if restore is not None:
             restore()
         self.graph = graph

@@ -21,6 +21,7 @@ import torch
 
 from .backend import (activation_ops, fused_attention_pure_dense, fused_ext, fused_kernels, layernorm_ops,
                       qgemm_w4a8_per_chn, qgemm_w4a8_per_group)
+from .persistent import record
 from .rope import rope_table
 from . import _lib
 
@@ -344,8 +345,7 @@ class DecodeRunner:
             torch.cuda.current_stream().wait_stream(s)
             try:
                 graph = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(graph):
-                    self._eager_step()
+                record(graph, self._eager_step)
                 self.graph = graph
             except RuntimeError as exc:  # (e.g. a collective that cannot be captured on this stack)
                 if self.tp_size == 1:
