@@ -1231,14 +1231,17 @@ GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool 
 struct PrefillPlan {
   int mb, kw, sk;
 };
-// sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs
+// sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs (omni_gemm_set_plan_override's K splits do, too)
 PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only);
 
 // shapes the straight-line kernel takes: whole channel tiles and K chunks (also of a K slice: a.kslice); it stores 16 B
 // per lane, so rows of an fp16 output must start 16-B aligned
+static inline bool exact_sizes(int M, int N, int K, int kslice) {
+  return M > 128 && N % 256 == 0 && K % KCHUNK == 0 && kslice % KCHUNK == 0 && (size_t)M * K < ((size_t)1 << 32);
+}
 static inline bool exact_shape(const GemmArgs& a, bool to_slab) {
   const bool out16 = to_slab || ((a.out_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0);
-  return a.M > 128 && a.N % 256 == 0 && a.K % KCHUNK == 0 && a.kslice % KCHUNK == 0 && (size_t)a.M * a.K < ((size_t)1 << 32) && out16;
+  return exact_sizes(a.M, a.N, a.K, a.kslice) && out16;
 }
 
 template <int MODE, int MB, int KW, bool TO_SLAB>

@@ -236,7 +236,7 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
     if (t < time) { time = t; best = PrefillPlan{mb, kw, split}; }
   };
   for (int mb = 8; mb >= 4; --mb) {
-    if (slab_only) {
+    if (slab_only || g_override_sk > 0) {
       offer(mb, 1, sk);
       continue;
     }
@@ -244,7 +244,7 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
     if (K % (2 * KCHUNK) == 0) offer(mb, 2, 1);
     if (sk > 1) offer(mb, 1, sk);
   }
-  if (mode == MODE_W8 && !slab_only && M >= TILES_M && tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < time)
+  if (mode == MODE_W8 && !slab_only && g_override_sk <= 0 && M >= TILES_M && tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < time)
     best = PrefillPlan{16, 1, 1};
   return best;
 }
@@ -266,6 +266,18 @@ extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int
   if (mb) *mb = pl.mb;
   if (waves) *waves = pl.waves;
   if (sk) *sk = pl.sk;
+}
+
+extern "C" int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int slabs_only, int* mb, int* kw, int* sk) {
+  using namespace omni;
+  if (M <= 128 || N < 64 || N % 64 || K < 64 || K % 64 || mode < 0 || mode > 2 || (slabs_only && M > 512)) return 0;
+  const GemmPlan pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, slabs_only != 0, mode == MODE_W8);
+  const bool exact = exact_sizes(M, N, K, pl.kslice);
+  const PrefillPlan pp = exact ? plan_prefill(M, N, K, mode, pl.sk, slabs_only != 0) : PrefillPlan{8, 1, pl.sk};
+  if (mb) *mb = pp.mb;
+  if (kw) *kw = pp.kw;
+  if (sk) *sk = pp.sk;
+  return exact ? 1 : 2;
 }
 
 // Would the row-kernel-free decode forms (omni_*_gemm_silu for gate_up, omni_*_gemm_partial_f16 for o / down) accept a layer

@@ -150,6 +150,50 @@ def test_gemm_plans_of_the_baseline_decode_shapes():
     assert lib.omni_gemm_rowfree_ok(16, 512, 512, 1024, 0) == 0            # more rows than hidden / 64 rider workgroups
 
 
+def _prefill_plan(M, N, K, mode, slabs_only=0):
+    import ctypes
+    from omniserve_amd import _lib
+    v = [ctypes.c_int(0) for _ in range(3)]
+    return (_lib.lib().omni_gemm_get_prefill_plan(M, N, K, mode, slabs_only, *map(ctypes.byref, v)), *(x.value for x in v))
+
+
+def test_prefill_plans_fit_the_kernels_and_the_scratch():
+    """What more than 128 rows run as (no GPU): the forms that exist, K slices only as many as the plan's scratch holds."""
+    import random
+    from omniserve_amd import _lib
+    lib, rng, seen = _lib.lib(), random.Random(5), set()
+    assert _prefill_plan(128, 4096, 4096, 0)[0] == 0 and _prefill_plan(513, 4096, 4096, 0, 1)[0] == 0 and _prefill_plan(200, 4096, 4096, 3)[0] == 0
+    for M, N, K in ((200, 320, 1024), (200, 512, 448), (4097, 64, 64)):
+        assert _prefill_plan(M, N, K, 0)[:3] == (2, 8, 1)
+    for _ in range(20000):
+        M = int(129 * 100 ** rng.random())
+        N, K, mode, slabs = 256 * rng.randint(1, 64), 256 * rng.randint(1, 32), rng.randrange(3), int(M <= 512 and rng.random() < 0.4)
+        which, mb, kw, sk = _prefill_plan(M, N, K, mode, slabs)
+        assert which == 1 and kw in (1, 2) and K % (256 * kw * sk) == 0
+        assert mb in (4, 5, 6, 7, 8) or (mb == 16 and mode == 2 and kw == sk == 1 and not slabs and M >= 256)
+        assert 16 * mb <= M                                   # the last tile starts at M less its height
+        if slabs:
+            assert kw == 1 and lib.omni_gemm_partial_workspace_bytes(M, N, K) >= sk * M * N * 4
+        elif sk > 1:
+            assert kw == 1 and lib.omni_gemm_workspace_bytes(M, N, K) >= sk * M * N * 4
+        seen.add((mb, kw, sk > 1))
+    assert seen >= {(mb, kw, False) for mb in range(4, 9) for kw in (1, 2)} | {(mb, 1, True) for mb in range(4, 9)} | {(16, 1, False)}
+
+
+def test_forced_k_splits_reach_the_prefill_plan():
+    from omniserve_amd import _lib
+    lib = _lib.lib()
+    for M, N, K in ((256, 6144, 4096), (256, 4096, 4096), (300, 512, 2048), (512, 4096, 4096)):
+        for mode in range(3):
+            for sk in (1, 2, 4):
+                lib.omni_gemm_set_plan_override(0, sk)
+                try:
+                    which, _, kw, got = _prefill_plan(M, N, K, mode)
+                finally:
+                    lib.omni_gemm_set_plan_override(0, 0)
+                assert (which, kw, got) == (1, 1, sk), (M, N, K, mode, sk)
+
+
 def test_release_library_reads_no_environment():
     """Release hygiene: the planner / debug knobs (OMNI_GEMV_DBG, OMNI_GEMV_NARROW, ...) exist only in
     -DOMNI_TUNING builds; the shipped library neither imports getenv nor carries their names."""

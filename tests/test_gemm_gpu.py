@@ -52,8 +52,9 @@ def test_per_chn_prefill_shapes(M, N, K):
 
 
 # Decode at batch 129 .. 512 (the reference's published A100 figure is quoted at bs = 256): few 128 x 256 tiles, so the plan
-# splits K over grid.y into int32 slabs + the slab epilogue (qgemm_plan.hip: down_proj 8 ways, o_proj / qkv 4 ways at
-# bs = 256; gate_up has 224 tiles and stays whole).  Ragged M (row tiles partly filled), all three flavours.
+# offers K slices over grid.y into int32 slabs + the slab epilogue (qgemm_plan.hip: down_proj 8 ways, o_proj / qkv 4 ways at
+# bs = 256; gate_up has 224 tiles and stays whole), with scratch for them; whether they run is plan_prefill's choice (forced, with
+# the tile heights: test_prefill_forms).  Ragged M (row tiles partly filled), all three flavours.
 FEW_TILE_SHAPES = [(256, 4096, 14336), (256, 6144, 4096), (256, 4096, 4096), (129, 4096, 14336), (300, 512, 2048), (512, 4096, 4096)]
 
 
@@ -396,7 +397,8 @@ def test_w8a8_whole_tiles(M, N, K):
 
 
 # Per-group weights whose second level is unpacked in 16-bit lanes (scales up to 17) in some chunks and in whole words (a scale above 17) in
-# others: the edge between the two forms, in the prefill kernel's tile heights and both of its K splits.
+# others: the edge between the two forms.  (Tiles of 64 rows whole and with K slices over the grid, 96 rows; 128 rows, which have the second
+# form only.  K in two parts inside a workgroup: test_per_group_scales_around_the_lane_limit_two_k_parts.)
 @pytest.mark.parametrize("M,N,K", [(140, 512, 1024), (333, 512, 2048), (300, 512, 768), (449, 16384, 256), (700, 16384, 256)])
 def test_per_group_scales_around_the_lane_limit(M, N, K):
     import omniserve_backend.qgemm_w4a8_per_group as mod
@@ -414,3 +416,82 @@ def test_per_group_scales_around_the_lane_limit(M, N, K):
     mod.gemm_forward_cuda(to_dev(a), to_dev(qw), to_dev(s2z), to_dev(s2s), to_dev(s1h), to_dev(sa), out)
     torch.cuda.synchronize()
     assert_f16_equal(out, want, "per_group M=%d N=%d K=%d" % (M, N, K))
+
+
+def _prefill_plan(mode, M, N, K, slabs_only=False):
+    """(rows / 16 of a tile, K parts inside a workgroup, K slices over the grid) of the straight-line kernels; None: the general kernel"""
+    import ctypes
+    from omniserve_amd import _lib
+    mb, kw, sk = (ctypes.c_int(0) for _ in range(3))
+    which = _lib.lib().omni_gemm_get_prefill_plan(M, N, K, MODES.index(mode), int(slabs_only), ctypes.byref(mb), ctypes.byref(kw), ctypes.byref(sk))
+    assert which in (1, 2)
+    return (mb.value, kw.value, sk.value) if which == 1 else None
+
+
+MODES = ["chn", "grp", "w8"]
+# Every instantiation of the straight-line kernels that plan_prefill takes somewhere, with the plan that is to run: whole K, two K parts that
+# meet in LDS, K slices over the grid with the slab epilogue.
+PREFILL_FORMS = [(m, *f) for m in MODES for f in (
+    (4, 1, 1, 129, 256, 256), (5, 1, 1, 324, 12288, 256), (7, 1, 1, 404, 12288, 256), (8, 1, 1, 449, 16384, 256),
+    (5, 1, 8, 129, 3072, 8192), (8, 1, 8, 229, 3072, 8192)) if not (m == "w8" and f[0] == 7)] + [
+    (m, *f) for m in MODES for f in ((6, 1, 1, 700, 16384, 256), (5, 2, 1, 513, 8192, 2048), (8, 2, 1, 449, 16384, 2048))] + [
+    ("chn", 4, 2, 1, 300, 512, 2048), ("chn", 6, 2, 1, 161, 28672, 4096), ("chn", 7, 2, 1, 385, 16384, 4096),
+    ("chn", 4, 1, 4, 129, 256, 4096), ("chn", 7, 1, 8, 164, 3072, 8192),
+    ("grp", 4, 2, 1, 700, 256, 2048), ("grp", 6, 2, 1, 333, 16384, 2048), ("grp", 7, 2, 1, 385, 16384, 2048),
+    ("grp", 4, 1, 2, 300, 512, 2048), ("grp", 6, 1, 8, 164, 6144, 8192), ("grp", 7, 1, 8, 164, 3072, 8192),
+    ("w8", 7, 1, 1, 484, 12288, 256), ("w8", 4, 2, 1, 300, 512, 2048), ("w8", 6, 2, 1, 333, 16384, 2048), ("w8", 7, 2, 1, 385, 16384, 2048),
+    ("w8", 4, 1, 4, 256, 4096, 4096), ("w8", 6, 1, 8, 164, 3072, 8192), ("w8", 7, 1, 8, 194, 3072, 8192),
+    ("w8", 16, 1, 1, 512, 18944, 1536), ("w8", 16, 1, 1, 2369, 17920, 1024)]      # the last: up to three 256 x 256 tiles per workgroup
+# ... and of the slab-only calls, which take the K slices as they are
+SLAB_FORMS = [(m, *f) for m in MODES for f in ((4, 4, 256, 4096, 4096), (5, 8, 129, 3072, 8192), (8, 8, 229, 3072, 8192), (5, 1, 324, 12288, 256))] + [
+    ("chn", 6, 8, 164, 6144, 8192), ("chn", 7, 8, 164, 3072, 8192), ("grp", 6, 8, 164, 6144, 8192), ("grp", 7, 8, 164, 3072, 8192),
+    ("w8", 6, 8, 164, 3072, 8192), ("w8", 7, 8, 194, 3072, 8192)]
+
+
+@pytest.mark.parametrize("mode,mb,kw,sk,M,N,K", PREFILL_FORMS)
+def test_prefill_forms(mode, mb, kw, sk, M, N, K):
+    assert _prefill_plan(mode, M, N, K) == (mb, kw, sk)
+    {"chn": lambda: _run_chn(M, N, K, seed=M, out_view=True), "grp": lambda: _run_grp(M, N, K, True), "w8": lambda: _run_w8(M, N, K)}[mode]()
+
+
+@pytest.mark.parametrize("mode,mb,sk,M,N,K", SLAB_FORMS)
+def test_prefill_slab_forms(mode, mb, sk, M, N, K):
+    """Sums of the slabs: the exact accumulators; what lies behind them stays as it was."""
+    from omniserve_amd.backend import fused_ext
+    assert _prefill_plan(mode, M, N, K, slabs_only=True) == (mb, 1, sk)
+    rng = np.random.default_rng(M + N)
+    a = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+    if mode == "w8":
+        w = rng.integers(-128, 128, size=(N, K), dtype=np.int8)
+        call, want = lambda s: fused_ext.gemm_partial_w8a8(to_dev(a), to_dev(w), s), w4a8._int_matmul_fast(a, w)
+    elif mode == "chn":
+        qw = rng.integers(-128, 128, size=(N, K // 2), dtype=np.int8)
+        call, want = lambda s: fused_ext.gemm_partial_per_chn(to_dev(a), to_dev(qw), s), w4a8.gemm_per_chn_acc(a, qw)
+    else:
+        u, z, s2, s1 = w4a8.synth_per_group(N, K, seed=M, wrap=True)
+        qw, _, s2s, s2z = w4a8.pack_per_group(u, z, s2, s1)
+        call = lambda s: fused_ext.gemm_partial_per_group(to_dev(a), to_dev(qw), to_dev(s2z), to_dev(s2s), s)      # noqa: E731
+        want = w4a8.gemm_per_group_acc(a, qw, s2z, s2s)
+    slab = torch.full((sk + 1, M, N), 7, dtype=torch.int32, device=dev())
+    assert call(slab) == sk
+    torch.cuda.synchronize()
+    assert (slab[sk:] == 7).all() and np.array_equal(slab[:sk].sum(dim=0).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("M,N,K,sk", [(140, 256, 4096, 2), (255, 256, 2048, 4), (300, 512, 2048, 2), (512, 4096, 4096, 2)])
+def test_prefill_forced_k_slices(mode, M, N, K, sk):
+    """omni_gemm_set_plan_override's K splits run as they are asked for"""
+    from omniserve_amd import _lib
+    _lib.lib().omni_gemm_set_plan_override(0, sk)
+    try:
+        assert _prefill_plan(mode, M, N, K)[1:] == (1, sk)
+        {"chn": lambda: _run_chn(M, N, K, seed=M), "grp": lambda: _run_grp(M, N, K, True), "w8": lambda: _run_w8(M, N, K)}[mode]()
+    finally:
+        _lib.lib().omni_gemm_set_plan_override(0, 0)
+
+
+@pytest.mark.parametrize("mb,M,N,K", [(4, 700, 256, 2048), (5, 513, 8192, 2048), (6, 333, 16384, 2048), (7, 385, 16384, 2048)])
+def test_per_group_scales_around_the_lane_limit_two_k_parts(mb, M, N, K):
+    assert _prefill_plan("grp", M, N, K) == (mb, 2, 1)
+    test_per_group_scales_around_the_lane_limit(M, N, K)
