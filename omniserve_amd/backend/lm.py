@@ -183,7 +183,7 @@ class LmOps:
 
     # ---- products ------------------------------------------------------------------------------------------------
     def _slices(self, x, w, epi):
-        """room for the sums of w's K slices"""
+        """room for the sums of w's K slices (kept by the caller until the call has enqueued what uses it)"""
         n = self._h.lm_gemm_rows_scratch(w.shape[0], w.shape[1], x.shape[0], epi)
         return torch.empty((n,), dtype=torch.float32, device=x.device) if n else None
 
@@ -198,7 +198,8 @@ class LmOps:
         part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), n, w.shape[1])
         epi = EPI_F32 if out_f32 else EPI_ELEM
         if T <= ROWS_MAX or n <= NARROW:
-            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, scale, epi, 0, _p(self._slices(x, w, epi)))
+            sums = self._slices(x, w, epi)
+            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, scale, epi, 0, _p(sums))
         else:
             self._call("lm_gemm_tiles", _c.byref(part), None, 1, None, None, None, 0, T, 0, 1, scale, epi, 0)
         return out
@@ -210,7 +211,8 @@ class LmOps:
         out = torch.empty((T, n), dtype=self.dtype, device=x.device)
         if T <= ROWS_MAX:
             part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), 2 * n, w.shape[1], bias=_p(bias))
-            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, 1.0, EPI_GLU, ACT[act], _p(self._slices(x, w, EPI_GLU)))
+            sums = self._slices(x, w, EPI_GLU)
+            self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, 1.0, EPI_GLU, ACT[act], _p(sums))
         else:
             y = self.matmul(x, w)
             self._call("lm_glu", _p(out), _ld(out), _p(y), _ld(y), _p(bias), T, n, ACT[act])
