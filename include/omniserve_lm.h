@@ -11,7 +11,7 @@
 extern "C" {
 #endif
 
-#define LM_ABI_VERSION 4
+#define LM_ABI_VERSION 5
 #define LM_NORM_LAYER 0
 #define LM_NORM_RMS 1
 #define LM_EPI_ELEM 0
@@ -57,6 +57,8 @@ int lm_attn_prefill(const void* q, int64_t ldq, const void* kc, int64_t k_page, 
                     int64_t v_page, int v_head, int v_row, const int* bt, int bt_stride, const int* entry,
                     const int* tiles, int n_tiles, const void* gate, int64_t ldg, void* o, int64_t ldo, float scale, int window, int H,
                     int G, int dk, int dv, void* stream);
+/* Query rows of a wave (16 or 32) that lm_attn_prefill takes for these sizes. */
+int lm_attn_prefill_rows(int dk, int dv, int n_tiles, int H);
 
 /* One token per sequence: rotation + value mixing + append + attention + gate.  part: f32 [B][H][nsplit][dv + 2] for nsplit > 1. */
 int lm_attn_decode(const void* qkv, int64_t ld, const void* v_first, int64_t ldv, float lambda, const float* freq, int half,

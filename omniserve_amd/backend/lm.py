@@ -19,7 +19,7 @@ ELEM = {torch.bfloat16: "bf16", torch.float32: "f32"}
 NORM = {"layer": 0, "rms": 1}
 ACT = {None: 0, "silu": 1, "gelu_tanh": 2, "sigmoid": 3}
 EPI_ELEM, EPI_F32, EPI_GLU, EPI_GATE = 0, 1, 2, 3
-ABI = 4
+ABI = 5
 ATTN_ROWS = 128          # query rows of one prefill tile
 PAGE = 64                # tokens per cache page
 ROWS_MAX = 64            # up to here a step's products stream the weights
@@ -39,6 +39,7 @@ PROTOTYPES = {
     "lm_gated_rms": (_i, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i, _i, _i, _f, _vp]),
     "lm_rope_append": (_i, [_vp, _i64, _vp, _i64, _f, _vp, _i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "lm_attn_prefill": (_i, [_vp, _i64, _vp, _i64, _i, _i, _vp, _i64, _i, _i, _vp, _i, _vp, _vp, _i, _vp, _i64, _vp, _i64, _f, _i, _i, _i, _i, _i, _vp]),
+    "lm_attn_prefill_rows": (_i, [_i, _i, _i, _i]),
     "lm_attn_decode": (_i, [_vp, _i64, _vp, _i64, _f, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i64, _vp, _i64, _vp, _i, _f, _i, _i, _i,
                             _i, _i, _i, _vp]),
     "lm_linear_prefill": (_i, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _i, _i, _i, _vp]),

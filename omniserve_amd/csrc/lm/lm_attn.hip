@@ -184,8 +184,7 @@ __global__ __launch_bounds__(64 * WAVES, attn_waves_per_simd(DK, DV)) void attn_
 }
 
 #if LM_ELEM == 0
-// The same with 32 query rows per wave (v_mfma_f32_32x32x16_bf16), four waves of 128 rows, two workgroups per CU: for head sizes whose
-// registers leave the kernel above two waves per SIMD.
+// The same with 32 query rows per wave (v_mfma_f32_32x32x16_bf16), four waves of 128 rows, two workgroups per CU.
 //
 // With eight waves of 16 rows there is one workgroup on a CU: its waves form scores, take exponentials and multiply by V in step, and
 // every one of them reads all of K and V out of LDS for 16 rows.  Two workgroups run against each other, and an operand read serves 32
@@ -196,9 +195,9 @@ __global__ __launch_bounds__(64 * WAVES, attn_waves_per_simd(DK, DV)) void attn_
 //   O^T = V^T P^T: a k step may take its 16 keys in any order that both operands agree on, so step j of a block takes the lane's own
 //   r = 8 j .. 8 j + 7: rows 16 j + 4 (lane / 32) + (0..3) and + 8 of V, two transposed reads.
 //
-// MI355X, 192 / 128, 16 heads, before -> here: 2 prompts of 8000 1424 -> 1078 us (850 TFLOP/s with the second operand of the probabilities counted),
-// 16 of 1024 273 -> 183, 48 of 150 (32 heads) 118 -> 92; 256 / 64 107 -> 81 and 64 / 256 126 -> 103 (4 x 2000, 8 heads).  128 / 128 has four
-// waves per SIMD above and stays there (one prompt of 7999 790 us, 841 with 32 rows per wave).
+// MI355X, 192 / 128, 16 heads, kernel above -> here: 2 prompts of 8000 1305 -> 920 us (990 TFLOP/s with the second operand of the probabilities
+// counted), 48 of 150 57 -> 46; 256 / 64 and 64 / 256 at 2 prompts of 8000, 6 and 8 heads: 579 -> 457 and 766 -> 580.  128 / 128 has four
+// waves per SIMD above and stays there (one prompt of 7999 790 us, 841 with 32 rows per wave).  attn_rows32 says where this one runs.
 template <int DK, int DV>
 struct Attn32 {
   static constexpr int KB = DK * 2, VB = DV * 2, TILE = PAGE * (KB + VB);
@@ -391,15 +390,23 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnArgs p) {
 }
 #endif
 
+// Which sizes have the 32-row form: sums up to 256 have four waves per SIMD in the 16-row form, sums above 320 leave LDS for one workgroup of
+// the 32-row form on a CU.  And it pays where workgroups share CUs: alone on one, its four waves have the SIMDs to themselves and wait for what eight
+// of the other form overlap.  (MI355X, 16 rows / 32 rows per wave: 256 workgroups -- 16 prompts of 100 behind 400, 1 of 2000, 16 heads of 192 / 128 --
+// 26.7 / 28.4 and 74.2 / 75.8 us, 128 rows behind 7000 241 / 246, 8 heads of 64 / 256 257 / 282; 288 workgroups, 3 prompts of 333 with 32
+// heads, 27.4 / 22.0.)
+constexpr bool has_rows32(int dk, int dv) { return !LM_ELEM && dk + dv == 320; }
+static bool attn_rows32(int dk, int dv, int64_t workgroups) { return has_rows32(dk, dv) && workgroups > 256; }
+
 template <int DK, int DV>
 static int launch(const AttnArgs& a, hipStream_t s) {
+  const int64_t total = (int64_t)a.n_tiles * a.H;
 #if LM_ELEM == 0
   static_assert(LM_ATTN_ROWS == 128, "four waves of 32 rows");
-  if constexpr (DK + DV == 320) {
+  if constexpr (has_rows32(DK, DV)) if (attn_rows32(DK, DV, total)) {
     auto k = attn_prefill32_kernel<DK, DV>;
     constexpr size_t lds = 2 * Attn32<DK, DV>::TILE;
     if (allow_lds(k, lds)) return LM_EINVAL;
-    const int64_t total = (int64_t)a.n_tiles * a.H;
     hipLaunchKernelGGL(k, dim3((unsigned)(8 * ((total + 7) / 8))), dim3(256), lds, s, a);
     return launch_status();
   }
@@ -409,7 +416,6 @@ static int launch(const AttnArgs& a, hipStream_t s) {
   constexpr size_t lds = (size_t)PAGE * (Gm::KB + Gm::VB) * (Gm::DB ? 2 : 1);
   auto k = attn_prefill_kernel<DK, DV, WAVES>;
   if (allow_lds(k, lds)) return LM_EINVAL;
-  const int64_t total = (int64_t)a.n_tiles * a.H;
   hipLaunchKernelGGL(k, dim3((unsigned)(8 * ((total + 7) / 8))), dim3(64 * WAVES), lds, s, a);
   return launch_status();
 }
@@ -417,6 +423,8 @@ static int launch(const AttnArgs& a, hipStream_t s) {
 }  // namespace lm
 
 using namespace lm;
+
+extern "C" int lm_attn_prefill_rows(int dk, int dv, int n_tiles, int H) { return attn_rows32(dk, dv, (int64_t)n_tiles * H) ? 32 : 16; }
 
 extern "C" int lm_attn_prefill(const void* q, int64_t ldq, const void* kc, int64_t k_page, int k_head, int k_row,
                                const void* vc, int64_t v_page, int v_head, int v_row, const int* bt, int bt_stride, const int* entry, const int* tiles, int n_tiles, const void* gate, int64_t ldg, void* o, int64_t ldo,

@@ -69,3 +69,18 @@ def test_prompt_attention(dtype, dk, dv, entries, window):
 @pytest.mark.parametrize("heads,kv_heads", [(3, 3), (8, 1), (16, 16)])
 def test_prompt_attention_heads_and_gate(heads, kv_heads):
     _run(torch.bfloat16, 192, 128, heads, kv_heads, [(150, 10), (97, 0)], 1 << 30, gated=True, seed=heads)
+
+
+def _rows_per_wave(dtype, dk, dv, heads, entries):
+    from omniserve_amd.backend.lm import lm_ops
+    return lm_ops(dtype)._h.lm_attn_prefill_rows(dk, dv, sum(-(-n // 128) for n, _ in entries), heads)
+
+
+# The 32-row form of bf16, which takes more than 256 workgroups: the same ends of tiles, pages and windows with as many heads, kv heads whole to an
+# XCD (8) and not (17, 136).
+@pytest.mark.parametrize("entries,window", [([(1, 0), (31, 0), (33, 5), (127, 64)], 1 << 30), ([(130, 0), (257, 190)], 1 << 30), ([(300, 0), (64, 127), (129, 300)], 100),
+                                            ([(200, 50)], 1), ([(385, 0)], 64)])
+@pytest.mark.parametrize("dk,dv,kv_heads,gated", [(192, 128, 8, False), (192, 128, 17, True), (192, 128, 136, False), (64, 256, 17, False), (256, 64, 8, True)])
+def test_prompt_attention_rows32(dk, dv, kv_heads, gated, entries, window):
+    assert _rows_per_wave(torch.bfloat16, dk, dv, 136, entries) == 32
+    _run(torch.bfloat16, dk, dv, 136, kv_heads, entries, window, gated=gated, seed=dk + kv_heads)

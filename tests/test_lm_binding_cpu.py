@@ -1,4 +1,5 @@
-"""The engine kernels' binding without a GPU: what a call passes by address lives until the call has been made."""
+"""The engine kernels' binding and plans without a GPU: what a call passes by address lives until the call has been made; which form of a
+kernel takes which sizes."""
 import weakref
 
 import pytest
@@ -42,3 +43,15 @@ def test_scratch_of_k_slices_outlives_its_call(ops, monkeypatch, call):
     ops._call = enqueue
     call(ops, torch.zeros(3, 256, dtype=torch.bfloat16), torch.zeros(64, 256, dtype=torch.bfloat16))
     assert seen == [("lm_gemm_rows", True)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_per_wave_of_prompt_attention(dtype):
+    """32 only where workgroups share compute units"""
+    rows = lm.lm_ops(dtype)._h.lm_attn_prefill_rows
+    for dk in (64, 128, 192, 256):
+        for dv in (64, 128, 256):
+            for tiles, heads in ((1, 32), (16, 16), (2, 128), (8, 32)):
+                assert rows(dk, dv, tiles, heads) == 16
+            for tiles, heads in ((9, 32), (126, 16), (43, 6)):
+                assert rows(dk, dv, tiles, heads) == (32 if dtype == torch.bfloat16 and dk + dv == 320 else 16)
