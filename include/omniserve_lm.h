@@ -156,6 +156,8 @@ int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int
                  int x_div, int max_rows, float scale, int epi, int act, float* part, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,
                   int max_tiles, int rows_a, int rows_b, int x_div, float scale, int epi, int act, void* stream);
+/* Channels of the tiles (128 or 256) that lm_gemm_tiles takes; max_tiles 0: one matrix over rows_a rows; n_b, k_b, rows_b: part b, or 0. */
+int lm_gemm_tile_channels(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b);
 
 int lm_argmax(int64_t* out, const float* z, int64_t ld, int rows, int n, void* stream);
 

@@ -3,7 +3,8 @@
 //
 //   lm_gemm_rows   few rows (decode): HBM bound.  A workgroup streams the weights of 16 - 80 channels of a group once, through an LDS
 //                  ring filled by DMA; the rows of x come the same way, shared by its waves.
-//   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 256 tiles, both operands by LDS-DMA, a workgroup per CU that takes tile after tile.
+//   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 256 tiles, both operands by LDS-DMA, a workgroup per CU that takes tile after tile;
+//                  256 x 128 where those are too few for the chip, or their last round too empty.
 //
 // Epilogues: element type, f32 times a factor, the gated unit act(gate + bias) * (up + bias) of a matrix whose rows alternate in
 // blocks of 16 between gate and up channels (both halves of a pair then sit in the same lane), or the product with sigmoid(gate).
@@ -380,10 +381,157 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs p, const floa
   store4<EPI>(pt, m, c, 0, v, p.scale);
 }
 
-constexpr int TM = LM_TILE_ROWS, TN = 256;                  // rows, channels of a tile
+// ---- many rows: 256 x 128 tiles -----------------------------------------------------------------------------------------------
+constexpr int TM = LM_TILE_ROWS;                            // rows of a tile
+static_assert(TM == 256, "the wave layouts");
+constexpr int HTN = 128;                                    // channels
+constexpr int HROWB = 64, HK = HROWB / (int)sizeof(elem_t);  // a stage: 64 bytes of k of every row
+constexpr int HSTAGE = (TM + HTN) * HROWB, HSTAGES = 3;
+
+// LDS rows of 64 bytes, four 16-byte slots and four rows to a 256-byte line: slot s of row r at s ^ (0, 2, 3, 1)[r / 4 % 4], with
+// the property Tile::swizzle has for fragment reads
+__device__ __forceinline__ int stage_swizzle(int row) {
+  const int q = (row >> 2) & 3;
+  return (((q ^ (q >> 1)) & 1) << 1) | (q >> 1);
+}
+
+// 4 waves, 128 rows x 64 channels each; three stages: while one multiplies, two are on their way.  Two workgroups share a CU where there are enough.
+// half_tiles() says where this one runs.
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_half_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[HSTAGES * HSTAGE];
+  __shared__ int y_row[TM];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l15 = lane & 15, l4 = lane >> 4;
+  // linear order: bands of row tiles, all channel tiles of a band before the next one; of both parts a contiguous range per XCD
+  const int nt_a = (p.a.n + HTN - 1) / HTN, nt_b = mt_b ? (p.b.n + HTN - 1) / HTN : 0;
+  const int wgs_b = 8 * ((mt_b * nt_b + 7) >> 3);
+  const bool is_b = (int)blockIdx.x < wgs_b;
+  const Part& pt = is_b ? p.b : p.a;
+  const int nt = is_b ? nt_b : nt_a, mts = is_b ? mt_b : mt_a;
+  const int id = xcd_contiguous(is_b ? blockIdx.x : blockIdx.x - wgs_b, mts * nt);
+  if (id < 0) return;
+  constexpr int GM = 4;
+  const int band = id / (GM * nt), in = id - band * GM * nt, bm = min(GM, mts - band * GM);
+  const int mi = band * GM + in % bm, ni = in / bm;
+  const int* perm = is_b ? nullptr : p.perm;
+  int first = mi * TM, rows, g = 0;
+  if (perm) {
+    const i32x4 t = *(const i32x4*)(p.tiles + 4 * mi);       // group, first place, rows
+    if (t[2] <= 0) return;
+    g = t[0];
+    first = t[1];
+    rows = t[2];
+  } else {
+    rows = min(TM, (is_b ? p.rows_b : p.rows_a) - first);
+  }
+  const int n0 = ni * HTN;
+  const elem_t* w = pt.w + (int64_t)g * pt.n * pt.k;
+  // pieces of 16 rows: lane -> (row lane / 4, physical slot lane % 4); a wave carries 2 of the weights' and 4 of x's
+  const elem_t *wsrc[2], *xsrc[4];
+  const int pr = lane >> 2, ps = (lane & 3) ^ stage_swizzle(pr);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = min(16 * (4 * wave + i) + pr, rows - 1);
+    const int xr = perm ? perm[first + r] / p.x_div : first + r;
+    xsrc[i] = pt.x + (int64_t)xr * pt.ldx + ps * FR;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wsrc[i] = w + (int64_t)min(n0 + 16 * (2 * wave + i) + pr, pt.n - 1) * pt.k + ps * FR;
+  y_row[tid] = tid < rows ? (perm ? perm[first + tid] : first + tid) : -1;
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const int uw = __builtin_amdgcn_readfirstlane(wave);
+  auto stage = [&](int st, int k0) {
+    const uint32_t dst = lds0 + st * HSTAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16_uncounted(wsrc[i] + k0, dst + 1024 * (2 * uw + i));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16_uncounted(xsrc[i] + k0, dst + HTN * HROWB + 1024 * (4 * uw + i));
+  };
+  const int wn = 64 * (wave & 1), wm = 128 * (wave >> 1);
+  f32x4 acc[4][8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = zero4();
+  const int nk = pt.k / HK;                                 // (>= 2: k is a multiple of 64)
+  const int lane_off = l15 * HROWB + ((l4 ^ stage_swizzle(l15)) << 4);
+  wait_pieces<0>();                                         // the compiler's own loads
+  stage(0, 0);
+  stage(1, HK);
+  int st = 0;
+  for (int t = 0; t < nk; ++t) {
+    if (t + 1 < nk) wait_pieces<6>();                       // stage t is there, the 6 pieces of t + 1 may still fly
+    else wait_pieces<0>();
+    __builtin_amdgcn_s_barrier();                           // ... for every wave, and everyone has left stage t - 1
+    asm volatile("" ::: "memory");
+    if (t + 2 < nk) stage(st == 0 ? 2 : st - 1, (t + 2) * HK);
+    const uint8_t* wt = lds + st * HSTAGE + wn * HROWB + lane_off;
+    const uint8_t* xt = lds + st * HSTAGE + (HTN + wm) * HROWB + lane_off;
+    frag_t a[4], b[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = *(const frag_t*)(wt + 16 * HROWB * i);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = *(const frag_t*)(xt + 16 * HROWB * j);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i][j] = mma(a[i], b[j], acc[i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    st = st == 2 ? 0 : st + 1;
+  }
+  __syncthreads();                                          // the stages are free
+  if constexpr (EPI == LM_EPI_F32) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int row = y_row[wm + 16 * j + l15];
+      if (row < 0) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = n0 + wn + 16 * i + 4 * l4;
+        if (c < pt.n) store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
+      }
+    }
+  } else {
+    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 32 rows of the wave's at a time
+    constexpr int OC = EPI == LM_EPI_GLU ? 32 : 64, PITCH = OC * (int)sizeof(elem_t) + 16, PPR = OC / FR;
+    static_assert(4 * 32 * PITCH <= HSTAGES * HSTAGE, "the waves' buffers");
+    uint8_t* buf = lds + wave * 32 * PITCH;
+#pragma unroll
+    for (int part = 0; part < 4; ++part) {
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) {
+        const int j = 2 * part + jj;
+#pragma unroll
+        for (int i = 0; i < 4; i += EPI == LM_EPI_GLU ? 2 : 1) {
+          f32x4 v = acc[i][j];
+          int c = 16 * i;
+          if constexpr (EPI == LM_EPI_GLU) {
+            c = 8 * i;
+            if (n0 + wn + 16 * i < pt.n) v = glu(pt, p.act, n0 + wn + 16 * i + 4 * l4, v, acc[i + 1][j]);
+          }
+          *(quad_t*)(buf + (16 * jj + l15) * PITCH + (c + 4 * l4) * (int)sizeof(elem_t)) = to_quad(v);
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 32 * PPR / 64; ++i) {
+        const int pc = 64 * i + lane, r = pc / PPR, q = pc % PPR;
+        const int row = y_row[wm + 32 * part + r], c = (EPI == LM_EPI_GLU ? (n0 + wn) / 2 : n0 + wn) + q * FR;
+        if (row >= 0 && c < (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n))
+          *(frag_t*)((elem_t*)pt.y + (int64_t)row * pt.ldy + c) = *(const frag_t*)(buf + r * PITCH + q * 16);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// ---- many rows: 256 x 256 tiles -----------------------------------------------------------------------------------------------
+constexpr int TN = 256;                                     // channels of a tile
 constexpr int SROWB = 128, SK = SROWB / (int)sizeof(elem_t); // a stage: 128 bytes of k of every row (whole lines of the L2)
 constexpr int STAGE = (TM + TN) * SROWB;
-static_assert(TM == 256, "the wave layout");
 
 // c += a b, c pinned (mfma_pinned.h)
 __device__ __forceinline__ void mma_in_place(f32x4& c, frag_t a, frag_t b) {
@@ -648,6 +796,35 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   }
 }
 
+// 256 x 128 tiles instead of 256 x 256?  Whichever has the smaller time in rounds of the latter (one workgroup per CU) by a model of both: on
+// the XCD with the most tiles, pairs of half tiles share a CU and take 0.95 - 1.25 rounds, the more the longer their K (1.05 with fewer than 48 rows in
+// a tile, where they wait for weights), a rest that is alone on its CUs 0.8.  What it is about: grids that leave CUs idle, and last rounds.
+// (MI355X, bf16, 256 x 256 / 256 x 128, us: to f32, 65 rows of 32000 x 4096 102 / 77, 300 rows 116 / 134, 1000 rows of 8192 x 4096 105 / 81, 2000
+// rows 109 / 144.  Experts: 12 rows each of 32 x 4096 x 1792 151 / 133, 130 rows 161 / 178, 550 rows 352 / 393; 64 x 2048 x 640 70 / 56, 77 / 76, 164 / 161.
+// f32, 65 rows of 4096 x 1024 234 / 129.  Over 336 such sizes the choice costs 0.1 % on average and 10 % at most against the better one.)
+// max_tiles > 0: rows sorted by group, of which there is a tile for every 256 and one per group.  Part b over rows_b rows: its tiles are the first that
+// workgroups of the whole form take, and where its K is longer those end later, by a third of it.
+static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {
+  const int row_tiles = max_tiles > 0 ? max_tiles : (rows_a + TM - 1) / TM;
+  const int64_t rows = max_tiles > 0 ? (int64_t)TM * max(0, max_tiles - groups) : rows_a;
+  auto per_xcd = [&](int tn) {
+    auto part = [&](int tiles, int c) { return ((int64_t)tiles * ((c + tn - 1) / tn) + 7) / 8; };
+    return part(row_tiles, n) + part((rows_b + TM - 1) / TM, n_b);
+  };
+  const int64_t per_h = per_xcd(HTN), per_f = per_xcd(TN);
+  const float pair = rows < (int64_t)48 * (max_tiles > 0 ? groups : row_tiles) ? 1.05f : 0.95f + 0.3f * (float)min((int64_t)k * (int)sizeof(elem_t), (int64_t)8192) / 8192.f;
+  const int64_t rest = per_h % 64;
+  const float half = (float)(per_h / 64) * pair + (rest == 0 ? 0.f : rest <= 32 ? 0.8f : pair);
+  const float late = rows_b > 0 && k_b > k ? ((float)k_b / (float)k - 1.f) / 3.f : 0.f;
+  return half <= (float)((per_f + 31) / 32) + late;
+}
+
+template <int EPI>
+static void launch_tiles(const GemmArgs& a, bool half, int64_t wgs, int mt_a, int mt_b, hipStream_t s) {
+  if (half) hipLaunchKernelGGL((gemm_half_tiles_kernel<EPI>), dim3((unsigned)wgs), dim3(256), 0, s, a, mt_a, mt_b);
+  else hipLaunchKernelGGL((gemm_tiles_kernel<EPI>), dim3((unsigned)min((int64_t)256, wgs)), dim3(256), 0, s, a, mt_a, mt_b);      // a workgroup per CU
+}
+
 static int check_part(const Part& p, int epi, int act) {
   if (!p.w || !p.x || !p.y || p.n <= 0 || p.k <= 0 || p.k % 64 || p.n % 16 || p.ldx < p.k || p.ldx % FR || p.ldy % FR) return LM_EINVAL;
   if (epi == LM_EPI_GLU && (p.n % 32 || (act != LM_ACT_SILU && act != LM_ACT_GELU_TANH))) return LM_EINVAL;
@@ -772,6 +949,10 @@ extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {
   return s > 1 ? (int64_t)s * rows * n : 0;
 }
 
+extern "C" int lm_gemm_tile_channels(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {
+  return half_tiles(n, k, groups, max_tiles, rows_a, n_b, k_b, rows_b) ? HTN : TN;
+}
+
 extern "C" int lm_gemm_tiles(const LmGemmPart* pa, const LmGemmPart* pb, int groups, const int* perm, const int* off,
                              const int* tiles, int max_tiles, int rows_a, int rows_b, int x_div,
                              float scale, int epi, int act, void* stream) {
@@ -781,13 +962,14 @@ extern "C" int lm_gemm_tiles(const LmGemmPart* pa, const LmGemmPart* pb, int gro
   if (perm && (!tiles || max_tiles <= 0)) return LM_EINVAL;
   a.tiles = perm ? tiles : nullptr;
   const int mt_a = perm ? max_tiles : (rows_a + TM - 1) / TM, mt_b = pb && rows_b > 0 ? (rows_b + TM - 1) / TM : 0;
-  const int64_t tiles_a = (int64_t)mt_a * ((a.a.n + TN - 1) / TN), tiles_b = mt_b ? (int64_t)mt_b * ((a.b.n + TN - 1) / TN) : 0;
+  const bool half = half_tiles(a.a.n, a.a.k, groups, perm ? max_tiles : 0, rows_a, a.b.n, a.b.k, mt_b ? rows_b : 0);
+  const int tn = half ? HTN : TN;
+  const int64_t tiles_a = (int64_t)mt_a * ((a.a.n + tn - 1) / tn), tiles_b = mt_b ? (int64_t)mt_b * ((a.b.n + tn - 1) / tn) : 0;
   if (tiles_a <= 0 || tiles_a + tiles_b > (1 << 30)) return LM_EINVAL;
-  // a workgroup per CU
-  const dim3 grid((unsigned)min((int64_t)256, 8 * ((tiles_a + 7) / 8 + (tiles_b + 7) / 8)));
+  const int64_t wgs = 8 * ((tiles_a + 7) / 8 + (tiles_b + 7) / 8);
   hipStream_t s = (hipStream_t)stream;
-  if (epi == LM_EPI_ELEM) hipLaunchKernelGGL((gemm_tiles_kernel<LM_EPI_ELEM>), grid, dim3(256), 0, s, a, mt_a, mt_b);
-  else if (epi == LM_EPI_F32) hipLaunchKernelGGL((gemm_tiles_kernel<LM_EPI_F32>), grid, dim3(256), 0, s, a, mt_a, mt_b);
-  else hipLaunchKernelGGL((gemm_tiles_kernel<LM_EPI_GLU>), grid, dim3(256), 0, s, a, mt_a, mt_b);
+  if (epi == LM_EPI_ELEM) launch_tiles<LM_EPI_ELEM>(a, half, wgs, mt_a, mt_b, s);
+  else if (epi == LM_EPI_F32) launch_tiles<LM_EPI_F32>(a, half, wgs, mt_a, mt_b, s);
+  else launch_tiles<LM_EPI_GLU>(a, half, wgs, mt_a, mt_b, s);
   return launch_status();
 }

@@ -55,3 +55,19 @@ def test_rows_per_wave_of_prompt_attention(dtype):
                 assert rows(dk, dv, tiles, heads) == 16
             for tiles, heads in ((9, 32), (126, 16), (43, 6)):
                 assert rows(dk, dv, tiles, heads) == (32 if dtype == torch.bfloat16 and dk + dv == 320 else 16)
+
+
+def test_tiles_of_prompt_products():
+    """Whole tiles where they fill the chip's rounds, half tiles where they leave units idle or wait for weights"""
+    channels = lm.lm_ops(torch.bfloat16)._h.lm_gemm_tile_channels
+    for n, k, rows, want in ((32000, 4096, 65, 128), (32000, 4096, 257, 256), (32000, 4096, 1000, 256), (4096, 2048, 300, 128), (8192, 4096, 1000, 128),
+                             (8192, 4096, 2000, 256), (1024, 4096, 2000, 128)):
+        assert channels(n, k, 1, 0, rows, 0, 0, 0) == want
+    tiles = lambda tokens, experts, top: lm.lm_ops(torch.bfloat16)._h.lm_route_max_tiles(tokens, experts, top)      # noqa: E731
+    for tokens, experts, top, n, k, n_b, k_b, want in (
+            (65, 32, 6, 4096, 1792, 4096, 3584, 128), (150, 32, 6, 3584, 4096, 7168, 4096, 128), (700, 32, 6, 4096, 1792, 4096, 3584, 128),
+            (700, 32, 6, 3584, 4096, 7168, 4096, 256), (1500, 32, 6, 4096, 1792, 4096, 3584, 256), (7999, 32, 6, 4096, 1792, 4096, 3584, 256),
+            (7999, 32, 6, 3584, 4096, 7168, 4096, 256), (100, 64, 8, 2048, 640, 2048, 1024, 128), (100, 64, 8, 1280, 2048, 2048, 2048, 128),
+            (4000, 64, 8, 1280, 2048, 2048, 2048, 256)):
+        assert channels(n, k, experts, tiles(tokens, experts, top), 0, n_b, k_b, tokens) == want, (tokens, n, k)
+    assert lm.lm_ops(torch.float32)._h.lm_gemm_tile_channels(4096, 1024, 1, 0, 65, 0, 0, 0) == 128

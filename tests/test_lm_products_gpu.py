@@ -141,3 +141,63 @@ def test_experts_of_a_prompt(tokens, E, top, ff, W, skew, dtype):
         down[t * top + c] = a[t * top + c] @ wod[e].t()
     _rows_close(y[:tokens * top], down, dtype)
     _rows_close(y[tokens * top:], acts.double() @ wd.double().t(), dtype)
+
+
+def _channels(ops, n, k, groups=1, max_tiles=0, rows=0, n_b=0, k_b=0, rows_b=0):
+    return ops._h.lm_gemm_tile_channels(n, k, groups, max_tiles, rows, n_b, k_b, rows_b)
+
+
+def _matrix_close(got, want, dtype):
+    """errors() of the whole result, on the GPU"""
+    want = want.float() if got.dtype == torch.float32 else want
+    assert ((got.double() - want).norm() / want.double().norm()) < TOL[dtype] and ((got.double() - want).abs().max() / want.double().square().mean().sqrt()) < 16 * TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k,channels", [(2000, 16112, 2048, 256), (3000, 16112, 1024, 256), (255, 32784, 1024, 256), (255, 32016, 1024, 128), (1000, 8160, 2048, 128), (4100, 16400, 64, 128), (2100, 4112, 192, 128)])
+def test_tiles_in_turn(m, n, k, channels, dtype):
+    """many rows to f32: whole and half tiles, two and three whole ones in turn on a workgroup"""
+    ops = _ops(dtype)
+    assert _channels(ops, n, k, rows=m) == channels
+    x, w = _randn(23, dtype, m, k + 64)[:, 64:], _randn(24, dtype, n, k) * k ** -0.5
+    guard = torch.full((m + 2, n), 7.0, device=DEV)
+    ops.matmul(x, w, out=guard[1:-1], out_f32=True)
+    _matrix_close(guard[1:-1], x.double() @ w.double().t(), torch.float32)
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("tokens,E,top,n,k,channels", [(70, 62, 3, 4096, 64, 256), (71, 62, 3, 3072, 128, 256), (66, 62, 3, 2048, 192, 256), (80, 62, 3, 4064, 1024, 256),
+                                                       (70, 64, 3, 1376, 64, 128), (700, 16, 4, 2080, 192, 128), (2800, 16, 4, 4096, 2048, 256)])
+@pytest.mark.parametrize("glu", [False, True])
+def test_experts_in_turn(tokens, E, top, n, k, channels, glu, dtype):
+    """Experts and a shared one: two to four whole tiles in turn on a workgroup, of one, two and more stages of k, experts without rows between them;
+    half tiles.  Every row, and what lies around the results stays as it was."""
+    ops = _ops(dtype)
+    max_tiles = ops._h.lm_route_max_tiles(tokens, E, top)
+    assert _channels(ops, n, k, E, max_tiles, n_b=544, k_b=k, rows_b=tokens) == channels
+    z = _randn(25, torch.float32, tokens, E)
+    z[:, E // 4:E // 2] -= 100                                           # nobody chooses these
+    wts, order = ops.route(z.contiguous(), torch.zeros((E,), device=DEV), E, top)
+    h, w, ws = _randn(26, dtype, tokens, k), _randn(27, dtype, E, n, k) * k ** -0.5, _randn(28, dtype, 544, k) * k ** -0.5
+    out = n // 2 if glu else n
+    y = torch.full((tokens * top + 2, out), 7.0, dtype=dtype, device=DEV)
+    ys = torch.full((tokens + 2, 272 if glu else 544), 7.0, dtype=dtype, device=DEV)
+    ops.grouped(order, tokens, h, w, y[1:-1], False, glu, (h, ws, ys[1:-1]))
+    for edge in (y[0], y[-1], ys[0], ys[-1]):
+        assert (edge == 7).all()
+
+    def product(x, m):
+        v = x.double() @ m.double().t()
+        if glu:
+            v = v.view(x.shape[0], m.shape[0] // 32, 2, 16)
+            v = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(x.shape[0], m.shape[0] // 2)
+        return v
+
+    ids = torch.argsort(-z, dim=1, stable=True)[:, :top]
+    want = torch.empty((tokens * top, out), dtype=torch.float64, device=DEV)
+    for e in range(E):
+        t, c = torch.nonzero(ids == e, as_tuple=True)
+        want[t * top + c] = product(h[t], w[e])
+    _rows_close(y[1:-1], want.cpu(), dtype)
+    _rows_close(ys[1:-1], product(h, ws).cpu(), dtype)
