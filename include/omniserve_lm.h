@@ -152,6 +152,9 @@ typedef struct {
 /* lm_gemm_rows, part (or null): lm_gemm_rows_scratch() f32 of scratch for one matrix over at most 64 rows, whose K may then be cut into
  * slices (0: it is not). */
 int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi);
+/* Channels per workgroup that lm_gemm_rows streams (0: the kernel without a stream) for `groups` matrices, without perm and part b; *slices: K
+ * slices, more than one only where `sliced` (there is scratch). */
+int lm_gemm_rows_channels(int groups, int n, int k, int rows, int epi, int sliced, int* slices);
 int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, int rows_a, int rows_b,
                  int x_div, int max_rows, float scale, int epi, int act, float* part, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,

@@ -62,6 +62,7 @@ PROTOTYPES = {
     "lm_route_max_tiles": (_i, [_i, _i, _i]),
     "lm_route": (_i, [_vp, _i64, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     "lm_gemm_rows_scratch": (_i64, [_i, _i, _i, _i]),
+    "lm_gemm_rows_channels": (_i, [_i] * 6 + [_c.POINTER(_i)]),
     "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp]),
     "lm_gemm_tiles": (_i, [_PP, _PP, _i, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp]),
     "lm_gemm_tile_channels": (_i, [_i] * 8),

@@ -2,7 +2,7 @@
 // experts is one group per expert over the tokens routed to it, plus one for the shared expert over all tokens.
 //
 //   lm_gemm_rows   few rows (decode): HBM bound.  A workgroup streams the weights of 16 - 80 channels of a group once, through an LDS
-//                  ring filled by DMA; the rows of x come the same way, shared by its waves.
+//                  ring filled by DMA; the rows of x come the same way, shared by its waves.  Small ones: operands straight to registers.
 //   lm_gemm_tiles  many rows (prefill): MFMA bound.  256 x 256 tiles, both operands by LDS-DMA, a workgroup per CU that takes tile after tile;
 //                  256 x 128 where those are too few for the chip, or their last round too empty.
 //
@@ -848,9 +848,9 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   return LM_OK;
 }
 
-template <int EPI>
+template <int NR, int MB, int EPI>
 static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s) {
-  constexpr int NR = 2, MB = 4, KW = 8;
+  constexpr int KW = 8;
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
   const dim3 grid((n + 16 * NR - 1) / (16 * NR), a.groups + has_b, a.perm ? 1 : (max_rows + 16 * MB - 1) / (16 * MB));
   hipLaunchKernelGGL((gemm_rows_kernel<NR, MB, KW, EPI>), grid, dim3(64 * KW), 0, s, a);
@@ -865,20 +865,20 @@ static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s
 // was measured the channels per workgroup matter most where n / 64 is far from a multiple of 256 (10816 x 4096, 48 rows: 26.5 us at 64,
 // 20.8 at 48; 4096 x 4096, 16 rows: 11.8 us at 64 and 4 slices, 9.8 at 16), slices where K is long (4096 x 14336, 48 rows: 40 us, 26
 // with 4).
-struct StreamPlan {
-  int nw, slices;
+struct RowsPlan {
+  int nw, slices;      // nw 0: gemm_rows_kernel
 };
-static StreamPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool sliced) {
-  StreamPlan best{4, 1};
+static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool sliced) {
+  RowsPlan best{4, 1};
   float time = 1e30f;
   const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
   for (int nw = 5; nw >= 1; --nw) {
     if (glu && nw != 4) continue;                          // (a gate block and its up block share a workgroup)
     const int64_t tiles = (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw));
-    for (int s = 1; s <= (sliced ? 8 : 1) && stages >= 4 * s; s *= 2) {
+    for (int s = 1; s <= (sliced ? 8 : 1) && (s == 1 || stages >= 4 * s); s *= 2) {
       float t = (float)((tiles * s + 255) / 256) * (float)((stages + s - 1) / s) * (0.07f * nw + 0.02f * mb + 0.02f);
       if (s > 1) t += 4.5f + (float)s * rows * n * 8.f / 5e6f;
-      if (t < time) { time = t; best = StreamPlan{nw, s}; }
+      if (t < time) { time = t; best = RowsPlan{nw, s}; }
     }
   }
   return best;
@@ -896,10 +896,8 @@ static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices,
 }
 
 template <int EPI>
-static int launch_stream(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
+static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part, hipStream_t s) {
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
-  // experts: how many have rows is not known here; 64 channels measured best from 60 to 1000 MB
-  const StreamPlan pl = a.perm || has_b ? StreamPlan{4, 1} : plan_stream(a.groups, n, a.a.k, max_rows, EPI == LM_EPI_GLU, part != nullptr);
   if constexpr (EPI == LM_EPI_GLU) {
     launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s);
   } else {
@@ -918,14 +916,37 @@ static int launch_stream(const GemmArgs& a, int max_rows, int has_b, float* part
   return launch_status();
 }
 
-// More than 64 rows come here with few channels (the router of a prompt) or one matrix per head: workgroups along the rows.
-template <int EPI>
-static int plan_rows(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
-  if constexpr (EPI != LM_EPI_GLU) {
-    if (max_rows > 64) return launch_rows<EPI>(a, max_rows, has_b, s);
+// Which kernel, and how dealt.  experts: groups by perm or two parts; how many of them have rows is not known here, and 64 channels measured best from
+// 60 to 1000 MB.  gemm_rows_kernel takes
+//   * more than 64 rows of few channels (the router of a prompt) or of one matrix per head: workgroups along the rows;
+//   * 33 - 64 rows where channels and K slices make too few workgroups: there too (MI355X, 64 rows: 64 x 2048 7.7 us in 8 slices, 6.1 so; 8 heads of
+//     128 x 512 4.2 / 3.8; but 16 heads of 128 x 256 3.7 / 4.7, and 128 x 4096 is better in slices);
+//   * up to 16 rows where a ring is only filled once (16 heads of 256 x 128 3.5 / 3.2, 4096 x 128 3.2 / 2.8; 4096 x 256 3.2 / 3.3; more workgroups
+//     than CUs take 64 channels each, 32 heads of 512 x 128 4.1 / 8.0);
+//   * the gated unit of up to 16 rows over few weights, whose stream of 64 channels per workgroup has too few workgroups (16 rows: 2048 x 512
+//     4.2 / 3.7 us, 4096 x 256 4.2 / 3.7, 2048 x 1024 6.4 / 6.3, 4096 x 1024 6.6 / 6.5).
+static RowsPlan plan_rows(int groups, int n, int k, int rows, int epi, bool experts, bool sliced) {
+  if (experts && (epi == LM_EPI_GLU || rows <= 64)) return RowsPlan{4, 1};
+  if (epi == LM_EPI_GLU) {
+    if (rows <= 16 && (int64_t)groups * n * k * (int)sizeof(elem_t) <= (4 << 20)) return RowsPlan{0, 1};
+    return plan_stream(groups, n, k, rows, true, sliced);
   }
+  if (rows > 64) return RowsPlan{0, 1};
+  const RowsPlan pl = plan_stream(groups, n, k, rows, false, sliced);
+  const int64_t bytes_k = (int64_t)k * (int)sizeof(elem_t), channels = (int64_t)groups * n;
+  if (rows > 32 && n <= 256 && channels <= 1024 && (pl.slices == 1 || bytes_k <= 4096)) return RowsPlan{0, 1};
+  if (rows <= 16 && bytes_k <= 512 && channels <= 4096) return RowsPlan{0, 1};
+  return pl;
+}
+
+template <int EPI>
+static int launch_few(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
   const bool one = a.groups == 1 && !a.perm && !has_b && max_rows <= 64 && max_rows == a.rows_a;
-  return launch_stream<EPI>(a, max_rows, has_b, one ? part : nullptr, s);
+  const RowsPlan pl = plan_rows(a.groups, has_b && a.b.n > a.a.n ? a.b.n : a.a.n, a.a.k, max_rows, EPI, a.perm || has_b, one && part != nullptr);
+  if (pl.nw > 0) return launch_stream<EPI>(a, has_b, pl, part, s);
+  if constexpr (EPI == LM_EPI_GLU) return launch_rows<2, 1, EPI>(a, max_rows, has_b, s);
+  else if (max_rows <= 64) return launch_rows<1, 1, EPI>(a, max_rows, has_b, s);
+  else return launch_rows<2, 4, EPI>(a, max_rows, has_b, s);
 }
 
 }  // namespace lm
@@ -938,15 +959,21 @@ extern "C" int lm_gemm_rows(const LmGemmPart* pa, const LmGemmPart* pb, int grou
   if (fill(a, pa, pb, groups, perm, off, rows_a, rows_b, x_div, scale, epi, act) || max_rows <= 0) return LM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   const int has_b = pb && rows_b > 0;
-  if (epi == LM_EPI_GLU) return plan_rows<LM_EPI_GLU>(a, max_rows, has_b, part, s);
-  if (epi == LM_EPI_GATE) return plan_rows<LM_EPI_GATE>(a, max_rows, has_b, part, s);
-  return epi == LM_EPI_F32 ? plan_rows<LM_EPI_F32>(a, max_rows, has_b, part, s) : plan_rows<LM_EPI_ELEM>(a, max_rows, has_b, part, s);
+  if (epi == LM_EPI_GLU) return launch_few<LM_EPI_GLU>(a, max_rows, has_b, part, s);
+  if (epi == LM_EPI_GATE) return launch_few<LM_EPI_GATE>(a, max_rows, has_b, part, s);
+  return epi == LM_EPI_F32 ? launch_few<LM_EPI_F32>(a, max_rows, has_b, part, s) : launch_few<LM_EPI_ELEM>(a, max_rows, has_b, part, s);
 }
 
 extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {
   if (n <= 0 || k <= 0 || rows <= 0 || rows > 64) return 0;
-  const int s = plan_stream(1, n, k, rows, epi == LM_EPI_GLU, true).slices;
+  const int s = plan_rows(1, n, k, rows, epi, false, true).slices;
   return s > 1 ? (int64_t)s * rows * n : 0;
+}
+
+extern "C" int lm_gemm_rows_channels(int groups, int n, int k, int rows, int epi, int sliced, int* slices) {
+  const RowsPlan pl = plan_rows(groups, n, k, rows, epi, false, sliced != 0);
+  if (slices) *slices = pl.slices;
+  return 16 * pl.nw;
 }
 
 extern "C" int lm_gemm_tile_channels(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {

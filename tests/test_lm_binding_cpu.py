@@ -71,3 +71,15 @@ def test_tiles_of_prompt_products():
             (4000, 64, 8, 1280, 2048, 2048, 2048, 256)):
         assert channels(n, k, experts, tiles(tokens, experts, top), 0, n_b, k_b, tokens) == want, (tokens, n, k)
     assert lm.lm_ops(torch.float32)._h.lm_gemm_tile_channels(4096, 1024, 1, 0, 65, 0, 0, 0) == 128
+
+
+def test_few_rows_of_short_k_spread_over_the_chip():
+    """K of one to three stages: as many workgroups as the channels make, not 64 channels each whatever their number"""
+    import ctypes
+    for dtype in (torch.bfloat16, torch.float32):
+        h, slices = lm.lm_ops(dtype)._h, ctypes.c_int(0)
+        for k in (64, 128, 192) if dtype == torch.bfloat16 else (64,):
+            assert h.lm_gemm_rows_channels(1, 4096, k, 20, 0, 1, ctypes.byref(slices)) == 16 and slices.value == 1
+            assert h.lm_gemm_rows_channels(16, 256, k, 17, 0, 0, None) == 16
+            assert h.lm_gemm_rows_channels(1, 4096, k, 15, 0, 1, ctypes.byref(slices)) == 0 and slices.value == 1
+            assert h.lm_gemm_rows_channels(32, 512, k, 16, 0, 0, None) == 64

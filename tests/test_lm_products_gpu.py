@@ -1,6 +1,8 @@
-"""The engine's products of few rows (csrc/lm/lm_gemm.hip): every width of a workgroup, K in parts and in slices, fewer stages than parts,
-row counts at the edges of 16, views with a row stride, the gated unit, one matrix per head, experts with many rows.  Against float64."""
-import numpy as np
+"""The engine's products (csrc/lm/lm_gemm.hip).  Few rows: every width of a workgroup, K in parts and in slices, fewer stages than parts, row counts
+at the edges of 16, views with a row stride, the gated unit, one matrix per head, experts with many rows.  Many rows: whole and half tiles, several in
+turn on a workgroup, experts without rows.  Against float64."""
+import ctypes
+
 import pytest
 import torch
 
@@ -48,6 +50,32 @@ def test_products(m, n, k, dtype):
     assert (guard[0] == 7).all() and (guard[-1] == 7).all()
     assert errors(ops.matmul(x, w, out_f32=True, scale=0.5).cpu().numpy(), 0.5 * want.cpu().numpy()).max() < 2e-6
     assert torch.equal(ops.matmul(x, w), ops.matmul(x, w))
+
+
+def _rows_plan(ops, groups, n, k, rows, epi=0, sliced=1):
+    slices = ctypes.c_int(0)
+    return ops._h.lm_gemm_rows_channels(groups, n, k, rows, epi, sliced, ctypes.byref(slices)), slices.value
+
+
+# Every width with whole rings and with fewer stages than the ring holds, in slices of K, in K parts (at most 256 workgroups) and without; the kernel
+# without a stream.  Channels that end inside a workgroup, row counts around 16.
+# (k of bf16; half of it in f32, whose stages hold half as many)
+WIDTHS = [(16, 1, 16, 4096, 1024), (16, 8, 17, 256, 4096), (32, 1, 33, 6224, 256), (32, 8, 64, 528, 3200), (48, 1, 48, 10816, 4096), (48, 1, 33, 10816, 512),
+          (64, 1, 64, 12352, 4096), (64, 1, 49, 32016, 128), (64, 8, 64, 2048, 6144), (80, 1, 48, 16448, 4096), (80, 1, 17, 16448, 256), (80, 8, 1, 12352, 4096),
+          (0, 1, 33, 64, 1024), (0, 1, 64, 240, 2048), (0, 1, 16, 4096, 128), (0, 1, 3, 528, 256)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("channels,slices,m,n,k", WIDTHS)
+def test_every_width(channels, slices, m, n, k, dtype):
+    ops, k = _ops(dtype), k // (1 if dtype == torch.bfloat16 else 2)
+    assert _rows_plan(ops, 1, n, k, m) == (channels, slices)
+    x, w = _randn(21, dtype, m, k + 64)[:, 64:], _randn(22, dtype, n, k) * k ** -0.5
+    want = x.double() @ w.double().t()
+    guard = torch.full((m + 2, n), 7.0, dtype=dtype, device=DEV)
+    _close(ops.matmul(x, w, out=guard[1:-1]), want, dtype)
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+    assert errors(ops.matmul(x, w, out_f32=True, scale=0.5).cpu().numpy(), 0.5 * want.cpu().numpy()).max() < 2e-6
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
