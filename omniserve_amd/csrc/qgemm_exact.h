@@ -87,8 +87,17 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
     const int t = xcd * per + min(xcd, more) + i;
     const int band = t / (p.tile_linear * p.tiles_n), in = t - band * p.tile_linear * p.tiles_n;
     const int rows = min(p.tile_linear, p.tiles_m - band * p.tile_linear);
-    tile_n = in / rows;
-    tile_m = band * p.tile_linear + in - tile_n * rows;
+    if (KW == 1 && !TO_SLAB && (p.tiles_m & 7) == 0) {
+      // whole bands of 8 row tiles: blocks of 8 x 8 tiles, along their rows -- neighbours share activations, which a band's columns would
+      // all read at once (MI355X, column / row order: 2048 rows of 28672 x 4096 185 / 177 us per-channel, 265 / 251 per-group; 4096 rows 359 / 354 and
+      // 512 / 496; 4096 x 14336 and 8192 x 8192 the same; bands of 6, 1501 rows, 140 / 142)
+      const int blk = in >> 6, cols = min(8, p.tiles_n - 8 * blk), i64 = in & 63, r = i64 / cols;
+      tile_n = 8 * blk + i64 - r * cols;
+      tile_m = band * 8 + r;
+    } else {
+      tile_n = in / rows;
+      tile_m = band * p.tile_linear + in - tile_n * rows;
+    }
   }
   const int ng = tile_n * WAVES + wave;  // 64-channel group of this wave
   // M need not be whole tiles: the last row tile starts at M - MT and computes the rows it shares with the one before a second time

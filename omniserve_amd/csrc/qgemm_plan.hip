@@ -204,8 +204,8 @@ static const TileCost kTileCost[3] = {
     {{3.5f, 6.5f, 4.7f}, {{1.63f, 1.80f, 1.88f, 2.12f, 2.24f}, {2.18f, 2.65f, 3.00f, 3.08f, 3.36f}, {1.22f, 1.36f, 1.48f, 1.62f, 1.78f}}},
 };
 
-static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, int chunks) {
-  auto t = [&](int kind) { return c.fix[kind] + c.chunk[kind][mb - 4] * (float)chunks; };
+static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, float chunks) {
+  auto t = [&](int kind) { return c.fix[kind] + c.chunk[kind][mb - 4] * chunks; };
   if (kw == 2) {      // (nothing runs beside the next one's start: 4 us more per further round)
     const long long rounds = (workgroups + 255) / 256;
     return (float)rounds * (t(2) + 4.f) - 4.f;
@@ -227,10 +227,13 @@ static float tiles_time(long long tiles, int stages) {
 PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) {
   const TileCost& c = kTileCost[mode];
   PrefillPlan best{8, 1, slab_only ? sk : 1};
+  // rows far apart are slower to read, but not where K slices read them at several places (512 rows of 8192 x 28672 per-channel: 1.08 us per chunk of
+  // two K parts, 0.83 at 14336; 256 rows of 7168 x 8192 W8A8 1.68, 1.25 at 4096: 126 and 58 us where slices take 105 and 47)
+  const float far = mode == MODE_W8 && K >= 8192 ? 1.2f : mode == MODE_CHN && K >= 16384 ? 1.17f : 1.f;
   float time = 1e30f;
   auto offer = [&](int mb, int kw, int split) {
     const long long tiles = (long long)((M + 16 * mb - 1) / (16 * mb)) * (N / 256) * split;
-    float t = grid_time(c, mb, kw, tiles, K / (split * KCHUNK));
+    float t = grid_time(c, mb, kw, tiles, (split == 1 ? far : 1.f) * (float)(K / (split * KCHUNK)));
     // the slabs written, read and reduced by a launch of their own
     if (split > 1 && !slab_only) t += 4.5f + (float)split * M * N * 8.f / 4.5e6f;
     if (t < time) { time = t; best = PrefillPlan{mb, kw, split}; }

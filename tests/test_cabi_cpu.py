@@ -180,6 +180,14 @@ def test_prefill_plans_fit_the_kernels_and_the_scratch():
     assert seen >= {(mb, kw, False) for mb in range(4, 9) for kw in (1, 2)} | {(mb, 1, True) for mb in range(4, 9)} | {(16, 1, False)}
 
 
+def test_prefill_plans_of_rows_far_apart():
+    """K slices over the grid where whole rows of that length read slowly, two K parts in a workgroup where they do not"""
+    for M, N, K, mode, sliced in ((512, 8192, 28672, 0, True), (450, 8192, 28672, 0, True), (256, 7168, 8192, 2, True), (300, 8192, 8192, 2, True),
+                                  (256, 4096, 4096, 0, False), (512, 4096, 4096, 2, False)):
+        _, _, kw, sk = _prefill_plan(M, N, K, mode)
+        assert (sk > 1) == sliced and kw == (1 if sliced else 2), (M, N, K, mode)
+
+
 def test_forced_k_splits_reach_the_prefill_plan():
     from omniserve_amd import _lib
     lib = _lib.lib()

@@ -495,3 +495,11 @@ def test_prefill_forced_k_slices(mode, M, N, K, sk):
 def test_per_group_scales_around_the_lane_limit_two_k_parts(mb, M, N, K):
     assert _prefill_plan("grp", M, N, K) == (mb, 2, 1)
     test_per_group_scales_around_the_lane_limit(M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,mb", [(512, 2304, 256, 4), (505, 4352, 256, 4), (1000, 2304, 768, 4), (1920, 2560, 256, 5)])
+@pytest.mark.parametrize("mode", MODES)
+def test_prefill_whole_bands(mode, M, N, K, mb):
+    """row tiles in whole bands of 8, whose blocks of 8 x 8 tiles end in one or two columns (and in none)"""
+    assert _prefill_plan(mode, M, N, K) == (mb, 1, 1) and -(-M // (16 * mb)) % 8 == 0
+    {"chn": lambda: _run_chn(M, N, K, seed=M, out_view=True), "grp": lambda: _run_grp(M, N, K, True), "w8": lambda: _run_w8(M, N, K)}[mode]()
