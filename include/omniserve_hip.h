@@ -51,7 +51,7 @@ void omni_gemm_set_plan_override(int waves, int sk);
  * sk > 0 forces its K split.  Per calling thread, like the override above. */
 void omni_gemm_set_midm_override(int mode, int sk);
 void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, int* sk);
-/* M > 128 (0 below), output rows 16-byte aligned.  mode: 0 per-channel W4A8, 1 per-group W4A8, 2 W8A8; slabs_only: omni_*_gemm_partial.
+/* M > 128 (0 below), operands and output rows 16-byte aligned (others go to the general kernel).  mode: 0 per-channel W4A8, 1 per-group W4A8, 2 W8A8; slabs_only: omni_*_gemm_partial.
  * Returns 1 for the straight-line kernels: *mb 16-row blocks of a tile (16: the 256 x 256 tiles of W8A8), *kw K parts inside a
  * workgroup, *sk K slices that go through the scratch (1: none but slabs_only's own).  2 for the general kernel (N % 256 or K % 256). */
 int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int slabs_only, int* mb, int* kw, int* sk);

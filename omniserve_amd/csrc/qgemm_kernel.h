@@ -1235,13 +1235,14 @@ struct PrefillPlan {
 PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only);
 
 // shapes the straight-line kernel takes: whole channel tiles and K chunks (also of a K slice: a.kslice); it stores 16 B
-// per lane, so rows of an fp16 output must start 16-B aligned
+// per lane, so rows of an fp16 output must start 16-B aligned, and so must both operands
 static inline bool exact_sizes(int M, int N, int K, int kslice) {
   return M > 128 && N % 256 == 0 && K % KCHUNK == 0 && kslice % KCHUNK == 0 && (size_t)M * K < ((size_t)1 << 32);
 }
 static inline bool exact_shape(const GemmArgs& a, bool to_slab) {
   const bool out16 = to_slab || ((a.out_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0);
-  return exact_sizes(a.M, a.N, a.K, a.kslice) && out16;
+  const bool in16 = ((reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W)) & 15) == 0;      // LDS-DMA takes whole 16-byte pieces
+  return exact_sizes(a.M, a.N, a.K, a.kslice) && out16 && in16;
 }
 
 template <int MODE, int MB, int KW, bool TO_SLAB>

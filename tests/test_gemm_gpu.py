@@ -503,3 +503,43 @@ def test_prefill_whole_bands(mode, M, N, K, mb):
     """row tiles in whole bands of 8, whose blocks of 8 x 8 tiles end in one or two columns (and in none)"""
     assert _prefill_plan(mode, M, N, K) == (mb, 1, 1) and -(-M // (16 * mb)) % 8 == 0
     {"chn": lambda: _run_chn(M, N, K, seed=M, out_view=True), "grp": lambda: _run_grp(M, N, K, True), "w8": lambda: _run_w8(M, N, K)}[mode]()
+
+
+def _shifted(a):
+    """The same values, contiguous, from 8 bytes behind a 16-byte boundary on"""
+    t = torch.from_numpy(np.ascontiguousarray(a)).to(dev())
+    base = torch.empty((t.numel() + 16,), dtype=t.dtype, device=dev())
+    out = base[8:8 + t.numel()].view(t.shape)
+    out.copy_(t)
+    assert out.data_ptr() % 16 == 8
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 256, 256), (300, 512, 768), (300, 512, 2048), (512, 18944, 1536)])
+@pytest.mark.parametrize("mode", MODES)
+def test_prefill_operands_between_boundaries(mode, M, N, K):
+    """operands that start between two 16-byte boundaries, which the straight-line kernels' DMA does not take"""
+    from omniserve_amd.backend import fused_ext, qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
+    a, sa, asum = _acts(M, K, M)
+    out = torch.empty((M, N), dtype=torch.float16, device=dev())
+    if mode == "chn":
+        u, z, s1 = w4a8.synth_per_channel(N, K, M)
+        qw, s1h, szh = w4a8.pack_per_channel(u, z, s1)
+        want = w4a8.gemm_per_chn(a, qw, s1h, sa, szh, asum)
+        qgemm_w4a8_per_chn.gemm_forward_cuda(_shifted(a), to_dev(qw), to_dev(s1h), to_dev(sa), to_dev(szh), to_dev(asum), out)
+    elif mode == "grp":
+        u, z, s2, s1 = w4a8.synth_per_group(N, K, seed=M, wrap=True)
+        qw, s1h, s2s, s2z = w4a8.pack_per_group(u, z, s2, s1)
+        want = w4a8.gemm_per_group(a, qw, s2z, s2s, s1h, sa)
+        qgemm_w4a8_per_group.gemm_forward_cuda(_shifted(a), to_dev(qw), to_dev(s2z), to_dev(s2s), to_dev(s1h), to_dev(sa), out)
+    else:
+        rng = np.random.default_rng(M)
+        w, sw = rng.integers(-128, 128, size=(N, K), dtype=np.int8), rng.uniform(0.001, 0.01, size=(N,)).astype(np.float16)
+        want = w4a8.gemm_w8a8(a, w, sw, sa)
+        qgemm_w8a8.w8a8_gemm_forward_cuda(_shifted(a), _shifted(w), to_dev(sw), to_dev(sa), out)
+        if M <= 300:
+            slab = torch.empty((8, M, N), dtype=torch.int32, device=dev())
+            sk = fused_ext.gemm_partial_w8a8(_shifted(a), _shifted(w), slab)
+            assert np.array_equal(slab[:sk].sum(dim=0).cpu().numpy(), w4a8._int_matmul_fast(a, w))
+    torch.cuda.synchronize()
+    assert_f16_equal(out, want, "%s M=%d N=%d K=%d" % (mode, M, N, K))
