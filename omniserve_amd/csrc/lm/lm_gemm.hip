@@ -942,7 +942,11 @@ static RowsPlan plan_rows(int groups, int n, int k, int rows, int epi, bool expe
 template <int EPI>
 static int launch_few(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
   const bool one = a.groups == 1 && !a.perm && !has_b && max_rows <= 64 && max_rows == a.rows_a;
-  const RowsPlan pl = plan_rows(a.groups, has_b && a.b.n > a.a.n ? a.b.n : a.a.n, a.a.k, max_rows, EPI, a.perm || has_b, one && part != nullptr);
+  RowsPlan pl = plan_rows(a.groups, has_b && a.b.n > a.a.n ? a.b.n : a.a.n, a.a.k, max_rows, EPI, a.perm || has_b, one && part != nullptr);
+  // the stream's DMA takes whole 16-byte pieces; loads into registers may start anywhere
+  uintptr_t at = (uintptr_t)a.a.w | (uintptr_t)a.a.x;
+  if (has_b) at |= (uintptr_t)a.b.w | (uintptr_t)a.b.x;
+  if (at & 15) pl = RowsPlan{0, 1};
   if (pl.nw > 0) return launch_stream<EPI>(a, has_b, pl, part, s);
   if constexpr (EPI == LM_EPI_GLU) return launch_rows<2, 1, EPI>(a, max_rows, has_b, s);
   else if (max_rows <= 64) return launch_rows<1, 1, EPI>(a, max_rows, has_b, s);

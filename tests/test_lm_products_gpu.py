@@ -229,3 +229,36 @@ def test_experts_in_turn(tokens, E, top, n, k, channels, glu, dtype):
         want[t * top + c] = product(h[t], w[e])
     _rows_close(y[1:-1], want.cpu(), dtype)
     _rows_close(ys[1:-1], product(h, ws).cpu(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m", [1, 20, 64])
+def test_few_rows_between_boundaries(m, dtype):
+    """x and w that start between two 16-byte boundaries, which the stream's DMA does not take: plain, gated, per head, experts"""
+    ops, shift = _ops(dtype), 8 // torch.empty((), dtype=dtype).element_size()
+
+    def between(seed, gain, *shape):      # (all rows of one size, unlike each other: errors() relates a row to the mean of all)
+        n = torch.Size(shape).numel()
+        t = (_randn(seed, torch.float32, n + 16) * gain).to(dtype)[shift:shift + n].view(shape)
+        assert t.data_ptr() % 16 == 8
+        return t
+
+    x, w, b = between(29, 1, m, 1024), _randn(30, dtype, 544, 1024) / 32, _randn(33, torch.float32, 544) * 0.1
+    ws = between(31, 1 / 32, 544, 1024)
+    want = x.double() @ ws.double().t()
+    _close(ops.matmul(x, ws), want, dtype)
+    _close(ops.matmul(x, w), x.double() @ w.double().t(), dtype)
+    y = (want + b.double()).view(m, 17, 2, 16)
+    got = ops.glu(x, ws, b, "gelu_tanh")
+    want = (torch.nn.functional.gelu(y[:, :, 0], approximate="tanh") * y[:, :, 1]).reshape(m, 272)
+    assert errors(got.float().cpu().numpy(), want.cpu().numpy()).max() < max(TOL[dtype], 5e-6)
+    wh, out = between(32, 1 / 16, 4, 128, 256), torch.empty((m, 512), dtype=dtype, device=DEV)
+    ops.head_products(x, wh, out, 256, 128)
+    _close(out, torch.cat([x[:, 256 * h:256 * h + 256].double() @ wh[h].double().t() for h in range(4)], dim=1), dtype)
+    z = _randn(34, torch.float32, m, 6)
+    wts, order = ops.route(z, torch.zeros((6,), device=DEV), 6, 3)
+    we, y, ys = _randn(35, dtype, 6, 192, 1024) / 32, torch.empty((m * 3, 192), dtype=dtype, device=DEV), torch.empty((m, 544), dtype=dtype, device=DEV)
+    ops.grouped(order, m, x, we, y, False, False, (x, ws, ys))
+    ids = torch.argsort(-z, dim=1, stable=True)[:, :3]
+    _close(y, torch.stack([x[t].double() @ we[ids[t, c]].double().t() for t in range(m) for c in range(3)]), dtype)
+    _close(ys, x.double() @ ws.double().t(), dtype)
