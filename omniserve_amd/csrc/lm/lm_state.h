@@ -5,9 +5,10 @@
 
 namespace lm {
 
-// The recurrent state of a decode step, read and written once.  Where it is larger than the L2s it is not kept there: what it would push out is
-// read again (MI355X, 32 heads of 128 x 128: 64 sequences 60 -> 49 us, 48 47 -> 38, 16 19.6 -> 15.8; one sequence 8.6 without keeping it, 8.0
-// with, so small states stay).
+// The recurrent state of a decode step, read and written once.  From 16 MB on (half of the L2s) it is not kept there: what it would push out is read
+// again.  (MI355X, heads of 128 x 128, kept / not, 300 MB of other reads in front: 8 MB 10.1 / 9.6 us gated, 12.7 / 12.1 delta rule; 16 MB 12.7 / 11.4 and
+// 15.4 / 13.7; 32 MB 20.2 / 17.0 and 23.1 / 19.7; 64 MB 34.1 / 29.0 and 39.3 / 35.6; a state still in the caches, heads of 256 x 256: 4 MB 10.2 / 12.1,
+// 12 MB 12.2 / 13.8, 16 MB 13.0 / 14.1, but 32.1 / 31.4 with the reads behind it.  One sequence, 2 MB, 7.6 / 7.9 then, so small states stay.)
 __host__ __device__ constexpr bool streams_state(int64_t sequences, int heads, int dk, int dv) {
   return sequences * heads * dk * dv * (int64_t)sizeof(float) >= (16 << 20);
 }

@@ -46,8 +46,11 @@ struct GemmArgs {
   int64_t out_stride;
   int kslice;             // k per split (multiple of 64)
   int tiles_m, tiles_n;   // > 0: 1-D grid with the XCD-aware tile order of w4a8_gemm_kernel
-  int tile_linear;        // 1 (with tiles_n > 0): workgroup w = tile (w % tiles_m, w / tiles_m) -- few row tiles; w4a8_gemm_exact_kernel and
-                          // w8a8_tiles_kernel: row tiles per band of their order (a field of its own would move the decode kernels' arguments)
+  // what the launched kernel reads in it (a field each would move the decode kernels' arguments):
+  //   w4a8_gemm_kernel: 1 (with tiles_n > 0): workgroup w = tile (w % tiles_m, w / tiles_m) -- few row tiles
+  //   w4a8_gemm_exact_kernel, w8a8_tiles_kernel: row tiles per band of their order
+  //   w4a8_midm_kernel: 1: rows of the output allow 16-byte stores
+  int tile_linear;
   // ---- row-kernel-free decode forms (fused extension; see w4a8_gemv_kernel EPI / A16) ----
   const half_t* A16;      // [M,K] fp16 activations quantised on the fly (A16 kernels; `A` unused)
   uint32_t* amax;         // [AMAX_WORDS] row-maximum candidates (common.h): EPI = 1 raises them, A16 reads them
