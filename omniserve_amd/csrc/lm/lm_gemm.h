@@ -1,0 +1,68 @@
+// What the products' kernels share: lm_gemm.hip and, in a file of their own, the 256 x 128 tiles.
+#pragma once
+#include "lm_common.h"
+#include "omniserve_lm.h"
+
+namespace lm {
+
+struct Part {        // a family of equally shaped groups
+  const elem_t* w;   // [groups][n][k]
+  const elem_t* x; int64_t ldx;
+  void* y; int64_t ldy;
+  int n, k;
+  int64_t gx, gy;            // without perm: columns of x / y between neighbouring groups
+  const float* bias;         // [n] added to the products of a gated unit (or null)
+  const elem_t* gate;        // LM_EPI_GATE: the factor's argument, laid out like y
+  int64_t ldg;
+};
+
+struct GemmArgs {
+  Part a, b;                  // a: groups 0 .. groups - 1 (rows by perm / off), b: one group over rows 0 .. rows_b - 1
+  int groups;
+  const int* perm;            // row of y for every sorted place (null: identity, rows_a rows)
+  const int* off;             // [groups + 1] sorted places of each group
+  int rows_a, rows_b;
+  int x_div;                  // x row = y row / x_div (tokens of (token, choice) pairs)
+  const int* tiles;           // lm_gemm_tiles with perm: (group, first place, rows, 0) of every row tile, rows 0: none
+  float scale;
+  int act;                    // of the gated unit
+};
+
+__device__ __forceinline__ f32x4 glu(const Part& pt, int act, int c, f32x4 gate, f32x4 up) {      // c: gate channel's row in w, a multiple of 4
+  if (pt.bias) {
+    gate += *(const f32x4*)(pt.bias + c);
+    up += *(const f32x4*)(pt.bias + c + 16);
+  }
+  f32x4 r;
+  if (act == LM_ACT_GELU_TANH) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = gelu_tanh(gate[e]) * up[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = silu(gate[e]) * up[e];
+  }
+  return r;
+}
+
+template <int EPI>
+__device__ __forceinline__ void store4(const Part& pt, int64_t row, int c, int64_t y0, f32x4 v, float scale) {
+  if constexpr (EPI == LM_EPI_ELEM || EPI == LM_EPI_GLU) {
+    *(quad_t*)((elem_t*)pt.y + row * pt.ldy + y0 + c) = to_quad(v);
+  } else if constexpr (EPI == LM_EPI_F32) {
+    *(f32x4*)((float*)pt.y + row * pt.ldy + y0 + c) = v * scale;
+  } else {
+    const f32x4 z = from_quad(*(const quad_t*)(pt.gate + row * pt.ldg + y0 + c));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] *= sigmoid(z[e]);
+    *(quad_t*)((elem_t*)pt.y + row * pt.ldy + y0 + c) = to_quad(v);
+  }
+}
+
+constexpr int TM = LM_TILE_ROWS;                            // rows of a tile
+static_assert(TM == 256, "the wave layouts");
+constexpr int HTN = 128;                                    // channels of a half tile
+
+// gemm_half_tiles_kernel<epi> over `wgs` workgroups; mt_a, mt_b: row tiles of both parts
+__attribute__((visibility("hidden"))) void launch_half_tiles(const GemmArgs& a, int epi, unsigned wgs, int mt_a, int mt_b, hipStream_t s);
+
+}  // namespace lm

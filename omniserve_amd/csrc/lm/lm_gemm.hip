@@ -8,9 +8,8 @@
 //
 // Epilogues: element type, f32 times a factor, the gated unit act(gate + bias) * (up + bias) of a matrix whose rows alternate in
 // blocks of 16 between gate and up channels (both halves of a pair then sit in the same lane), or the product with sigmoid(gate).
-#include "lm_common.h"
+#include "lm_gemm.h"
 #include "mfma_pinned.h"
-#include "omniserve_lm.h"
 
 namespace lm {
 
@@ -19,59 +18,6 @@ template <int J, typename F>
 __device__ __forceinline__ void countdown(F&& f) {      // f(J), f(J - 1), ..., f(0)
   f(Int<J>{});
   if constexpr (J > 0) countdown<J - 1>(f);
-}
-
-struct Part {        // a family of equally shaped groups
-  const elem_t* w;   // [groups][n][k]
-  const elem_t* x; int64_t ldx;
-  void* y; int64_t ldy;
-  int n, k;
-  int64_t gx, gy;            // without perm: columns of x / y between neighbouring groups
-  const float* bias;         // [n] added to the products of a gated unit (or null)
-  const elem_t* gate;        // LM_EPI_GATE: the factor's argument, laid out like y
-  int64_t ldg;
-};
-
-struct GemmArgs {
-  Part a, b;                  // a: groups 0 .. groups - 1 (rows by perm / off), b: one group over rows 0 .. rows_b - 1
-  int groups;
-  const int* perm;            // row of y for every sorted place (null: identity, rows_a rows)
-  const int* off;             // [groups + 1] sorted places of each group
-  int rows_a, rows_b;
-  int x_div;                  // x row = y row / x_div (tokens of (token, choice) pairs)
-  const int* tiles;           // lm_gemm_tiles with perm: (group, first place, rows, 0) of every row tile, rows 0: none
-  float scale;
-  int act;                    // of the gated unit
-};
-
-__device__ __forceinline__ f32x4 glu(const Part& pt, int act, int c, f32x4 gate, f32x4 up) {      // c: gate channel's row in w, a multiple of 4
-  if (pt.bias) {
-    gate += *(const f32x4*)(pt.bias + c);
-    up += *(const f32x4*)(pt.bias + c + 16);
-  }
-  f32x4 r;
-  if (act == LM_ACT_GELU_TANH) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = gelu_tanh(gate[e]) * up[e];
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = silu(gate[e]) * up[e];
-  }
-  return r;
-}
-
-template <int EPI>
-__device__ __forceinline__ void store4(const Part& pt, int64_t row, int c, int64_t y0, f32x4 v, float scale) {
-  if constexpr (EPI == LM_EPI_ELEM || EPI == LM_EPI_GLU) {
-    *(quad_t*)((elem_t*)pt.y + row * pt.ldy + y0 + c) = to_quad(v);
-  } else if constexpr (EPI == LM_EPI_F32) {
-    *(f32x4*)((float*)pt.y + row * pt.ldy + y0 + c) = v * scale;
-  } else {
-    const f32x4 z = from_quad(*(const quad_t*)(pt.gate + row * pt.ldg + y0 + c));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] *= sigmoid(z[e]);
-    *(quad_t*)((elem_t*)pt.y + row * pt.ldy + y0 + c) = to_quad(v);
-  }
 }
 
 // A workgroup owns NR 16-channel blocks; its KW waves split K and meet in LDS.  16 MB rows at a time; blockIdx.z takes every
@@ -381,153 +327,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs p, const floa
   store4<EPI>(pt, m, c, 0, v, p.scale);
 }
 
-// ---- many rows: 256 x 128 tiles -----------------------------------------------------------------------------------------------
-constexpr int TM = LM_TILE_ROWS;                            // rows of a tile
-static_assert(TM == 256, "the wave layouts");
-constexpr int HTN = 128;                                    // channels
-constexpr int HROWB = 64, HK = HROWB / (int)sizeof(elem_t);  // a stage: 64 bytes of k of every row
-constexpr int HSTAGE = (TM + HTN) * HROWB, HSTAGES = 3;
-
-// LDS rows of 64 bytes, four 16-byte slots and four rows to a 256-byte line: slot s of row r at s ^ (0, 2, 3, 1)[r / 4 % 4], with
-// the property Tile::swizzle has for fragment reads
-__device__ __forceinline__ int stage_swizzle(int row) {
-  const int q = (row >> 2) & 3;
-  return (((q ^ (q >> 1)) & 1) << 1) | (q >> 1);
-}
-
-// 4 waves, 128 rows x 64 channels each; three stages: while one multiplies, two are on their way.  Two workgroups share a CU where there are enough.
-// half_tiles() says where this one runs.
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_half_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[HSTAGES * HSTAGE];
-  __shared__ int y_row[TM];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l15 = lane & 15, l4 = lane >> 4;
-  // linear order: bands of row tiles, all channel tiles of a band before the next one; of both parts a contiguous range per XCD
-  const int nt_a = (p.a.n + HTN - 1) / HTN, nt_b = mt_b ? (p.b.n + HTN - 1) / HTN : 0;
-  const int wgs_b = 8 * ((mt_b * nt_b + 7) >> 3);
-  const bool is_b = (int)blockIdx.x < wgs_b;
-  const Part& pt = is_b ? p.b : p.a;
-  const int nt = is_b ? nt_b : nt_a, mts = is_b ? mt_b : mt_a;
-  const int id = xcd_contiguous(is_b ? blockIdx.x : blockIdx.x - wgs_b, mts * nt);
-  if (id < 0) return;
-  constexpr int GM = 4;
-  const int band = id / (GM * nt), in = id - band * GM * nt, bm = min(GM, mts - band * GM);
-  const int mi = band * GM + in % bm, ni = in / bm;
-  const int* perm = is_b ? nullptr : p.perm;
-  int first = mi * TM, rows, g = 0;
-  if (perm) {
-    const i32x4 t = *(const i32x4*)(p.tiles + 4 * mi);       // group, first place, rows
-    if (t[2] <= 0) return;
-    g = t[0];
-    first = t[1];
-    rows = t[2];
-  } else {
-    rows = min(TM, (is_b ? p.rows_b : p.rows_a) - first);
-  }
-  const int n0 = ni * HTN;
-  const elem_t* w = pt.w + (int64_t)g * pt.n * pt.k;
-  // pieces of 16 rows: lane -> (row lane / 4, physical slot lane % 4); a wave carries 2 of the weights' and 4 of x's
-  const elem_t *wsrc[2], *xsrc[4];
-  const int pr = lane >> 2, ps = (lane & 3) ^ stage_swizzle(pr);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = min(16 * (4 * wave + i) + pr, rows - 1);
-    const int xr = perm ? perm[first + r] / p.x_div : first + r;
-    xsrc[i] = pt.x + (int64_t)xr * pt.ldx + ps * FR;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = w + (int64_t)min(n0 + 16 * (2 * wave + i) + pr, pt.n - 1) * pt.k + ps * FR;
-  y_row[tid] = tid < rows ? (perm ? perm[first + tid] : first + tid) : -1;
-  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
-  const int uw = __builtin_amdgcn_readfirstlane(wave);
-  auto stage = [&](int st, int k0) {
-    const uint32_t dst = lds0 + st * HSTAGE;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_uncounted(wsrc[i] + k0, dst + 1024 * (2 * uw + i));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dma16_uncounted(xsrc[i] + k0, dst + HTN * HROWB + 1024 * (4 * uw + i));
-  };
-  const int wn = 64 * (wave & 1), wm = 128 * (wave >> 1);
-  f32x4 acc[4][8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = zero4();
-  const int nk = pt.k / HK;                                 // (>= 2: k is a multiple of 64)
-  const int lane_off = l15 * HROWB + ((l4 ^ stage_swizzle(l15)) << 4);
-  wait_pieces<0>();                                         // the compiler's own loads
-  stage(0, 0);
-  stage(1, HK);
-  int st = 0;
-  for (int t = 0; t < nk; ++t) {
-    if (t + 1 < nk) wait_pieces<6>();                       // stage t is there, the 6 pieces of t + 1 may still fly
-    else wait_pieces<0>();
-    __builtin_amdgcn_s_barrier();                           // ... for every wave, and everyone has left stage t - 1
-    asm volatile("" ::: "memory");
-    if (t + 2 < nk) stage(st == 0 ? 2 : st - 1, (t + 2) * HK);
-    const uint8_t* wt = lds + st * HSTAGE + wn * HROWB + lane_off;
-    const uint8_t* xt = lds + st * HSTAGE + (HTN + wm) * HROWB + lane_off;
-    frag_t a[4], b[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = *(const frag_t*)(wt + 16 * HROWB * i);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b[j] = *(const frag_t*)(xt + 16 * HROWB * j);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][j] = mma(a[i], b[j], acc[i][j]);
-    __builtin_amdgcn_s_setprio(0);
-    st = st == 2 ? 0 : st + 1;
-  }
-  __syncthreads();                                          // the stages are free
-  if constexpr (EPI == LM_EPI_F32) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int row = y_row[wm + 16 * j + l15];
-      if (row < 0) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = n0 + wn + 16 * i + 4 * l4;
-        if (c < pt.n) store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
-      }
-    }
-  } else {
-    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 32 rows of the wave's at a time
-    constexpr int OC = EPI == LM_EPI_GLU ? 32 : 64, PITCH = OC * (int)sizeof(elem_t) + 16, PPR = OC / FR;
-    static_assert(4 * 32 * PITCH <= HSTAGES * HSTAGE, "the waves' buffers");
-    uint8_t* buf = lds + wave * 32 * PITCH;
-#pragma unroll
-    for (int part = 0; part < 4; ++part) {
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const int j = 2 * part + jj;
-#pragma unroll
-        for (int i = 0; i < 4; i += EPI == LM_EPI_GLU ? 2 : 1) {
-          f32x4 v = acc[i][j];
-          int c = 16 * i;
-          if constexpr (EPI == LM_EPI_GLU) {
-            c = 8 * i;
-            if (n0 + wn + 16 * i < pt.n) v = glu(pt, p.act, n0 + wn + 16 * i + 4 * l4, v, acc[i + 1][j]);
-          }
-          *(quad_t*)(buf + (16 * jj + l15) * PITCH + (c + 4 * l4) * (int)sizeof(elem_t)) = to_quad(v);
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int i = 0; i < 32 * PPR / 64; ++i) {
-        const int pc = 64 * i + lane, r = pc / PPR, q = pc % PPR;
-        const int row = y_row[wm + 32 * part + r], c = (EPI == LM_EPI_GLU ? (n0 + wn) / 2 : n0 + wn) + q * FR;
-        if (row >= 0 && c < (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n))
-          *(frag_t*)((elem_t*)pt.y + (int64_t)row * pt.ldy + c) = *(const frag_t*)(buf + r * PITCH + q * 16);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
-}
-
 // ---- many rows: 256 x 256 tiles -----------------------------------------------------------------------------------------------
 constexpr int TN = 256;                                     // channels of a tile
 constexpr int SROWB = 128, SK = SROWB / (int)sizeof(elem_t); // a stage: 128 bytes of k of every row (whole lines of the L2)
@@ -821,7 +620,7 @@ static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int 
 
 template <int EPI>
 static void launch_tiles(const GemmArgs& a, bool half, int64_t wgs, int mt_a, int mt_b, hipStream_t s) {
-  if (half) hipLaunchKernelGGL((gemm_half_tiles_kernel<EPI>), dim3((unsigned)wgs), dim3(256), 0, s, a, mt_a, mt_b);
+  if (half) launch_half_tiles(a, EPI, (unsigned)wgs, mt_a, mt_b, s);
   else hipLaunchKernelGGL((gemm_tiles_kernel<EPI>), dim3((unsigned)min((int64_t)256, wgs)), dim3(256), 0, s, a, mt_a, mt_b);      // a workgroup per CU
 }
 
