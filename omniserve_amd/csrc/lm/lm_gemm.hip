@@ -596,11 +596,11 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
 }
 
 // 256 x 128 tiles instead of 256 x 256?  Whichever has the smaller time in rounds of the latter (one workgroup per CU) by a model of both: on
-// the XCD with the most tiles, pairs of half tiles share a CU and take 0.95 - 1.25 rounds, the more the longer their K (1.05 with fewer than 48 rows in
-// a tile, where they wait for weights), a rest that is alone on its CUs 0.8.  What it is about: grids that leave CUs idle, and last rounds.
+// the XCD with the most tiles, pairs of half tiles share a CU and take 0.97 - 1.26 rounds, the more the longer their K and the fewer rows of them are empty
+// (1.05 with fewer than 48 rows in a tile, where they wait for weights), a rest that is alone on its CUs 0.8.  What it is about: grids that leave CUs idle, and last rounds.
 // (MI355X, bf16, 256 x 256 / 256 x 128, us: to f32, 65 rows of 32000 x 4096 102 / 77, 300 rows 116 / 134, 1000 rows of 8192 x 4096 105 / 81, 2000
 // rows 109 / 144.  Experts: 12 rows each of 32 x 4096 x 1792 151 / 133, 130 rows 161 / 178, 550 rows 352 / 393; 64 x 2048 x 640 70 / 56, 77 / 76, 164 / 161.
-// f32, 65 rows of 4096 x 1024 234 / 129.  Over 336 such sizes the choice costs 0.1 % on average and 10 % at most against the better one.)
+// f32, 65 rows of 4096 x 1024 234 / 129.  Over 408 such sizes the choice costs 0.2 % on average and 6 % at most against the better one.)
 // max_tiles > 0: rows sorted by group, of which there is a tile for every 256 and one per group.  Part b over rows_b rows: its tiles are the first that
 // workgroups of the whole form take, and where its K is longer those end later, by a third of it.
 static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {
@@ -611,7 +611,9 @@ static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int 
     return part(row_tiles, n) + part((rows_b + TM - 1) / TM, n_b);
   };
   const int64_t per_h = per_xcd(HTN), per_f = per_xcd(TN);
-  const float pair = rows < (int64_t)48 * (max_tiles > 0 ? groups : row_tiles) ? 1.05f : 0.95f + 0.3f * (float)min((int64_t)k * (int)sizeof(elem_t), (int64_t)8192) / 8192.f;
+  const int64_t places = max_tiles > 0 ? groups : row_tiles;
+  const float pair = rows < 48 * places ? 1.05f
+                                        : (rows < 1000 * places ? 0.97f : 1.01f) + 0.25f * (float)min((int64_t)k * (int)sizeof(elem_t), (int64_t)8192) / 8192.f;
   const int64_t rest = per_h % 64;
   const float half = (float)(per_h / 64) * pair + (rest == 0 ? 0.f : rest <= 32 ? 0.8f : pair);
   const float late = rows_b > 0 && k_b > k ? ((float)k_b / (float)k - 1.f) / 3.f : 0.f;
