@@ -48,6 +48,20 @@ __device__ __forceinline__ void lds_dma_rows(const void* sbase, uint32_t voff, u
   else OMNI_DMA_ROWS(OMNI_DMA_NEXT OMNI_DMA_NEXT OMNI_DMA_NEXT OMNI_DMA_NEXT OMNI_DMA_NEXT OMNI_DMA_NEXT OMNI_DMA_NEXT);
 }
 
+// Eight pieces of the wave's own 32 rows (128-row tiles of KW = 1): piece i = rows 4 i .. 4 i + 3, lane offset v[i & 3] from base0 (i < 4) or base1,
+// 16 rows on; LDS image from lds_dst + i * 1024.  With it hipcc keeps the weight ring where it lies: in the form above it copies ring registers at
+// the end of every chunk, behind waits for loads that it has just requested (MI355X, that form / this one: per-channel 4096 rows of 28672 x 4096 343 / 338
+// us, 8192 of 8192 x 8192 386 / 378; per-group 4096 of 28672 x 4096 487 / 471, 8192 of 6144 x 4096 215 / 207).
+__device__ __forceinline__ void lds_dma_own_rows(const void* base0, const void* base1, const uint32_t (&v)[4], uint32_t lds_dst) {
+  uint32_t keep;
+#define OMNI_DMA_OWN(V, B) "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %" #V ", %" #B "\n\t"
+  asm volatile("s_nop 4\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %1\n\t"
+               OMNI_DMA_OWN(4, 1) OMNI_DMA_OWN(5, 1) OMNI_DMA_OWN(6, 1) OMNI_DMA_OWN(3, 2) OMNI_DMA_OWN(4, 2) OMNI_DMA_OWN(5, 2) OMNI_DMA_OWN(6, 2)
+               "s_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(base0), "s"(base1), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(lds_dst) : "memory", "scc");
+#undef OMNI_DMA_OWN
+}
+
 // TO_SLAB (decode batches of 129 .. 512 rows: few tiles): the workgroup takes K slice blockIdx.y of p.kslice (a whole number of chunks)
 // and stores its int32 accumulators to slab[blockIdx.y][M][N] for splitk_epilogue_kernel / a slab consumer.
 template <int MODE, int MB, int KW, bool TO_SLAB = false>
@@ -133,13 +147,19 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
   // ---- activations ---------------------------------------------------------------------------------------
   // LDS row m = 256 B, piece q at slot q ^ (m & 15), written by LDS-DMA: piece i of wave w covers rows i * 16 + w * 4 + dr of the tile,
   // lane -> (dr = lane >> 4, LDS slot ds = lane & 15), so the source piece is ds ^ (w * 4 + dr), the same for every i
-  const int drow = wave * 4 + (lane >> 4);
-  const uint32_t dvo = (uint32_t)drow * (uint32_t)p.K + (uint32_t)(((lane & 15) ^ drow) << 4);
+  // (OWN: piece i of wave w covers rows 32 w + 4 i + dr, source piece ds ^ (4 (i & 3) + dr)).  The address is formed from the kernel's arguments in
+  // every chunk: a base kept outside the loop brings the copies back.
+  constexpr bool OWN = MB == 8 && KW == 1;
+  const int drow = OWN ? lane >> 4 : wave * 4 + (lane >> 4);
+  uint32_t dvo[4];
+#pragma unroll
+  for (int i = 0; i < (OWN ? 4 : 1); ++i) dvo[i] = (uint32_t)(4 * i + drow) * (uint32_t)p.K + (uint32_t)(((lane & 15) ^ (4 * i + drow)) << 4);
   const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)smem + (uint32_t)part * (2 * MT * KCHUNK);
-  const uint8_t* const arows = reinterpret_cast<const uint8_t*>(p.A) + (size_t)m0 * p.K + k0;
   auto dma_chunk = [&](int chunk, int buf) {
-    lds_dma_rows<MB>(arows + (size_t)chunk * KCHUNK, dvo, (uint32_t)p.K * 16u,
-                     __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)buf * (MT * KCHUNK) + (uint32_t)wave * 1024));
+    const uint8_t* const src = reinterpret_cast<const uint8_t*>(p.A) + (size_t)(m0 + (OWN ? 32 * wave : 0)) * p.K + (size_t)k0 + (size_t)chunk * KCHUNK;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)buf * (MT * KCHUNK) + (uint32_t)wave * (OWN ? 8192 : 1024));
+    if constexpr (OWN) lds_dma_own_rows(src, src + (size_t)16 * p.K, dvo, dst);
+    else lds_dma_rows<MB>(src, dvo[0], (uint32_t)p.K * 16u, dst);
   };
   // B-operand address of row block 0 at k-step 0 (per lane); row block mb adds an immediate
   const uint32_t boff = (uint32_t)part * (2 * MT * KCHUNK) + (uint32_t)(lane & 15) * 256 + (uint32_t)(((lane >> 4) ^ (lane & 15)) << 4);
@@ -203,7 +223,8 @@ __global__ __launch_bounds__(256 * KW, 2) void w4a8_gemm_exact_kernel(GemmArgs p
     }
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VM_AFTER_DMA) : "memory");   // my pieces of chunk c landed
     __syncthreads();          // chunk c is visible in lds[c & 1]; everybody is done reading lds[(c + 1) & 1]
-    const uint8_t* abuf = smem + (c & 1) * (MT * KCHUNK);
+    // (so written, and not smem + (c & 1) * ..., the per-group kernel waits for step 1's weights in front of the next requests and not for those, too)
+    const uint8_t* abuf = reinterpret_cast<uint8_t (*)[MT * KCHUNK]>(smem)[c & 1];
 
     const bool small = MODE == MODE_GRP && MB < 8 && grp_scales_small(gs[0], gs[1]);      // (MB = 8 has no registers for both forms)
     // unpack (+ lane transpose / per-group dequant) of k-step s into MFMA A operands
