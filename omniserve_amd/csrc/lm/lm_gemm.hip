@@ -196,10 +196,19 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 #pragma unroll
     for (int i = 0; i < XP; ++i) dma16_uncounted(xsrc[i] + t * (KW * RB), dst + WST + 1024 * xp[i]);
   };
-  // sums of 4 stages and the sum of those: shorter chains of f32 additions than K / 32
+  // sums of 4 stages (2, 1, half a one) and the sum of those: chains of f32 additions no longer than an eighth of K
+  const int chain = k >= 64 * KSTEP ? 3 : k >= 32 * KSTEP ? 1 : 0;
+  const bool halves = k < 16 * KSTEP;
   f32x4 acc[MB], total[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) acc[m] = total[m] = zero4();
+  auto end_chain = [&] {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      total[m] += acc[m];
+      acc[m] = zero4();
+    }
+  };
   auto multiply = [&](int t) {
     const uint8_t* wt = lds + (t % R) * ST + wave * (16 * RB);
     const uint8_t* xt = lds + (t % R) * ST + WST;
@@ -211,16 +220,12 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
       for (int m = 0; m < MB; ++m) b[v][m] = *(const frag_t*)(xt + 16 * m * RB + T::slot(l15, 4 * v + l4));
     }
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
+    for (int v = 0; v < 2; ++v) {
 #pragma unroll
       for (int m = 0; m < MB; ++m) acc[m] = mma(a[v], b[v][m], acc[m]);
-    if ((t & 3) == 3) {
-#pragma unroll
-      for (int m = 0; m < MB; ++m) {
-        total[m] += acc[m];
-        acc[m] = zero4();
-      }
+      if (v == 0 && halves) end_chain();
     }
+    if ((t & chain) == chain) end_chain();
   };
   const int nst = (s1 - s0 - h + KW - 1) / KW;
   wait_pieces<0>();                                        // the compiler's own loads
