@@ -654,9 +654,8 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   return LM_OK;
 }
 
-template <int NR, int MB, int EPI>
+template <int NR, int MB, int EPI, int KW = 8>
 static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s) {
-  constexpr int KW = 8;
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
   const dim3 grid((n + 16 * NR - 1) / (16 * NR), a.groups + has_b, a.perm ? 1 : (max_rows + 16 * MB - 1) / (16 * MB));
   hipLaunchKernelGGL((gemm_rows_kernel<NR, MB, KW, EPI>), grid, dim3(64 * KW), 0, s, a);
@@ -723,25 +722,33 @@ static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part,
 }
 
 // Which kernel, and how dealt.  experts: groups by perm or two parts; how many of them have rows is not known here, and 64 channels measured best from
-// 60 to 1000 MB.  gemm_rows_kernel takes
+// 60 to 1000 MB.  gemm_rows_kernel takes (figures: MI355X, us, stream / gemm_rows_kernel, bf16 where nothing else is said)
 //   * more than 64 rows of few channels (the router of a prompt) or of one matrix per head: workgroups along the rows;
-//   * 33 - 64 rows where channels and K slices make too few workgroups: there too (MI355X, 64 rows: 64 x 2048 7.7 us in 8 slices, 6.1 so; 8 heads of
+//   * 33 - 64 rows where channels and K slices make too few workgroups: there too (64 rows: 64 x 2048 7.7 in 8 slices / 6.1; 8 heads of
 //     128 x 512 4.2 / 3.8; but 16 heads of 128 x 256 3.7 / 4.7, and 128 x 4096 is better in slices);
-//   * up to 16 rows where a ring is only filled once (16 heads of 256 x 128 3.5 / 3.2, 4096 x 128 3.2 / 2.8; 4096 x 256 3.2 / 3.3; more workgroups
-//     than CUs take 64 channels each, 32 heads of 512 x 128 4.1 / 8.0);
+//   * up to 16 rows where a ring is only filled once: up to 4096 channels (16 heads of 256 x 128 3.5 / 3.2, 4096 x 128 3.2 / 2.8; 4096 x 256 3.2 / 3.3; f32
+//     4096 x 192 4.0 / 3.6, 16 heads of 128 x 256 3.7 / 3.3, and at 32 rows 4.0 / 3.5), 9600 to 16384 of K up to 128 with 32 channels per
+//     workgroup (32 heads of 512 x 128 3.8 / 3.8, weights in the caches 3.5 / 3.0; of 512 x 64 3.3 / 2.9; 512 x 256 4.4 / 4.8; 32000 x 128 4.5 / 5.8);
+//   * up to 16 tokens of few small experts, which leave the stream too few workgroups (1 and 16 tokens, 2 of 8 x 1024 x 1024 5.5 / 3.9 and 6.7 / 6.4, of
+//     512 x 512 4.4 / 3.2 and 4.7 / 3.5; but 4 of 16 x 1024 x 512 5.2 / 8.6 at 16);
 //   * the gated unit of up to 16 rows over few weights, whose stream of 64 channels per workgroup has too few workgroups (16 rows: 2048 x 512
-//     4.2 / 3.7 us, 4096 x 256 4.2 / 3.7, 2048 x 1024 6.4 / 6.3, 4096 x 1024 6.6 / 6.5).
+//     4.7 / 3.9, 4096 x 256 4.2 / 3.7, 2048 x 1024 6.4 / 6.1, 4096 x 1024 6.5 / 6.2; 1024 x 2048 9.1 / 9.2; f32 2048 x 1024 9.3 / 10.2), with short K also of more rows (17 and 32 rows: 2048 x 512 4.8 /
+//     4.4 and 4.9 / 4.6, 4096 x 512 4.9 / 4.5 and 5.0 / 4.6; 1024 x 512 4.2 / 4.4; 64 rows 5.7 / 5.8; f32 13.3 / 11.4).
 static RowsPlan plan_rows(int groups, int n, int k, int rows, int epi, bool experts, bool sliced) {
+  const int64_t bytes_k = (int64_t)k * (int)sizeof(elem_t), channels = (int64_t)groups * n;
+  if (experts && epi != LM_EPI_GLU && rows <= 16 && channels <= 8192) return RowsPlan{0, 1};
   if (experts && (epi == LM_EPI_GLU || rows <= 64)) return RowsPlan{4, 1};
   if (epi == LM_EPI_GLU) {
-    if (rows <= 16 && (int64_t)groups * n * k * (int)sizeof(elem_t) <= (4 << 20)) return RowsPlan{0, 1};
+    if (rows <= 16 && channels * bytes_k <= (bytes_k <= 2048 ? 8 << 20 : 4 << 20)) return RowsPlan{0, 1};
+    if (rows <= (LM_ELEM ? 64 : 32) && k <= 512 && channels >= 2048 && channels <= 4096) return RowsPlan{0, 1};
     return plan_stream(groups, n, k, rows, true, sliced);
   }
   if (rows > 64) return RowsPlan{0, 1};
   const RowsPlan pl = plan_stream(groups, n, k, rows, false, sliced);
-  const int64_t bytes_k = (int64_t)k * (int)sizeof(elem_t), channels = (int64_t)groups * n;
   if (rows > 32 && n <= 256 && channels <= 1024 && (pl.slices == 1 || bytes_k <= 4096)) return RowsPlan{0, 1};
-  if (rows <= 16 && bytes_k <= 512 && channels <= 4096) return RowsPlan{0, 1};
+  if (k <= 256 && n <= 256 && channels <= 2048 && rows <= 32) return RowsPlan{0, 1};
+  if (rows <= 16 && channels <= 4096 && k <= 256 && bytes_k <= 768) return RowsPlan{0, 1};
+  if (rows <= 16 && channels >= 9600 && channels <= 16384 && k <= 128) return RowsPlan{0, 1};
   return pl;
 }
 
@@ -754,9 +761,15 @@ static int launch_few(const GemmArgs& a, int max_rows, int has_b, float* part, h
   if (has_b) at |= (uintptr_t)a.b.w | (uintptr_t)a.b.x;
   if (at & 15) pl = RowsPlan{0, 1};
   if (pl.nw > 0) return launch_stream<EPI>(a, has_b, pl, part, s);
-  if constexpr (EPI == LM_EPI_GLU) return launch_rows<2, 1, EPI>(a, max_rows, has_b, s);
-  else if (max_rows <= 64) return launch_rows<1, 1, EPI>(a, max_rows, has_b, s);
-  else return launch_rows<2, 4, EPI>(a, max_rows, has_b, s);
+  if constexpr (EPI == LM_EPI_GLU) {
+    if (max_rows <= 16) return launch_rows<2, 1, EPI>(a, max_rows, has_b, s);
+    else if (max_rows <= 32) return launch_rows<2, 2, EPI>(a, max_rows, has_b, s);
+    else return launch_rows<2, 4, EPI>(a, max_rows, has_b, s);
+  } else {
+    if (max_rows > 64) return launch_rows<2, 4, EPI>(a, max_rows, has_b, s);
+    else if (max_rows <= 16 && (int64_t)a.groups * a.a.n > 4096 && !a.perm) return launch_rows<2, 1, EPI, 4>(a, max_rows, has_b, s);
+    else return launch_rows<1, 1, EPI>(a, max_rows, has_b, s);
+  }
 }
 
 }  // namespace lm

@@ -82,4 +82,5 @@ def test_few_rows_of_short_k_spread_over_the_chip():
             assert h.lm_gemm_rows_channels(1, 4096, k, 20, 0, 1, ctypes.byref(slices)) == 16 and slices.value == 1
             assert h.lm_gemm_rows_channels(16, 256, k, 17, 0, 0, None) == 16
             assert h.lm_gemm_rows_channels(1, 4096, k, 15, 0, 1, ctypes.byref(slices)) == 0 and slices.value == 1
-            assert h.lm_gemm_rows_channels(32, 512, k, 16, 0, 0, None) == 64
+            assert h.lm_gemm_rows_channels(32, 512, k, 17, 0, 0, None) == 64
+            assert h.lm_gemm_rows_channels(32, 512, k, 16, 0, 0, None) == (0 if k <= 128 else 64)

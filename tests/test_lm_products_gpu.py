@@ -264,6 +264,53 @@ def test_few_rows_between_boundaries(m, dtype):
     _close(ys, x.double() @ ws.double().t(), dtype)
 
 
+# What goes around the stream: 32 channels per workgroup (short K of many channels, some past the last whole workgroup), 16 rows in turn (heads of few
+# channels), the gated unit in 16 - 64 rows at once.
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("heads,n,k,m", [(1, 9616, 64, 16), (1, 16368, 128, 9), (32, 512, 128, 1), (36, 272, 64, 16), (8, 256, 256, 17), (16, 128, 192, 32)])
+def test_short_k(heads, n, k, m, dtype):
+    ops = _ops(dtype)
+    assert _rows_plan(ops, heads, n, k, m, sliced=heads == 1) == (0, 1)
+    x, w = _randn(36, dtype, m, heads * k), _randn(37, dtype, heads, n, k) * k ** -0.5
+    gate, guard = _randn(38, dtype, m, heads * n), torch.full((m + 2, heads * n), 7.0, dtype=dtype, device=DEV)
+    want = torch.cat([x[:, h * k:(h + 1) * k].double() @ w[h].double().t() for h in range(heads)], dim=1)
+    _close(ops.head_products(x, w, guard[1:-1], k, n), want, dtype)
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+    got = ops.head_products(x, w, guard[1:-1], k, n, gate=gate)
+    assert errors(got.float().cpu().numpy(), (want * torch.sigmoid(gate.double())).cpu().numpy()).max() < max(TOL[dtype], 5e-6)
+    if heads == 1:
+        assert errors(ops.matmul(x, w[0], out_f32=True, scale=0.5).cpu().numpy(), 0.5 * want.cpu().numpy()).max() < 2e-6
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k", [(1, 2080, 512), (17, 2048, 512), (32, 4096, 448), (31, 2080, 64), (33, 2080, 512), (64, 4096, 512)])
+def test_small_gated_units(m, n, k, dtype):
+    ops = _ops(dtype)
+    assert (_rows_plan(ops, 1, n, k, m, epi=2)[0] == 0) == (m <= 32 or dtype == torch.float32)
+    x, w, b = _randn(39, dtype, m, k), _randn(40, dtype, n, k) * k ** -0.5, _randn(41, torch.float32, n) * 0.1
+    y = (x.double() @ w.double().t() + b.double()).view(m, n // 32, 2, 16)
+    want = (torch.nn.functional.gelu(y[:, :, 0], approximate="tanh") * y[:, :, 1]).reshape(m, n // 2)
+    assert errors(ops.glu(x, w, b, "gelu_tanh").float().cpu().numpy(), want.cpu().numpy()).max() < max(TOL[dtype], 5e-6)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("tokens", [1, 5, 16])
+@pytest.mark.parametrize("E,n", [(24, 400), (16, 512), (5, 80)])
+def test_experts_of_few_tokens(E, n, tokens, dtype):
+    """more than 8192 channels (the stream) and fewer, a part b that ends before and behind the experts' channels"""
+    ops, top, W = _ops(dtype), 3, 320
+    z = _randn(42, torch.float32, tokens, E)
+    wts, order = ops.route(z, torch.zeros((E,), device=DEV), E, top)
+    h, w, ws = _randn(43, dtype, tokens, W), _randn(44, dtype, E, n, W) * W ** -0.5, _randn(45, dtype, 432, W) * W ** -0.5
+    y, ys = torch.full((tokens * top + 2, n), 7.0, dtype=dtype, device=DEV), torch.full((tokens + 2, 432), 7.0, dtype=dtype, device=DEV)
+    ops.grouped(order, tokens, h, w, y[1:-1], False, False, (h, ws, ys[1:-1]))
+    for t in (y, ys):
+        assert (t[0] == 7).all() and (t[-1] == 7).all()
+    ids = torch.argsort(-z, dim=1, stable=True)[:, :top]
+    _close(y[1:-1], torch.stack([h[t].double() @ w[ids[t, c]].double().t() for t in range(tokens) for c in range(top)]), dtype)
+    _close(ys[1:-1], h.double() @ ws.double().t(), dtype)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("n,k", [(4096, 64), (4096, 128), (4096, 192), (2048, 320), (4096, 640), (4096, 1088), (10816, 1536), (2048, 4096)])
 def test_sums_of_the_stream_are_as_exact(n, k, dtype):
