@@ -230,12 +230,16 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
   // rows far apart are slower to read, but not where K slices read them at several places (512 rows of 8192 x 28672 per-channel: 1.08 us per chunk of
   // two K parts, 0.83 at 14336; 256 rows of 7168 x 8192 W8A8 1.68, 1.25 at 4096: 126 and 58 us where slices take 105 and 47)
   const float far = mode == MODE_W8 && K >= 8192 ? 1.2f : mode == MODE_CHN && K >= 16384 ? 1.17f : 1.f;
+  // whole bands of 8 full row tiles go in an order of their own (w4a8_gemm_exact_kernel): 4096 rows of 8192 x 28672 per-channel 607 us, 632 with K in two
+  // parts; 4096 of 10240 x 8192 per-group 336, 346 in tiles of 112 rows; 8192 of 5120 x 13824 546, 563
+  const float whole = mode != MODE_W8 && M % 1024 == 0 ? 0.96f : 1.f;
   float time = 1e30f;
   auto offer = [&](int mb, int kw, int split) {
     const long long tiles = (long long)((M + 16 * mb - 1) / (16 * mb)) * (N / 256) * split;
     float t = grid_time(c, mb, kw, tiles, (split == 1 ? far : 1.f) * (float)(K / (split * KCHUNK)));
     // the slabs written, read and reduced by a launch of their own
     if (split > 1 && !slab_only) t += 4.5f + (float)split * M * N * 8.f / 4.5e6f;
+    if (mb == 8 && kw == 1 && split == 1) t *= whole;
     if (t < time) { time = t; best = PrefillPlan{mb, kw, split}; }
   };
   for (int mb = 8; mb >= 4; --mb) {
