@@ -163,7 +163,9 @@ __device__ __forceinline__ void wait_stage() {
 
 // rows (at most 16 MB) of x times 16 NW channels of w, stages s0 .. s1 - 1 of k, into red [KW][16 MB][16 NW + 4]: part h of the
 // workgroup's waves takes every KW-th stage through a ring of its own
-template <int MB, int NW, int KW>
+// SHORT: k may be below CHAIN_K.
+constexpr int CHAIN_K = 64 * KSTEP;
+template <int MB, int NW, int KW, bool SHORT>
 __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int n, int64_t k, int n0, const elem_t* x, int64_t ldx,
                                               const int* perm, int div, int rows, int s0, int s1) {
   constexpr int WST = 16 * NW * RB, XST = 16 * MB * RB, ST = WST + XST, R0 = ring_bytes<NW, KW> / ST;
@@ -196,9 +198,10 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 #pragma unroll
     for (int i = 0; i < XP; ++i) dma16_uncounted(xsrc[i] + t * (KW * RB), dst + WST + 1024 * xp[i]);
   };
-  // sums of 4 stages (2, 1, half a one) and the sum of those: chains of f32 additions no longer than an eighth of K
-  const int chain = k >= 64 * KSTEP ? 3 : k >= 32 * KSTEP ? 1 : 0;
-  const bool halves = k < 16 * KSTEP;
+  // sums of 4 stages (2, 1, half a one) and the sum of those: chains of f32 additions no longer than an eighth of K.  (A form of its own for long K: with
+  // the choice in it that one took 3 - 7 % more, 16 tokens of 8 of 64 x 1280 x 2048 52.8 -> 55.5 us.)
+  const int chain = !SHORT || k >= CHAIN_K ? 3 : k >= CHAIN_K / 2 ? 1 : 0;
+  const bool halves = SHORT && k < CHAIN_K / 4;
   f32x4 acc[MB], total[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) acc[m] = total[m] = zero4();
@@ -260,7 +263,7 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 
 // A workgroup: 16 NW channels of a group, rows 0 .. 16 MB - 1 of it, K slice blockIdx.z.  With several slices (one group) the f32 sums of a
 // slice go to part [slice][rows][n] and gemm_reduce_kernel finishes them.
-template <int EPI, int NW, int KW>
+template <int EPI, int NW, int KW, bool SHORT>
 __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, float* part) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[KW * ring_bytes<NW, KW>];
   constexpr int RC = 16 * NW, NT = 64 * NW * KW;
@@ -282,10 +285,10 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
     const int here = min(64, rows - m0), mb = (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
     const int* pm = perm ? perm + m0 : nullptr;
-    if (mb == 1) stream_stages<1, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else if (mb == 2) stream_stages<2, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else if (mb == 3) stream_stages<3, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else stream_stages<4, NW, KW>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    if (mb == 1) stream_stages<1, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 2) stream_stages<2, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 3) stream_stages<3, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else stream_stages<4, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     const float* red = (const float*)lds;
     auto sum = [&](int m, int c) {
       f32x4 v = *(const f32x4*)&red[m * (RC + 4) + c];
@@ -690,14 +693,20 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
 }
 
 // K parts inside a workgroup where there is no second one to run beside it on its CU
-template <int EPI, int NW>
-static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+template <int EPI, int NW, bool SHORT>
+static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
   constexpr int KW = NW <= 2 ? 4 : 2;
   if ((int64_t)grid.x * grid.y * grid.z <= 256)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW>), grid, dim3(64 * NW * KW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT>), grid, dim3(64 * NW * KW), 0, s, a, part);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1>), grid, dim3(64 * NW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT>), grid, dim3(64 * NW), 0, s, a, part);
+}
+
+template <int EPI, int NW>
+static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+  if (a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K)) launch_stream_form<EPI, NW, true>(a, n, has_b, slices, part, s);
+  else launch_stream_form<EPI, NW, false>(a, n, has_b, slices, part, s);
 }
 
 template <int EPI>
