@@ -16,6 +16,7 @@
 #include "row_reduce.h"
 #include "row_kernels.h"
 #include "tp_comm.h"
+#include "norm_rows.h"
 #include <cstdlib>
 
 namespace omni {
@@ -541,6 +542,10 @@ static inline PrefetchArgs take_prefetch(int tokens) {
   if (tokens >= ROWS_MANY) pf.blocks = 0;    // many-row launches are bandwidth-bound themselves: nothing idles
   return pf;
 }
+// norm_pairs_kernel's rows (norm_rows.hip has both sides); K slabs within 32-bit offsets of their first byte
+static inline bool norm_pairs_ok(int tokens, int hidden, int sk = 1) {
+  return tokens < ROWS_MANY && hidden % 1024 == 0 && hidden <= 8192 && (unsigned long long)sk * tokens * hidden * sizeof(int32_t) < 1ull << 32;
+}
 // (kernels without a PrefetchArgs parameter)
 #define OMNI_V2_LAUNCH_PLAIN(KERNEL, tokens, hidden, elems, ...)                                                \
   do {                                                                                                          \
@@ -651,6 +656,11 @@ extern "C" int omni_rms_norm_general(void* out_i8, const void* in_f16, const voi
   if (!out_i8 || !in_f16 || !weight_f16 || !scale_f16 || tokens < 0 || hidden < 1) return OMNI_EINVAL;
   if (hidden > VPT * NT_MAX) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
+  if (norm_pairs_ok(tokens, hidden)) {
+    norm_pairs_plain(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, nullptr, (half_t*)scale_f16, eps}, (const half_t*)in_f16, tokens, hidden,
+                     take_prefetch(tokens), (hipStream_t)stream);
+    return omni_launch_status();
+  }
   {
     const int nv = norm_block(hidden, true);
     if (v2_ok(hidden, nv)) {
@@ -677,6 +687,11 @@ extern "C" int omni_rms_norm_general_fuse_sum(void* out_i8, const void* in_f16,
     return OMNI_EINVAL;
   if (hidden > VPT * NT_MAX) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
+  if (norm_pairs_ok(tokens, hidden)) {
+    norm_pairs_plain(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps}, (const half_t*)in_f16, tokens,
+                     hidden, take_prefetch(tokens), (hipStream_t)stream);
+    return omni_launch_status();
+  }
   {
     const int nv = norm_block(hidden, true);
     if (v2_ok(hidden, nv)) {
@@ -756,6 +771,11 @@ extern "C" int omni_add_rms_norm_general_fuse_sum(void* out_i8, void* residual_f
     return OMNI_EINVAL;
   if (hidden > VPT * NT_MAX) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
+  if (norm_pairs_ok(tokens, hidden)) {
+    norm_pairs_add(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps}, (half_t*)residual_f16,
+                   (const half_t*)delta_f16, tokens, hidden, take_prefetch(tokens), (hipStream_t)stream);
+    return omni_launch_status();
+  }
   {
     const int nv = norm_block(hidden, true);
     if (v2_ok(hidden, nv)) {
@@ -858,21 +878,16 @@ extern "C" int omni_splitk_add_rms_norm_general_fuse_sum(void* out_i8, void* res
   const int nv = norm_block(hidden, true);
   if (!v2_ok(hidden, nv)) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
+  if (norm_pairs_ok(tokens, hidden, sk)) {
+    norm_pairs_slabs(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps},
+                     NormSlabs{(half_t*)residual_f16, (const int32_t*)slab_i32, (size_t)tokens * hidden, sk, (const half_t*)wscales_f16,
+                               (const half_t*)w_szs_f16, (const half_t*)ascales_in_f16, (const half_t*)a_ssums_in_f16},
+                     tokens, hidden, take_prefetch(tokens), (hipStream_t)stream);
+    return omni_launch_status();
+  }
   SrcSlabAddChn src{(half_t*)residual_f16, (const int32_t*)slab_i32, (size_t)tokens * hidden, sk, hidden,
                     (const half_t*)wscales_f16, (const half_t*)w_szs_f16, (const half_t*)ascales_in_f16,
                     (const half_t*)a_ssums_in_f16, (half_t)0.0f, (half_t)0.0f};
-  if (tokens < ROWS_MANY && hidden > 512 * VT && hidden <= 512 * 2 * VT) {
-    // decode-size rows of 4097 .. 8192 columns (Llama-2-70B): two vectors per thread with BATCHED requests -- the unbatched
-    // source made the second vector's slab loads a second memory round trip of the row chain
-    typedef SrcSlabAddT<true, true> SrcB;
-    SrcB srcb{src.res, src.slab, src.sstride, src.sk, src.stride, src.wscales, src.wsz, src.ascales, src.asum, (half_t)0.0f, (half_t)0.0f};
-    const PrefetchArgs pf = take_prefetch(tokens);
-    size_t lds = (size_t)hidden * sizeof(float);
-    if (pf.blocks > 0 && lds < 8 * 1024) lds = 8 * 1024;
-    hipLaunchKernelGGL((general_norm_v2_kernel<512, 2, true, SrcB>), dim3(tokens + pf.blocks), dim3(512), lds, (hipStream_t)stream,
-                       (int8_t*)out_i8, srcb, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps, hidden, nv, pf);
-    return omni_launch_status();
-  }
   const bool v2_batched = false;
   #undef KQ_
   #define KQ_(RT_, RV_) general_norm_v2_kernel<RT_, RV_, true, SrcSlabAddChn>
@@ -893,6 +908,13 @@ extern "C" int omni_splitk_w8_add_rms_norm_general_fuse_sum(void* out_i8, void* 
   const int nv = norm_block(hidden, true);
   if (!v2_ok(hidden, nv)) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
+  if (norm_pairs_ok(tokens, hidden, sk)) {
+    norm_pairs_slabs(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps},
+                     NormSlabs{(half_t*)residual_f16, (const int32_t*)slab_i32, (size_t)tokens * hidden, sk, (const half_t*)wscales_f16, nullptr,
+                               (const half_t*)ascales_in_f16, nullptr},
+                     tokens, hidden, take_prefetch(tokens), (hipStream_t)stream);
+    return omni_launch_status();
+  }
   SrcSlabAddW8 src{(half_t*)residual_f16, (const int32_t*)slab_i32, (size_t)tokens * hidden, sk, hidden,
                    (const half_t*)wscales_f16, (const half_t*)nullptr, (const half_t*)ascales_in_f16,
                    (const half_t*)nullptr, (half_t)0.0f, (half_t)0.0f};

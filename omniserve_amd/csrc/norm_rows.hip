@@ -1,0 +1,311 @@
+// rms_norm_general[_fuse_sum] with per-token quantisation for rows of 1024 .. 8192 channels in whole 1024s, fewer than ROWS_MANY of them (reference:
+// kernels/csrc/layernorm_kernels.cu:58-331).  Everything else stays on general_norm_v2_kernel (row_kernels.h), to whose bits this kernel keeps.
+//
+// At these sizes a row is one compute unit's serial chain -- requests, two reductions, codes -- and the launch lasts as long as that chain.
+// The reference's order of additions (1024 virtual threads, thread t adds up channels t, t + 1024, ..; a butterfly over 32 threads, one over
+// their 32 sums) is what general_norm_v2_kernel replays out of an LDS copy of the row, by two of its eight waves, behind a barrier, twice.  Here the
+// threads own the channels as the virtual threads do: thread p holds 2 p and 2 p + 1 of every 1024, so that
+//
+//  * the per-thread sums are formed in registers as the values appear: no copy, no replay, no barrier in front of them;
+//  * a virtual warp is a row of 16 lanes: its butterfly is four DPP additions; the one over the 32 sums reads 16 bytes of LDS and is four more;
+//  * the row maximum and the sum of the normalised values cross the workgroup together: two barriers in all instead of seven.
+//
+// MI355X, inside the captured step of the 8B model (4096 channels), general_norm_v2_kernel -> this one, us: 1 row, 8 slabs 8.3 -> 6.5; 16 rows, 8 slabs 8.0
+// -> 6.3; first layer, no slabs, 6.3 -> 5.5.  What is left: the first load (the slabs come from other XCDs' launches; 128 KiB of them into one compute
+// unit) and a launch's ends.
+#include "common.h"
+#include "norm_rows.h"
+
+namespace omni {
+
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+// One row's array behind a scalar descriptor: an access is one instruction with the lane's bytes and a scalar offset, and no address arithmetic
+// in vector registers (global loads of this many arrays got two additions each).
+struct RowArray {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ explicit RowArray(const void* base) : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xFFFFFFFFu, 0x00020000)) {}
+  __device__ __forceinline__ v2h pair(uint32_t lane, uint32_t scalar) const {
+    return __builtin_bit_cast(v2h, __builtin_amdgcn_raw_buffer_load_b32(r, lane, scalar, 0));
+  }
+  __device__ __forceinline__ v2i two(uint32_t lane, uint32_t scalar) const {
+    return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, lane, scalar, 0));
+  }
+  __device__ __forceinline__ void put(uint32_t lane, uint32_t scalar, v2h v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, lane, scalar, 0);
+  }
+  __device__ __forceinline__ void put16(uint32_t lane, uint32_t scalar, uint16_t v) const { __builtin_amdgcn_raw_buffer_store_b16(v, r, lane, scalar, 0); }
+};
+
+// of more than 8 slabs, those whose requests are in flight together
+template <int C>
+constexpr int MANY_SLABS = C <= 4 ? 16 : 12;
+
+// The norm's weights, requested first, are waited for here, in front of the residual's stores: a wait behind those would be for them, too
+template <int C>
+__device__ __forceinline__ void arrived(v2h (&g)[C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) asm volatile("" : "+v"(g[c]));
+}
+
+// residual += h(epilogue(sum of the K slabs)); ZP: ((acc * sw) * sa) - (sz * as), else acc * (sw * sa)
+template <bool ZP>
+struct PairSlabs {
+  NormSlabs s;
+  __device__ __forceinline__ void pin() const {
+    asm volatile("" ::"s"(s.res), "s"(s.slab), "s"(s.sstride), "s"(s.sk), "s"(s.wscales), "s"(s.wsz), "s"(s.ascales), "s"(s.asum));
+  }
+  // SK: slabs whose requests all go out in front of the first addition (those beyond s.sk read slab 0 again); a form of its own for each, to the
+  // end: joined before the additions, hipcc waits for every load at the join
+  template <int C, int SK>
+  __device__ __forceinline__ void values_of(int row, uint32_t at, v2h (&g)[C], float (&x)[C][2]) const {
+    const half_t sa_h = s.ascales[row];
+    half_t as_h = (half_t)0.0f;
+    if constexpr (ZP) as_h = s.asum[row];
+    const RowArray res(s.res + (size_t)row * (1024 * C)), slab(s.slab + (size_t)row * (1024 * C)), ws(s.wscales), wz(s.wsz);
+    const uint32_t step = (uint32_t)(s.sstride * 4);
+    v2i t[SK][C];
+#pragma unroll
+    for (int k = 0; k < SK; ++k)
+#pragma unroll
+      for (int c = 0; c < C; ++c) t[k][c] = slab.two(2 * at, (SK <= 8 || k < s.sk ? k * step : 0) + 4096 * c);
+    v2h a[C], sw[C], sz[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      a[c] = res.pair(at, 2048 * c);
+      sw[c] = ws.pair(at, 2048 * c);
+      if constexpr (ZP) sz[c] = wz.pair(at, 2048 * c);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // every request in front of the first wait
+    arrived(g);
+    v2i acc[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = t[0][c];      // integers: any order is exact
+#pragma unroll
+    for (int k = 1; k < SK; ++k)
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[c] += SK <= 8 || k < s.sk ? t[k][c] : (v2i){0, 0};
+    if constexpr (SK > 8)
+      for (int k = SK; k < s.sk; ++k)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[c] += slab.two(2 * at, k * step + 4096 * c);
+    const float sa = (float)sa_h, as = (float)as_h;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      v2h o;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {      // the product's own epilogue (qgemm_kernel.h), each step rounded to f32
+        half_t ep;
+        if constexpr (ZP) {
+          float v = (float)acc[c][e] * (float)sw[c][e];
+          v = v * sa;
+          const float z = (float)sz[c][e] * as;
+          ep = (half_t)rounded_f32(v - z);
+        } else {
+          const float sc = (float)sw[c][e] * sa;
+          ep = (half_t)rounded_f32((float)acc[c][e] * sc);
+        }
+        o[e] = (half_t)((float)a[c][e] + (float)ep);
+        x[c][e] = (float)o[e];
+      }
+      res.put(at, 2048 * c, o);
+    }
+  }
+  template <int C>
+  __device__ __forceinline__ void values(int row, int p, v2h (&g)[C], float (&x)[C][2]) const {
+    const uint32_t at = 4 * p;      // bytes of a pair of halves
+    switch (s.sk) {
+      case 1: return values_of<C, 1>(row, at, g, x);
+      case 2: return values_of<C, 2>(row, at, g, x);
+      case 3: return values_of<C, 3>(row, at, g, x);
+      case 4: return values_of<C, 4>(row, at, g, x);
+      case 5: return values_of<C, 5>(row, at, g, x);
+      case 6: return values_of<C, 6>(row, at, g, x);
+      case 7: return values_of<C, 7>(row, at, g, x);
+      case 8: return values_of<C, 8>(row, at, g, x);
+      default: return values_of<C, MANY_SLABS<C>>(row, at, g, x);
+    }
+  }
+};
+
+struct PairAdd {      // residual += delta
+  half_t* res;
+  const half_t* delta;
+  __device__ __forceinline__ void pin() const { asm volatile("" ::"s"(res), "s"(delta)); }
+  template <int C>
+  __device__ __forceinline__ void values(int row, int p, v2h (&g)[C], float (&x)[C][2]) const {
+    const RowArray r(res + (size_t)row * (1024 * C)), d(delta + (size_t)row * (1024 * C));
+    const uint32_t at = 4 * p;
+    v2h a[C], b[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      a[c] = r.pair(at, 2048 * c);
+      b[c] = d.pair(at, 2048 * c);
+    }
+    arrived(g);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      v2h o;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        o[e] = (half_t)((float)a[c][e] + (float)b[c][e]);
+        x[c][e] = (float)o[e];
+      }
+      r.put(at, 2048 * c, o);
+    }
+  }
+};
+
+struct PairPlain {
+  const half_t* in;
+  __device__ __forceinline__ void pin() const { asm volatile("" ::"s"(in)); }
+  template <int C>
+  __device__ __forceinline__ void values(int row, int p, v2h (&g)[C], float (&x)[C][2]) const {
+    const RowArray r(in + (size_t)row * (1024 * C));
+    v2h a[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) a[c] = r.pair(4 * p, 2048 * c);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) x[c][e] = (float)a[c][e];
+  }
+};
+
+// The sum over lanes l ^ 8, ^ 4, ^ 2, ^ 1 of a row of 16, in this order (behind the first addition the values repeat every 8 lanes, so that a
+// rotation by 4 finds the partner), in every lane
+__device__ __forceinline__ float row16_sum(float v) {
+  v = v + dpp_mov<0x128>(v);      // row_ror:8
+  v = v + dpp_mov<0x124>(v);      // row_ror:4
+  v = v + lane_xor2(v);
+  return v + lane_xor1(v);
+}
+
+// LDS is published, stores to memory are not waited for (__syncthreads waits for the residual's here)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int C, bool FUSE_SUM, typename Src>
+__global__ __launch_bounds__(512) void norm_pairs_kernel(int8_t* __restrict__ out, Src src, const half_t* __restrict__ gamma, half_t* __restrict__ sum_out,
+                                                         half_t* __restrict__ scale_out, float eps, PrefetchArgs pf) {
+  constexpr int H = 1024 * C;
+  __shared__ __attribute__((aligned(16))) float lds[8 * 256];      // 1 KiB a wave for fetching workgroups; a row's uses the first 104 words
+  // one batch of scalar loads for the test below and the row's path
+  src.pin();
+  asm volatile("" ::"s"(out), "s"(gamma), "s"(sum_out), "s"(scale_out), "s"(eps), "s"(pf.blocks), "s"(pf.first_block));
+  if (pf.blocks > 0 && (int)blockIdx.x >= pf.first_block) {      // extra workgroups: the next product's weights into L2
+    prefetch_weights_to_l2(pf, lds);
+    return;
+  }
+  const int p = threadIdx.x, lane = p & 63, wave = p >> 6, row = blockIdx.x;
+  const RowArray gains(gamma);
+  v2h g[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) g[c] = gains.pair(4 * p, 2048 * c);
+  float x[C][2];
+  src.template values<C>(row, p, g, x);
+
+  // sum and sum of squares: the virtual thread's, the virtual warp's, the row's
+  float s[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      s[0][e] = s[0][e] + x[c][e];
+      s[1][e] = s[1][e] + x[c][e] * x[c][e];
+    }
+  auto warp_sum = [&](float (&v)[2]) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[e] = row16_sum(v[e]);
+    return v[0] + v[1];
+  };
+  const int vw = 4 * wave + (lane >> 4);                          // virtual warp; its sums lie beside those of vw ^ 16
+  float* const r1 = lds;                                          // [16][sum, sum, square, square]
+  float* const r2 = lds + 64;                                     // [16][2] sums of the normalised values, then 8 maxima
+  {
+    const float w0 = warp_sum(s[0]), w1 = warp_sum(s[1]);
+    if ((lane & 15) == 0) {
+      r1[(vw & 15) * 4 + (vw >> 4)] = w0;
+      r1[(vw & 15) * 4 + 2 + (vw >> 4)] = w1;
+    }
+  }
+  lds_barrier();
+  const v4f q4 = *reinterpret_cast<const v4f*>(r1 + (lane & 15) * 4);
+  const float mean = row16_sum(q4[0] + q4[1]) / (float)H;
+  const float rstd = 1.0f / __builtin_sqrtf(row16_sum(q4[2] + q4[3]) / (float)H + eps);
+
+  float amax = (float)(half_t)1e-6f;
+  float hs[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      float y = (x[c][e] - mean) * rstd;
+      y = rounded_f32(y * (float)g[c][e]);
+      x[c][e] = y;
+      const float yh = (float)(half_t)y;
+      amax = __builtin_fmaxf(amax, __builtin_fabsf(yh));
+      if constexpr (FUSE_SUM) hs[e] = (float)(half_t)(hs[e] + yh);      // the reference adds these up in fp16
+    }
+  amax = wave_max64(amax);
+  if (lane == 0) r2[32 + wave] = amax;
+  if constexpr (FUSE_SUM) {
+    const float w = warp_sum(hs);
+    if ((lane & 15) == 0) r2[(vw & 15) * 2 + (vw >> 4)] = w;
+  }
+  lds_barrier();
+  amax = r2[32 + (lane & 7)];
+  amax = __builtin_fmaxf(amax, lane_xor1(amax));
+  amax = __builtin_fmaxf(amax, lane_xor2(amax));
+  amax = __builtin_fmaxf(amax, dpp_mov<0x141>(amax));             // the other half of 8 lanes, mirrored
+  if (p == 0) scale_out[row] = (half_t)(amax / 127.0f);
+  const float q = 127.0f / amax;
+  const RowArray codes(out + (size_t)row * H);
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    codes.put16(2 * p, 1024 * c,
+          (uint16_t)((uint32_t)(uint8_t)rni_sat_s8(x[c][0] * q) | ((uint32_t)(uint8_t)rni_sat_s8(x[c][1] * q) << 8)));
+  if constexpr (FUSE_SUM) {
+    const float tot = row16_sum(r2[(lane & 15) * 2] + r2[(lane & 15) * 2 + 1]);
+    if (p == 0) sum_out[row] = (half_t)tot;
+  }
+}
+
+template <bool FUSE_SUM, typename Src>
+static void launch_pairs(const NormOut& o, const Src& src, int tokens, int hidden, const PrefetchArgs& pf, hipStream_t st) {
+  const dim3 grid(tokens + pf.blocks), block(512);
+  switch (hidden >> 10) {
+#define OMNI_NORM_PAIRS(C_) \
+  case C_: hipLaunchKernelGGL((norm_pairs_kernel<C_, FUSE_SUM, Src>), grid, block, 0, st, o.out, src, o.gamma, o.sum, o.scale, o.eps, pf); break
+    OMNI_NORM_PAIRS(1);
+    OMNI_NORM_PAIRS(2);
+    OMNI_NORM_PAIRS(3);
+    OMNI_NORM_PAIRS(4);
+    OMNI_NORM_PAIRS(5);
+    OMNI_NORM_PAIRS(6);
+    OMNI_NORM_PAIRS(7);
+    OMNI_NORM_PAIRS(8);
+#undef OMNI_NORM_PAIRS
+  }
+}
+template <typename Src>
+static void launch_pairs(const NormOut& o, const Src& src, int tokens, int hidden, const PrefetchArgs& pf, hipStream_t st) {
+  if (o.sum) launch_pairs<true>(o, src, tokens, hidden, pf, st);
+  else launch_pairs<false>(o, src, tokens, hidden, pf, st);
+}
+
+void norm_pairs_slabs(const NormOut& o, const NormSlabs& s, int tokens, int hidden, const PrefetchArgs& pf, hipStream_t st) {
+  if (s.wsz) launch_pairs<true>(o, PairSlabs<true>{s}, tokens, hidden, pf, st);
+  else launch_pairs(o, PairSlabs<false>{s}, tokens, hidden, pf, st);
+}
+void norm_pairs_add(const NormOut& o, half_t* res, const half_t* delta, int tokens, int hidden, const PrefetchArgs& pf, hipStream_t st) {
+  launch_pairs(o, PairAdd{res, delta}, tokens, hidden, pf, st);
+}
+void norm_pairs_plain(const NormOut& o, const half_t* in, int tokens, int hidden, const PrefetchArgs& pf, hipStream_t st) {
+  launch_pairs(o, PairPlain{in}, tokens, hidden, pf, st);
+}
+
+}  // namespace omni

@@ -77,10 +77,9 @@ class LServeDecodeRunner:
         # L2 weight prefetch riding on the row kernels (see omniserve_amd/runtime.py; a hint, results unaffected)
         prefetch_default = prefetch_mb is None
         if prefetch_mb is None:
-            # round 2 (quantiser row kernels as carriers): 4-5 % SLOWER at batch 1 with W8A8 weights, so it was off; with the
-            # row-kernel-free layer (norms and the wide merge as the carriers) 24-64 MiB measure 1.5-2 % FASTER per step
-            # (3.11-3.13 -> 3.05-3.07 ms, tools/r03_call60/61.sh); 8-16 MiB are neutral
-            prefetch_mb = 32.0 if self.fused else 0.0
+            # a norm's own chain at batch 1 takes as long as fetching 16 MiB: four steps at 100 000 tokens 2.03 ms, 2.04 with 32 MiB, 2.085 with 60
+            # (with the quantiser row kernels as carriers the prefetch is 4-5 % slower at batch 1: off there, see below)
+            prefetch_mb = 16.0 if self.fused else 0.0
         self.prefetch_bytes = int(float(prefetch_mb) * (1 << 20)) if self.fused else 0
         self.prefetch_blocks = int(prefetch_blocks)
         # (the wide merge as a carrier for o_proj's 16.8 MB costs it 2.8 us where o_proj gains 1.1: 3.07 -> 3.05 ms without)

@@ -192,16 +192,16 @@ class DecodeRunner:
                       fused_ext.norm_gemm_fused_ok(batch, (self.hl + 2 * self.kl) * cfg.head_dim, cfg.hidden, cfg.group_size, False) and
                       fused_ext.norm_gemm_fused_ok(batch, 2 * self.il, cfg.hidden, cfg.group_size, True))
         if prefetch_mb is None:
-            # measured (profiles/r02_*): +6-7 % at bs = 16 with 28-40 MiB per row kernel (the L2s hold 32 MiB; the
-            # excess lands in MALL), nothing at bs = 128, -4 % at bs = 64 where the row kernels are no longer idle
+            # A row kernel lasts as long as what it fetches where that is more than its rows' own chain: 16 MiB take the 6 us that a norm of
+            # 4096 channels takes, down_proj's 29.6 MB made it 8.  Step of 8 layers, 40 -> 16 MiB (14 and 18 the same, 24 and 12 1 % slower), us: 1 sequence
+            # 485 -> 474, 16 545 -> 536, 28 700 -> 673, 9 g128 643 -> 627, 6 of the 70B shape 643 -> 628.
             # (batch 33..64: 12 MiB per carrier measured best at configs[2] -- 3.50 -> 3.43 ms per step, 24 MiB and more lose.
             #  A tensor-parallel shard's projections are small enough to be fetched whole: one Llama-2-70B TP = 8 rank at
-            #  bs = 128 7.22-7.26 -> 6.59-6.65 ms per step with 12 .. 48 MiB.  Other batches > 64: not measured, off)
-            dflt = 40.0 if batch <= 32 else (12.0 if batch <= 64 else (24.0 if self.tp_size > 1 else 0.0))
+            #  bs = 128 7.22-7.26 -> 6.59-6.65 ms per step with 12 .. 48 MiB.  Other batches > 64: nothing gained, off)
+            dflt = 16.0 if batch <= 32 else (12.0 if batch <= 64 else (24.0 if self.tp_size > 1 else 0.0))
             prefetch_mb = dflt if self.fused else 0.0
         self.prefetch_bytes = int(float(prefetch_mb) * (1 << 20)) if self.fused else 0
-        # (fetching workgroups per carrier: 240 was round 2's optimum; with down_proj's 29.6 MB on the norm in front of gate_up
-        #  128-192 measure 1.7 % faster per step at bs = 16 -- 2.28 -> 2.24 ms --, 64-96 slower; bs = 64 / TP / LServe: flat)
+        # (fetching workgroups per carrier: 128, 224 and 320 measure up to 2 % slower per step at 1, 16, 28 and 61 sequences; TP / LServe: flat)
         self.prefetch_blocks = int(prefetch_blocks)
         self.weight_policy = int(weight_policy) if self.prefetch_bytes > 0 else 0
         c = cfg
@@ -289,10 +289,10 @@ class DecodeRunner:
         self.ngf_err = torch.zeros((4,), dtype=torch.int32, device=device)      # sticky: a hand-off wait gave up (check())
         self.tickets = fused_ext.new_tickets(device)      # ticket words of the single-launch attention (this runner's stream)
         self.ngf_clk = {}     # timeline probe (tools/pairs_ab.py): {(layer, site): int64 [grid, 8]} handed to that launch
-        # level 3: the norm in front of gate_up prefetches ALL of DOWN's weights (29.6 MB fit the 32 MB of L2s) instead of
+        # level 3: the norm in front of gate_up prefetches DOWN's weights (as much of them as the budget holds) instead of
         # the head of gate_up's 58.7 MB; gate_up then streams cold with non-temporal loads (they do not displace the
         # prefetched lines) and down reads L2: 2.322-2.334 -> 2.294-2.314 ms per step on the same box (profiles/r03_g;
-        # l3_prefetch_down=0: round 3's first arrangement, 2: gate_up with plain loads -- slower, 2.35)
+        # l3_prefetch_down=0: the head of gate_up's, 2: gate_up with plain loads -- slower, 2.35)
         self.pf_down = int(l3_prefetch_down)
         # fused level >= 2: the qkv projection leaves int32 split-K slabs and the decode attention applies its epilogue in
         # its first load trip (fused_ext.decode_arm_qkv_slabs): no slab epilogue launch between the two.  "auto": on exactly

@@ -381,3 +381,65 @@ def test_decode_step_begin_is_three_torch_ops():
     torch.cuda.synchronize()
     assert torch.isnan(out[3].float()).all() and torch.equal(out[4], table[idx[4]])
     assert torch.equal(lengths.cpu(), torch.arange(101, 117, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("hidden,sk", [(1024, 1), (2048, 2), (3072, 3), (4096, 4), (5120, 5), (6144, 6), (7168, 7), (8192, 8), (4096, 9), (4096, 16),
+                                       (2048, 17), (8192, 13), (8192, 11)])
+@pytest.mark.parametrize("zero_points", [True, False])
+def test_norm_of_slabs_in_whole_kilochannels(hidden, sk, zero_points):
+    """residual += epilogue(sum of sk slabs), norm, codes, scale, sum: every width and count of slabs that has a form of its own, and a count beyond"""
+    from omniserve_amd.backend import fused_ext
+    rng = np.random.default_rng(hidden + sk)
+    M = 3
+    slab = rng.integers(-40000, 40000, (sk, M, hidden), dtype=np.int32)
+    resid, g = _x(M, hidden, 6, 2.0), (1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float16)
+    sw, sz = rng.uniform(0.0005, 0.004, hidden).astype(np.float16), rng.uniform(0.0, 0.02, hidden).astype(np.float16)
+    sa, asum = rng.uniform(0.005, 0.02, M).astype(np.float16), rng.uniform(-40, 40, M).astype(np.float16)
+    f = np.float32
+    acc = slab.astype(np.int64).sum(0).astype(np.int32).astype(f)
+    if zero_points:
+        ep = ((acc * f(sw)) * f(sa)[:, None] - f(sz) * f(asum)[:, None]).astype(np.float16)
+    else:
+        ep = (acc * (f(sw) * f(sa)[:, None])).astype(np.float16)
+    xs = (f(resid) + f(ep)).astype(np.float16)
+    qo, so, smo = oe.rms_norm_general(xs, g, 1e-5, True)
+    slab_d, x, g_d, sw_d, sz_d, sa_d, as_d = map(to_dev, (slab, resid, g, sw, sz, sa, asum))
+    q = torch.empty((M, hidden), dtype=torch.int8, device=dev())
+    sc, sm = (torch.empty((M,), dtype=torch.float16, device=dev()) for _ in range(2))
+    if zero_points:
+        fused_ext.splitk_add_rms_norm_general_fuse_sum(q, x, slab_d, sk, sw_d, sa_d, sz_d, as_d, g_d, sm, sc, 1e-5)
+    else:
+        fused_ext.splitk_w8_add_rms_norm_general_fuse_sum(q, x, slab_d, sk, sw_d, sa_d, g_d, sm, sc, 1e-5)
+    torch.cuda.synchronize()
+    assert_f16_equal(x, xs, "residual")
+    assert np.array_equal(q.cpu().numpy(), qo)
+    assert_f16_equal(sc, so, "scale")
+    assert_f16_equal(sm, smo, "sum")
+
+
+@pytest.mark.parametrize("hidden", [1024, 7168, 8192, 9216])      # (9216: beyond the kernel's widths)
+@pytest.mark.parametrize("tokens", [2, 1023])
+def test_norm_in_whole_kilochannels(hidden, tokens):
+    """the plain and the adding form, with and without the row sum"""
+    import omniserve_backend.layernorm_ops as ln
+    from omniserve_amd.backend import fused_ext
+    x, d = _x(tokens, hidden, 1, 2.0), _x(tokens, hidden, 2, 1.0)
+    g = (1.0 + 0.1 * np.random.default_rng(3).standard_normal(hidden)).astype(np.float16)
+    xs = (x.astype(np.float32) + d.astype(np.float32)).astype(np.float16)
+    q = torch.empty((tokens, hidden), dtype=torch.int8, device=dev())
+    sc, sm = (torch.empty((tokens,), dtype=torch.float16, device=dev()) for _ in range(2))
+    for rows, add in ((x, None), (xs, d)):
+        for want_sum in (True, False):
+            r = to_dev(x)
+            qo, so, smo = oe.rms_norm_general(rows, g, 1e-5, want_sum)
+            if add is not None:
+                fused_ext.add_rms_norm_general_fuse_sum(q, r, to_dev(add), to_dev(g), sm if want_sum else None, sc, 1e-5)
+                assert_f16_equal(r, xs, "residual")
+            elif want_sum:
+                ln.rms_norm_general_fuse_sum(q, r, to_dev(g), sm, sc, 1e-5, True)
+            else:
+                ln.rms_norm_general(q, r, to_dev(g), sc, 1e-5, True)
+            assert np.array_equal(q.cpu().numpy(), qo)
+            assert_f16_equal(sc, so, "scale")
+            if want_sum:
+                assert_f16_equal(sm, smo, "sum")
