@@ -550,6 +550,19 @@ int omni_w4a8_per_group_norm_gemm_fused(void* codes_i8, void* residual_f16, cons
                                         void* amax_slots_u32, void* sync_u32, void* err_u32, int M, int N, int K, void* clk_u64,
                                         void* stream);
 
+/* Fused extension: residual_out = residual + h(epilogue(sum of sk split-K slabs)) (slab_i32 NULL: the residual as it is, nothing stored) ->
+ * rms_norm_general[_fuse_sum] -> the projection, for one or two rows of 2048, 3072 or 4096 channels, as ONE launch in which every workgroup forms the
+ * rows by itself (csrc/norm_product.hip).  Bit-identical to omni_splitk_[w8_]add_rms_norm_general_fuse_sum (omni_rms_norm_general[_fuse_sum]) and
+ * omni_w4a8_per_*_gemm / omni_w8a8_gemm, or with amax_slots_u32 (out = act [M, N/2]) omni_*_gemm_silu.  mode: 0 per-channel W4A8 (p_wszs, p_asums and
+ * w_szs required), 1 per-group W4A8 (zeros_i8, scales_i8 required), 2 W8A8; the projection before (p_*) has the same mode.  residual_out_f16 must
+ * be another buffer than residual_f16.  Replaces llama_w4a8_unpad.py:410-415,425-432 at these sizes.
+ * omni_norm_product_ok: 1 where the form exists; k_before: K of the omni_*_gemm_partial[_f16] whose slabs are consumed (0: none). */
+int omni_norm_product_ok(int M, int N, int K, int mode, int silu, int k_before);
+int omni_norm_product(int mode, const void* residual_f16, void* residual_out_f16, const void* slab_i32, int sk, const void* p_wscales_f16,
+                      const void* p_ascales_f16, const void* p_wszs_f16, const void* p_asums_f16, const void* gamma_f16, float eps,
+                      const void* weight, const void* zeros_i8, const void* scales_i8, const void* wscales_f16, const void* w_szs_f16,
+                      void* out_f16, int64_t out_row_stride, void* amax_slots_u32, int M, int N, int K, void* stream);
+
 /* Fused extension (round 4): omni_kv4_decode_attention_partial + omni_attn_merge_f16_amax as ONE launch.  Every split
  * workgroup writes its partial through, takes a ticket of its (sequence, head group), and the last arriver merges the splits
  * (the merge kernels' arithmetic), stores the fp16 [B, Hq * 128] output and raises the row maxima; an armed L2 prefetch rides

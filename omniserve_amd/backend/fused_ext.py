@@ -459,6 +459,37 @@ def select_topk_pages(out, scores, subs_per_page, total_pages, k):
     _lib.check(rc, "fused_ext.select_topk_pages")
 
 
+# ---- one or two rows: norm and product in one launch, every workgroup with the rows (csrc/norm_product.hip) ------------
+def norm_product_ok(M, N, K, mode, silu=False, k_before=0):
+    """True where norm_product exists.  mode: 0 W4A8 per-channel, 1 per-group, 2 W8A8; k_before: K of the projection whose slabs it
+    consumes (0: none)."""
+    return _lib.lib().omni_norm_product_ok(int(M), int(N), int(K), int(mode), int(bool(silu)), int(k_before)) == 1
+
+
+def norm_product(residual, gamma, epsilon, lin, out, residual_out=None, slab=None, sk=0, producer=None, p_ascales=None, p_asums=None,
+                 amax=None):
+    """residual_out = residual + epilogue(sum of `sk` slabs of `producer`) (no slab: the residual as it is), rms_norm_general[_fuse_sum] of it,
+    out = lin(codes) (amax given: out = silu_and_mul(lin(codes)) [M, N/2], row maxima raised): one launch, the bits of the two or three calls.
+    `lin` / `producer`: W4A8 (qweight, s1_scales, s1_szeros or s2_zeros / s2_scales) or W8A8 layers (weight, dequant_scale) of one kind."""
+    _lib.require_cuda(residual, gamma, out, residual_out, slab, p_ascales, p_asums, amax)
+    M, K = residual.shape
+    if hasattr(lin, "dequant_scale"):
+        mode, w, scale, zero, s2z, s2s = 2, lin.weight, lin.dequant_scale, None, None, None
+    elif lin.group == -1:
+        mode, w, scale, zero, s2z, s2s = 0, lin.qweight, lin.s1_scales, lin.s1_szeros, None, None
+    else:
+        mode, w, scale, zero, s2z, s2s = 1, lin.qweight, lin.s1_scales, None, lin.s2_zeros, lin.s2_scales
+    p_scale = p_zero = None
+    if slab is not None:
+        p_scale = producer.dequant_scale if mode == 2 else producer.s1_scales
+        p_zero = producer.s1_szeros if mode == 0 else None
+    rc = _lib.lib().omni_norm_product(
+        mode, residual.data_ptr(), _ptr(residual_out), _ptr(slab), int(sk), _ptr(p_scale), _ptr(p_ascales), _ptr(p_zero),
+        _ptr(p_asums) if mode == 0 else None, gamma.data_ptr(), float(epsilon), w.data_ptr(), _ptr(s2z), _ptr(s2s), scale.data_ptr(),
+        _ptr(zero), out.data_ptr(), out.stride(0), _ptr(amax), M, w.shape[0], K, _lib.current_stream())
+    _lib.check(rc, "fused_ext.norm_product")
+
+
 # ---- round 6: (norm -> GEMV) pairs as one launch (csrc/norm_gemv_fused.h) -------------------------------------------
 NGF_SYNC_WORDS = 32     # per call site: arrival counter + the rows' {scale, sum} pairs; zeroed by the caller before every launch
 

@@ -1,0 +1,309 @@
+// residual += the product before, norm, quantisation and the next product as ONE launch, for one or two rows: the decode layer's two edges
+// input_layernorm -> qkv_proj and post_attention_layernorm -> gate_up_proj (+ silu_and_mul) (reference: llama_w4a8_unpad.py:410-432).
+//
+// As two launches (norm_rows.hip, then the GEMV) one compute unit works through the row for 6 us while the others wait, and only then are the product's
+// first weights requested.  Handing the row over inside a launch costs what the boundary between two does (norm_gemv_fused.h).  But a row or two
+// are little enough for EVERY workgroup of the product to form by itself: 50 - 200 KiB of slabs out of its L2, requested in front of the first
+// weights, so that the whole chain -- requests, two reductions, codes -- passes while the weights are on their way, and nothing waits for
+// another workgroup.  Each row's codes, scale and sum are the bits that the two launches give (norm_pairs.h: the same additions in the same order).
+//
+//  * the product is row_product.h's.  gate_up: 32 gate channels and their 32 up channels a workgroup (twice as many, so that a compute unit has one of
+//    224 workgroups and the others fetch down_proj's weights: the same 14 us, and down gains what this loses).
+//  * qkv: 32 channels a workgroup, so that 6144 channels make 192 workgroups instead of 96.
+//  * the new residual goes to a buffer of its own (workgroup 0 stores it): other workgroups still read the old one.
+//
+// MI355X, 8B model, us a layer, two launches -> one: W4A8 1 row qkv 6.5 + 5.5 -> 7.7, gate_up 6.5 + 12.0 -> 13.7 (down_proj, whose weights the norm
+// no longer fetches, 6.8 -> 8.7); the step of 8 layers 472 -> 419 us, 2 rows 511 -> 490; with groups of 128 604 -> 500 and 620 -> 557.  W8A8 1
+// row: gate_up 6.5 + 24.5 -> 27.3; four LServe steps of 4 layers 2037 -> 1818.  Two rows
+// gain little enough that more are left to the two launches.
+#include "row_product.h"
+
+namespace omni {
+
+struct NormProductArgs {
+  const half_t* res;
+  half_t* res_out;          // with slabs
+  const int32_t* slab;      // [sk][M][K]
+  int sk;
+  const half_t *p_wscales, *p_wsz, *p_ascales, *p_asum;
+  const half_t* gamma;
+  float eps;
+  const uint8_t *W, *s2s, *s2z;
+  const half_t *wscales, *wsz;
+  half_t* out;
+  uint32_t* amax;
+  long long out_stride;
+  int M, N;
+};
+
+// C: K / 1024.  SK: slabs whose requests go out together (those beyond sk read slab 0 again); 0: the residual as it is.  ROWS: M.
+template <int MODE, int EPI, int BLOCKS, int C, int SK, int ROWS>
+__global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(NormProductArgs p) {
+  constexpr bool ZP = MODE == MODE_CHN, W8 = MODE == MODE_W8;
+  constexpr int K = 1024 * C, KPART = K / RP_WAVES;
+  // units requested in front of the rows' first wait, and (the slabs' registers are free then) all that fly together
+  constexpr bool WIDE = ROWS * SK * C > 16;
+  constexpr int FIRST_MAX = W8 ? (EPI ? 1 : 2) : EPI && WIDE ? 3 : 4, RING_MAX = W8 ? 2 : FIRST_MAX;
+  typedef RowProduct<MODE, EPI ? LAYOUT_GATE : LAYOUT_ROWS32, BLOCKS, KPART, RING_MAX, ROWS> Product;
+  constexpr int FIRST = FIRST_MAX < Product::RING ? FIRST_MAX : Product::RING;
+  constexpr int PITCH = K + 64;
+  constexpr int LDS_PARTS = ROWS * PITCH, LDS_RED = LDS_PARTS + Product::PART_BYTES, LDS_ALL = LDS_RED + ROWS * 512;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_ALL];
+  uint8_t* const codes = lds;
+  uint8_t* const parts = lds + LDS_PARTS;
+  float (*red)[128] = reinterpret_cast<float (*)[128]>(lds + LDS_RED);
+  asm volatile("" ::"s"(p.res), "s"(p.slab), "s"(p.sk), "s"(p.p_wscales), "s"(p.p_wsz), "s"(p.p_ascales), "s"(p.p_asum), "s"(p.gamma), "s"(p.W),
+               "s"(p.wscales), "s"(p.wsz), "s"(p.N));
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ng = blockIdx.x;
+  const uint32_t at = 4 * tid;
+
+  // ---- requests: the rows ----
+  v2h g[C], a[ROWS][C], sw[C], sz[C];
+  v2i t[ROWS][SK ? SK : 1][C];
+  half_t sa_h[ROWS], as_h[ROWS];
+  {
+    const RowArray gains(p.gamma), ws(p.p_wscales), wz(p.p_wsz);
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) {
+      if constexpr (SK > 0) {
+        const RowArray slab(p.slab + (size_t)m * K);
+        const uint32_t step = ROWS * K * 4;
+#pragma unroll
+        for (int k = 0; k < SK; ++k)
+#pragma unroll
+          for (int c = 0; c < C; ++c) t[m][k][c] = slab.two(2 * at, (k < p.sk ? k * step : 0) + 4096 * c);
+        sa_h[m] = p.p_ascales[m];
+        if constexpr (ZP) as_h[m] = p.p_asum[m];
+      }
+      const RowArray res(p.res + (size_t)m * K);
+#pragma unroll
+      for (int c = 0; c < C; ++c) a[m][c] = res.pair(at, 2048 * c);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if constexpr (SK > 0) {
+        sw[c] = ws.pair(at, 2048 * c);
+        if constexpr (ZP) sz[c] = wz.pair(at, 2048 * c);
+      }
+      g[c] = gains.pair(at, 2048 * c);
+    }
+  }
+  // ---- ... the scales of the channel that this lane finishes ----
+  int chan;
+  if constexpr (EPI) chan = ((lane >> 3) & 1) * (p.N / 2) + ng * 32 + (lane >> 4) * 8 + (lane & 7);
+  else chan = ng * 32 + (lane & 31);
+  const half_t sw_own = p.wscales[chan];
+  half_t sz_own = (half_t)0.0f;
+  if constexpr (ZP) sz_own = p.wsz[chan];
+  // ---- ... and the weights ----
+  Product product;
+  product.open(p.W, p.s2s, p.s2z, p.N, K, ng * BLOCKS, wave * KPART);
+  __builtin_amdgcn_sched_barrier(0);      // what the rows need returns first: loads return in order
+#pragma unroll
+  for (int u = 0; u < FIRST; ++u) product.request(u);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the rows (norm_rows.hip, step by step) ----
+  float x[ROWS][C][2];
+  v2h o[ROWS][C];
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      o[m][c] = a[m][c];
+      if constexpr (SK > 0) {
+        v2i acc = t[m][0][c];
+#pragma unroll
+        for (int k = 1; k < SK; ++k) acc += k < p.sk ? t[m][k][c] : (v2i){0, 0};
+        const float sa = (float)sa_h[m];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          half_t ep;
+          if constexpr (ZP) ep = epilogue<MODE_CHN>(acc[e], (float)sw[c][e], sa, (float)sz[c][e], (float)as_h[m]);
+          else ep = epilogue<MODE_W8>(acc[e], (float)sw[c][e], sa, 0.0f, 0.0f);
+          o[m][c][e] = (half_t)((float)a[m][c][e] + (float)ep);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) x[m][c][e] = (float)o[m][c][e];
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = FIRST; u < Product::RING; ++u) product.request(u);
+  __builtin_amdgcn_sched_barrier(0);
+  const int vw = 4 * wave + (lane >> 4);
+  auto warp_sum = [&](float v0, float v1) { return row16_sum(v0) + row16_sum(v1); };
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    float s[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        s[0][e] = s[0][e] + x[m][c][e];
+        s[1][e] = s[1][e] + x[m][c][e] * x[m][c][e];
+      }
+    const float w0 = warp_sum(s[0][0], s[0][1]), w1 = warp_sum(s[1][0], s[1][1]);
+    if ((lane & 15) == 0) {
+      red[m][(vw & 15) * 4 + (vw >> 4)] = w0;
+      red[m][(vw & 15) * 4 + 2 + (vw >> 4)] = w1;
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    const v4f q4 = *reinterpret_cast<const v4f*>(&red[m][(lane & 15) * 4]);
+    const float mean = row16_sum(q4[0] + q4[1]) / (float)K;
+    const float rstd = 1.0f / __builtin_sqrtf(row16_sum(q4[2] + q4[3]) / (float)K + p.eps);
+    float amax = (float)(half_t)1e-6f, hs[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float y = (x[m][c][e] - mean) * rstd;
+        y = rounded_f32(y * (float)g[c][e]);
+        x[m][c][e] = y;
+        const float yh = (float)(half_t)y;
+        amax = __builtin_fmaxf(amax, __builtin_fabsf(yh));
+        if constexpr (ZP) hs[e] = (float)(half_t)(hs[e] + yh);
+      }
+    amax = wave_max64(amax);
+    if (lane == 0) red[m][96 + wave] = amax;
+    if constexpr (ZP) {
+      const float w = warp_sum(hs[0], hs[1]);
+      if ((lane & 15) == 0) red[m][64 + (vw & 15) * 2 + (vw >> 4)] = w;
+    }
+  }
+  lds_barrier();
+  float row_scale[ROWS], row_sum[ROWS];
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    float amax = red[m][96 + (lane & 7)];
+    amax = __builtin_fmaxf(amax, lane_xor1(amax));
+    amax = __builtin_fmaxf(amax, lane_xor2(amax));
+    amax = __builtin_fmaxf(amax, dpp_mov<0x141>(amax));
+    row_scale[m] = (float)(half_t)(amax / 127.0f);
+    row_sum[m] = 0.0f;
+    if constexpr (ZP) row_sum[m] = (float)(half_t)row16_sum(red[m][64 + (lane & 15) * 2] + red[m][64 + (lane & 15) * 2 + 1]);
+    const float q = 127.0f / amax;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const uint32_t two = (uint32_t)(uint8_t)rni_sat_s8(x[m][c][0] * q) | ((uint32_t)(uint8_t)rni_sat_s8(x[m][c][1] * q) << 8);
+      *reinterpret_cast<uint16_t*>(codes + m * PITCH + code_place<MODE>(1024 * c + 2 * tid)) = (uint16_t)two;
+    }
+  }
+  lds_barrier();
+
+  product.multiply(codes + wave * KPART, PITCH);
+  product.leave(parts, wave);
+  lds_barrier();
+  if (wave < ROWS) {      // (a wave finishes a row, a lane a channel)
+    const int m = wave;
+    float scale = row_scale[0], sum = row_sum[0];
+#pragma unroll
+    for (int i = 1; i < ROWS; ++i)
+      if (m == i) {
+        scale = row_scale[i];
+        sum = row_sum[i];
+      }
+    int total;
+    if constexpr (EPI) total = Product::total(parts, lane >> 4, lane & 15, m);
+    else if constexpr (W8) total = Product::total(parts, (lane >> 4) & 1, lane & 15, m);
+    else total = Product::total(parts, (lane >> 3) & 3, (lane & 7) + 8 * (lane >> 5), 2 * m + (lane >> 5));
+    if constexpr (Product::PAIRED) total += __shfl_xor(total, 32, 64);
+    const half_t h = epilogue<MODE == MODE_GRP ? MODE_W8 : MODE>(total, (float)sw_own, scale, (float)sz_own, sum);
+    half_t* const out = p.out + (size_t)m * p.out_stride;
+    if constexpr (EPI) {
+      const int up = __shfl_xor((int)__builtin_bit_cast(uint16_t, h), 8, 64);
+      const half_t act = silu_mul_h(h, __builtin_bit_cast(half_t, (uint16_t)up));      // (of lanes with a gate channel)
+      const bool gate = !(lane & 8);
+      if (gate) out[chan] = act;
+      const float top = wave_max64(gate ? __builtin_fabsf((float)act) : 0.0f);
+      if (lane == 0) amax_raise(p.amax, m, ng >> 3, top);
+    } else if (lane < 32) {
+      out[chan] = h;
+    }
+  }
+  if constexpr (SK > 0) {
+    if (blockIdx.x == 0) {
+#pragma unroll
+      for (int m = 0; m < ROWS; ++m)
+#pragma unroll
+        for (int c = 0; c < C; ++c) RowArray(p.res_out + (size_t)m * K).put(at, 2048 * c, o[m][c]);
+    }
+  }
+}
+
+}  // namespace omni
+using namespace omni;
+
+namespace {
+
+template <int MODE, int EPI, int BLOCKS, int C, int SK>
+void launch_rows(const NormProductArgs& p, hipStream_t st) {
+  const dim3 grid(EPI ? p.N / 64 : p.N / 32), block(RP_THREADS);
+  if constexpr (MODE != MODE_W8 && SK <= 8) {      // (two rows with int8 weights, or of 16 slabs, do not fit the registers)
+    if (p.M == 2) {
+      hipLaunchKernelGGL((norm_product_kernel<MODE, EPI, BLOCKS, C, SK, 2>), grid, block, 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((norm_product_kernel<MODE, EPI, BLOCKS, C, SK, 1>), grid, block, 0, st, p);
+}
+template <int MODE, int C>
+void launch_slabs(const NormProductArgs& p, hipStream_t st) {
+  constexpr int CHANNELS32 = MODE == MODE_W8 ? 2 : 4;
+  if (p.amax) {
+    if (p.sk <= 2) launch_rows<MODE, 1, 4, C, 2>(p, st);
+    else launch_rows<MODE, 1, 4, C, 4>(p, st);
+  } else if (!p.slab) {
+    launch_rows<MODE, 0, CHANNELS32, C, 0>(p, st);
+  } else if (p.sk <= 8) {
+    launch_rows<MODE, 0, CHANNELS32, C, 8>(p, st);
+  } else {
+    launch_rows<MODE, 0, CHANNELS32, C, 16>(p, st);
+  }
+}
+template <int MODE>
+int launch(const NormProductArgs& p, int K, hipStream_t st) {
+  switch (K >> 10) {
+    case 2: launch_slabs<MODE, 2>(p, st); break;
+    case 3: launch_slabs<MODE, 3>(p, st); break;
+    default: launch_slabs<MODE, 4>(p, st); break;
+  }
+  return omni_launch_status();
+}
+
+}  // namespace
+
+static bool sizes_ok(int M, int N, int K, int mode, bool silu, int sk) {
+  if (mode < 0 || mode > 2 || M < 1 || M > (mode == MODE_W8 ? 1 : 2) || K % 1024 || K < 2048 || K > 4096 || N < 64 || N % (silu ? 128 : 64)) return false;
+  return silu ? sk >= 1 && sk <= 4 : sk >= 0 && sk <= (M == 1 ? 16 : 8);
+}
+
+extern "C" int omni_norm_product_ok(int M, int N, int K, int mode, int silu, int k_before) {
+  if (!sizes_ok(M, N, K, mode, silu != 0, 1)) return 0;
+  const int kalign = mode == MODE_GRP ? 128 : 64;
+  if (k_before == 0) return !silu;
+  if (k_before < kalign || k_before % kalign) return 0;
+  return sizes_ok(M, N, K, mode, silu != 0, plan_gemm(M, K, k_before, kalign, true, mode == MODE_W8).sk);
+}
+
+extern "C" int omni_norm_product(int mode, const void* residual_f16, void* residual_out_f16, const void* slab_i32, int sk, const void* p_wscales_f16,
+                                 const void* p_ascales_f16, const void* p_wszs_f16, const void* p_asums_f16, const void* gamma_f16, float eps,
+                                 const void* weight, const void* zeros_i8, const void* scales_i8, const void* wscales_f16, const void* w_szs_f16,
+                                 void* out_f16, int64_t out_row_stride, void* amax_slots_u32, int M, int N, int K, void* stream) {
+  if (!residual_f16 || !gamma_f16 || !weight || !wscales_f16 || !out_f16 || !sizes_ok(M, N, K, mode, amax_slots_u32 != nullptr, slab_i32 ? sk : 0))
+    return OMNI_EINVAL;
+  if (mode == MODE_CHN && !w_szs_f16) return OMNI_EINVAL;
+  if (mode == MODE_GRP && (!zeros_i8 || !scales_i8)) return OMNI_EINVAL;
+  if (slab_i32 && (sk < 1 || !p_wscales_f16 || !p_ascales_f16 || !residual_out_f16 || residual_out_f16 == residual_f16)) return OMNI_EINVAL;
+  if (slab_i32 && mode == MODE_CHN && (!p_wszs_f16 || !p_asums_f16)) return OMNI_EINVAL;
+  const NormProductArgs p{(const half_t*)residual_f16, (half_t*)residual_out_f16, (const int32_t*)slab_i32, sk, (const half_t*)p_wscales_f16,
+                          (const half_t*)p_wszs_f16, (const half_t*)p_ascales_f16, (const half_t*)p_asums_f16, (const half_t*)gamma_f16, eps,
+                          (const uint8_t*)weight, (const uint8_t*)scales_i8, (const uint8_t*)zeros_i8, (const half_t*)wscales_f16,
+                          (const half_t*)w_szs_f16, (half_t*)out_f16, (uint32_t*)amax_slots_u32, out_row_stride, M, N};
+  hipStream_t st = (hipStream_t)stream;
+  if (mode == MODE_CHN) return launch<MODE_CHN>(p, K, st);
+  return mode == MODE_GRP ? launch<MODE_GRP>(p, K, st) : launch<MODE_W8>(p, K, st);
+}

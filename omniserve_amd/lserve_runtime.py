@@ -63,12 +63,12 @@ class LServeDecodeRunner:
     def __init__(self, cfg: LlamaConfig, batch: int, context: int, max_new: int, device, seed=0, kv_format="kv8",
                  streaming_ratio=0.5, sink=128, local=256, budget_tokens=4096, selector_interval=4,
                  sub_chunk_per_block=4, use_graph=True, fused=True, prefetch_mb=None, ctx_sink=128, ctx_local=8192,
-                 prefetch_blocks=160, arm_o=False, defer=True, qkv_slabs=True, rowfree=True):
+                 prefetch_blocks=160, arm_o=False, defer=True, qkv_slabs=True, rowfree=True, own_rows=True):
         """fused: use the opt-in fused entry points (residual add + norm + quant, silu*mul + quant) -- bit-identical to the
         reference call sequence, three launches fewer per layer.  fused=True (or 3) also takes the
         row-kernel-free forms where they apply (batch <= 16: the attention merge leaves fp16 + row maxima, gate_up runs
         with the SiLU*mul epilogue, o_proj / down_proj quantise on the fly -- runtime.py's fusion level 3 for the W8A8
-        layers); fused=2 keeps the quantiser row kernels.  prefetch_mb / prefetch_blocks / arm_o / defer / qkv_slabs / rowfree: the
+        layers); fused=2 keeps the quantiser row kernels.  prefetch_mb / prefetch_blocks / arm_o / defer / qkv_slabs / rowfree / own_rows: the
         A/B switches of the step (this module reads no environment)."""
         c = cfg
         self.cfg, self.B, self.device = cfg, batch, device
@@ -190,6 +190,10 @@ class LServeDecodeRunner:
         if self.rowfree:
             self.attn_f16 = torch.empty((B, Hq * d), dtype=f16, device=device)
             self.amax = torch.zeros((c.layers, 2, fused_ext.AMAX_WORDS), dtype=torch.int32, device=device)
+        # one or two rows: each norm and the product behind it are one launch, which leaves the new residual in the other of two buffers
+        self.own_rows = (self.rowfree and bool(own_rows) and fused_ext.norm_product_ok(B, qkv_n, c.hidden, 2, False, c.inter) and
+                         fused_ext.norm_product_ok(B, 2 * c.inter, c.hidden, 2, True, Hq * d))
+        self._x2 = torch.empty_like(self.x) if self.own_rows else None
         self.qkv_buf = torch.empty((B, qkv_n), dtype=f16, device=device)
         self.proj_buf = torch.empty((B, c.hidden), dtype=f16, device=device)
         self.gate_up_buf = torch.empty((B, 2 * c.inter), dtype=f16, device=device)
@@ -225,8 +229,11 @@ class LServeDecodeRunner:
         `self.lengths`; `hist` only sizes RoPE tables, split plans and the selector's padded output)."""
         c, B = self.cfg, self.B
         Hq, Hk, d = c.heads, c.kv_heads, c.head_dim
+        own, x, spare = self.own_rows, self.x, self._x2
+        if own:
+            x, spare = spare, x      # (an odd number of changes: the last residual is in self.x)
         if self.fused:     # embedding rows + lengths += 1 + the step's row-maximum slots zeroed: one launch
-            fused_ext.decode_step_begin(self.x, self.embed, self.tokens, self.lengths, self.amax if self.rowfree else None)
+            fused_ext.decode_step_begin(x, self.embed, self.tokens, self.lengths, self.amax if self.rowfree else None)
         else:
             self.lengths.add_(1)
             torch.index_select(self.embed, 0, self.tokens, out=self.x)
@@ -240,8 +247,14 @@ class LServeDecodeRunner:
         sm = None          # W8A8: nobody reads a row sum (rms_norm_general / invoke_quant upstream): the fused kernels skip it
         rowfree = self.rowfree
         for li, L in enumerate(self.layers):
-            self._arm(L["qkv"])
-            if pending is not None:       # residual += down_proj(previous layer) [deferred epilogue], norm + quant
+            if not own:
+                self._arm(L["qkv"])
+            if own and pending is not None:
+                fused_ext.norm_product(x, L["ln1"], c.eps, L["qkv"], self.qkv_buf, spare, self.slab, pending[0], pending[1], sq)
+                x, spare, pending = spare, x, None
+            elif own:
+                fused_ext.norm_product(x, L["ln1"], c.eps, L["qkv"], self.qkv_buf)
+            elif pending is not None:       # residual += down_proj(previous layer) [deferred epilogue], norm + quant
                 fused_ext.splitk_w8_add_rms_norm_general_fuse_sum(self.q_hidden, self.x, self.slab, pending[0],
                                                                   pending[1].dequant_scale, sq, L["ln1"], sm, sc, c.eps)
                 pending = None
@@ -249,7 +262,9 @@ class LServeDecodeRunner:
                 fused_ext.add_rms_norm_general_fuse_sum(self.q_hidden, self.x, self.proj_buf, L["ln1"], sm, sc, c.eps)
             else:
                 layernorm_ops.rms_norm_general(self.q_hidden, self.x, L["ln1"], sc, c.eps, True)
-            if self.qkv_slabs and not select:   # slabs only: the attention applies the projection's epilogue (the page
+            if own:
+                pass
+            elif self.qkv_slabs and not select:   # slabs only: the attention applies the projection's epilogue (the page
                 lin = L["qkv"]                  # selector of a refresh step reads fp16 q / k: regular GEMM there)
                 sk_q = fused_ext.gemm_partial_w8a8(self.q_hidden, lin.weight, self.slab)
                 fused_ext.decode_arm_qkv_slabs(self.slab, sk_q, B, lin.n, 0, Hq * d, (Hq + Hk) * d, lin.dequant_scale, sc)
@@ -309,6 +324,12 @@ class LServeDecodeRunner:
                 sk = fused_ext.gemm_partial_w8a8(self.q_attn, L["o"].weight, self.slab)
             else:
                 L["o"].forward(self.q_attn, sq, self.proj_buf)
+            if own:
+                fused_ext.norm_product(x, L["ln2"], c.eps, L["gate_up"], self.mlp_act, spare, self.slab, sk, L["o"], sq,
+                                       amax=self.amax[li, 1])
+                x, spare = spare, x
+                pending = (fused_ext.gemm_partial_f16_w8a8(self.mlp_act, self.amax[li, 1], L["down"].weight, self.slab, sq), L["down"])
+                continue
             if not (rowfree and li < nl - 1):     # (the SiLU-epilogue form pairs gate / up rows: no prefetch descriptor)
                 self._arm(L["gate_up"])
             # (letting that norm carry the head of down_proj's 58.7 MB instead measured slower: 3.09 -> 3.21 ms per step)
@@ -339,7 +360,11 @@ class LServeDecodeRunner:
                 L["down"].forward(self.q_inter, sq, self.proj_buf)
                 if not self.fused or li == nl - 1:
                     self.x.add_(self.proj_buf)
-        layernorm_ops.rms_norm(self.normed, self.x, self.final_norm, c.eps, False)
+        if pending is not None:     # the last layer's down projection: epilogue + residual add inside the final norm
+            fused_ext.splitk_add_rms_norm(self.normed, self.x, self.slab, pending[0], pending[1].dequant_scale, sq, None, None,
+                                          self.final_norm, c.eps)
+        else:
+            layernorm_ops.rms_norm(self.normed, self.x, self.final_norm, c.eps, False)
         logits = torch.matmul(self.normed, self.lm_head.t())
         fused_ext.argmax(self.tokens, logits)
 

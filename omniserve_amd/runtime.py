@@ -122,7 +122,8 @@ class DecodeRunner:
     def __init__(self, cfg: LlamaConfig, batch: int, context: int, max_new: int, device, seed=0,
                  use_graph=True, fused=True, tp_rank=0, tp_size=1, tp_group=None, shard_full=False,
                  prefetch_mb=None, prefetch_blocks=160, weight_policy=1, tp_comm=None, max_fused=4, tp_l2_attn=True,
-                 l3_prefetch_down=1, qkv_slabs="auto", attn_single=True, arm_qkv=True, arm_o=True, l3_last=True):
+                 l3_prefetch_down=1, qkv_slabs="auto", attn_single=True, arm_qkv=True, arm_o=True, l3_last=True,
+                 own_rows=True):
         """tp_size > 1: Megatron-style tensor parallelism (omniserve_amd/tp.py): qkv / gate_up column-parallel,
         o / down row-parallel, attention by kv head, one fp16 sum all-reduce of the [B, hidden] projection after
         o_proj and after down_proj.  shard_full=True builds the full layers from the seed and keeps this
@@ -130,7 +131,7 @@ class DecodeRunner:
         are drawn (bench: synthetic weights, no point in materialising 70B parameters per rank).
         The A/B switches of the decode step are constructor arguments (this module reads no environment): max_fused caps the
         fusion level the runner may pick; tp_l2_attn / qkv_slabs ("auto", True, False) / attn_single / arm_qkv / arm_o /
-        l3_prefetch_down (0, 1, 2) / l3_last select the forms described where they are used below."""
+        l3_prefetch_down (0, 1, 2) / l3_last / own_rows select the forms described where they are used below."""
         self.cfg, self.B, self.device = cfg, batch, device
         self.tp_rank, self.tp_size, self.tp_group = int(tp_rank), int(tp_size), tp_group
         # tp_comm = "peer": the decode step's collectives run on the library's own peer-mapped all-reduce (tp.PeerComm: one
@@ -317,6 +318,12 @@ class DecodeRunner:
         # level 3 also in the LAST layer: its down projection's slabs are consumed by the model's final norm
         # (fused_ext.splitk_add_rms_norm) instead of GEMV epilogue + residual add + rms_norm (l3_last=False: off, A/B)
         self.last_l3 = self.fused >= 3 and self.tp_size == 1 and self.comm is None and bool(l3_last)
+        # one or two rows: each norm and the product behind it are one launch, which leaves the new residual in the other of two buffers
+        mode = 0 if c.group_size == -1 else 1
+        self.own_rows = (self.last_l3 and not self.pairs and not self.qkv_slabs and bool(own_rows) and
+                         fused_ext.norm_product_ok(B, qkv_n, c.hidden, mode, False, il) and
+                         fused_ext.norm_product_ok(B, 2 * il, c.hidden, mode, True, hl * d))
+        self._x2 = torch.empty_like(self.x) if self.own_rows else None
         self.normed = torch.empty((B, c.hidden), dtype=f16, device=device)
         self.lengths = torch.full((B,), context, dtype=torch.int32, device=device)
         self.tokens = torch.randint(0, c.vocab, (B,), device=device, generator=gen)
@@ -433,12 +440,16 @@ class DecodeRunner:
     def _eager_step_body(self):
         # one decoder layer at decode shape = llama_w4a8_unpad.py:406-438
         c = self.cfg
+        nl = len(self.layers)
+        own, x, spare = self.own_rows, self.x, self._x2
+        if own:
+            x, spare = spare, x      # (an odd number of changes: the last residual is in self.x)
         if self.fused:     # one launch: embedding rows (torch's index_select takes 12.6 us for 16 rows) + lengths += 1 + the
-            fused_ext.decode_step_begin(self.x, self.embed, self.tokens, self.lengths,      # step's row-maximum slots zeroed
+            fused_ext.decode_step_begin(x, self.embed, self.tokens, self.lengths,      # step's row-maximum slots zeroed
                                         self._step_words if self.fused >= 3 else None)
         else:
             self.lengths.add_(1)
-            torch.index_select(self.embed, 0, self.tokens, out=self.x)
+            torch.index_select(self.embed, 0, self.tokens, out=x)
         B = self.B
         hq, hk, d = self.hl, self.kl, c.head_dim     # this rank's heads
         sA, mA = self.act_scale2, self.act_sum2   # scales / sums produced by quant-type kernels
@@ -447,7 +458,6 @@ class DecodeRunner:
         if not per_chn:    # g128: no activation sums anywhere (llama_w4a8_unpad.py:81,212-215,395-401): the reference calls
             mA = mB = None # rms_norm_general / invoke_quant, and the fused entry points skip the second row reduction
         pending = None                             # (sk, linear) of a down_proj whose epilogue is deferred
-        nl = len(self.layers)
         for li, L in enumerate(self.layers):
             qa_h, qa_i = self._q_hidden, self._q_inter
             l3 = self.fused >= 3 and (li < nl - 1 or self.last_l3)     # row-kernel-free MLP half in this layer
@@ -463,9 +473,16 @@ class DecodeRunner:
                 else:
                     fused_ext.norm_gemm_fused(qa_h, self.x, L["ln1"], mB, sB, c.eps, L["qkv"], self.qkv_buf, self.ngf_sync[li, 0],
                                               self.ngf_err)
+            elif own:
+                if pending is not None:
+                    sk, lin = pending
+                    fused_ext.norm_product(x, L["ln1"], c.eps, L["qkv"], self.qkv_buf, spare, self.slab, sk, lin, sA, mA)
+                    x, spare, pending = spare, x, None
+                else:
+                    fused_ext.norm_product(x, L["ln1"], c.eps, L["qkv"], self.qkv_buf)
             elif self.arm_qkv:
                 self._arm(L["qkv"], deferred=self.qkv_slabs)
-            if self.pairs and l3:
+            if own or self.pairs and l3:
                 pass
             elif pending is not None:     # residual += down_proj(prev layer) [deferred epilogue], norm + quant
                 sk, lin = pending
@@ -479,7 +496,7 @@ class DecodeRunner:
                 layernorm_ops.rms_norm_general_fuse_sum(qa_h, self.x, L["ln1"], mB, sB, c.eps, True)
             else:
                 layernorm_ops.rms_norm_general(qa_h, self.x, L["ln1"], sB, c.eps, True)
-            if self.pairs and l3:
+            if own or self.pairs and l3:
                 pass
             elif self.qkv_slabs:      # slabs only; the attention kernel reads q / k / v from them (qkv_buf: shapes only)
                 lin = L["qkv"]
@@ -519,6 +536,12 @@ class DecodeRunner:
                     fused_ext.norm_gemm_fused(qa_h, self.x, L["ln2"], mB, sB, c.eps, G, self.mlp_act, self.ngf_sync[li, 1],
                                               self.ngf_err, slab=self.slab, sk=sk, producer=L["o"], p_ascales=sA, p_asums=mA,
                                               amax=self.amax[li, 1], clk=self.ngf_clk.get((li, 1)))
+                    pending = (self._partial_f16(self.mlp_act, self.amax[li, 1], L["down"], mA, sA), L["down"])
+                    continue
+                if own:
+                    fused_ext.norm_product(x, L["ln2"], c.eps, L["gate_up"], self.mlp_act, spare, self.slab, sk, L["o"], sA, mA,
+                                           self.amax[li, 1])
+                    x, spare = spare, x
                     pending = (self._partial_f16(self.mlp_act, self.amax[li, 1], L["down"], mA, sA), L["down"])
                     continue
                 if l3 and self.pf_down:
