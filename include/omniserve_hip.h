@@ -556,8 +556,14 @@ int omni_w4a8_per_group_norm_gemm_fused(void* codes_i8, void* residual_f16, cons
  * omni_w4a8_per_*_gemm / omni_w8a8_gemm, or with amax_slots_u32 (out = act [M, N/2]) omni_*_gemm_silu.  mode: 0 per-channel W4A8 (p_wszs, p_asums and
  * w_szs required), 1 per-group W4A8 (zeros_i8, scales_i8 required), 2 W8A8; the projection before (p_*) has the same mode.  residual_out_f16 must
  * be another buffer than residual_f16.  Replaces llama_w4a8_unpad.py:410-415,425-432 at these sizes.
- * omni_norm_product_ok: 1 where the form exists; k_before: K of the omni_*_gemm_partial[_f16] whose slabs are consumed (0: none). */
+ * omni_norm_product_ok: 1 where the form exists; k_before: K of the omni_act_product, or
+ * where that has not the size of the omni_*_gemm_partial_f16, whose slabs are consumed (0: none).
+ * omni_act_product: omni_*_gemm_partial_f16 for one or two rows (W8A8: one) in K slices of its own, omni_act_product_slices of them (0: not its size;
+ * csrc/act_product.hip); the slabs' sums are the same.  sum_f16 may be NULL.  act and weight 16-byte aligned. */
 int omni_norm_product_ok(int M, int N, int K, int mode, int silu, int k_before);
+int omni_act_product_slices(int M, int N, int K, int mode);
+int omni_act_product(int mode, const void* act_f16, const void* amax_slots_u32, const void* weight, const void* zeros_i8, const void* scales_i8,
+                     void* slab_i32, size_t slab_bytes, void* sum_f16, void* scale_f16, int M, int N, int K, void* stream);
 int omni_norm_product(int mode, const void* residual_f16, void* residual_out_f16, const void* slab_i32, int sk, const void* p_wscales_f16,
                       const void* p_ascales_f16, const void* p_wszs_f16, const void* p_asums_f16, const void* gamma_f16, float eps,
                       const void* weight, const void* zeros_i8, const void* scales_i8, const void* wscales_f16, const void* w_szs_f16,

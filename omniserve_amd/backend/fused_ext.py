@@ -466,6 +466,31 @@ def norm_product_ok(M, N, K, mode, silu=False, k_before=0):
     return _lib.lib().omni_norm_product_ok(int(M), int(N), int(K), int(mode), int(bool(silu)), int(k_before)) == 1
 
 
+def _mode_and_weights(lin):
+    """mode, weights, scales, scaled zero points (per-channel), second-level zeros and scales (per-group) of a W4A8 or W8A8 layer"""
+    if hasattr(lin, "dequant_scale"):
+        return 2, lin.weight, lin.dequant_scale, None, None, None
+    if lin.group == -1:
+        return 0, lin.qweight, lin.s1_scales, lin.s1_szeros, None, None
+    return 1, lin.qweight, lin.s1_scales, None, lin.s2_zeros, lin.s2_scales
+
+
+def act_product_ok(M, N, K, mode):
+    return _lib.lib().omni_act_product_slices(int(M), int(N), int(K), int(mode)) > 0
+
+
+def act_product(act, amax, lin, slab, sum_out, scale_out):
+    """gemm_partial_f16_* of one or two rows in K slices of its own (csrc/act_product.hip): returns their number, the slabs' sums are the same."""
+    _lib.require_cuda(act, amax, slab, sum_out, scale_out)
+    M, K = act.shape
+    mode, w, _, _, s2z, s2s = _mode_and_weights(lin)
+    rc = _lib.lib().omni_act_product(mode, act.data_ptr(), amax.data_ptr(), w.data_ptr(), _ptr(s2z), _ptr(s2s), slab.data_ptr(),
+                                     slab.numel() * slab.element_size(), _ptr(sum_out), scale_out.data_ptr(), M, w.shape[0], K,
+                                     _lib.current_stream())
+    _lib.check(rc, "fused_ext.act_product")
+    return _lib.lib().omni_act_product_slices(M, w.shape[0], K, mode)
+
+
 def norm_product(residual, gamma, epsilon, lin, out, residual_out=None, slab=None, sk=0, producer=None, p_ascales=None, p_asums=None,
                  amax=None):
     """residual_out = residual + epilogue(sum of `sk` slabs of `producer`) (no slab: the residual as it is), rms_norm_general[_fuse_sum] of it,
@@ -473,12 +498,7 @@ def norm_product(residual, gamma, epsilon, lin, out, residual_out=None, slab=Non
     `lin` / `producer`: W4A8 (qweight, s1_scales, s1_szeros or s2_zeros / s2_scales) or W8A8 layers (weight, dequant_scale) of one kind."""
     _lib.require_cuda(residual, gamma, out, residual_out, slab, p_ascales, p_asums, amax)
     M, K = residual.shape
-    if hasattr(lin, "dequant_scale"):
-        mode, w, scale, zero, s2z, s2s = 2, lin.weight, lin.dequant_scale, None, None, None
-    elif lin.group == -1:
-        mode, w, scale, zero, s2z, s2s = 0, lin.qweight, lin.s1_scales, lin.s1_szeros, None, None
-    else:
-        mode, w, scale, zero, s2z, s2s = 1, lin.qweight, lin.s1_scales, None, lin.s2_zeros, lin.s2_scales
+    mode, w, scale, zero, s2z, s2s = _mode_and_weights(lin)
     p_scale = p_zero = None
     if slab is not None:
         p_scale = producer.dequant_scale if mode == 2 else producer.s1_scales

@@ -286,7 +286,8 @@ extern "C" int omni_norm_product_ok(int M, int N, int K, int mode, int silu, int
   const int kalign = mode == MODE_GRP ? 128 : 64;
   if (k_before == 0) return !silu;
   if (k_before < kalign || k_before % kalign) return 0;
-  return sizes_ok(M, N, K, mode, silu != 0, plan_gemm(M, K, k_before, kalign, true, mode == MODE_W8).sk);
+  const int slices = act_product_slices(M, K, k_before, mode);
+  return sizes_ok(M, N, K, mode, silu != 0, slices ? slices : plan_gemm(M, K, k_before, kalign, true, mode == MODE_W8).sk);
 }
 
 extern "C" int omni_norm_product(int mode, const void* residual_f16, void* residual_out_f16, const void* slab_i32, int sk, const void* p_wscales_f16,

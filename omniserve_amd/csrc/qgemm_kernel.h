@@ -1222,6 +1222,8 @@ struct GemmPlan {
   int midm;    // 1: w4a8_midm_kernel (qgemm_midm.h): 128 channels x mb * 16 rows per workgroup, mz row tiles in grid.z
 };
 
+int act_product_slices(int M, int N, int K, int mode);      // act_product.hip's K slices; 0: not its size
+
 // Tuning hook (tests / bench sweeps): waves<=0 and sk<=0 restore the heuristic.
 extern "C" void omni_gemm_set_plan_override(int waves, int sk);
 // mode: -1 heuristic, 0 never the mid-M kernel, 1 wherever its shape conditions hold; sk > 0 forces its K split

@@ -24,20 +24,21 @@ __device__ __forceinline__ uint32_t code_place(uint32_t k) {
 }
 
 // BLOCKS: 16-row operand blocks of the workgroup (packed weights: whole tile rows, 4 blocks to a pair).  KPART: k of a wave.  RING: units (of UNIT k) that
-// fly together.
-template <int MODE, int LAYOUT, int BLOCKS, int KPART, int RING_MAX, int ROWS>
+// fly together.  NT: packed weights load non-temporally (false: they lie in L2).
+template <int MODE, int LAYOUT, int BLOCKS, int KPART, int RING_MAX, int ROWS, bool NT = true>
 struct RowProduct {
   static constexpr bool W8 = MODE == MODE_W8, PAIRED = !W8 && LAYOUT == LAYOUT_ROWS32;
   static constexpr int PAIRS = BLOCKS / 4;                                  // tile-row pairs (ROWS32: the one tile row)
   static_assert(W8 || BLOCKS % 4 == 0, "whole tile rows");
   static constexpr int UNIT = (PAIRED || W8) && KPART % 128 == 0 ? 128 : 64, UNITS = KPART / UNIT;
-  static_assert(KPART % UNIT == 0 && (!PAIRED || UNIT == 128) && (MODE != MODE_GRP || KPART % 128 == 0), "whole units");
+  static_assert(KPART % UNIT == 0 && (!PAIRED || UNIT == 128), "whole units");
   static constexpr int HALVES = W8 ? UNIT / 64 : 1;
   static constexpr int LOADS = W8 ? HALVES * BLOCKS : 2 * PAIRS;            // 16-byte loads of a unit
   static constexpr int RING = UNITS < RING_MAX ? UNITS : RING_MAX;
   static constexpr int COLS = ROWS * (PAIRED ? 2 : 1);
   static constexpr int PART_BYTES = RP_WAVES * BLOCKS * 4 * COLS * 16;
-  static constexpr int GROUPS = MODE == MODE_GRP ? KPART / 128 : 1;
+  static constexpr int PER = KPART % 128 ? 1 : 128 / UNIT;                  // units that share their group's parameters
+  static constexpr int GROUPS = MODE == MODE_GRP ? UNITS / PER : 1;
 
   uint4 wq[RING][LOADS];
   uint32_t gs[PAIRS ? PAIRS : 1][GROUPS], gz[PAIRS ? PAIRS : 1][GROUPS];
@@ -76,7 +77,7 @@ struct RowProduct {
         for (int t = 0; t < PAIRS; ++t)
 #pragma unroll
           for (int i = 0; i < GROUPS; ++i) {
-            const size_t off = (size_t)(k0 / 128 + i) * N + (trow + t * pair) * 32 + lc * 4;
+            const size_t off = (size_t)((k0 + i * PER * UNIT) / 128) * N + (trow + t * pair) * 32 + lc * 4;
             gs[t][i] = *reinterpret_cast<const uint32_t*>(s2s + off);
             gz[t][i] = *reinterpret_cast<const uint32_t*>(s2z + off);
           }
@@ -90,7 +91,7 @@ struct RowProduct {
     for (int j = 0; j < LOADS; ++j) {
       const uint8_t* src = base + (W8 ? j / HALVES : j >> 1) * step + (W8 ? place(u) * UNIT + (j % HALVES) * 64 : (u * (UNIT / 32) + (j & 1)) * 512);
       v4i v;
-      if constexpr (W8) v = *reinterpret_cast<const v4i*>(src);             // (non-temporal, a line's second half is fetched again: 31 us, not 28)
+      if constexpr (W8 || !NT) v = *reinterpret_cast<const v4i*>(src);             // (non-temporal, a line's second half is fetched again: 31 us, not 28)
       else v = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(src));
       wq[u % RING][j] = make_uint4((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]);
     }
@@ -121,7 +122,6 @@ struct RowProduct {
 #pragma unroll
               for (int q = 0; q < 4; ++q) w[q] = (d[j][q] >> (4 * i)) & 0x0F0F0F0Fu;
               if constexpr (MODE == MODE_GRP) {
-                constexpr int PER = 128 / UNIT;
                 const uint32_t sc = (gs[t][u / PER] >> (8 * (i * 2 + j))) & 0xFFu;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) w[q] = w[q] * sc;

@@ -216,6 +216,12 @@ class LServeDecodeRunner:
             fused_ext.prefetch_arm_gemm(lin.weight, self.B, lin.n, lin.k, 2 | 0x20, deferred, self.prefetch_bytes,
                                         self.prefetch_blocks)
 
+    def _partial_f16(self, act, amax, lin, scale_out):
+        """o_proj / down_proj from fp16 activations and their row maxima: int32 slabs in self.slab, returns their number."""
+        if self.own_rows and fused_ext.act_product_ok(self.B, lin.n, lin.k, 2):
+            return fused_ext.act_product(act, amax, lin, self.slab, None, scale_out)
+        return fused_ext.gemm_partial_f16_w8a8(act, amax, lin.weight, self.slab, scale_out)
+
     # one decode step; `select` = this step refreshes the page selection (every `interval`-th step upstream)
     def _eager_step(self, hist: int, select: bool):
         try:
@@ -319,7 +325,7 @@ class LServeDecodeRunner:
             if not self.fused:
                 fused_kernels.invoke_quant(self.q_attn, out.view(B, Hq * d), sq)
             if rowfree:
-                sk = fused_ext.gemm_partial_f16_w8a8(self.attn_f16, self.amax[li, 0], L["o"].weight, self.slab, sq)
+                sk = self._partial_f16(self.attn_f16, self.amax[li, 0], L["o"], sq)
             elif self.defer:
                 sk = fused_ext.gemm_partial_w8a8(self.q_attn, L["o"].weight, self.slab)
             else:
@@ -328,7 +334,7 @@ class LServeDecodeRunner:
                 fused_ext.norm_product(x, L["ln2"], c.eps, L["gate_up"], self.mlp_act, spare, self.slab, sk, L["o"], sq,
                                        amax=self.amax[li, 1])
                 x, spare = spare, x
-                pending = (fused_ext.gemm_partial_f16_w8a8(self.mlp_act, self.amax[li, 1], L["down"].weight, self.slab, sq), L["down"])
+                pending = (self._partial_f16(self.mlp_act, self.amax[li, 1], L["down"], sq), L["down"])
                 continue
             if not (rowfree and li < nl - 1):     # (the SiLU-epilogue form pairs gate / up rows: no prefetch descriptor)
                 self._arm(L["gate_up"])
@@ -344,8 +350,7 @@ class LServeDecodeRunner:
             if rowfree and li < nl - 1:     # gate_up with the SiLU*mul epilogue; down_proj quantises on the fly
                 G = L["gate_up"]
                 fused_ext.gemm_silu_w8a8(self.q_hidden, G.weight, G.dequant_scale, sc, self.mlp_act, self.amax[li, 1])
-                pending = (fused_ext.gemm_partial_f16_w8a8(self.mlp_act, self.amax[li, 1], L["down"].weight, self.slab,
-                                                           sq), L["down"])
+                pending = (self._partial_f16(self.mlp_act, self.amax[li, 1], L["down"], sq), L["down"])
                 continue
             L["gate_up"].forward(self.q_hidden, sc, self.gate_up_buf)
             self._arm(L["down"], self.defer and li < nl - 1)

@@ -406,6 +406,8 @@ class DecodeRunner:
     def _partial_f16(self, act, amax, lin, sum_out, scale_out):
         """Level 3: o_proj / down_proj from fp16 activations + row maxima (codes computed inside the GEMV; sums / scales by
         rider workgroups): int32 split-K slabs in self.slab, returns the slab count."""
+        if self.own_rows and fused_ext.act_product_ok(self.B, lin.n, lin.k, 0 if lin.group == -1 else 1):
+            return fused_ext.act_product(act, amax, lin, self.slab, sum_out, scale_out)
         if lin.group == -1:
             return fused_ext.gemm_partial_f16_per_chn(act, amax, lin.qweight, self.slab, sum_out, scale_out)
         return fused_ext.gemm_partial_f16_per_group(act, amax, lin.qweight, lin.s2_zeros, lin.s2_scales, self.slab,
