@@ -17,6 +17,7 @@
 #include "row_kernels.h"
 #include "tp_comm.h"
 #include "norm_rows.h"
+#include "argmax_key.h"
 #include <cstdlib>
 
 namespace omni {
@@ -1100,23 +1101,6 @@ extern "C" int omni_tp_add_rms_norm_general_fuse_sum(void* out_i8, void* residua
 // finishes.  torch's generic reduce kernel takes 47 us for [16, 128256] inside the decode step; this takes ~6.
 // ------------------------------------------------------------------------------------------
 constexpr int ARGMAX_CHUNKS = 32;
-
-__device__ __forceinline__ unsigned long long argmax_key(uint32_t h16, uint32_t idx) {
-  uint32_t h = h16 & 0xFFFFu;
-  if (h == 0x8000u) h = 0;                                   // -0 == +0
-  const uint32_t k = (h & 0x8000u) ? (~h & 0xFFFFu) : (h | 0x8000u);
-  return ((unsigned long long)k << 32) | (unsigned long long)(0xFFFFFFFFu - idx);
-}
-
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    const uint32_t lo = __shfl_xor((uint32_t)v, m, 64), hi = __shfl_xor((uint32_t)(v >> 32), m, 64);
-    const unsigned long long o = ((unsigned long long)hi << 32) | lo;
-    v = o > v ? o : v;
-  }
-  return v;
-}
 
 __global__ __launch_bounds__(256) void argmax_partial_kernel(const half_t* __restrict__ x, int64_t row_stride, int cols,
                                                              unsigned long long* __restrict__ part) {

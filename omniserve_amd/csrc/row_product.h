@@ -45,10 +45,9 @@ struct RowProduct {
   v4i acc[BLOCKS];
   const uint8_t* base;      // of the lane
   long long step;           // packed: from a tile-row pair to the next; int8: from a block of rows to the next
-  int turn;                 // int8: the unit that this workgroup begins with
+  int turn;                 // the unit that this workgroup begins with
 
   __device__ __forceinline__ int place(int u) const {      // of the u-th unit in the wave's K
-    if constexpr (!W8) return u;
     const int v = u + turn;
     return v < UNITS ? v : v - UNITS;
   }
@@ -56,7 +55,9 @@ struct RowProduct {
   // first: the workgroup's first operand block of all; k0: the wave's first k
   __device__ __forceinline__ void open(const uint8_t* W, const uint8_t* s2s, const uint8_t* s2z, int N, int K, int first, int k0) {
     const int lane = threadIdx.x & 63, lx = (lane >> 3) & 1, lc = lane & 7, le = lane >> 4;
-    turn = (first / BLOCKS >> 3) % UNITS;      // (rows lie whole KiBs apart: workgroups in step would all ask the same channels of the memory; 28.6 us, not 27.3)
+// (workgroups in step ask the same channels of the memory: gate_up W8A8 28.9 us, turned 27.6, W4A8 14.3 and 13.8.  Not per-group weights, 16.2 and 17.6, and not
+    // ROWS64: W8A8 down_proj 12.3 and 13.5, o_proj behind its prefetch 4.1 and 4.7)
+    turn = MODE == MODE_GRP || LAYOUT == LAYOUT_ROWS64 ? 0 : (int)(blockIdx.x >> 3) % UNITS;
     if constexpr (W8) {
       if constexpr (LAYOUT == LAYOUT_GATE) {
         base = W + (size_t)(lx * (N / 2) + first * 8 + lc) * K + le * 16 + k0;
@@ -89,7 +90,7 @@ struct RowProduct {
   __device__ __forceinline__ void request(int u) {
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
-      const uint8_t* src = base + (W8 ? j / HALVES : j >> 1) * step + (W8 ? place(u) * UNIT + (j % HALVES) * 64 : (u * (UNIT / 32) + (j & 1)) * 512);
+      const uint8_t* src = base + (W8 ? j / HALVES : j >> 1) * step + (W8 ? place(u) * UNIT + (j % HALVES) * 64 : (place(u) * (UNIT / 32) + (j & 1)) * 512);
       v4i v;
       if constexpr (W8 || !NT) v = *reinterpret_cast<const v4i*>(src);             // (non-temporal, a line's second half is fetched again: 31 us, not 28)
       else v = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(src));

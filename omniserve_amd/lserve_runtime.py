@@ -370,8 +370,7 @@ class LServeDecodeRunner:
                                           self.final_norm, c.eps)
         else:
             layernorm_ops.rms_norm(self.normed, self.x, self.final_norm, c.eps, False)
-        logits = torch.matmul(self.normed, self.lm_head.t())
-        fused_ext.argmax(self.tokens, logits)
+        fused_ext.head_argmax(self.tokens, self.normed, self.lm_head)
 
     # ---- context stage ------------------------------------------------------------------------------------------------
     def prefill(self, tokens=None, hidden=None, seq_len=None, chunk=16384):
@@ -468,7 +467,7 @@ class LServeDecodeRunner:
             self.page_idx = [torch.zeros((B, Hq, npick), dtype=torch.int32, device=dev) for _ in self.layers]
         last = x[Lp - 1::Lp].contiguous()
         layernorm_ops.rms_norm(self.normed, last, self.final_norm, c.eps, False)
-        fused_ext.argmax(self.tokens, torch.matmul(self.normed, self.lm_head.t()))
+        fused_ext.head_argmax(self.tokens, self.normed, self.lm_head)
         return x
 
     def step(self):

@@ -606,11 +606,14 @@ class DecodeRunner:
                                           lin.s1_szeros if per_chn else None, mA if per_chn else None, self.final_norm, c.eps)
         else:
             layernorm_ops.rms_norm(self.normed, self.x, self.final_norm, c.eps, False)
-        logits = torch.matmul(self.normed, self.lm_head.t())
+        self._greedy()
+
+    def _greedy(self):
+        """self.tokens <- argmax of the head's logits of self.normed"""
         if self.fused:
-            fused_ext.argmax(self.tokens, logits)      # same result as torch.argmax, 6 us instead of 47
+            fused_ext.head_argmax(self.tokens, self.normed, self.lm_head)
         else:
-            self.tokens.copy_(torch.argmax(logits, dim=-1))
+            self.tokens.copy_(torch.argmax(torch.matmul(self.normed, self.lm_head.t()), dim=-1))
 
     # ---- prefill (context stage) ---------------------------------------------------------------------------
     def prefill(self, prompt_len=None, tokens=None):
@@ -687,8 +690,7 @@ class DecodeRunner:
         last = x.view(B, L, c.hidden)[:, L - 1]
         self.x.copy_(last)
         layernorm_ops.rms_norm(self.normed, self.x, self.final_norm, c.eps, False)
-        logits = torch.matmul(self.normed, self.lm_head.t())
-        self.tokens.copy_(torch.argmax(logits, dim=-1))
+        self._greedy()
         self.lengths.fill_(L)
 
     def _all_reduce(self, buf):
