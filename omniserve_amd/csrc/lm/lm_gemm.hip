@@ -153,7 +153,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(GemmArgs p) {
 // -> 26 (117 MB: 4.5 TB/s), 28672 x 4096 75 -> 49, 32 experts at 60 tokens (998 MB) 278 -> 172 us (5.8 TB/s).  A stage is consumed behind one
 // barrier; R - 1 more are on their way.
 constexpr int RB = 128;                // bytes of k of a stage's rows
-template <int NW, int KW> constexpr int ring_bytes = KW > 1 ? (144 << 10) / KW : NW <= 4 ? 64 << 10 : 80 << 10;      // of one K part
+template <int NW, int KW> constexpr int ring_bytes = KW > 1 ? (144 << 10) / KW : NW <= 4 ? 64 << 10 : NW == 5 ? 80 << 10 : 144 << 10;      // of one K part
 
 // at most N pieces of this wave still fly, and its LDS reads have been answered
 template <int N>
@@ -163,9 +163,9 @@ __device__ __forceinline__ void wait_stage() {
 
 // rows (at most 16 MB) of x times 16 NW channels of w, stages s0 .. s1 - 1 of k, into red [KW][16 MB][16 NW + 4]: part h of the
 // workgroup's waves takes every KW-th stage through a ring of its own
-// SHORT: k may be below CHAIN_K.
+// SHORT: k may be below CHAIN_K.  TURN: see gemm_stream_kernel.
 constexpr int CHAIN_K = 64 * KSTEP;
-template <int MB, int NW, int KW, bool SHORT>
+template <int MB, int NW, int KW, bool SHORT, bool TURN>
 __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int n, int64_t k, int n0, const elem_t* x, int64_t ldx,
                                               const int* perm, int div, int rows, int s0, int s1) {
   constexpr int WST = 16 * NW * RB, XST = 16 * MB * RB, ST = WST + XST, R0 = ring_bytes<NW, KW> / ST;
@@ -191,12 +191,15 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
     xsrc[i] = (const uint8_t*)(x + row * ldx) + (int64_t)(s0 + h) * RB + ((ps ^ T::swizzle(r)) << 4);
   }
   const uint32_t base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
-  auto stage = [&](int t) {                                // stage t of this part
+  const int nst = (s1 - s0 - h + KW - 1) / KW;
+  const int turn = TURN && gridDim.z == 1 && nst > 0 ? (int)(blockIdx.x >> 3) * 2 % nst : 0;
+  auto stage = [&](int t) {                                // the t-th stage of this part
     const uint32_t dst = base + (uint32_t)(t % R) * ST;
+    const int at = (!TURN || t + turn < nst ? t + turn : t + turn - nst) * (KW * RB);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16_stream(wsrc[i] + t * (KW * RB), dst + 2048 * wave + 1024 * i);
+    for (int i = 0; i < 2; ++i) dma16_stream(wsrc[i] + at, dst + 2048 * wave + 1024 * i);
 #pragma unroll
-    for (int i = 0; i < XP; ++i) dma16_uncounted(xsrc[i] + t * (KW * RB), dst + WST + 1024 * xp[i]);
+    for (int i = 0; i < XP; ++i) dma16_uncounted(xsrc[i] + at, dst + WST + 1024 * xp[i]);
   };
   // sums of 4 stages (2, 1, half a one) and the sum of those: chains of f32 additions no longer than an eighth of K.  (A form of its own for long K: with
   // the choice in it that one took 3 - 7 % more, 16 tokens of 8 of 64 x 1280 x 2048 52.8 -> 55.5 us.)
@@ -230,7 +233,6 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
     }
     if ((t & chain) == chain) end_chain();
   };
-  const int nst = (s1 - s0 - h + KW - 1) / KW;
   wait_pieces<0>();                                        // the compiler's own loads
 #pragma unroll
   for (int t = 0; t < R - 1; ++t)
@@ -281,14 +283,19 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
   const int stages = pt.k * (int)sizeof(elem_t) / RB, slice = blockIdx.z, slices = gridDim.z;
   const int s0 = stages * slice / slices, s1 = stages * (slice + 1) / slices;
   const int div = is_b ? 1 : p.x_div;
+  // Rows lie whole KiBs apart: workgroups in step ask the same channels of the memory, so each begins 256 bytes further in k than the one before it on its
+  // XCD (MI355X: 28672 x 4096 at 48 rows 50.4 -> 47.0 us, 32000 x 4096 54.3 -> 49.8, 32000 x 2048 at 16 rows 26.3 -> 22.7).  Heads and wide dense gated units
+  // only: the sums' order changes with it, and what a router reads keeps its order, so that near ties choose as they did (experts would gain 3 %: 16 tokens
+  // of 8 of 64 x 1280 x 2048 54.2 -> 52.6); K slices begin at places of their own (4096 x 14336 in 4 of them 24.7, turned 25.3).
+  constexpr bool TURN = EPI == LM_EPI_F32 || (EPI == LM_EPI_GLU && NW == 8);
   for (int m0 = 0; m0 < rows; m0 += 64) {
     const int here = min(64, rows - m0), mb = (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
     const int* pm = perm ? perm + m0 : nullptr;
-    if (mb == 1) stream_stages<1, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else if (mb == 2) stream_stages<2, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else if (mb == 3) stream_stages<3, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else stream_stages<4, NW, KW, SHORT>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    if (mb == 1) stream_stages<1, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 2) stream_stages<2, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 3) stream_stages<3, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else stream_stages<4, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     const float* red = (const float*)lds;
     auto sum = [&](int m, int c) {
       f32x4 v = *(const f32x4*)&red[m * (RC + 4) + c];
@@ -672,7 +679,9 @@ static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s
 // 256 more: 16448 channels at 48 rows take 42 us as 257 tiles of 64, 30 as 206 of 80), and slices cost the launch that adds them.  By what
 // was measured the channels per workgroup matter most where n / 64 is far from a multiple of 256 (10816 x 4096, 48 rows: 26.5 us at 64,
 // 20.8 at 48; 4096 x 4096, 16 rows: 11.8 us at 64 and 4 slices, 9.8 at 16), slices where K is long (4096 x 14336, 48 rows: 40 us, 26
-// with 4).
+// with 4).  128 channels, bf16: 2.5 us for a ring of 144 KiB that nothing runs beside, but x comes in half as often, and 224 or 250 workgroups are one round where 448
+// or 500 are two (28672 x 4096, 64 / 128 channels: 1 row 38.0 / 37.3 us, 48 rows 45.5 / 38.2, 64 rows 47.4 / 39.3; 32000 x 4096, 48 rows 45.2 / 42.9;
+// 32000 x 2048, 16 rows 22.0 / 24.3; 96 and 112 channels nowhere the fastest).
 struct RowsPlan {
   int nw, slices;      // nw 0: gemm_rows_kernel
 };
@@ -680,11 +689,12 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
   RowsPlan best{4, 1};
   float time = 1e30f;
   const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
-  for (int nw = 5; nw >= 1; --nw) {
-    if (glu && nw != 4) continue;                          // (a gate block and its up block share a workgroup)
+  for (int nw = LM_ELEM ? 5 : 8; nw >= 1; --nw) {
+    if (nw == 6 || nw == 7 || (glu && nw % 4)) continue;   // (a gate block and its up block share a workgroup)
     const int64_t tiles = (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw));
     for (int s = 1; s <= (sliced ? 8 : 1) && (s == 1 || stages >= 4 * s); s *= 2) {
       float t = (float)((tiles * s + 255) / 256) * (float)((stages + s - 1) / s) * (0.07f * nw + 0.02f * mb + 0.02f);
+      if (nw == 8) t += 2.5f;
       if (s > 1) t += 4.5f + (float)s * rows * n * 8.f / 5e6f;
       if (t < time) { time = t; best = RowsPlan{nw, s}; }
     }
@@ -696,8 +706,8 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
 template <int EPI, int NW, bool SHORT>
 static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
-  constexpr int KW = NW <= 2 ? 4 : 2;
-  if ((int64_t)grid.x * grid.y * grid.z <= 256)
+  constexpr int KW = NW <= 2 ? 4 : NW <= 5 ? 2 : 1;
+  if (KW > 1 && (int64_t)grid.x * grid.y * grid.z <= 256)
     hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT>), grid, dim3(64 * NW * KW), 0, s, a, part);
   else
     hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT>), grid, dim3(64 * NW), 0, s, a, part);
@@ -713,9 +723,13 @@ template <int EPI>
 static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part, hipStream_t s) {
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
   if constexpr (EPI == LM_EPI_GLU) {
-    launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s);
+    if (LM_ELEM == 0 && pl.nw == 8) launch_stream_tiles<EPI, LM_ELEM == 0 ? 8 : 4>(a, n, has_b, pl.slices, part, s);
+    else launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s);
   } else {
     switch (pl.nw) {
+#if LM_ELEM == 0
+      case 8: launch_stream_tiles<EPI, 8>(a, n, has_b, pl.slices, part, s); break;
+#endif
       case 1: launch_stream_tiles<EPI, 1>(a, n, has_b, pl.slices, part, s); break;
       case 2: launch_stream_tiles<EPI, 2>(a, n, has_b, pl.slices, part, s); break;
       case 3: launch_stream_tiles<EPI, 3>(a, n, has_b, pl.slices, part, s); break;

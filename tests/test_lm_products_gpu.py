@@ -78,6 +78,22 @@ def test_every_width(channels, slices, m, n, k, dtype):
     assert errors(ops.matmul(x, w, out_f32=True, scale=0.5).cpu().numpy(), 0.5 * want.cpu().numpy()).max() < 2e-6
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 32032, 2048), (17, 28704, 4160), (1, 32768, 4096), (48, 28672, 4096)])
+def test_workgroups_of_128_channels(m, n, k):
+    """bf16 only: one round of them; channels that end inside one, uneven stages, the gated unit"""
+    ops = _ops(torch.bfloat16)
+    assert _rows_plan(ops, 1, n, k, m) == (128, 1) and _rows_plan(ops, 1, n, k, m, 2) == (128, 1)
+    x, w = _randn(31, torch.bfloat16, m, k + 64)[:, 64:], _randn(32, torch.bfloat16, n, k) * k ** -0.5
+    want = x.double() @ w.double().t()
+    guard = torch.full((m + 2, n), 7.0, device=DEV)
+    ops.matmul(x, w, out=guard[1:-1], out_f32=True)
+    assert errors(guard[1:-1].cpu().numpy(), want.cpu().numpy()).max() < 2e-6
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+    y = want.view(m, n // 32, 2, 16)
+    unit = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(m, n // 2)
+    assert errors(ops.glu(x, w, None, "silu").float().cpu().numpy(), unit.cpu().numpy()).max() < TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("m,n,k", [(1, 16, 64), (16, 1040, 128), (33, 2064, 192), (64, 512, 4160), (48, 9216, 64)])
 def test_gated_unit(m, n, k, dtype):
