@@ -43,7 +43,8 @@ size_t omni_gemm_partial_workspace_bytes(int M, int N, int K);
 
 /* Tuning / introspection hooks (tests and bench sweeps; not used by the serving path):
  * override the decode-shape plan (waves per workgroup: 1 or 4; K splits; M > 128: K slices over the grid where the plan may
- * have them), 0/0 restores the heuristic; query the plan the library would use.  M > 128: that plan says what scratch the call
+ * have them, and waves = 16: per-group products of 256 rows or more in 256 x 256 tiles wherever K >= 512 and they are not split),
+ * 0/0 restores the heuristic; query the plan the library would use.  M > 128: that plan says what scratch the call
  * brings; omni_gemm_get_prefill_plan says which tiles run and whether they use it. */
 void omni_gemm_set_plan_override(int waves, int sk);
 /* The mid-M kernel (M = 33 .. 128, csrc/qgemm_midm.h; the regime of gemm_cuda.cu:621-655's 32x64x128 / 64x64x64 tiles):
@@ -53,7 +54,8 @@ void omni_gemm_set_midm_override(int mode, int sk);
 void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, int* sk);
 /* M > 128 (0 below), operands and output rows 16-byte aligned (others go to the general kernel).  mode: 0 per-channel W4A8, 1 per-group W4A8, 2 W8A8; slabs_only: omni_*_gemm_partial.
  * Returns 1 for the straight-line kernels: *mb 16-row blocks of a tile (16: the 256 x 256 tiles of W8A8), *kw K parts inside a
- * workgroup, *sk K slices that go through the scratch (1: none but slabs_only's own).  2 for the general kernel (N % 256 or K % 256). */
+ * workgroup, *sk K slices that go through the scratch (1: none but slabs_only's own);
+ * per-group: what runs where its own 256 x 256 tiles (csrc/qgemm_group_tiles.h) are not the faster choice.  2 for the general kernel (N % 256 or K % 256). */
 int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int slabs_only, int* mb, int* kw, int* sk);
 /* 1 when the row-kernel-free decode forms below (omni_*_gemm_silu for gate_up [2*inter, hidden], omni_*_gemm_partial_f16
  * for o [hidden, attn_dim] and down [hidden, inter]) accept a layer of these dimensions at M rows, 0 otherwise: the plan

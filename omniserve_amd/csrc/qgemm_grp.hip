@@ -1,6 +1,16 @@
 // omni_w4a8_per_group_gemm: instantiates the g128 per-group W4A8 kernels (see qgemm_kernel.h).
 #include "qgemm_kernel.h"
+#include "qgemm_group_tiles.h"
 using namespace omni;
+
+void omni::launch_group_tiles(const GemmArgs& a, hipStream_t st) {      // a workgroup per CU
+  GemmArgs b = a;
+  b.tiles_n = b.N / TILES_N;
+  b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
+  const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
+  b.tile_linear = (b.tiles_m + bands - 1) / bands;
+  hipLaunchKernelGGL(w4a8_group_tiles_kernel, dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+}
 
 extern "C" int omni_w4a8_per_group_gemm(const void* in_feats, const void* qweight, const void* zeros,
                                         const void* scales_i8, const void* wscales, const void* ascales,

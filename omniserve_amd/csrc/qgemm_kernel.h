@@ -1232,9 +1232,10 @@ extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool w8 = false);
 
 // w4a8_gemm_exact_kernel's tile height (16-row blocks; 16: w8a8_tiles_kernel), K parts inside a workgroup, K slices over the grid (1: no
-// slabs)
+// slabs); group_tiles: w4a8_group_tiles_kernel instead of all that
 struct PrefillPlan {
   int mb, kw, sk;
+  bool group_tiles = false;
 };
 // sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs (omni_gemm_set_plan_override's K splits do, too)
 PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only);
@@ -1281,6 +1282,9 @@ static void launch_tiles(GemmArgs b, hipStream_t st) {
   hipLaunchKernelGGL((w8a8_tiles_kernel<MODE>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
 }
 
+// qgemm_grp.hip
+void launch_group_tiles(const GemmArgs& a, hipStream_t st);
+
 // prefill regime (M > 128): chunked LDS staging, weights through L2
 template <int MODE>
 static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
@@ -1289,6 +1293,13 @@ static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
     if constexpr (MODE == MODE_W8) {
       if (pp.mb == 16) {
         launch_tiles<MODE>(a, st);
+        return;
+      }
+    }
+    if constexpr (MODE == MODE_GRP) {
+      // (a lane's parameters are four bytes)
+      if (pp.group_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
+        launch_group_tiles(a, st);
         return;
       }
     }
