@@ -539,13 +539,14 @@ struct DeltaDecodeArgs {
   int H, G;
 };
 
+// Bound by the states read and written; heads vary first over the grid, as in gla_decode_kernel (48 sequences of 32 heads x 128 x 128: 44.2 -> 40.6 us).
 template <int DK, int DV, bool STREAM>
 __global__ __launch_bounds__(4 * DV) void delta_decode_kernel(DeltaDecodeArgs p) {
   constexpr int TH = 4 * DV, COLS = DV / 4, ROWS = DK / STATE_GROUPS;
   __shared__ __attribute__((aligned(16))) float qkv[2 * DK + DV];
   __shared__ float unit[2];
   __shared__ f32x4 red[2][STATE_GROUPS][COLS];
-  const int b = blockIdx.x, h = blockIdx.y, g = h / (p.H / p.G), tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
+  const int h = blockIdx.x, b = blockIdx.y, g = h / (p.H / p.G), tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
   const int ps = p.pos[b];
   if (ps < 0) return;
   const int slot = p.slot[b], channels = 2 * p.G * DK + p.H * DV;
@@ -662,9 +663,9 @@ extern "C" int lm_delta_decode(const void* x, int64_t ld, void* o, int64_t ldo, 
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
     if (streams_state(B, H, K, V))                                                                           \
-      hipLaunchKernelGGL((delta_decode_kernel<K, V, true>), dim3(B, H), dim3(4 * V), 0, s, a);               \
+      hipLaunchKernelGGL((delta_decode_kernel<K, V, true>), dim3(H, B), dim3(4 * V), 0, s, a);               \
     else                                                                                                     \
-      hipLaunchKernelGGL((delta_decode_kernel<K, V, false>), dim3(B, H), dim3(4 * V), 0, s, a);              \
+      hipLaunchKernelGGL((delta_decode_kernel<K, V, false>), dim3(H, B), dim3(4 * V), 0, s, a);              \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)

@@ -370,13 +370,15 @@ struct GlaDecodeArgs {
   int H;
 };
 
+// Bound by the states read and written.  Heads vary first over the grid: neighbouring workgroups take neighbouring states, where sequences first would have
+// them all a slot apart, on the same memory channels at a time (48 sequences of 32 heads x 128 x 128, 201 MB: 46.3 -> 40.6 us, 5.0 TB/s).
 template <int DK, int DV, bool STREAM>
 __global__ __launch_bounds__(4 * DV) void gla_decode_kernel(GlaDecodeArgs p) {
   constexpr int TH = 4 * DV, COLS = DV / 4, ROWS = DK / STATE_GROUPS;
   static_assert(TH == COLS * STATE_GROUPS, "layout");
   __shared__ float qs[DK], ks[DK], as[DK];
   __shared__ f32x4 red[STATE_GROUPS][COLS];
-  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
+  const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
   const int ps = p.pos[b];
   if (ps < 0) return;
   const elem_t* row = p.x + (int64_t)b * p.ld;
@@ -466,9 +468,9 @@ extern "C" int lm_gla_decode(const void* x, int64_t ld, void* o, int64_t ldo, fl
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
     if (streams_state(B, H, K, V))                                                                           \
-      hipLaunchKernelGGL((gla_decode_kernel<K, V, true>), dim3(B, H), dim3(4 * V), 0, s, a);                 \
+      hipLaunchKernelGGL((gla_decode_kernel<K, V, true>), dim3(H, B), dim3(4 * V), 0, s, a);                 \
     else                                                                                                     \
-      hipLaunchKernelGGL((gla_decode_kernel<K, V, false>), dim3(B, H), dim3(4 * V), 0, s, a);                \
+      hipLaunchKernelGGL((gla_decode_kernel<K, V, false>), dim3(H, B), dim3(4 * V), 0, s, a);                \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)
