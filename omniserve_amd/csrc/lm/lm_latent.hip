@@ -170,15 +170,16 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void latent_decode_kernel(Laten
     qa[i] = (float)pos * p.freq[d];
   }
   // The first tile is on its way while the rest is prepared (what the compiler loads behind it only makes the loop's first wait
-  // stricter) -- but behind the new row where this workgroup brings it: every one whose part holds the newest tile writes the row
-  // (equal bytes).
+  // stricter) -- but behind the new row where that is in it and this workgroup brings it: every one whose part holds the newest tile
+  // writes the row (equal bytes).
   const int slot = p.slot[b];
-  const bool append = tb == nt && ta < tb && slot >= 0 && p.src_col >= 0;
+  const bool append = tb == nt && ta < tb && slot >= 0 && p.src_col >= 0, one = append && ta == nt - 1;
+  if (ta < tb && !one) stage(ta);
   if (append) {
     latent_row(row + p.src_col, p.w, p.eps, p.freq, p.half, pos, p.cache + (int64_t)slot * ROW, p.R, RP, TP, red);
     __syncthreads();    // (makes it visible to the other waves of this workgroup)
   }
-  if (ta < tb) stage(ta);
+  if (one) stage(ta);
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     const int hh = (256 * i + tid) / (TP / 2), d = (256 * i + tid) % (TP / 2);
@@ -281,9 +282,13 @@ static int launch_blocks(const LatentDecodeArgs& a, int B, hipStream_t s) {
   return launch_status();
 }
 
+// 16 heads a workgroup while all of those are on the chip at once (two a CU for 16-bit rows of 512 + 64): a workgroup is a chain of short steps, and each is half as long; 32 heads read
+// the keys once (MI355X, 32 heads, without splits, 32 | 16 heads a workgroup, us: 48 sequences of 150 keys 17.2 | 14.0, of 400 30.9 | 24.7; 128 of 900, two
+// splits, 54 | 52; 256 of 30 11.9 | 13.4, of 400 38.7 | 36.1, of 2000 167 | 156; 288 of 150 26.0 | 31.7, of 1500 142 | 195).
 template <int RP, int TP>
 static int launch(const LatentDecodeArgs& a, int B, hipStream_t s) {
-  return a.H > 16 ? launch_blocks<RP, TP, 2>(a, B, s) : launch_blocks<RP, TP, 1>(a, B, s);
+  constexpr int64_t AT_ONCE = 256 * ((160 * 1024) / (int)(LatentGeom<RP, TP, 1>::LDS + 64));
+  return a.H <= 16 || (int64_t)B * ((a.H + 15) / 16) * a.nsplit <= AT_ONCE ? launch_blocks<RP, TP, 1>(a, B, s) : launch_blocks<RP, TP, 2>(a, B, s);
 }
 
 static int check(int64_t ld, int64_t src_col, const float* w, int half, int H, int dk, int q_rot, int R, int Rp, int Tp) {
