@@ -444,7 +444,8 @@ int omni_kv_min_max_pool(const void* k_f16, const void* kv_pointers_i64, const v
 /* Replaces omniserve_backend.fused_attention_selector.single_query_page_selector
  *   (sparse_utils/KVPageSelector/fused_kv_page_selector.cpp:262-334): for retrieval heads,
  *   out[b,h,c] = fp16( sum_d max(q_d*kmax[c,d], q_d*kmin[c,d]) ) over the sub-chunks c of the history
- *   (q rotated at position lengths[b]-1); out fp16 [B,Hq,padded_sub_chunks] must be zero filled. */
+ *   (q rotated at position lengths[b]-1); out fp16 [B,Hq,padded_sub_chunks]: the
+ *   rest, and streaming heads, zero. */
 int omni_kv_page_selector(void* out_f16, const void* q_f16, int64_t q_stride, const void* kv_pointers_i64,
                           const void* retrieval_head_flags_i32, const void* head_rank_table_i32,
                           const void* lengths_i32, int batch, int max_blocks, int num_heads, int num_kv_heads,

@@ -29,7 +29,8 @@ def single_query_page_selector(q, k, v, retrieval_kv_pointers, streaming_kv_poin
     n_sub = (int(timestep) + tokens_per_sub_chunk - 1) // tokens_per_sub_chunk
     group = tokens_per_block // tokens_per_sub_chunk
     padded = (n_sub + group - 1) // group * group
-    out = torch.zeros((B, Hq, padded), dtype=q.dtype, device=q.device)
+    # (the kernel writes the zeros, too; a stand-in of the library on the host need not)
+    out = (torch.zeros if q.device.type == "cpu" else torch.empty)((B, Hq, padded), dtype=q.dtype, device=q.device)
     scale = 1.0 if rotary_embedding_scale == 1.0 else 1.0 / float(rotary_embedding_scale)
     table = rope_table(int(timestep) + 1, D, float(rotary_base), scale, q.device)
     rc = _lib.lib().omni_kv_page_selector(out.data_ptr(), q.data_ptr(), q.stride(0), retrieval_kv_pointers.data_ptr(),

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void kv_min_max_pool_kernel(PoolArgs p) {
 }
 
 struct SelArgs {
-  half_t* out;                // [B, Hq, padded_sub_chunks] (zero filled by the caller)
+  half_t* out;                // [B, Hq, padded_sub_chunks]
   const half_t* q; int64_t q_stride;
   const int64_t* kv_pointers; // retrieval table [B,2,max_blocks]
   const int* retrieval_head_flags; const int* head_rank_table; const int* lengths;
@@ -65,13 +65,14 @@ struct SelArgs {
   int row_bytes;              // Dh/2 (KV4 pages) or Dh (KV8 pages)
 };
 
-// Page selector.  One workgroup per (block of SEL_PB pages, kv head, sequence) scores ALL q heads of the kv
+// Page selector.  One workgroup per (block of PB pages, kv head, sequence) scores ALL q heads of the kv
 // head's GQA group from one pass over the page statistics (the reference walks them once per q head).  A team
 // of 16 lanes (= one DPP row; 8 dims per lane, one 16-B load of kmax and of kmin) owns a sub-chunk; a team keeps
-// 8 sub-chunks = 16 loads in flight.  Per-lane sums run over e = 0..7 and the team butterfly over xor 8, 4, 2, 1
+// PB / 4 sub-chunks, two loads each, in flight.  Per-lane sums run over e = 0..7 and the team butterfly over xor 8, 4, 2, 1
 // exactly as KVPageSelectorTemplate.hpp:482-493, so the fp32 sums (and the fp16 scores) are bit-identical.
-constexpr int SEL_PB = 32;     // pages per workgroup
-constexpr int SEL_UN = 8;      // sub-chunks in flight per team
+// PB: pages per workgroup, 8 while the chip takes that many workgroups in a few rounds, 16 beyond (8 | 16 | 32 pages, 8 kv heads of 128, 64-token pages of 4 sub-chunks,
+// us: 8000 tokens 4.1 | 5.1 | 7.3, 100000 tokens 9.2 | 10.0 | 11.0, four sequences of that 26.3 | 27.0 | 30.3, eight 47.2 | 45.6 | 48.8, eight of 128000 62 | 57 | 60).
+constexpr int SEL_MANY = 8192;
 
 __device__ __forceinline__ float team_xor4(float v, int lane) {
   const float up = dpp_mov<0x104>(v);    // row_shl:4 : lane i reads lane i+4
@@ -79,21 +80,26 @@ __device__ __forceinline__ float team_xor4(float v, int lane) {
   return (lane & 4) ? dn : up;
 }
 
-template <int G>
+template <int G, int SEL_PB>
 __global__ __launch_bounds__(256) void kv_page_selector_kernel(SelArgs p) {
+  constexpr int SEL_UN = SEL_PB / 4;             // sub-chunks in flight per team (all of a workgroup's where a page has four)
   __shared__ __attribute__((aligned(16))) half_t q_lds[G * SDH];
   __shared__ int64_t page_lds[SEL_PB];
   const int hk = blockIdx.y, b = blockIdx.z;
-  if (p.retrieval_head_flags[hk] == 0) return;   // streaming heads: scores stay zero
   const int rank = p.head_rank_table[hk];
   const int tlen = p.lengths[b] - 1;
   const int tid = threadIdx.x, lane = tid & 63;
   const int subs = p.tpb / p.sub;
-  const int n_sub = (tlen + p.sub - 1) / p.sub;
+  const int n_sub = p.retrieval_head_flags[hk] == 0 ? 0 : (tlen + p.sub - 1) / p.sub;      // streaming heads: no scores
   const int page0 = blockIdx.x * SEL_PB;
   const int c0 = page0 * subs;
-  if (c0 >= n_sub) return;
   const int h0 = hk * G;
+  // its sub-chunks without a score: zero
+  const int c1 = min(c0 + SEL_PB * subs, p.padded);
+  for (int i = max(c0, n_sub) + tid; i < c1; i += 256)
+#pragma unroll
+    for (int g = 0; g < G; ++g) p.out[((size_t)b * p.num_heads + h0 + g) * p.padded + i] = (half_t)0.0f;
+  if (c0 >= n_sub) return;
   if (tid < SEL_PB) {
     const int pg = page0 + tid;
     page_lds[tid] = (pg < p.max_blocks && pg * subs < n_sub) ? p.kv_pointers[(size_t)b * 2 * p.max_blocks + pg] : 0;
@@ -344,12 +350,15 @@ extern "C" int omni_kv_page_selector(void* out_f16, const void* q_f16, int64_t q
   const int subs = tokens_per_block / tokens_per_sub_chunk;
   const int pages = (padded_sub_chunks + subs - 1) / subs;
   if (pages == 0) return OMNI_OK;
-  dim3 grid((pages + SEL_PB - 1) / SEL_PB, num_kv_heads, batch);
+  const bool many = (long long)((pages + 7) / 8) * num_kv_heads * batch > SEL_MANY;
+  const int pb = many ? 16 : 8;
+  dim3 grid((pages + pb - 1) / pb, num_kv_heads, batch);
+  auto launch = [&](auto* few, auto* lots) { hipLaunchKernelGGL(many ? lots : few, grid, dim3(256), 0, (hipStream_t)stream, a); };
   switch (group) {
-    case 1: hipLaunchKernelGGL(kv_page_selector_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
-    case 2: hipLaunchKernelGGL(kv_page_selector_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
-    case 4: hipLaunchKernelGGL(kv_page_selector_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
-    case 8: hipLaunchKernelGGL(kv_page_selector_kernel<8>, grid, dim3(256), 0, (hipStream_t)stream, a); break;
+    case 1: launch(kv_page_selector_kernel<1, 8>, kv_page_selector_kernel<1, 16>); break;
+    case 2: launch(kv_page_selector_kernel<2, 8>, kv_page_selector_kernel<2, 16>); break;
+    case 4: launch(kv_page_selector_kernel<4, 8>, kv_page_selector_kernel<4, 16>); break;
+    case 8: launch(kv_page_selector_kernel<8, 8>, kv_page_selector_kernel<8, 16>); break;
     default: return OMNI_EINVAL;
   }
   return omni_launch_status();
