@@ -1168,7 +1168,7 @@ struct DecodePlan {
 static thread_local int g_override_nsplit = 0;   // tuning hook, see omni_kv4_decode_set_split_override
 
 static DecodePlan plan_decode(int batch, int num_heads, int num_kv_heads, int max_context, int tokens_per_block,
-                              bool per_q_head = false, bool allow_g8 = false, int sweep = 32 * DEC_WAVES) {
+                              bool per_q_head = false, bool allow_g8 = false, bool fine = false) {
   DecodePlan pl;
   const int group = num_heads / num_kv_heads;
   pl.g = group >= 4 ? 4 : group;  // group in {1,2,4,8,...}
@@ -1194,14 +1194,20 @@ static DecodePlan plan_decode(int batch, int num_heads, int num_kv_heads, int ma
   int s_hi = 2048 / wgs_per_split + 1;
   if (s_hi < 2 * s_lo + 8) s_hi = 2 * s_lo + 8;
   if (s_hi > max_s) s_hi = max_s;
-  int s = s_lo;
-  long long best = -1;
-  for (int n = s_lo; n <= s_hi; ++n) {
+  const int sweep = (fine ? 64 : 32) * DEC_WAVES;
+  auto cost = [&](int n, bool whole) {
     const long long rounds = ((long long)wgs_per_split * n + OMNI_FLASH_SLOTS - 1) / OMNI_FLASH_SLOTS;
     const int st = split_tokens(n);
-    const long long cost = rounds * ((st <= sweep ? st : (st + sweep - 1) / sweep * sweep) + 192) + (sweep > 32 * DEC_WAVES ? 34 : 30) * n;
-    if (best < 0 || cost < best) { best = cost; s = n; }
+    if (!whole) return rounds * (st + 192);
+    return rounds * ((st <= sweep ? st : (st + sweep - 1) / sweep * sweep) + 192) + (fine ? 34 : 30) * n;
+  };
+  int plain = s_lo, s = s_lo;
+  for (int n = s_lo + 1; n <= s_hi; ++n) {
+    if (cost(n, false) < cost(plain, false)) plain = n;
+    if (cost(n, true) < cost(s, true)) s = n;
   }
+  // (another order of the merge's sums only where it is worth a fifth: below that the two measure the same)
+  if (!fine && 5 * cost(plain, true) <= 6 * cost(s, true)) s = plain;
   if (g_override_nsplit > 0) s = g_override_nsplit;
   if (s > max_s) s = max_s;
   if (s < 1) s = 1;
@@ -1620,7 +1626,7 @@ static int decode_fg_common(
   }
   if (span > max_context && !sparse) span = max_context;
   if (span < 1) span = 1;
-  const DecodePlan pl = plan_decode(batch, num_heads, num_kv_heads, span, tokens_per_block, sparse, false, 64 * DEC_WAVES);
+  const DecodePlan pl = plan_decode(batch, num_heads, num_kv_heads, span, tokens_per_block, sparse, false, true);
   if ((long long)pl.nsplit * pl.split_tokens < span) return OMNI_EINVAL;
   if (pl.lds_bytes > 160 * 1024) return OMNI_EINVAL;
   const size_t need = (size_t)batch * num_heads * pl.nsplit * (DH + 2) * sizeof(float);
