@@ -1168,7 +1168,7 @@ struct DecodePlan {
 static thread_local int g_override_nsplit = 0;   // tuning hook, see omni_kv4_decode_set_split_override
 
 static DecodePlan plan_decode(int batch, int num_heads, int num_kv_heads, int max_context, int tokens_per_block,
-                              bool per_q_head = false, bool allow_g8 = false, bool fine = false) {
+                              bool per_q_head = false, bool allow_g8 = false) {
   DecodePlan pl;
   const int group = num_heads / num_kv_heads;
   pl.g = group >= 4 ? 4 : group;  // group in {1,2,4,8,...}
@@ -1184,30 +1184,18 @@ static DecodePlan plan_decode(int batch, int num_heads, int num_kv_heads, int ma
   // ceil(W*s / 512) rounds of about (tokens per split + a fixed prologue/epilogue worth ~192 tokens) each; pick
   // the split count that minimises that product (a 17-way split of 64 (sequence, head) pairs was 3 rounds of 1936
   // tokens where 24 splits are 3 rounds of 1376).  A single split skips the merge kernel.
-  // The four waves sweep 128 tokens at a time (`sweep`; fine-grained instantiations 256), so a longer split costs whole sweeps; and the merge reads
-  // the splits of a head one behind another, 0.24 us each (30 tokens' worth; 0.27 where it is a launch of its own behind the fine-grained ones,
-  // whose 4096 tokens are then 8 splits, not 16: LServe's decode of 12000 tokens 1603 -> 1553 us).  Without | with both terms, us per step of 8 layers of
-  // 32 / 8 heads: one sequence of 1500 tokens 419 | 399, 3000 482 | 411 (47 splits, 12), 6000 512 | 424, 16000 525 | 465, two of 3000 515 | 463,
-  // three of 1000 503 | 487; 4 layers of 64 / 8 heads, one of 3000 677 | 614; no change for 16 and more sequences.
   int s_lo = 1;
   while (s_lo < max_s && split_tokens(s_lo) > st_cap) ++s_lo;
   int s_hi = 2048 / wgs_per_split + 1;
   if (s_hi < 2 * s_lo + 8) s_hi = 2 * s_lo + 8;
   if (s_hi > max_s) s_hi = max_s;
-  const int sweep = (fine ? 64 : 32) * DEC_WAVES;
-  auto cost = [&](int n, bool whole) {
+  int s = s_lo;
+  long long best = -1;
+  for (int n = s_lo; n <= s_hi; ++n) {
     const long long rounds = ((long long)wgs_per_split * n + OMNI_FLASH_SLOTS - 1) / OMNI_FLASH_SLOTS;
-    const int st = split_tokens(n);
-    if (!whole) return rounds * (st + 192);
-    return rounds * ((st <= sweep ? st : (st + sweep - 1) / sweep * sweep) + 192) + (fine ? 34 : 30) * n;
-  };
-  int plain = s_lo, s = s_lo;
-  for (int n = s_lo + 1; n <= s_hi; ++n) {
-    if (cost(n, false) < cost(plain, false)) plain = n;
-    if (cost(n, true) < cost(s, true)) s = n;
+    const long long cost = rounds * (split_tokens(n) + 192);
+    if (best < 0 || cost < best) { best = cost; s = n; }
   }
-  // (another order of the merge's sums only where it is worth a fifth: below that the two measure the same)
-  if (!fine && 5 * cost(plain, true) <= 6 * cost(s, true)) s = plain;
   if (g_override_nsplit > 0) s = g_override_nsplit;
   if (s > max_s) s = max_s;
   if (s < 1) s = 1;
@@ -1626,7 +1614,7 @@ static int decode_fg_common(
   }
   if (span > max_context && !sparse) span = max_context;
   if (span < 1) span = 1;
-  const DecodePlan pl = plan_decode(batch, num_heads, num_kv_heads, span, tokens_per_block, sparse, false, true);
+  const DecodePlan pl = plan_decode(batch, num_heads, num_kv_heads, span, tokens_per_block, sparse);
   if ((long long)pl.nsplit * pl.split_tokens < span) return OMNI_EINVAL;
   if (pl.lds_bytes > 160 * 1024) return OMNI_EINVAL;
   const size_t need = (size_t)batch * num_heads * pl.nsplit * (DH + 2) * sizeof(float);
