@@ -163,7 +163,11 @@ __device__ __forceinline__ void wait_stage() {
 
 // rows (at most 16 MB) of x times 16 NW channels of w, stages s0 .. s1 - 1 of k, into red [KW][16 MB][16 NW + 4]: part h of the
 // workgroup's waves takes every KW-th stage through a ring of its own
-// SHORT: k may be below CHAIN_K.  TURN: see gemm_stream_kernel.
+// SHORT: k may be below CHAIN_K.
+// TURN: rows lie whole KiBs apart, and workgroups in step ask the same channels of the memory.  So the workgroups of an XCD begin with different numbers (`early`) of
+// K's last chains of stages, whose sums wait in registers for those in front of them: the additions keep their order, and a channel's sum does not hang
+// on its place.  (MI355X, without | with: 28672 x 4096 at 48 rows 48.9 | 39.9 us, 32000 x 4096 59.7 | 43.4, 32000 x 2048 at 16 rows 25.4 | 22.9; each workgroup
+// 256 bytes further than the one before it and an order of its own, 38.5, 42.1, 21.5; at most 8 and 4 chains 40.1, 45.1, 22.4.)
 constexpr int CHAIN_K = 64 * KSTEP;
 template <int MB, int NW, int KW, bool SHORT, bool TURN>
 __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int n, int64_t k, int n0, const elem_t* x, int64_t ldx,
@@ -192,10 +196,12 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
   }
   const uint32_t base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int nst = (s1 - s0 - h + KW - 1) / KW;
-  const int turn = TURN && gridDim.z == 1 && nst > 0 ? (int)(blockIdx.x >> 3) * 2 % nst : 0;
-  auto stage = [&](int t) {                                // the t-th stage of this part
+  constexpr int EARLY = !TURN || SHORT ? 0 : NW == 5 ? (MB <= 2 ? 7 : 4) : MB <= 2 ? 15 : 7;      // (as the registers have room; of 80 channels 3 waves share a SIMD's)
+  const int early = EARLY ? max(0, min((int)(blockIdx.x >> 3) % (EARLY + 1), (nst + 3) / 4 - 3)) : 0;      // (12 stages or more stay behind them, R - 1 <= 9)
+  const int turn = early ? 4 * ((nst + 3) / 4 - early) : 0, first = early ? nst - turn : 0;      // first: stages of those chains
+  auto stage = [&](int t) {                                // the t-th stage that this part takes
     const uint32_t dst = base + (uint32_t)(t % R) * ST;
-    const int at = (!TURN || t + turn < nst ? t + turn : t + turn - nst) * (KW * RB);
+    const int at = (EARLY == 0 || t + turn < nst ? t + turn : t + turn - nst) * (KW * RB);
 #pragma unroll
     for (int i = 0; i < 2; ++i) dma16_stream(wsrc[i] + at, dst + 2048 * wave + 1024 * i);
 #pragma unroll
@@ -205,7 +211,7 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
   // the choice in it that one took 3 - 7 % more, 16 tokens of 8 of 64 x 1280 x 2048 52.8 -> 55.5 us.)
   const int chain = !SHORT || k >= CHAIN_K ? 3 : k >= CHAIN_K / 2 ? 1 : 0;
   const bool halves = SHORT && k < CHAIN_K / 4;
-  f32x4 acc[MB], total[MB];
+  f32x4 acc[MB], total[MB], later[EARLY + 1][MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) acc[m] = total[m] = zero4();
   auto end_chain = [&] {
@@ -231,19 +237,37 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
       for (int m = 0; m < MB; ++m) acc[m] = mma(a[v], b[v][m], acc[m]);
       if (v == 0 && halves) end_chain();
     }
-    if ((t & chain) == chain) end_chain();
+  };
+  auto multiply_on = [&](int t) {                          // ... of the chains that are added up at once
+    multiply(t);
+    if (((t - first) & chain) == chain) end_chain();
   };
   wait_pieces<0>();                                        // the compiler's own loads
 #pragma unroll
   for (int t = 0; t < R - 1; ++t)
     if (t < nst) stage(t);
   int t = 0;
-  for (; t + R - 1 < nst; ++t) {                           // R - 2 stages fly behind stage t
+  auto next = [&] {                                        // R - 2 stages fly behind stage t
     wait_stage<(R - 2) * P>();
     __builtin_amdgcn_s_barrier();                          // stage t is there for every wave, everyone has left stage t - 1
     asm volatile("" ::: "memory");
     stage(t + R - 1);
-    multiply(t);
+  };
+#pragma unroll
+  for (int c = 0; c < EARLY; ++c) {
+    for (const int end = c < early ? min(t + 4, first) : t; t < end; ++t) {
+      next();
+      multiply(t);
+    }
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      later[c][m] = acc[m];
+      acc[m] = zero4();
+    }
+  }
+  for (; t + R - 1 < nst; ++t) {
+    next();
+    multiply_on(t);
   }
   // the last R - 1 stages: j fly behind this one
   auto last = [&](auto jt) {
@@ -252,10 +276,15 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
     wait_stage<J * P>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    multiply(nst - 1 - J);
+    multiply_on(nst - 1 - J);
   };
   countdown<R - 2>(last);
   if (KW > 1 && nst < (s1 - s0 + KW - 1) / KW) __builtin_amdgcn_s_barrier();      // (other parts have a stage more)
+#pragma unroll
+  for (int c = 0; c < EARLY; ++c)
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+      if (c < early) total[m] += later[c][m];
   __syncthreads();                                         // the rings are free
   float* red = (float*)(lds - h * ring_bytes<NW, KW>) + h * (16 * MB * (16 * NW + 4));
 #pragma unroll
@@ -283,11 +312,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
   const int stages = pt.k * (int)sizeof(elem_t) / RB, slice = blockIdx.z, slices = gridDim.z;
   const int s0 = stages * slice / slices, s1 = stages * (slice + 1) / slices;
   const int div = is_b ? 1 : p.x_div;
-  // Rows lie whole KiBs apart: workgroups in step ask the same channels of the memory, so each begins 256 bytes further in k than the one before it on its
-  // XCD (MI355X: 28672 x 4096 at 48 rows 50.4 -> 47.0 us, 32000 x 4096 54.3 -> 49.8, 32000 x 2048 at 16 rows 26.3 -> 22.7).  Heads and wide dense gated units
-  // only: the sums' order changes with it, and what a router reads keeps its order, so that near ties choose as they did (experts would gain 3 %: 16 tokens
-  // of 8 of 64 x 1280 x 2048 54.2 -> 52.6); K slices begin at places of their own (4096 x 14336 in 4 of them 24.7, turned 25.3).
-  constexpr bool TURN = EPI == LM_EPI_F32 || (EPI == LM_EPI_GLU && NW == 8);
+  constexpr bool TURN = EPI == LM_EPI_F32 || (EPI == LM_EPI_GLU && NW == 8);      // heads and wide dense gated units
   for (int m0 = 0; m0 < rows; m0 += 64) {
     const int here = min(64, rows - m0), mb = (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
@@ -680,8 +705,8 @@ static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s
 // was measured the channels per workgroup matter most where n / 64 is far from a multiple of 256 (10816 x 4096, 48 rows: 26.5 us at 64,
 // 20.8 at 48; 4096 x 4096, 16 rows: 11.8 us at 64 and 4 slices, 9.8 at 16), slices where K is long (4096 x 14336, 48 rows: 40 us, 26
 // with 4).  128 channels, bf16: 2.5 us for a ring of 144 KiB that nothing runs beside, but x comes in half as often, and 224 or 250 workgroups are one round where 448
-// or 500 are two (28672 x 4096, 64 / 128 channels: 1 row 38.0 / 37.3 us, 48 rows 45.5 / 38.2, 64 rows 47.4 / 39.3; 32000 x 4096, 48 rows 45.2 / 42.9;
-// 32000 x 2048, 16 rows 22.0 / 24.3; 96 and 112 channels nowhere the fastest).
+// or 500 are two (heads and gated units, whose workgroups begin with different chains; 28672 x 4096, 64 / 128 channels: 16 rows 42.3 / 37.1 us, 48 rows 48.3 / 39.9, 64
+// rows 51.8 / 41.5; 32000 x 4096, 80 / 128: 48 rows 52.0 / 43.4; 32000 x 2048, 16 rows 25.4 / 22.9; 96 and 112 channels nowhere the fastest).
 struct RowsPlan {
   int nw, slices;      // nw 0: gemm_rows_kernel
 };
@@ -689,16 +714,20 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
   RowsPlan best{4, 1};
   float time = 1e30f;
   const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
-  for (int nw = LM_ELEM ? 5 : 8; nw >= 1; --nw) {
-    if (nw == 6 || nw == 7 || (glu && nw % 4)) continue;   // (a gate block and its up block share a workgroup)
+  for (int nw = 5; nw >= 1; --nw) {
+    if (glu && nw != 4) continue;                          // (a gate block and its up block share a workgroup)
     const int64_t tiles = (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw));
     for (int s = 1; s <= (sliced ? 8 : 1) && (s == 1 || stages >= 4 * s); s *= 2) {
       float t = (float)((tiles * s + 255) / 256) * (float)((stages + s - 1) / s) * (0.07f * nw + 0.02f * mb + 0.02f);
-      if (nw == 8) t += 2.5f;
       if (s > 1) t += 4.5f + (float)s * rows * n * 8.f / 5e6f;
       if (t < time) { time = t; best = RowsPlan{nw, s}; }
     }
   }
+  // 128 channels only in place of workgroups that take K in one chain of stages, as they do: the same order of sums
+  auto tiles = [&](int nw) { return (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw)); };
+  if (LM_ELEM == 0 && best.slices == 1 && tiles(best.nw) > 256 &&
+      (float)((tiles(8) + 255) / 256) * (float)stages * (0.07f * 8 + 0.02f * mb + 0.02f) + 2.5f < time)
+    best.nw = 8;
   return best;
 }
 
@@ -715,6 +744,9 @@ static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, 
 
 template <int EPI, int NW>
 static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+  if constexpr (EPI == LM_EPI_F32) {      // (slices begin at places of their own, and what they leave is the same)
+    if (slices > 1) return launch_stream_tiles<LM_EPI_ELEM, NW>(a, n, has_b, slices, part, s);
+  }
   if (a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K)) launch_stream_form<EPI, NW, true>(a, n, has_b, slices, part, s);
   else launch_stream_form<EPI, NW, false>(a, n, has_b, slices, part, s);
 }

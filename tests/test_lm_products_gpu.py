@@ -342,3 +342,29 @@ def test_sums_of_the_stream_are_as_exact(n, k, dtype):
     assert _rows_plan(ops, 1, n, k, m)[0] > 0 and x.data_ptr() % 16 == 0 and inside.data_ptr() % 16 == 8
     stream, plain = ((ops.matmul(a, w, out_f32=True).double() - want).norm().item() for a in (x, inside))
     assert 0 < stream < 1.02 * plain, (stream / want.norm().item(), plain / want.norm().item())
+
+
+# experts of a router (16 channels a workgroup), heads of 80 and of 128 channels a workgroup, in K parts and in slices
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("m,n,k", [(1, 256, 2048), (16, 512, 2048), (48, 512, 1024), (3, 4096, 4096), (5, 16448, 2048), (48, 32000, 4096), (1, 32768, 2048)])
+def test_equal_channels_have_equal_sums(m, n, k, dtype):
+    """A channel's sum does not hang on its place: experts or words with the same weights are as likely as each other."""
+    ops = _ops(dtype)
+    x, w = _randn(41, dtype, m, k), _randn(42, dtype, 32, k).repeat(n // 32, 1)
+    y = ops.matmul(x, w, out_f32=True).view(m, n // 32, 32)
+    assert torch.equal(y, y[:, :1].expand_as(y))
+
+
+def test_equal_channels_have_equal_gated_units():
+    """... nor does a gated unit of 128 channels a workgroup"""
+    ops, m, n, k = _ops(torch.bfloat16), 48, 28672, 4096
+    assert _rows_plan(ops, 1, n, k, m, 2) == (128, 1)
+    y = ops.glu(_randn(43, torch.bfloat16, m, k), _randn(44, torch.bfloat16, 32, k).repeat(n // 32, 1), None, "silu").view(m, n // 32, 16)
+    assert torch.equal(y, y[:, :1].expand_as(y))
+
+
+@pytest.mark.parametrize("epi,n,k,m,narrow", [(0, 43536, 4096, 1, (80, 4)), (0, 28688, 8192, 1, (80, 2)), (0, 11136, 14336, 49, (48, 1)), (0, 16384, 28672, 64, (64, 1)),
+                                               (2, 34848, 4096, 1, (64, 4)), (2, 57376, 4096, 1, (64, 8))])
+def test_128_channels_keep_the_order_of_sums(epi, n, k, m, narrow):
+    """Workgroups of 128 channels take K in one chain of stages: they stand in for narrower ones that do, too, not for those with K slices or K parts."""
+    assert _rows_plan(_ops(torch.bfloat16), 1, n, k, m, epi) == narrow
