@@ -5,10 +5,11 @@
 // the address path takes at 15 bytes a clock).  A workgroup has 64 channels; a stage is 128 bytes of k of them and of the rows, consumed behind one
 // barrier while as many more as 64 KiB hold are on their way; two workgroups to a compute unit.  The logits stay inside: a workgroup leaves one key a row.
 //
-// MI355X, with the argmax, against the vendor's product and omni_argmax_f16: 32000 x 4096 60.3 - 62.0 -> 43.6 - 44.2 us (1 - 16 rows; 6.3 TB/s without the launch that
-// finishes), 58.9 -> 52 (64 rows); 16000 x 8192 54.7 -> 45.5, at 64 rows no faster.
+// MI355X, with the argmax, against the vendor's product and omni_argmax_f16: 32000 x 4096 61.0 - 62.5 -> 42.8 us (1 - 16 rows; 6.4 TB/s without the launch that
+// finishes), 61.9 -> 53.4 (64 rows); 16000 x 8192 55 - 56 -> 49, at 64 rows no faster.
 //
-// f32 sums of 256 products each, added up: no further from 64 bits than one chain.
+// f32 sums of 256 products each, added up in the order of k: no further from 64 bits than one chain, and the same for equal weights wherever they stand, so that the first
+// of equal rows is the one that is found.
 #include "qgemm_kernel.h"
 #include "argmax_key.h"
 
@@ -42,6 +43,7 @@ __global__ __launch_bounds__(256) void head_argmax_kernel(HeadArgs p) {
   constexpr int MB = (EIGHTS + 1) / 2, W_BYTES = HEAD_CHANNELS * 128, STAGE = W_BYTES + EIGHTS * 1024;
   constexpr int XP = (EIGHTS + 3) / 4, P = 2 + XP;            // pieces of x, and all, that a wave requests for a stage (some of x twice: the same bytes)
   constexpr int R = (64 << 10) / STAGE;
+  constexpr int EARLY = MB <= 2 ? 15 : 7;                     // as the registers have room
   static_assert((R - 2) * P <= 63, "vmcnt");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[R * STAGE];
   __shared__ unsigned long long best[4][16 * MB];
@@ -64,9 +66,11 @@ __global__ __launch_bounds__(256) void head_argmax_kernel(HeadArgs p) {
   const uint8_t* const wbase = reinterpret_cast<const uint8_t*>(p.w + (size_t)n0 * p.K);
   const uint8_t* const xbase = reinterpret_cast<const uint8_t*>(p.x);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds);
-  // rows lie whole KiBs apart: workgroups in step would all ask the same channels of the memory, so each begins at another k (MI355X, 1 and 16 rows, with and
-  // without: 32000 x 4096 43.6 and 49.8 us, 16000 x 8192 45 - 46 and 54 - 55; 256 bytes apart instead of 640 44 and 47)
-  const int turn = (int)(blockIdx.x >> 3) * 5 % nst;
+  // Rows lie whole KiBs apart: workgroups in step would all ask the same channels of the memory, so they begin with different numbers (`early`) of K's last chains,
+  // whose sums wait for those in front of them.  (MI355X, 1 and 16 rows, at most 1, 4, 8, 15 chains: 32000 x 4096 50.7, 44 - 47, 43 - 46, 42 - 45 us, 128256 x 4096
+  // 186 - 192, 174 - 179, 169 - 172, 164; beginning 640 bytes apart with orders of their own 44 and 166.  64 rows, 7 and 15 chains: 52 and 61.)
+  const int chains = (nst + HEAD_CHAIN - 1) / HEAD_CHAIN, early = max(0, min((int)(blockIdx.x >> 3) % (EARLY + 1), chains - 3));
+  const int turn = early ? HEAD_CHAIN * (chains - early) : 0, first = early ? nst - turn : 0;      // first: stages of those chains
   auto stage = [&](int t) {
     const size_t at = (size_t)(t + turn < nst ? t + turn : t + turn - nst) * 128;
     const uint32_t dst = lds0 + (uint32_t)(t % R) * STAGE;
@@ -82,7 +86,7 @@ __global__ __launch_bounds__(256) void head_argmax_kernel(HeadArgs p) {
   uint32_t xoff[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) xoff[h] = EIGHTS == 1 ? (uint32_t)(l15 & 7) * 128 + (((4 * h + l4) ^ tiles_swizzle(l15 & 7)) << 4) : off[h];
-  v4f acc[MB], total[MB];
+  v4f acc[MB], total[MB], later[EARLY][MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) acc[m] = total[m] = (v4f){0.f, 0.f, 0.f, 0.f};
   auto multiply = [&](int t) {
@@ -95,29 +99,55 @@ __global__ __launch_bounds__(256) void head_argmax_kernel(HeadArgs p) {
       for (int m = 0; m < MB; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, *reinterpret_cast<const f16x8*>(xt + 2048 * m + xoff[h]), acc[m], 0, 0, 0);
     }
-    if ((t & (HEAD_CHAIN - 1)) == HEAD_CHAIN - 1) {
-#pragma unroll
-      for (int m = 0; m < MB; ++m) {
-        total[m] += acc[m];
-        acc[m] = (v4f){0.f, 0.f, 0.f, 0.f};
-      }
-    }
   };
 #pragma unroll
   for (int t = 0; t < R - 1; ++t)
     if (t < nst) stage(t);
   int t = 0;
-  for (; t + R - 1 < nst; ++t) {
+  auto step = [&] {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * P) : "memory");
     __builtin_amdgcn_s_barrier();                             // stage t is there for every wave, everyone has left stage t - 1
     asm volatile("" ::: "memory");
     stage(t + R - 1);
     multiply(t);
+    ++t;
+  };
+#pragma unroll
+  for (int c = 0; c < EARLY; ++c) {
+    const int end = c < early ? min(t + HEAD_CHAIN, first) : t;
+    while (t < end) step();                                   // (more than R - 1 stages follow)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      later[c][m] = acc[m];
+      acc[m] = (v4f){0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  auto end_chain = [&] {                                      // ... behind stage t - 1
+    if (((t - first) & (HEAD_CHAIN - 1)) != 0) return;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      total[m] += acc[m];
+      acc[m] = (v4f){0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  while (t + R - 1 < nst) {
+    step();
+    end_chain();
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();                               // the rest is there
   asm volatile("" ::: "memory");
-  for (; t < nst; ++t) multiply(t);
+  while (t < nst) {
+    multiply(t++);
+    end_chain();
+  }
+#pragma unroll
+  for (int m = 0; m < MB; ++m) total[m] += acc[m];
+#pragma unroll
+  for (int c = 0; c < EARLY; ++c) {
+    for (int m = 0; m < MB; ++m)
+      if (c < early) total[m] += later[c][m];
+  }
 
   // the lane's four channels of row l15 of each block
 #pragma unroll
@@ -126,7 +156,7 @@ __global__ __launch_bounds__(256) void head_argmax_kernel(HeadArgs p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int n = n0 + 16 * wave + 4 * l4 + e;
-      const half_t h = (half_t)(total[m][e] + acc[m][e]);
+      const half_t h = (half_t)total[m][e];
       const unsigned long long k = n < p.V ? argmax_key(__builtin_bit_cast(uint16_t, h), n) : 0;
       key = k > key ? k : key;
     }

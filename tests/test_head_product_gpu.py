@@ -41,3 +41,21 @@ def test_head_argmax_takes_the_first_of_equal_logits_and_nan_as_the_largest():
     w[131] = -0.0                                            # (and 0 from below: -0 == +0)
     fused_ext.head_argmax(out, x, w)
     assert out.tolist() == [131, 131]
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 64])
+@pytest.mark.parametrize("V,K", [(32000, 4096), (9000, 448), (16000, 8192)])
+def test_head_argmax_takes_the_first_of_equal_rows(M, V, K):
+    """Words with the same weights have the same logit wherever they stand: sums of cancelling products, whose f32 rounding is far above the fp16 logit's"""
+    from omniserve_amd.backend import fused_ext
+    w = torch.empty((V, K), dtype=torch.float16, device=dev())
+    out = torch.empty((M,), dtype=torch.int64, device=dev())
+    for seed in range(12):
+        g = torch.Generator(device=dev()).manual_seed(seed)
+        x = torch.randn((K,), generator=g, device=dev()) + 1.0
+        r = torch.randn((K,), generator=g, device=dev())
+        r = (r - (r @ x) / (x @ x) * x).half()
+        w.fill_(-1.0)
+        w[[100, 5000, V - 1]] = r
+        fused_ext.head_argmax(out, x.half().repeat(M, 1), w)
+        assert out.tolist() == [100] * M, seed
