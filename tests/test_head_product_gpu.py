@@ -59,3 +59,18 @@ def test_head_argmax_takes_the_first_of_equal_rows(M, V, K):
         w[[100, 5000, V - 1]] = r
         fused_ext.head_argmax(out, x.half().repeat(M, 1), w)
         assert out.tolist() == [100] * M, seed
+
+
+@pytest.mark.parametrize("M", [1, 5])
+def test_head_argmax_of_strided_operands(M):
+    """A head that is a view -- transposed, or columns of something wider -- goes through torch.matmul."""
+    from omniserve_amd.backend import fused_ext
+    g = torch.Generator(device=dev()).manual_seed(M)
+    out = torch.empty((M,), dtype=torch.int64, device=dev())
+    for x, w in ((torch.randn((M, 256), generator=g, device=dev()).half(), torch.randn((256, 700), generator=g, device=dev()).half().t()),
+                 (torch.randn((M, 320), generator=g, device=dev()).half()[:, 64:], torch.randn((700, 320), generator=g, device=dev()).half()[:, :256])):
+        fused_ext.head_argmax(out, x, w)
+        logits = x.double() @ w.double().T
+        top = logits.amax(dim=1)
+        # fp16 logits, that of the largest and that of the chosen one (2^-11 each)
+        assert torch.all(top - logits.gather(1, out[:, None])[:, 0] <= 2.0 ** -10 * top.abs() + 1e-5)
