@@ -313,6 +313,7 @@ int omni_argmax_f16(void* out_i64, const void* logits_f16, int64_t row_stride, i
 /* The greedy head in one: out[r] = omni_argmax_f16 of the fp16 logits x[r, :] w^T (fp16 x [M, K], w [V, K]; f32 sums, in one order for all rows of w), which are not stored.  x and w 16-byte
  * aligned; omni_head_argmax_workspace_bytes = 0: not its size (M <= 64, K % 64 == 0). */
 size_t omni_head_argmax_workspace_bytes(int M, int V, int K);
+int omni_head_argmax_faster(int M, int V, int K);      /* 1: faster than a product and omni_argmax_f16 */
 int omni_head_argmax_f16(void* out_i64, const void* x_f16, const void* w_f16, int M, int V, int K, void* workspace, size_t workspace_bytes,
                          void* stream);
 

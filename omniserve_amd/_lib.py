@@ -97,6 +97,7 @@ PROTOTYPES = {
     "omni_gather_rows_f16": (_i, [_vp, _vp, _vp, _i, _i, _i64, _vp]),
     "omni_argmax_workspace_bytes": (_sz, [_i]),
     "omni_head_argmax_workspace_bytes": (_sz, [_i, _i, _i]),
+    "omni_head_argmax_faster": (_i, [_i, _i, _i]),
     "omni_head_argmax_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp, _sz, _vp]),
     "omni_argmax_f16": (_i, [_vp, _vp, _i64, _i, _i, _vp, _sz, _vp]),
     "omni_kv4_prefill_write_fine_grained": (_i, [_vp] * 7 + [_i] * 15 + [_vp, _i, _i, _vp]),

@@ -445,19 +445,18 @@ def argmax(out, logits):
 
 
 def head_argmax(out, x, weight):
-    """out int64 [rows] = argmax of the fp16 logits x @ weight.T: few contiguous rows in one product that keeps its logits to itself (csrc/head_product.hip),
-    others through torch.matmul and argmax."""
+    """out int64 [rows] = argmax of the fp16 logits x @ weight.T: in one product that keeps its logits to itself (csrc/head_product.hip) for contiguous operands of
+    sizes where that is the faster way, others through torch.matmul and argmax."""
     _lib.require_cuda(out, x, weight)
     if any(t.dtype != torch.float16 or t.dim() != 2 for t in (x, weight)) or x.shape[1] != weight.shape[1]:
         raise RuntimeError("head_argmax: fp16 x [rows, hidden] and weight [vocab, hidden] expected")
     if out.dtype != torch.int64 or out.numel() != x.shape[0] or not out.is_contiguous():
         raise RuntimeError("head_argmax: out must be a contiguous int64 [rows] tensor")
     (M, K), V = x.shape, weight.shape[0]
-    need = _lib.lib().omni_head_argmax_workspace_bytes(M, V, K)
-    if need == 0 or (x.data_ptr() | weight.data_ptr()) % 16 or not x.is_contiguous() or not weight.is_contiguous():
+    if not _lib.lib().omni_head_argmax_faster(M, V, K) or (x.data_ptr() | weight.data_ptr()) % 16 or not x.is_contiguous() or not weight.is_contiguous():
         argmax(out, torch.matmul(x, weight.t()))
         return
-    ws = _lib.workspace(need, x.device, "argmax")
+    ws = _lib.workspace(_lib.lib().omni_head_argmax_workspace_bytes(M, V, K), x.device, "argmax")
     rc = _lib.lib().omni_head_argmax_f16(out.data_ptr(), x.data_ptr(), weight.data_ptr(), M, V, K, ws.data_ptr(), ws.numel(), _lib.current_stream())
     _lib.check(rc, "fused_ext.head_argmax")
 

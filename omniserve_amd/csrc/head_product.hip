@@ -205,6 +205,18 @@ extern "C" size_t omni_head_argmax_workspace_bytes(int M, int V, int K) {
   return (size_t)M * head_groups(V) * sizeof(unsigned long long);
 }
 
+// Where this measured faster than the vendor's product and omni_argmax_f16 (MI355X, 13 vocabularies of 500 - 64000 x 9 K of 512 - 8192, us, this | those).  A workgroup
+// alone takes 5 us for 1024 of K, whatever V: 500 x 4096 21 | 13, 8000 x 4096 23 | 22 at 1 row, 31 | 24 at 64; 10000 x 4096 23 | 25 and 31 | 32; 4000 x 2048 14 | 14.  The
+// vendor's product loses where rows lie whole 4 KiBs apart and is good where they do not: 17 rows and more, 32000 x 5120 61 | 63 and 71 | 65, 50000 x 5120 108 | 96 and
+// 129 | 102, 24000 x 3072 41 | 38 at 64 rows; x 4096 54 | 60, 94 | 87, 50 | 54.
+extern "C" int omni_head_argmax_faster(int M, int V, int K) {
+  if (omni_head_argmax_workspace_bytes(M, V, K) == 0) return 0;
+  const bool many = M > 32;
+  if (M > 16 && K % 2048 != 0 && K > (many ? 1024 : 4096)) return 0;
+  if (K <= (many ? 1024 : 2048)) return V >= (many ? 2 : 1) * K;
+  return V >= (many ? (K <= 2048 ? 10000 : 16000) : (K <= 4096 ? 10000 : 12000));
+}
+
 extern "C" int omni_head_argmax_f16(void* out_i64, const void* x_f16, const void* w_f16, int M, int V, int K, void* workspace, size_t workspace_bytes,
                                     void* stream) {
   const size_t need = omni_head_argmax_workspace_bytes(M, V, K);
