@@ -662,10 +662,8 @@ extern "C" int lm_delta_decode(const void* x, int64_t ld, void* o, int64_t ldo, 
   hipStream_t s = (hipStream_t)stream;
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
-    if (streams_state(B, H, K, V))                                                                           \
-      hipLaunchKernelGGL((delta_decode_kernel<K, V, true>), dim3(H, B), dim3(4 * V), 0, s, a);               \
-    else                                                                                                     \
-      hipLaunchKernelGGL((delta_decode_kernel<K, V, false>), dim3(H, B), dim3(4 * V), 0, s, a);              \
+    const auto run = streams_state(B, H, K, V) ? delta_decode_kernel<K, V, true> : delta_decode_kernel<K, V, false>; \
+    in_places(a, B, [&](const DeltaDecodeArgs& p, int n) { hipLaunchKernelGGL(run, dim3(H, n), dim3(4 * V), 0, s, p); }); \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)

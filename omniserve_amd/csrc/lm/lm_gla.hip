@@ -467,10 +467,8 @@ extern "C" int lm_gla_decode(const void* x, int64_t ld, void* o, int64_t ldo, fl
   hipStream_t s = (hipStream_t)stream;
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
-    if (streams_state(B, H, K, V))                                                                           \
-      hipLaunchKernelGGL((gla_decode_kernel<K, V, true>), dim3(H, B), dim3(4 * V), 0, s, a);                 \
-    else                                                                                                     \
-      hipLaunchKernelGGL((gla_decode_kernel<K, V, false>), dim3(H, B), dim3(4 * V), 0, s, a);                \
+    const auto run = streams_state(B, H, K, V) ? gla_decode_kernel<K, V, true> : gla_decode_kernel<K, V, false>; \
+    in_places(a, B, [&](const GlaDecodeArgs& p, int n) { hipLaunchKernelGGL(run, dim3(H, n), dim3(4 * V), 0, s, p); }); \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)

@@ -8,6 +8,7 @@
 // Long portions are cut into segments that run in parallel: a first pass forms what each segment adds to the state, the second
 // starts every segment from the decayed sum of those before it.
 #include "lm_common.h"
+#include "lm_state.h"
 #include "omniserve_lm.h"
 
 namespace lm {
@@ -333,7 +334,9 @@ extern "C" int lm_linear_decode(const void* x, int64_t ld, void* o, int64_t ldo,
                                 const float* log2_decay, int B, int H, int dk, int dv, int act, void* stream) {
   if (B <= 0 || H <= 0 || (dk != 64 && dk != 128 && dk != 256) || (dv != 64 && dv != 128 && dv != 256) || ld % 4 || ldo % 4)
     return LM_EINVAL;
-  hipLaunchKernelGGL(linear_decode_kernel, dim3(H, B), dim3(256), 0, (hipStream_t)stream, (const elem_t*)x, ld, (elem_t*)o, ldo, state,
-                     slot, pos, log2_decay, H, dk, dv, act);
+  struct Args { const elem_t* x; int64_t ld; elem_t* o; int64_t ldo; const int *slot, *pos; };
+  in_places(Args{(const elem_t*)x, ld, (elem_t*)o, ldo, slot, pos}, B, [&](const Args& a, int n) {
+    hipLaunchKernelGGL(linear_decode_kernel, dim3(H, n), dim3(256), 0, (hipStream_t)stream, a.x, ld, a.o, ldo, state, a.slot, a.pos, log2_decay, H, dk, dv, act);
+  });
   return launch_status();
 }

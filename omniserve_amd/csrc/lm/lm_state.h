@@ -5,6 +5,20 @@
 
 namespace lm {
 
+// A grid's second dimension, the places of the batch, ends at 65535: more go in launches of their own (a third dimension and its test in the kernel: a step of one
+// sequence 4.1 -> 4.3 us).  a: the kernel's arguments, of which x, o, slot and pos go from place to place.
+constexpr int STATE_PLACES = 32768;
+template <typename Args, typename Launch>
+static void in_places(Args a, int B, Launch launch) {
+  for (; B > 0; B -= STATE_PLACES) {
+    launch(a, min(B, STATE_PLACES));
+    a.x += STATE_PLACES * a.ld;
+    a.o += STATE_PLACES * a.ldo;
+    a.slot += STATE_PLACES;
+    a.pos += STATE_PLACES;
+  }
+}
+
 // The recurrent state of a decode step, read and written once.  From 16 MB on (half of the L2s) it is not kept there: what it would push out is read
 // again.  (MI355X, heads of 128 x 128, kept / not, 300 MB of other reads in front: 8 MB 10.1 / 9.6 us gated, 12.7 / 12.1 delta rule; 16 MB 12.7 / 11.4 and
 // 15.4 / 13.7; 32 MB 20.2 / 17.0 and 23.1 / 19.7; 64 MB 34.1 / 29.0 and 39.3 / 35.6; a state still in the caches, heads of 256 x 256: 4 MB 10.2 / 12.1,

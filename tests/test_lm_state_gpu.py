@@ -46,3 +46,37 @@ def test_streamed_state(layer, batch, heads, dk, dv, positions):
     torch.cuda.synchronize()
     assert torch.equal(whole, split) and torch.equal(one, parts) and torch.equal(one_ring, parts_ring)
     assert not torch.equal(one, state) and whole.float().abs().sum() > 0
+
+
+@pytest.mark.parametrize("layer", ["linear", "gla", "delta"])
+def test_more_than_65535_places(layer):
+    """A batch of mostly empty places, the last of them beyond what the second dimension of a grid may count: the sequences in it as in a batch of their own."""
+    from omniserve_amd.backend.lm import lm_ops
+    ops = lm_ops(torch.bfloat16)
+    batch, dk, dv = 65600, 64, 64
+    rows = [0, 65535, batch - 1]
+    gen = torch.Generator(device=dev()).manual_seed(5)
+    rnd = lambda *shape: torch.randn(*shape, device=dev(), generator=gen)      # noqa: E731
+    qkv = 2 * dk + dv
+    few, st0, rg0 = rnd(3, qkv + dv + 64).bfloat16(), rnd(3, 1, dk, dv) * 0.1, rnd(3, 4, qkv)
+    x = torch.zeros((batch, few.shape[1]), dtype=torch.bfloat16, device=dev())
+    x[rows] = few
+    pos, slot = torch.full((batch,), -1, dtype=torch.int32, device=dev()), torch.zeros((batch,), dtype=torch.int32, device=dev())
+    pos[rows], slot[rows] = 2, torch.arange(3, dtype=torch.int32, device=dev())
+    w, a2, bias, conv, a_log, dt_bias, decay = rnd(dv), rnd(dk, 16).bfloat16() * 0.1, rnd(dk), rnd(4, qkv) * 0.5, rnd(1), rnd(1), -rnd(1).abs()
+
+    def run(xs, sl, ps):
+        o, st, rg = torch.zeros((xs.shape[0], dv), dtype=torch.bfloat16, device=dev()), st0.clone(), rg0.clone()
+        if layer == "linear":
+            ops.linear_decode(xs, o, st, sl, ps, decay, 1, dk, dv, "silu")
+        elif layer == "gla":
+            ops.gla_decode(xs, o, st, sl, ps, qkv + dv, a2, bias, 16.0, dk ** -0.5, qkv, w, dv, 1e-6, 1, dk, dv)
+        else:
+            ops.delta_decode(xs, o, st, rg, sl, ps, conv, 1e-6, dk ** -0.5, qkv + dv, a_log, dt_bias, qkv, w, dv, 1e-6, 1, 1, dk, dv)
+        torch.cuda.synchronize()
+        return o, st, rg
+
+    o, *after = run(x, slot, pos)
+    want, *want_after = run(few, slot[rows].contiguous(), pos[rows].contiguous())
+    assert torch.equal(o[rows], want) and not o[1:65535].any()
+    assert all(torch.equal(a, b) for a, b in zip(after, want_after))
