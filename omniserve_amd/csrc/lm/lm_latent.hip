@@ -282,12 +282,14 @@ static int launch_blocks(const LatentDecodeArgs& a, int B, hipStream_t s) {
   return launch_status();
 }
 
-// 16 heads a workgroup while all of those are on the chip at once (two a CU for 16-bit rows of 512 + 64): a workgroup is a chain of short steps, and each is half as long; 32 heads read
-// the keys once (MI355X, 32 heads, without splits, 32 | 16 heads a workgroup, us: 48 sequences of 150 keys 17.2 | 14.0, of 400 30.9 | 24.7; 128 of 900, two
-// splits, 54 | 52; 256 of 30 11.9 | 13.4, of 400 38.7 | 36.1, of 2000 167 | 156; 288 of 150 26.0 | 31.7, of 1500 142 | 195).
+// 16 heads a workgroup while all of those are on the chip at once, three a CU at most: a workgroup is a chain of short steps, and each is half as long; 32 heads read
+// the keys once, which is worth more where four and more share a CU's memory path (MI355X, 32 heads, rows of 16 bits, without splits, 32 | 16 heads a workgroup, us, by latent
+// columns: 512, 48 sequences of 150 keys 18.5 | 14.8, of 400 37.1 | 30.4, 256 of 30 11.7 | 13.3, of 400 42.9 | 40.4, of 1500 124 | 115; 256, 384 of 30 10.6 | 11.2, of 84
+// 15.3 | 14.2, of 1500 86.3 | 88.7; 128, 384 of 400 24.7 | 24.0, 512 of it 26.4 | 28.2, 768 of it 34.3 | 47.1; 64, 384 of 400 22.0 | 20.1, 512 of it 22.6 | 23.8, 1024
+// of it 34.5 | 42.2).
 template <int RP, int TP>
 static int launch(const LatentDecodeArgs& a, int B, hipStream_t s) {
-  constexpr int64_t AT_ONCE = 256 * ((160 * 1024) / (int)(LatentGeom<RP, TP, 1>::LDS + 64));
+  constexpr int BY_LDS = (160 * 1024) / (int)(LatentGeom<RP, TP, 1>::LDS + 64), AT_ONCE = 256 * (BY_LDS < 3 ? BY_LDS : 3);
   return a.H <= 16 || (int64_t)B * ((a.H + 15) / 16) * a.nsplit <= AT_ONCE ? launch_blocks<RP, TP, 1>(a, B, s) : launch_blocks<RP, TP, 2>(a, B, s);
 }
 

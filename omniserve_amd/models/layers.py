@@ -438,7 +438,7 @@ class LatentAttention(Mixer):
         return ops.matmul(o, self.w_out)
 
     def splits(self, b) -> int:
-        """Parts of the keys per (sequence, 32 heads): a workgroup per CU, two if each gets 1024 keys; at least 256 keys each (a part
+        """Parts of the keys per (sequence, 32 heads, as one workgroup or as two of 16): a workgroup per CU, two if each gets 1024 keys; at least 256 keys each (a part
         leaves a latent of f32 per head)."""
         groups, keys = max(b.n_decode * ((self.s.heads + 31) // 32), 1), b.max_context
         return max(1, min(max(256 // groups, min(512 // groups, keys // 1024)), keys // 256, 64))
