@@ -368,17 +368,17 @@ struct GlaDecodeArgs {
   int n;
   float eps;
   int H;
+  bool heads_first;      // over the grid
 };
 
-// Bound by the states read and written.  Heads vary first over the grid: neighbouring workgroups take neighbouring states, where sequences first would have
-// them all a slot apart, on the same memory channels at a time (48 sequences of 32 heads x 128 x 128, 201 MB: 46.3 -> 40.6 us, 5.0 TB/s).
+// Bound by the states read and written (48 sequences of 32 heads x 128 x 128, 201 MB: 40.6 us, 5.0 TB/s).
 template <int DK, int DV, bool STREAM>
 __global__ __launch_bounds__(4 * DV) void gla_decode_kernel(GlaDecodeArgs p) {
   constexpr int TH = 4 * DV, COLS = DV / 4, ROWS = DK / STATE_GROUPS;
   static_assert(TH == COLS * STATE_GROUPS, "layout");
   __shared__ float qs[DK], ks[DK], as[DK];
   __shared__ f32x4 red[STATE_GROUPS][COLS];
-  const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
+  const int h = p.heads_first ? blockIdx.x : blockIdx.y, b = p.heads_first ? blockIdx.y : blockIdx.x, tid = threadIdx.x, col = tid % COLS, grp = tid / COLS;
   const int ps = p.pos[b];
   if (ps < 0) return;
   const elem_t* row = p.x + (int64_t)b * p.ld;
@@ -463,12 +463,12 @@ extern "C" int lm_gla_decode(const void* x, int64_t ld, void* o, int64_t ldo, fl
   if (B <= 0 || H <= 0 || n <= 0 || n > dv || ld % FR || ldo % 4 || low_col % FR || g_col % 4 || rp <= 0 || rp % FR || !(inv_tau > 0.f))
     return LM_EINVAL;
   GlaDecodeArgs a{(const elem_t*)x, ld, (elem_t*)o, ldo, state, slot, pos, low_col, (const elem_t*)a2, bias, rp, inv_tau, scale, g_col, w,
-                  n, eps, H};
+                  n, eps, H, heads_first(B, H)};
   hipStream_t s = (hipStream_t)stream;
 #define LM_CASE(K, V)                                                                                        \
   if (dk == K && dv == V) {                                                                                  \
     const auto run = streams_state(B, H, K, V) ? gla_decode_kernel<K, V, true> : gla_decode_kernel<K, V, false>; \
-    in_places(a, B, [&](const GlaDecodeArgs& p, int n) { hipLaunchKernelGGL(run, dim3(H, n), dim3(4 * V), 0, s, p); }); \
+    in_places(a, B, [&](const GlaDecodeArgs& p, int n) { hipLaunchKernelGGL(run, state_grid(p, n), dim3(4 * V), 0, s, p); }); \
     return launch_status();                                                                                  \
   }
   LM_CASE(64, 64) LM_CASE(64, 128) LM_CASE(64, 256) LM_CASE(128, 64) LM_CASE(128, 128) LM_CASE(128, 256)

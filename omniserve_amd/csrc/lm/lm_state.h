@@ -5,7 +5,15 @@
 
 namespace lm {
 
-// A grid's second dimension, the places of the batch, ends at 65535: more go in launches of their own (a third dimension and its test in the kernel: a step of one
+// Heads or places of the batch first over the grid.  Heads first, neighbouring workgroups take neighbouring states, where places first have them a slot apart, on the
+// same memory channels at a time; but while all workgroups are on the chip at once, places first are as fast or faster.  (MI355X, heads of 128 x 128 in the steps of a
+// model, us, gated / delta rule, places | heads first: 128 heads in all 7.4 | 7.4 / 9.1 | 9.1, 256 9.1 | 9.2 / 10.2 | 10.8, 384 11.8 | 13.1 / 12.6 | 12.2, 512 14.2 | 14.0 / 15.2 |
+// 15.6, 768 21.8 | 19.8 / 23.7 | 20.4, 1536 45 | 40.6 / 44 | 40.6.)
+static inline bool heads_first(int64_t B, int H) { return B * H > 512; }
+template <typename Args>
+static inline dim3 state_grid(const Args& a, int places) { return a.heads_first ? dim3(a.H, places) : dim3(places, a.H); }
+
+// A grid's second dimension, which may be the places of the batch, ends at 65535: more go in launches of their own (a third dimension and its test in the kernel: a step of one
 // sequence 4.1 -> 4.3 us).  a: the kernel's arguments, of which x, o, slot and pos go from place to place.
 constexpr int STATE_PLACES = 32768;
 template <typename Args, typename Launch>
