@@ -492,6 +492,20 @@ def _mode_and_weights(lin):
     return 1, lin.qweight, lin.s1_scales, None, lin.s2_zeros, lin.s2_scales
 
 
+def _want(what, ok):
+    if not ok:
+        raise RuntimeError(what)
+
+
+def _rows(t, n, dtype=torch.float16):
+    """a contiguous tensor of at least n values"""
+    return t is not None and t.dtype == dtype and t.is_contiguous() and t.numel() >= n
+
+
+def _lin_k(mode, w):
+    return w.shape[1] * (1 if mode == 2 else 2)
+
+
 def act_product_ok(M, N, K, mode):
     return _lib.lib().omni_act_product_slices(int(M), int(N), int(K), int(mode)) > 0
 
@@ -499,8 +513,12 @@ def act_product_ok(M, N, K, mode):
 def act_product(act, amax, lin, slab, sum_out, scale_out):
     """gemm_partial_f16_* of one or two rows in K slices of its own (csrc/act_product.hip): returns their number, the slabs' sums are the same."""
     _lib.require_cuda(act, amax, slab, sum_out, scale_out)
-    M, K = act.shape
     mode, w, _, _, s2z, s2s = _mode_and_weights(lin)
+    _want("act_product: act must be a contiguous fp16 [M, K] tensor", act.dtype == torch.float16 and act.dim() == 2 and act.is_contiguous() and act.shape[1] == _lin_k(mode, w))
+    M, K = act.shape
+    _want("act_product: amax must come from new_amax_slots", _rows(amax, AMAX_WORDS, torch.int32))
+    _want("act_product: slab must be contiguous", slab.is_contiguous())
+    _want("act_product: sum_out (or None) and scale_out must be contiguous fp16 [M] tensors", _rows(scale_out, M) and (sum_out is None or _rows(sum_out, M)))
     rc = _lib.lib().omni_act_product(mode, act.data_ptr(), amax.data_ptr(), w.data_ptr(), _ptr(s2z), _ptr(s2s), slab.data_ptr(),
                                      slab.numel() * slab.element_size(), _ptr(sum_out), scale_out.data_ptr(), M, w.shape[0], K,
                                      _lib.current_stream())
@@ -514,12 +532,24 @@ def norm_product(residual, gamma, epsilon, lin, out, residual_out=None, slab=Non
     out = lin(codes) (amax given: out = silu_and_mul(lin(codes)) [M, N/2], row maxima raised): one launch, the bits of the two or three calls.
     `lin` / `producer`: W4A8 (qweight, s1_scales, s1_szeros or s2_zeros / s2_scales) or W8A8 layers (weight, dequant_scale) of one kind."""
     _lib.require_cuda(residual, gamma, out, residual_out, slab, p_ascales, p_asums, amax)
-    M, K = residual.shape
     mode, w, scale, zero, s2z, s2s = _mode_and_weights(lin)
+    _want("norm_product: residual must be a contiguous fp16 [M, K] tensor", residual.dtype == torch.float16 and residual.dim() == 2 and residual.is_contiguous() and
+          residual.shape[1] == _lin_k(mode, w))
+    M, K = residual.shape
+    _want("norm_product: gamma must be a contiguous fp16 [K] tensor", _rows(gamma, K))
+    _want("norm_product: out must be fp16 [M, N], or [M, N/2] with amax, with contiguous rows", out.dtype == torch.float16 and out.dim() == 2 and out.stride(1) == 1 and
+          tuple(out.shape) == (M, w.shape[0] // (1 if amax is None else 2)))
+    _want("norm_product: amax must come from new_amax_slots", amax is None or _rows(amax, AMAX_WORDS, torch.int32))
     p_scale = p_zero = None
     if slab is not None:
+        _want("norm_product: the producer must be of lin's kind", _mode_and_weights(producer)[0] == mode)
         p_scale = producer.dequant_scale if mode == 2 else producer.s1_scales
         p_zero = producer.s1_szeros if mode == 0 else None
+        _want("norm_product: the producer must have K channels", _rows(p_scale, K) and (mode != 0 or _rows(p_zero, K)))
+        _want("norm_product: slab must be contiguous and hold sk [M, K] sums", slab.is_contiguous() and slab.numel() * slab.element_size() >= int(sk) * M * K * 4)
+        _want("norm_product: p_ascales, and with zero points p_asums, must be contiguous fp16 [M] tensors", _rows(p_ascales, M) and (mode != 0 or _rows(p_asums, M)))
+        _want("norm_product: residual_out must be a contiguous fp16 [M, K] tensor of its own", _rows(residual_out, M * K) and
+              abs(residual_out.data_ptr() - residual.data_ptr()) >= 2 * M * K)
     rc = _lib.lib().omni_norm_product(
         mode, residual.data_ptr(), _ptr(residual_out), _ptr(slab), int(sk), _ptr(p_scale), _ptr(p_ascales), _ptr(p_zero),
         _ptr(p_asums) if mode == 0 else None, gamma.data_ptr(), float(epsilon), w.data_ptr(), _ptr(s2z), _ptr(s2s), scale.data_ptr(),

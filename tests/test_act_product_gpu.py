@@ -55,3 +55,20 @@ def test_act_product_refuses_what_it_does_not_cover():
     ok = fused_ext.act_product_ok
     assert not ok(3, 4096, 4096, 0) and not ok(2, 4096, 4096, 2) and not ok(1, 4096 + 32, 4096, 0) and not ok(1, 4096, 4096 + 512, 0)
     assert not ok(1, 4096, 1024 * 43, 0)                             # a slice of 4 would be 11008: no whole steps; of 1 too long
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_act_product_refuses_buffers_that_do_not_fit(mode):
+    from omniserve_amd.backend import fused_ext
+    g = torch.Generator(device=dev())
+    g.manual_seed(mode)
+    N, K = 128, 2048
+    f16 = lambda *s: torch.zeros(s, dtype=torch.float16, device=dev())      # noqa: E731
+    good = dict(act=f16(1, K), amax=fused_ext.new_amax_slots(1, dev()), lin=_Layer(N, K, mode, g), slab=torch.empty((64 << 10,), dtype=torch.uint8, device=dev()),
+                sum_out=f16(1) if mode == 0 else None, scale_out=f16(1))
+    fused_ext.act_product(**good)
+    for change in (dict(act=f16(1, K).float()), dict(act=f16(1, 2 * K)[:, ::2]), dict(act=f16(1, K // 2)), dict(act=f16(1, 2 * K)), dict(act=f16(K)), dict(amax=good["amax"][:-1]),
+                   dict(amax=good["amax"].float()), dict(slab=good["slab"][:64]), dict(slab=good["slab"].view(2, -1)[:, ::2]), dict(scale_out=f16(0)), dict(scale_out=f16(1).float()),
+                   dict(sum_out=f16(0)), dict(sum_out=f16(1).float())):
+        with pytest.raises(RuntimeError):
+            fused_ext.act_product(**{**good, **change})

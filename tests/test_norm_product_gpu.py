@@ -99,3 +99,28 @@ def test_norm_product_refuses_what_it_does_not_cover():
     assert not ok(1, 6144 + 32, 4096, 0) and not ok(1, 28672 + 64, 4096, 0, True, 4096)
     assert not ok(2, 6144, 4096, 2, False, 4096)          # two rows with int8 weights
     assert not ok(1, 28672, 4096, 0, True)                # gate_up always consumes slabs
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_norm_product_refuses_buffers_that_do_not_fit(mode):
+    """wrong types, strides and sizes, which the kernel would read or write past"""
+    from omniserve_amd.backend import fused_ext
+    g = torch.Generator(device=dev())
+    g.manual_seed(mode)
+    H, N, sk = 2048, 256, 3
+    f16 = lambda *s: torch.zeros(s, dtype=torch.float16, device=dev())      # noqa: E731
+    x = f16(1, 2 * H)
+    good = dict(residual=x[:, :H], gamma=f16(H), epsilon=1e-5, lin=_Layer(N, H, mode, g), out=f16(1, N), residual_out=f16(1, H), slab=torch.zeros((sk, 1, H), dtype=torch.int32, device=dev()),
+                sk=sk, producer=_Layer(H, 256, mode, g), p_ascales=f16(1), p_asums=f16(1))
+    fused_ext.norm_product(**good)
+    silu = dict(out=f16(1, N // 2), amax=fused_ext.new_amax_slots(1, dev()))
+    fused_ext.norm_product(**{**good, **silu})
+    bad = [dict(residual=x[:, :H].float()), dict(residual=f16(1, H // 2)), dict(residual=f16(1, 2 * H)[:, ::2]), dict(gamma=f16(H - 1)), dict(gamma=f16(2 * H)[::2]), dict(out=f16(1, N - 1)),
+           dict(out=f16(1, N // 2)), dict(out=f16(1, 2 * N)[:, ::2]), dict(out=f16(1, N).float()), dict(sk=sk + 1), dict(slab=good["slab"][:2]), dict(producer=_Layer(H // 2, 256, mode, g)),
+           dict(producer=_Layer(H, 256, 0 if mode == 2 else 2, g)), dict(residual_out=None), dict(residual_out=x[:, :H]), dict(residual_out=x[:, 64:H + 64]), dict(residual_out=f16(1, H - 64)),
+           dict(p_ascales=None), dict(p_ascales=f16(1).float()), {**silu, "out": f16(1, N)}, {**silu, "amax": silu["amax"][:-1]}, {**silu, "amax": silu["amax"].float()}]
+    if mode == 0:
+        bad += [dict(p_asums=None), dict(p_asums=f16(0))]
+    for change in bad:
+        with pytest.raises(RuntimeError):
+            fused_ext.norm_product(**{**good, **change})
