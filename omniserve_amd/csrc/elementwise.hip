@@ -543,8 +543,9 @@ static inline PrefetchArgs take_prefetch(int tokens) {
   if (tokens >= ROWS_MANY) pf.blocks = 0;    // many-row launches are bandwidth-bound themselves: nothing idles
   return pf;
 }
-// norm_pairs_kernel's rows (norm_rows.hip has both sides); K slabs within 32-bit offsets of their first byte
-static inline bool norm_pairs_ok(int tokens, int hidden, int sk = 1) {
+// norm_pairs_kernel's rows (norm_rows.hip has both sides); K slabs within 32-bit offsets of their first byte, and without zero points few enough
+static inline bool norm_pairs_ok(int tokens, int hidden, int sk = 1, bool zero_points = true) {
+  if (!zero_points && sk > (hidden <= 2048 ? 24 : hidden <= 6144 ? 16 : 12)) return false;
   return tokens < ROWS_MANY && hidden % 1024 == 0 && hidden <= 8192 && (unsigned long long)sk * tokens * hidden * sizeof(int32_t) < 1ull << 32;
 }
 // (kernels without a PrefetchArgs parameter)
@@ -909,7 +910,7 @@ extern "C" int omni_splitk_w8_add_rms_norm_general_fuse_sum(void* out_i8, void* 
   const int nv = norm_block(hidden, true);
   if (!v2_ok(hidden, nv)) return OMNI_EINVAL;
   if (tokens == 0) return OMNI_OK;
-  if (norm_pairs_ok(tokens, hidden, sk)) {
+  if (norm_pairs_ok(tokens, hidden, sk, false)) {
     norm_pairs_slabs(NormOut{(int8_t*)out_i8, (const half_t*)weight_f16, (half_t*)sum_f16, (half_t*)scale_f16, eps},
                      NormSlabs{(half_t*)residual_f16, (const int32_t*)slab_i32, (size_t)tokens * hidden, sk, (const half_t*)wscales_f16, nullptr,
                                (const half_t*)ascales_in_f16, nullptr},

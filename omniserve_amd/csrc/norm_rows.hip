@@ -12,7 +12,9 @@
 //
 // MI355X, inside the captured step of the 8B model (4096 channels), general_norm_v2_kernel -> this one, us: 1 row, 8 slabs 8.3 -> 6.5; 16 rows, 8 slabs 8.0
 // -> 6.3; first layer, no slabs, 6.3 -> 5.5.  What is left: the first load (the slabs come from other XCDs' launches; 128 KiB of them into one compute
-// unit) and a launch's ends.
+// unit) and a launch's ends.  Rows alone, at 1, 128, 512 and 1023 of them: 4096 channels, no slabs, 4.3, 4.9, 6.3, 10.8 -> 3.0, 3.4, 4.2, 6.7; 4 slabs 6.3, 6.9, 15.7, 28.8
+// -> 4.4, 4.9, 11.3, 21.1; 8192 channels, 8 slabs 9.0, 11.2, 32.5, 68 -> 8.1, 9.2, 27.3, 59.  Many slabs take a second trip: behind the product of 28672 x 8192 with its
+// 14 slabs the two 32.5 -> 32.2, behind the int8 one with 28 72.3 -> 75.5 (16 slabs of int8 products, 1 and 16 rows: 4096 channels -0.1 and -0.2, 8192 +1.9 and +1.1).
 #include "norm_pairs.h"
 #include "norm_rows.h"
 
