@@ -55,8 +55,11 @@ void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, in
 /* M > 128 (0 below), operands and output rows 16-byte aligned (others go to the general kernel).  mode: 0 per-channel W4A8, 1 per-group W4A8, 2 W8A8; slabs_only: omni_*_gemm_partial.
  * Returns 1 for the straight-line kernels: *mb 16-row blocks of a tile (16: the 256 x 256 tiles of W8A8), *kw K parts inside a
  * workgroup, *sk K slices that go through the scratch (1: none but slabs_only's own);
- * per-group: what runs where its own 256 x 256 tiles (csrc/qgemm_group_tiles.h) are not the faster choice.  2 for the general kernel (N % 256 or K % 256). */
+ * per-group: what runs where omni_gemm_prefill_group_tiles is 0.  2 for the general kernel (N % 256 or K % 256). */
 int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int slabs_only, int* mb, int* kw, int* sk);
+/* 1 where omni_w4a8_per_group_gemm of these sizes runs in 256 x 256 tiles (csrc/qgemm_group_tiles.h), its operands aligned as above and its second-level scales and
+ * zero points on whole dwords. */
+int omni_gemm_prefill_group_tiles(int M, int N, int K);
 /* 1 when the row-kernel-free decode forms below (omni_*_gemm_silu for gate_up [2*inter, hidden], omni_*_gemm_partial_f16
  * for o [hidden, attn_dim] and down [hidden, inter]) accept a layer of these dimensions at M rows, 0 otherwise: the plan
  * conditions those entry points check at launch, for a driver that picks its fusion level up front.

@@ -299,6 +299,13 @@ extern "C" int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int sla
   return exact ? 1 : 2;
 }
 
+extern "C" int omni_gemm_prefill_group_tiles(int M, int N, int K) {
+  using namespace omni;
+  if (M <= 128 || N < 64 || N % 64 || K < 64 || K % 64) return 0;
+  const GemmPlan pl = plan_gemm(M, N, K, 128, false, false);
+  return exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, MODE_GRP, pl.sk, false).group_tiles;
+}
+
 // Would the row-kernel-free decode forms (omni_*_gemm_silu for gate_up, omni_*_gemm_partial_f16 for o / down) accept a layer
 // with these dimensions?  The same plan conditions launch_gemm_silu / launch_gemm_partial_f16 check at launch (one place to
 // keep in step: qgemm_kernel.h), so that a driver can choose its fusion level BEFORE its first step instead of running into

@@ -188,6 +188,29 @@ def test_prefill_plans_of_rows_far_apart():
         assert (sk > 1) == sliced and kw == (1 if sliced else 2), (M, N, K, mode)
 
 
+def test_per_group_prefill_takes_256_x_256_tiles_where_they_are_faster():
+    from omniserve_amd import _lib
+    from tests import test_gemm_gpu as forms
+    lib = _lib.lib()
+    tiles = lib.omni_gemm_prefill_group_tiles
+    for M, N, K in ((2331, 28672, 4096), (2331, 4096, 14336), (512, 28672, 4096), (511, 26624, 1536), (8000, 8192, 28672)):
+        assert tiles(M, N, K) == 1, (M, N, K)
+    # few tiles on the chip; short K; too few rows; channels or K that are no whole tiles
+    for M, N, K in ((2331, 4096, 4096), (1800, 4096, 14336), (1024, 6144, 4096), (8000, 2048, 512), (8000, 28672, 256), (255, 28672, 4096), (128, 28672, 4096), (2331, 28672 + 64, 4096),
+                    (2331, 28672, 4096 + 128)):
+        assert tiles(M, N, K) == 0, (M, N, K)
+    # what the tests of the other kernel name by its plan runs there
+    for form in forms.PREFILL_FORMS:
+        if form[0] == "grp":
+            assert tiles(*form[4:]) == 0, form
+    for waves, sk, want in ((16, 0, 1), (0, 2, 0), (16, 2, 0)):
+        lib.omni_gemm_set_plan_override(waves, sk)
+        try:
+            assert tiles(300, 256, 1536) == want and tiles(2331, 28672, 4096) == want and tiles(300, 256, 256) == 0
+        finally:
+            lib.omni_gemm_set_plan_override(0, 0)
+
+
 def test_forced_k_splits_reach_the_prefill_plan():
     from omniserve_amd import _lib
     lib = _lib.lib()

@@ -20,7 +20,17 @@ def tiles():
 @pytest.mark.parametrize("M,N,K,wrap,shift", [(256, 256, 512, False, 0), (257, 256, 768, True, 0), (511, 512, 1024, False, 0), (512, 256, 1280, True, 0), (2100, 8192, 512, False, 0),
                                               (300, 256, 1536, True, 1)])
 def test_group_tiles(tiles, M, N, K, wrap, shift):
+    _run(M, N, K, wrap, shift)
+
+
+def test_group_tiles_by_the_rule():
+    _run(511, 26624, 1536, True, 0)
+
+
+def _run(M, N, K, wrap, shift):
     import omniserve_backend.qgemm_w4a8_per_group as mod
+    from omniserve_amd import _lib
+    assert _lib.lib().omni_gemm_prefill_group_tiles(M, N, K) == 1
     u, z, s2, s1 = w4a8.synth_per_group(N, K, seed=M + K, wrap=wrap)
     qw, s1h, s2s, s2z = w4a8.pack_per_group(u, z, s2, s1)
     g = torch.Generator().manual_seed(M)
