@@ -1483,7 +1483,11 @@ static int launch_gemm_silu(GemmArgs a, hipStream_t st) {
   OMNI_GEMV_SET_DBG(a);
   // int8 rows load plainly: a wave takes 64 bytes of each, and non-temporally a line's other half comes from memory again (28672 x 4096, 4 rows 26.8 ->
   // 24.7 us, 16 rows 28.7 -> 26.8; 4096 x 14336 below 16.5 -> 15.7)
-  return (take_prefetched_weight(a.W) || MODE == MODE_W8) ? launch_gemv_silu_nt<MODE, false>(a, pl, st) : launch_gemv_silu_nt<MODE, true>(a, pl, st);
+  const bool plain = take_prefetched_weight(a.W);
+  if constexpr (MODE != MODE_W8) {
+    if (!plain) return launch_gemv_silu_nt<MODE, true>(a, pl, st);
+  }
+  return launch_gemv_silu_nt<MODE, false>(a, pl, st);
 }
 
 template <int MODE, bool NT>
@@ -1515,7 +1519,11 @@ static int launch_gemm_partial_f16(GemmArgs a, void* slab, size_t slab_bytes, in
   a.kslice = pl.kslice;
   *sk_out = pl.sk;
   OMNI_GEMV_SET_DBG(a);
-  return (take_prefetched_weight(a.W) || MODE == MODE_W8) ? launch_gemv_f16_nt<MODE, false>(a, pl, st) : launch_gemv_f16_nt<MODE, true>(a, pl, st);
+  const bool plain = take_prefetched_weight(a.W);      // (int8 rows: always, see launch_gemm_silu)
+  if constexpr (MODE != MODE_W8) {
+    if (!plain) return launch_gemv_f16_nt<MODE, true>(a, pl, st);
+  }
+  return launch_gemv_f16_nt<MODE, false>(a, pl, st);
 }
 
 // Deferred-epilogue variant (fused extension): only the int32 split-K slabs are produced; the consumer
