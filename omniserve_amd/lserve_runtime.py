@@ -191,7 +191,7 @@ class LServeDecodeRunner:
             self.attn_f16 = torch.empty((B, Hq * d), dtype=f16, device=device)
             self.amax = torch.zeros((c.layers, 2, fused_ext.AMAX_WORDS), dtype=torch.int32, device=device)
         # one or two rows: each norm and the product behind it are one launch, which leaves the new residual in the other of two buffers
-        self.own_rows = (self.rowfree and bool(own_rows) and fused_ext.norm_product_ok(B, qkv_n, c.hidden, 2, False, c.inter) and
+        self.own_rows = (self.rowfree and bool(own_rows) and c.layers > 0 and fused_ext.norm_product_ok(B, qkv_n, c.hidden, 2, False, c.inter) and
                          fused_ext.norm_product_ok(B, 2 * c.inter, c.hidden, 2, True, Hq * d))
         self._x2 = torch.empty_like(self.x) if self.own_rows else None
         self.qkv_buf = torch.empty((B, qkv_n), dtype=f16, device=device)

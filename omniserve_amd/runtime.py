@@ -318,9 +318,9 @@ class DecodeRunner:
         # level 3 also in the LAST layer: its down projection's slabs are consumed by the model's final norm
         # (fused_ext.splitk_add_rms_norm) instead of GEMV epilogue + residual add + rms_norm (l3_last=False: off, A/B)
         self.last_l3 = self.fused >= 3 and self.tp_size == 1 and self.comm is None and bool(l3_last)
-        # one or two rows: each norm and the product behind it are one launch, which leaves the new residual in the other of two buffers
+        # one or two rows: each norm and the product behind it are one launch, which leaves the new residual in the other of two buffers (without layers nothing does)
         mode = 0 if c.group_size == -1 else 1
-        self.own_rows = (self.last_l3 and not self.pairs and not self.qkv_slabs and bool(own_rows) and
+        self.own_rows = (self.last_l3 and not self.pairs and not self.qkv_slabs and bool(own_rows) and c.layers > 0 and
                          fused_ext.norm_product_ok(B, qkv_n, c.hidden, mode, False, il) and
                          fused_ext.norm_product_ok(B, 2 * il, c.hidden, mode, True, hl * d))
         self._x2 = torch.empty_like(self.x) if self.own_rows else None

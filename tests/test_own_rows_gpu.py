@@ -59,3 +59,12 @@ def test_prefill_and_steps_behind_it():
         r.prefill(70, tokens=torch.arange(140, device=dev()))
         out.append(_state(r, 3))
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_a_model_without_layers():
+    out = []
+    for own in (False, True):
+        r = DecodeRunner(_config(0, 4096), batch=1, context=70, max_new=8, device=dev(), seed=3, use_graph=False, own_rows=own)
+        assert not r.own_rows
+        out.append(_state(r, 2))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
