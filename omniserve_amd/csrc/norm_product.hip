@@ -12,7 +12,7 @@
 //  * qkv: 32 channels a workgroup, so that 6144 channels make 192 workgroups instead of 96.
 //  * the new residual goes to a buffer of its own (workgroup 0 stores it): other workgroups still read the old one.
 //
-// MI355X, 8B model, us a layer, two launches -> one: W4A8 1 row qkv 6.5 + 5.5 -> 7.7, gate_up 6.5 + 12.0 -> 13.7 (down_proj, whose weights the norm
+// MI355X, 8B model, us a layer, two launches -> one: W4A8 1 row qkv 6.5 + 5.5 -> 6.7, gate_up 6.5 + 12.0 -> 13.7 (down_proj, whose weights the norm
 // no longer fetches, 6.8 -> 8.7); the step of 8 layers 472 -> 419 us, 2 rows 511 -> 490; with groups of 128 604 -> 500 and 620 -> 557.  W8A8 1
 // row: gate_up 6.5 + 24.5 -> 27.3; four LServe steps of 4 layers 2037 -> 1818.  Two rows
 // gain little enough that more are left to the two launches.
@@ -36,7 +36,9 @@ struct NormProductArgs {
   int M, N;
 };
 
-// C: K / 1024.  SK: slabs whose requests go out together (those beyond sk read slab 0 again); 0: the residual as it is.  ROWS: M.
+// C: K / 1024.  SK: slabs whose requests go out together (those beyond sk read slab 0 again, so there are forms for 2, 4, 8 and 16: qkv of 12288 channels behind one slab of two
+// rows in the form for 8, 1048 us a step of 16 layers of 4096 / 11008, 921 in that for 2; the 8B model's step of 16 layers behind 4, 1 and 2 rows, 680 -> 662 and 782 -> 750); 0: the
+// residual as it is.  ROWS: M.
 template <int MODE, int EPI, int BLOCKS, int C, int SK, int ROWS>
 __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(NormProductArgs p) {
   constexpr bool ZP = MODE == MODE_CHN, W8 = MODE == MODE_W8;
@@ -258,6 +260,10 @@ void launch_slabs(const NormProductArgs& p, hipStream_t st) {
     else launch_rows<MODE, 1, 4, C, 4>(p, st);
   } else if (!p.slab) {
     launch_rows<MODE, 0, CHANNELS32, C, 0>(p, st);
+  } else if (p.sk <= 2) {
+    launch_rows<MODE, 0, CHANNELS32, C, 2>(p, st);
+  } else if (p.sk <= 4) {
+    launch_rows<MODE, 0, CHANNELS32, C, 4>(p, st);
   } else if (p.sk <= 8) {
     launch_rows<MODE, 0, CHANNELS32, C, 8>(p, st);
   } else {

@@ -62,6 +62,7 @@ def _two_calls(x, gamma, lin, out, silu, amax, prod, slab, sk, p_a, p_sum):
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("M,N,H,sk,silu", [(1, 64, 4096, 0, False), (2, 6144, 4096, 0, False), (1, 6144, 4096, 7, False), (2, 192, 4096, 8, False),
                                            (1, 192, 4096, 14, False), (1, 64, 2048, 16, False), (2, 2560, 3072, 1, False), (1, 320, 2048, 5, False),
+                                           (1, 12288, 4096, 1, False), (2, 192, 4096, 2, False), (1, 320, 3072, 3, False), (2, 6144, 2048, 4, False),
                                            (1, 28672, 4096, 2, True), (2, 28672, 4096, 4, True), (2, 128, 2048, 1, True), (1, 8448, 3072, 3, True),
                                            (1, 16512, 2048, 2, True), (2, 22016, 4096, 3, True)])
 def test_norm_product_gives_the_bits_of_the_calls_it_replaces(mode, M, N, H, sk, silu):
