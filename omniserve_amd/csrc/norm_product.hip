@@ -105,7 +105,7 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
   for (int u = 0; u < FIRST; ++u) product.request(u);
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- the rows (norm_rows.hip, step by step) ----
+  // ---- the rows ----
   float x[ROWS][C][2];
   v2h o[ROWS][C];
 #pragma unroll
@@ -133,66 +133,23 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
 #pragma unroll
   for (int u = FIRST; u < Product::RING; ++u) product.request(u);
   __builtin_amdgcn_sched_barrier(0);
-  const int vw = 4 * wave + (lane >> 4);
-  auto warp_sum = [&](float v0, float v1) { return row16_sum(v0) + row16_sum(v1); };
+  const PairPlace place(tid);
 #pragma unroll
-  for (int m = 0; m < ROWS; ++m) {
-    float s[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        s[0][e] = s[0][e] + x[m][c][e];
-        s[1][e] = s[1][e] + x[m][c][e] * x[m][c][e];
-      }
-    const float w0 = warp_sum(s[0][0], s[0][1]), w1 = warp_sum(s[1][0], s[1][1]);
-    if ((lane & 15) == 0) {
-      red[m][(vw & 15) * 4 + (vw >> 4)] = w0;
-      red[m][(vw & 15) * 4 + 2 + (vw >> 4)] = w1;
-    }
-  }
+  for (int m = 0; m < ROWS; ++m) pair_sums<C>(x[m], red[m], place);
   lds_barrier();
 #pragma unroll
-  for (int m = 0; m < ROWS; ++m) {
-    const v4f q4 = *reinterpret_cast<const v4f*>(&red[m][(lane & 15) * 4]);
-    const float mean = row16_sum(q4[0] + q4[1]) / (float)K;
-    const float rstd = 1.0f / __builtin_sqrtf(row16_sum(q4[2] + q4[3]) / (float)K + p.eps);
-    float amax = (float)(half_t)1e-6f, hs[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        float y = (x[m][c][e] - mean) * rstd;
-        y = rounded_f32(y * (float)g[c][e]);
-        x[m][c][e] = y;
-        const float yh = (float)(half_t)y;
-        amax = __builtin_fmaxf(amax, __builtin_fabsf(yh));
-        if constexpr (ZP) hs[e] = (float)(half_t)(hs[e] + yh);
-      }
-    amax = wave_max64(amax);
-    if (lane == 0) red[m][96 + wave] = amax;
-    if constexpr (ZP) {
-      const float w = warp_sum(hs[0], hs[1]);
-      if ((lane & 15) == 0) red[m][64 + (vw & 15) * 2 + (vw >> 4)] = w;
-    }
-  }
+  for (int m = 0; m < ROWS; ++m) pair_normalise<C, ZP>(x[m], g, p.eps, red[m], place);
   lds_barrier();
   float row_scale[ROWS], row_sum[ROWS];
 #pragma unroll
   for (int m = 0; m < ROWS; ++m) {
-    float amax = red[m][96 + (lane & 7)];
-    amax = __builtin_fmaxf(amax, lane_xor1(amax));
-    amax = __builtin_fmaxf(amax, lane_xor2(amax));
-    amax = __builtin_fmaxf(amax, dpp_mov<0x141>(amax));
+    const float amax = pair_top(red[m], place);
     row_scale[m] = (float)(half_t)(amax / 127.0f);
     row_sum[m] = 0.0f;
-    if constexpr (ZP) row_sum[m] = (float)(half_t)row16_sum(red[m][64 + (lane & 15) * 2] + red[m][64 + (lane & 15) * 2 + 1]);
+    if constexpr (ZP) row_sum[m] = (float)pair_total(red[m], place);
     const float q = 127.0f / amax;
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const uint32_t two = (uint32_t)(uint8_t)rni_sat_s8(x[m][c][0] * q) | ((uint32_t)(uint8_t)rni_sat_s8(x[m][c][1] * q) << 8);
-      *reinterpret_cast<uint16_t*>(codes + m * PITCH + code_place<MODE>(1024 * c + 2 * tid)) = (uint16_t)two;
-    }
+    for (int c = 0; c < C; ++c) *reinterpret_cast<uint16_t*>(codes + m * PITCH + code_place<MODE>(1024 * c + 2 * tid)) = pair_codes(x[m][c], q);
   }
   lds_barrier();
 

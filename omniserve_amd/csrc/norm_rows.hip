@@ -159,7 +159,7 @@ template <int C, bool FUSE_SUM, typename Src>
 __global__ __launch_bounds__(512) void norm_pairs_kernel(int8_t* __restrict__ out, Src src, const half_t* __restrict__ gamma, half_t* __restrict__ sum_out,
                                                          half_t* __restrict__ scale_out, float eps, PrefetchArgs pf) {
   constexpr int H = 1024 * C;
-  __shared__ __attribute__((aligned(16))) float lds[8 * 256];      // 1 KiB a wave for fetching workgroups; a row's uses the first 104 words
+  __shared__ __attribute__((aligned(16))) float lds[8 * 256];      // 1 KiB a wave for fetching workgroups; a row's uses the first PAIR_RED words
   // one batch of scalar loads for the test below and the row's path
   src.pin();
   asm volatile("" ::"s"(out), "s"(gamma), "s"(sum_out), "s"(scale_out), "s"(eps), "s"(pf.blocks), "s"(pf.first_block));
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(512) void norm_pairs_kernel(int8_t* __restrict__ ou
     prefetch_weights_to_l2(pf, lds);
     return;
   }
-  const int p = threadIdx.x, lane = p & 63, wave = p >> 6, row = blockIdx.x;
+  const int p = threadIdx.x, row = blockIdx.x;
   const RowArray gains(gamma);
   v2h g[C];
 #pragma unroll
@@ -175,69 +175,20 @@ __global__ __launch_bounds__(512) void norm_pairs_kernel(int8_t* __restrict__ ou
   float x[C][2];
   src.template values<C>(row, p, g, x);
 
-  // sum and sum of squares: the virtual thread's, the virtual warp's, the row's
-  float s[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-#pragma unroll
-  for (int c = 0; c < C; ++c)
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      s[0][e] = s[0][e] + x[c][e];
-      s[1][e] = s[1][e] + x[c][e] * x[c][e];
-    }
-  auto warp_sum = [&](float (&v)[2]) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e) v[e] = row16_sum(v[e]);
-    return v[0] + v[1];
-  };
-  const int vw = 4 * wave + (lane >> 4);                          // virtual warp; its sums lie beside those of vw ^ 16
-  float* const r1 = lds;                                          // [16][sum, sum, square, square]
-  float* const r2 = lds + 64;                                     // [16][2] sums of the normalised values, then 8 maxima
-  {
-    const float w0 = warp_sum(s[0]), w1 = warp_sum(s[1]);
-    if ((lane & 15) == 0) {
-      r1[(vw & 15) * 4 + (vw >> 4)] = w0;
-      r1[(vw & 15) * 4 + 2 + (vw >> 4)] = w1;
-    }
-  }
+  const PairPlace place(p);
+  pair_sums<C>(x, lds, place);
   lds_barrier();
-  const v4f q4 = *reinterpret_cast<const v4f*>(r1 + (lane & 15) * 4);
-  const float mean = row16_sum(q4[0] + q4[1]) / (float)H;
-  const float rstd = 1.0f / __builtin_sqrtf(row16_sum(q4[2] + q4[3]) / (float)H + eps);
-
-  float amax = (float)(half_t)1e-6f;
-  float hs[2] = {0.0f, 0.0f};
-#pragma unroll
-  for (int c = 0; c < C; ++c)
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      float y = (x[c][e] - mean) * rstd;
-      y = rounded_f32(y * (float)g[c][e]);
-      x[c][e] = y;
-      const float yh = (float)(half_t)y;
-      amax = __builtin_fmaxf(amax, __builtin_fabsf(yh));
-      if constexpr (FUSE_SUM) hs[e] = (float)(half_t)(hs[e] + yh);      // the reference adds these up in fp16
-    }
-  amax = wave_max64(amax);
-  if (lane == 0) r2[32 + wave] = amax;
-  if constexpr (FUSE_SUM) {
-    const float w = warp_sum(hs);
-    if ((lane & 15) == 0) r2[(vw & 15) * 2 + (vw >> 4)] = w;
-  }
+  pair_normalise<C, FUSE_SUM>(x, g, eps, lds, place);
   lds_barrier();
-  amax = r2[32 + (lane & 7)];
-  amax = __builtin_fmaxf(amax, lane_xor1(amax));
-  amax = __builtin_fmaxf(amax, lane_xor2(amax));
-  amax = __builtin_fmaxf(amax, dpp_mov<0x141>(amax));             // the other half of 8 lanes, mirrored
+  const float amax = pair_top(lds, place);
   if (p == 0) scale_out[row] = (half_t)(amax / 127.0f);
   const float q = 127.0f / amax;
   const RowArray codes(out + (size_t)row * H);
 #pragma unroll
-  for (int c = 0; c < C; ++c)
-    codes.put16(2 * p, 1024 * c,
-          (uint16_t)((uint32_t)(uint8_t)rni_sat_s8(x[c][0] * q) | ((uint32_t)(uint8_t)rni_sat_s8(x[c][1] * q) << 8)));
+  for (int c = 0; c < C; ++c) codes.put16(2 * p, 1024 * c, pair_codes(x[c], q));
   if constexpr (FUSE_SUM) {
-    const float tot = row16_sum(r2[(lane & 15) * 2] + r2[(lane & 15) * 2 + 1]);
-    if (p == 0) sum_out[row] = (half_t)tot;
+    const half_t tot = pair_total(lds, place);
+    if (p == 0) sum_out[row] = tot;
   }
 }
 
