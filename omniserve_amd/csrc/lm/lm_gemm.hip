@@ -294,7 +294,7 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 
 // A workgroup: 16 NW channels of a group, rows 0 .. 16 MB - 1 of it, K slice blockIdx.z.  With several slices (one group) the f32 sums of a
 // slice go to part [slice][rows][n] and gemm_reduce_kernel finishes them.
-template <int EPI, int NW, int KW, bool SHORT>
+template <int EPI, int NW, int KW, bool SHORT, bool TURN>
 __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, float* part) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[KW * ring_bytes<NW, KW>];
   constexpr int RC = 16 * NW, NT = 64 * NW * KW;
@@ -312,7 +312,6 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
   const int stages = pt.k * (int)sizeof(elem_t) / RB, slice = blockIdx.z, slices = gridDim.z;
   const int s0 = stages * slice / slices, s1 = stages * (slice + 1) / slices;
   const int div = is_b ? 1 : p.x_div;
-  constexpr bool TURN = EPI == LM_EPI_F32 || (EPI == LM_EPI_GLU && NW == 8);      // heads and wide dense gated units
   for (int m0 = 0; m0 < rows; m0 += 64) {
     const int here = min(64, rows - m0), mb = (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
@@ -704,9 +703,10 @@ static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s
 // 256 more: 16448 channels at 48 rows take 42 us as 257 tiles of 64, 30 as 206 of 80), and slices cost the launch that adds them.  By what
 // was measured the channels per workgroup matter most where n / 64 is far from a multiple of 256 (10816 x 4096, 48 rows: 26.5 us at 64,
 // 20.8 at 48; 4096 x 4096, 16 rows: 11.8 us at 64 and 4 slices, 9.8 at 16), slices where K is long (4096 x 14336, 48 rows: 40 us, 26
-// with 4).  128 channels, bf16: 2.5 us for a ring of 144 KiB that nothing runs beside, but x comes in half as often, and 224 or 250 workgroups are one round where 448
-// or 500 are two (heads and gated units, whose workgroups begin with different chains; 28672 x 4096, 64 / 128 channels: 16 rows 42.3 / 37.1 us, 48 rows 48.3 / 39.9, 64
-// rows 51.8 / 41.5; 32000 x 4096, 80 / 128: 48 rows 52.0 / 43.4; 32000 x 2048, 16 rows 25.4 / 22.9; 96 and 112 channels nowhere the fastest).
+// with 4).  128 channels, bf16: 2 us a round for a ring of 144 KiB that nothing runs beside, but x comes in half as often, and 224 or 250 workgroups are one round where 448
+// or 500 are two (heads and gated units; 28672 x 4096, 64 / 128 channels: 16 rows 42.3 / 37.1 us, 48 rows 48.3 / 39.9, 64 rows 51.8 / 41.5; 32000 x 4096, 80 / 128: 48 rows
+// 52.0 / 43.4; 32000 x 2048, 16 rows 25.4 / 22.9; two and four rounds of few rows and short K lose: 64000 x 2048 at 1 row 45.9 / 48.5, 128256 x 1024 43.1 / 46.7; 96 and
+// 112 channels nowhere the fastest).
 struct RowsPlan {
   int nw, slices;      // nw 0: gemm_rows_kernel
 };
@@ -726,29 +726,34 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
   // 128 channels only in place of workgroups that take K in one chain of stages, as they do: the same order of sums
   auto tiles = [&](int nw) { return (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw)); };
   if (LM_ELEM == 0 && best.slices == 1 && tiles(best.nw) > 256 &&
-      (float)((tiles(8) + 255) / 256) * (float)stages * (0.07f * 8 + 0.02f * mb + 0.02f) + 2.5f < time)
+      (float)((tiles(8) + 255) / 256) * ((float)stages * (0.07f * 8 + 0.02f * mb + 0.02f) + 2.f) + 0.5f < time)
     best.nw = 8;
   return best;
 }
 
 // K parts inside a workgroup where there is no second one to run beside it on its CU
-template <int EPI, int NW, bool SHORT>
+template <int EPI, int NW, bool SHORT, bool TURN = false>
 static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
   constexpr int KW = NW <= 2 ? 4 : NW <= 5 ? 2 : 1;
   if (KW > 1 && (int64_t)grid.x * grid.y * grid.z <= 256)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT>), grid, dim3(64 * NW * KW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT, TURN>), grid, dim3(64 * NW * KW), 0, s, a, part);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT>), grid, dim3(64 * NW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT, TURN>), grid, dim3(64 * NW), 0, s, a, part);
 }
+
+// bf16: heads, and gated units of 128 channels, in one slice: workgroups that begin at different k where rows lie whole 4 KiBs apart and are enough to be bound by the memory's
+// channels.  (MI355X, in step | so, 16 rows, f32 results, us: 16448 x 4096 27.9 | 24.6, 40960 x 4096 63.0 | 55.3, 8192 x 8192 33.5 | 28.1, 8192 x 4096 16.6 | 16.0; other rows 2 - 5 % the
+// other way: 24576 x 2560 23.2 | 24.4, 36864 x 3072 37.6 | 39.0; small products, the router's among them, by 0.6 us: 512 x 2048 5.4 | 6.0, 4096 x 4096 9.5 | 10.1.)
+[[maybe_unused]] static bool turns(int n, int64_t k, int slices) { return slices == 1 && k % 2048 == 0 && n * k >= 24 << 20; }
 
 template <int EPI, int NW>
 static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
-  if constexpr (EPI == LM_EPI_F32) {      // (slices begin at places of their own, and what they leave is the same)
-    if (slices > 1) return launch_stream_tiles<LM_EPI_ELEM, NW>(a, n, has_b, slices, part, s);
+  if (a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K)) return launch_stream_form<EPI, NW, true>(a, n, has_b, slices, part, s);
+  if constexpr (LM_ELEM == 0 && (EPI == LM_EPI_F32 || (EPI == LM_EPI_GLU && NW == 8))) {
+    if (turns(n, a.a.k, slices)) return launch_stream_form<EPI, NW, false, true>(a, n, has_b, slices, part, s);
   }
-  if (a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K)) launch_stream_form<EPI, NW, true>(a, n, has_b, slices, part, s);
-  else launch_stream_form<EPI, NW, false>(a, n, has_b, slices, part, s);
+  launch_stream_form<EPI, NW, false>(a, n, has_b, slices, part, s);
 }
 
 template <int EPI>
