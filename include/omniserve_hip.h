@@ -421,7 +421,8 @@ int omni_prefill_attention_block_streaming(void* out_f16, const void* q_f16, con
                                            int max_seqlen_q, int num_heads, int num_kv_heads, int head_dim,
                                            const void* head_mask_type_i32, const void* streaming_info_i32, void* stream);
 /* Tuning / test hook: 0 = 16 query rows per wave (16x16x32 MFMA, default), 1 = 32 rows per wave (32x32x16 MFMA), 2 = the 16-row
- * form on the 8-wave ping-pong schedule (waves 4-7 one segment behind waves 0-3; same results within the attention tolerance). */
+ * form on the 8-wave ping-pong schedule (waves 4-7 one segment behind waves 0-3; same results within the attention tolerance),
+ * 3 / 4 = the 16-row form in workgroups of 64 / 128 rows whatever the size (0 takes the one that is faster: the same bits). */
 void omni_prefill_set_variant(int variant);
 
 /* Tuning hook: over how many XCDs the query tiles of one kv head are spread when streaming heads are present

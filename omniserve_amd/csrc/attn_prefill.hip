@@ -79,16 +79,21 @@ __device__ __forceinline__ int first_local_key(int qpos, int local, int g) { ret
 // head costs O(L^2), a streaming head O(L * window); with whole kv heads pinned to XCDs the XCDs that drew streaming heads
 // idle for most of the launch).  kv heads are taken dense-first: sorted position pos, part j -> XCD (pos * W + j) % 8.
 // Returns false for the padding workgroups of a part that has fewer tiles.
+// LONG_FIRST: the longest tiles of all sequences first instead of one sequence after the other, every other 32 workgroups of an XCD (one for each of its CUs)
+// backwards, so that the CU with the longest of one turn gets the shortest of the next.
+template <bool LONG_FIRST = false>
 __device__ __forceinline__ bool prefill_map_block(const PrefillArgs& p, int& b, int& h, int& qt) {
   const int W = p.xcd_split, Hk = p.num_kv_heads, G = p.num_heads / Hk;
   const int P = (Hk * W) >> 3;                       // (kv head, part) pairs per XCD
   const int R = (p.q_tiles + W - 1) / W;             // tile rows of a part
   const int wid = blockIdx.x, xcd = wid & 7;
   int slot = wid >> 3;
+  if (LONG_FIRST && (slot & 32) && (slot | 31) < (int)(gridDim.x >> 3)) slot ^= 31;
   const int u = slot % G; slot /= G;
   const int i = slot % P; slot /= P;
-  const int r = slot % R;
-  b = slot / R;
+  const int batch = LONG_FIRST ? (int)(gridDim.x >> 3) / (G * P * R) : 1;
+  const int r = LONG_FIRST ? slot / batch : slot % R;
+  b = LONG_FIRST ? slot % batch : slot / R;
   const int idx = xcd + 8 * i, pos = idx / W, j = idx - pos * W;
   qt = p.q_tiles - 1 - (r * W + j);                  // long (late) query tiles first
   int kvh = pos;
@@ -240,8 +245,9 @@ void prefill_attn_kernel(PrefillArgs p) {
     if (kb_next < k_hi) PREFILL_DMA_TILE(kb_next, B ? ktile0 : ktile1, B ? vtile0 : vtile1);
 #endif
     __builtin_amdgcn_sched_barrier(0);
-    // does any (row, key) pair of this workgroup's tile need the mask?  (workgroup-uniform)
-    bool full = (kb + PKT <= len_k) && (q_first + PQROWS <= len_q);
+    // does any (row, key) pair of this workgroup's tile need the mask?  (workgroup-uniform; a row past the sequence is a copy of its last
+    // one and never stored: the last query tile, the longest, took the mask for every key -- 1501 tokens 56.6 -> 44.6 us)
+    bool full = kb + PKT <= len_k;
     if (p.causal) full = full && (kb + PKT - 1 <= q_first + off);
     if (streaming) full = full && ((kb + PKT <= sink) || (kb >= first_local_key(q_last + off, local, gl)));
     // ---- online softmax (per query row = per lane column), probabilities straight into the B operand ----------
@@ -361,6 +367,219 @@ void prefill_attn_kernel(PrefillArgs p) {
 #undef PREFILL_DMA_TILE
 
 // ------------------------------------------------------------------------------------------------------------------------
+// The stages of a tile for one wave of 16 rows, as in the kernel above: scores of 64 keys, their softmax, the product with V.
+__device__ __forceinline__ void rows16_scores(const uint8_t* kt, int l15, int l4, const v8h (&qb)[4], v4f (&st)[4]) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) st[u] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int key = 16 * u + l15;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const v8h a = *reinterpret_cast<const v8h*>(kt + key * PKROW + (((4 * s + l4) ^ l15) << 4));
+      st[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[s], st[u], 0, 0, 0);
+    }
+  }
+}
+// full: no (row, key) pair of the workgroup's tile needs the mask
+__device__ __forceinline__ void rows16_softmax(bool full, int kb, int l4, int qrow, int off, int len_q, int len_k, int causal, bool streaming, int sink,
+                                               int local, int gl, const v4f (&st)[4], v8h (&pb)[2], float& m_run, float& l_run, v4f (&oacc)[8]) {
+  const float scale2 = 0.08838834764831845f * 1.4426950408889634f;
+  float tmax = -1e30f, m_new, alpha, psum = 0.0f;
+  if (full) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmax = __builtin_fmaxf(tmax, st[u][r]);
+    tmax = rows4_max(tmax);
+    m_new = __builtin_fmaxf(m_run, tmax * scale2);
+    alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(st[e >> 2][e & 3], scale2, -m_new));
+      pb[e >> 3][e & 7] = (half_t)pe;
+      psum += pe;
+    }
+  } else {
+    bool okv[16];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = kb + 16 * u + 4 * l4 + r;
+        const int qpos = qrow + off;
+        int ok = (int)(key < len_k) & (int)(qrow < len_q);
+        ok &= (int)(!causal) | (int)(key <= qpos);
+        ok &= (int)(!streaming) | (int)(key < sink) | (int)(key >= first_local_key(qpos, local, gl));
+        okv[4 * u + r] = ok != 0;
+        tmax = __builtin_fmaxf(tmax, ok ? st[u][r] : -1e30f);
+      }
+    tmax = rows4_max(tmax);
+    m_new = __builtin_fmaxf(m_run, tmax * scale2);
+    alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float pe = okv[e] ? __builtin_amdgcn_exp2f(__builtin_fmaf(st[e >> 2][e & 3], scale2, -m_new)) : 0.0f;
+      pb[e >> 3][e & 7] = (half_t)pe;
+      psum += pe;
+    }
+  }
+  l_run = l_run * alpha + psum;
+  if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) oacc[c] *= alpha;
+  }
+  m_run = m_new;
+}
+__device__ __forceinline__ void rows16_values(const uint8_t* vt, int tr_a0, const v8h (&pb)[2], v4f (&oacc)[8]) {
+  v8h a16[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int kk = i >> 3, c = i & 7;
+    const uint8_t* src = vt + (32 * kk) * PVROW + (tr_a0 ^ (c << 5));
+    const pv4hp lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+        (__attribute__((address_space(3))) pv4hp*)(__attribute__((address_space(3))) void*)(src));
+    const pv4hp hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+        (__attribute__((address_space(3))) pv4hp*)(__attribute__((address_space(3))) void*)(src + 16 * PVROW));
+    a16[i] = (v8h){(half_t)lo[0], (half_t)lo[1], (half_t)lo[2], (half_t)lo[3],
+                   (half_t)hi[0], (half_t)hi[1], (half_t)hi[2], (half_t)hi[3]};
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) oacc[i & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a16[i], pb[i >> 3], oacc[i & 7], 0, 0, 0);
+  __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+  for (int i = 0; i < 13; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+}
+
+// ------------------------------------------------------------------------------------------------------------------------
+// Few query tiles: 64 query rows a workgroup, four waves of 16, ONE K and ONE V buffer (32 KB of LDS, four workgroups on a CU).
+//
+// Where the 128-row kernel has about one workgroup on a CU, its eight waves go through scores, softmax and values in step (1.6 us a tile of 64
+// keys) and its longest query tile is the launch.  Here four workgroups of a CU, each at its own place, cover one another's waits; K of the next tile
+// is requested as soon as everyone has formed this one's scores and flies under softmax and values, V of it behind the values and flies under
+// the next scores and softmax.  The price is K and V brought in once per 64 rows, which is what large launches are short of.  A row meets the same
+// tiles in the same order: the same bits.
+// MI355X, 32 / 8 heads, 128 rows / here, us: one prompt of 129 tokens 9.6 / 7.9, 333 14.0 / 12.0, 1501 44.6 / 40.7, 2048 60.5 / 58.0, 4000 179 / 180, 8192 617 / 691;
+// 7 x 333 31.4 / 25.4, 16 x 375 57 / 48, 16 x 100 13.7 / 12.6, 4 x 1500 116 / 117; 3 x 801, 28 / 4 heads, 43.0 / 32.9.  (Two K and two V buffers, two
+// workgroups a CU: 1501 37.0, but 7 x 333 29.2, 16 x 375 59; two K buffers, three workgroups: 39.2, 25.6, 51.  Tiles sequence after sequence instead of
+// long ones first: 7 x 333 27.5, 3 x 801 37.6.)
+constexpr int SM_WAVES = 4, SM_ROWS = 16 * SM_WAVES;
+constexpr int SM_PIECES = PKT * 16 / (64 * SM_WAVES);      // 1-KiB pieces of a K (or V) tile per wave
+__global__ __launch_bounds__(64 * SM_WAVES, 4) __attribute__((amdgpu_waves_per_eu(4, 4), amdgpu_num_vgpr(128)))
+void prefill_attn_small_kernel(PrefillArgs p) {
+  __shared__ __attribute__((aligned(16))) uint8_t ktile[PKTILE];
+  __shared__ __attribute__((aligned(16))) uint8_t vtile[PVTILE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, l4 = lane >> 4;
+  int b = blockIdx.z, h = blockIdx.y, qt = gridDim.x - 1 - blockIdx.x;
+  if (p.q_tiles > 0 && !prefill_map_block<true>(p, b, h, qt)) return;
+  const int hk = h / (p.num_heads / p.num_kv_heads);
+  const int q_begin = p.cu_q[b], len_q = p.cu_q[b + 1] - q_begin;
+  const int k_begin = p.cu_k[b], len_k = p.cu_k[b + 1] - k_begin;
+  const int q_first = qt * SM_ROWS;
+  if (q_first >= len_q) return;
+  const int q_last = min(q_first + SM_ROWS, len_q) - 1;
+  const int off = len_k - len_q;
+  const bool streaming = p.head_mask_type != nullptr && p.head_mask_type[h] < 0;
+  const int gl = p.gran_log2;
+  const int sink = streaming ? p.streaming_info[2 * h] << gl : 0;
+  const int local = streaming ? p.streaming_info[2 * h + 1] : 0;
+  const int qrow = q_first + 16 * wave + l15;
+  const int k_hi = p.causal ? min(len_k, q_last + off + 1) : len_k;
+  const int win_lo = streaming ? first_local_key(q_first + off, local, gl) : 0;
+  auto next_tile = [&](int kb) {
+    while (kb < k_hi && streaming && kb >= sink && kb + PKT <= win_lo) kb += PKT;
+    return kb;
+  };
+  const uint8_t* kbase = reinterpret_cast<const uint8_t*>(p.k + (size_t)k_begin * p.k_stride + (size_t)hk * PDH);
+  const uint8_t* vbase = reinterpret_cast<const uint8_t*>(p.v + (size_t)k_begin * p.v_stride + (size_t)hk * PDH);
+  const uint32_t kstride_b = (uint32_t)(p.k_stride * 2), vstride_b = (uint32_t)(p.v_stride * 2);
+  // (source-side swizzles of the kernel above: K slot ^ (row & 15), V slot ^ 2 (row & 7))
+  auto request = [&](const uint8_t* base, uint32_t stride, int kb, uint8_t* tile, bool v) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));      // per-piece constants of the lane are formed here, not kept across the loop
+#pragma unroll
+    for (int i = 0; i < SM_PIECES; ++i) {
+      const int row = 4 * SM_PIECES * wave + 4 * i + (ln >> 4);
+      const uint32_t r = (uint32_t)min(kb + row, len_k - 1);
+      lds_dma16_untracked(base + ((uint64_t)r * stride + (uint32_t)(((ln & 15) ^ (v ? 2 * (row & 7) : row & 15)) << 4)),
+                          tile + (4 * SM_PIECES * wave + 4 * i) * PKROW);
+    }
+  };
+  // everyone has read the tile that is requested next; own reads are waited for first
+  auto barrier_read = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  int kb = next_tile(0);
+  if (kb < k_hi) {
+    request(kbase, kstride_b, kb, ktile, false);
+    request(vbase, vstride_b, kb, vtile, true);
+  }
+  v8h qb[4];
+  {
+    const int qr_c = qrow < len_q ? qrow : (len_q - 1);
+    const half_t* qp = p.q + (size_t)(q_begin + qr_c) * p.q_stride + (size_t)h * PDH + 8 * l4;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qb[s] = *reinterpret_cast<const v8h*>(qp + 32 * s);
+  }
+  v4f oacc[8];
+  float m_run = -1e30f, l_run = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) oacc[c] = (v4f){0.f, 0.f, 0.f, 0.f};
+  const int trow = 4 * l4 + (l15 >> 2);
+  const int tr_a0 = (trow * PVROW + (l15 & 3) * 8) | ((trow & 7) << 5);
+  lds_dma_wait_all();
+  __syncthreads();
+  while (kb < k_hi) {
+    const int kb_next = next_tile(kb + PKT);
+    const bool more = kb_next < k_hi;
+    v4f st[4];
+    v8h pb[2];
+    __builtin_amdgcn_s_setprio(1);
+    rows16_scores(ktile, l15, l4, qb, st);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_read();
+    if (more) request(kbase, kstride_b, kb_next, ktile, false);
+    __builtin_amdgcn_sched_barrier(0);
+    bool full = kb + PKT <= len_k;
+    if (p.causal) full = full && (kb + PKT - 1 <= q_first + off);
+    if (streaming) full = full && ((kb + PKT <= sink) || (kb >= first_local_key(q_last + off, local, gl)));
+    rows16_softmax(full, kb, l4, qrow, off, len_q, len_k, p.causal, streaming, sink, local, gl, st, pb, m_run, l_run, oacc);
+    __builtin_amdgcn_sched_barrier(0);
+    // V of this tile has landed: behind it only the SM_PIECES requests of the next K are in flight (none behind the last tile)
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SM_PIECES) : "memory");
+    else lds_dma_wait_all();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_setprio(1);
+    rows16_values(vtile, tr_a0, pb, oacc);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    lds_dma_wait_all();       // the next K tile
+    barrier_read();
+    if (more) request(vbase, vstride_b, kb_next, vtile, true);
+    kb = kb_next;
+  }
+  const float l = rows4_sum(l_run);
+  if (qrow >= len_q) return;
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  half_t* op = p.out + ((size_t)(q_begin + qrow) * p.num_heads + h) * PDH + 4 * l4;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<v4h_t*>(op + c * 16) = (v4h_t){(half_t)(oacc[c][0] * inv), (half_t)(oacc[c][1] * inv), (half_t)(oacc[c][2] * inv),
+                                                     (half_t)(oacc[c][3] * inv)};
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------------------
 // Ping-pong form of the 16-row kernel (omni_prefill_set_variant(2)).  Same tiles, layouts and arithmetic; what changes is WHEN the
 // two halves of the workgroup do what.  In the form above all eight waves run S -> softmax -> P.V in step behind one barrier per
 // tile, so on every SIMD the softmax's VALU issue and the MFMAs of the wave pair ADD UP instead of overlapping (profiles/r02_f:
@@ -412,7 +631,6 @@ void prefill_attn_pp_kernel(PrefillArgs p) {
   const int gl = p.gran_log2;
   const int sink = streaming ? p.streaming_info[2 * h] << gl : 0;
   const int local = streaming ? p.streaming_info[2 * h + 1] : 0;
-  const float scale2 = 0.08838834764831845f * 1.4426950408889634f;
   const int qrow = q0 + l15;
   v8h qb[4];
   {
@@ -438,93 +656,15 @@ void prefill_attn_pp_kernel(PrefillArgs p) {
   const int trow = 4 * l4 + (l15 >> 2);
   const int tr_a0 = (trow * PVROW + (l15 & 3) * 8) | ((trow & 7) << 5);
 
-  // ---- the three stages of a tile (the 16-row kernel's own code) ---------------------------------------------------------
-  auto stage_s = [&](const uint8_t* kt, v4f (&st)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) st[u] = (v4f){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int key = 16 * u + l15;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const v8h a = *reinterpret_cast<const v8h*>(kt + key * PKROW + (((4 * s + l4) ^ l15) << 4));
-        st[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[s], st[u], 0, 0, 0);
-      }
-    }
-  };
+  // ---- the three stages of a tile --------------------------------------------------------------------------------------
+  auto stage_s = [&](const uint8_t* kt, v4f (&st)[4]) { rows16_scores(kt, l15, l4, qb, st); };
   auto stage_softmax = [&](int kb, const v4f (&st)[4], v8h (&pb)[2]) {
-    bool full = (kb + PKT <= len_k) && (q_first + PQROWS <= len_q);
+    bool full = kb + PKT <= len_k;
     if (p.causal) full = full && (kb + PKT - 1 <= q_first + off);
     if (streaming) full = full && ((kb + PKT <= sink) || (kb >= first_local_key(q_last + off, local, gl)));
-    float tmax = -1e30f, m_new, alpha, psum = 0.0f;
-    if (full) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) tmax = __builtin_fmaxf(tmax, st[u][r]);
-      tmax = rows4_max(tmax);
-      m_new = __builtin_fmaxf(m_run, tmax * scale2);
-      alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(st[e >> 2][e & 3], scale2, -m_new));
-        pb[e >> 3][e & 7] = (half_t)pe;
-        psum += pe;
-      }
-    } else {
-      bool okv[16];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kb + 16 * u + 4 * l4 + r;
-          const int qpos = qrow + off;
-          int ok = (int)(key < len_k) & (int)(qrow < len_q);
-          ok &= (int)(!p.causal) | (int)(key <= qpos);
-          ok &= (int)(!streaming) | (int)(key < sink) | (int)(key >= first_local_key(qpos, local, gl));
-          okv[4 * u + r] = ok != 0;
-          tmax = __builtin_fmaxf(tmax, ok ? st[u][r] : -1e30f);
-        }
-      tmax = rows4_max(tmax);
-      m_new = __builtin_fmaxf(m_run, tmax * scale2);
-      alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float pe = okv[e] ? __builtin_amdgcn_exp2f(__builtin_fmaf(st[e >> 2][e & 3], scale2, -m_new)) : 0.0f;
-        pb[e >> 3][e & 7] = (half_t)pe;
-        psum += pe;
-      }
-    }
-    l_run = l_run * alpha + psum;
-    if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) oacc[c] *= alpha;
-    }
-    m_run = m_new;
+    rows16_softmax(full, kb, l4, qrow, off, len_q, len_k, p.causal, streaming, sink, local, gl, st, pb, m_run, l_run, oacc);
   };
-  auto stage_pv = [&](const uint8_t* vt, const v8h (&pb)[2]) {
-    v8h a16[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int kk = i >> 3, c = i & 7;
-      const uint8_t* src = vt + (32 * kk) * PVROW + (tr_a0 ^ (c << 5));
-      const pv4hp lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
-          (__attribute__((address_space(3))) pv4hp*)(__attribute__((address_space(3))) void*)(src));
-      const pv4hp hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
-          (__attribute__((address_space(3))) pv4hp*)(__attribute__((address_space(3))) void*)(src + 16 * PVROW));
-      a16[i] = (v8h){(half_t)lo[0], (half_t)lo[1], (half_t)lo[2], (half_t)lo[3],
-                     (half_t)hi[0], (half_t)hi[1], (half_t)hi[2], (half_t)hi[3]};
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[i & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a16[i], pb[i >> 3], oacc[i & 7], 0, 0, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-#pragma unroll
-    for (int i = 0; i < 13; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-  };
+  auto stage_pv = [&](const uint8_t* vt, const v8h (&pb)[2]) { rows16_values(vt, tr_a0, pb, oacc); };
   // barrier that opens a B segment: this wave's DMA pieces have landed, then everybody's
   auto barrier_landed = [&]() {
     lds_dma_wait_all();
@@ -816,7 +956,7 @@ void prefill_attn32_kernel(PrefillArgs p) {
     kb = kb_next;
   };
   auto is_full = [&](int kb_) {
-    bool full = (kb_ + PKT <= len_k) && (q_first + P32ROWS <= len_q);
+    bool full = kb_ + PKT <= len_k;
     if (p.causal) full = full && (kb_ + PKT - 1 <= q_first + off);
     if (streaming) full = full && ((kb_ + PKT <= sink) || (kb_ >= first_local_key(q_last + off, local, gl)));
     return full;
@@ -852,14 +992,21 @@ void prefill_attn32_kernel(PrefillArgs p) {
 using namespace omni;
 
 static thread_local int g_prefill_variant = OMNI_PREFILL_MFMA32;
-// Tuning / test hook: 0 = the 16-row form (default), 1 = the 32-row form.  Same results within the attention tolerance.
-extern "C" void omni_prefill_set_variant(int variant) { g_prefill_variant = (variant == 1 || variant == 2) ? variant : 0; }
+// Tuning / test hook: 0 = by size (default): 128-row workgroups or, of few tiles, 64-row ones; 1 = the 32-row form, 2 = the ping-pong form, 3 / 4 = always
+// 64 / 128 rows.  Same results within the attention tolerance (0, 3 and 4: the same bits).
+extern "C" void omni_prefill_set_variant(int variant) { g_prefill_variant = (variant >= 1 && variant <= 4) ? variant : 0; }
 #ifndef OMNI_PREFILL_XCD_SPLIT_MASKED
 #define OMNI_PREFILL_XCD_SPLIT_MASKED 8
 #endif
 static thread_local int g_prefill_xcd_split = 0;
 // Tuning hook: XCDs that share one kv head's query tiles when streaming heads are present (0 = default, else 1 / 2 / 4 / 8).
 extern "C" void omni_prefill_set_xcd_split(int w) { g_prefill_xcd_split = (w == 1 || w == 2 || w == 4 || w == 8) ? w : 0; }
+
+// 64-row workgroups?  Less than one round of two 128-row ones on every CU, or short prompts (figures at prefill_attn_small_kernel); longer keys than
+// queries, which the host cannot see (another array of offsets), count as long ones.
+static bool small_tiles(int batch, int max_seqlen_q, int num_heads, bool self) {
+  return (self && max_seqlen_q <= 1024) || (long long)batch * num_heads * ((max_seqlen_q + PQROWS - 1) / PQROWS) < 512;
+}
 
 static int prefill_attention_common(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16,
                                     int64_t q_stride, int64_t k_stride, int64_t v_stride,
@@ -880,8 +1027,9 @@ static int prefill_attention_common(void* out_f16, const void* q_f16, const void
   a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.causal = causal;
   a.gran_log2 = gran_log2;
   const bool form32 = g_prefill_variant == 1;
+  const bool small = g_prefill_variant == 3 || (g_prefill_variant == 0 && small_tiles(batch, max_seqlen_q, num_heads, cu_seqlens_q_i32 == cu_seqlens_k_i32));
   const int rows_per_wg = form32 ? P32ROWS : PQROWS;
-  const int q_tiles = (max_seqlen_q + rows_per_wg - 1) / rows_per_wg;
+  const int q_tiles = (max_seqlen_q + rows_per_wg - 1) / rows_per_wg * (small ? PQROWS / SM_ROWS : 1);
   dim3 grid(q_tiles, num_heads, batch);
   a.q_tiles = 0;
   a.xcd_split = 1;
@@ -900,6 +1048,7 @@ static int prefill_attention_common(void* out_f16, const void* q_f16, const void
     }
   }
   if (form32) hipLaunchKernelGGL(prefill_attn32_kernel, grid, dim3(64 * P32W), 0, (hipStream_t)stream, a);
+  else if (small) hipLaunchKernelGGL(prefill_attn_small_kernel, grid, dim3(64 * SM_WAVES), 0, (hipStream_t)stream, a);
   else if (g_prefill_variant == 2) hipLaunchKernelGGL(prefill_attn_pp_kernel, grid, dim3(64 * PWAVES), 0, (hipStream_t)stream, a);
   else hipLaunchKernelGGL(prefill_attn_kernel, grid, dim3(64 * PWAVES), 0, (hipStream_t)stream, a);
   return omni_launch_status();
