@@ -24,6 +24,8 @@ extern "C" {
 #define LM_ACT_SIGMOID 3
 #define LM_TILE_ROWS 256 /* rows of one lm_gemm_tiles tile */
 #define LM_ATTN_ROWS 128 /* query rows of one lm_attn_prefill tile */
+#define LM_CHOOSE_TOKENS 32 /* tokens of one lm_norm_choose at most */
+#define LM_MAX_TOP 16 /* experts of a token at most */
 
 int lm_abi_version(void);
 int lm_elem_bytes(void);
@@ -131,6 +133,13 @@ int lm_route_max_tiles(int tokens, int experts, int top);
 int lm_route(const float* z, int64_t ldz, const float* bias, int tokens, int experts, int top, float* wts, int* off, int* perm,
              int* tiles, int* scratch_i32, void* stream);
 
+/* Few tokens: lm_residual_norm (x += norm(y; post); h = norm(x; next), h of ldh = k elements), the router's product of h (router [experts, up to a multiple of 16][k], zero
+ * rows behind the last expert) and the choice of lm_route in one launch -> wts [tokens][top], ids [tokens][top] (experts).  lm_norm_choose_ok: for these sizes. */
+int lm_norm_choose_ok(int tokens, int k, int experts, int top);
+int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy, const float* post_w, const float* post_b, const float* next_w, const float* next_b,
+                   void* h, int64_t ldh, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top,
+                   float* wts, int* ids, void* stream);
+
 /* y = x w^T for one or many matrices w [groups][n][k].  perm null: rows_a rows, group g reads x from column g * gx and writes y
  * from column g * gy (several groups: lm_gemm_rows only).  Else group g has the places off[g] .. off[g + 1] of perm; a place's y
  * row is perm[place], its x row perm[place] / x_div.  b (optional): one more matrix over rows 0 .. rows_b - 1 of its own x and y.
@@ -157,6 +166,11 @@ int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi);
 int lm_gemm_rows_channels(int groups, int n, int k, int rows, int epi, int sliced, int* slices);
 int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, int rows_a, int rows_b,
                  int x_div, int max_rows, float scale, int epi, int act, float* part, void* stream);
+/* The same over choices that are not sorted: group g has the pairs (token * top + choice) whose entry of ids is g; a pair's y row is its number, its x row that or (x_is_pairs
+ * 0) its token.  b over rows 0 .. tokens - 1.  Outputs are those of lm_gemm_rows with lm_route's order.  lm_gemm_chosen_ok: for these sizes; epi LM_EPI_ELEM or LM_EPI_GLU. */
+int lm_gemm_chosen_ok(int groups, int n, int k, int tokens, int top, int epi);
+int lm_gemm_chosen(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* ids, int tokens, int top, int x_is_pairs, float scale, int epi,
+                   int act, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,
                   int max_tiles, int rows_a, int rows_b, int x_div, float scale, int epi, int act, void* stream);
 /* Channels of the tiles (128 or 256) that lm_gemm_tiles takes; max_tiles 0: one matrix over rows_a rows; n_b, k_b, rows_b: part b, or 0. */

@@ -61,6 +61,10 @@ PROTOTYPES = {
     "lm_route_scratch_words": (_i64, [_i, _i, _i]),
     "lm_route_max_tiles": (_i, [_i, _i, _i]),
     "lm_route": (_i, [_vp, _i64, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "lm_norm_choose_ok": (_i, [_i] * 4),
+    "lm_norm_choose": (_i, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _i, _f, _vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
+    "lm_gemm_chosen_ok": (_i, [_i] * 6),
+    "lm_gemm_chosen": (_i, [_PP, _PP, _i, _vp, _i, _i, _i, _f, _i, _i, _vp]),
     "lm_gemm_rows_scratch": (_i64, [_i, _i, _i, _i]),
     "lm_gemm_rows_channels": (_i, [_i] * 6 + [_c.POINTER(_i)]),
     "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp]),
@@ -245,15 +249,38 @@ class LmOps:
         self._call("lm_route", _p(z), _ld(z), _p(bias), T, experts, top, _p(wts), _p(off), _p(perm), _p(tiles), _p(scratch))
         return wts, (off, perm, tiles, max_tiles, top)
 
+    def chooses(self, tokens, router, experts, top, w_in, w_out):
+        """Do norm_choose and products over its unsorted choices exist for these sizes?  w_in, w_out: all experts' matrices"""
+        ok = self._h.lm_gemm_chosen_ok
+        return bool(self._h.lm_norm_choose_ok(tokens, router.shape[1], experts, top) and ok(*w_in.shape, tokens, top, EPI_GLU)
+                    and ok(*w_out.shape, tokens, top, EPI_ELEM))
+
+    def norm_choose(self, x, n, kind, eps, y, post, next, h, router, bias, experts, top):
+        """residual_norm, the router's product of h and route in one launch -> (weights [T, top], the choices for grouped)"""
+        T = x.shape[0]
+        if not (h.is_contiguous() and router.is_contiguous() and h.shape == (T, router.shape[1]) and router.shape[0] == (experts + 15) // 16 * 16):
+            raise ValueError("norm_choose: h [tokens, k] and router [experts (a multiple of 16), k], both contiguous")
+        wts = torch.empty((T, top), dtype=torch.float32, device=x.device)
+        ids = torch.empty((T, top), dtype=torch.int32, device=x.device)
+        post = post or (None, None)
+        self._call("lm_norm_choose", _p(x), _ld(x), _p(y), _ld(y), _p(post[0]), _p(post[1]), _p(next[0]), _p(next[1]), _p(h), _ld(h), T, n, NORM[kind], eps,
+                   _p(router), _p(bias), router.shape[1], experts, top, _p(wts), _p(ids))
+        return wts, ids
+
     def grouped(self, order, tokens, x, w, y, x_is_pairs, glu, extra=None):
-        """Expert products: w [experts, n, k]; x rows per token or per (token, choice); extra = (x, w, y) of the shared expert."""
-        off, perm, tiles, max_tiles, top = order
+        """Expert products: w [experts, n, k]; x rows per token or per (token, choice); extra = (x, w, y) of the shared expert.  order: route's, or
+        the choices of norm_choose."""
         a = _Part(_p(w), _p(x), _ld(x), _p(y), _ld(y), w.shape[1], w.shape[2])
         b = None
         if extra is not None:
             b = _Part(_p(extra[1]), _p(extra[0]), _ld(extra[0]), _p(extra[2]), _ld(extra[2]), extra[1].shape[0], extra[1].shape[1])
         pb = None if b is None else _c.byref(b)
-        epi, div, rb = (EPI_GLU if glu else EPI_ELEM), (1 if x_is_pairs else top), (tokens if b is not None else 0)
+        epi = EPI_GLU if glu else EPI_ELEM
+        if torch.is_tensor(order):
+            self._call("lm_gemm_chosen", _c.byref(a), pb, w.shape[0], _p(order), tokens, order.shape[1], int(x_is_pairs), 1.0, epi, ACT["silu"])
+            return
+        off, perm, tiles, max_tiles, top = order
+        div, rb = (1 if x_is_pairs else top), (tokens if b is not None else 0)
         if tiles is None:
             self._call("lm_gemm_rows", _c.byref(a), pb, w.shape[0], _p(perm), _p(off), 0, rb, div, tokens, 1.0, epi, ACT["silu"], None)
         else:

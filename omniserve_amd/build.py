@@ -40,7 +40,7 @@ FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=
 
 LM_CSRC = os.path.join(CSRC, "lm")
 LM_SOURCES = ["lm_rows.hip", "lm_gemm.hip", "lm_route.hip", "lm_attn.hip", "lm_attn_decode.hip", "lm_linear_attn.hip",
-              "lm_latent.hip", "lm_gla.hip", "lm_delta.hip", "lm_gemm_half.hip"]
+              "lm_latent.hip", "lm_gla.hip", "lm_delta.hip", "lm_gemm_half.hip", "lm_norm_choose.hip"]
 LM_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", *NO_PACKED_F32, "-Wall", "-Wno-unused-function",
             "-I" + LM_CSRC, "-I" + INCLUDE]
 LM_ELEM = {"bf16": 0, "f32": 1}        # -DLM_ELEM=<n>

@@ -5,6 +5,13 @@
 
 namespace lm {
 
+template <int N> struct Int { static constexpr int value = N; };
+template <int J, typename F>
+__device__ __forceinline__ void countdown(F&& f) {      // f(J), f(J - 1), ..., f(0)
+  f(Int<J>{});
+  if constexpr (J > 0) countdown<J - 1>(f);
+}
+
 struct Part {        // a family of equally shaped groups
   const elem_t* w;   // [groups][n][k]
   const elem_t* x; int64_t ldx;
@@ -26,6 +33,8 @@ struct GemmArgs {
   const int* tiles;           // lm_gemm_tiles with perm: (group, first place, rows, 0) of every row tile, rows 0: none
   float scale;
   int act;                    // of the gated unit
+  const int* ids;             // chosen form: the expert of every (token, choice) pair, from which a workgroup finds its own (perm, off: null)
+  int pairs;
 };
 
 __device__ __forceinline__ f32x4 glu(const Part& pt, int act, int c, f32x4 gate, f32x4 up) {      // c: gate channel's row in w, a multiple of 4

@@ -13,13 +13,6 @@
 
 namespace lm {
 
-template <int N> struct Int { static constexpr int value = N; };
-template <int J, typename F>
-__device__ __forceinline__ void countdown(F&& f) {      // f(J), f(J - 1), ..., f(0)
-  f(Int<J>{});
-  if constexpr (J > 0) countdown<J - 1>(f);
-}
-
 // A workgroup owns NR 16-channel blocks; its KW waves split K and meet in LDS.  16 MB rows at a time; blockIdx.z takes every
 // gridDim.z-th such part.
 template <int NR, int MB, int KW, int EPI>
@@ -294,9 +287,12 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 
 // A workgroup: 16 NW channels of a group, rows 0 .. 16 MB - 1 of it, K slice blockIdx.z.  With several slices (one group) the f32 sums of a
 // slice go to part [slice][rows][n] and gemm_reduce_kernel finishes them.
-template <int EPI, int NW, int KW, bool SHORT, bool TURN>
+// IDS: the rows of a group are the pairs whose expert it is: every wave looks through the choices (a load per 64 pairs, all at once), one of them notes
+// the places.  Their order does not matter: a row's sums are its own.
+template <int EPI, int NW, int KW, bool SHORT, bool TURN, bool IDS = false>
 __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, float* part) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[KW * ring_bytes<NW, KW>];
+  __shared__ int own[IDS ? LM_CHOOSE_TOKENS : 1];
   constexpr int RC = 16 * NW, NT = 64 * NW * KW;
   const int g = blockIdx.y, tid = threadIdx.x;
   const bool is_b = g >= p.groups;
@@ -305,19 +301,44 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
   if (n0 >= pt.n) return;
   int first = 0, rows = is_b ? p.rows_b : p.rows_a;
   const int* perm = is_b ? nullptr : p.perm;
-  if (perm) { first = p.off[g]; rows = p.off[g + 1] - first; perm += first; }
+  if (IDS && !is_b) {
+    const int lane = tid & 63;
+    rows = 0;
+    auto look = [&](auto chunks) {
+      constexpr int CHUNKS = decltype(chunks)::value;
+      int e[CHUNKS];
+#pragma unroll
+      for (int i = 0; i < CHUNKS; ++i) e[i] = p.ids[min(64 * i + lane, p.pairs - 1)];
+#pragma unroll
+      for (int i = 0; i < CHUNKS; ++i) {
+        const bool it = e[i] == g && 64 * i + lane < p.pairs;
+        const uint64_t mine = __builtin_amdgcn_ballot_w64(it);
+        const int at = rows + __builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0));
+        if (tid < 64 && it && at < LM_CHOOSE_TOKENS) own[at] = 64 * i + lane;
+        rows += __builtin_popcountll(mine);
+      }
+    };
+    if (p.pairs <= 128) look(Int<2>{});
+    else look(Int<LM_CHOOSE_TOKENS * LM_MAX_TOP / 64>{});
+    rows = min(rows, LM_CHOOSE_TOKENS);      // (a token chooses an expert once)
+    perm = own;
+    if (rows > 0) __syncthreads();
+  } else if (perm) {
+    first = p.off[g]; rows = p.off[g + 1] - first; perm += first;
+  }
   if (rows <= 0) return;
   const elem_t* w = pt.w + (is_b ? 0 : (int64_t)g * pt.n * pt.k);
   const int64_t x0 = is_b || perm ? 0 : g * pt.gx, y0 = is_b || perm ? 0 : g * pt.gy;
   const int stages = pt.k * (int)sizeof(elem_t) / RB, slice = blockIdx.z, slices = gridDim.z;
   const int s0 = stages * slice / slices, s1 = stages * (slice + 1) / slices;
   const int div = is_b ? 1 : p.x_div;
-  for (int m0 = 0; m0 < rows; m0 += 64) {
+  static_assert(!IDS || LM_CHOOSE_TOKENS <= 32, "rows of a chosen group");
+  for (int m0 = 0; m0 < (IDS ? 1 : rows); m0 += 64) {
     const int here = min(64, rows - m0), mb = (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
     const int* pm = perm ? perm + m0 : nullptr;
     if (mb == 1) stream_stages<1, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
-    else if (mb == 2) stream_stages<2, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (IDS || mb == 2) stream_stages<2, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     else if (mb == 3) stream_stages<3, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     else stream_stages<4, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     const float* red = (const float*)lds;
@@ -684,7 +705,7 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   a.b = pb ? conv(pb) : Part{};
   if (check_part(a.a, epi, act) || (pb && check_part(a.b, epi, act))) return LM_EINVAL;
   a.groups = groups; a.perm = perm; a.off = off; a.rows_a = rows_a; a.rows_b = pb ? rows_b : 0; a.x_div = perm ? x_div : 1;
-  a.tiles = nullptr; a.scale = scale; a.act = act;
+  a.tiles = nullptr; a.scale = scale; a.act = act; a.ids = nullptr; a.pairs = 0;
   return LM_OK;
 }
 
@@ -732,14 +753,14 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
 }
 
 // K parts inside a workgroup where there is no second one to run beside it on its CU
-template <int EPI, int NW, bool SHORT, bool TURN = false>
+template <int EPI, int NW, bool SHORT, bool TURN = false, bool IDS = false>
 static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
   constexpr int KW = NW <= 2 ? 4 : NW <= 5 ? 2 : 1;
   if (KW > 1 && (int64_t)grid.x * grid.y * grid.z <= 256)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT, TURN>), grid, dim3(64 * NW * KW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT, TURN, IDS>), grid, dim3(64 * NW * KW), 0, s, a, part);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT, TURN>), grid, dim3(64 * NW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT, TURN, IDS>), grid, dim3(64 * NW), 0, s, a, part);
 }
 
 // bf16: heads, and gated units of 128 channels, in one slice: workgroups that begin at different k where rows lie whole 4 KiBs apart and are enough to be bound by the memory's
@@ -845,6 +866,40 @@ extern "C" int lm_gemm_rows(const LmGemmPart* pa, const LmGemmPart* pb, int grou
   if (epi == LM_EPI_GLU) return launch_few<LM_EPI_GLU>(a, max_rows, has_b, part, s);
   if (epi == LM_EPI_GATE) return launch_few<LM_EPI_GATE>(a, max_rows, has_b, part, s);
   return epi == LM_EPI_F32 ? launch_few<LM_EPI_F32>(a, max_rows, has_b, part, s) : launch_few<LM_EPI_ELEM>(a, max_rows, has_b, part, s);
+}
+
+// are the products of a mixture of experts those of gemm_stream_kernel with 64 channels?
+static bool chosen_streams(int groups, int n, int k, int tokens, int epi) { return plan_rows(groups, n, k, tokens, epi, true, false).nw == 4; }
+
+extern "C" int lm_gemm_chosen_ok(int groups, int n, int k, int tokens, int top, int epi) {
+  return LM_ELEM == 0 && groups > 0 && n > 0 && k > 0 && tokens > 0 && tokens <= LM_CHOOSE_TOKENS && top > 0 && top <= LM_MAX_TOP && (epi == LM_EPI_GLU || epi == LM_EPI_ELEM) &&
+         chosen_streams(groups, n, k, tokens, epi);
+}
+
+extern "C" int lm_gemm_chosen(const LmGemmPart* pa, const LmGemmPart* pb, int groups, const int* ids, int tokens, int top, int x_is_pairs, float scale, int epi, int act,
+                              void* stream) {
+#if LM_ELEM == 0
+  GemmArgs a;
+  if (!ids || tokens <= 0 || top <= 0 || fill(a, pa, pb, groups, nullptr, nullptr, 0, tokens, x_is_pairs ? 1 : top, scale, epi, act)) return LM_EINVAL;
+  const int has_b = pb != nullptr, n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
+  if (!lm_gemm_chosen_ok(groups, n, a.a.k, tokens, top, epi)) return LM_EINVAL;
+  uintptr_t at = (uintptr_t)a.a.w | (uintptr_t)a.a.x;
+  if (has_b) at |= (uintptr_t)a.b.w | (uintptr_t)a.b.x;
+  if (at & 15) return LM_EINVAL;
+  a.ids = ids; a.pairs = tokens * top; a.x_div = x_is_pairs ? 1 : top;
+  hipStream_t s = (hipStream_t)stream;
+  const bool is_short = a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K);
+  if (epi == LM_EPI_GLU) {
+    if (is_short) launch_stream_form<LM_EPI_GLU, 4, true, false, true>(a, n, has_b, 1, nullptr, s);
+    else launch_stream_form<LM_EPI_GLU, 4, false, false, true>(a, n, has_b, 1, nullptr, s);
+  } else {
+    if (is_short) launch_stream_form<LM_EPI_ELEM, 4, true, false, true>(a, n, has_b, 1, nullptr, s);
+    else launch_stream_form<LM_EPI_ELEM, 4, false, false, true>(a, n, has_b, 1, nullptr, s);
+  }
+  return launch_status();
+#else
+  return LM_EINVAL;
+#endif
 }
 
 extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {

@@ -559,10 +559,15 @@ class MixtureOfExperts:
             self.shared_in = pair_rows(w.matrix("shared.gate", s.shared_ff, width), w.matrix("shared.up", s.shared_ff, width), self.FS, W)
             self.shared_out = padded(w.matrix("shared.down", width, s.shared_ff), W, self.FS)
 
-    def __call__(self, h):
-        """-> (rows by (token, choice), then by token for the shared expert; arguments of LmOps.residual_norm that sum them)"""
+    def chooses(self, tokens):
+        """Can the norm in front of it choose the experts too (LmOps.norm_choose)?"""
+        return self.ops.chooses(tokens, self.router, self.s.experts, self.s.top, self.w_in, self.w_out)
+
+    def __call__(self, h, chosen=None):
+        """-> (rows by (token, choice), then by token for the shared expert; arguments of LmOps.residual_norm that sum them).  chosen: what
+        LmOps.norm_choose returned."""
         s, ops, T = self.s, self.ops, h.shape[0]
-        wts, order = ops.route(ops.matmul(h, self.router, out_f32=True), self.bias, s.experts, s.top)
+        wts, order = chosen or ops.route(ops.matmul(h, self.router, out_f32=True), self.bias, s.experts, s.top)
         pairs, new = T * s.top, lambda r, c: torch.empty((r, c), dtype=h.dtype, device=h.device)      # noqa: E731
         act, y = new(pairs, self.F), new(pairs + (T if s.shared_ff else 0), self.W)
         up = down = None
@@ -668,8 +673,11 @@ class Decoder(EngineModel):
                 y = L.mixer(h, b, *cache.state[self._state[i]])
             form, post = {}, L.post
             if L.ff is not None:
-                norm(y=y, post=post, next=L.ff_pre, h=h)
-                y, form = L.ff(h)
+                if L.ff_pre and isinstance(L.ff, MixtureOfExperts) and L.ff.chooses(T):
+                    y, form = L.ff(h, ops.norm_choose(x, spec.width, spec.norm, spec.eps, y, post, L.ff_pre, h, L.ff.router, L.ff.bias, L.ff.s.experts, L.ff.s.top))
+                else:
+                    norm(y=y, post=post, next=L.ff_pre, h=h)
+                    y, form = L.ff(h)
                 post = L.ff_post
             if i < last:
                 norm(y=y, post=post, next=self.layers[i + 1].pre, h=h, **form)
