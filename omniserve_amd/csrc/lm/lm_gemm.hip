@@ -289,7 +289,8 @@ __device__ __forceinline__ void stream_stages(uint8_t* lds, const elem_t* w, int
 // slice go to part [slice][rows][n] and gemm_reduce_kernel finishes them.
 // IDS: the rows of a group are the pairs whose expert it is: every wave looks through the choices (a load per 64 pairs, all at once), one of them notes
 // the places.  Their order does not matter: a row's sums are its own.
-template <int EPI, int NW, int KW, bool SHORT, bool TURN, bool IDS = false>
+// ROWS16: blocks of 16 rows that there are (0: up to four).
+template <int EPI, int NW, int KW, bool SHORT, bool TURN, bool IDS, int ROWS16>
 __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, float* part) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[KW * ring_bytes<NW, KW>];
   __shared__ int own[IDS ? LM_CHOOSE_TOKENS : 1];
@@ -334,10 +335,11 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
   const int div = is_b ? 1 : p.x_div;
   static_assert(!IDS || LM_CHOOSE_TOKENS <= 32, "rows of a chosen group");
   for (int m0 = 0; m0 < (IDS ? 1 : rows); m0 += 64) {
-    const int here = min(64, rows - m0), mb = (here + 15) >> 4;
+    const int here = min(64, rows - m0), mb = ROWS16 ? ROWS16 : (here + 15) >> 4;
     const elem_t* x = pt.x + x0 + (perm ? 0 : m0 * pt.ldx);
     const int* pm = perm ? perm + m0 : nullptr;
-    if (mb == 1) stream_stages<1, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    if constexpr (ROWS16 > 0) stream_stages<ROWS16, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
+    else if (mb == 1) stream_stages<1, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     else if (IDS || mb == 2) stream_stages<2, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     else if (mb == 3) stream_stages<3, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
     else stream_stages<4, NW, KW, SHORT, TURN>(lds, w, pt.n, pt.k, n0, x, pt.ldx, pm, div, here, s0, s1);
@@ -753,14 +755,39 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
 }
 
 // K parts inside a workgroup where there is no second one to run beside it on its CU
-template <int EPI, int NW, bool SHORT, bool TURN = false, bool IDS = false>
-static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+template <int EPI, int NW, bool SHORT, bool TURN, bool IDS, int ROWS16>
+static void launch_stream_rows(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   const dim3 grid((n + 16 * NW - 1) / (16 * NW), a.groups + has_b, slices);
   constexpr int KW = NW <= 2 ? 4 : NW <= 5 ? 2 : 1;
   if (KW > 1 && (int64_t)grid.x * grid.y * grid.z <= 256)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT, TURN, IDS>), grid, dim3(64 * NW * KW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, KW, SHORT, TURN, IDS, ROWS16>), grid, dim3(64 * NW * KW), 0, s, a, part);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT, TURN, IDS>), grid, dim3(64 * NW), 0, s, a, part);
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI, NW, 1, SHORT, TURN, IDS, ROWS16>), grid, dim3(64 * NW), 0, s, a, part);
+}
+// One matrix, or one per head: a kernel for the very number of row blocks.  A kernel with all four in it keeps more in registers than it has scalar ones.
+// (MI355X, bf16, 64 rows, all in one | this: 28672 x 4096 gated 41.9 | 40.8 us, 12352 x 4096 28.0 | 26.1, 10816 x 4096 24.6 | 23.5, 32000 x 4096 45.9 | 44.4; 16 rows of 32000 x 2048
+// 23.7 | 23.2, of 2048 x 2048 6.1 | 5.9.)  Experts' rows are known on the device only.
+template <int EPI, int NW, bool SHORT, bool TURN = false, bool IDS = false>
+static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
+  if constexpr (!IDS && LM_ELEM == 0) {
+    if (!a.perm && !has_b && a.rows_a > 64) {      // (in one slice)
+      for (int m = 0; m < a.rows_a; m += 64) {
+        GemmArgs c = a;
+        c.rows_a = min(64, a.rows_a - m);
+        c.a.x += m * a.a.ldx;
+        c.a.y = (uint8_t*)a.a.y + m * a.a.ldy * (EPI == LM_EPI_F32 ? (int64_t)sizeof(float) : (int64_t)sizeof(elem_t));
+        if (EPI == LM_EPI_GATE) c.a.gate += m * a.a.ldg;
+        launch_stream_form<EPI, NW, SHORT, TURN, IDS>(c, n, has_b, slices, part, s);
+      }
+      return;
+    }
+    const int blocks = a.perm || has_b ? 0 : (a.rows_a + 15) / 16;
+    if (blocks == 1) return launch_stream_rows<EPI, NW, SHORT, TURN, IDS, 1>(a, n, has_b, slices, part, s);
+    if (blocks == 2) return launch_stream_rows<EPI, NW, SHORT, TURN, IDS, 2>(a, n, has_b, slices, part, s);
+    if (blocks == 3) return launch_stream_rows<EPI, NW, SHORT, TURN, IDS, 3>(a, n, has_b, slices, part, s);
+    if (blocks == 4) return launch_stream_rows<EPI, NW, SHORT, TURN, IDS, 4>(a, n, has_b, slices, part, s);
+  }
+  if constexpr (NW == 4 || LM_ELEM != 0) launch_stream_rows<EPI, NW, SHORT, TURN, IDS, 0>(a, n, has_b, slices, part, s);      // (experts: 64 channels a workgroup)
 }
 
 // bf16: heads, and gated units of 128 channels, in one slice: workgroups that begin at different k where rows lie whole 4 KiBs apart and are enough to be bound by the memory's
