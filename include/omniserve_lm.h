@@ -42,6 +42,11 @@ int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const void* embed
                      const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n, int kind, int store_x, float eps,
                      void* stream);
 
+/* The same with y as lm_gemm_sums leaves it: f32 sums [slices][sum_rows][ld] of K slices, added up and rounded to elem first. */
+int lm_residual_norm_sums(float* x, int64_t ldx, const float* sums, int64_t ld, int slices, int sum_rows, const float* y_bias, const float* post_w,
+                          const float* post_b, const float* next_w, const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n,
+                          int kind, int store_x, float eps, void* stream);
+
 /* out = rms_norm(o) * w * sigmoid(gate); n real columns of cols */
 int lm_gated_rms(void* out, int64_t ldo, const void* o, int64_t ldi, const void* gate, int64_t ldg, const float* w, int rows, int cols,
                  int n, float eps, void* stream);
@@ -171,6 +176,9 @@ int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int
 int lm_gemm_chosen_ok(int groups, int n, int k, int tokens, int top, int epi);
 int lm_gemm_chosen(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* ids, int tokens, int top, int x_is_pairs, float scale, int epi,
                    int act, void* stream);
+/* lm_gemm_rows of one matrix whose K is cut into slices (lm_gemm_rows_scratch() > 0 for LM_EPI_ELEM; w and x at multiples of 16 bytes), without the addition of the
+ * slices' sums [slices][rows][n]; y of the part is not written. */
+int lm_gemm_sums(const LmGemmPart* a, int rows, float* sums, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,
                   int max_tiles, int rows_a, int rows_b, int x_div, float scale, int epi, int act, void* stream);
 /* Channels of the tiles (128 or 256) that lm_gemm_tiles takes; max_tiles 0: one matrix over rows_a rows; n_b, k_b, rows_b: part b, or 0. */

@@ -36,6 +36,7 @@ PROTOTYPES = {
     "lm_abi_version": (_i, []),
     "lm_elem_bytes": (_i, []),
     "lm_residual_norm": (_i, [_vp, _i64, _vp, _vp, _f, _vp, _i64, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i, _i, _i, _i, _f, _vp]),
+    "lm_residual_norm_sums": (_i, [_vp, _i64, _vp, _i64, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i, _i, _i, _i, _f, _vp]),
     "lm_gated_rms": (_i, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i, _i, _i, _f, _vp]),
     "lm_rope_append": (_i, [_vp, _i64, _vp, _i64, _f, _vp, _i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "lm_attn_prefill": (_i, [_vp, _i64, _vp, _i64, _i, _i, _vp, _i64, _i, _i, _vp, _i, _vp, _vp, _i, _vp, _i64, _vp, _i64, _f, _i, _i, _i, _i, _i, _vp]),
@@ -65,6 +66,7 @@ PROTOTYPES = {
     "lm_norm_choose": (_i, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _i, _f, _vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "lm_gemm_chosen_ok": (_i, [_i] * 6),
     "lm_gemm_chosen": (_i, [_PP, _PP, _i, _vp, _i, _i, _i, _f, _i, _i, _vp]),
+    "lm_gemm_sums": (_i, [_PP, _i, _vp, _vp]),
     "lm_gemm_rows_scratch": (_i64, [_i, _i, _i, _i]),
     "lm_gemm_rows_channels": (_i, [_i] * 6 + [_c.POINTER(_i)]),
     "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp]),
@@ -105,12 +107,18 @@ class LmOps:
 
     def residual_norm(self, x, n, kind, eps, *, tokens=None, embed=None, embed_scale=1.0, y=None, y_bias=None, experts=None, post=None,
                       next=None, h=None, rows=None, store_x=True):
-        """experts: (pair weights [tokens, top], shared) when y holds expert rows; post / next: (weight, bias or None); h without
-        next: the new residual itself."""
+        """y: rows, or what sums returned; experts: (pair weights [tokens, top], shared) when y holds expert rows; post / next: (weight, bias
+        or None); h without next: the new residual itself."""
         pw, shared = experts if experts is not None else (None, False)
         top = pw.shape[1] if pw is not None else 0
         pairs = pw.numel() if pw is not None else 0
         post, nxt = post or (None, None), next or (None, None)
+        if y is not None and y.dim() == 3:
+            if tokens is not None or pw is not None:
+                raise ValueError("K slices of a product are neither embeddings nor expert rows")
+            self._call("lm_residual_norm_sums", _p(x), _ld(x), _p(y), y.shape[2], y.shape[0], y.shape[1], _p(y_bias), _p(post[0]), _p(post[1]), _p(nxt[0]), _p(nxt[1]),
+                       _p(h), _ld(h), _p(rows), x.shape[0] if rows is None else rows.numel(), n, NORM[kind], int(store_x), eps)
+            return
         self._call("lm_residual_norm", _p(x), _ld(x), _p(tokens), _p(embed), embed_scale, _p(y), _ld(y), _p(y_bias), _p(pw), top, pairs, int(bool(shared)),
                    _p(post[0]), _p(post[1]), _p(nxt[0]), _p(nxt[1]), _p(h), _ld(h), _p(rows),
                    x.shape[0] if rows is None else rows.numel(), n, NORM[kind], int(store_x), eps)
@@ -209,6 +217,16 @@ class LmOps:
             self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, scale, epi, 0, _p(sums))
         else:
             self._call("lm_gemm_tiles", _c.byref(part), None, 1, None, None, None, 0, T, 0, 1, scale, epi, 0)
+        return out
+
+    def sums(self, x, w):
+        """x w^T for residual_norm: where few rows are multiplied in K slices, their f32 sums [slices, T, n] (residual_norm adds them up: a launch less), else matmul's rows"""
+        T, (n, k) = x.shape[0], w.shape
+        room = self._h.lm_gemm_rows_scratch(n, k, T, EPI_ELEM) if T <= ROWS_MAX and (_p(x) | _p(w)) % 16 == 0 else 0
+        if room == 0:
+            return self.matmul(x, w)
+        out = torch.empty((room // (T * n), T, n), dtype=torch.float32, device=x.device)
+        self._call("lm_gemm_sums", _c.byref(_Part(_p(w), _p(x), _ld(x), _p(out), n, n, k)), T, _p(out))
         return out
 
     def glu(self, x, w, bias, act):

@@ -35,6 +35,7 @@ struct GemmArgs {
   int act;                    // of the gated unit
   const int* ids;             // chosen form: the expert of every (token, choice) pair, from which a workgroup finds its own (perm, off: null)
   int pairs;
+  int leave;                  // the K slices' sums stay as they are
 };
 
 __device__ __forceinline__ f32x4 glu(const Part& pt, int act, int c, f32x4 gate, f32x4 up) {      // c: gate channel's row in w, a multiple of 4

@@ -707,7 +707,7 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   a.b = pb ? conv(pb) : Part{};
   if (check_part(a.a, epi, act) || (pb && check_part(a.b, epi, act))) return LM_EINVAL;
   a.groups = groups; a.perm = perm; a.off = off; a.rows_a = rows_a; a.rows_b = pb ? rows_b : 0; a.x_div = perm ? x_div : 1;
-  a.tiles = nullptr; a.scale = scale; a.act = act; a.ids = nullptr; a.pairs = 0;
+  a.tiles = nullptr; a.scale = scale; a.act = act; a.ids = nullptr; a.pairs = 0; a.leave = 0;
   return LM_OK;
 }
 
@@ -822,7 +822,7 @@ static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part,
       default: launch_stream_tiles<EPI, 5>(a, n, has_b, pl.slices, part, s); break;
     }
   }
-  if (pl.slices > 1) {
+  if (pl.slices > 1 && !a.leave) {
     const int64_t q = (int64_t)a.rows_a * ((EPI == LM_EPI_GLU ? n / 2 : n) / 4);
     hipLaunchKernelGGL((gemm_reduce_kernel<EPI>), dim3((unsigned)((q + 255) / 256)), dim3(256), 0, s, a, part, pl.slices);
   }
@@ -927,6 +927,15 @@ extern "C" int lm_gemm_chosen(const LmGemmPart* pa, const LmGemmPart* pb, int gr
 #else
   return LM_EINVAL;
 #endif
+}
+
+extern "C" int lm_gemm_sums(const LmGemmPart* pa, int rows, float* sums, void* stream) {
+  GemmArgs a;
+  if (fill(a, pa, nullptr, 1, nullptr, nullptr, rows, 0, 1, 1.f, LM_EPI_ELEM, 0) || rows <= 0 || rows > 64 || !sums || ((uintptr_t)a.a.w | (uintptr_t)a.a.x) % 16) return LM_EINVAL;
+  const RowsPlan pl = plan_rows(1, a.a.n, a.a.k, rows, LM_EPI_ELEM, false, true);
+  if (pl.nw == 0 || pl.slices < 2) return LM_EINVAL;
+  a.leave = 1;
+  return launch_stream<LM_EPI_ELEM>(a, 0, pl, sums, (hipStream_t)stream);
 }
 
 extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {

@@ -185,7 +185,7 @@ extern "C" int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy,
   if (slices == 0 || !x || !y || !next_w || !h || !router || !wts || !ids || n <= 0 || n > ldx || ldx % 4 || ldh != k || ldx > k || ldh < n || ldy % 4 ||
       ((uintptr_t)router | (uintptr_t)h) % 16)
     return LM_EINVAL;
-  const ResidualArgs a{x, ldx, nullptr, nullptr, 1.f, (const elem_t*)y, ldy, nullptr, nullptr, 0, 0, 0, post_w, post_b, next_w, next_b, (elem_t*)h, ldh, nullptr, n, kind, 1, eps};
+  const ResidualArgs a{x, ldx, nullptr, nullptr, 1.f, (const elem_t*)y, ldy, nullptr, 0, 0, nullptr, nullptr, 0, 0, 0, post_w, post_b, next_w, next_b, (elem_t*)h, ldh, nullptr, n, kind, 1, eps};
   hipStream_t s = (hipStream_t)stream;
   const elem_t* rt = (const elem_t*)router;
   const int nb = (experts + 15) / 16;

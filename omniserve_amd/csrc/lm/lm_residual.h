@@ -60,6 +60,8 @@ struct ResidualArgs {
   const int* tokens; const elem_t* embed;    // tokens: the residual starts as these rows of the table [vocab][ldx] ...
   float embed_scale;                         // ... times this
   const elem_t* y; int64_t ldy;              // sublayer output (or null): added to the residual
+  const float* sums; int slices;             // ... or the f32 sums of its product's K slices, [slices][sum_rows][ldy]
+  int64_t sum_rows;
   const float* y_bias;                       // added to y (or null)
   const float* pair_w; int top, pairs0, shared;   // top > 0: y holds expert outputs by (token, choice), see moe_sum
   const float *post_w, *post_b;              // norm of the sublayer output before it is added (or null)
@@ -84,7 +86,28 @@ __device__ __forceinline__ void residual_row(const ResidualArgs& p, Row<TH>& row
     if (c >= p.n) continue;
     x[i] = er ? p.embed_scale * from_quad(*(const quad_t*)(er + c)) : *(const f32x4*)(xr + c);
   }
-  if (p.y) {
+  if (p.y || p.sums) {
+    if (p.sums) {         // added up and rounded as gemm_reduce_kernel does
+      constexpr int B = NV == 1 ? 4 : NV == 2 ? 2 : 1;      // slices in flight
+      const float* sr = p.sums + (int64_t)t * p.ldy;
+      const int64_t next = p.sum_rows * p.ldy;
+      for (int k0 = 0; k0 < p.slices; k0 += B) {
+        f32x4 v[B][NV];
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int c = 4 * (TH * i + tid);
+            v[k][i] = c < p.n && k0 + k < p.slices ? *(const f32x4*)(sr + (k0 + k) * next + c) : zero4();
+          }
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+#pragma unroll
+          for (int i = 0; i < NV; ++i) y[i] += v[k][i];
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) y[i] = from_quad(to_quad(y[i]));
+    }
     if (p.top > 0) {      // weighted sum of the chosen experts' rows (+ the shared expert's)
       const int64_t p0 = (int64_t)t * p.top;
       constexpr int B = NV >= 8 ? 1 : NV >= 4 ? 2 : 4;      // rows in flight
@@ -108,7 +131,7 @@ __device__ __forceinline__ void residual_row(const ResidualArgs& p, Row<TH>& row
           for (int i = 0; i < NV; ++i) y[i] += w[b] * from_quad(v[b][i]);
       }
     }
-    if (p.top == 0 || p.shared) {
+    if (!p.sums && (p.top == 0 || p.shared)) {
       const elem_t* yr = p.y + (int64_t)(p.top > 0 ? p.pairs0 + t : t) * p.ldy;
 #pragma unroll
       for (int i = 0; i < NV; ++i) {

@@ -194,17 +194,8 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int64_t* out, const float*
 
 using namespace lm;
 
-extern "C" int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const void* embed, float embed_scale, const void* y,
-                                int64_t ldy, const float* y_bias, const float* pair_w, int top, int pairs0, int shared, const float* post_w, const float* post_b,
-                                const float* next_w, const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n,
-                                int kind, int store_x, float eps, void* stream) {
-  if (n_rows <= 0 || n <= 0 || n > ldx || ldx % 4 || (tokens && !embed) || (next_w && !h) || (h && (ldh % 4 || ldh < n)) || top < 0 ||
-      (top > 0 && (!y || !pair_w)))
-    return LM_EINVAL;
-  ResidualArgs a{x, ldx, tokens, (const elem_t*)embed, embed_scale, (const elem_t*)y, ldy, y_bias, pair_w, top, pairs0, shared, post_w, post_b, next_w,
-                 next_b, (elem_t*)h, ldh, rows, n, kind, store_x, eps};
-  hipStream_t s = (hipStream_t)stream;
-  const int64_t cols = ldx > ldh ? ldx : ldh;
+static int launch_residual(const ResidualArgs& a, int n_rows, hipStream_t s) {
+  const int64_t cols = a.ldx > a.ldh ? a.ldx : a.ldh;
 #define LM_CASE(TH, NV) \
   if (cols <= 4 * TH * NV) { hipLaunchKernelGGL((residual_norm_kernel<TH, NV>), dim3(n_rows), dim3(TH), 0, s, a); return launch_status(); }
   LM_CASE(256, 1)
@@ -214,6 +205,27 @@ extern "C" int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const 
   LM_CASE(256, 2) LM_CASE(256, 4) LM_CASE(256, 8) LM_CASE(256, 16)
 #undef LM_CASE
   return LM_EINVAL;
+}
+
+extern "C" int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const void* embed, float embed_scale, const void* y,
+                                int64_t ldy, const float* y_bias, const float* pair_w, int top, int pairs0, int shared, const float* post_w, const float* post_b,
+                                const float* next_w, const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n,
+                                int kind, int store_x, float eps, void* stream) {
+  if (n_rows <= 0 || n <= 0 || n > ldx || ldx % 4 || (tokens && !embed) || (next_w && !h) || (h && (ldh % 4 || ldh < n)) || top < 0 ||
+      (top > 0 && (!y || !pair_w)))
+    return LM_EINVAL;
+  const ResidualArgs a{x, ldx, tokens, (const elem_t*)embed, embed_scale, (const elem_t*)y, ldy, nullptr, 0, 0, y_bias, pair_w, top, pairs0, shared, post_w, post_b, next_w,
+                 next_b, (elem_t*)h, ldh, rows, n, kind, store_x, eps};
+  return launch_residual(a, n_rows, (hipStream_t)stream);
+}
+
+extern "C" int lm_residual_norm_sums(float* x, int64_t ldx, const float* sums, int64_t ld, int slices, int sum_rows, const float* y_bias, const float* post_w,
+                                     const float* post_b, const float* next_w, const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n, int kind,
+                                     int store_x, float eps, void* stream) {
+  if (n_rows <= 0 || n <= 0 || n > ldx || ldx % 4 || (next_w && !h) || (h && (ldh % 4 || ldh < n)) || !sums || slices <= 0 || ld < n || ld % 4 || sum_rows <= 0) return LM_EINVAL;
+  const ResidualArgs a{x, ldx, nullptr, nullptr, 1.f, nullptr, ld, sums, slices, sum_rows, y_bias, nullptr, 0, 0, 0, post_w, post_b, next_w, next_b, (elem_t*)h, ldh, rows, n, kind,
+                       store_x, eps};
+  return launch_residual(a, n_rows, (hipStream_t)stream);
 }
 
 extern "C" int lm_gated_rms(void* out, int64_t ldo, const void* o, int64_t ldi, const void* gate, int64_t ldg, const float* w,

@@ -538,8 +538,8 @@ class Dense:
         self.b_out = w.vector("down.b", width, W)
 
     def __call__(self, h):
-        """-> (rows without the last bias, arguments of LmOps.residual_norm that add it)"""
-        return self.ops.matmul(self.ops.glu(h, self.w_in, self.b_in, self.s.act), self.w_out), {"y_bias": self.b_out}
+        """-> (rows without the last bias, or LmOps.sums of them; arguments of LmOps.residual_norm that add it)"""
+        return self.ops.sums(self.ops.glu(h, self.w_in, self.b_in, self.s.act), self.w_out), {"y_bias": self.b_out}
 
 
 class MixtureOfExperts:

@@ -1,0 +1,35 @@
+"""A product's K slices added up by the norm behind it: the same bits as the product's own rows and the norm over those."""
+import pytest
+import torch
+
+from omniserve_amd.backend.lm import lm_ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T", [1, 17, 48, 64])
+@pytest.mark.parametrize("n,k,real", [(4096, 14336, 4096), (1024, 8192, 1000), (2048, 6144, 2044), (8192, 16384, 8192), (512, 512, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_same_bits(T, n, k, real, dtype):
+    ops = lm_ops(dtype)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n + k)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")      # noqa: E731
+    w, a, x0 = (k ** -0.5 * rnd(n, k)).to(dtype), rnd(T, k).to(dtype), rnd(T, n)
+    pad = lambda v: torch.nn.functional.pad(v[:real], (0, n - real))      # noqa: E731
+    w[real:] = 0
+    bias, post, nxt = pad(0.1 * rnd(n)), (pad(1 + 0.1 * rnd(n)), pad(0.1 * rnd(n))), (pad(1 + 0.1 * rnd(n)), None)
+    rows = torch.arange(T - 1, -1, -2, dtype=torch.int32, device="cuda")
+    y = ops.matmul(a, w)
+    s = ops.sums(a, w)
+    assert (s.dim() == 3) == (ops._h.lm_gemm_rows_scratch(n, k, T, 0) > 0)
+    for kw in (dict(kind="rms", y_bias=bias, post=post), dict(kind="layer", next=nxt), dict(kind="rms", y_bias=bias, post=post, next=nxt, rows=rows, store_x=False)):
+        kw = dict(kw)
+        kind = kw.pop("kind")
+        out = []
+        for v in (y, s):
+            x, h = x0.clone(), torch.zeros((T if "rows" not in kw else rows.numel(), n), dtype=dtype, device="cuda")
+            ops.residual_norm(x, real, kind, 1e-5, y=v, h=h, **kw)
+            out.append((x, h))
+        torch.cuda.synchronize()
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), kw.keys()
