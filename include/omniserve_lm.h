@@ -139,10 +139,11 @@ int lm_route(const float* z, int64_t ldz, const float* bias, int tokens, int exp
              int* tiles, int* scratch_i32, void* stream);
 
 /* Few tokens: lm_residual_norm (x += norm(y; post); h = norm(x; next), h of ldh = k elements), the router's product of h (router [experts, up to a multiple of 16][k], zero
- * rows behind the last expert) and the choice of lm_route in one launch -> wts [tokens][top], ids [tokens][top] (experts).  lm_norm_choose_ok: for these sizes. */
+ * rows behind the last expert) and the choice of lm_route in one launch -> wts [tokens][top], ids [tokens][top] (experts).  pos (or null): a token whose entry is
+ * negative is none: weights 0, experts -1, x and h as they are.  lm_norm_choose_ok: for these sizes. */
 int lm_norm_choose_ok(int tokens, int k, int experts, int top);
 int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy, const float* post_w, const float* post_b, const float* next_w, const float* next_b,
-                   void* h, int64_t ldh, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top,
+                   void* h, int64_t ldh, const int* pos, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top,
                    float* wts, int* ids, void* stream);
 
 /* y = x w^T for one or many matrices w [groups][n][k].  perm null: rows_a rows, group g reads x from column g * gx and writes y

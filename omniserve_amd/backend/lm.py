@@ -63,7 +63,7 @@ PROTOTYPES = {
     "lm_route_max_tiles": (_i, [_i, _i, _i]),
     "lm_route": (_i, [_vp, _i64, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     "lm_norm_choose_ok": (_i, [_i] * 4),
-    "lm_norm_choose": (_i, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _i, _f, _vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
+    "lm_norm_choose": (_i, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i, _i, _i, _f, _vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "lm_gemm_chosen_ok": (_i, [_i] * 6),
     "lm_gemm_chosen": (_i, [_PP, _PP, _i, _vp, _i, _i, _i, _f, _i, _i, _vp]),
     "lm_gemm_sums": (_i, [_PP, _i, _vp, _vp]),
@@ -273,15 +273,16 @@ class LmOps:
         return bool(self._h.lm_norm_choose_ok(tokens, router.shape[1], experts, top) and ok(*w_in.shape, tokens, top, EPI_GLU)
                     and ok(*w_out.shape, tokens, top, EPI_ELEM))
 
-    def norm_choose(self, x, n, kind, eps, y, post, next, h, router, bias, experts, top):
-        """residual_norm, the router's product of h and route in one launch -> (weights [T, top], the choices for grouped)"""
+    def norm_choose(self, x, n, kind, eps, y, post, next, h, router, bias, experts, top, pos=None):
+        """residual_norm, the router's product of h and route in one launch -> (weights [T, top], the choices for grouped).  pos: places with a
+        negative one are empty (their rows stay as they are and choose nothing)"""
         T = x.shape[0]
         if not (h.is_contiguous() and router.is_contiguous() and h.shape == (T, router.shape[1]) and router.shape[0] == (experts + 15) // 16 * 16):
             raise ValueError("norm_choose: h [tokens, k] and router [experts (a multiple of 16), k], both contiguous")
         wts = torch.empty((T, top), dtype=torch.float32, device=x.device)
         ids = torch.empty((T, top), dtype=torch.int32, device=x.device)
         post = post or (None, None)
-        self._call("lm_norm_choose", _p(x), _ld(x), _p(y), _ld(y), _p(post[0]), _p(post[1]), _p(next[0]), _p(next[1]), _p(h), _ld(h), T, n, NORM[kind], eps,
+        self._call("lm_norm_choose", _p(x), _ld(x), _p(y), _ld(y), _p(post[0]), _p(post[1]), _p(next[0]), _p(next[1]), _p(h), _ld(h), _p(pos), T, n, NORM[kind], eps,
                    _p(router), _p(bias), router.shape[1], experts, top, _p(wts), _p(ids))
         return wts, ids
 

@@ -6,7 +6,8 @@
 // to those who need it: a workgroup of lm_gemm_chosen finds its expert's pairs among the choices.
 //
 // MI355X, bf16, us, norm + router product + choice -> here: 16 tokens, 64 experts, width 2048 4.5 + 4.4 + 6.9 -> 9.8 (in a step of a model 18.6 -> 11.1), 32 tokens 4.5 + 5.2 + 11.5 ->
-// 9.8, one 4.3 + 4.4 + 5.5 -> 9.6; 16 tokens, 32 experts, width 4096 5.5 + 6.6 + 4.9 -> 12.6.
+// 9.8, one 4.3 + 4.4 + 5.5 -> 9.6; 16 tokens, 32 experts, width 4096 5.5 + 6.6 + 4.9 -> 12.6.  A step's empty places choose nothing: 20 steps of
+// a model of 6 such layers, 5 sequences in 8 places, 35.6 ms -> 34.6 by the launch and 33.2 by the experts that are not read.
 //
 // The logits' sums are those of gemm_stream_kernel with 16 channels and four K parts, one product and one addition after the other: a near tie
 // between experts falls as it does there.
@@ -21,7 +22,7 @@ constexpr int KPARTS = 4, STAGE_B = 128, SLICES = 8;      // K parts of a slice;
 
 // NB: blocks of 16 experts.  Stage s belongs to K part s % 4; four stages (one of each part) are a group, a slot of the ring.
 template <int TH, int NB>
-__global__ __launch_bounds__(TH) void norm_choose_kernel(ResidualArgs p, const elem_t* router, const float* bias, int k, int slices, int experts, int top,
+__global__ __launch_bounds__(TH) void norm_choose_kernel(ResidualArgs p, const int* pos, const elem_t* router, const float* bias, int k, int slices, int experts, int top,
                                                          float* wts, int* ids) {
   constexpr int WAVES = TH / 64, STAGE = NB * 16 * STAGE_B, GROUP = KPARTS * STAGE, R = NB <= 2 ? 8 : 4;
   constexpr int PIECES = GROUP / 1024, P = (PIECES + WAVES - 1) / WAVES;      // of a group, and a wave's (some twice: the same bytes)
@@ -32,6 +33,13 @@ __global__ __launch_bounds__(TH) void norm_choose_kernel(ResidualArgs p, const e
   __shared__ int count[WAVES][64];
   elem_t* const hrow = (elem_t*)(lds + R * GROUP);
   const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l15 = lane & 15, l4 = lane >> 4;
+  if (pos && pos[r] < 0) {      // an empty place of a captured step: it chooses no expert, whose weights would be read for it
+    if (tid < top) {
+      ids[(int64_t)r * top + tid] = -1;
+      wts[(int64_t)r * top + tid] = 0.f;
+    }
+    return;
+  }
   const uint32_t base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int groups = k / (KPARTS * STAGE_B / (int)sizeof(elem_t)), own = groups / slices;      // own: of a slice
   // piece i of the wave: eight rows of a stage; lane -> (row lane / 8, slot lane % 8)
@@ -149,11 +157,11 @@ __global__ __launch_bounds__(TH) void norm_choose_kernel(ResidualArgs p, const e
 }
 
 template <int TH, int NB>
-static int launch_choose(const ResidualArgs& a, const elem_t* router, const float* bias, int k, int slices, int experts, int top, float* wts, int* ids, int tokens,
+static int launch_choose(const ResidualArgs& a, const int* pos, const elem_t* router, const float* bias, int k, int slices, int experts, int top, float* wts, int* ids, int tokens,
                          hipStream_t s) {
   const size_t lds = (size_t)(NB <= 2 ? 8 : 4) * KPARTS * NB * 16 * STAGE_B + (size_t)k * sizeof(elem_t);
   if (allow_lds(norm_choose_kernel<TH, NB>, lds)) return LM_EINVAL;
-  hipLaunchKernelGGL((norm_choose_kernel<TH, NB>), dim3(tokens), dim3(TH), lds, s, a, router, bias, k, slices, experts, top, wts, ids);
+  hipLaunchKernelGGL((norm_choose_kernel<TH, NB>), dim3(tokens), dim3(TH), lds, s, a, pos, router, bias, k, slices, experts, top, wts, ids);
   return launch_status();
 }
 #endif
@@ -178,7 +186,7 @@ static int choose_slices(int tokens, int k, int experts, int top) {
 extern "C" int lm_norm_choose_ok(int tokens, int k, int experts, int top) { return choose_slices(tokens, k, experts, top) > 0; }
 
 extern "C" int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy, const float* post_w, const float* post_b, const float* next_w, const float* next_b, void* h,
-                              int64_t ldh, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top, float* wts, int* ids,
+                              int64_t ldh, const int* pos, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top, float* wts, int* ids,
                               void* stream) {
 #if LM_ELEM == 0
   const int slices = choose_slices(tokens, k, experts, top);
@@ -189,7 +197,7 @@ extern "C" int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy,
   hipStream_t s = (hipStream_t)stream;
   const elem_t* rt = (const elem_t*)router;
   const int nb = (experts + 15) / 16;
-#define LM_CASE(TH, NB) if (nb == NB && k <= 4 * TH) return launch_choose<TH, NB>(a, rt, bias, k, slices, experts, top, wts, ids, tokens, s);
+#define LM_CASE(TH, NB) if (nb == NB && k <= 4 * TH) return launch_choose<TH, NB>(a, pos, rt, bias, k, slices, experts, top, wts, ids, tokens, s);
   LM_CASE(512, 1) LM_CASE(512, 2) LM_CASE(512, 3) LM_CASE(512, 4) LM_CASE(1024, 1) LM_CASE(1024, 2) LM_CASE(1024, 3) LM_CASE(1024, 4)
 #undef LM_CASE
 #endif

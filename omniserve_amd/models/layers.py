@@ -674,7 +674,7 @@ class Decoder(EngineModel):
             form, post = {}, L.post
             if L.ff is not None:
                 if L.ff_pre and isinstance(L.ff, MixtureOfExperts) and L.ff.chooses(T):
-                    y, form = L.ff(h, ops.norm_choose(x, spec.width, spec.norm, spec.eps, y, post, L.ff_pre, h, L.ff.router, L.ff.bias, L.ff.s.experts, L.ff.s.top))
+                    y, form = L.ff(h, ops.norm_choose(x, spec.width, spec.norm, spec.eps, y, post, L.ff_pre, h, L.ff.router, L.ff.bias, L.ff.s.experts, L.ff.s.top, b.pos))
                 else:
                     norm(y=y, post=post, next=L.ff_pre, h=h)
                     y, form = L.ff(h)

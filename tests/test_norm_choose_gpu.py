@@ -62,3 +62,21 @@ def test_sizes_that_it_leaves():
     for T, experts, k in ((33, 64, 2048), (16, 65, 2048), (16, 64, 1024), (16, 64, 8192), (16, 64, 2112)):
         assert not ops.chooses(T, shape((experts + 15) // 16 * 16, k), experts, 8, *big)
     assert not lm_ops(torch.float32).chooses(16, shape(64, 2048), 64, 8, *big)
+
+
+def test_empty_places_choose_nothing():
+    ops, T, k, experts, top = lm_ops(torch.bfloat16), 8, 2048, 64, 8
+    m = _inputs(T, k, k, experts, 640, 1024, 3, False)
+    pos = torch.tensor([4, -1, 0, 7, -1, -1, 9, 1], dtype=torch.int32, device=DEV)
+    full, out = pos >= 0, []
+    for p in (None, pos):
+        x, h = m["x"].clone(), torch.zeros((T, k), dtype=torch.bfloat16, device=DEV)
+        wts, ids = ops.norm_choose(x, k, "layer", 1e-5, m["y"], m["post"], m["next"], h, m["router"], m["bias"], experts, top, p)
+        act = torch.full((T * top, 640), -3.0, dtype=torch.bfloat16, device=DEV)
+        ops.grouped(ids, T, h, m["w_in"], act, False, True)
+        out.append((x, h, wts, ids, act.view(T, top, -1)))
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.equal(a[full], b[full])
+    x, h, wts, ids, act = out[1]
+    assert torch.equal(x[~full], m["x"][~full]) and not h[~full].any() and not wts[~full].any() and (ids[~full] == -1).all() and (act[~full] == -3).all()
