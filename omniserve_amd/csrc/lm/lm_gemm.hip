@@ -430,11 +430,15 @@ __device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag
 // MI355X, bf16, before: 256 x 128 tiles of 64-byte stages, a workgroup per tile, two of them on a CU.  7999
 // tokens, 6 of 32 experts of 1792, width 4096: 2407 -> 1883 us up (998 TFLOP/s with the rows of the half empty tiles not counted), 1084 ->
 // 938 down; 6733 tokens, 8 of 64 experts of 640, width 2048: 410 -> 382 up, 256 -> 259 down; 8192 x 7168 x 4096 to f32: 569 -> 469.
+// Ahead of the requests a wave touches 32 lines of the stage behind them (touch_lines32): 64 rows of each operand a workgroup, the others by the workgroups
+// of the band and of the neighbouring columns; where a band's tiles are several experts', their weights' other rows come untouched.  7999 tokens as
+// above: 1687 -> 1644 up, 947 -> 920 down.
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
   constexpr bool DIRECT = EPI == LM_EPI_F32 || sizeof(elem_t) == 4;      // accumulators straight to memory
+  constexpr bool TOUCH = sizeof(elem_t) == 2;                            // (f32's products take too long to wait for memory)
   constexpr int OC = EPI == LM_EPI_GLU ? 64 : 128, PITCH = OC * (int)sizeof(elem_t) + 16, OUT = DIRECT ? 0 : 4 * 16 * PITCH;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE + OUT];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE + OUT + 128];
   __shared__ int y_rows[2][TM];
   typedef Tile<SROWB> T;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -450,6 +454,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   const uint8_t* xsrc[8];
   uint32_t woff[8];                                         // from the tile's first channel
   const uint8_t* wbase = nullptr;
+  const uint8_t* soon = nullptr;                            // the lane's line of the stage behind the one requested last: of the weights (lanes 0 - 15) or of x
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const uint32_t dst0 = __builtin_amdgcn_readfirstlane(lds0 + 64 * SROWB * wave);
   auto dst = [&](int t, int i) { return dst0 + (t & 1) * STAGE + 1024 * (i & 7) + (i < 8 ? 0 : TN * SROWB); };      // of piece i
@@ -498,10 +503,17 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
         const int xr = perm ? perm[first + rc] / x_div : first + rc;
         xsrc[i] = (const uint8_t*)(pt.x + (int64_t)xr * pt.ldx) + ((ps ^ T::swizzle(r)) << 4);
       }
+      {
+        const int r = 64 * ((ol & 16 ? in / bm : mi) & 3) + 16 * wave + (ol & 15), rc = first + min(r, rows - 1);
+        const int xr = perm ? perm[rc] / x_div : rc;
+        soon = (ol & 16 ? (const uint8_t*)(pt.x + (int64_t)xr * pt.ldx) : wbase + (uint32_t)min(r, pt.n - 1 - n0) * (uint32_t)(pt.k * (int)sizeof(elem_t))) +
+               SROWB * min(2, ns - 1);
+      }
       y_row[otid] = otid < rows ? (perm ? perm[first + otid] : first + otid) : -1;
       wait_pieces<0>();                                     // the compiler's own loads
       stage(0);
       if (ns > 1) stage(1);
+      if constexpr (TOUCH) touch_lines32(soon, lds0 + 2 * STAGE + OUT);
       at += (int)gridDim.x >> 3;
       return true;
     }
@@ -541,7 +553,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       four(Int<0>{}, 4, j);
     }
     // stage t + 1 is there for every wave, and everyone has stage t in registers
-    if constexpr (MORE) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if constexpr (DMA && TOUCH) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)" ::: "memory");      // (behind its requests only lines are touched)
+    else if constexpr (MORE) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -567,7 +580,11 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
         four(Int<1>{}, 4, j);
       }
     }
-    if constexpr (DMA) wbase += SROWB;
+    if constexpr (DMA) {
+      wbase += SROWB;
+      soon += SROWB & (t + 3 < ns ? -1 : 0);
+      if constexpr (TOUCH) touch_lines32(soon, lds0 + 2 * STAGE + OUT);
+    }
   };
 
   int parity = 0;
@@ -578,8 +595,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{z, z, z, z};
-    // stage 0 is there: of what was requested last -- stage 1, or stores of the tile before -- 16 may still fly
-    if (ns > 1) wait_pieces<16>();
+    // stage 0 is there: of what was requested last -- stage 1 and lines, or stores of the tile before -- 16 (17) may still fly
+    if (ns > 1) wait_pieces<16 + TOUCH>();
     else wait_pieces<0>();
     __syncthreads();
     const int fl = lane_here();

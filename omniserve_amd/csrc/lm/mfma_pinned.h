@@ -23,6 +23,14 @@
                  : "memory");                                                                                               \
   } while (0)
 
+// The lines at 32 lanes' addresses (the first 32's) into the XCD's L2: a dword of each goes to 128 bytes of LDS that nobody reads, as one piece of vmcnt.
+// For tiles that many compute units of an XCD read at about the same time: their requests come half a stage before they are needed, enough for what the L2
+// holds and not for what it has to fetch; ahead of them each unit touches its share of what they have in common.  Whole waves only.  (No gain where a stage
+// takes longer for its operands to be unpacked: the 4-bit group-wise tiles, 320 us of 28672 x 4096 and 2331 rows without, 322 with.)
+__device__ __forceinline__ void touch_lines32(const void* src, uint32_t lds_sink) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dword %0, off\n\ts_mov_b32 exec_hi, -1" ::"v"(src), "s"(lds_sink) : "memory", "m0");
+}
+
 // a value the optimiser knows nothing about: what is computed from it is computed where it stands, not kept across a loop
 __device__ __forceinline__ int opaque(int v) {
   asm volatile("" : "+v"(v));

@@ -7,12 +7,16 @@
 //
 //  * stages of 128 bytes of k (64 KB), two of them: the fragments of a half stage are read while the half before it multiplies, the stage
 //    after next is requested as soon as every wave has the current one in registers.
+//  * ahead of the requests a wave touches 32 lines of the stage behind them (touch_lines32): 64 rows of each operand a workgroup, the other rows by
+//    those of the 32 workgroups of an XCD that have the same rows or channels (four of a band, and four neighbouring columns).
 //  * a workgroup takes tile after tile of its XCD; the first two stages of the next one are on their way while it stores this one.
 //
 // Integer sums and the general kernel's epilogue: the same bits.
 //
-// MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 656 -> 561 (2510 TOPS); what
-// is left of the 5 POPS nominal: the clock under this load and, at 28672 channels, 690 MB of results.
+// MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 656 -> 561 (2510 TOPS).  With lines touched
+// ahead 1206 -> 1118 and 512 -> 487 (two stages ahead 1134 and 489; every workgroup its whole tile 1168 and 535; the operands of all tiles the first one's, so
+// that the L2 has everything, 983 and 445; no requests at all 934 and 398; no LDS reads 1182 and 498): what is left of the 5 POPS nominal is the clock under this load,
+// 8 us at the ends of a tile, which 4096 of K show, and the L2.
 #pragma once
 #include "lm/mfma_pinned.h"
 
@@ -40,8 +44,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
   static_assert(MODE == MODE_W8, "rows of int8 weights");
   constexpr int PITCH = 128 * 2 + 16;                       // a row of the write-back buffers: a wave's 128 channels
   // one object: the stages, four write-back buffers of 16 rows, the scales of two tiles
-  constexpr int LDS_OUT = 2 * TILES_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SC + 2 * 1024];
+  constexpr int LDS_OUT = 2 * TILES_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH, LDS_SINK = LDS_SC + 2 * 1024;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SINK + 128];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = 128 * (wave & 1), wm = 128 * (wave >> 1);
   // XCD x takes the x-th contiguous eighth of the tiles, counted down the columns of bands of row tiles (as w4a8_gemm_exact_kernel)
@@ -69,6 +73,10 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     abase += TILES_K;
   };
   const int ns = p.K / TILES_K;                             // even
+  uint32_t ahead = 0;                                       // the lane's row that it touches ahead, of the weights (lanes 0 - 15) or the activations
+  const uint32_t sink = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds + LDS_SINK);
+  // the lines of the stage behind the one requested last (left: there is one, else that one's)
+  auto touch = [&](bool left) { touch_lines32((lane_here() & 16 ? abase : wbase) + ahead - (left ? 0 : TILES_K), sink); };
   int m0 = 0, n0 = 0;
   uint16_t sw_next = 0, sa_next = 0;                        // the thread's channel's and row's scales of the tile opened last
   // requests the next tile's first two stages; false: there is none.  The last row tile starts at M - 256: the rows that it shares with the
@@ -80,6 +88,10 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     at += (int)gridDim.x >> 3;
     n0 = tn * TILES_N;
     m0 = min((band * p.tile_linear + in - tn * rows) * TILES_M, p.M - TILES_M);
+    {
+      const int l = lane_here();
+      ahead = (uint32_t)(64 * ((l & 16 ? tn : in) & 3) + 16 * wave + (l & 15)) * (uint32_t)p.K;      // (in % rows: rows is four in all bands but the last)
+    }
     wbase = p.W + (size_t)n0 * p.K;
     abase = (const uint8_t*)p.A + (size_t)m0 * p.K;
     const int tid = 64 * wave + lane_here();
@@ -87,6 +99,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     sa_next = ((const uint16_t*)p.ascales)[m0 + tid];
     stage(0);
     stage(1);
+    touch(2 < ns);
     return true;
   };
   // ... its scales in LDS: 256 channels', 256 rows'
@@ -127,7 +140,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
       four(IntTag<0>{}, 4, j);
     }
     // stage t + 1 is there for every wave, and everyone has stage t in registers
-    if constexpr (MORE) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if constexpr (MORE && DMA) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)" ::: "memory");      // (behind its requests only lines are touched)
+    else if constexpr (MORE) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -153,6 +167,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     if constexpr (DMA) {
       wbase += TILES_K;
       abase += TILES_K;
+      touch(t + 3 < ns);
     }
   };
 
@@ -165,8 +180,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[i][j] = (v4i){z, z, z, z};
-    // stage 0 is there: of what was requested last -- stage 1, or stores of the tile before -- 16 may still fly
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    // stage 0 is there: of what was requested last -- stage 1 and lines, or stores of the tile before -- 17 may still fly
+    asm volatile("s_waitcnt vmcnt(17)" ::: "memory");
     __syncthreads();
     const int fl = lane_here();
 #pragma unroll
