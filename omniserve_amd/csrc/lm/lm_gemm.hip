@@ -436,7 +436,7 @@ __device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
   constexpr bool DIRECT = EPI == LM_EPI_F32 || sizeof(elem_t) == 4;      // accumulators straight to memory
-  constexpr bool TOUCH = sizeof(elem_t) == 2;                            // (f32's products take too long to wait for memory)
+  constexpr bool TOUCH = sizeof(elem_t) == 2;                            // (f32's products take too long for memory and ends of tiles to matter)
   constexpr int OC = EPI == LM_EPI_GLU ? 64 : 128, PITCH = OC * (int)sizeof(elem_t) + 16, OUT = DIRECT ? 0 : 4 * 16 * PITCH;
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE + OUT + 128];
   __shared__ int y_rows[2][TM];
@@ -532,15 +532,18 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
     a[U][i] = *(const frag_t*)(lds + (t & 1) * STAGE + 16 * SROWB * i + off[U] + wn * SROWB);
   };
   f32x4 acc[8][8];
-  // Stage t: MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products: a burst of
+  // Stage t: FRESH: the tile's first (its accumulators were not zeroed: 256 instructions of a lone wave), MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products: a burst of
   // them fills the queues of the address path and the LDS, and the lone wave, which issues in order, waits there with its matrix
   // unit idle.  No condition inside: reads and products have to share a basic block.
-  auto step = [&](int t, auto more, auto dma) {
-    constexpr bool MORE = decltype(more)::value, DMA = decltype(dma)::value;
+  auto step = [&](int t, auto fresh, auto more, auto dma) {
+    constexpr bool FRESH = decltype(fresh)::value, MORE = decltype(more)::value, DMA = decltype(dma)::value;
     auto four = [&](auto half, int i0, int j) {
       constexpr int U = decltype(half)::value;
 #pragma unroll
-      for (int i = i0; i < i0 + 4; ++i) mma_in_place(acc[i][j], a[U][i], b[U][j]);
+      for (int i = i0; i < i0 + 4; ++i) {
+        if constexpr (FRESH && U == 0) OMNI_MFMA_FRESH("v_mfma_f32_16x16x32_bf16", acc[i][j], a[U][i], b[U][j]);
+        else mma_in_place(acc[i][j], a[U][i], b[U][j]);
+      }
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
@@ -590,11 +593,6 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   int parity = 0;
   bool open = open_tile(y_rows[0]);
   while (open) {
-    const float z = __builtin_bit_cast(float, opaque(0));   // (no register of zeros across the tiles)
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{z, z, z, z};
     // stage 0 is there: of what was requested last -- stage 1 and lines, or stores of the tile before -- 16 (17) may still fly
     if (ns > 1) wait_pieces<16 + TOUCH>();
     else wait_pieces<0>();
@@ -608,12 +606,22 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       fetch_a(0, Int<0>{}, i);
     }
     int t = 0;
-    for (; t + 2 < ns; ++t) step(t, Int<1>{}, Int<1>{});
+    if (TOUCH && ns > 2) {
+      step(0, Int<TOUCH>{}, Int<1>{}, Int<1>{});
+      t = 1;
+    } else {
+      const float z = __builtin_bit_cast(float, opaque(0));
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{z, z, z, z};
+    }
+    for (; t + 2 < ns; ++t) step(t, Int<0>{}, Int<1>{}, Int<1>{});
     if (t + 1 < ns) {
-      step(t, Int<1>{}, Int<0>{});
+      step(t, Int<0>{}, Int<1>{}, Int<0>{});
       ++t;
     }
-    step(t, Int<0>{}, Int<0>{});                            // (behind its barrier both stages are free)
+    step(t, Int<0>{}, Int<0>{}, Int<0>{});                  // (behind its barrier both stages are free)
     accumulators_settle(acc);
 
     const Part& pt = is_b ? p.b : p.a;

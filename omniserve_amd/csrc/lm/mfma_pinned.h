@@ -11,6 +11,9 @@
 
 #define OMNI_MFMA_PINNED(OP, c, a, b) asm volatile(OP " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b))
 
+// c = a b
+#define OMNI_MFMA_FRESH(OP, c, a, b) asm volatile(OP " %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b))
+
 // ADDR: "%10" with a scalar base and src a 32-bit offset from it, "off" with src an address (base is then ignored).  M0 is the compiler's:
 // saved and restored.
 #define OMNI_MFMA3_DMA16(OP, ADDR, c0, c1, c2, a0, a1, a2, b, src, base, lds_dst)                                            \

@@ -217,7 +217,7 @@ static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, 
 // w8a8_tiles_kernel: rounds of a tile per CU.  A stage takes 0.95 us where few CUs have a tile and 1.4 where all have one; 8 us a tile for its
 // ends, which is what short K loses here.  (MI355X, this kernel against the best tile height of the other: 12001 rows of 28672 x 4096 1193 us /
 // 1403, of 4096 x 14336 561 / 656, of 16640 x 1024 237 / 252, of 16384 x 256 116 / 111; 2331 rows of 6144 x 4096 51 / 62; 1501 rows of 4096 x
-// 14336, 96 tiles, 128 / 95.)
+// 14336, 96 tiles, 128 / 95.  From 512 of K: the kernel's first stage and its last two are not the same.)
 static float tiles_time(long long tiles, int stages) {
   const long long rounds = tiles / 256;
   const float rest = (float)(tiles - rounds * 256) / 256.f;
@@ -261,7 +261,7 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
     if (K % (2 * KCHUNK) == 0) offer(mb, 2, 1);
     if (sk > 1) offer(mb, 1, sk);
   }
-  if (mode == MODE_W8 && !slab_only && g_override_sk <= 0 && M >= TILES_M && tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < time)
+  if (mode == MODE_W8 && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K && tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < time)
     best = PrefillPlan{16, 1, 1};
   if (mode == MODE_GRP && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K)
     best.group_tiles = g_override_waves == 16 || group_tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < 0.98f * time;

@@ -13,10 +13,11 @@
 //
 // Integer sums and the general kernel's epilogue: the same bits.
 //
+//  * the stores stream: 256 workgroups write 33 MB at the ends of their tiles, as much as all L2s hold, which keep the operands.
 // MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 656 -> 561 (2510 TOPS).  With lines touched
 // ahead 1206 -> 1118 and 512 -> 487 (two stages ahead 1134 and 489; every workgroup its whole tile 1168 and 535; the operands of all tiles the first one's, so
 // that the L2 has everything, 983 and 445; no requests at all 934 and 398; no LDS reads 1182 and 498): what is left of the 5 POPS nominal is the clock under this load,
-// 8 us at the ends of a tile, which 4096 of K show, and the L2.
+// the ends of a tile, which 4096 of K show, and the L2.  Streaming stores 1038 -> 1013 and 470 -> 461, no zeroing of accumulators 1013 -> 996 and 460 -> 459.
 #pragma once
 #include "lm/mfma_pinned.h"
 
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     wbase += TILES_K;
     abase += TILES_K;
   };
-  const int ns = p.K / TILES_K;                             // even
+  const int ns = p.K / TILES_K;                             // even, four or more
   uint32_t ahead = 0;                                       // the lane's row that it touches ahead, of the weights (lanes 0 - 15) or the activations
   const uint32_t sink = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)lds + LDS_SINK);
   // the lines of the stage behind the one requested last (left: there is one, else that one's)
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     sa_next = ((const uint16_t*)p.ascales)[m0 + tid];
     stage(0);
     stage(1);
-    touch(2 < ns);
+    touch(true);
     return true;
   };
   // ... its scales in LDS: 256 channels', 256 rows'
@@ -120,14 +121,17 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     b[U][i] = *(const v4i*)(lds + (t & 1) * TILES_STAGE + 16 * TILES_K * i + off[U] + (TILES_N + wm) * TILES_K);
   };
 #define OMNI_TILES_OP "v_mfma_i32_16x16x64_i8"
-  // Stage t: MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products (a burst of them
+  // Stage t: FRESH: the tile's first (no accumulators are zeroed: 256 instructions of a lone wave), MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products (a burst of them
   // fills the queues, where the lone wave, which issues in order, waits).  No condition inside: one basic block.
-  auto step = [&](int t, auto more, auto dma) {
-    constexpr bool MORE = decltype(more)::value, DMA = decltype(dma)::value;
+  auto step = [&](int t, auto fresh, auto more, auto dma) {
+    constexpr bool FRESH = decltype(fresh)::value, MORE = decltype(more)::value, DMA = decltype(dma)::value;
     auto four = [&](auto half, int i0, int j) {
       constexpr int U = decltype(half)::value;
 #pragma unroll
-      for (int i = i0; i < i0 + 4; ++i) OMNI_MFMA_PINNED(OMNI_TILES_OP, acc[i][j], a[U][i], b[U][j]);
+      for (int i = i0; i < i0 + 4; ++i) {
+        if constexpr (FRESH && U == 0) OMNI_MFMA_FRESH(OMNI_TILES_OP, acc[i][j], a[U][i], b[U][j]);
+        else OMNI_MFMA_PINNED(OMNI_TILES_OP, acc[i][j], a[U][i], b[U][j]);
+      }
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
@@ -175,11 +179,6 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
   bool open = open_tile();
   if (open) park(0);
   while (open) {
-    const int z = opaque(0);                                // (no register of zeros across the tiles)
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = (v4i){z, z, z, z};
     // stage 0 is there: of what was requested last -- stage 1 and lines, or stores of the tile before -- 17 may still fly
     asm volatile("s_waitcnt vmcnt(17)" ::: "memory");
     __syncthreads();
@@ -191,13 +190,14 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
       fetch_b(0, IntTag<0>{}, i);
       fetch_a(0, IntTag<0>{}, i);
     }
-    int t = 0;
-    for (; t + 2 < ns; ++t) step(t, BoolTag<true>{}, BoolTag<true>{});
+    int t = 1;
+    step(0, BoolTag<true>{}, BoolTag<true>{}, BoolTag<true>{});
+    for (; t + 2 < ns; ++t) step(t, BoolTag<false>{}, BoolTag<true>{}, BoolTag<true>{});
     if (t + 1 < ns) {                                       // (always: it keeps the two steps in blocks of their own)
-      step(t, BoolTag<true>{}, BoolTag<false>{});
+      step(t, BoolTag<false>{}, BoolTag<true>{}, BoolTag<false>{});
       ++t;
     }
-    step(t, BoolTag<false>{}, BoolTag<false>{});            // (behind its barrier both stages are free)
+    step(t, BoolTag<false>{}, BoolTag<false>{}, BoolTag<false>{});      // (behind its barrier both stages are free)
     accumulators_settle(acc);
 
     // the results, packed; then the next tile; then the stores.  The arithmetic of the general kernel: both scales' product, the sum times
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * i + e4;
-        *(uint4*)(out + (size_t)(16 * j + r) * p.out_stride + e15 * 8) = *(const uint4*)(buf + r * PITCH + e15 * 16);
+        __builtin_nontemporal_store(*(const v4i*)(buf + r * PITCH + e15 * 16), (v4i*)(out + (size_t)(16 * j + r) * p.out_stride + e15 * 8));
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
