@@ -278,6 +278,16 @@ int omni_w4a8_per_chn_gemm_silu(const void* in_feats, const void* qweight, const
 int omni_w4a8_per_group_gemm_silu(const void* in_feats, const void* qweight, const void* zeros, const void* scales_i8,
                                   const void* wscales, const void* ascales, void* act_f16, void* amax_slots_u32, int M,
                                   int N, int K, void* stream);
+/* The same for prompts (more than 128 rows): act_f16 [M, N/2] alone, bit for bit what the product and silu_and_mul leave, in the tiles that the product of these sizes
+ * runs in.  omni_gemm_silu_rows_ok (mode 0: per-channel, 1: per-group, 2: W8A8): 1 where they have the unit -- one pass over K by a whole workgroup, N and K multiples
+ * of 256, rows and weights 16-byte aligned (second-level parameters of the 256 x 256 tiles 4); OMNI_EINVAL elsewhere. */
+int omni_gemm_silu_rows_ok(int M, int N, int K, int mode);
+int omni_w4a8_per_chn_gemm_silu_rows(const void* in_feats, const void* qweight, const void* wscales, const void* ascales, const void* w_szs,
+                                     const void* a_ssums, void* act_f16, int M, int N, int K, void* stream);
+int omni_w4a8_per_group_gemm_silu_rows(const void* in_feats, const void* qweight, const void* zeros, const void* scales_i8, const void* wscales,
+                                       const void* ascales, void* act_f16, int M, int N, int K, void* stream);
+int omni_w8a8_gemm_silu_rows(const void* in_feats, const void* weight, const void* wscales, const void* ascales, void* act_f16, int M, int N, int K,
+                             void* stream);
 int omni_w4a8_per_chn_gemm_partial_f16(const void* act_f16, const void* amax_slots_u32, const void* qweight,
                                        void* slab_i32, size_t slab_bytes, void* sum_f16, void* scale_f16, int M, int N,
                                        int K, int* sk_out, void* stream);

@@ -57,6 +57,10 @@ PROTOTYPES = {
     "omni_w4a8_per_chn_gemm_partial": (_i, [_vp, _vp, _vp, _sz, _i, _i, _i, _c.POINTER(_i), _vp]),
     "omni_w4a8_per_chn_gemm_silu": (_i, [_vp] * 8 + [_i, _i, _i, _vp]),
     "omni_w4a8_per_group_gemm_silu": (_i, [_vp] * 8 + [_i, _i, _i, _vp]),
+    "omni_gemm_silu_rows_ok": (_i, [_i, _i, _i, _i]),
+    "omni_w4a8_per_chn_gemm_silu_rows": (_i, [_vp] * 7 + [_i, _i, _i, _vp]),
+    "omni_w4a8_per_group_gemm_silu_rows": (_i, [_vp] * 7 + [_i, _i, _i, _vp]),
+    "omni_w8a8_gemm_silu_rows": (_i, [_vp] * 5 + [_i, _i, _i, _vp]),
     "omni_w4a8_per_chn_gemm_partial_f16": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _i, _i, _i, _c.POINTER(_i), _vp]),
     "omni_w4a8_per_group_gemm_partial_f16": (_i, [_vp] * 6 + [_sz, _vp, _vp, _i, _i, _i, _c.POINTER(_i), _vp]),
     "omni_kv4_decode_attention_f16_amax": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp,

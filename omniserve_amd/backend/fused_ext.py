@@ -224,6 +224,32 @@ def gemm_silu_per_group(in_feats, qweight, s2_zeros, s2_scales, wscales, ascales
     _lib.check(rc, "fused_ext.gemm_silu_per_group")
 
 
+def gate_up_rows(out, in_feats, weight, operands, gate_up, input_sum, scale):
+    """gate_up projection, silu_and_mul and invoke_quant[_fuse_sum] (input_sum=None: without the sum) of many rows -> int8 out [M, N/2] and its scale, bit for bit
+    those calls'.  Where the product's tiles have the unit it leaves fp16 [M, N/2] in `gate_up` (room for [M, N], contiguous) instead of both halves.
+    operands: per-channel (wscales, ascales, w_szs, a_ssums), per-group (s2_zeros, s2_scales, wscales, ascales), W8A8 (wscales, ascales)."""
+    from . import fused_kernels, qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
+    _lib.require_cuda(out, in_feats, weight, gate_up, scale, *operands)
+    (M, K), N, h = in_feats.shape, weight.shape[0], _lib.lib()
+    w8 = len(operands) == 2
+    group = not w8 and operands[0].dim() == 2 and operands[0].dtype == torch.int8
+    name, product = (("omni_w8a8_gemm_silu_rows", qgemm_w8a8.w8a8_gemm_forward_cuda) if w8 else
+                     ("omni_w4a8_per_group_gemm_silu_rows", qgemm_w4a8_per_group.gemm_forward_cuda) if group else
+                     ("omni_w4a8_per_chn_gemm_silu_rows", qgemm_w4a8_per_chn.gemm_forward_cuda))
+    if (h.omni_gemm_silu_rows_ok(M, N, K, 2 if w8 else int(group)) and gate_up.is_contiguous() and in_feats.is_contiguous() and
+            (gate_up.data_ptr() | in_feats.data_ptr() | weight.data_ptr()) % 16 == 0 and not (group and (operands[0].data_ptr() | operands[1].data_ptr()) % 4)):
+        act = gate_up.view(-1)[:M * (N // 2)].view(M, N // 2)
+        _lib.check(getattr(h, name)(in_feats.data_ptr(), weight.data_ptr(), *(t.data_ptr() for t in operands), act.data_ptr(), M, N, K, _lib.current_stream()),
+                   "fused_ext.gate_up_rows")
+        if input_sum is None:
+            fused_kernels.invoke_quant(out, act, scale)
+        else:
+            fused_kernels.invoke_quant_fuse_sum(out, act, input_sum, scale)
+        return
+    product(in_feats, weight, *operands, gate_up)
+    silu_mul_quant_fuse_sum(out, gate_up, input_sum, scale)
+
+
 def gemm_partial_f16_per_chn(act, amax, qweight, slab, sum_out, scale_out):
     """o / down projection straight from fp16 activations: the int8 codes invoke_quant_fuse_sum(act) would produce are
     computed inside the GEMV from `amax` (row maxima left by the producer of `act`); writes int32 split-K slabs (returns

@@ -105,6 +105,25 @@ __device__ __forceinline__ half_t silu_mul_h(half_t a, half_t b) {
   return (half_t)((float)s * (float)b);
 }
 
+// four channels of one row: g, u packed -> silu(g) u
+__device__ __forceinline__ uint2 silu_mul_h4(uint2 g, uint2 u) {
+  uint32_t r[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t gv = h ? g.y : g.x, uv = h ? u.y : u.x;
+    const half_t lo = silu_mul_h(__builtin_bit_cast(half_t, (uint16_t)gv), __builtin_bit_cast(half_t, (uint16_t)uv));
+    const half_t hi = silu_mul_h(__builtin_bit_cast(half_t, (uint16_t)(gv >> 16)), __builtin_bit_cast(half_t, (uint16_t)(uv >> 16)));
+    r[h] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | (uint32_t)__builtin_bit_cast(uint16_t, hi) << 16;
+  }
+  return make_uint2(r[0], r[1]);
+}
+// Gate channels in lanes 0 - 31 and the up channels of the same place in lanes 32 - 63, of two row blocks -> silu(gate) up of the first block in lanes 0 - 31, of
+// the second in the others (no lane idles).
+__device__ __forceinline__ uint2 silu_mul_blocks(uint2 first, uint2 second) {
+  const auto x = __builtin_amdgcn_permlane32_swap(first.x, second.x, false, false), y = __builtin_amdgcn_permlane32_swap(first.y, second.y, false, false);
+  return silu_mul_h4(make_uint2((uint32_t)x[0], (uint32_t)y[0]), make_uint2((uint32_t)x[1], (uint32_t)y[1]));
+}
+
 // four fp16 values (two packed dwords) -> the four int8 codes rni_sat_s8(f32(x) * q), packed little-endian, for a row
 // whose multiplier is q = 127 / max|x| (quant_multiplier below).  2.25 VALU per element instead of 5.75 for the
 // literal rint / NaN test / clamp / convert / pack sequence:

@@ -1251,39 +1251,41 @@ static inline bool exact_shape(const GemmArgs& a, bool to_slab) {
   return exact_sizes(a.M, a.N, a.K, a.kslice) && out16 && in16;
 }
 
-template <int MODE, int MB, int KW, bool TO_SLAB>
+template <int MODE, int MB, int KW, bool TO_SLAB, bool SILU = false>
 static void launch_exact_tile(GemmArgs b, int sk, hipStream_t st) {
   b.tiles_n = b.N / 256;
   b.tiles_m = (b.M + MB * 16 - 1) / (MB * 16);
   const int bands = (b.tiles_m + 7) / 8;
   b.tile_linear = (b.tiles_m + bands - 1) / bands;
   const int tiles = b.tiles_m * b.tiles_n;
-  hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, MB, KW, TO_SLAB>), dim3((tiles + 7) / 8 * 8, sk, 1), dim3(256 * KW), 0, st, b);
+  hipLaunchKernelGGL((w4a8_gemm_exact_kernel<MODE, MB, KW, TO_SLAB, SILU>), dim3((tiles + 7) / 8 * 8, sk, 1), dim3(256 * KW), 0, st, b);
 }
 
-template <int MODE, int KW, bool TO_SLAB>
+template <int MODE, int KW, bool TO_SLAB, bool SILU = false>
 static void launch_exact_rows(const GemmArgs& a, int mb, int sk, hipStream_t st) {
   switch (mb) {
-    case 4: launch_exact_tile<MODE, 4, KW, TO_SLAB>(a, sk, st); break;
-    case 5: launch_exact_tile<MODE, 5, KW, TO_SLAB>(a, sk, st); break;
-    case 6: launch_exact_tile<MODE, 6, KW, TO_SLAB>(a, sk, st); break;
-    case 7: launch_exact_tile<MODE, 7, KW, TO_SLAB>(a, sk, st); break;
-    default: launch_exact_tile<MODE, 8, KW, TO_SLAB>(a, sk, st); break;
+    case 4: launch_exact_tile<MODE, 4, KW, TO_SLAB, SILU>(a, sk, st); break;
+    case 5: launch_exact_tile<MODE, 5, KW, TO_SLAB, SILU>(a, sk, st); break;
+    case 6: launch_exact_tile<MODE, 6, KW, TO_SLAB, SILU>(a, sk, st); break;
+    case 7: launch_exact_tile<MODE, 7, KW, TO_SLAB, SILU>(a, sk, st); break;
+    default: launch_exact_tile<MODE, 8, KW, TO_SLAB, SILU>(a, sk, st); break;
   }
 }
 
 // a workgroup per CU
-template <int MODE>
+template <int MODE, bool SILU = false>
 static void launch_tiles(GemmArgs b, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;
   b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
   const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
   b.tile_linear = (b.tiles_m + bands - 1) / bands;
-  hipLaunchKernelGGL((w8a8_tiles_kernel<MODE>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+  hipLaunchKernelGGL((w8a8_tiles_kernel<MODE, SILU>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
 }
 
 // qgemm_grp.hip
-void launch_group_tiles(const GemmArgs& a, hipStream_t st);
+void launch_group_tiles(const GemmArgs& a, bool silu, hipStream_t st);
+// qgemm_plan.hip: does omni_*_gemm_silu_rows take these sizes?  pp: its plan
+bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp);
 
 // prefill regime (M > 128): chunked LDS staging, weights through L2
 template <int MODE>
@@ -1299,7 +1301,7 @@ static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
     if constexpr (MODE == MODE_GRP) {
       // (a lane's parameters are four bytes)
       if (pp.group_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
-        launch_group_tiles(a, st);
+        launch_group_tiles(a, false, st);
         return;
       }
     }
@@ -1488,6 +1490,27 @@ static int launch_gemm_silu(GemmArgs a, hipStream_t st) {
     if (!plain) return launch_gemv_silu_nt<MODE, true>(a, pl, st);
   }
   return launch_gemv_silu_nt<MODE, false>(a, pl, st);
+}
+
+// The same for prompts: out = silu(gate) up fp16 [M, N/2], bit for bit what the product and silu_and_mul leave, in the products' own tiles.
+template <int MODE>
+static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
+  GemmPlan pl;
+  PrefillPlan pp;
+  if (!silu_rows_plan(a.M, a.N, a.K, MODE, &pl, &pp)) return OMNI_EINVAL;
+  a.kslice = pl.kslice;
+  if (!exact_shape(a, false)) return OMNI_EINVAL;
+  if constexpr (MODE == MODE_W8) {
+    launch_tiles<MODE, true>(a, st);
+  } else {
+    bool tiles = pp.group_tiles;
+    if (tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) != 0) return OMNI_EINVAL;
+    if constexpr (MODE == MODE_GRP) {
+      if (tiles) launch_group_tiles(a, true, st);
+    }
+    if (!tiles) launch_exact_rows<MODE, 1, false, true>(a, pp.mb, 1, st);
+  }
+  return omni_launch_status();
 }
 
 template <int MODE, bool NT>

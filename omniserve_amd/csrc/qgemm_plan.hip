@@ -268,7 +268,23 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
   return best;
 }
 
+// One pass over K by the kernels that have the unit: the tiles, and w4a8_gemm_exact_kernel of one K part.
+bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp) {
+  if (M <= 128 || N < 256 || K < 64 || mode < MODE_CHN || mode > MODE_W8) return false;
+  if (N % 256 != 0 || K % KCHUNK != 0) return false;
+  *pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
+  if (pl->midm || !exact_sizes(M, N, K, pl->kslice)) return false;
+  *pp = plan_prefill(M, N, K, mode, pl->sk, false);
+  return mode == MODE_W8 ? pp->mb == 16 : pp->group_tiles || (pp->sk == 1 && pp->kw == 1);
+}
+
 }  // namespace omni
+
+extern "C" int omni_gemm_silu_rows_ok(int M, int N, int K, int mode) {
+  omni::GemmPlan pl;
+  omni::PrefillPlan pp;
+  return omni::silu_rows_plan(M, N, K, mode, &pl, &pp) ? 1 : 0;
+}
 
 extern "C" void omni_gemm_set_plan_override(int waves, int sk) {
   omni::g_override_waves = waves;

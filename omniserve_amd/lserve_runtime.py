@@ -448,10 +448,11 @@ class LServeDecodeRunner:
                 layernorm_ops.rms_norm_general(q_hidden, x, L["ln2"], scale, c.eps, True)
             for s0 in range(0, T, ch):
                 n = min(ch, T - s0)
-                L["gate_up"].forward(q_hidden[s0:s0 + n], scale[s0:s0 + n], gate_up[:n])
-                if self.fused:             # SiLU*mul + quant without the fp16 round trip (bit-identical)
-                    fused_ext.silu_mul_quant_fuse_sum(q_inter[:n], gate_up[:n], sums, scale[:n])
+                G = L["gate_up"]
+                if self.fused:             # SiLU*mul in the product where it can be, without the fp16 round trip to the quantiser elsewhere (bit-identical)
+                    fused_ext.gate_up_rows(q_inter[:n], q_hidden[s0:s0 + n], G.weight, (G.dequant_scale, scale[s0:s0 + n]), gate_up[:n], sums, scale[:n])
                 else:
+                    G.forward(q_hidden[s0:s0 + n], scale[s0:s0 + n], gate_up[:n])
                     activation_ops.silu_and_mul(mlp_act[:n], gate_up[:n])
                     fused_kernels.invoke_quant(q_inter[:n], mlp_act[:n], scale[:n])
                 L["down"].forward(q_inter[:n], scale[:n], proj[s0:s0 + n])

@@ -77,8 +77,7 @@ class QServeLlama(EngineModel):
                 fused_kernels.invoke_quant(qa, o, sa)
             L["o"].forward(qa, sa, ma, proj)
             fused_ext.add_rms_norm_general_fuse_sum(qh, x, proj, L["ln2"], mn, sn, c.eps)
-            L["gate_up"].forward(qh, sn, mn, gu)
-            fused_ext.silu_mul_quant_fuse_sum(qi, gu, ma, sa)
+            fused_ext.gate_up_rows(qi, qh, L["gate_up"].qweight, L["gate_up"].operands(sn, mn), gu, ma, sa)
             L["down"].forward(qi, sa, ma, proj)
         return x.add_(proj)
 

@@ -74,6 +74,10 @@ class W4A8Linear:
             self.s2_scales = s2.to(torch.int8)
             self.s2_zeros = (-(z * s2)).to(torch.int8)
 
+    def operands(self, scales, sums):
+        """what its product takes beside the codes and packed weights"""
+        return (self.s1_scales, scales, self.s1_szeros, sums) if self.group == -1 else (self.s2_zeros, self.s2_scales, self.s1_scales, scales)
+
     def forward(self, x_i8, scales, sums, out):
         if self.group == -1:
             qgemm_w4a8_per_chn.gemm_forward_cuda(x_i8, self.qweight, self.s1_scales, scales, self.s1_szeros, sums, out)
@@ -682,8 +686,7 @@ class DecodeRunner:
             Ly["o"].forward(qa, sA, mA, proj)
             self._all_reduce(proj)
             fused_ext.add_rms_norm_general_fuse_sum(qh, x, proj, Ly["ln2"], mB, sB, c.eps)
-            Ly["gate_up"].forward(qh, sB, mB, gu)
-            fused_ext.silu_mul_quant_fuse_sum(qi, gu, mA, sA)
+            fused_ext.gate_up_rows(qi, qh, Ly["gate_up"].qweight, Ly["gate_up"].operands(sB, mB), gu, mA, sA)
             Ly["down"].forward(qi, sA, mA, proj)
             self._all_reduce(proj)
         x.add_(proj)
