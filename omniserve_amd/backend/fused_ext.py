@@ -237,6 +237,7 @@ def gate_up_rows(out, in_feats, weight, operands, gate_up, input_sum, scale):
                      ("omni_w4a8_per_group_gemm_silu_rows", qgemm_w4a8_per_group.gemm_forward_cuda) if group else
                      ("omni_w4a8_per_chn_gemm_silu_rows", qgemm_w4a8_per_chn.gemm_forward_cuda))
     if (h.omni_gemm_silu_rows_ok(M, N, K, 2 if w8 else int(group)) and gate_up.is_contiguous() and in_feats.is_contiguous() and
+            (N <= 32768 or M >= 1024) and      # (few rows wider than that: only the unit's quantiser has a kernel of whole rows)
             (gate_up.data_ptr() | in_feats.data_ptr() | weight.data_ptr()) % 16 == 0 and not (group and (operands[0].data_ptr() | operands[1].data_ptr()) % 4)):
         act = gate_up.view(-1)[:M * (N // 2)].view(M, N // 2)
         _lib.check(getattr(h, name)(in_feats.data_ptr(), weight.data_ptr(), *(t.data_ptr() for t in operands), act.data_ptr(), M, N, K, _lib.current_stream()),

@@ -25,17 +25,6 @@ extern "C" int omni_w4a8_per_chn_gemm_partial(const void* in_feats, const void* 
   return launch_gemm_partial<MODE_CHN>(a, slab_i32, slab_bytes, sk_out, (hipStream_t)stream);
 }
 
-extern "C" int omni_w4a8_per_chn_gemm_silu_rows(const void* in_feats, const void* qweight, const void* wscales, const void* ascales, const void* w_szs,
-                                                const void* a_ssums, void* act_f16, int M, int N, int K, void* stream) {
-  if (!in_feats || !qweight || !wscales || !ascales || !w_szs || !a_ssums || !act_f16) return OMNI_EINVAL;
-  GemmArgs a{};
-  a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)qweight;
-  a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
-  a.wsz = (const half_t*)w_szs; a.asum = (const half_t*)a_ssums;
-  a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_CHN>(a, (hipStream_t)stream);
-}
-
 // Fused extension: gate_up projection + silu_and_mul in one kernel (act fp16 [M, N/2]) + row maxima of |act|.
 extern "C" int omni_w4a8_per_chn_gemm_silu(const void* in_feats, const void* qweight, const void* wscales,
                                            const void* ascales, const void* w_szs, const void* a_ssums, void* act_f16,

@@ -398,4 +398,14 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
 #undef OMNI_GT_FENCE
 }
 
+// a workgroup per CU
+template <bool SILU>
+static void launch_group_tiles_as(GemmArgs b, hipStream_t st) {
+  b.tiles_n = b.N / TILES_N;
+  b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
+  const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
+  b.tile_linear = (b.tiles_m + bands - 1) / bands;
+  hipLaunchKernelGGL(w4a8_group_tiles_kernel<SILU>, dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+}
+
 }  // namespace omni

@@ -3,16 +3,7 @@
 #include "qgemm_group_tiles.h"
 using namespace omni;
 
-void omni::launch_group_tiles(const GemmArgs& a, bool silu, hipStream_t st) {      // a workgroup per CU
-  GemmArgs b = a;
-  b.tiles_n = b.N / TILES_N;
-  b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
-  const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
-  b.tile_linear = (b.tiles_m + bands - 1) / bands;
-  const dim3 grid(std::min(256, (tiles + 7) / 8 * 8));
-  if (silu) hipLaunchKernelGGL(w4a8_group_tiles_kernel<true>, grid, dim3(256), 0, st, b);
-  else hipLaunchKernelGGL(w4a8_group_tiles_kernel<false>, grid, dim3(256), 0, st, b);
-}
+void omni::launch_group_tiles(const GemmArgs& a, hipStream_t st) { launch_group_tiles_as<false>(a, st); }
 
 extern "C" int omni_w4a8_per_group_gemm(const void* in_feats, const void* qweight, const void* zeros,
                                         const void* scales_i8, const void* wscales, const void* ascales,
@@ -52,17 +43,6 @@ extern "C" int omni_w4a8_per_group_gemm_silu(const void* in_feats, const void* q
   a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
   a.amax = (uint32_t*)amax_slots_u32;
   return launch_gemm_silu<MODE_GRP>(a, (hipStream_t)stream);
-}
-
-extern "C" int omni_w4a8_per_group_gemm_silu_rows(const void* in_feats, const void* qweight, const void* zeros, const void* scales_i8, const void* wscales,
-                                                  const void* ascales, void* act_f16, int M, int N, int K, void* stream) {
-  if (!in_feats || !qweight || !zeros || !scales_i8 || !wscales || !ascales || !act_f16) return OMNI_EINVAL;
-  GemmArgs a{};
-  a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)qweight;
-  a.s2s = (const uint8_t*)scales_i8; a.s2z = (const uint8_t*)zeros;
-  a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
-  a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_GRP>(a, (hipStream_t)stream);
 }
 
 extern "C" int omni_w4a8_per_group_gemm_partial_f16(const void* act_f16, const void* amax_slots_u32, const void* qweight,

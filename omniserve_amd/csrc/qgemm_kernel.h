@@ -1283,7 +1283,7 @@ static void launch_tiles(GemmArgs b, hipStream_t st) {
 }
 
 // qgemm_grp.hip
-void launch_group_tiles(const GemmArgs& a, bool silu, hipStream_t st);
+void launch_group_tiles(const GemmArgs& a, hipStream_t st);
 // qgemm_plan.hip: does omni_*_gemm_silu_rows take these sizes?  pp: its plan
 bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp);
 
@@ -1301,7 +1301,7 @@ static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st
     if constexpr (MODE == MODE_GRP) {
       // (a lane's parameters are four bytes)
       if (pp.group_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
-        launch_group_tiles(a, false, st);
+        launch_group_tiles(a, st);
         return;
       }
     }
@@ -1490,27 +1490,6 @@ static int launch_gemm_silu(GemmArgs a, hipStream_t st) {
     if (!plain) return launch_gemv_silu_nt<MODE, true>(a, pl, st);
   }
   return launch_gemv_silu_nt<MODE, false>(a, pl, st);
-}
-
-// The same for prompts: out = silu(gate) up fp16 [M, N/2], bit for bit what the product and silu_and_mul leave, in the products' own tiles.
-template <int MODE>
-static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
-  GemmPlan pl;
-  PrefillPlan pp;
-  if (!silu_rows_plan(a.M, a.N, a.K, MODE, &pl, &pp)) return OMNI_EINVAL;
-  a.kslice = pl.kslice;
-  if (!exact_shape(a, false)) return OMNI_EINVAL;
-  if constexpr (MODE == MODE_W8) {
-    launch_tiles<MODE, true>(a, st);
-  } else {
-    bool tiles = pp.group_tiles;
-    if (tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) != 0) return OMNI_EINVAL;
-    if constexpr (MODE == MODE_GRP) {
-      if (tiles) launch_group_tiles(a, true, st);
-    }
-    if (!tiles) launch_exact_rows<MODE, 1, false, true>(a, pp.mb, 1, st);
-  }
-  return omni_launch_status();
 }
 
 template <int MODE, bool NT>

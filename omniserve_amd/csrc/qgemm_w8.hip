@@ -37,16 +37,6 @@ extern "C" int omni_w8a8_gemm_silu(const void* in_feats, const void* weight, con
   return launch_gemm_silu<MODE_W8>(a, (hipStream_t)stream);
 }
 
-extern "C" int omni_w8a8_gemm_silu_rows(const void* in_feats, const void* weight, const void* wscales, const void* ascales, void* act_f16, int M, int N, int K,
-                                        void* stream) {
-  if (!in_feats || !weight || !wscales || !ascales || !act_f16) return OMNI_EINVAL;
-  GemmArgs a{};
-  a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)weight;
-  a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
-  a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_W8>(a, (hipStream_t)stream);
-}
-
 // Fused extension: split-K partial sums of a W8A8 projection whose int8 input is quantised on the fly from fp16
 // activations (invoke_quant's arithmetic) with the row maxima its producer left; rider workgroups write the scales.
 extern "C" int omni_w8a8_gemm_partial_f16(const void* act_f16, const void* amax_slots_u32, const void* weight,
