@@ -345,8 +345,8 @@ struct SrcSilu {  // h(h(silu(gate)) * up) of a [2d] row
 // latency chain: spread it over 8 waves), <128, 4> / <256, 8> when there are many rows (prefill: 4x / 2x more rows
 // resident per CU, the kernel becomes bandwidth-bound instead of chain-bound).  hidden <= RT * RV * 8.
 
-// quant[_fuse_sum] (NV = min(hidden,1024)) with a pluggable source
-template <int RT, int RV, bool FUSE_SUM, typename Src>
+// quant[_fuse_sum] (NV = min(hidden,1024)) with a pluggable source.  HALF: the row's LDS copy is fp16, of a source whose values that holds.
+template <int RT, int RV, bool FUSE_SUM, typename Src, bool HALF = false>
 __global__ __launch_bounds__(RT) void quant_v2_kernel(int8_t* __restrict__ out, Src src0,
                                                        half_t* __restrict__ sum_out, half_t* __restrict__ scale_out,
                                                        int hidden, int nv, PrefetchArgs pf) {
@@ -391,7 +391,12 @@ __global__ __launch_bounds__(RT) void quant_v2_kernel(int8_t* __restrict__ out, 
       x[it][e] = ok ? x[it][e] : 0.0f;
       amax = __builtin_fmaxf(amax, __builtin_fabsf(x[it][e]));
     }
-    if (FUSE_SUM && ok) {
+    if constexpr (HALF) {
+      v8h h;
+#pragma unroll
+      for (int e = 0; e < VT; ++e) h[e] = (half_t)x[it][e];
+      if (ok) *reinterpret_cast<v8h*>(reinterpret_cast<half_t*>(xs) + i) = h;
+    } else if (FUSE_SUM && ok) {
       *reinterpret_cast<v4f*>(xs + i) = (v4f){x[it][0], x[it][1], x[it][2], x[it][3]};
       *reinterpret_cast<v4f*>(xs + i + 4) = (v4f){x[it][4], x[it][5], x[it][6], x[it][7]};
     }
@@ -411,7 +416,8 @@ __global__ __launch_bounds__(RT) void quant_v2_kernel(int8_t* __restrict__ out, 
   OMNI_CLK(12);
   if constexpr (FUSE_SUM) {
     float s[1][VT], tot[1];
-    ordered_partials<1>(xs, p, nv, hidden, s, [](float (&v)[1][VT], int e, float val) { v[0][e] = v[0][e] + val; });
+    if constexpr (HALF) ordered_sums(reinterpret_cast<const half_t*>(xs), p, nv, hidden, s);
+    else ordered_partials<1>(xs, p, nv, hidden, s, [](float (&v)[1][VT], int e, float val) { v[0][e] = v[0][e] + val; });
     tree_sum8<1>(s, red, p, nv >> 5, tot);
     if (p == 0) sum_out[blockIdx.x] = (half_t)tot[0];
   }
@@ -587,6 +593,16 @@ static inline int norm_block(int hidden, bool round32) {
   return b;
 }
 
+// Many rows of more than 8192, quantised with their sum: f32 copies would leave a CU two rows of 14336 (57 KB each).  (MI355X, f32 / fp16: quant_fuse_sum of 14336, 1501 rows
+// 18.3 / 16.1 us, 5000 46.1 / 36.3, 12001 113.3 / 92.5; of 16384, 1100 rows 16.2 / 14.9; of 8192, 1501 rows 10.1 / 10.6.)
+template <typename Src>
+static bool quant_half_copy(int8_t* out, const Src& src, half_t* sum, half_t* scale, int tokens, int hidden, int nv, hipStream_t st) {
+  if (tokens < ROWS_MANY || hidden <= 8192 || hidden > 256 * 8 * VT) return false;
+  const PrefetchArgs pf = take_prefetch(tokens);      // (no rider beside many rows)
+  hipLaunchKernelGGL((quant_v2_kernel<256, 8, true, Src, true>), dim3(tokens), dim3(256), (size_t)hidden * sizeof(half_t), st, out, src, sum, scale, hidden, nv, pf);
+  return true;
+}
+
 }  // namespace omni
 
 using namespace omni;
@@ -618,6 +634,8 @@ extern "C" int omni_quant_fuse_sum(void* out_i8, const void* in_f16, void* sum_f
   if (tokens == 0) return OMNI_OK;
   const int nv = norm_block(hidden, false);
   if (v2_ok(hidden, nv)) {
+    if (quant_half_copy((int8_t*)out_i8, SrcPlain{(const half_t*)in_f16, hidden}, (half_t*)sum_f16, (half_t*)scale_f16, tokens, hidden, nv, (hipStream_t)stream))
+      return omni_launch_status();
     #undef KQ_
     #define KQ_(RT_, RV_) quant_v2_kernel<RT_, RV_, true, SrcPlain>
     OMNI_V2_LAUNCH(KQ_, tokens, hidden, hidden, (int8_t*)out_i8, SrcPlain{(const half_t*)in_f16, hidden},
@@ -819,6 +837,8 @@ extern "C" int omni_silu_mul_quant_fuse_sum(void* out_i8, const void* in_f16, vo
     const int nv = norm_block(d, false);
     if (v2_ok(d, nv)) {
       if (sum_f16) {
+        if (quant_half_copy((int8_t*)out_i8, SrcSilu{(const half_t*)in_f16, d}, (half_t*)sum_f16, (half_t*)scale_f16, tokens, d, nv, (hipStream_t)stream))
+          return omni_launch_status();
         #undef KQ_
         #define KQ_(RT_, RV_) quant_v2_kernel<RT_, RV_, true, SrcSilu>
         OMNI_V2_LAUNCH(KQ_, tokens, d, d, (int8_t*)out_i8, SrcSilu{(const half_t*)in_f16, d},

@@ -98,4 +98,24 @@ __device__ __forceinline__ void ordered_partials(const float* xs, int p, int nv,
   }
 }
 
+// the row sum from an fp16 copy that holds the values exactly: ordered_partials<1> of additions
+__device__ __forceinline__ void ordered_sums(const half_t* xs, int p, int nv, int hidden, float (&v)[1][VT]) {
+#pragma unroll
+  for (int e = 0; e < VT; ++e) v[0][e] = 0.0f;
+  if (VT * p < nv) {
+    for (int i = VT * p; i < hidden; i += 4 * nv) {
+      v8h a[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const v8h*>(xs + ((i + c * nv) < hidden ? i + c * nv : i));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if ((i + c * nv) < hidden) {
+#pragma unroll
+          for (int e = 0; e < VT; ++e) v[0][e] = v[0][e] + (float)a[c][e];
+        }
+      }
+    }
+  }
+}
+
 }  // namespace omni
