@@ -40,7 +40,14 @@ struct NormProductArgs {
 // rows in the form for 8, 1048 us a step of 16 layers of 4096 / 11008, 921 in that for 2; the 8B model's step of 16 layers behind 4, 1 and 2 rows, 680 -> 662 and 782 -> 750); 0: the
 // residual as it is.  ROWS: M.
 template <int MODE, int EPI, int BLOCKS, int C, int SK, int ROWS>
-__global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(NormProductArgs p) {
+struct NormProduct {
+  constexpr static int K = 1024 * C, PITCH = K + 64, PART_BYTES = RowProduct<MODE, EPI ? LAYOUT_GATE : LAYOUT_ROWS32, BLOCKS, K / RP_WAVES, 1, ROWS>::PART_BYTES;
+  constexpr static int LDS_BYTES = ROWS * PITCH + PART_BYTES + ROWS * 512;
+};
+
+// first: the workgroup's first operand block of all; ng: its place in the grid
+template <int MODE, int EPI, int BLOCKS, int C, int SK, int ROWS>
+__device__ __forceinline__ void norm_product(const NormProductArgs& p, uint8_t* lds, int first, int ng) {
   constexpr bool ZP = MODE == MODE_CHN, W8 = MODE == MODE_W8;
   constexpr int K = 1024 * C, KPART = K / RP_WAVES;
   // units requested in front of the rows' first wait, and (the slabs' registers are free then) all that fly together
@@ -49,14 +56,13 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
   typedef RowProduct<MODE, EPI ? LAYOUT_GATE : LAYOUT_ROWS32, BLOCKS, KPART, RING_MAX, ROWS> Product;
   constexpr int FIRST = FIRST_MAX < Product::RING ? FIRST_MAX : Product::RING;
   constexpr int PITCH = K + 64;
-  constexpr int LDS_PARTS = ROWS * PITCH, LDS_RED = LDS_PARTS + Product::PART_BYTES, LDS_ALL = LDS_RED + ROWS * 512;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_ALL];
+  constexpr int LDS_PARTS = ROWS * PITCH, LDS_RED = LDS_PARTS + Product::PART_BYTES;
   uint8_t* const codes = lds;
   uint8_t* const parts = lds + LDS_PARTS;
   float (*red)[128] = reinterpret_cast<float (*)[128]>(lds + LDS_RED);
   asm volatile("" ::"s"(p.res), "s"(p.slab), "s"(p.sk), "s"(p.p_wscales), "s"(p.p_wsz), "s"(p.p_ascales), "s"(p.p_asum), "s"(p.gamma), "s"(p.W),
                "s"(p.wscales), "s"(p.wsz), "s"(p.N));
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ng = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t at = 4 * tid;
 
   // ---- requests: the rows ----
@@ -92,14 +98,15 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
   }
   // ---- ... the scales of the channel that this lane finishes ----
   int chan;
-  if constexpr (EPI) chan = ((lane >> 3) & 1) * (p.N / 2) + ng * 32 + (lane >> 4) * 8 + (lane & 7);
+  const int block = min(lane >> 4, BLOCKS - 1);
+  if constexpr (EPI) chan = ((lane >> 3) & 1) * (p.N / 2) + (first + block) * 8 + (lane & 7);
   else chan = ng * 32 + (lane & 31);
   const half_t sw_own = p.wscales[chan];
   half_t sz_own = (half_t)0.0f;
   if constexpr (ZP) sz_own = p.wsz[chan];
   // ---- ... and the weights ----
   Product product;
-  product.open(p.W, p.s2s, p.s2z, p.N, K, ng * BLOCKS, wave * KPART);
+  product.open(p.W, p.s2s, p.s2z, p.N, K, first, wave * KPART);
   __builtin_amdgcn_sched_barrier(0);      // what the rows need returns first: loads return in order
 #pragma unroll
   for (int u = 0; u < FIRST; ++u) product.request(u);
@@ -166,7 +173,7 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
         sum = row_sum[i];
       }
     int total;
-    if constexpr (EPI) total = Product::total(parts, lane >> 4, lane & 15, m);
+    if constexpr (EPI) total = Product::total(parts, block, lane & 15, m);
     else if constexpr (W8) total = Product::total(parts, (lane >> 4) & 1, lane & 15, m);
     else total = Product::total(parts, (lane >> 3) & 3, (lane & 7) + 8 * (lane >> 5), 2 * m + (lane >> 5));
     if constexpr (Product::PAIRED) total += __shfl_xor(total, 32, 64);
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
     if constexpr (EPI) {
       const int up = __shfl_xor((int)__builtin_bit_cast(uint16_t, h), 8, 64);
       const half_t act = silu_mul_h(h, __builtin_bit_cast(half_t, (uint16_t)up));      // (of lanes with a gate channel)
-      const bool gate = !(lane & 8);
+      const bool gate = !(lane & 8) && (lane >> 4) < BLOCKS;
       if (gate) out[chan] = act;
       const float top = wave_max64(gate ? __builtin_fabsf((float)act) : 0.0f);
       if (lane == 0) amax_raise(p.amax, m, ng >> 3, top);
@@ -184,13 +191,30 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
     }
   }
   if constexpr (SK > 0) {
-    if (blockIdx.x == 0) {
+    if (ng == 0) {
 #pragma unroll
       for (int m = 0; m < ROWS; ++m)
 #pragma unroll
         for (int c = 0; c < C; ++c) RowArray(p.res_out + (size_t)m * K).put(at, 2048 * c, o[m][c]);
     }
   }
+}
+
+template <int MODE, int EPI, int BLOCKS, int C, int SK, int ROWS>
+__global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(NormProductArgs p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[NormProduct<MODE, EPI, BLOCKS, C, SK, ROWS>::LDS_BYTES];
+  norm_product<MODE, EPI, BLOCKS, C, SK, ROWS>(p, lds, (int)blockIdx.x * BLOCKS, blockIdx.x);
+}
+
+// gate_up of int8 weights in two workgroups a compute unit: the first `wide` of them take four blocks of eight gate and eight up channels, the others three.  448
+// workgroups of four leave a quarter of the units with one, and a unit takes in its weights at a rate of its own.  (MI355X, 28672 x
+// 4096: four LServe steps of 4 layers 1607 -> 1585 us.  Packed weights hold two blocks in a byte and cannot be dealt in threes.)
+template <int C, int SK>
+__global__ __launch_bounds__(RP_THREADS, 4) void gate_up_even_kernel(NormProductArgs p, int wide) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[NormProduct<MODE_W8, 1, 4, C, SK, 1>::LDS_BYTES];
+  const int ng = blockIdx.x;
+  if (ng < wide) norm_product<MODE_W8, 1, 4, C, SK, 1>(p, lds, 4 * ng, ng);
+  else norm_product<MODE_W8, 1, 3, C, SK, 1>(p, lds, 3 * ng + wide, ng);
 }
 
 }  // namespace omni
@@ -201,6 +225,13 @@ namespace {
 template <int MODE, int EPI, int BLOCKS, int C, int SK>
 void launch_rows(const NormProductArgs& p, hipStream_t st) {
   const dim3 grid(EPI ? p.N / 64 : p.N / 32), block(RP_THREADS);
+  if constexpr (MODE == MODE_W8 && EPI) {
+    const int wide = p.N / 16 - 3 * 512;
+    if (wide > 0 && wide < 512) {
+      hipLaunchKernelGGL((gate_up_even_kernel<C, SK>), dim3(512), block, 0, st, p, wide);
+      return;
+    }
+  }
   if constexpr (MODE != MODE_W8 && SK <= 8) {      // (two rows with int8 weights, or of 16 slabs, do not fit the registers)
     if (p.M == 2) {
       hipLaunchKernelGGL((norm_product_kernel<MODE, EPI, BLOCKS, C, SK, 2>), grid, block, 0, st, p);
