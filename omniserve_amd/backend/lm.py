@@ -230,33 +230,18 @@ class LmOps:
         return out
 
     def glu(self, x, w, bias, act):
-        """act(x gate^T + bias) * (x up^T + bias); w [2 n, k] (and its bias) in alternating blocks of 16 gate and up channels.  One launch for few
-        rows and where the tiles do well (_unit_in_tiles), else the vendor product and a row kernel."""
+        """act(x gate^T + bias) * (x up^T + bias); w [2 n, k] (and its bias) in alternating blocks of 16 gate and up channels.  Few
+        rows: one launch; many: the vendor product and a row kernel."""
         T, n = x.shape[0], w.shape[0] // 2
         out = torch.empty((T, n), dtype=self.dtype, device=x.device)
         if T <= ROWS_MAX:
             part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), 2 * n, w.shape[1], bias=_p(bias))
             sums = self._slices(x, w, EPI_GLU)
             self._call("lm_gemm_rows", _c.byref(part), None, 1, None, None, T, 0, 1, T, 1.0, EPI_GLU, ACT[act], _p(sums))
-        elif self._unit_in_tiles(x, w):
-            part = _Part(_p(w), _p(x), _ld(x), _p(out), _ld(out), 2 * n, w.shape[1], bias=_p(bias))
-            self._call("lm_gemm_tiles", _c.byref(part), None, 1, None, None, None, 0, T, 0, 1, 1.0, EPI_GLU, ACT[act])
         else:
             y = self.matmul(x, w)
             self._call("lm_glu", _p(out), _ld(out), _p(y), _ld(y), _p(bias), T, n, ACT[act])
         return out
-
-    def _unit_in_tiles(self, x, w):
-        """Is a gated unit of many rows faster in tiles that hold gate and up?  The vendor's product is up to a tenth faster than the tiles, the
-        unit's rows of their own take 5 - 40 % of it: the more the shorter K.  So: short K, or rounds of 256 tiles that are full enough.  (MI355X, product
-        and rows / tiles, us: 15963 rows of 12288 x 2048 700 / 630 (between a prompt's other launches 707 / 690); 7150 of 28672 x 4096, 12.3 rounds, 1272 / 1272; 1000 of it, 1.75 rounds, 206 / 192; 700 of it,
-        1.3 rounds, 168 / 178; 3000 of 12288 x 2048, 2.25 rounds, 154 / 167; 5000 of 16384 x 1024 196 / 156; 700 of 57344 x 8192 549 / 600.  Over 127
-        sizes of 130 rows and more the rule takes 9 % less time than without the tiles, the better of the two 11 %; no size loses more than 8 %.)"""
-        T, (n, k) = x.shape[0], w.shape
-        if self.dtype != torch.bfloat16 or k % 64 or n % 32 or not w.is_contiguous() or (_p(x) | _p(w)) % 16 or _ld(x) % 8:
-            return False
-        rounds = ((T + 255) // 256 * ((n + 255) // 256) + 255) // 256
-        return T >= 128 and (k <= 1536 or T * n >= (0.65 + 0.1 * k / 2048) * rounds * (256 << 16))
 
     def head_products(self, x, w, out, x_step, out_step, gate=None):
         """One matrix per head, w [heads, n, k]: head h reads x from column h * x_step and writes out from column h * out_step;

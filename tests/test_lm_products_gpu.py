@@ -368,3 +368,13 @@ def test_equal_channels_have_equal_gated_units():
 def test_128_channels_keep_the_order_of_sums(epi, n, k, m, narrow):
     """Workgroups of 128 channels take K in one chain of stages: they stand in for narrower ones that do, too, not for those with K slices or K parts."""
     assert _rows_plan(_ops(torch.bfloat16), 1, n, k, m, epi) == narrow
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 32, 64), (1000, 14336, 2048), (2000, 6144, 2048), (300, 1024, 512)])
+def test_gated_unit_of_many_rows_has_the_bits_of_product_and_unit(m, n, k):
+    """Gate and up of more than 64 rows are the product's rows, rounded to the element type, whatever the number of rows."""
+    ops = _ops(torch.bfloat16)
+    x, w, b = _randn(61, torch.bfloat16, m, k), _randn(62, torch.bfloat16, 2 * n, k) * k ** -0.5, _randn(63, torch.float32, 2 * n)
+    y, want = ops.matmul(x, w), torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+    ops._call("lm_glu", want.data_ptr(), n, y.data_ptr(), 2 * n, b.data_ptr(), m, n, 1)
+    assert torch.equal(ops.glu(x, w, b, "silu"), want)
