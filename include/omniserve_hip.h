@@ -434,6 +434,8 @@ int omni_prefill_attention_block_streaming(void* out_f16, const void* q_f16, con
  * form on the 8-wave ping-pong schedule (waves 4-7 one segment behind waves 0-3; same results within the attention tolerance),
  * 3 / 4 = the 16-row form in workgroups of 64 / 128 rows whatever the size (0 takes the one that is faster: the same bits). */
 void omni_prefill_set_variant(int variant);
+/* Query rows of a workgroup (64 or 128) that form 0 takes; same_offsets: queries and keys have one array of offsets; 0: no such sizes. */
+int omni_prefill_attention_rows(int batch, int max_seqlen_q, int num_heads, int num_kv_heads, int causal, int same_offsets, int streaming_heads);
 
 /* Tuning hook: over how many XCDs the query tiles of one kv head are spread when streaming heads are present
  * (head_mask_type != NULL): 1, 2, 4 or 8; 0 = the default (8).  Results do not depend on it. */

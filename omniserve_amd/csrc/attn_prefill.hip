@@ -461,7 +461,7 @@ __device__ __forceinline__ void rows16_values(const uint8_t* vt, int tr_a0, cons
 // Where the 128-row kernel has about one workgroup on a CU, its eight waves go through scores, softmax and values in step (1.6 us a tile of 64
 // keys) and its longest query tile is the launch.  Here four workgroups of a CU, each at its own place, cover one another's waits; K of the next tile
 // is requested as soon as everyone has formed this one's scores and flies under softmax and values, V of it behind the values and flies under
-// the next scores and softmax.  The price is K and V brought in once per 64 rows, which is what large launches are short of.  A row meets the same
+// the next scores and softmax.  The price is K and V brought in once per 64 rows, which is what large launches are short of (small_tiles).  A row meets the same
 // tiles in the same order: the same bits.
 // MI355X, 32 / 8 heads, 128 rows / here, us: one prompt of 129 tokens 9.6 / 7.9, 333 14.0 / 12.0, 1501 44.6 / 40.7, 2048 60.5 / 58.0, 4000 179 / 180, 8192 617 / 691;
 // 7 x 333 31.4 / 25.4, 16 x 375 57 / 48, 16 x 100 13.7 / 12.6, 4 x 1500 116 / 117; 3 x 801, 28 / 4 heads, 43.0 / 32.9.  (Two K and two V buffers, two
@@ -1002,10 +1002,25 @@ static thread_local int g_prefill_xcd_split = 0;
 // Tuning hook: XCDs that share one kv head's query tiles when streaming heads are present (0 = default, else 1 / 2 / 4 / 8).
 extern "C" void omni_prefill_set_xcd_split(int w) { g_prefill_xcd_split = (w == 1 || w == 2 || w == 4 || w == 8) ? w : 0; }
 
-// 64-row workgroups?  Less than one round of two 128-row ones on every CU, or short prompts (figures at prefill_attn_small_kernel); longer keys than
-// queries, which the host cannot see (another array of offsets), count as long ones.
-static bool small_tiles(int batch, int max_seqlen_q, int num_heads, bool self) {
-  return (self && max_seqlen_q <= 1024) || (long long)batch * num_heads * ((max_seqlen_q + PQROWS - 1) / PQROWS) < 512;
+// 64-row workgroups (prefill_attn_small_kernel)?  They bring K and V in once per 64 rows, in an order that takes all sequences' tiles of one length together.  So:
+// causal prompts over their own keys (keys of another array of offsets are more than the host can see: 512 queries behind 8192, 32768 and 100000 keys take 162, 609 and 1972 us
+// with 128 rows, 177, 690 and 2540 with 64), up to 1024 of them or less than one round of two 128-row workgroups on every CU, and
+//   * all heads dense: keys and values of at most 60 MB for every query head of a kv head, up to 240, which the caches hold between the tiles that share them (32 / 32 heads, 128 / 64 rows, us: 4 x 1000
+//     62.4 / 58.7, 66 MB; 16 x 333 54.1 / 57.6, 87 MB; 16 x 1024 227 / 356; 64 x 1024 898 / 2044; 32 / 16 heads 64 x 512, 268 MB, 332 / 329, 64 x 1024 962 / 1234; 32 / 8 heads
+//     16 x 1024, 67 MB, 232 / 226; 64 / 8 heads 64 x 1024, 268 MB, 1863 / 1915);
+//   * streaming heads among them: four query heads a kv head, or up to 512 queries (32 / 32 heads: 1 x 1024 31.8 / 33.2, 16 x 1024 288 / 355, 16 x 512 202 / 146; 32 / 8 heads: 16 x 1000 256 / 226).
+// Not causal: 1024 28.2 / 32.6, 7 x 333 33.8 / 35.7, 16 x 1000 359 / 394.  (MI355X; 960 sizes of 1 - 64 heads: none that
+// the rule takes is slower by more than 2 %, but those of up to 64 tokens, 5 - 6 us, by 0.1 - 0.3.)
+static bool small_tiles(int batch, int max_seqlen_q, int num_heads, int num_kv_heads, bool causal, bool self, bool streaming) {
+  if (!causal || !self || (max_seqlen_q > 1024 && (long long)batch * num_heads * ((max_seqlen_q + PQROWS - 1) / PQROWS) >= 512)) return false;
+  const int share = num_heads / num_kv_heads;
+  if (streaming) return share >= 4 || max_seqlen_q <= 512;
+  return (long long)batch * max_seqlen_q * num_kv_heads * (2 * PDH * (int)sizeof(half_t)) <= 60'000'000LL * min(share, 4);
+}
+
+extern "C" int omni_prefill_attention_rows(int batch, int max_seqlen_q, int num_heads, int num_kv_heads, int causal, int same_offsets, int streaming_heads) {
+  if (batch < 1 || max_seqlen_q < 1 || num_kv_heads < 1 || num_heads < num_kv_heads) return 0;
+  return small_tiles(batch, max_seqlen_q, num_heads, num_kv_heads, causal != 0, same_offsets != 0, streaming_heads != 0) ? SM_ROWS : PQROWS;
 }
 
 static int prefill_attention_common(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16,
@@ -1027,7 +1042,7 @@ static int prefill_attention_common(void* out_f16, const void* q_f16, const void
   a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.causal = causal;
   a.gran_log2 = gran_log2;
   const bool form32 = g_prefill_variant == 1;
-  const bool small = g_prefill_variant == 3 || (g_prefill_variant == 0 && small_tiles(batch, max_seqlen_q, num_heads, cu_seqlens_q_i32 == cu_seqlens_k_i32));
+  const bool small = g_prefill_variant == 3 || (g_prefill_variant == 0 && small_tiles(batch, max_seqlen_q, num_heads, num_kv_heads, causal != 0, cu_seqlens_q_i32 == cu_seqlens_k_i32, head_mask_type_i32 != nullptr));
   const int rows_per_wg = form32 ? P32ROWS : PQROWS;
   const int q_tiles = (max_seqlen_q + rows_per_wg - 1) / rows_per_wg * (small ? PQROWS / SM_ROWS : 1);
   dim3 grid(q_tiles, num_heads, batch);
