@@ -229,14 +229,17 @@ def gate_up_rows(out, in_feats, weight, operands, gate_up, input_sum, scale):
     those calls'.  Where the product's tiles have the unit it leaves fp16 [M, N/2] in `gate_up` (room for [M, N], contiguous) instead of both halves.
     operands: per-channel (wscales, ascales, w_szs, a_ssums), per-group (s2_zeros, s2_scales, wscales, ascales), W8A8 (wscales, ascales)."""
     from . import fused_kernels, qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
-    _lib.require_cuda(out, in_feats, weight, gate_up, scale, *operands)
-    (M, K), N, h = in_feats.shape, weight.shape[0], _lib.lib()
-    w8 = len(operands) == 2
-    group = not w8 and operands[0].dim() == 2 and operands[0].dtype == torch.int8
+    from ._gemm_common import check_gemm_io
+    w8, h = len(operands) == 2, _lib.lib()
+    M, N, K, _ = check_gemm_io(in_feats, weight, gate_up, packed=not w8)
+    _lib.require_cuda(out, scale, input_sum, *operands)
+    group = not w8 and operands[0].dim() == 2
+    if group and (tuple(operands[0].shape) != (K // 128, N) or tuple(operands[1].shape) != (K // 128, N)):
+        raise RuntimeError("per-group gemm: zeros/scales_i8 must be [K/128, N]")
     name, product = (("omni_w8a8_gemm_silu_rows", qgemm_w8a8.w8a8_gemm_forward_cuda) if w8 else
                      ("omni_w4a8_per_group_gemm_silu_rows", qgemm_w4a8_per_group.gemm_forward_cuda) if group else
                      ("omni_w4a8_per_chn_gemm_silu_rows", qgemm_w4a8_per_chn.gemm_forward_cuda))
-    if (h.omni_gemm_silu_rows_ok(M, N, K, 2 if w8 else int(group)) and gate_up.is_contiguous() and in_feats.is_contiguous() and
+    if (h.omni_gemm_silu_rows_ok(M, N, K, 2 if w8 else int(group)) and gate_up.is_contiguous() and
             (N <= 32768 or M >= 1024) and      # (few rows wider than that: only the unit's quantiser has a kernel of whole rows)
             (gate_up.data_ptr() | in_feats.data_ptr() | weight.data_ptr()) % 16 == 0 and not (group and (operands[0].data_ptr() | operands[1].data_ptr()) % 4)):
         act = gate_up.view(-1)[:M * (N // 2)].view(M, N // 2)
