@@ -228,30 +228,35 @@ def gate_up_rows(out, in_feats, weight, operands, gate_up, input_sum, scale):
     """gate_up projection, silu_and_mul and invoke_quant[_fuse_sum] (input_sum=None: without the sum) of many rows -> int8 out [M, N/2] and its scale, bit for bit
     those calls'.  Where the product's tiles have the unit it leaves fp16 [M, N/2] in `gate_up` (room for [M, N], contiguous) instead of both halves.
     operands: per-channel (wscales, ascales, w_szs, a_ssums), per-group (s2_zeros, s2_scales, wscales, ascales), W8A8 (wscales, ascales)."""
-    from . import fused_kernels, qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
+    w8 = len(operands) == 2
+    group = not w8 and operands[0].dim() == 2
+    f = _lib.fast()
+    if f is not None:      # a prompt's layers are launched eagerly, and a short one's by a host that is behind: one call
+        call = f.gate_up_w8a8 if w8 else f.gate_up_w4a8_per_group if group else f.gate_up_w4a8_per_chn
+        return call(out, in_feats, weight, *operands, gate_up, input_sum, scale)
+    from . import qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
     from ._gemm_common import check_gemm_io
-    w8, h = len(operands) == 2, _lib.lib()
     M, N, K, _ = check_gemm_io(in_feats, weight, gate_up, packed=not w8)
     _lib.require_cuda(out, scale, input_sum, *operands)
-    group = not w8 and operands[0].dim() == 2
     if group and (tuple(operands[0].shape) != (K // 128, N) or tuple(operands[1].shape) != (K // 128, N)):
         raise RuntimeError("per-group gemm: zeros/scales_i8 must be [K/128, N]")
-    name, product = (("omni_w8a8_gemm_silu_rows", qgemm_w8a8.w8a8_gemm_forward_cuda) if w8 else
-                     ("omni_w4a8_per_group_gemm_silu_rows", qgemm_w4a8_per_group.gemm_forward_cuda) if group else
-                     ("omni_w4a8_per_chn_gemm_silu_rows", qgemm_w4a8_per_chn.gemm_forward_cuda))
-    if (h.omni_gemm_silu_rows_ok(M, N, K, 2 if w8 else int(group)) and gate_up.is_contiguous() and
-            (N <= 32768 or M >= 1024) and      # (few rows wider than that: only the unit's quantiser has a kernel of whole rows)
-            (gate_up.data_ptr() | in_feats.data_ptr() | weight.data_ptr()) % 16 == 0 and not (group and (operands[0].data_ptr() | operands[1].data_ptr()) % 4)):
-        act = gate_up.view(-1)[:M * (N // 2)].view(M, N // 2)
-        _lib.check(getattr(h, name)(in_feats.data_ptr(), weight.data_ptr(), *(t.data_ptr() for t in operands), act.data_ptr(), M, N, K, _lib.current_stream()),
-                   "fused_ext.gate_up_rows")
-        if input_sum is None:
-            fused_kernels.invoke_quant(out, act, scale)
-        else:
-            fused_kernels.invoke_quant_fuse_sum(out, act, input_sum, scale)
-        return
-    product(in_feats, weight, *operands, gate_up)
-    silu_mul_quant_fuse_sum(out, gate_up, input_sum, scale)
+    h, st = _lib.lib(), _lib.current_stream()
+    unit, product = ((h.omni_w8a8_gemm_silu_rows, qgemm_w8a8.w8a8_gemm_forward_cuda) if w8 else
+                     (h.omni_w4a8_per_group_gemm_silu_rows, qgemm_w4a8_per_group.gemm_forward_cuda) if group else
+                     (h.omni_w4a8_per_chn_gemm_silu_rows, qgemm_w4a8_per_chn.gemm_forward_cuda))
+    # the entry refuses sizes without the unit, and rows and weights between two boundaries; few rows of more than 16384 channels: only the unit's quantiser has a
+    # kernel of whole rows
+    rc = -22
+    if gate_up.is_contiguous() and (N <= 32768 or M >= 1024):
+        rc = unit(in_feats.data_ptr(), weight.data_ptr(), *(t.data_ptr() for t in operands), gate_up.data_ptr(), M, N, K, st)
+    if rc == -22:
+        product(in_feats, weight, *operands, gate_up)
+        return silu_mul_quant_fuse_sum(out, gate_up, input_sum, scale)
+    if rc == 0 and input_sum is None:
+        rc = h.omni_quant(out.data_ptr(), gate_up.data_ptr(), scale.data_ptr(), M, N // 2, st)
+    elif rc == 0:
+        rc = h.omni_quant_fuse_sum(out.data_ptr(), gate_up.data_ptr(), input_sum.data_ptr(), scale.data_ptr(), M, N // 2, st)
+    _lib.check(rc, "fused_ext.gate_up_rows")
 
 
 def gemm_partial_f16_per_chn(act, amax, qweight, slab, sum_out, scale_out):

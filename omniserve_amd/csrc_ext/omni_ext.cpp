@@ -84,12 +84,17 @@ void gemm_w4a8_per_chn(const torch::Tensor& in, const torch::Tensor& w, const to
        "qgemm_w4a8_per_chn.gemm_forward_cuda");
 }
 
+inline void check_second_level(const torch::Tensor& zeros, const torch::Tensor& scales_i8, const GemmIO& g) {
+  need_cuda(zeros, "gemm_forward"); need_cuda(scales_i8, "gemm_forward");
+  TORCH_CHECK(zeros.dim() == 2 && zeros.size(0) == g.K / 128 && zeros.size(1) == g.N && scales_i8.dim() == 2 &&
+              scales_i8.size(0) == g.K / 128 && scales_i8.size(1) == g.N, "per-group gemm: zeros/scales_i8 must be [K/128, N]");
+}
+
 void gemm_w4a8_per_group(const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& zeros, const torch::Tensor& scales_i8,
                          const torch::Tensor& wscales, const torch::Tensor& ascales, torch::Tensor out) {
   const GemmIO g = check_gemm_io(in, w, out, true);
-  need_cuda(zeros, "gemm_forward"); need_cuda(scales_i8, "gemm_forward"); need_cuda(wscales, "gemm_forward"); need_cuda(ascales, "gemm_forward");
-  TORCH_CHECK(zeros.dim() == 2 && zeros.size(0) == g.K / 128 && zeros.size(1) == g.N && scales_i8.dim() == 2 &&
-              scales_i8.size(0) == g.K / 128 && scales_i8.size(1) == g.N, "per-group gemm: zeros/scales_i8 must be [K/128, N]");
+  check_second_level(zeros, scales_i8, g);
+  need_cuda(wscales, "gemm_forward"); need_cuda(ascales, "gemm_forward");
   fail(with_scratch(g, in, [&](void* ws, size_t n) {
          return omni_w4a8_per_group_gemm(in.data_ptr(), w.data_ptr(), zeros.data_ptr(), scales_i8.data_ptr(), wscales.data_ptr(), ascales.data_ptr(),
                                          out.data_ptr(), g.M, g.N, g.K, g.stride, ws, n, stream_of(in)); }),
@@ -103,6 +108,60 @@ void gemm_w8a8(const torch::Tensor& in, const torch::Tensor& w, const torch::Ten
          return omni_w8a8_gemm(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), out.data_ptr(), g.M, g.N, g.K, g.stride,
                                ws, n, stream_of(in)); }),
        "qgemm_w8a8.w8a8_gemm_forward_cuda");
+}
+
+// fused_ext.gate_up_rows: gate_up, silu_and_mul and their quantiser (sum: none without).  The product with the unit in its tiles where there is one -- its entry refuses
+// other sizes, and rows and weights between two boundaries --, which leaves [M, N/2] at the start of gate_up; else the product and the unit's own quantiser.
+template <class Unit, class Product>
+void gate_up(const GemmIO& g, const torch::Tensor& in, torch::Tensor& out, torch::Tensor& gate_up, const c10::optional<torch::Tensor>& sum, torch::Tensor& scale,
+             Unit unit, Product product) {
+  need_cuda(out, "gate_up_rows"); need_cuda(scale, "gate_up_rows");
+  if (sum) need_cuda(*sum, "gate_up_rows");
+  void* const s = sum ? sum->data_ptr() : nullptr;
+  void* const st = stream_of(in);
+  // (few rows of more than 16384 channels: only the unit's quantiser has a kernel of whole rows)
+  const int rc = gate_up.is_contiguous() && (g.N <= 32768 || g.M >= 1024) ? unit(st) : -22;
+  if (rc == -22) {
+    product();
+    fail(omni_silu_mul_quant_fuse_sum(out.data_ptr(), gate_up.data_ptr(), s, scale.data_ptr(), g.M, g.N / 2, st), "fused_ext.gate_up_rows");
+    return;
+  }
+  fail(rc, "fused_ext.gate_up_rows");
+  if (s) fail(omni_quant_fuse_sum(out.data_ptr(), gate_up.data_ptr(), s, scale.data_ptr(), g.M, g.N / 2, st), "fused_ext.gate_up_rows");
+  else fail(omni_quant(out.data_ptr(), gate_up.data_ptr(), scale.data_ptr(), g.M, g.N / 2, st), "fused_ext.gate_up_rows");
+}
+
+void gate_up_w4a8_per_chn(torch::Tensor out, const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& wscales, const torch::Tensor& ascales,
+                          const torch::Tensor& w_szs, const torch::Tensor& a_ssums, torch::Tensor gu, const c10::optional<torch::Tensor>& sum, torch::Tensor scale) {
+  const GemmIO g = check_gemm_io(in, w, gu, true);
+  need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows"); need_cuda(w_szs, "gate_up_rows"); need_cuda(a_ssums, "gate_up_rows");
+  gate_up(g, in, out, gu, sum, scale,
+          [&](void* st) {
+            return omni_w4a8_per_chn_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), w_szs.data_ptr(), a_ssums.data_ptr(),
+                                                    gu.data_ptr(), g.M, g.N, g.K, st); },
+          [&] { gemm_w4a8_per_chn(in, w, wscales, ascales, w_szs, a_ssums, gu); });
+}
+
+void gate_up_w4a8_per_group(torch::Tensor out, const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& zeros, const torch::Tensor& scales_i8,
+                            const torch::Tensor& wscales, const torch::Tensor& ascales, torch::Tensor gu, const c10::optional<torch::Tensor>& sum, torch::Tensor scale) {
+  const GemmIO g = check_gemm_io(in, w, gu, true);
+  check_second_level(zeros, scales_i8, g);
+  need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
+  gate_up(g, in, out, gu, sum, scale,
+          [&](void* st) {
+            return omni_w4a8_per_group_gemm_silu_rows(in.data_ptr(), w.data_ptr(), zeros.data_ptr(), scales_i8.data_ptr(), wscales.data_ptr(), ascales.data_ptr(),
+                                                      gu.data_ptr(), g.M, g.N, g.K, st); },
+          [&] { gemm_w4a8_per_group(in, w, zeros, scales_i8, wscales, ascales, gu); });
+}
+
+void gate_up_w8a8(torch::Tensor out, const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& wscales, const torch::Tensor& ascales, torch::Tensor gu,
+                  const c10::optional<torch::Tensor>& sum, torch::Tensor scale) {
+  const GemmIO g = check_gemm_io(in, w, gu, false);
+  need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
+  gate_up(g, in, out, gu, sum, scale,
+          [&](void* st) {
+            return omni_w8a8_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), gu.data_ptr(), g.M, g.N, g.K, st); },
+          [&] { gemm_w8a8(in, w, wscales, ascales, gu); });
 }
 
 // fp16 row kernels (the other element types and the static-scale overloads stay on the ctypes mirror)
@@ -188,6 +247,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_w4a8_per_chn", &gemm_w4a8_per_chn);
   m.def("gemm_w4a8_per_group", &gemm_w4a8_per_group);
   m.def("gemm_w8a8", &gemm_w8a8);
+  m.def("gate_up_w4a8_per_chn", &gate_up_w4a8_per_chn);
+  m.def("gate_up_w4a8_per_group", &gate_up_w4a8_per_group);
+  m.def("gate_up_w8a8", &gate_up_w8a8);
   m.def("rms_norm_general_fuse_sum_f16", &rms_norm_general_fuse_sum_f16);
   m.def("rms_norm_general_f16", &rms_norm_general_f16);
   m.def("rms_norm_f16", &rms_norm_f16);

@@ -281,8 +281,8 @@ def test_fast_binding_is_built_and_exports_the_routed_functions():
     _lib.lib()
     e = importlib.import_module("omniserve_amd._omni_ext")
     assert e.abi_version() == _lib.lib().omni_abi_version()
-    for name in ("gemm_w4a8_per_chn", "gemm_w4a8_per_group", "gemm_w8a8", "rms_norm_general_fuse_sum_f16", "rms_norm_general_f16",
-                 "rms_norm_f16", "quant_fuse_sum_f16", "quant_f16", "silu_and_mul_f16", "decode_attention_kv4"):
+    for name in ("gemm_w4a8_per_chn", "gemm_w4a8_per_group", "gemm_w8a8", "gate_up_w4a8_per_chn", "gate_up_w4a8_per_group", "gate_up_w8a8",
+                 "rms_norm_general_fuse_sum_f16", "rms_norm_general_f16", "rms_norm_f16", "quant_fuse_sum_f16", "quant_f16", "silu_and_mul_f16", "decode_attention_kv4"):
         assert callable(getattr(e, name))
     import torch
     if not torch.cuda.is_available():

@@ -67,6 +67,26 @@ def test_gemms_agree(M, N, K):
     assert (r1[0][0] == 7).all() and (r1[0][M + 1] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K,mode", [(136, 1024, 512, 0), (700, 16384, 256, 0), (136, 1024, 512, 1), (700, 16384, 256, 1), (300, 512, 768, 2), (2700, 28672, 1024, 2)])
+def test_gate_up_rows_agree(M, N, K, mode):
+    """with the unit in the product's tiles and without"""
+    from omniserve_amd.backend import fused_ext
+    from tests.test_silu_rows_gpu import _case
+    x, w, ops = _case(M, N, K, mode)
+
+    def run():
+        q = torch.full((M, N // 2), 77, dtype=torch.int8, device=dev())
+        s, m = torch.zeros((M,), dtype=torch.float16, device=dev()), torch.zeros((M,), dtype=torch.float16, device=dev())
+        gu = torch.full((M, N), 7.0, dtype=torch.float16, device=dev())
+        assert fused_ext.gate_up_rows(q, x, w, ops, gu, None if mode == 2 else m, s) is None
+        with pytest.raises(RuntimeError):
+            fused_ext.gate_up_rows(q, x, w[:, :-16], ops, gu, m, s)
+        return q, s, m, gu
+    r0, r1 = _both(run)
+    _eq(r0, r1)
+    assert (r1[0] != 77).any() and bool((r1[3].view(-1)[M * N // 2:] == 7).all()) == bool(_lib.lib().omni_gemm_silu_rows_ok(M, N, K, mode))
+
+
 @pytest.mark.parametrize("tokens,hidden", [(16, 4096), (1, 4096), (300, 5120), (16, 14336)])
 def test_row_kernels_agree(tokens, hidden):
     import omniserve_backend.activation_ops as act

@@ -10,18 +10,25 @@ from omniserve_amd.backend import fused_ext
 M, N, K = 300, 512, 256
 
 
+class Names(list):
+    pass
+
+
 @pytest.fixture
 def launches(monkeypatch):
     """A library that takes every call and notes its name"""
-    names = []
+    names = Names()
 
     class Library:
+        answers = {"omni_gemm_workspace_bytes": 1}
+
         def __getattr__(self, name):
-            return lambda *a: names.append(name) or int(name.endswith("_ok"))
+            return lambda *a: names.append(name) or self.answers.get(name, 0)
 
     monkeypatch.setattr(_lib, "_lib", Library())
     monkeypatch.setattr(_lib, "require_cuda", lambda *t: None)
     monkeypatch.setattr(_lib, "current_stream", lambda: 0)
+    names.library = _lib._lib
     return names
 
 
@@ -52,4 +59,17 @@ def test_operands_of_the_product_are_checked(mode, launches):
         del launches[:]
         with pytest.raises(RuntimeError):
             fused_ext.gate_up_rows(**vars(c))
-        assert not [n for n in launches if not n.endswith("_ok")], what
+        assert not launches, what
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_the_library_is_not_asked_before_it_is_called(mode, launches, monkeypatch):
+    """Host time counts where prompts are short: a call for the unit and one for the quantiser; one that refuses and the two that stand in for it"""
+    kind = ("w4a8_per_chn", "w4a8_per_group", "w8a8")[mode]
+    fused_ext.gate_up_rows(**vars(_call(mode)))
+    assert launches == ["omni_%s_gemm_silu_rows" % kind, "omni_quant_fuse_sum" if mode == 0 else "omni_quant"]
+    monkeypatch.setitem(launches.library.answers, launches[0], -22)
+    monkeypatch.setattr(_lib, "workspace", lambda *a: torch.zeros(1, dtype=torch.uint8))
+    del launches[:]
+    fused_ext.gate_up_rows(**vars(_call(mode)))
+    assert [n for n in launches if n != "omni_gemm_workspace_bytes"] == ["omni_%s_gemm_silu_rows" % kind, "omni_%s_gemm" % kind, "omni_silu_mul_quant_fuse_sum"]
