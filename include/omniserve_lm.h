@@ -26,6 +26,7 @@ extern "C" {
 #define LM_ATTN_ROWS 128 /* query rows of one lm_attn_prefill tile */
 #define LM_CHOOSE_TOKENS 32 /* tokens of one lm_norm_choose at most */
 #define LM_MAX_TOP 16 /* experts of a token at most */
+#define LM_NO_EXPERTS_BITS 0x80000000u /* -0 */
 
 int lm_abi_version(void);
 int lm_elem_bytes(void);
@@ -36,7 +37,8 @@ int lm_elem_bytes(void);
  *   x += norm(y; post_w, post_b)           (post_w null: x += y;  y null: nothing added)
  *   h = norm(x; next_w, next_b)            (next_w null: h = x;  h null: none)
  * kind: LM_NORM_LAYER / LM_NORM_RMS over the first n columns.  Expert rows: (token, choice) pair t * top + k of y, weight
- * pair_w of the same index; shared != 0: row pairs0 + t is added with weight one.  rows: row r of h belongs to token rows[r]. */
+ * pair_w of the same index (up to 256 rows of more than 1024 elements, the first weight -0: the token has
+ * no expert rows, whatever is in their memory); shared != 0: row pairs0 + t is added with weight one.  rows: row r of h belongs to token rows[r]. */
 int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const void* embed, float embed_scale, const void* y, int64_t ldy,
                      const float* y_bias, const float* pair_w, int top, int pairs0, int shared, const float* post_w, const float* post_b, const float* next_w,
                      const float* next_b, void* h, int64_t ldh, const int* rows, int n_rows, int n, int kind, int store_x, float eps,
@@ -140,7 +142,7 @@ int lm_route(const float* z, int64_t ldz, const float* bias, int tokens, int exp
 
 /* Few tokens: lm_residual_norm (x += norm(y; post); h = norm(x; next), h of ldh = k elements), the router's product of h (router [experts, up to a multiple of 16][k], zero
  * rows behind the last expert) and the choice of lm_route in one launch -> wts [tokens][top], ids [tokens][top] (experts).  pos (or null): a token whose entry is
- * negative is none: weights 0, experts -1, x and h as they are.  lm_norm_choose_ok: for these sizes. */
+ * negative is none: weights -0, experts -1 (lm_gemm_chosen writes no rows of its pairs), x and h as they are.  lm_norm_choose_ok: for these sizes. */
 int lm_norm_choose_ok(int tokens, int k, int experts, int top);
 int lm_norm_choose(float* x, int64_t ldx, const void* y, int64_t ldy, const float* post_w, const float* post_b, const float* next_w, const float* next_b,
                    void* h, int64_t ldh, const int* pos, int tokens, int n, int kind, float eps, const void* router, const float* bias, int k, int experts, int top,

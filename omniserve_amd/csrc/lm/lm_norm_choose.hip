@@ -36,7 +36,7 @@ __global__ __launch_bounds__(TH) void norm_choose_kernel(ResidualArgs p, const i
   if (pos && pos[r] < 0) {      // an empty place of a captured step: it chooses no expert, whose weights would be read for it
     if (tid < top) {
       ids[(int64_t)r * top + tid] = -1;
-      wts[(int64_t)r * top + tid] = 0.f;
+      wts[(int64_t)r * top + tid] = __builtin_bit_cast(float, LM_NO_EXPERTS_BITS);
     }
     return;
   }

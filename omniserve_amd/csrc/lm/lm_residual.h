@@ -125,6 +125,8 @@ __device__ __forceinline__ void residual_row(const ResidualArgs& p, Row<TH>& row
             v[b][i] = c < p.n ? *(const quad_t*)(yr + c) : to_quad(zero4());
           }
         }
+        // (behind the requests, which bring the weights, too; TH > 256: the forms of few rows, for which lm_norm_choose is)
+        if (TH > 256 && k0 == 0 && __builtin_bit_cast(uint32_t, w[0]) == LM_NO_EXPERTS_BITS) break;
 #pragma unroll
         for (int b = 0; b < B; ++b)
 #pragma unroll

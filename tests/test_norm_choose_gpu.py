@@ -80,3 +80,34 @@ def test_empty_places_choose_nothing():
         assert torch.equal(a[full], b[full])
     x, h, wts, ids, act = out[1]
     assert torch.equal(x[~full], m["x"][~full]) and not h[~full].any() and not wts[~full].any() and (ids[~full] == -1).all() and (act[~full] == -3).all()
+
+
+@pytest.mark.parametrize("shared_ff", [0, 1024])
+def test_rows_that_nobody_wrote_stay_out_of_the_residual(shared_ff):
+    """An empty place's pairs have no rows: whatever bits their memory holds, the norm behind adds none of them"""
+    ops, T, k, experts, top = lm_ops(torch.bfloat16), 8, 2048, 64, 8
+    m = _inputs(T, k, k, experts, 640, 1024, 5, False)
+    pos = torch.tensor([4, -1, 0, 7, -1, -1, 9, 1], dtype=torch.int32, device=DEV)
+    full, out = pos >= 0, []
+    for p in (None, pos):
+        x, h = m["x"].clone(), torch.ones((T, k), dtype=torch.bfloat16, device=DEV)
+        wts, ids = ops.norm_choose(x, k, "layer", 1e-5, m["y"], m["post"], m["next"], h, m["router"], m["bias"], experts, top, p)
+        new = lambda *s: torch.full(s, float("nan"), dtype=torch.bfloat16, device=DEV)      # noqa: E731
+        act, act_s, y = new(T * top, 640), new(T, 1024), new(T * top + (T if shared_ff else 0), k)
+        up, down = ((h, m["shared_in"], act_s), (act_s, m["shared_out"], y[T * top:])) if shared_ff else (None, None)
+        ops.grouped(ids, T, h, m["w_in"], act, False, True, up)
+        ops.grouped(ids, T, act, m["w_out"], y, True, False, down)
+        if p is not None:
+            assert y[:T * top].view(T, top, k)[~full].isnan().all()
+        ops.residual_norm(x, k, "layer", 1e-5, y=y, experts=(wts, bool(shared_ff)), post=m["post"], next=m["next"], h=h)
+        out.append((x, h))
+    # weights of 0 behind others are weights: what their rows hold counts
+    wts = torch.tensor([[0.5, 0.0]] * T, device=DEV)
+    y = torch.ones((2 * T, k), dtype=torch.bfloat16, device=DEV)
+    y[1::4] = float("nan")
+    x = m["x"].clone()
+    ops.residual_norm(x, k, "rms", 1e-5, y=y, experts=(wts, False))
+    torch.cuda.synchronize()
+    assert x[::2].isnan().all() and torch.equal(x[1::2], m["x"][1::2] + 0.5)
+    for a, b in zip(*out):
+        assert torch.equal(a[full], b[full]) and b.isfinite().all()
