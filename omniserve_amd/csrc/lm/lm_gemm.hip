@@ -795,7 +795,7 @@ static void launch_stream_rows(const GemmArgs& a, int n, int has_b, int slices, 
 template <int EPI, int NW, bool SHORT, bool TURN = false, bool IDS = false>
 static void launch_stream_form(const GemmArgs& a, int n, int has_b, int slices, float* part, hipStream_t s) {
   if constexpr (!IDS && LM_ELEM == 0) {
-    if (!a.perm && !has_b && a.rows_a > 64) {      // (in one slice)
+    if (!a.perm && !has_b && a.rows_a > 64) {      // (in one slice; more rows than a caller's max_rows said, or gated units of more)
       for (int m = 0; m < a.rows_a; m += 64) {
         GemmArgs c = a;
         c.rows_a = min(64, a.rows_a - m);
@@ -832,6 +832,7 @@ static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices,
 template <int EPI>
 static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part, hipStream_t s) {
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
+  if (LM_ELEM == 0 && (a.perm || has_b) && pl.nw != 4) return LM_EINVAL;      // (no such kernels: launch_stream_form)
   if constexpr (EPI == LM_EPI_GLU) {
     if (LM_ELEM == 0 && pl.nw == 8) launch_stream_tiles<EPI, LM_ELEM == 0 ? 8 : 4>(a, n, has_b, pl.slices, part, s);
     else launch_stream_tiles<EPI, 4>(a, n, has_b, pl.slices, part, s);
