@@ -31,7 +31,11 @@
 // holds and not for what it has to fetch; ahead of them each unit touches its share of what they have in common.  Whole waves only.  (No gain where a stage
 // takes longer for its operands to be unpacked: the 4-bit group-wise tiles, 320 us of 28672 x 4096 and 2331 rows without, 322 with.)
 __device__ __forceinline__ void touch_lines32(const void* src, uint32_t lds_sink) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dword %0, off\n\ts_mov_b32 exec_hi, -1" ::"v"(src), "s"(lds_sink) : "memory", "m0");
+  uint32_t keep_m0;      // (M0 is the compiler's)
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 exec_hi, -1\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep_m0)
+               : "v"(src), "s"(lds_sink)
+               : "memory");
 }
 
 // a value the optimiser knows nothing about: what is computed from it is computed where it stands, not kept across a loop
