@@ -109,6 +109,8 @@ int omni_quant(void* out_i8, const void* in_f16, void* scale_f16, int tokens, in
  *   (fused_kernels.cu:97-142,255-271): as omni_quant plus sum = h(sum_i x_i) (f32 tree). */
 int omni_quant_fuse_sum(void* out_i8, const void* in_f16, void* sum_f16, void* scale_f16,
                         int tokens, int hidden, void* stream);
+/* Bytes (2 or 4) of an element of the row that its kernel keeps for the sum (omni_silu_mul_quant_fuse_sum's too): the same results. */
+int omni_quant_sum_copy_bytes(int tokens, int hidden);
 
 /* Replaces omniserve_backend.layernorm_ops.rms_norm (use_quant = false)
  *   (kernels/csrc/layernorm_kernels.cu:335-365,409-430). */

@@ -35,6 +35,7 @@ PROTOTYPES = {
     "omni_w4a8_per_group_gemm": (_i, [_vp] * 7 + [_i, _i, _i, _i64, _vp, _sz, _vp]),
     "omni_w8a8_gemm": (_i, [_vp] * 5 + [_i, _i, _i, _i64, _vp, _sz, _vp]),
     "omni_quant": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
+    "omni_quant_sum_copy_bytes": (_i, [_i, _i]),
     "omni_quant_fuse_sum": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),
     "omni_rms_norm": (_i, [_vp, _vp, _vp, _f, _i, _i, _vp]),
     "omni_rms_norm_general": (_i, [_vp, _vp, _vp, _vp, _f, _i, _i, _vp]),

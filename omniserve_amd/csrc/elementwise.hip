@@ -593,11 +593,15 @@ static inline int norm_block(int hidden, bool round32) {
   return b;
 }
 
-// Many rows of more than 8192, quantised with their sum: f32 copies would leave a CU two rows of 14336 (57 KB each).  (MI355X, f32 / fp16: quant_fuse_sum of 14336, 1501 rows
-// 18.3 / 16.1 us, 5000 46.1 / 36.3, 12001 113.3 / 92.5; of 16384, 1100 rows 16.2 / 14.9; of 8192, 1501 rows 10.1 / 10.6.)
+// Many rows, quantised with their sum, of which a CU's LDS holds two as f32 copies (54 KB each) and five to six as fp16.  Up to three f32 copies the eight waves of a CU more gain
+// less than the conversions cost.  (MI355X, f32 / fp16, us: quant_fuse_sum of 14336, 1501 rows 18.2 / 16.0, 5000 47.7 / 36.8, 12001 114.6 / 93.1; of 13824, 1501 rows 18.0 / 15.7;
+// of 16384, 1100 rows 16.6 / 15.5; but of 9216, 1024 rows 8.4 / 8.9, of 12288, 1100 rows 11.6 / 11.9, and silu's 12001 rows of 12288 130 / 143, of 11008 117 / 127.)
+static bool quant_half_ok(int tokens, int hidden) {
+  return tokens >= ROWS_MANY && hidden <= 256 * 8 * VT && 3 * (hidden * (int)sizeof(float) + 512) > 160 * 1024;
+}
 template <typename Src>
 static bool quant_half_copy(int8_t* out, const Src& src, half_t* sum, half_t* scale, int tokens, int hidden, int nv, hipStream_t st) {
-  if (tokens < ROWS_MANY || hidden <= 8192 || hidden > 256 * 8 * VT) return false;
+  if (!quant_half_ok(tokens, hidden)) return false;
   const PrefetchArgs pf = take_prefetch(tokens);      // (no rider beside many rows)
   hipLaunchKernelGGL((quant_v2_kernel<256, 8, true, Src, true>), dim3(tokens), dim3(256), (size_t)hidden * sizeof(half_t), st, out, src, sum, scale, hidden, nv, pf);
   return true;
@@ -626,6 +630,8 @@ extern "C" int omni_quant(void* out_i8, const void* in_f16, void* scale_f16, int
                      (half_t*)scale_f16, hidden);
   return omni_launch_status();
 }
+
+extern "C" int omni_quant_sum_copy_bytes(int tokens, int hidden) { return quant_half_ok(tokens, hidden) ? 2 : 4; }
 
 extern "C" int omni_quant_fuse_sum(void* out_i8, const void* in_f16, void* sum_f16, void* scale_f16,
                                    int tokens, int hidden, void* stream) {
