@@ -588,6 +588,8 @@ int omni_w4a8_per_group_norm_gemm_fused(void* codes_i8, void* residual_f16, cons
  * omni_act_product: omni_*_gemm_partial_f16 for one or two rows (W8A8: one) in K slices of its own, omni_act_product_slices of them (0: not its size;
  * csrc/act_product.hip); the slabs' sums are the same.  sum_f16 may be NULL.  act and weight 16-byte aligned. */
 int omni_norm_product_ok(int M, int N, int K, int mode, int silu, int k_before);
+/* Workgroups that omni_norm_product launches (0: not its size): int8 gate_up of some widths takes two on every compute unit. */
+int omni_norm_product_workgroups(int M, int N, int K, int mode, int silu);
 int omni_act_product_slices(int M, int N, int K, int mode);
 int omni_act_product(int mode, const void* act_f16, const void* amax_slots_u32, const void* weight, const void* zeros_i8, const void* scales_i8,
                      void* slab_i32, size_t slab_bytes, void* sum_f16, void* scale_f16, int M, int N, int K, void* stream);

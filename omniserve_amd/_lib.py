@@ -111,6 +111,7 @@ PROTOTYPES = {
     "omni_kv4_decode_attention_fine_grained": (_i, [_vp, _vp, _vp, _vp, _i64, _i64] + [_vp] * 6 + [_i] * 16 + [_vp, _i, _vp, _sz, _vp]),
     "omni_kv8_prefill_write_per_tensor": (_i, [_vp] * 8 + [_i] * 15 + [_vp, _i, _i, _vp]),
     "omni_kv8_decode_attention_per_tensor": (_i, [_vp, _vp, _vp, _vp, _i64, _i64] + [_vp] * 8 + [_i] * 16 + [_vp, _i, _vp, _sz, _vp]),
+    "omni_norm_product_workgroups": (_i, [_i] * 5),
     "omni_norm_product_ok": (_i, [_i] * 6),
     "omni_act_product_slices": (_i, [_i] * 4),
     "omni_act_product": (_i, [_i] + [_vp] * 6 + [_c.c_size_t, _vp, _vp, _i, _i, _i, _vp]),
