@@ -1009,10 +1009,11 @@ extern "C" void omni_prefill_set_xcd_split(int w) { g_prefill_xcd_split = (w == 
 //     62.4 / 58.7, 66 MB; 16 x 333 54.1 / 57.6, 87 MB; 16 x 1024 227 / 356; 64 x 1024 898 / 2044; 32 / 16 heads 64 x 512, 268 MB, 332 / 329, 64 x 1024 962 / 1234; 32 / 8 heads
 //     16 x 1024, 67 MB, 232 / 226; 64 / 8 heads 64 x 1024, 268 MB, 1863 / 1915);
 //   * streaming heads among them: four query heads a kv head, or up to 512 queries (32 / 32 heads: 1 x 1024 31.8 / 33.2, 16 x 1024 288 / 355, 16 x 512 202 / 146; 32 / 8 heads: 16 x 1000 256 / 226).
-// Not causal: 1024 28.2 / 32.6, 7 x 333 33.8 / 35.7, 16 x 1000 359 / 394.  (MI355X; 960 sizes of 1 - 64 heads: none that
-// the rule takes is slower by more than 2 %, but those of up to 64 tokens, 5 - 6 us, by 0.1 - 0.3.)
+// Not causal: 1024 28.2 / 32.6, 7 x 333 33.8 / 35.7, 16 x 1000 359 / 394.  One tile of keys, dense heads and no second 128-row workgroup on a CU: nothing to cover (32 / 8 heads of 48 tokens: 1
+// sequence 5.56 / 5.63, 8 6.01 / 6.16, 16 7.98 / 7.63).  (MI355X; 1300 sizes of 1 - 64 heads: none that the rule takes is slower by more than 2 %.)
 static bool small_tiles(int batch, int max_seqlen_q, int num_heads, int num_kv_heads, bool causal, bool self, bool streaming) {
-  if (!causal || !self || (max_seqlen_q > 1024 && (long long)batch * num_heads * ((max_seqlen_q + PQROWS - 1) / PQROWS) >= 512)) return false;
+  const long long wgs = (long long)batch * num_heads * ((max_seqlen_q + PQROWS - 1) / PQROWS);
+  if (!causal || !self || (max_seqlen_q > 1024 && wgs >= 512) || (!streaming && max_seqlen_q <= PKT && wgs <= 256)) return false;
   const int share = num_heads / num_kv_heads;
   if (streaming) return share >= 4 || max_seqlen_q <= 512;
   return (long long)batch * max_seqlen_q * num_kv_heads * (2 * PDH * (int)sizeof(half_t)) <= 60'000'000LL * min(share, 4);

@@ -217,10 +217,10 @@ def test_prefill_attention_of_64_rows_is_left_where_it_is_slower():
     rows = _lib.lib().omni_prefill_attention_rows
     #      batch, queries, heads, kv heads, causal, same offsets, streaming heads
     for a in ((1, 1501, 32, 8, 1, 1, 0), (7, 333, 32, 8, 1, 1, 0), (4, 900, 32, 32, 1, 1, 0), (16, 1024, 32, 8, 1, 1, 0), (1, 1024, 32, 8, 1, 1, 0), (16, 1000, 32, 8, 1, 1, 1),
-              (16, 512, 32, 32, 1, 1, 1)):
+              (16, 512, 32, 32, 1, 1, 1), (1, 65, 32, 8, 1, 1, 0), (9, 64, 32, 8, 1, 1, 0), (1, 64, 32, 8, 1, 1, 1)):
         assert rows(*a) == 64, a
     for a in ((1, 512, 32, 8, 1, 0, 0), (1, 1900, 32, 8, 1, 0, 0), (1, 64, 32, 8, 1, 0, 1), (1, 1024, 32, 8, 0, 1, 0), (7, 333, 32, 8, 0, 1, 0), (64, 1024, 32, 32, 1, 1, 0), (16, 333, 32, 32, 1, 1, 0),
-              (64, 1024, 32, 16, 1, 1, 0), (64, 1024, 64, 8, 1, 1, 0), (1, 1024, 32, 32, 1, 1, 1), (16, 1000, 32, 16, 1, 1, 1), (1, 8192, 32, 8, 1, 1, 0)):
+              (64, 1024, 32, 16, 1, 1, 0), (64, 1024, 64, 8, 1, 1, 0), (1, 1024, 32, 32, 1, 1, 1), (16, 1000, 32, 16, 1, 1, 1), (1, 8192, 32, 8, 1, 1, 0), (1, 64, 32, 8, 1, 1, 0), (8, 64, 32, 8, 1, 1, 0)):
         assert rows(*a) == 128, a
     assert rows(0, 1, 32, 8, 1, 1, 0) == 0 and rows(1, 0, 32, 8, 1, 1, 0) == 0 and rows(1, 1, 8, 32, 1, 1, 0) == 0
 
