@@ -593,11 +593,12 @@ static inline int norm_block(int hidden, bool round32) {
   return b;
 }
 
-// Many rows, quantised with their sum, of which a CU's LDS holds two as f32 copies (54 KB each) and five to six as fp16.  Up to three f32 copies the eight waves of a CU more gain
-// less than the conversions cost.  (MI355X, f32 / fp16, us: quant_fuse_sum of 14336, 1501 rows 18.2 / 16.0, 5000 47.7 / 36.8, 12001 114.6 / 93.1; of 13824, 1501 rows 18.0 / 15.7;
-// of 16384, 1100 rows 16.6 / 15.5; but of 9216, 1024 rows 8.4 / 8.9, of 12288, 1100 rows 11.6 / 11.9, and silu's 12001 rows of 12288 130 / 143, of 11008 117 / 127.)
+// Many rows, quantised with their sum, of which a CU's LDS (160 KB in pieces of 1280 bytes) holds two as f32 copies and five to six as fp16.  Up to three f32 copies the waves that are more
+// gain less than the conversions cost.  (MI355X, f32 / fp16, us, rows that no cache holds: quant_fuse_sum of 14336, 1501 rows 20.1 / 17.9, 5000 52.0 / 42.8, 12001 118.5 / 94.4; of 13504, 1501 rows
+// 19.8 / 17.4; of 16384, 1100 rows 18.3 / 17.2; but of 9216, 1024 rows 10.4 / 10.8, of 12288, 1100 rows 13.3 / 14.2, and silu's 12001 rows of 12288 131 / 144, of 11008 117 / 127.)
 static bool quant_half_ok(int tokens, int hidden) {
-  return tokens >= ROWS_MANY && hidden <= 256 * 8 * VT && 3 * (hidden * (int)sizeof(float) + 512) > 160 * 1024;
+  constexpr int PIECE = 1280, THREE = 160 * 1024 / 3 / PIECE * PIECE;      // of an LDS with three workgroups, a row and 384 bytes each
+  return tokens >= ROWS_MANY && hidden <= 256 * 8 * VT && hidden * (int)sizeof(float) + 384 > THREE;
 }
 template <typename Src>
 static bool quant_half_copy(int8_t* out, const Src& src, half_t* sum, half_t* scale, int tokens, int hidden, int nv, hipStream_t st) {

@@ -228,9 +228,9 @@ def test_prefill_attention_of_64_rows_is_left_where_it_is_slower():
 def test_quantiser_keeps_fp16_rows_only_where_three_f32_rows_do_not_fit():
     from omniserve_amd import _lib
     size = _lib.lib().omni_quant_sum_copy_bytes
-    for tokens, hidden in ((1024, 13536), (1024, 13824), (1501, 14336), (12001, 14336), (1024, 16384)):
+    for tokens, hidden in ((1024, 13376), (1024, 13824), (1501, 14336), (12001, 14336), (1024, 16384)):
         assert size(tokens, hidden) == 2, (tokens, hidden)
-    for tokens, hidden in ((1023, 14336), (1024, 13504), (1024, 9216), (12001, 11008), (12001, 12288), (1024, 16392), (16, 14336)):
+    for tokens, hidden in ((1023, 14336), (1024, 13344), (1024, 9216), (12001, 11008), (12001, 12288), (1024, 16392), (16, 14336)):
         assert size(tokens, hidden) == 4, (tokens, hidden)
 
 
