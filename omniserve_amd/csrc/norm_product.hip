@@ -209,11 +209,11 @@ __global__ __launch_bounds__(RP_THREADS, EPI ? 4 : 2) void norm_product_kernel(N
 // gate_up of int8 weights in two workgroups a compute unit: the first `wide` of them take four blocks of eight gate and eight up channels, the others three.  448
 // workgroups of four leave a quarter of the units with one, and a unit takes in its weights at a rate of its own.  (MI355X, 28672 x
 // 4096: four LServe steps of 4 layers 1607 -> 1585 us.  Packed weights hold two blocks in a byte and cannot be dealt in threes.  Where: more than three blocks for each of the 512, but not
-// so many that few units are left with one; rows that take long enough to come in.  Workgroups of four / this, us, one slab: 24704 x 4096 21.7 / 18.3, 28672 21.0 / 19.9,
-// 29696 22.2 / 22.7; 24704 x 3072 15.9 / 14.8, 28672 16.4 / 15.7, 29696 16.5 / 16.6; but 26624 x 2048 10.4 / 11.2, 30720 10.6 / 12.3 with two slabs.)
-static int even_wide(int N, int K) {      // the first that take four blocks, 0: all take four
+// so many that few units are left with one.  Workgroups of four / this, us, one slab, weights that no cache holds: 24704 x 4096 26.3 / 23.4, 28672 26.7 / 25.2, 29696 27.3 / 27.2; 24704 x 2048 12.5 / 11.6,
+// 28672 12.6 / 12.2, 29696 12.9 / 13.2, 30720 13.0 / 13.3.  Of weights in the last cache rows of 2048 take 10.4 / 11.2 at 26624; a step's come from memory.)
+static int even_wide(int N) {      // the first that take four blocks, 0: all take four
   const int wide = N / 16 - 3 * 512;
-  return K >= 3072 && wide > 0 && wide <= 256 ? wide : 0;
+  return wide > 0 && wide <= 256 ? wide : 0;
 }
 template <int C, int SK>
 __global__ __launch_bounds__(RP_THREADS, 4) void gate_up_even_kernel(NormProductArgs p, int wide) {
@@ -231,8 +231,8 @@ namespace {
 template <int MODE, int EPI, int BLOCKS, int C, int SK>
 void launch_rows(const NormProductArgs& p, hipStream_t st) {
   const dim3 grid(EPI ? p.N / 64 : p.N / 32), block(RP_THREADS);
-  if constexpr (MODE == MODE_W8 && EPI && C >= 3) {
-    if (const int wide = even_wide(p.N, 1024 * C)) {
+  if constexpr (MODE == MODE_W8 && EPI) {
+    if (const int wide = even_wide(p.N)) {
       hipLaunchKernelGGL((gate_up_even_kernel<C, SK>), dim3(512), block, 0, st, p, wide);
       return;
     }
@@ -282,7 +282,7 @@ static bool sizes_ok(int M, int N, int K, int mode, bool silu, int sk) {
 
 extern "C" int omni_norm_product_workgroups(int M, int N, int K, int mode, int silu) {
   if (!sizes_ok(M, N, K, mode, silu != 0, 1)) return 0;
-  if (mode == MODE_W8 && silu && even_wide(N, K)) return 512;
+  if (mode == MODE_W8 && silu && even_wide(N)) return 512;
   return silu ? N / 64 : N / 32;
 }
 
