@@ -24,6 +24,7 @@ ATTN_ROWS = 128          # query rows of one prefill tile
 PAGE = 64                # tokens per cache page
 ROWS_MAX = 64            # up to here a step's products stream the weights
 NARROW = 128             # products of so few channels do for any number of rows
+CHOOSE_TOKENS = 32       # tokens of one norm_choose at most
 
 
 class _Part(_c.Structure):
@@ -269,6 +270,8 @@ class LmOps:
 
     def chooses(self, tokens, router, experts, top, w_in, w_out):
         """Do norm_choose and products over its unsorted choices exist for these sizes?  w_in, w_out: all experts' matrices"""
+        if tokens > CHOOSE_TOKENS:      # (a prompt's host asks the library nothing)
+            return False
         ok = self._h.lm_gemm_chosen_ok
         return bool(self._h.lm_norm_choose_ok(tokens, router.shape[1], experts, top) and ok(*w_in.shape, tokens, top, EPI_GLU)
                     and ok(*w_out.shape, tokens, top, EPI_ELEM))

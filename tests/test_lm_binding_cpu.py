@@ -84,3 +84,12 @@ def test_few_rows_of_short_k_spread_over_the_chip():
             assert h.lm_gemm_rows_channels(1, 4096, k, 15, 0, 1, ctypes.byref(slices)) == 0 and slices.value == 1
             assert h.lm_gemm_rows_channels(32, 512, k, 17, 0, 0, None) == 64
             assert h.lm_gemm_rows_channels(32, 512, k, 16, 0, 0, None) == (0 if k <= 128 else 64)
+
+
+def test_prompts_do_not_ask_for_the_choice_in_one_launch(ops):
+    """Prompts are launched eagerly: what no number of tokens above 32 has is not asked for in every layer"""
+    real = lm.lm_ops(torch.bfloat16)
+    w = lambda *s: torch.empty(s, dtype=torch.bfloat16, device="meta")      # noqa: E731
+    sizes = (w(64, 2048), 64, 8, w(64, 1280, 2048), w(64, 2048, 640))
+    assert real.chooses(lm.CHOOSE_TOKENS, *sizes) and not real._h.lm_norm_choose_ok(lm.CHOOSE_TOKENS + 1, 2048, 64, 8)
+    assert ops.chooses(lm.CHOOSE_TOKENS + 1, *sizes) is False      # (its library has no such query)
