@@ -37,7 +37,7 @@ int lm_elem_bytes(void);
  *   x += norm(y; post_w, post_b)           (post_w null: x += y;  y null: nothing added)
  *   h = norm(x; next_w, next_b)            (next_w null: h = x;  h null: none)
  * kind: LM_NORM_LAYER / LM_NORM_RMS over the first n columns.  Expert rows: (token, choice) pair t * top + k of y, weight
- * pair_w of the same index (up to 256 rows of more than 1024 elements, the first weight -0: the token has
+ * pair_w of the same index (up to 256 rows of more than 1024 elements, all of a token's weights -0: it has
  * no expert rows, whatever is in their memory); shared != 0: row pairs0 + t is added with weight one.  rows: row r of h belongs to token rows[r]. */
 int lm_residual_norm(float* x, int64_t ldx, const int* tokens, const void* embed, float embed_scale, const void* y, int64_t ldy,
                      const float* y_bias, const float* pair_w, int top, int pairs0, int shared, const float* post_w, const float* post_b, const float* next_w,

@@ -114,10 +114,13 @@ __device__ __forceinline__ void residual_row(const ResidualArgs& p, Row<TH>& row
       for (int k0 = 0; k0 < p.top; k0 += B) {
         quad_t v[B][NV];
         float w[B];
+        uint32_t some = 0;
 #pragma unroll
         for (int b = 0; b < B; ++b) {
           const int k = min(k0 + b, p.top - 1);
-          w[b] = k0 + b < p.top ? p.pair_w[p0 + k] : 0.f;
+          const float pw = p.pair_w[p0 + k];
+          some |= __builtin_bit_cast(uint32_t, pw) ^ LM_NO_EXPERTS_BITS;
+          w[b] = k0 + b < p.top ? pw : 0.f;
           const elem_t* yr = p.y + (p0 + k) * p.ldy;
 #pragma unroll
           for (int i = 0; i < NV; ++i) {
@@ -126,7 +129,7 @@ __device__ __forceinline__ void residual_row(const ResidualArgs& p, Row<TH>& row
           }
         }
         // (behind the requests, which bring the weights, too; TH > 256: the forms of few rows, for which lm_norm_choose is)
-        if (TH > 256 && k0 == 0 && __builtin_bit_cast(uint32_t, w[0]) == LM_NO_EXPERTS_BITS) break;
+        if (TH > 256 && some == 0) continue;
 #pragma unroll
         for (int b = 0; b < B; ++b)
 #pragma unroll

@@ -111,3 +111,16 @@ def test_rows_that_nobody_wrote_stay_out_of_the_residual(shared_ff):
     assert x[::2].isnan().all() and torch.equal(x[1::2], m["x"][1::2] + 0.5)
     for a, b in zip(*out):
         assert torch.equal(a[full], b[full]) and b.isfinite().all()
+
+
+@pytest.mark.parametrize("top", [1, 2, 4, 5, 8, 9])
+@pytest.mark.parametrize("k", [1024, 2048, 4096])
+def test_weights_of_minus_zero_are_weights(top, k):
+    """... but where a token has no other: a row behind them counts, wherever it stands"""
+    ops = lm_ops(torch.bfloat16)
+    x0 = torch.randn((top, k), device=DEV)
+    y = torch.randn((top * top, k), device=DEV).bfloat16()
+    x, wts = x0.clone(), torch.full((top, top), -0.0, device=DEV)
+    wts.fill_diagonal_(0.5)
+    ops.residual_norm(x, k, "rms", 1e-5, y=y, experts=(wts, False))
+    assert torch.equal(x, x0 + 0.5 * y.view(top, top, k).diagonal().T.float())
