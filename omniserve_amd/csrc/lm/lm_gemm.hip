@@ -685,9 +685,10 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
 // 256 x 128 tiles instead of 256 x 256?  Whichever has the smaller time in rounds of the latter (one workgroup per CU) by a model of both: on
 // the XCD with the most tiles, pairs of half tiles share a CU and take 0.97 - 1.26 rounds, the more the longer their K and the fewer rows of them are empty
 // (1.05 with fewer than 48 rows in a tile, where they wait for weights), a rest that is alone on its CUs 0.8.  What it is about: grids that leave CUs idle, and last rounds.
-// (MI355X, bf16, 256 x 256 / 256 x 128, us: to f32, 65 rows of 32000 x 4096 102 / 77, 300 rows 116 / 134, 1000 rows of 8192 x 4096 105 / 81, 2000
-// rows 109 / 144.  Experts: 12 rows each of 32 x 4096 x 1792 151 / 133, 130 rows 161 / 178, 550 rows 352 / 393; 64 x 2048 x 640 70 / 56, 77 / 76, 164 / 161.
-// f32, 65 rows of 4096 x 1024 234 / 129.  Over 408 such sizes the choice costs 0.2 % on average and 6 % at most against the better one.)
+// (MI355X, bf16, 256 x 256 / 256 x 128, us: to f32, 65 rows of 32000 x 4096 103 / 84, 300 rows 110 / 133, 1000 rows of 8192 x 4096 79 / 72, 2000
+// rows 103 / 138.  Experts: 12 rows each of 32 x 4096 x 1792 145 / 131, 131 rows 158 / 176, 750 rows 415 / 498; 64 x 2048 x 640, 8, 87 and 500 rows, 62 / 49, 62 / 58, 152 / 156.
+// f32, 65 rows of 4096 x 1024 234 / 129.  Over 113 bf16 sizes the choice costs 0.4 % on average and 9 % at most, 700 tokens' two of 16 experts of 4096 x 4096, 209 us for 192, against the
+// better one.)
 // max_tiles > 0: rows sorted by group, of which there is a tile for every 256 and one per group.  Part b over rows_b rows: its tiles are the first that
 // workgroups of the whole form take, and where its K is longer those end later, by a third of it.
 static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {

@@ -170,8 +170,9 @@ static int launch_choose(const ResidualArgs& a, const int* pos, const elem_t* ro
 
 using namespace lm;
 
-// Sizes that it has: rows of 1028 - 4096 elements, which lm_residual_norm takes in one piece of a workgroup too, and up to 64 experts (512 KB and more would take
-// longer through every token's CU than in launches of their own); the router's product as lm_gemm_rows deals it to 16 channels and four K parts.
+// Sizes that it has: rows of 2048 - 4096 elements in multiples of 256 (a group of the ring: a stage of 64 of each of four K parts), of which every K slice has equally many
+// groups, and up to 64 experts (512 KB and more would take longer through every token's CU than in launches of their own); the router's product as lm_gemm_rows deals it to
+// 16 channels and four K parts.  Below 2048 of K that product adds its stages up in shorter chains, which are not built here; a row of 4096 is one piece of 1024 threads.
 // K slices of the router's product, or 0: there is no such launch
 static int choose_slices(int tokens, int k, int experts, int top) {
 #if LM_ELEM == 0

@@ -215,9 +215,11 @@ static float grid_time(const TileCost& c, int mb, int kw, long long workgroups, 
 }
 
 // w8a8_tiles_kernel: rounds of a tile per CU.  A stage takes 0.95 us where few CUs have a tile and 1.4 where all have one; 8 us a tile for its
-// ends, which is what short K loses here.  (MI355X, this kernel against the best tile height of the other: 12001 rows of 28672 x 4096 1193 us /
-// 1403, of 4096 x 14336 561 / 656, of 16640 x 1024 237 / 252, of 16384 x 256 116 / 111; 2331 rows of 6144 x 4096 51 / 62; 1501 rows of 4096 x
-// 14336, 96 tiles, 128 / 95.  From 512 of K: the kernel's first stage and its last two are not the same.)
+// ends, which is what short K loses here.  (MI355X, this kernel against the best tiles of the other: 12001 rows of 28672 x 4096 1057 us / 1406, of 4096 x 14336 499 / 681, of
+// 16640 x 1024 213 / 252, of 16384 x 512 152 / 158; 2331 rows of 6144 x 4096 52 / 66; 1501 rows of 4096 x 14336, 96 tiles, 149 / 112.  The stages' times are those of the kernel
+// before its lines were touched ahead; with them it is up to a tenth faster, and sizes at the line go to the slower one: over 142 sizes of 300 - 12001 rows the rule takes 1.4 % more
+// time than the better of the two, 8000 rows of 2048 x 2048 41 us for 32, 1501 of 16640 x 1024 43 for 35, 1024 of 8192 x 28672 255 for 229.  From 512 of K: the kernel's first
+// stage and its last two are not the same.)
 static float tiles_time(long long tiles, int stages) {
   const long long rounds = tiles / 256;
   const float rest = (float)(tiles - rounds * 256) / 256.f;

@@ -8,16 +8,20 @@
 //  * stages of 128 bytes of k (64 KB), two of them: the fragments of a half stage are read while the half before it multiplies, the stage
 //    after next is requested as soon as every wave has the current one in registers.
 //  * ahead of the requests a wave touches 32 lines of the stage behind them (touch_lines32): 64 rows of each operand a workgroup, the other rows by
-//    those of the 32 workgroups of an XCD that have the same rows or channels (four of a band, and four neighbouring columns).
+//    those of the 32 workgroups of an XCD that have the same rows (four neighbouring columns) or channels: as many as a band has row tiles.  Four of them touch all
+//    channels; bands of three, which 5, 6 and 9 row tiles make, leave a quarter to the requests.
 //  * a workgroup takes tile after tile of its XCD; the first two stages of the next one are on their way while it stores this one.
 //
 // Integer sums and the general kernel's epilogue: the same bits.
 //
 //  * the stores stream: 256 workgroups write 33 MB at the ends of their tiles, as much as all L2s hold, which keep the operands.
-// MI355X, 12001 rows, before -> here: 28672 x 4096 1403 -> 1193 us (2360 TOPS), 6144 x 4096 295 -> 249, 4096 x 14336 656 -> 561 (2510 TOPS).  With lines touched
-// ahead 1206 -> 1118 and 512 -> 487 (two stages ahead 1134 and 489; every workgroup its whole tile 1168 and 535; the operands of all tiles the first one's, so
-// that the L2 has everything, 983 and 445; no requests at all 934 and 398; no LDS reads 1182 and 498): what is left of the 5 POPS nominal is the clock under this load,
-// the ends of a tile, which 4096 of K show, and the L2.  Streaming stores 1038 -> 1013 and 470 -> 461, no zeroing of accumulators 1013 -> 996 and 460 -> 459.
+// MI355X, us, 12001 rows of 28672 x 4096 | 4096 x 14336, what is compared in turn on one box (boxes differ by a tenth, by the card's power):
+//  * w4a8_gemm_exact_kernel's best tiles -> here 1406 -> 1057 (2670 TOPS) | 681 -> 499 (2820 TOPS); of 6144 x 4096 304 -> 245;
+//  * without -> with lines touched ahead 1206 -> 1118 | 512 -> 487 (two stages ahead 1134 | 489; every workgroup its whole tile 1168 | 535; the operands of all tiles the first
+//    one's, so that the L2 has everything, 983 | 445; no requests at all 934 | 398; no LDS reads 1182 | 498); a line of the tile that is there anyway -> the lines ahead 1067 -> 1056 |
+//    516 -> 500, and of 28672 x 4096 in bands of four 1024 rows 113 -> 105, 2048 213 -> 200, in bands of three 1501 163 -> 157, 2100 217 -> 216; of 4096 x 14336 2100 166 -> 150, 2331 166 -> 131;
+//  * results stored -> streamed 1038 -> 1013 | 470 -> 461, accumulators zeroed -> not 1013 -> 996 | 460 -> 459.
+// What is left of the 5 POPS nominal is the clock under this load, the ends of a tile, which 4096 of K show, and the L2.
 #pragma once
 #include "lm/mfma_pinned.h"
 
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     n0 = tn * (SILU ? TILES_N / 2 : TILES_N);
     m0 = min((band * p.tile_linear + in - tn * rows) * TILES_M, p.M - TILES_M);
     {
-      const int l = lane_here();                            // (in % rows: rows is four in all bands but the last)
+      const int l = lane_here();                            // (in & 3: in % rows where rows is four)
       const uint8_t *aq = (const uint8_t*)p.A + (size_t)(m0 + 64 * (tn & 3)) * p.K, *wq = p.W + (size_t)(n0 + quarter(in & 3)) * p.K;
       soon = (l & 16 ? aq : wq) + ((uint32_t)(16 * wave + (l & 15)) * (uint32_t)p.K + 2 * TILES_K);
     }
