@@ -309,17 +309,17 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_stream_kernel(GemmArgs p, f
       constexpr int CHUNKS = decltype(chunks)::value;
       int e[CHUNKS];
 #pragma unroll
-      for (int i = 0; i < CHUNKS; ++i) e[i] = p.ids[min(64 * i + lane, p.pairs - 1)];
+      for (int i = 0; i < CHUNKS; ++i) e[i] = p.off[min(64 * i + lane, p.rows_a - 1)];
 #pragma unroll
       for (int i = 0; i < CHUNKS; ++i) {
-        const bool it = e[i] == g && 64 * i + lane < p.pairs;
+        const bool it = e[i] == g && 64 * i + lane < p.rows_a;
         const uint64_t mine = __builtin_amdgcn_ballot_w64(it);
         const int at = rows + __builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0));
         if (tid < 64 && it && at < LM_CHOOSE_TOKENS) own[at] = 64 * i + lane;
         rows += __builtin_popcountll(mine);
       }
     };
-    if (p.pairs <= 128) look(Int<2>{});
+    if (p.rows_a <= 128) look(Int<2>{});
     else look(Int<LM_CHOOSE_TOKENS * LM_MAX_TOP / 64>{});
     rows = min(rows, LM_CHOOSE_TOKENS);      // (a token chooses an expert once)
     perm = own;
@@ -432,7 +432,8 @@ __device__ __forceinline__ void mma3_dma16(f32x4& c0, f32x4& c1, f32x4& c2, frag
 // 938 down; 6733 tokens, 8 of 64 experts of 640, width 2048: 410 -> 382 up, 256 -> 259 down; 8192 x 7168 x 4096 to f32: 569 -> 469.
 // Ahead of the requests a wave touches 32 lines of the stage behind them (touch_lines32): 64 rows of each operand a workgroup, the others by the workgroups
 // of the band and of the neighbouring columns; where a band's tiles are several experts', their weights' other rows come untouched.  7999 tokens as
-// above: 1687 -> 1644 up, 947 -> 920 down.
+// above: 1687 -> 1644 up, 947 -> 920 down.  To f32, 30 sizes of 300 - 4100 rows: 0.94x on average, 2000 rows of 16384 x 4096 236 -> 198, but 1000 of 32000 x 4096 229 -> 239, 2000 of
+// 8192 x 4096 99 -> 102 (of the two steps, no zeroing alone 0.998x).
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a, int mt_b) {
   constexpr bool DIRECT = EPI == LM_EPI_F32 || sizeof(elem_t) == 4;      // accumulators straight to memory
@@ -733,7 +734,7 @@ static int fill(GemmArgs& a, const LmGemmPart* pa, const LmGemmPart* pb, int gro
   a.b = pb ? conv(pb) : Part{};
   if (check_part(a.a, epi, act) || (pb && check_part(a.b, epi, act))) return LM_EINVAL;
   a.groups = groups; a.perm = perm; a.off = off; a.rows_a = rows_a; a.rows_b = pb ? rows_b : 0; a.x_div = perm ? x_div : 1;
-  a.tiles = nullptr; a.scale = scale; a.act = act; a.ids = nullptr; a.pairs = 0; a.leave = 0;
+  a.tiles = nullptr; a.scale = scale; a.act = act;
   return LM_OK;
 }
 
@@ -831,7 +832,7 @@ static void launch_stream_tiles(const GemmArgs& a, int n, int has_b, int slices,
 }
 
 template <int EPI>
-static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part, hipStream_t s) {
+static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part, hipStream_t s, bool leave = false) {      // leave: the K slices' sums stay as they are
   const int n = has_b && a.b.n > a.a.n ? a.b.n : a.a.n;
   if (LM_ELEM == 0 && (a.perm || has_b) && pl.nw != 4) return LM_EINVAL;      // (no such kernels: launch_stream_form)
   if constexpr (EPI == LM_EPI_GLU) {
@@ -849,7 +850,7 @@ static int launch_stream(const GemmArgs& a, int has_b, RowsPlan pl, float* part,
       default: launch_stream_tiles<EPI, 5>(a, n, has_b, pl.slices, part, s); break;
     }
   }
-  if (pl.slices > 1 && !a.leave) {
+  if (pl.slices > 1 && !leave) {
     const int64_t q = (int64_t)a.rows_a * ((EPI == LM_EPI_GLU ? n / 2 : n) / 4);
     hipLaunchKernelGGL((gemm_reduce_kernel<EPI>), dim3((unsigned)((q + 255) / 256)), dim3(256), 0, s, a, part, pl.slices);
   }
@@ -940,7 +941,7 @@ extern "C" int lm_gemm_chosen(const LmGemmPart* pa, const LmGemmPart* pb, int gr
   uintptr_t at = (uintptr_t)a.a.w | (uintptr_t)a.a.x;
   if (has_b) at |= (uintptr_t)a.b.w | (uintptr_t)a.b.x;
   if (at & 15) return LM_EINVAL;
-  a.ids = ids; a.pairs = tokens * top; a.x_div = x_is_pairs ? 1 : top;
+  a.off = ids; a.rows_a = tokens * top; a.x_div = x_is_pairs ? 1 : top;
   hipStream_t s = (hipStream_t)stream;
   const bool is_short = a.a.k < CHAIN_K || (has_b && a.b.k < CHAIN_K);
   if (epi == LM_EPI_GLU) {
@@ -961,8 +962,7 @@ extern "C" int lm_gemm_sums(const LmGemmPart* pa, int rows, float* sums, void* s
   if (fill(a, pa, nullptr, 1, nullptr, nullptr, rows, 0, 1, 1.f, LM_EPI_ELEM, 0) || rows <= 0 || rows > 64 || !sums || ((uintptr_t)a.a.w | (uintptr_t)a.a.x) % 16) return LM_EINVAL;
   const RowsPlan pl = plan_rows(1, a.a.n, a.a.k, rows, LM_EPI_ELEM, false, true);
   if (pl.nw == 0 || pl.slices < 2) return LM_EINVAL;
-  a.leave = 1;
-  return launch_stream<LM_EPI_ELEM>(a, 0, pl, sums, (hipStream_t)stream);
+  return launch_stream<LM_EPI_ELEM>(a, 0, pl, sums, (hipStream_t)stream, true);
 }
 
 extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {
