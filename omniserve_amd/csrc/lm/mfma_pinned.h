@@ -49,6 +49,15 @@ __device__ __forceinline__ int lane_here() {
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
   return v;
 }
+// at the start of a block behind a branch: the accumulators come into it where they are (a value that is read in other blocks than its own is moved to vector registers in
+// front of the branch)
+template <typename V, int N, int M>
+__device__ __forceinline__ void accumulators_stay(V (&c)[N][M]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(c[i][j])::"memory");
+}
 template <typename V, int N, int M>
 __device__ __forceinline__ void accumulators_settle(V (&c)[N][M]) {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");

@@ -14,8 +14,11 @@
 // 336 / 396; 2331 rows of 28672 x 4096 318 / 342.  The matrix units are busy half of the time, as in the W8A8 tiles; unpacking in 8.5 operations a word took
 // 2 - 3 % more, letting the stores of a tile fly into the next one nothing less.
 //
+// SHARE: K of the last round's tiles shared out (tile_share.h).
+//
 // Integer sums and the general kernel's epilogue: the same bits.
 #pragma once
+#include "tile_share.h"
 
 namespace omni {
 
@@ -32,16 +35,18 @@ constexpr int GT_ACT = TILES_M * TILES_K, GT_W = TILES_N * TILES_K / 2, GT_PAR =
 
 // SILU: out = silu(gate) up of a [gate | up] weight, [M][N / 2]: of a wave's 64 channels the first 32 are gate channels, the others the up channels of the same place.  (2331 rows of
 // 28672 x 4096: the product takes 307 us either way, the quantiser behind it 31 -> 18.)
-template <bool SILU>
-__global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
+template <bool SILU, bool SHARE>
+__global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, TileShare share) {
   constexpr int PITCH = 64 * 2 + 16;                        // a row of the write-back buffers: a wave's 64 channels
   constexpr int LDS_OUT = GT_BUFS * GT_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SC + 2 * 1024];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SC + 2 * 1024 + (SHARE ? 16 : 0)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // (tile order: w8a8_tiles_kernel's)
   const int tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x & 7;
   const int own = (tiles >> 3) + (xcd < (tiles & 7)), first = xcd * (tiles >> 3) + min(xcd, tiles & 7);
   int at = blockIdx.x >> 3;
+  const int all_stages = p.K / TILES_K;
+  TileParts parts(own, all_stages);                         // (SHARE)
 
   // a wave's part of a stage: 64 rows of the activations, 8 a piece (lane: row lane / 8, slot lane % 8), and its two tile rows of weights, 2 KB each
   uint32_t src[8], wsrc[4];
@@ -82,25 +87,35 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
     dma_params(buf);
     advance();
   };
-  const int ns = p.K / TILES_K;
-  int m0 = 0, n0 = 0;
+  int m0 = 0, n0 = 0, ns = all_stages;                      // ns: stages of the tile opened last
   uint16_t sw_next = 0, sa_next = 0;                        // the thread's channel's and row's scales of the tile opened last
   // (the last row tile starts at M - 256: the rows that it shares with the one before are computed twice, to the same bits)
   auto open_tile = [&]() __attribute__((always_inline)) {
-    if (at >= own) return false;
-    const int id = first + at, band = id / (p.tile_linear * p.tiles_n), in = id - band * p.tile_linear * p.tiles_n;
+    int k0 = 0;
+    if constexpr (SHARE) {
+      if (!parts.next(at)) return false;
+      k0 = parts.k0;
+      ns = parts.stages;
+    } else {
+      if (at >= own) return false;
+    }
+    const int id = first + (SHARE ? parts.tile : at), band = id / (p.tile_linear * p.tiles_n), in = id - band * p.tile_linear * p.tiles_n;
     const int rows = min(p.tile_linear, p.tiles_m - band * p.tile_linear), tn = in / rows;
     at += (int)gridDim.x >> 3;
     n0 = tn * (SILU ? TILES_N / 2 : TILES_N);
     m0 = min((band * p.tile_linear + in - tn * rows) * TILES_M, p.M - TILES_M);
-    wbase = p.W + (size_t)n0 * (p.K / 2);
-    abase = (const uint8_t*)p.A + (size_t)m0 * p.K;
+    wbase = p.W + (size_t)n0 * (p.K / 2) + k0 * (4 * 512);
+    abase = (const uint8_t*)p.A + (size_t)m0 * p.K + k0 * TILES_K;
     const int tid = 64 * wave + lane_here();
     // (lane l of 64 channels: the first of the wave's and, SILU, the other half's)
     auto channel = [&](int l) __attribute__((always_inline)) { return SILU ? n0 + 32 * wave + (l & 31) + (l >> 5) * (p.N >> 1) : n0 + 64 * wave + l; };
-    par = ((tid & 16) ? p.s2z : p.s2s) + channel(4 * (tid & 15));
+    par = ((tid & 16) ? p.s2z : p.s2s) + (size_t)k0 * p.N + channel(4 * (tid & 15));
     sw_next = ((const uint16_t*)p.wscales)[channel(lane_here())];
     sa_next = ((const uint16_t*)p.ascales)[m0 + tid];
+    if constexpr (SHARE) {
+      wbase = wave_uniform(wbase);
+      abase = wave_uniform(abase);
+    }
 #pragma unroll
     for (int i = 0; i < GT_BUFS; ++i) stage(i * GT_STAGE);
     return true;
@@ -287,6 +302,10 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
     // a tile takes the same time)
     asm volatile("s_waitcnt vmcnt(13)" ::: "memory");
     __syncthreads();
+    if constexpr (SHARE) {
+      wbase = wave_uniform(wbase);
+      abase = wave_uniform(abase);
+    }
     const int fl = lane_here();
 #pragma unroll
     for (int u = 0; u < 2; ++u) off[u] = (fl & 15) * TILES_K + (((4 * u + (fl >> 4)) ^ tiles_swizzle(fl & 15)) << 4);
@@ -337,30 +356,58 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
     const int chan = (i0 >> 3) * 32 + (i0 & 7);             // of block 0
     const uint8_t* scales = lds + LDS_SC + 1024 * parity;
     half_t* const out = p.out + (size_t)m0 * p.out_stride + n0 + (SILU ? 32 : 64) * wave;
-    uint2 packed[16][4];                                    // [row block][channel block]
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint2 w = *(const uint2*)(scales + 2 * (64 * wave + chan + 8 * i));
-      const uint32_t wv[2] = {w.x, w.y};
-      float sw[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float sa = (float)*(const half_t*)(scales + 512 + 2 * (16 * j + e15));
-        uint32_t h[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          v2f r = (v2f){(float)acc[i][j][2 * e] * (sw[2 * e] * sa), (float)acc[i][j][2 * e + 1] * (sw[2 * e + 1] * sa)};
-          asm volatile("" : "+v"(r));
-          h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
-          asm volatile("" : "+v"(h[e]));
+    bool opened = false;
+    const TileParts mine = parts;
+    if constexpr (SHARE) {
+      if (mine.shared()) {
+        const bool last = mine.finishes(share, lds + LDS_SC + 2 * 1024, acc, [&] {
+          opened = true;
+          open = open_tile();
+        });
+        if (!last) {
+          parity ^= 1;
+          if (open) park(parity);
+          continue;
         }
-        packed[j][i] = make_uint2(h[0], h[1]);
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
-    open = open_tile();
+    uint2 packed[16][4];                                    // [row block][channel block]
+    auto pack = [&](auto add) __attribute__((always_inline)) {
+      constexpr bool ADD = decltype(add)::value;
+      if constexpr (SHARE) accumulators_stay(acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v4i x[8];
+        const uint2 w = *(const uint2*)(scales + 2 * (64 * wave + chan + 8 * i));
+        const uint32_t wv[2] = {w.x, w.y};
+        float sw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          if constexpr (ADD) if (j % 8 == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            mine.others(share, 16 * i + j, x);
+            accumulators_stay(acc);
+          }
+          const float sa = (float)*(const half_t*)(scales + 512 + 2 * (16 * j + e15));
+          uint32_t h[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int c0 = acc[i][j][2 * e] + (ADD ? x[j & 7][2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? x[j & 7][2 * e + 1] : 0);
+            v2f r = (v2f){(float)c0 * (sw[2 * e] * sa), (float)c1 * (sw[2 * e + 1] * sa)};
+            asm volatile("" : "+v"(r));
+            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
+            asm volatile("" : "+v"(h[e]));
+          }
+          packed[j][i] = make_uint2(h[0], h[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (SHARE && mine.shared()) pack(BoolTag<SHARE>{});
+    else pack(BoolTag<false>{});
+    if (!opened) open = open_tile();
     // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's 64 channels at a time
     uint8_t* rows = lds + LDS_OUT + wave * 16 * PITCH;
     if constexpr (SILU) {      // two row blocks at a time; lanes l and l ^ 16 have a block's eight channels
@@ -400,12 +447,13 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p) {
 
 // a workgroup per CU
 template <bool SILU>
-static void launch_group_tiles_as(GemmArgs b, hipStream_t st) {
+static void launch_group_tiles_as(GemmArgs b, const TileShare& share, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;
   b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
   const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
   b.tile_linear = (b.tiles_m + bands - 1) / bands;
-  hipLaunchKernelGGL(w4a8_group_tiles_kernel<SILU>, dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+  if (share.sums) hipLaunchKernelGGL((w4a8_group_tiles_kernel<SILU, true>), dim3(256), dim3(256), 0, st, b, share);
+  else hipLaunchKernelGGL((w4a8_group_tiles_kernel<SILU, false>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b, share);
 }
 
 }  // namespace omni

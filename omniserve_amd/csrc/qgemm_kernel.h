@@ -21,6 +21,7 @@
 #pragma once
 #include "common.h"
 #include "row_reduce.h"
+#include "tile_share.h"
 
 namespace omni {
 
@@ -1232,13 +1233,14 @@ extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool w8 = false);
 
 // w4a8_gemm_exact_kernel's tile height (16-row blocks; 16: w8a8_tiles_kernel), K parts inside a workgroup, K slices over the grid (1: no
-// slabs); group_tiles: w4a8_group_tiles_kernel instead of all that
+// slabs); group_tiles: w4a8_group_tiles_kernel instead of all that; share: either of the 256 x 256 kernels, K of the last round's tiles shared out (tile_share.h)
 struct PrefillPlan {
   int mb, kw, sk;
-  bool group_tiles = false;
+  bool group_tiles = false, share = false;
 };
 // sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs (omni_gemm_set_plan_override's K splits do, too)
-PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only);
+// scratch: there is memory for shared tiles
+PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, bool scratch = false);
 
 // shapes the straight-line kernel takes: whole channel tiles and K chunks (also of a K slice: a.kslice); it stores 16 B
 // per lane, so rows of an fp16 output must start 16-B aligned, and so must both operands
@@ -1272,36 +1274,39 @@ static void launch_exact_rows(const GemmArgs& a, int mb, int sk, hipStream_t st)
   }
 }
 
-// a workgroup per CU
+// a workgroup per CU; share.sums: with K of the last round's tiles shared out
 template <int MODE, bool SILU = false>
-static void launch_tiles(GemmArgs b, hipStream_t st) {
+static void launch_tiles(GemmArgs b, const TileShare& share, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;
   b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
   const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
   b.tile_linear = (b.tiles_m + bands - 1) / bands;
-  hipLaunchKernelGGL((w8a8_tiles_kernel<MODE, SILU>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b);
+  if (share.sums) hipLaunchKernelGGL((w8a8_tiles_kernel<MODE, SILU, true>), dim3(8 * SHARE_PER), dim3(256), 0, st, b, share);
+  else hipLaunchKernelGGL((w8a8_tiles_kernel<MODE, SILU>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b, share);
 }
 
 // qgemm_grp.hip
-void launch_group_tiles(const GemmArgs& a, hipStream_t st);
+void launch_group_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st);
+// qgemm_plan.hip: the scratch that omni_gemm_arm_share left for this thread's next product
+TileShare take_armed_share();
 // qgemm_plan.hip: does omni_*_gemm_silu_rows take these sizes?  pp: its plan
-bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp);
+bool silu_rows_plan(int M, int N, int K, int mode, bool scratch, GemmPlan* pl, PrefillPlan* pp);
 
 // prefill regime (M > 128): chunked LDS staging, weights through L2
 template <int MODE>
-static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
+static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, const TileShare& share, hipStream_t st) {
   if (exact_shape(a, false)) {
-    const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false);
+    const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false, share.sums != nullptr);
     if constexpr (MODE == MODE_W8) {
       if (pp.mb == 16) {
-        launch_tiles<MODE>(a, st);
+        launch_tiles<MODE>(a, pp.share ? share : TileShare{}, st);
         return;
       }
     }
     if constexpr (MODE == MODE_GRP) {
       // (a lane's parameters are four bytes)
       if (pp.group_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
-        launch_group_tiles(a, st);
+        launch_group_tiles(a, pp.share ? share : TileShare{}, st);
         return;
       }
     }
@@ -1430,6 +1435,7 @@ static void launch_gemv(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
 
 template <int MODE>
 static int launch_gemm(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
+  const TileShare share = take_armed_share();
   if (a.M < 1 || a.N % 64 != 0 || a.K % 64 != 0 || a.K < 64) return OMNI_EINVAL;
   if (MODE == MODE_GRP && a.K % 128 != 0) return OMNI_EINVAL;
   GemmPlan pl = plan_gemm(a.M, a.N, a.K, MODE == MODE_GRP ? 128 : 64, false, MODE == MODE_W8);
@@ -1450,7 +1456,7 @@ static int launch_gemm(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
     return omni_launch_status();
   }
   if (a.M > 128) {
-    launch_prefill<MODE>(a, pl, st);
+    launch_prefill<MODE>(a, pl, share, st);
   } else {
     switch (pl.mb) {
       case 1: launch_gemv<MODE, 1>(a, pl, st); break;

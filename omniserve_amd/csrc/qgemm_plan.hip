@@ -1,5 +1,7 @@
 // Host-side tiling / split-K planning for the W4A8 / W8A8 GEMMs (shared by the three GEMM TUs).
 #include "qgemm_kernel.h"
+#include <atomic>
+#include <chrono>
 
 namespace omni {
 
@@ -31,6 +33,13 @@ PrefetchArgs take_armed_prefetch() {
   PrefetchArgs pf = g_armed_prefetch;
   g_armed_prefetch = PrefetchArgs{};
   return pf;
+}
+
+static thread_local TileShare g_armed_share = {};
+TileShare take_armed_share() {
+  const TileShare s = g_armed_share;
+  g_armed_share = TileShare{};
+  return s;
 }
 
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred, bool w8) {
@@ -236,7 +245,18 @@ static float group_tiles_time(long long tiles, int stages) {
   return (float)rounds * (8.f + 1.65f * (float)stages) + (rest > 0.f ? 8.f + (1.3f + 0.35f * rest) * (float)stages : 0.f);
 }
 
-PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) {
+// The same with K of the last round's tiles shared out (the rounds in front of it as above): every CU at work for the stages of a head, and 17 us for a second part's sums and two more ends, 4 for each
+// part more.  1e30f: it has nothing
+// to share.  (MI355X, whole tiles / shared, us: per-group 2331 rows of 4096 x 14336, 20 tiles of an XCD, 181 / 152; 3000, 24 tiles, 181 / 164; 6000, 32 + 16, 342 / 300; 2331 of 28672 x 4096, 4 x 32 + 12, 284 / 278;
+// 1500, 2 x 32 + 20, 167 / 172, 3000 of 4096 x 4096, 24 tiles, 54 / 61.)
+static float shared_time(long long tiles, int stages, float stage) {
+  const int left = (int)((tiles + 7) / 8 % SHARE_PER);
+  const ShareSplit sp = share_split(left, stages);
+  if (left == 0 || sp.head == stages) return 1e30f;
+  return (float)((tiles + 7) / 8 / SHARE_PER) * (8.f + stage * (float)stages) + 17.f + 4.f * (float)(sp.used - left - 1) / (float)left + stage * (float)sp.head;
+}
+
+PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, bool scratch) {
   const TileCost& c = kTileCost[mode];
   PrefillPlan best{8, 1, slab_only ? sk : 1};
   // rows far apart are slower to read, but not where K slices read them at several places (512 rows of 8192 x 28672 per-channel: 1.08 us per chunk of
@@ -263,21 +283,29 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only) 
     if (K % (2 * KCHUNK) == 0) offer(mb, 2, 1);
     if (sk > 1) offer(mb, 1, sk);
   }
-  if (mode == MODE_W8 && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K && tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < time)
-    best = PrefillPlan{16, 1, 1};
-  if (mode == MODE_GRP && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K)
-    best.group_tiles = g_override_waves == 16 || group_tiles_time((long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N), K / TILES_K) < 0.98f * time;
+  if (mode != MODE_CHN && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K) {
+    const long long tiles = (long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N);
+    const int stages = K / TILES_K;
+    const float whole = mode == MODE_W8 ? tiles_time(tiles, stages) : group_tiles_time(tiles, stages);
+    const bool take = mode == MODE_W8 ? whole < time : g_override_waves == 16 || whole < 0.98f * time;
+    const bool share = scratch && shared_time(tiles, stages, mode == MODE_W8 ? 1.4f : 1.65f) < (take ? whole : 0.93f * time) - 4.f;      // (the models' errors)
+    if ((take || share) && mode == MODE_W8) best = PrefillPlan{16, 1, 1};
+    best.group_tiles = (take || share) && mode == MODE_GRP;
+    best.share = share;
+  }
   return best;
 }
 
 // One pass over K by the kernels that have the unit: the tiles, and w4a8_gemm_exact_kernel of one K part.
-bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp) {
+bool silu_rows_plan(int M, int N, int K, int mode, bool scratch, GemmPlan* pl, PrefillPlan* pp) {
   if (M <= 128 || N < 256 || K < 64 || mode < MODE_CHN || mode > MODE_W8) return false;
   if (N % 256 != 0 || K % KCHUNK != 0) return false;
   *pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
   if (pl->midm || !exact_sizes(M, N, K, pl->kslice)) return false;
   *pp = plan_prefill(M, N, K, mode, pl->sk, false);
-  return mode == MODE_W8 ? pp->mb == 16 : pp->group_tiles || (pp->sk == 1 && pp->kw == 1);
+  if (mode == MODE_W8 ? pp->mb != 16 : !pp->group_tiles && (pp->sk != 1 || pp->kw != 1)) return false;
+  if (scratch) *pp = plan_prefill(M, N, K, mode, pl->sk, false, true);
+  return true;
 }
 
 }  // namespace omni
@@ -285,7 +313,7 @@ bool silu_rows_plan(int M, int N, int K, int mode, GemmPlan* pl, PrefillPlan* pp
 extern "C" int omni_gemm_silu_rows_ok(int M, int N, int K, int mode) {
   omni::GemmPlan pl;
   omni::PrefillPlan pp;
-  return omni::silu_rows_plan(M, N, K, mode, &pl, &pp) ? 1 : 0;
+  return omni::silu_rows_plan(M, N, K, mode, false, &pl, &pp) ? 1 : 0;
 }
 
 extern "C" void omni_gemm_set_plan_override(int waves, int sk) {
@@ -322,6 +350,24 @@ extern "C" int omni_gemm_prefill_group_tiles(int M, int N, int K) {
   if (M <= 128 || N < 64 || N % 64 || K < 64 || K % 64) return 0;
   const GemmPlan pl = plan_gemm(M, N, K, 128, false, false);
   return exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, MODE_GRP, pl.sk, false).group_tiles;
+}
+
+extern "C" size_t omni_gemm_share_bytes(int M, int N, int K, int mode) {
+  using namespace omni;
+  if (M < TILES_M || N < TILES_N || K < 4 * TILES_K || (mode != MODE_GRP && mode != MODE_W8)) return 0;
+  const GemmPlan pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
+  return !pl.midm && exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, mode, pl.sk, false, true).share ? SHARE_BYTES : 0;
+}
+
+extern "C" int omni_gemm_arm_share(void* scratch, size_t bytes) {
+  using namespace omni;
+  g_armed_share = TileShare{};
+  if (!scratch) return OMNI_OK;
+  if (bytes < SHARE_BYTES || (reinterpret_cast<uintptr_t>(scratch) & 15) != 0) return OMNI_EINVAL;
+  static std::atomic<unsigned long long> launches{(unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count()};
+  g_armed_share = TileShare{static_cast<v4i*>(scratch), reinterpret_cast<unsigned long long*>(static_cast<char*>(scratch) + SHARE_SUMS),
+                            launches.fetch_add(1, std::memory_order_relaxed) << 8};
+  return OMNI_OK;
 }
 
 // Would the row-kernel-free decode forms (omni_*_gemm_silu for gate_up, omni_*_gemm_partial_f16 for o / down) accept a layer

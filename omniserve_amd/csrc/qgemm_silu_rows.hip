@@ -7,18 +7,20 @@ using namespace omni;
 // out = silu(gate) up fp16 [M, N/2], bit for bit what the product and silu_and_mul leave, in the products' own tiles.
 template <int MODE>
 static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
+  TileShare share = take_armed_share();
   GemmPlan pl;
   PrefillPlan pp;
-  if (!silu_rows_plan(a.M, a.N, a.K, MODE, &pl, &pp)) return OMNI_EINVAL;
+  if (!silu_rows_plan(a.M, a.N, a.K, MODE, share.sums != nullptr, &pl, &pp)) return OMNI_EINVAL;
   a.kslice = pl.kslice;
+  if (!pp.share) share = TileShare{};
   if (!exact_shape(a, false)) return OMNI_EINVAL;
   if constexpr (MODE == MODE_W8) {
-    launch_tiles<MODE, true>(a, st);
+    launch_tiles<MODE, true>(a, share, st);
   } else {
     const bool tiles = pp.group_tiles;
     if (tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) != 0) return OMNI_EINVAL;
     if constexpr (MODE == MODE_GRP) {
-      if (tiles) launch_group_tiles_as<true>(a, st);
+      if (tiles) launch_group_tiles_as<true>(a, share, st);
     }
     if (!tiles) launch_exact_rows<MODE, 1, false, true>(a, pp.mb, 1, st);
   }

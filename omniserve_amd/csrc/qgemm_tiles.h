@@ -47,19 +47,21 @@ __device__ __forceinline__ void tiles_dma16(uint32_t src, const void* base, uint
 // SILU: out = silu(gate) up of a [gate | up] weight, [M][N / 2]: rows 0 - 63 and 128 - 191 of a tile are 128 gate channels, the others the up channels of the same place, so that
 // a wave has both.  Half the stores pay for the exponentials; what it saves is the other half's way
 // through memory: 12001 rows of 28672 x 4096, the quantiser behind the product 156 -> 90 us, both 1.03x of a whole prompt.
-template <int MODE, bool SILU = false>
-__global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
+// SHARE: tile_share.h.
+template <int MODE, bool SILU = false, bool SHARE = false>
+__global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShare share) {
   static_assert(MODE == MODE_W8, "rows of int8 weights");
   constexpr int PITCH = 128 * 2 + 16;                       // a row of the write-back buffers: a wave's 128 channels
   // one object: the stages, four write-back buffers of 16 rows, the scales of two tiles
   constexpr int LDS_OUT = 2 * TILES_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH, LDS_SINK = LDS_SC + 2 * 1024;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SINK + 128];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SINK + 128 + (SHARE ? 16 : 0)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = 128 * (wave & 1), wm = 128 * (wave >> 1);
   // XCD x takes the x-th contiguous eighth of the tiles, counted down the columns of bands of row tiles (as w4a8_gemm_exact_kernel)
   const int tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x & 7;
   const int own = (tiles >> 3) + (xcd < (tiles & 7)), first = xcd * (tiles >> 3) + min(xcd, tiles & 7);
   int at = blockIdx.x >> 3;
+  TileParts parts(own, p.K / TILES_K);                      // (SHARE)
 
   // a wave's part of a stage: 64 rows of the weights and 64 of the activations, 8 a piece (lane: row lane / 8, slot lane % 8)
   uint32_t src[8];
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     wbase += TILES_K;
     abase += TILES_K;
   };
-  const int ns = p.K / TILES_K;                             // even, four or more
+  int ns = p.K / TILES_K;                                   // stages of the part opened last: four or more
   // first channel of a quarter of the tile's rows, from the tile's
   auto quarter = [&](int q) { return SILU ? 64 * (q >> 1) + (q & 1) * (p.N >> 1) : 64 * q; };
   const uint8_t* soon = nullptr;                            // the lane's line of the stage behind the one requested last: of the weights (lanes 0 - 15) or the activations
@@ -90,8 +92,15 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
   // requests the next tile's first two stages; false: there is none.  The last row tile starts at M - 256: the rows that it shares with the
   // one before are computed twice, to the same bits.
   auto open_tile = [&]() {
-    if (at >= own) return false;
-    const int id = first + at, band = id / (p.tile_linear * p.tiles_n), in = id - band * p.tile_linear * p.tiles_n;
+    int k0 = 0;
+    if constexpr (SHARE) {
+      if (!parts.next(at)) return false;
+      k0 = parts.k0 * TILES_K;
+      ns = parts.stages;
+    } else {
+      if (at >= own) return false;
+    }
+    const int id = first + (SHARE ? parts.tile : at), band = id / (p.tile_linear * p.tiles_n), in = id - band * p.tile_linear * p.tiles_n;
     const int rows = min(p.tile_linear, p.tiles_m - band * p.tile_linear), tn = in / rows;
     at += (int)gridDim.x >> 3;
     n0 = tn * (SILU ? TILES_N / 2 : TILES_N);
@@ -99,10 +108,14 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     {
       const int l = lane_here();                            // (in & 3: in % rows where rows is four)
       const uint8_t *aq = (const uint8_t*)p.A + (size_t)(m0 + 64 * (tn & 3)) * p.K, *wq = p.W + (size_t)(n0 + quarter(in & 3)) * p.K;
-      soon = (l & 16 ? aq : wq) + ((uint32_t)(16 * wave + (l & 15)) * (uint32_t)p.K + 2 * TILES_K);
+      soon = (l & 16 ? aq : wq) + ((uint32_t)(16 * wave + (l & 15)) * (uint32_t)p.K + k0 + 2 * TILES_K);
     }
-    wbase = p.W + (int64_t)__builtin_amdgcn_readfirstlane(n0 + (quarter(wave) - 64 * wave)) * p.K;      // (its rows' offsets hold 64 * wave)
-    abase = (const uint8_t*)p.A + (size_t)m0 * p.K;
+    wbase = p.W + (int64_t)__builtin_amdgcn_readfirstlane(n0 + (quarter(wave) - 64 * wave)) * p.K + k0;      // (its rows' offsets hold 64 * wave)
+    abase = (const uint8_t*)p.A + (size_t)m0 * p.K + k0;
+    if constexpr (SHARE) {
+      wbase = wave_uniform(wbase);
+      abase = wave_uniform(abase);
+    }
     const int tid = 64 * wave + lane_here();
     sw_next = ((const uint16_t*)p.wscales)[n0 + quarter(wave) + lane_here()];
     sa_next = ((const uint16_t*)p.ascales)[m0 + tid];
@@ -191,6 +204,10 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     // stage 0 is there: of what was requested last -- stage 1 and lines, or stores of the tile before -- 17 may still fly
     asm volatile("s_waitcnt vmcnt(17)" ::: "memory");
     __syncthreads();
+    if constexpr (SHARE) {
+      wbase = wave_uniform(wbase);
+      abase = wave_uniform(abase);
+    }
     const int fl = lane_here();
 #pragma unroll
     for (int u = 0; u < 2; ++u) off[u] = (fl & 15) * TILES_K + (((4 * u + (fl >> 4)) ^ tiles_swizzle(fl & 15)) << 4);
@@ -214,34 +231,61 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p) {
     const int el = lane_here(), e15 = el & 15, e4 = el >> 4;
     const uint8_t* sc = lds + LDS_SC + 1024 * parity;
     half_t* const out = p.out + (size_t)(m0 + wm) * p.out_stride + n0 + (SILU ? wn / 2 : wn);
-    uint2 packed[8][8];                                     // [row block][channel block]
-    float sa[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sa[j] = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint2 w = *(const uint2*)(sc + 2 * (wn + 16 * i + 4 * e4));
-      const uint32_t wv[2] = {w.x, w.y};
-      float sw[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        typedef float v2f __attribute__((ext_vector_type(2)));
-        typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-        uint32_t h[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          v2f r = (v2f){(float)acc[i][j][2 * e] * (sw[2 * e] * sa[j]), (float)acc[i][j][2 * e + 1] * (sw[2 * e + 1] * sa[j])};
-          asm volatile("" : "+v"(r));
-          h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
-          asm volatile("" : "+v"(h[e]));                    // (converted here, not where it is stored: half the registers)
+    bool opened = false;
+    const TileParts mine = parts;
+    if constexpr (SHARE) {
+      if (mine.shared()) {
+        const bool last = mine.finishes(share, lds + LDS_SINK + 128, acc, [&] {
+          opened = true;
+          open = open_tile();
+        });
+        if (!last) {
+          parity ^= 1;
+          if (open) park(parity);
+          continue;
         }
-        packed[j][i] = make_uint2(h[0], h[1]);
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
-    open = open_tile();
+    uint2 packed[8][8];                                     // [row block][channel block]
+    auto pack = [&](auto add) __attribute__((always_inline)) {
+      constexpr bool ADD = decltype(add)::value;
+      if constexpr (SHARE) accumulators_stay(acc);
+      float sa[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sa[j] = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v4i x[8];
+        if constexpr (ADD) {
+          mine.others(share, 8 * i, x);
+          accumulators_stay(acc);
+        }
+        const uint2 w = *(const uint2*)(sc + 2 * (wn + 16 * i + 4 * e4));
+        const uint32_t wv[2] = {w.x, w.y};
+        float sw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          typedef float v2f __attribute__((ext_vector_type(2)));
+          typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+          uint32_t h[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int c0 = acc[i][j][2 * e] + (ADD ? x[j][2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? x[j][2 * e + 1] : 0);
+            v2f r = (v2f){(float)c0 * (sw[2 * e] * sa[j]), (float)c1 * (sw[2 * e + 1] * sa[j])};
+            asm volatile("" : "+v"(r));
+            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
+            asm volatile("" : "+v"(h[e]));                    // (converted here, not where it is stored: half the registers)
+          }
+          packed[j][i] = make_uint2(h[0], h[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (SHARE && mine.shared()) pack(BoolTag<SHARE>{});
+    else pack(BoolTag<false>{});
+    if (!opened) open = open_tile();
     // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
     uint8_t* buf = lds + LDS_OUT + wave * 16 * PITCH;
 #pragma unroll

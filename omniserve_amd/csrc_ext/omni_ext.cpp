@@ -74,6 +74,16 @@ inline int with_scratch(const GemmIO& g, const torch::Tensor& like, F call) {
   return rc;
 }
 
+// Scratch for a prompt's product whose last round's tiles share out their K (mode 1: per-group, 2: W8A8), from the caching allocator, in the order of the stream it is launched on: the tensor lives until
+// the launch.  Undefined where nothing is shared.
+inline torch::Tensor arm_share(const GemmIO& g, int mode, const torch::Tensor& like) {
+  const size_t n = omni_gemm_share_bytes(g.M, g.N, g.K, mode);
+  if (n == 0) return torch::Tensor();
+  torch::Tensor t = torch::empty({(int64_t)n}, torch::TensorOptions().dtype(torch::kUInt8).device(like.device()));
+  fail(omni_gemm_arm_share(t.data_ptr(), n), "gemm_forward");
+  return t;
+}
+
 void gemm_w4a8_per_chn(const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& wscales, const torch::Tensor& ascales,
                        const torch::Tensor& w_szs, const torch::Tensor& a_ssums, torch::Tensor out) {
   const GemmIO g = check_gemm_io(in, w, out, true);
@@ -96,6 +106,7 @@ void gemm_w4a8_per_group(const torch::Tensor& in, const torch::Tensor& w, const 
   check_second_level(zeros, scales_i8, g);
   need_cuda(wscales, "gemm_forward"); need_cuda(ascales, "gemm_forward");
   fail(with_scratch(g, in, [&](void* ws, size_t n) {
+         const torch::Tensor share = arm_share(g, 1, in);
          return omni_w4a8_per_group_gemm(in.data_ptr(), w.data_ptr(), zeros.data_ptr(), scales_i8.data_ptr(), wscales.data_ptr(), ascales.data_ptr(),
                                          out.data_ptr(), g.M, g.N, g.K, g.stride, ws, n, stream_of(in)); }),
        "qgemm_w4a8_per_group.gemm_forward_cuda");
@@ -105,6 +116,7 @@ void gemm_w8a8(const torch::Tensor& in, const torch::Tensor& w, const torch::Ten
   const GemmIO g = check_gemm_io(in, w, out, false);
   need_cuda(wscales, "gemm_forward"); need_cuda(ascales, "gemm_forward");
   fail(with_scratch(g, in, [&](void* ws, size_t n) {
+         const torch::Tensor share = arm_share(g, 2, in);
          return omni_w8a8_gemm(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), out.data_ptr(), g.M, g.N, g.K, g.stride,
                                ws, n, stream_of(in)); }),
        "qgemm_w8a8.w8a8_gemm_forward_cuda");
@@ -149,6 +161,7 @@ void gate_up_w4a8_per_group(torch::Tensor out, const torch::Tensor& in, const to
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
+            const torch::Tensor share = arm_share(g, 1, in);
             return omni_w4a8_per_group_gemm_silu_rows(in.data_ptr(), w.data_ptr(), zeros.data_ptr(), scales_i8.data_ptr(), wscales.data_ptr(), ascales.data_ptr(),
                                                       gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w4a8_per_group(in, w, zeros, scales_i8, wscales, ascales, gu); });
@@ -160,6 +173,7 @@ void gate_up_w8a8(torch::Tensor out, const torch::Tensor& in, const torch::Tenso
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
+            const torch::Tensor share = arm_share(g, 2, in);
             return omni_w8a8_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w8a8(in, w, wscales, ascales, gu); });
 }

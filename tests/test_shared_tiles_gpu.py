@@ -1,0 +1,88 @@
+"""Prompts' per-group and W8A8 products whose last round's tiles share out their K (csrc/tile_share.h): one tile of an XCD and many, two parts of a tile and many, with and without whole
+rounds in front, parts of the fewest stages, row tiles that share rows.  Against the same product with whole tiles: the same bits, whatever the scratch holds, launch after launch."""
+import pytest
+import torch
+
+from tests.test_silu_rows_gpu import GRP, W8, _case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+#        mode, rows, N, K                         tiles of an XCD's last round (of 32), parts
+SIZES = [(GRP, 2331, 4096, 14336), (W8, 2331, 4096, 14336),           # 20, two and three
+         (GRP, 2791, 6144, 8192), (W8, 2791, 6144, 8192),             # 1 behind a round, five: the most
+         (W8, 2133, 8192, 28672), (GRP, 4200, 4096, 14336),           # 4 and 2 behind a whole round
+         (GRP, 6000, 4096, 14336), (W8, 6000, 4096, 14336),           # 16 behind one: two
+         (GRP, 3165, 4096, 14336), (W8, 3000, 4096, 28672),           # 26, 24: one workgroup has the ends of several tiles
+         (GRP, 1570, 5120, 13824), (W8, 653, 4096, 14336)]            # 18 (some XCDs 17), 6
+UNIT = [(GRP, 2331, 28672, 4096), (GRP, 1500, 16384, 8192), (W8, 2100, 16384, 16384)]
+
+
+def _calls(mode, M, N, K, unit):
+    from omniserve_amd import _lib
+    h, (x, w, ops) = _lib.lib(), _case(M, N, K, mode)
+    need = h.omni_gemm_share_bytes(M, N, K, mode)
+    fn = {(GRP, False): h.omni_w4a8_per_group_gemm, (W8, False): h.omni_w8a8_gemm, (GRP, True): h.omni_w4a8_per_group_gemm_silu_rows, (W8, True): h.omni_w8a8_gemm_silu_rows}[mode, unit]
+    ws = torch.empty((max(h.omni_gemm_workspace_bytes(M, N, K), 1),), dtype=torch.uint8, device=DEV)
+
+    def call(out, scratch=None):
+        if scratch is not None:
+            assert h.omni_gemm_arm_share(scratch.data_ptr(), scratch.numel()) == 0
+        a = [t.data_ptr() for t in (x, w) + ops] + [out.data_ptr(), M, N, K]
+        a += [] if unit else [N, ws.data_ptr(), ws.numel()]
+        assert fn(*a, _lib.current_stream()) == 0
+        return out
+    n = N // 2 if unit else N
+    return need, call, lambda: torch.full((M, n), 7.0, dtype=torch.half, device=DEV), (x, w, ops, ws)
+
+
+@pytest.mark.parametrize("mode,M,N,K,unit", [s + (False,) for s in SIZES] + [s + (True,) for s in UNIT])
+def test_parts_add_up_to_the_whole(mode, M, N, K, unit):
+    need, call, out, keep = _calls(mode, M, N, K, unit)
+    assert need > 0
+    want = call(out())
+    assert torch.isfinite(want).all() and want.abs().sum() > 0
+    scratch = torch.randint(0, 256, (need,), dtype=torch.uint8, device=DEV)
+    for fill in (None, 0, 255, None):      # what was there, and what the launch before left
+        if fill is not None:
+            scratch.fill_(fill)
+        assert torch.equal(call(out(), scratch), want)
+    assert torch.equal(call(out()), want)      # one launch an arming
+
+
+def test_captured_launches_run_again():
+    need, call, out, keep = _calls(GRP, 2331, 4096, 14336, False)
+    want, got, scratch = call(out()), out(), torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    call(got, scratch)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(got, scratch)
+        call(got, scratch)
+    for _ in range(4):
+        got.fill_(7)
+        g.replay()
+        assert torch.equal(got, want)
+        assert torch.equal(call(out(), scratch), want)
+
+
+def test_mirror_takes_them_on_two_streams():
+    """The functions that allocate the scratch themselves, side by side"""
+    from omniserve_amd.backend import qgemm_w4a8_per_group
+    need, call, out, (x, w, ops, ws) = _calls(GRP, 2331, 4096, 14336, False)
+    want, streams, got = call(out()), [torch.cuda.Stream(), torch.cuda.Stream()], [[out() for _ in range(6)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for i in range(6):
+        for s, o in zip(streams, got):
+            with torch.cuda.stream(s):
+                qgemm_w4a8_per_group.gemm_forward_cuda(x, w, *ops, o[i])
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for os in got for o in os)
+
+
+def test_what_is_refused():
+    from omniserve_amd import _lib
+    h = _lib.lib()
+    t = torch.empty((1 << 20,), dtype=torch.uint8, device=DEV)
+    assert h.omni_gemm_arm_share(t.data_ptr(), t.numel()) != 0 and h.omni_gemm_arm_share(None, 0) == 0
+    for M, N, K, mode in ((2331, 4096, 14336, 0), (255, 4096, 14336, 1), (4000, 4096, 14336, 1), (2331, 4096, 512, 1), (2331, 4100, 14336, 2), (0, 0, 0, 1)):
+        assert h.omni_gemm_share_bytes(M, N, K, mode) == 0
