@@ -71,6 +71,14 @@ constexpr int TM = LM_TILE_ROWS;                            // rows of a tile
 static_assert(TM == 256, "the wave layouts");
 constexpr int HTN = 128;                                    // channels of a half tile
 
+// Row tiles with rows in them: experts fill fewer than the host has to reckon with (lm_route_max_tiles), and the tail without rows, of a tenth of the tiles with 32 experts and 8000 tokens, a sixth
+// with 64 of fewer, would be the last XCD's alone, the others' rounds the longer for it (us, whole tiles, 7999 tokens, 6 of 32 experts of 1792, width 4096, up 1612 -> 1593, down 888 -> 840; 900 tokens
+// 400 -> 314; 8 of 64 experts of 640, width 2048, 5800 tokens, up, 327 -> 277.  The half tiles, a workgroup each, wait for the entry: 1 - 2 % longer, and keep their order).  The last entry says how many, if it has no rows itself.
+__device__ __forceinline__ int row_tiles(const int* tiles, int max_tiles) {
+  const i32x4 last = *(const i32x4*)(tiles + 4 * (max_tiles - 1));
+  return last[2] > 0 || last[3] <= 0 ? max_tiles : min(last[3], max_tiles);
+}
+
 // gemm_half_tiles_kernel<epi> over `wgs` workgroups; mt_a, mt_b: row tiles of both parts
 __attribute__((visibility("hidden"))) void launch_half_tiles(const GemmArgs& a, int epi, unsigned wgs, int mt_a, int mt_b, hipStream_t s);
 

@@ -445,6 +445,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // linear order of a part: bands of row tiles, all channel tiles of a band before the next one; an XCD has a contiguous range of both
   // parts, its workgroups take the tiles of it in turn
+  if (p.perm) mt_a = row_tiles(p.tiles, mt_a);
   const int nt_a = (p.a.n + TN - 1) / TN, nt_b = mt_b ? (p.b.n + TN - 1) / TN : 0;
   const int per_a = (mt_a * nt_a + 7) >> 3, per_b = (mt_b * nt_b + 7) >> 3, xcd = blockIdx.x & 7;
   const int own_b = max(0, min(per_b, mt_b * nt_b - xcd * per_b)), own = own_b + max(0, min(per_a, mt_a * nt_a - xcd * per_a));
@@ -688,6 +689,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
 // (1.05 with fewer than 48 rows in a tile, where they wait for weights), a rest that is alone on its CUs 0.8.  What it is about: grids that leave CUs idle, and last rounds.
 // (MI355X, bf16, 256 x 256 / 256 x 128, us: to f32, 65 rows of 32000 x 4096 103 / 84, 300 rows 110 / 133, 1000 rows of 8192 x 4096 79 / 72, 2000
 // rows 103 / 138.  Experts: 12 rows each of 32 x 4096 x 1792 145 / 131, 131 rows 158 / 176, 750 rows 415 / 498; 64 x 2048 x 640, 8, 87 and 500 rows, 62 / 49, 62 / 58, 152 / 156.
+// With the rows' tiles shared out evenly (row_tiles): 300 tokens, 6 of 32 experts of 1792, width 4096, up, 229 / 303 (before: whole 311), 1200 331 / 542 and, down, 205 / 292, 2000 509 / 715 and 294 / 351; 8 of
+// 64 experts of 640, width 2048, 2000 tokens 129 / 212 and 83 / 117, 5800 276 / 388 and 201 / 234.  Over those 44 sizes the choice costs 0.1 % on average, 3.9 % before.
 // f32, 65 rows of 4096 x 1024 234 / 129.  Over 113 bf16 sizes the choice costs 0.4 % on average and 9 % at most, 700 tokens' two of 16 experts of 4096 x 4096, 209 us for 192, against the
 // better one.)
 // max_tiles > 0: rows sorted by group, of which there is a tile for every 256 and one per group.  Part b over rows_b rows: its tiles are the first that
@@ -695,11 +698,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
 static bool half_tiles(int n, int k, int groups, int max_tiles, int rows_a, int n_b, int k_b, int rows_b) {
   const int row_tiles = max_tiles > 0 ? max_tiles : (rows_a + TM - 1) / TM;
   const int64_t rows = max_tiles > 0 ? (int64_t)TM * max(0, max_tiles - groups) : rows_a;
-  auto per_xcd = [&](int tn) {
+  auto per_xcd = [&](int tn, int tiles_a) {
     auto part = [&](int tiles, int c) { return ((int64_t)tiles * ((c + tn - 1) / tn) + 7) / 8; };
-    return part(row_tiles, n) + part((rows_b + TM - 1) / TM, n_b);
+    return part(tiles_a, n) + part((rows_b + TM - 1) / TM, n_b);
   };
-  const int64_t per_h = per_xcd(HTN), per_f = per_xcd(TN);
+  // (the whole tiles' XCDs share out those that have rows, of experts that differ as many as their mean has and 0.45 more; the half tiles' those that may have.  Of fewer than 144 rows of each
+  // expert, 48 of 8 KB of K, which wait for weights, the difference is not made)
+  const int filled = max_tiles > 0 && rows >= (k * (int)sizeof(elem_t) >= 8192 ? 48 : 144) * (int64_t)groups ? min(max_tiles, (int)((float)groups * fmaxf(1.f, (float)rows / (float)(TM * groups) + 0.45f))) : row_tiles;
+  const int64_t per_h = per_xcd(HTN, row_tiles), per_f = per_xcd(TN, filled);
   const int64_t places = max_tiles > 0 ? groups : row_tiles;
   const float pair = rows < 48 * places ? 1.05f
                                         : (rows < 1000 * places ? 0.97f : 1.01f) + 0.25f * (float)min((int64_t)k * (int)sizeof(elem_t), (int64_t)8192) / 8192.f;

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void route_choose_kernel(const float* z, int64
   }
 }
 
-// ... offsets and row tiles (entries past the last tile: no rows) ...
+// ... offsets and row tiles (entries past the last tile: no rows, and how many tiles there are) ...
 __global__ __launch_bounds__(512) void route_offsets_kernel(const int* count, int experts, int max_tiles, int* off, int* tiles) {
   __shared__ int s_off[MAX_EXPERTS], s_tile[MAX_EXPERTS];
   const int e = threadIdx.x, c = e < experts ? count[e] : 0, nt = (c + LM_TILE_ROWS - 1) / LM_TILE_ROWS;
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(512) void route_offsets_kernel(const int* count, in
     for (int i = 0; i < nt; ++i) out[t + i] = (i32x4){e, o + LM_TILE_ROWS * i, min(LM_TILE_ROWS, c - LM_TILE_ROWS * i), 0};
     if (e == experts - 1) off[experts] = s_off[e];
   }
-  for (int t = s_tile[511] + e; t < max_tiles; t += 512) out[t] = (i32x4){0, 0, 0, 0};
+  for (int t = s_tile[511] + e; t < max_tiles; t += 512) out[t] = (i32x4){0, 0, 0, s_tile[511]};
 }
 
 // ... and the pairs in their places
