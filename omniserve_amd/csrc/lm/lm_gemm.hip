@@ -449,7 +449,9 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   const int nt_a = (p.a.n + TN - 1) / TN, nt_b = mt_b ? (p.b.n + TN - 1) / TN : 0;
   const int per_a = (mt_a * nt_a + 7) >> 3, per_b = (mt_b * nt_b + 7) >> 3, xcd = blockIdx.x & 7;
   const int own_b = max(0, min(per_b, mt_b * nt_b - xcd * per_b)), own = own_b + max(0, min(per_a, mt_a * nt_a - xcd * per_a));
-  int at = blockIdx.x >> 3;                                 // in the XCD's range
+  // in the XCD's range: a place further among its workgroups with every turn, so that a row of short tiles in every band is not always the same ones'
+  const int turn = (int)gridDim.x >> 3;
+  int place = blockIdx.x >> 3, turns = 0;
 
   // pieces of 8 rows: lane -> (row lane / 8, physical slot lane % 8); a wave carries 8 of the weights' and 8 of x's.  (A row of the tile past
   // the matrix: its last one again; none of it is stored.)
@@ -471,11 +473,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
     }
     wbase += SROWB;
   };
-  bool is_b = false;
+  bool is_b = false, few_next = false;
   int n0 = 0, ns = 0;
   // the next tile with rows from place `at` on: its rows of y, its first two stages requested; false: there is none
   auto open_tile = [&](int (&y_row)[TM]) {
-    for (; at < own; at += (int)gridDim.x >> 3) {
+    while (turns + place < own) {
+      const int at = turns + place;
+      turns += turn;
+      place = place + 1 == turn ? 0 : place + 1;
       is_b = at < own_b;
       const Part& pt = is_b ? p.b : p.a;
       const int nt = is_b ? nt_b : nt_a, mts = is_b ? mt_b : mt_a;
@@ -498,12 +503,19 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       n0 = in / bm * TN;
       ns = pt.k / SK;
       wbase = (const uint8_t*)(pt.w + ((int64_t)g * pt.n + n0) * pt.k);
+      int xr[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int r = 64 * wave + 8 * i + pr, rc = min(r, rows - 1);
+        const int rc = first + min(64 * wave + 8 * i + pr, rows - 1);
+        xr[i] = perm ? perm[rc] : rc;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 64 * wave + 8 * i + pr;
         woff[i] = (uint32_t)min(r, pt.n - 1 - n0) * (uint32_t)(pt.k * (int)sizeof(elem_t)) + ((ps ^ T::swizzle(r)) << 4);
-        const int xr = perm ? perm[first + rc] / x_div : first + rc;
-        xsrc[i] = (const uint8_t*)(pt.x + (int64_t)xr * pt.ldx) + ((ps ^ T::swizzle(r)) << 4);
+        xsrc[i] = (const uint8_t*)(pt.x + (int64_t)(perm ? xr[i] / x_div : xr[i]) * pt.ldx) + ((ps ^ T::swizzle(r)) << 4);
+        __builtin_amdgcn_sched_barrier(0);                  // (not eight divisions at once beside the results of the tile before)
       }
       {
         const int r = 64 * ((ol & 16 ? in / bm : mi) & 3) + 16 * wave + (ol & 15), rc = first + min(r, rows - 1);
@@ -516,13 +528,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       stage(0);
       if (ns > 1) stage(1);
       if constexpr (TOUCH) touch_lines32(soon, lds0 + 2 * STAGE + OUT);
-      at += (int)gridDim.x >> 3;
+      few_next = rows <= TM / 2;
       return true;
     }
     return false;
   };
 
-  const int wn = 128 * (wave & 1), wm = 128 * (wave >> 1);
+  const int wn = 128 * (wave & 1);
+  int wm = 0;                                               // the wave's first row
   int off[2];                                               // of a fragment of half u inside 16 rows
   frag_t a[2][8], b[2][8];
   auto fetch_b = [&](int t, auto half, int i) {
@@ -537,7 +550,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
   // Stage t: FRESH: the tile's first (its accumulators were not zeroed: 256 instructions of a lone wave), MORE: there is a stage t + 1, DMA: and a stage t + 2.  Requests and reads go out one by one between the products: a burst of
   // them fills the queues of the address path and the LDS, and the lone wave, which issues in order, waits there with its matrix
   // unit idle.  No condition inside: reads and products have to share a basic block.
-  auto step = [&](int t, auto fresh, auto more, auto dma) {
+  auto step = [&](int t, auto blocks, auto fresh, auto more, auto dma) {
+    constexpr int NJ = decltype(blocks)::value;            // blocks of 16 rows of the wave: 8, or 4 of a tile of up to 128 rows
     constexpr bool FRESH = decltype(fresh)::value, MORE = decltype(more)::value, DMA = decltype(dma)::value;
     auto four = [&](auto half, int i0, int j) {
       constexpr int U = decltype(half)::value;
@@ -549,11 +563,12 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       fetch_b(t, Int<1>{}, j);
+      if constexpr (NJ == 4) fetch_a(t, Int<1>{}, 2 * j);
       __builtin_amdgcn_sched_barrier(0);
       four(Int<0>{}, 0, j);
-      fetch_a(t, Int<1>{}, j);
+      fetch_a(t, Int<1>{}, NJ == 4 ? 2 * j + 1 : j);
       __builtin_amdgcn_sched_barrier(0);
       four(Int<0>{}, 4, j);
     }
@@ -564,22 +579,31 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if constexpr (MORE) fetch_b(t + 1, Int<0>{}, j);
+    for (int j = 0; j < NJ; ++j) {
+      constexpr int PER = 8 / NJ;                           // pieces of each operand with a block of rows
+      if constexpr (MORE) {
+        fetch_b(t + 1, Int<0>{}, j);
+        if constexpr (PER == 2) fetch_a(t + 1, Int<0>{}, 2 * j);
+      }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (DMA) {
-        mma3_dma16<true>(acc[0][j], acc[1][j], acc[2][j], a[1][0], a[1][1], a[1][2], b[1][j], woff[j], wbase, dst(t, j));
+        mma3_dma16<true>(acc[0][j], acc[1][j], acc[2][j], a[1][0], a[1][1], a[1][2], b[1][j], woff[PER * j], wbase, dst(t, PER * j));
         mma_in_place(acc[3][j], a[1][3], b[1][j]);
+        if constexpr (PER == 2) dma16_uncounted(wbase + woff[2 * j + 1 & 7], dst(t, 2 * j + 1));
         __builtin_amdgcn_sched_barrier(0);
       } else {
         four(Int<1>{}, 0, j);
       }
-      if constexpr (MORE) fetch_a(t + 1, Int<0>{}, j);
+      if constexpr (MORE) fetch_a(t + 1, Int<0>{}, PER * j + PER - 1);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (DMA) {
-        mma3_dma16<false>(acc[4][j], acc[5][j], acc[6][j], a[1][4], a[1][5], a[1][6], b[1][j], xsrc[j], nullptr, dst(t, 8 + j));
-        xsrc[j] += SROWB;
+        mma3_dma16<false>(acc[4][j], acc[5][j], acc[6][j], a[1][4], a[1][5], a[1][6], b[1][j], xsrc[PER * j], nullptr, dst(t, 8 + PER * j));
+        xsrc[PER * j] += SROWB;
         mma_in_place(acc[7][j], a[1][7], b[1][j]);
+        if constexpr (PER == 2) {
+          dma16_uncounted(xsrc[2 * j + 1 & 7], dst(t, 8 + 2 * j + 1));
+          xsrc[2 * j + 1 & 7] += SROWB;
+        }
         __builtin_amdgcn_sched_barrier(0);
       } else {
         four(Int<1>{}, 4, j);
@@ -599,85 +623,92 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(GemmArgs p, int mt_a
     if (ns > 1) wait_pieces<16 + TOUCH>();
     else wait_pieces<0>();
     __syncthreads();
+    const bool few = few_next;
+    wm = (few ? 64 : 128) * (wave >> 1);
     const int fl = lane_here();
 #pragma unroll
     for (int u = 0; u < 2; ++u) off[u] = T::slot(fl & 15, 4 * u + (fl >> 4));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      fetch_b(0, Int<0>{}, i);
-      fetch_a(0, Int<0>{}, i);
-    }
-    int t = 0;
-    if (TOUCH && ns > 2) {
-      step(0, Int<TOUCH>{}, Int<1>{}, Int<1>{});
-      t = 1;
-    } else {
-      const float z = __builtin_bit_cast(float, opaque(0));
+    auto products = [&](auto blocks) __attribute__((always_inline)) {
+      constexpr int NJ = decltype(blocks)::value;
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{z, z, z, z};
-    }
-    for (; t + 2 < ns; ++t) step(t, Int<0>{}, Int<1>{}, Int<1>{});
-    if (t + 1 < ns) {
-      step(t, Int<0>{}, Int<1>{}, Int<0>{});
-      ++t;
-    }
-    step(t, Int<0>{}, Int<0>{}, Int<0>{});                  // (behind its barrier both stages are free)
+        for (int j = NJ; j < 8; ++j) asm volatile("" : "=a"(acc[i][j]));      // (nothing: no value of the tile before is carried along)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i < NJ) fetch_b(0, Int<0>{}, i);
+        fetch_a(0, Int<0>{}, i);
+      }
+      int t = 0;
+      if (TOUCH && ns > 2) {
+        step(0, blocks, Int<TOUCH>{}, Int<1>{}, Int<1>{});
+        t = 1;
+      } else {
+        const float z = __builtin_bit_cast(float, opaque(0));
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{z, z, z, z};
+      }
+      for (; t + 2 < ns; ++t) step(t, blocks, Int<0>{}, Int<1>{}, Int<1>{});
+      if (t + 1 < ns) {
+        step(t, blocks, Int<0>{}, Int<1>{}, Int<0>{});
+        ++t;
+      }
+      step(t, blocks, Int<0>{}, Int<0>{}, Int<0>{});        // (behind its barrier both stages are free)
+    };
+    if (few) products(Int<4>{});
+    else products(Int<8>{});
     accumulators_settle(acc);
 
     const Part& pt = is_b ? p.b : p.a;
     const int el = lane_here(), e15 = el & 15, e4 = el >> 4;
     const int c0 = n0 + wn;                                 // the wave's first channel
     const int* y_row = y_rows[parity];
-    // the results, packed; then the next tile
-    constexpr int NI = EPI == LM_EPI_GLU ? 4 : 8;
-    quad_t out[DIRECT ? 1 : 8][NI];
-    if constexpr (!DIRECT) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          if constexpr (EPI == LM_EPI_GLU) out[j][i] = to_quad(glu(pt, p.act, min(c0 + 32 * i, pt.n - 32) + 4 * e4, acc[2 * i][j], acc[2 * i + 1][j]));
-          else out[j][i] = to_quad(acc[i][j]);
-        }
-      open = open_tile(y_rows[parity ^ 1]);
-    }
+    const int span = few ? 64 : 128;                        // the wave's rows (behind them is what other tiles left)
+    // the next tile's requests, then the results: they stay in the accumulation registers until they are stored
+    open = open_tile(y_rows[parity ^ 1]);
+    accumulators_stay(acc);
     if constexpr (DIRECT) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int row = y_row[wm + 16 * j + e15];
-        if (row < 0) continue;
+        const int row = 16 * j < span ? y_row[wm + 16 * j + e15] : -1;
+        if (row >= 0) {
 #pragma unroll
-        for (int i = 0; i < 8; i += EPI == LM_EPI_GLU ? 2 : 1) {
-          const int c = c0 + 16 * i + 4 * e4;
-          if (c >= pt.n) continue;
-          if constexpr (EPI == LM_EPI_GLU) store4<EPI>(pt, row, (c0 + 16 * i) / 2 + 4 * e4, 0, glu(pt, p.act, c, acc[i][j], acc[i + 1][j]), p.scale);
-          else store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
+          for (int i = 0; i < 8; i += EPI == LM_EPI_GLU ? 2 : 1) {
+            const int c = c0 + 16 * i + 4 * e4;
+            if (c >= pt.n) continue;
+            if constexpr (EPI == LM_EPI_GLU) store4<EPI>(pt, row, (c0 + 16 * i) / 2 + 4 * e4, 0, glu(pt, p.act, c, acc[i][j], acc[i + 1][j]), p.scale);
+            else store4<EPI>(pt, row, c, 0, acc[i][j], p.scale);
+          }
         }
-        __builtin_amdgcn_sched_barrier(0);                  // (no addresses of later rows kept beside the accumulators)
+        accumulators_stay(acc);                             // (no addresses of later rows kept beside them either)
       }
-      open = open_tile(y_rows[parity ^ 1]);
     } else {
       // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
-      constexpr int PPR = OC / FR;
+      constexpr int PPR = OC / FR, NI = EPI == LM_EPI_GLU ? 4 : 8;
       uint8_t* buf = lds + 2 * STAGE + wave * 16 * PITCH;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) *(quad_t*)(buf + e15 * PITCH + (16 * i + 4 * e4) * (int)sizeof(elem_t)) = out[j][i];
+        for (int i = 0; i < NI; ++i) {
+          quad_t v;
+          if constexpr (EPI == LM_EPI_GLU) v = to_quad(glu(pt, p.act, min(c0 + 32 * i, pt.n - 32) + 4 * e4, acc[2 * i][j], acc[2 * i + 1][j]));
+          else v = to_quad(acc[i][j]);
+          *(quad_t*)(buf + e15 * PITCH + (16 * i + 4 * e4) * (int)sizeof(elem_t)) = v;
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < 16 * PPR / 64; ++i) {
           const int pc = 64 * i + el, r = pc / PPR, q = pc % PPR;
-          const int row = y_row[wm + 16 * j + r], c = (EPI == LM_EPI_GLU ? c0 / 2 : c0) + q * FR;
+          const int row = 16 * j < span ? y_row[wm + 16 * j + r] : -1, c = (EPI == LM_EPI_GLU ? c0 / 2 : c0) + q * FR;
           if (row >= 0 && c < (EPI == LM_EPI_GLU ? pt.n / 2 : pt.n))
             *(frag_t*)((elem_t*)pt.y + (int64_t)row * pt.ldy + c) = *(const frag_t*)(buf + r * PITCH + q * 16);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        accumulators_stay(acc);
       }
     }
     parity ^= 1;
