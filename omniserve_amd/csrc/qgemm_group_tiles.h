@@ -14,6 +14,9 @@
 // 336 / 396; 2331 rows of 28672 x 4096 318 / 342.  The matrix units are busy half of the time, as in the W8A8 tiles; unpacking in 8.5 operations a word took
 // 2 - 3 % more, letting the stores of a tile fly into the next one nothing less.
 //
+// The next tile's requests go out before the results are scaled, which wait in the accumulation registers (accumulators_stay): 2331 rows of 28672 x 4096 with the unit 291 -> 279 us, of 6144 x 4096
+// 59.5 -> 56.8, 6000 rows of 28672 x 4096 620 -> 600.
+//
 // SHARE: K of the last round's tiles shared out (tile_share.h).
 //
 // Integer sums and the general kernel's epilogue: the same bits.
@@ -351,13 +354,13 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     step(buf, 0, BoolTag<false>{}, BoolTag<false>{});       // (behind its barrier all buffers are free)
     accumulators_settle(acc);
 
-    // the results, packed; then the next tile; then the stores (w8a8_tiles_kernel's arithmetic)
+    // the next tile's requests, then the results, which stay in the accumulation registers until they are stored (w8a8_tiles_kernel's arithmetic)
     const int el = lane_here(), e15 = el & 15, i0 = (el >> 4) * 4;
     const int chan = (i0 >> 3) * 32 + (i0 & 7);             // of block 0
     const uint8_t* scales = lds + LDS_SC + 1024 * parity;
     half_t* const out = p.out + (size_t)m0 * p.out_stride + n0 + (SILU ? 32 : 64) * wave;
-    bool opened = false;
     const TileParts mine = parts;
+    bool opened = false;
     if constexpr (SHARE) {
       if (mine.shared()) {
         const bool last = mine.finishes(share, lds + LDS_SC + 2 * 1024, acc, [&] {
@@ -371,73 +374,70 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
         }
       }
     }
-    uint2 packed[16][4];                                    // [row block][channel block]
-    auto pack = [&](auto add) __attribute__((always_inline)) {
+    if (!opened) open = open_tile();
+    uint8_t* rows = lds + LDS_OUT + wave * 16 * PITCH;
+    auto store = [&](auto add) __attribute__((always_inline)) {
       constexpr bool ADD = decltype(add)::value;
-      if constexpr (SHARE) accumulators_stay(acc);
+      accumulators_stay(acc);
+      float sw[4][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        v4i x[8];
         const uint2 w = *(const uint2*)(scales + 2 * (64 * wave + chan + 8 * i));
         const uint32_t wv[2] = {w.x, w.y};
-        float sw[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+        for (int e = 0; e < 4; ++e) sw[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+      }
+      v4i x[16];                                            // ADD: of four blocks of rows
+      uint2 h[2][4];                                        // [row block][channel block]
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          if constexpr (ADD) if (j % 8 == 0) {
-            __builtin_amdgcn_sched_barrier(0);
-            mine.others(share, 16 * i + j, x);
-            accumulators_stay(acc);
-          }
-          const float sa = (float)*(const half_t*)(scales + 512 + 2 * (16 * j + e15));
-          uint32_t h[2];
+      for (int j = 0; j < 16; ++j) {
+        if constexpr (ADD) if (j % 4 == 0) {
+          mine.others(share, [&](int q) { return 16 * (q & 3) + j + (q >> 2); }, x);
+          accumulators_stay(acc);
+        }
+        const float sa = (float)*(const half_t*)(scales + 512 + 2 * (16 * j + e15));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t hw[2];
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
-            const int c0 = acc[i][j][2 * e] + (ADD ? x[j & 7][2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? x[j & 7][2 * e + 1] : 0);
-            v2f r = (v2f){(float)c0 * (sw[2 * e] * sa), (float)c1 * (sw[2 * e + 1] * sa)};
+            const v4i& y = x[4 * (j & 3) + i];
+            const int c0 = acc[i][j][2 * e] + (ADD ? y[2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? y[2 * e + 1] : 0);
+            v2f r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
             asm volatile("" : "+v"(r));
-            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
-            asm volatile("" : "+v"(h[e]));
+            hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
           }
-          packed[j][i] = make_uint2(h[0], h[1]);
+          h[j & 1][i] = make_uint2(hw[0], hw[1]);
+        }
+        if constexpr (SILU) {      // two row blocks at a time; lanes l and l ^ 16 have a block's eight channels
+          if (j & 1) {
+            const int odd = (el >> 4) & 1;
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+              const uint2 v = silu_mul_blocks(h[0][i], h[1][i]), y = silu_mul_blocks(h[0][i + 1], h[1][i + 1]);
+              const auto lo = __builtin_amdgcn_permlane16_swap(v.x, y.x, false, false), hi = __builtin_amdgcn_permlane16_swap(v.y, y.y, false, false);
+              *(uint4*)(out + (size_t)(16 * (j - 1) + 16 * (el >> 5) + e15) * p.out_stride + 8 * (i + odd)) =
+                  make_uint4((uint32_t)lo[0], (uint32_t)hi[0], (uint32_t)lo[1], (uint32_t)hi[1]);
+            }
+          }
+        } else {      // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's 64 channels at a time
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *(uint2*)(rows + e15 * PITCH + (chan + 8 * i) * 2) = h[j & 1][i];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int r = 8 * i + (el >> 3);
+            *(uint4*)(out + (size_t)(16 * j + r) * p.out_stride + (el & 7) * 8) = *(const uint4*)(rows + r * PITCH + (el & 7) * 16);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    if (SHARE && mine.shared()) pack(BoolTag<SHARE>{});
-    else pack(BoolTag<false>{});
-    if (!opened) open = open_tile();
-    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's 64 channels at a time
-    uint8_t* rows = lds + LDS_OUT + wave * 16 * PITCH;
-    if constexpr (SILU) {      // two row blocks at a time; lanes l and l ^ 16 have a block's eight channels
-      const int odd = (el >> 4) & 1;
-#pragma unroll
-      for (int j = 0; j < 16; j += 2) {
-#pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          const uint2 x = silu_mul_blocks(packed[j][i], packed[j + 1][i]), y = silu_mul_blocks(packed[j][i + 1], packed[j + 1][i + 1]);
-          const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false), hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
-          *(uint4*)(out + (size_t)(16 * j + 16 * (el >> 5) + e15) * p.out_stride + 8 * (i + odd)) = make_uint4((uint32_t)lo[0], (uint32_t)hi[0], (uint32_t)lo[1], (uint32_t)hi[1]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < (SILU ? 0 : 16); ++j) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *(uint2*)(rows + e15 * PITCH + (chan + 8 * i) * 2) = packed[j][i];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = 8 * i + (el >> 3);
-        *(uint4*)(out + (size_t)(16 * j + r) * p.out_stride + (el & 7) * 8) = *(const uint4*)(rows + r * PITCH + (el & 7) * 16);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    if (SHARE && mine.shared()) store(BoolTag<SHARE>{});
+    else store(BoolTag<false>{});
     parity ^= 1;
     if (open) park(parity);
   }

@@ -21,6 +21,7 @@
 //    one's, so that the L2 has everything, 983 | 445; no requests at all 934 | 398; no LDS reads 1182 | 498); a line of the tile that is there anyway -> the lines ahead 1067 -> 1056 |
 //    516 -> 500, and of 28672 x 4096 in bands of four 1024 rows 113 -> 105, 2048 213 -> 200, in bands of three 1501 163 -> 157, 2100 217 -> 216; of 4096 x 14336 2100 166 -> 150, 2331 166 -> 131;
 //  * results stored -> streamed 1038 -> 1013 | 470 -> 461, accumulators zeroed -> not 1013 -> 996 | 460 -> 459.
+//  * the next tile requested behind -> before the scaling of the results, 30 sizes of 290 - 7900 rows, 1.009x on average (single rounds with the unit lose 1 %), 12001 rows 1047 -> 1043 | 491 -> 497.
 // What is left of the 5 POPS nominal is the clock under this load, the ends of a tile, which 4096 of K show, and the L2.
 #pragma once
 #include "lm/mfma_pinned.h"
@@ -226,13 +227,13 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
     step(t, BoolTag<false>{}, BoolTag<false>{}, BoolTag<false>{});      // (behind its barrier both stages are free)
     accumulators_settle(acc);
 
-    // the results, packed; then the next tile; then the stores.  The arithmetic of the general kernel: both scales' product, the sum times
-    // it, each rounded to f32, then to fp16 -- opaque in between, or hipcc folds the last two into one rounding.
+    // The next tile's requests, then the results, which stay in the accumulation registers until they are stored.  The arithmetic of the general kernel: both scales' product, the sum times it, each
+    // rounded to f32, then to fp16 -- opaque in between, or hipcc folds the last two into one rounding.
     const int el = lane_here(), e15 = el & 15, e4 = el >> 4;
     const uint8_t* sc = lds + LDS_SC + 1024 * parity;
     half_t* const out = p.out + (size_t)(m0 + wm) * p.out_stride + n0 + (SILU ? wn / 2 : wn);
-    bool opened = false;
     const TileParts mine = parts;
+    bool opened = false;
     if constexpr (SHARE) {
       if (mine.shared()) {
         const bool last = mine.finishes(share, lds + LDS_SINK + 128, acc, [&] {
@@ -246,64 +247,60 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
         }
       }
     }
-    uint2 packed[8][8];                                     // [row block][channel block]
-    auto pack = [&](auto add) __attribute__((always_inline)) {
+    if (!opened) open = open_tile();
+    uint8_t* buf = lds + LDS_OUT + wave * 16 * PITCH;
+    auto store = [&](auto add) __attribute__((always_inline)) {
       constexpr bool ADD = decltype(add)::value;
-      if constexpr (SHARE) accumulators_stay(acc);
-      float sa[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sa[j] = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
+      accumulators_stay(acc);
+      float sw[8][4];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        v4i x[8];
-        if constexpr (ADD) {
-          mine.others(share, 8 * i, x);
-          accumulators_stay(acc);
-        }
         const uint2 w = *(const uint2*)(sc + 2 * (wn + 16 * i + 4 * e4));
         const uint32_t wv[2] = {w.x, w.y};
-        float sw[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+        for (int e = 0; e < 4; ++e) sw[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+      }
+      // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
+      v4i x[16];                                            // ADD: of two blocks of rows
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (ADD) if (j % 2 == 0) {
+          mine.others(share, [&](int q) { return 8 * (q & 7) + j + (q >> 3); }, x);
+          accumulators_stay(acc);
+        }
+        const float sa = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
+        uint2 h[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
           typedef float v2f __attribute__((ext_vector_type(2)));
           typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-          uint32_t h[2];
+          uint32_t hw[2];
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
-            const int c0 = acc[i][j][2 * e] + (ADD ? x[j][2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? x[j][2 * e + 1] : 0);
-            v2f r = (v2f){(float)c0 * (sw[2 * e] * sa[j]), (float)c1 * (sw[2 * e + 1] * sa[j])};
+            const v4i& y = x[8 * (j & 1) + i];
+            const int c0 = acc[i][j][2 * e] + (ADD ? y[2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? y[2 * e + 1] : 0);
+            v2f r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
             asm volatile("" : "+v"(r));
-            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
-            asm volatile("" : "+v"(h[e]));                    // (converted here, not where it is stored: half the registers)
+            hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
           }
-          packed[j][i] = make_uint2(h[0], h[1]);
+          h[i] = make_uint2(hw[0], hw[1]);
         }
+#pragma unroll
+        for (int i = 0; i < (SILU ? 4 : 8); ++i) *(uint2*)(buf + e15 * PITCH + (16 * i + 4 * e4) * 2) = SILU ? silu_mul_h4(h[i], h[i + 4 & 7]) : h[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < (SILU ? 2 : 4); ++i) {
+          const int r = SILU ? 8 * i + (el >> 3) : 4 * i + e4, q = SILU ? el & 7 : e15;
+          __builtin_nontemporal_store(*(const v4i*)(buf + r * PITCH + q * 16), (v4i*)(out + (size_t)(16 * j + r) * p.out_stride + q * 8));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    if (SHARE && mine.shared()) pack(BoolTag<SHARE>{});
-    else pack(BoolTag<false>{});
-    if (!opened) open = open_tile();
-    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
-    uint8_t* buf = lds + LDS_OUT + wave * 16 * PITCH;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-#pragma unroll
-      for (int i = 0; i < (SILU ? 4 : 8); ++i)
-        *(uint2*)(buf + e15 * PITCH + (16 * i + 4 * e4) * 2) = SILU ? silu_mul_h4(packed[j][i], packed[j][i + 4 & 7]) : packed[j][i];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int i = 0; i < (SILU ? 2 : 4); ++i) {
-        const int r = SILU ? 8 * i + (el >> 3) : 4 * i + e4, q = SILU ? el & 7 : e15;
-        __builtin_nontemporal_store(*(const v4i*)(buf + r * PITCH + q * 16), (v4i*)(out + (size_t)(16 * j + r) * p.out_stride + q * 8));
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    if (SHARE && mine.shared()) store(BoolTag<SHARE>{});
+    else store(BoolTag<false>{});
     parity ^= 1;
     if (open) park(parity);
   }

@@ -141,25 +141,25 @@ struct TileParts {
     if (tid == 0) __hip_atomic_store(mark, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
   }
-  // x: the other parts' sums of pieces first .. first + M - 1
-  template <int M>
-  __device__ __forceinline__ void others(const TileShare& p, int first, v4i (&x)[M]) const {
+  // x[q]: the other parts' sums of piece number(q)
+  template <int M, class Number>
+  __device__ __forceinline__ void others(const TileShare& p, Number number, v4i (&x)[M]) const {
     const int tid = threadIdx.x;
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(p.sums, 0, (int)SHARE_SUMS, 0x00020000);
-    auto piece = [&](uint32_t at, int j) { return __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, at + (first + j) * 4096, 16); };
+    auto piece = [&](uint32_t at, int q) { return __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, at + number(q) * 4096, 16); };
     // (the first of them is this one or another)
     int s = me() < 0 ? lo : -1;
     uint32_t at = place(s);
 #pragma unroll
-    for (int j = 0; j < M; ++j) x[j] = piece(at, j);
+    for (int q = 0; q < M; ++q) x[q] = piece(at, q);
     for (s = max(s + 1, lo); s <= hi; ++s) {
       if (s == me()) continue;
       at = place(s);
       v4i y[M];
 #pragma unroll
-      for (int j = 0; j < M; ++j) y[j] = piece(at, j);
+      for (int q = 0; q < M; ++q) y[q] = piece(at, q);
 #pragma unroll
-      for (int j = 0; j < M; ++j) x[j] += y[j];
+      for (int q = 0; q < M; ++q) x[q] += y[q];
     }
   }
 };
