@@ -40,7 +40,7 @@ int omni_abi_version(void);
  * ABI 4 (omni_abi_version): ABI 3 had one query for both (which pinned an M x N slab for plain calls at M = 129..512). */
 size_t omni_gemm_workspace_bytes(int M, int N, int K);
 size_t omni_gemm_partial_workspace_bytes(int M, int N, int K);
-/* Prompts' per-group (mode 1) and W8A8 (2) products, with or without silu_and_mul: scratch with which the last round's tiles share out their K, 0 where that gains nothing.  The
+/* Prompts' per-channel (mode 0), per-group (1) and W8A8 (2) products, with or without silu_and_mul: scratch with which the last round's tiles share out their K, 0 where that gains nothing.  The
  * same bits with and without.  omni_gemm_arm_share: the next of these products that this thread enqueues may use the scratch (16-byte aligned, any contents), until it has run; any other of
  * them takes the arming back. */
 size_t omni_gemm_share_bytes(int M, int N, int K, int mode);
@@ -48,7 +48,7 @@ int omni_gemm_arm_share(void* scratch, size_t bytes);
 
 /* Tuning / introspection hooks (tests and bench sweeps; not used by the serving path):
  * override the decode-shape plan (waves per workgroup: 1 or 4; K splits; M > 128: K slices over the grid where the plan may
- * have them, and waves = 16: per-group products of 256 rows or more in 256 x 256 tiles wherever K >= 512 and they are not split),
+ * have them, and waves = 16: W4A8 products of 256 rows or more in 256 x 256 tiles wherever K >= 512 and they are not split),
  * 0/0 restores the heuristic; query the plan the library would use.  M > 128: that plan says what scratch the call
  * brings; omni_gemm_get_prefill_plan says which tiles run and whether they use it. */
 void omni_gemm_set_plan_override(int waves, int sk);
@@ -60,11 +60,12 @@ void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int* waves, in
 /* M > 128 (0 below), operands and output rows 16-byte aligned (others go to the general kernel).  mode: 0 per-channel W4A8, 1 per-group W4A8, 2 W8A8; slabs_only: omni_*_gemm_partial.
  * Returns 1 for the straight-line kernels: *mb 16-row blocks of a tile (16: the 256 x 256 tiles of W8A8), *kw K parts inside a
  * workgroup, *sk K slices that go through the scratch (1: none but slabs_only's own);
- * per-group: what runs where omni_gemm_prefill_group_tiles is 0.  2 for the general kernel (N % 256 or K % 256). */
+ * per-channel, per-group: what runs where omni_gemm_prefill_channel_tiles, omni_gemm_prefill_group_tiles are 0.  2 for the general kernel (N % 256 or K % 256). */
 int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int slabs_only, int* mb, int* kw, int* sk);
 /* 1 where omni_w4a8_per_group_gemm of these sizes runs in 256 x 256 tiles (csrc/qgemm_group_tiles.h), its operands aligned as above and its second-level scales and
- * zero points on whole dwords. */
+ * zero points on whole dwords; the other one: omni_w4a8_per_chn_gemm. */
 int omni_gemm_prefill_group_tiles(int M, int N, int K);
+int omni_gemm_prefill_channel_tiles(int M, int N, int K);
 /* 1 when the row-kernel-free decode forms below (omni_*_gemm_silu for gate_up [2*inter, hidden], omni_*_gemm_partial_f16
  * for o [hidden, attn_dim] and down [hidden, inter]) accept a layer of these dimensions at M rows, 0 otherwise: the plan
  * conditions those entry points check at launch, for a driver that picks its fusion level up front.

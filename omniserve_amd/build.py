@@ -26,7 +26,7 @@ OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libomniserve_hip.so")
 ARCH = "gfx950"
 SOURCES = ["qgemm_plan.hip", "qgemm_chn.hip", "qgemm_grp.hip", "qgemm_w8.hip", "qgemm_silu_rows.hip",
-           "elementwise.hip", "norm_rows.hip", "offpath.hip", "kv_cache.hip", "attn_prefill.hip", "sparse_utils.hip", "tp_comm.hip", "row_dtypes.hip", "norm_gemv_fused.hip",
+           "qgemm_chn_tiles.hip", "elementwise.hip", "norm_rows.hip", "offpath.hip", "kv_cache.hip", "attn_prefill.hip", "sparse_utils.hip", "tp_comm.hip", "row_dtypes.hip", "norm_gemv_fused.hip",
            "norm_product.hip", "act_product.hip", "head_product.hip"]
 # no packed-f32 instructions: some of their forms have returned wrong results on this hardware
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -1,4 +1,4 @@
-// Per-group W4A8 prefill GEMM in 256-row x 256-channel tiles: M >= 256, N % 256 == 0, K % 256 == 0, K >= 512.  (included by qgemm_grp.hip)
+// W4A8 prefill GEMM in 256-row x 256-channel tiles: M >= 256, N % 256 == 0, K % 256 == 0, K >= 512.  (included by qgemm_grp.hip, qgemm_chn_tiles.hip and qgemm_silu_rows.hip)
 //
 // What bounds w4a8_gemm_exact_kernel per-group is the second level: 5.5 operations (9.5 where a scale is above 17) for each word of four weights, done again for
 // every 64 - 128 rows, beside products that leave three issue slots each.  Here a wave has 64 channels and all 256 rows of the tile, so that a word is
@@ -17,6 +17,10 @@
 // The next tile's requests go out before the results are scaled, which wait in the accumulation registers (accumulators_stay): 2331 rows of 28672 x 4096 with the unit 291 -> 279 us, of 6144 x 4096
 // 59.5 -> 56.8, 6000 rows of 28672 x 4096 620 -> 600.
 //
+// Per-channel (MODE_CHN) there is no second level: a word is a shift and a mask, a stage has no parameters, and 64 products wait for nothing but their operands: 1.24 us a stage with all CUs at
+// work, 0.98 with few, where the package's power lets the clock be higher.  What it gains on w4a8_gemm_exact_kernel is operands brought in half as often, where its tiles fill whole rounds: us, 4000
+// rows of 4096 x 14336 162 -> 148 (3190 TOPS), of 28672 x 4096 with the unit 340 -> 331, of 8192 x 8192 188 -> 175, of 8192 x 28672 664 -> 572.
+//
 // SHARE: K of the last round's tiles shared out (tile_share.h).
 //
 // Integer sums and the general kernel's epilogue: the same bits.
@@ -25,7 +29,7 @@
 
 namespace omni {
 
-constexpr int GT_ACT = TILES_M * TILES_K, GT_W = TILES_N * TILES_K / 2, GT_PAR = 4 * 256, GT_STAGE = GT_ACT + GT_W + GT_PAR, GT_BUFS = 3;
+constexpr int GT_ACT = TILES_M * TILES_K, GT_W = TILES_N * TILES_K / 2, GT_PAR = 4 * 256, GT_BUFS = 3;
 
 // A word of four weights, u * scale + zero per byte, as the general form has it: the whole word's product, in which a byte's overflow goes into the next,
 // then four byte additions.  In full-rate operations, 6.5 a word where a quarter-rate multiplication and the additions one by one are 9.5, and without a
@@ -38,11 +42,14 @@ constexpr int GT_ACT = TILES_M * TILES_K, GT_W = TILES_N * TILES_K / 2, GT_PAR =
 
 // SILU: out = silu(gate) up of a [gate | up] weight, [M][N / 2]: of a wave's 64 channels the first 32 are gate channels, the others the up channels of the same place.  (2331 rows of
 // 28672 x 4096: the product takes 307 us either way, the quantiser behind it 31 -> 18.)
-template <bool SILU, bool SHARE>
-__global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, TileShare share) {
+template <int MODE, bool SILU, bool SHARE>
+__global__ __launch_bounds__(256, 1) void w4a8_tiles_kernel(GemmArgs p, TileShare share) {
+  static_assert(MODE == MODE_CHN || MODE == MODE_GRP, "packed weights");
+  constexpr bool GRP = MODE == MODE_GRP;
+  constexpr int GT_STAGE = GT_ACT + GT_W + (GRP ? GT_PAR : 0), PIECES = GRP ? 13 : 12;
   constexpr int PITCH = 64 * 2 + 16;                        // a row of the write-back buffers: a wave's 64 channels
-  constexpr int LDS_OUT = GT_BUFS * GT_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SC + 2 * 1024 + (SHARE ? 16 : 0)];
+  constexpr int LDS_OUT = GT_BUFS * GT_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH, SC = GRP ? 1024 : 2048;      // (SC: scales of 256 channels and 256 rows, CHN: zero points and sums too)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_SC + 2 * SC + (SHARE ? 16 : 0)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // (tile order: w8a8_tiles_kernel's)
   const int tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x & 7;
@@ -82,16 +89,16 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
   auto advance = [&]() __attribute__((always_inline)) {
     wbase += 4 * 512;
     abase += TILES_K;
-    par += p.N;
+    if constexpr (GRP) par += p.N;
   };
   auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 12; ++i) tiles_dma16(i < 8 ? src[i & 7] : wsrc[i & 3], i < 8 ? abase : wbase, dst(buf, i));
-    dma_params(buf);
+    if constexpr (GRP) dma_params(buf);
     advance();
   };
   int m0 = 0, n0 = 0, ns = all_stages;                      // ns: stages of the tile opened last
-  uint16_t sw_next = 0, sa_next = 0;                        // the thread's channel's and row's scales of the tile opened last
+  uint16_t sw_next = 0, sa_next = 0, sz_next = 0, as_next = 0;      // the thread's channel's and row's scales of the tile opened last; CHN: zero point and sum
   // (the last row tile starts at M - 256: the rows that it shares with the one before are computed twice, to the same bits)
   auto open_tile = [&]() __attribute__((always_inline)) {
     int k0 = 0;
@@ -112,9 +119,13 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     const int tid = 64 * wave + lane_here();
     // (lane l of 64 channels: the first of the wave's and, SILU, the other half's)
     auto channel = [&](int l) __attribute__((always_inline)) { return SILU ? n0 + 32 * wave + (l & 31) + (l >> 5) * (p.N >> 1) : n0 + 64 * wave + l; };
-    par = ((tid & 16) ? p.s2z : p.s2s) + (size_t)k0 * p.N + channel(4 * (tid & 15));
+    if constexpr (GRP) par = ((tid & 16) ? p.s2z : p.s2s) + (size_t)k0 * p.N + channel(4 * (tid & 15));
     sw_next = ((const uint16_t*)p.wscales)[channel(lane_here())];
     sa_next = ((const uint16_t*)p.ascales)[m0 + tid];
+    if constexpr (!GRP) {
+      sz_next = ((const uint16_t*)p.wsz)[channel(lane_here())];
+      as_next = ((const uint16_t*)p.asum)[m0 + tid];
+    }
     if constexpr (SHARE) {
       wbase = wave_uniform(wbase);
       abase = wave_uniform(abase);
@@ -125,9 +136,13 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
   };
   // ... its scales in LDS: 256 channels', 256 rows'
   auto park = [&](int parity) __attribute__((always_inline)) {
-    uint16_t* s = (uint16_t*)(lds + LDS_SC + 1024 * parity) + 64 * wave + lane_here();
+    uint16_t* s = (uint16_t*)(lds + LDS_SC + SC * parity) + 64 * wave + lane_here();
     s[0] = sw_next;
     s[256] = sa_next;
+    if constexpr (!GRP) {
+      s[512] = sz_next;
+      s[768] = as_next;
+    }
   };
 
   int off[2], woff = 0, poff = 0;                           // of a fragment of half u inside 16 rows; of a piece of the wave's weights; of its parameters
@@ -229,6 +244,36 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
   auto half = [&](auto hu, int same, int next, auto has_next, auto has_raw, auto dma) __attribute__((always_inline)) {
     constexpr int U = decltype(hu)::value;
     constexpr bool NEXT = decltype(has_next)::value, RAW = decltype(has_raw)::value, DMA = decltype(dma)::value;
+    if constexpr (!GRP) {      // (a group of four has five others)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        OMNI_GT_FENCE();
+        product(hu, 0, j);
+        if constexpr (NEXT) nibbles(j);
+        OMNI_GT_FENCE();
+        if (DMA && j < PIECES) product_dma(hu, 1, j, j, same);
+        else product(hu, 1, j);
+        if constexpr (NEXT) {
+          a[U ^ 1][block_of(j)][j & 3] = (int)gx;
+          if (j < 12 && j % 3 == 0) fetch_b(U ? next : same, IntTag<U ^ 1>{}, 12 + j / 3);
+        }
+        OMNI_GT_FENCE();
+        product(hu, 2, j);
+        if constexpr (NEXT) {
+          if (j < 12) fetch_b(U ? next : same, IntTag<U ^ 1>{}, j);
+          if (j == 6) turn(1);
+        }
+        OMNI_GT_FENCE();
+        product(hu, 3, j);
+        if constexpr (RAW) {
+          if (j == 8 || j == 9) fetch_raw(next, IntTag<U>{}, j - 8);
+          if (j == 14) turn(0);
+        }
+      }
+      OMNI_GT_FENCE();
+      if constexpr (DMA) advance();
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       OMNI_GT_FENCE();
@@ -301,9 +346,9 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
         c = (v4i){zero, zero, zero, zero};
         asm volatile("" : "+a"(c));                         // (here, not between the first products, behind whose writes hipcc would not wait)
       }
-    // stages 0 and 1 are there: of what was requested last -- a stage, or stores of the tile before -- 13 may still fly (let fly all 32 stores,
+    // stages 0 and 1 are there: of what was requested last -- a stage, or stores of the tile before -- 13 (CHN 12) may still fly (let fly all 32 stores,
     // a tile takes the same time)
-    asm volatile("s_waitcnt vmcnt(13)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
     __syncthreads();
     if constexpr (SHARE) {
       wbase = wave_uniform(wbase);
@@ -314,7 +359,7 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     for (int u = 0; u < 2; ++u) off[u] = (fl & 15) * TILES_K + (((4 * u + (fl >> 4)) ^ tiles_swizzle(fl & 15)) << 4);
     woff = 4096 * wave + ((fl >> 3) & 1) * 2048 + ((fl & 7) * 4 + (fl >> 4)) * 16;
     poff = 256 * wave + 4 * (fl & 15);
-    fetch_params(0);
+    if constexpr (GRP) fetch_params(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) fetch_raw(0, IntTag<0>{}, j);
 #pragma unroll
@@ -327,6 +372,11 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     for (int j = 0; j < 2; ++j) fetch_raw(0, IntTag<1>{}, j);
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
+      if constexpr (!GRP) {
+        nibbles(w);
+        a[0][block_of(w)][w & 3] = (int)gx;
+        continue;
+      }
       if ((w & 3) == 0) {
         scale(w);
         zero_point(w);
@@ -340,8 +390,10 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
       a[0][block_of(w)][w & 3] = to;
     }
     turn(0);
-    scale(0);
-    zero_point(0);
+    if constexpr (GRP) {
+      scale(0);
+      zero_point(0);
+    }
     int t = 0, buf = 0;
     do {                                                    // (at least once: zeros on a way around it would be kept beside the accumulators)
       step(buf, after(buf), BoolTag<true>{}, BoolTag<true>{});
@@ -357,13 +409,13 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     // the next tile's requests, then the results, which stay in the accumulation registers until they are stored (w8a8_tiles_kernel's arithmetic)
     const int el = lane_here(), e15 = el & 15, i0 = (el >> 4) * 4;
     const int chan = (i0 >> 3) * 32 + (i0 & 7);             // of block 0
-    const uint8_t* scales = lds + LDS_SC + 1024 * parity;
+    const uint8_t* scales = lds + LDS_SC + SC * parity;
     half_t* const out = p.out + (size_t)m0 * p.out_stride + n0 + (SILU ? 32 : 64) * wave;
     const TileParts mine = parts;
     bool opened = false;
     if constexpr (SHARE) {
       if (mine.shared()) {
-        const bool last = mine.finishes(share, lds + LDS_SC + 2 * 1024, acc, [&] {
+        const bool last = mine.finishes(share, lds + LDS_SC + 2 * SC, acc, [&] {
           opened = true;
           open = open_tile();
         });
@@ -379,14 +431,18 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
     auto store = [&](auto add) __attribute__((always_inline)) {
       constexpr bool ADD = decltype(add)::value;
       accumulators_stay(acc);
-      float sw[4][4];
+      float sw[4][4], sz[4][4];
+      auto channels = [&](int at, float (&to)[4][4]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint2 w = *(const uint2*)(scales + 2 * (64 * wave + chan + 8 * i));
-        const uint32_t wv[2] = {w.x, w.y};
+        for (int i = 0; i < 4; ++i) {
+          const uint2 w = *(const uint2*)(scales + at + 2 * (64 * wave + chan + 8 * i));
+          const uint32_t wv[2] = {w.x, w.y};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sw[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
-      }
+          for (int e = 0; e < 4; ++e) to[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+        }
+      };
+      channels(0, sw);
+      if constexpr (!GRP) channels(1024, sz);
       v4i x[16];                                            // ADD: of four blocks of rows
       uint2 h[2][4];                                        // [row block][channel block]
 #pragma unroll
@@ -396,6 +452,7 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
           accumulators_stay(acc);
         }
         const float sa = (float)*(const half_t*)(scales + 512 + 2 * (16 * j + e15));
+        const float as = GRP ? 0.f : (float)*(const half_t*)(scales + (GRP ? 0 : 1536) + 2 * (16 * j + e15));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           uint32_t hw[2];
@@ -403,7 +460,9 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
           for (int e = 0; e < 2; ++e) {
             const v4i& y = x[4 * (j & 3) + i];
             const int c0 = acc[i][j][2 * e] + (ADD ? y[2 * e] : 0), c1 = acc[i][j][2 * e + 1] + (ADD ? y[2 * e + 1] : 0);
-            v2f r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
+            v2f r;
+            if constexpr (GRP) r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
+            else r = (v2f){(float)c0 * sw[i][2 * e] * sa - sz[i][2 * e] * as, (float)c1 * sw[i][2 * e + 1] * sa - sz[i][2 * e + 1] * as};
             asm volatile("" : "+v"(r));
             hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
           }
@@ -446,14 +505,14 @@ __global__ __launch_bounds__(256, 1) void w4a8_group_tiles_kernel(GemmArgs p, Ti
 }
 
 // a workgroup per CU
-template <bool SILU>
-static void launch_group_tiles_as(GemmArgs b, const TileShare& share, hipStream_t st) {
+template <int MODE, bool SILU>
+static void launch_w4_tiles_as(GemmArgs b, const TileShare& share, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;
   b.tiles_m = (b.M + TILES_M - 1) / TILES_M;
   const int bands = (b.tiles_m + 3) / 4, tiles = b.tiles_m * b.tiles_n;
   b.tile_linear = (b.tiles_m + bands - 1) / bands;
-  if (share.sums) hipLaunchKernelGGL((w4a8_group_tiles_kernel<SILU, true>), dim3(256), dim3(256), 0, st, b, share);
-  else hipLaunchKernelGGL((w4a8_group_tiles_kernel<SILU, false>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b, share);
+  if (share.sums) hipLaunchKernelGGL((w4a8_tiles_kernel<MODE, SILU, true>), dim3(256), dim3(256), 0, st, b, share);
+  else hipLaunchKernelGGL((w4a8_tiles_kernel<MODE, SILU, false>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b, share);
 }
 
 }  // namespace omni

@@ -3,7 +3,7 @@
 #include "qgemm_group_tiles.h"
 using namespace omni;
 
-void omni::launch_group_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st) { launch_group_tiles_as<false>(a, share, st); }
+void omni::launch_group_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st) { launch_w4_tiles_as<MODE_GRP, false>(a, share, st); }
 
 extern "C" int omni_w4a8_per_group_gemm(const void* in_feats, const void* qweight, const void* zeros,
                                         const void* scales_i8, const void* wscales, const void* ascales,

@@ -1233,10 +1233,10 @@ extern "C" void omni_gemm_get_plan(int M, int N, int K, int kalign, int* mb, int
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred = false, bool w8 = false);
 
 // w4a8_gemm_exact_kernel's tile height (16-row blocks; 16: w8a8_tiles_kernel), K parts inside a workgroup, K slices over the grid (1: no
-// slabs); group_tiles: w4a8_group_tiles_kernel instead of all that; share: either of the 256 x 256 kernels, K of the last round's tiles shared out (tile_share.h)
+// slabs); w4_tiles: w4a8_tiles_kernel instead of all that; share: either of the 256 x 256 kernels, K of the last round's tiles shared out (tile_share.h)
 struct PrefillPlan {
   int mb, kw, sk;
-  bool group_tiles = false, share = false;
+  bool w4_tiles = false, share = false;
 };
 // sk: the K slices plan_gemm offers; slab_only: the caller wants that many slabs (omni_gemm_set_plan_override's K splits do, too)
 // scratch: there is memory for shared tiles
@@ -1285,8 +1285,9 @@ static void launch_tiles(GemmArgs b, const TileShare& share, hipStream_t st) {
   else hipLaunchKernelGGL((w8a8_tiles_kernel<MODE, SILU>), dim3(std::min(256, (tiles + 7) / 8 * 8)), dim3(256), 0, st, b, share);
 }
 
-// qgemm_grp.hip
+// qgemm_grp.hip, qgemm_chn_tiles.hip
 void launch_group_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st);
+void launch_chn_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st);
 // qgemm_plan.hip: the scratch that omni_gemm_arm_share left for this thread's next product
 TileShare take_armed_share();
 // qgemm_plan.hip: does omni_*_gemm_silu_rows take these sizes?  pp: its plan
@@ -1305,8 +1306,14 @@ static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, const TileShar
     }
     if constexpr (MODE == MODE_GRP) {
       // (a lane's parameters are four bytes)
-      if (pp.group_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
+      if (pp.w4_tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) == 0) {
         launch_group_tiles(a, pp.share ? share : TileShare{}, st);
+        return;
+      }
+    }
+    if constexpr (MODE == MODE_CHN) {
+      if (pp.w4_tiles) {
+        launch_chn_tiles(a, pp.share ? share : TileShare{}, st);
         return;
       }
     }

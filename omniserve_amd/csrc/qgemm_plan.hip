@@ -235,25 +235,30 @@ static float tiles_time(long long tiles, int stages) {
   return 3.f + (float)rounds * (8.f + 1.4f * (float)stages) + (rest > 0.f ? 8.f + (0.95f + 0.45f * rest * rest) * (float)stages : 0.f);
 }
 
-// w4a8_group_tiles_kernel: the same, a stage of 1.3 us where few CUs have a tile and 1.65 where all have one.  (MI355X, this kernel against the other's best: 8000 rows
+// w4a8_tiles_kernel, per-group: the same, a stage of 1.3 us where few CUs have a tile and 1.65 where all have one.  (MI355X, this kernel against the other's best: 8000 rows
 // of 8192 x 28672 1560 us / 1914, of 28672 x 4096 845 / 971, of 16384 x 1024 185 / 187, of 2048 x 512 21 / 20; 2331 rows of 4096 x 14336, 160 tiles, 178 / 192; 1800
 // rows of it, 128 tiles, 158 / 128; 1024 rows of 6144 x 4096, 96 tiles, 53 / 36.  Over 150 sizes of 257 - 8000 rows the rule takes 10 % less time than without
 // this kernel, the better of the two 10.2 %.)
-static float group_tiles_time(long long tiles, int stages) {
+static float w4_tiles_time(int mode, long long tiles, int stages) {
   const long long rounds = tiles / 256;
   const float rest = (float)(tiles - rounds * 256) / 256.f;
+  // per-channel: 0.98 and 1.24.  (MI355X, us, the best of w4a8_gemm_exact_kernel / here: 4096 rows of 4096 x 14336 162 / 149, of 28672 x 4096 346 / 328, 4000 of 8192 x 28672 664 / 572, of 8192 x 8192
+  // 188 / 175; 1280 of 28672 x 4096 118 / 133, 3000 of 6144 x 4096 65 / 86, 1500 of 4096 x 4096 26 / 42.)
+  if (mode == MODE_CHN) return (float)rounds * (9.f + 1.24f * (float)stages) + (rest > 0.f ? 9.f + (0.98f + 0.27f * rest * rest) * (float)stages : 0.f);
   return (float)rounds * (8.f + 1.65f * (float)stages) + (rest > 0.f ? 8.f + (1.3f + 0.35f * rest) * (float)stages : 0.f);
 }
 
-// The same with K of the last round's tiles shared out (the rounds in front of it as above): every CU at work for the stages of a head, and 17 us for a second part's sums and two more ends, 4 for each
+// The same with K of the last round's tiles shared out (the rounds in front of it as above): every CU at work for the stages of a head, and 17 us (per-channel 21) for a second part's sums and two more ends, 4 for each
 // part more.  1e30f: it has nothing
 // to share.  (MI355X, whole tiles / shared, us: per-group 2331 rows of 4096 x 14336, 20 tiles of an XCD, 181 / 152; 3000, 24 tiles, 181 / 164; 6000, 32 + 16, 342 / 300; 2331 of 28672 x 4096, 4 x 32 + 12, 284 / 278;
-// 1500, 2 x 32 + 20, 167 / 172, 3000 of 4096 x 4096, 24 tiles, 54 / 61.)
-static float shared_time(long long tiles, int stages, float stage) {
+// 1500, 2 x 32 + 20, 167 / 172, 3000 of 4096 x 4096, 24 tiles, 54 / 61; per-channel 3000 of
+// 4096 x 14336 137 / 128, 6000 265 / 237, 5000 264 / 209, 1000 of 8192 x 28672, 16 tiles, 241 / 165; 1501 of 28672 x 4096 with the unit, 2 x 32 + 20, 140 / 145.)
+static float shared_time(int mode, long long tiles, int stages) {
+  const float stage = mode == MODE_GRP ? 1.65f : mode == MODE_W8 ? 1.4f : 1.24f, ends = mode == MODE_CHN ? 9.f : 8.f, more = mode == MODE_CHN ? 21.f : 17.f;
   const int left = (int)((tiles + 7) / 8 % SHARE_PER);
   const ShareSplit sp = share_split(left, stages);
   if (left == 0 || sp.head == stages) return 1e30f;
-  return (float)((tiles + 7) / 8 / SHARE_PER) * (8.f + stage * (float)stages) + 17.f + 4.f * (float)(sp.used - left - 1) / (float)left + stage * (float)sp.head;
+  return (float)((tiles + 7) / 8 / SHARE_PER) * (ends + stage * (float)stages) + more + 4.f * (float)(sp.used - left - 1) / (float)left + stage * (float)sp.head;
 }
 
 PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, bool scratch) {
@@ -264,14 +269,14 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, 
   const float far = mode == MODE_W8 && K >= 8192 ? 1.2f : mode == MODE_CHN && K >= 16384 ? 1.17f : 1.f;
   // whole bands of 8 full row tiles go in an order of their own (w4a8_gemm_exact_kernel): 4096 rows of 8192 x 28672 per-channel 607 us, 632 with K in two
   // parts; 4096 of 10240 x 8192 per-group 336, 346 in tiles of 112 rows; 8192 of 5120 x 13824 546, 563
-  const float whole = mode != MODE_W8 && M % 1024 == 0 ? 0.96f : 1.f;
+  const float whole_bands = mode != MODE_W8 && M % 1024 == 0 ? 0.96f : 1.f;
   float time = 1e30f;
   auto offer = [&](int mb, int kw, int split) {
     const long long tiles = (long long)((M + 16 * mb - 1) / (16 * mb)) * (N / 256) * split;
     float t = grid_time(c, mb, kw, tiles, (split == 1 ? far : 1.f) * (float)(K / (split * KCHUNK)));
     // the slabs written, read and reduced by a launch of their own
     if (split > 1 && !slab_only) t += 4.5f + (float)split * M * N * 8.f / 4.5e6f;
-    if (mb == 8 && kw == 1 && split == 1) t *= whole;
+    if (mb == 8 && kw == 1 && split == 1) t *= whole_bands;
     if (t < time) { time = t; best = PrefillPlan{mb, kw, split}; }
   };
   for (int mb = 8; mb >= 4; --mb) {
@@ -283,14 +288,21 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, 
     if (K % (2 * KCHUNK) == 0) offer(mb, 2, 1);
     if (sk > 1) offer(mb, 1, sk);
   }
-  if (mode != MODE_CHN && !slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K) {
+  if (!slab_only && g_override_sk <= 0 && M >= TILES_M && K >= 4 * TILES_K) {
     const long long tiles = (long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N);
     const int stages = K / TILES_K;
-    const float whole = mode == MODE_W8 ? tiles_time(tiles, stages) : group_tiles_time(tiles, stages);
-    const bool take = mode == MODE_W8 ? whole < time : g_override_waves == 16 || whole < 0.98f * time;
-    const bool share = scratch && shared_time(tiles, stages, mode == MODE_W8 ? 1.4f : 1.65f) < (take ? whole : 0.93f * time) - 4.f;      // (the models' errors)
+    const float whole = mode == MODE_W8 ? tiles_time(tiles, stages) : w4_tiles_time(mode, tiles, stages);
+    // (the models' errors: per-channel the other kernel takes 1.05 - 1.15 of the time above where all CUs are at work, in whole bands of 8 row tiles too: 4096 rows of 4096 x 14336 136 us, in truth 162)
+    if (mode == MODE_CHN) {
+      const long long places = best.kw == 1 && best.sk == 1 ? 512 : 0, grid = (long long)((M + 16 * best.mb - 1) / (16 * best.mb)) * (N / 256);
+      const float busy = places ? (float)grid / (float)((grid + places - 1) / places * places) : 1.f;
+      if (best.mb == 8 && best.kw == 1 && best.sk == 1) time /= whole_bands;
+      time *= 1.f + 0.08f * std::max(0.f, (busy - 0.8f) / 0.2f);
+    }
+    const bool take = mode == MODE_W8 ? whole < time : g_override_waves == 16 || whole < (mode == MODE_GRP ? 0.98f : 0.985f) * time;      // (per-channel 1501 rows of 28672 x 4096, 0.994 here, 147 / 145 us in a prompt, whose step is no faster for it)
+    const bool share = scratch && shared_time(mode, tiles, stages) < (take ? whole : (mode == MODE_CHN ? 1.f : 0.93f) * time) - 4.f;
     if ((take || share) && mode == MODE_W8) best = PrefillPlan{16, 1, 1};
-    best.group_tiles = (take || share) && mode == MODE_GRP;
+    best.w4_tiles = (take || share) && mode != MODE_W8;
     best.share = share;
   }
   return best;
@@ -303,7 +315,7 @@ bool silu_rows_plan(int M, int N, int K, int mode, bool scratch, GemmPlan* pl, P
   *pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
   if (pl->midm || !exact_sizes(M, N, K, pl->kslice)) return false;
   *pp = plan_prefill(M, N, K, mode, pl->sk, false);
-  if (mode == MODE_W8 ? pp->mb != 16 : !pp->group_tiles && (pp->sk != 1 || pp->kw != 1)) return false;
+  if (mode == MODE_W8 ? pp->mb != 16 : !pp->w4_tiles && (pp->sk != 1 || pp->kw != 1)) return false;
   if (scratch) *pp = plan_prefill(M, N, K, mode, pl->sk, false, true);
   return true;
 }
@@ -345,16 +357,18 @@ extern "C" int omni_gemm_get_prefill_plan(int M, int N, int K, int mode, int sla
   return exact ? 1 : 2;
 }
 
-extern "C" int omni_gemm_prefill_group_tiles(int M, int N, int K) {
+static int prefill_w4_tiles(int M, int N, int K, int mode) {
   using namespace omni;
   if (M <= 128 || N < 64 || N % 64 || K < 64 || K % 64) return 0;
-  const GemmPlan pl = plan_gemm(M, N, K, 128, false, false);
-  return exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, MODE_GRP, pl.sk, false).group_tiles;
+  const GemmPlan pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, false);
+  return exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, mode, pl.sk, false).w4_tiles;
 }
+extern "C" int omni_gemm_prefill_group_tiles(int M, int N, int K) { return prefill_w4_tiles(M, N, K, omni::MODE_GRP); }
+extern "C" int omni_gemm_prefill_channel_tiles(int M, int N, int K) { return prefill_w4_tiles(M, N, K, omni::MODE_CHN); }
 
 extern "C" size_t omni_gemm_share_bytes(int M, int N, int K, int mode) {
   using namespace omni;
-  if (M < TILES_M || N < TILES_N || K < 4 * TILES_K || (mode != MODE_GRP && mode != MODE_W8)) return 0;
+  if (M < TILES_M || N < TILES_N || K < 4 * TILES_K || mode < MODE_CHN || mode > MODE_W8) return 0;
   const GemmPlan pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
   return !pl.midm && exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, mode, pl.sk, false, true).share ? SHARE_BYTES : 0;
 }

@@ -17,12 +17,10 @@ static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
   if constexpr (MODE == MODE_W8) {
     launch_tiles<MODE, true>(a, share, st);
   } else {
-    const bool tiles = pp.group_tiles;
-    if (tiles && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) != 0) return OMNI_EINVAL;
-    if constexpr (MODE == MODE_GRP) {
-      if (tiles) launch_group_tiles_as<true>(a, share, st);
-    }
-    if (!tiles) launch_exact_rows<MODE, 1, false, true>(a, pp.mb, 1, st);
+    const bool tiles = pp.w4_tiles;
+    if (tiles && MODE == MODE_GRP && ((reinterpret_cast<uintptr_t>(a.s2s) | reinterpret_cast<uintptr_t>(a.s2z)) & 3) != 0) return OMNI_EINVAL;
+    if (tiles) launch_w4_tiles_as<MODE, true>(a, share, st);
+    else launch_exact_rows<MODE, 1, false, true>(a, pp.mb, 1, st);
   }
   return omni_launch_status();
 }

@@ -74,7 +74,7 @@ inline int with_scratch(const GemmIO& g, const torch::Tensor& like, F call) {
   return rc;
 }
 
-// Scratch for a prompt's product whose last round's tiles share out their K (mode 1: per-group, 2: W8A8), from the caching allocator, in the order of the stream it is launched on: the tensor lives until
+// Scratch for a prompt's product whose last round's tiles share out their K (mode 0: per-channel, 1: per-group, 2: W8A8), from the caching allocator, in the order of the stream it is launched on: the tensor lives until
 // the launch.  Undefined where nothing is shared.
 inline torch::Tensor arm_share(const GemmIO& g, int mode, const torch::Tensor& like) {
   const size_t n = omni_gemm_share_bytes(g.M, g.N, g.K, mode);
@@ -89,6 +89,7 @@ void gemm_w4a8_per_chn(const torch::Tensor& in, const torch::Tensor& w, const to
   const GemmIO g = check_gemm_io(in, w, out, true);
   need_cuda(wscales, "gemm_forward"); need_cuda(ascales, "gemm_forward"); need_cuda(w_szs, "gemm_forward"); need_cuda(a_ssums, "gemm_forward");
   fail(with_scratch(g, in, [&](void* ws, size_t n) {
+         const torch::Tensor share = arm_share(g, 0, in);
          return omni_w4a8_per_chn_gemm(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), w_szs.data_ptr(), a_ssums.data_ptr(),
                                        out.data_ptr(), g.M, g.N, g.K, g.stride, ws, n, stream_of(in)); }),
        "qgemm_w4a8_per_chn.gemm_forward_cuda");
@@ -149,6 +150,7 @@ void gate_up_w4a8_per_chn(torch::Tensor out, const torch::Tensor& in, const torc
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows"); need_cuda(w_szs, "gate_up_rows"); need_cuda(a_ssums, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
+            const torch::Tensor share = arm_share(g, 0, in);
             return omni_w4a8_per_chn_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), w_szs.data_ptr(), a_ssums.data_ptr(),
                                                     gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w4a8_per_chn(in, w, wscales, ascales, w_szs, a_ssums, gu); });

@@ -1,9 +1,9 @@
-"""Prompts' per-group and W8A8 products whose last round's tiles share out their K (csrc/tile_share.h): one tile of an XCD and many, two parts of a tile and many, with and without whole
+"""Prompts' products whose last round's tiles share out their K (csrc/tile_share.h): one tile of an XCD and many, two parts of a tile and many, with and without whole
 rounds in front, parts of the fewest stages, row tiles that share rows.  Against the same product with whole tiles: the same bits, whatever the scratch holds, launch after launch."""
 import pytest
 import torch
 
-from tests.test_silu_rows_gpu import GRP, W8, _case
+from tests.test_silu_rows_gpu import CHN, GRP, W8, _case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -13,15 +13,16 @@ SIZES = [(GRP, 2331, 4096, 14336), (W8, 2331, 4096, 14336),           # 20, two 
          (W8, 2133, 8192, 28672), (GRP, 4200, 4096, 14336),           # 4 and 2 behind a whole round
          (GRP, 6000, 4096, 14336), (W8, 6000, 4096, 14336),           # 16 behind one: two
          (GRP, 3165, 4096, 14336), (W8, 3000, 4096, 28672),           # 26, 24: one workgroup has the ends of several tiles
-         (GRP, 1570, 5120, 13824), (W8, 653, 4096, 14336)]            # 18 (some XCDs 17), 6
-UNIT = [(GRP, 2331, 28672, 4096), (GRP, 1500, 16384, 8192), (W8, 2100, 16384, 16384)]
+         (GRP, 1570, 5120, 13824), (W8, 653, 4096, 14336),            # 18 (some XCDs 17), 6
+         (CHN, 2830, 4096, 28672), (CHN, 2140, 8192, 28672)]          # 24; 4 behind a whole round
+UNIT = [(CHN, 2600, 16384, 16384), (GRP, 2331, 28672, 4096), (GRP, 1500, 16384, 8192), (W8, 2100, 16384, 16384)]
 
 
 def _calls(mode, M, N, K, unit):
     from omniserve_amd import _lib
     h, (x, w, ops) = _lib.lib(), _case(M, N, K, mode)
     need = h.omni_gemm_share_bytes(M, N, K, mode)
-    fn = {(GRP, False): h.omni_w4a8_per_group_gemm, (W8, False): h.omni_w8a8_gemm, (GRP, True): h.omni_w4a8_per_group_gemm_silu_rows, (W8, True): h.omni_w8a8_gemm_silu_rows}[mode, unit]
+    fn = {(CHN, False): h.omni_w4a8_per_chn_gemm, (CHN, True): h.omni_w4a8_per_chn_gemm_silu_rows, (GRP, False): h.omni_w4a8_per_group_gemm, (W8, False): h.omni_w8a8_gemm, (GRP, True): h.omni_w4a8_per_group_gemm_silu_rows, (W8, True): h.omni_w8a8_gemm_silu_rows}[mode, unit]
     ws = torch.empty((max(h.omni_gemm_workspace_bytes(M, N, K), 1),), dtype=torch.uint8, device=DEV)
 
     def call(out, scratch=None):
@@ -84,5 +85,5 @@ def test_what_is_refused():
     h = _lib.lib()
     t = torch.empty((1 << 20,), dtype=torch.uint8, device=DEV)
     assert h.omni_gemm_arm_share(t.data_ptr(), t.numel()) != 0 and h.omni_gemm_arm_share(None, 0) == 0
-    for M, N, K, mode in ((2331, 4096, 14336, 0), (255, 4096, 14336, 1), (4000, 4096, 14336, 1), (2331, 4096, 512, 1), (2331, 4100, 14336, 2), (0, 0, 0, 1)):
+    for M, N, K, mode in ((2331, 4096, 14336, 3), (255, 4096, 14336, 1), (4000, 4096, 14336, 1), (2331, 4096, 512, 1), (2331, 4100, 14336, 2), (0, 0, 0, 1)):
         assert h.omni_gemm_share_bytes(M, N, K, mode) == 0
