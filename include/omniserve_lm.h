@@ -179,8 +179,9 @@ int lm_gemm_rows(const LmGemmPart* a, const LmGemmPart* b, int groups, const int
 int lm_gemm_chosen_ok(int groups, int n, int k, int tokens, int top, int epi);
 int lm_gemm_chosen(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* ids, int tokens, int top, int x_is_pairs, float scale, int epi,
                    int act, void* stream);
-/* lm_gemm_rows of one matrix whose K is cut into slices (lm_gemm_rows_scratch() > 0 for LM_EPI_ELEM; w and x at multiples of 16 bytes), without the addition of the
- * slices' sums [slices][rows][n]; y of the part is not written. */
+/* lm_gemm_rows of one matrix whose K is cut into slices, without the addition of the slices' sums [slices][rows][n]; y of the part is not written; w and x at multiples of 16 bytes.
+ * lm_gemm_sums_room: how many f32 the sums are (0: no slices).  Where lm_gemm_rows has slices, too (lm_gemm_rows_scratch() > 0 for LM_EPI_ELEM), they are its. */
+int64_t lm_gemm_sums_room(int n, int k, int rows);
 int lm_gemm_sums(const LmGemmPart* a, int rows, float* sums, void* stream);
 int lm_gemm_tiles(const LmGemmPart* a, const LmGemmPart* b, int groups, const int* perm, const int* off, const int* tiles,
                   int max_tiles, int rows_a, int rows_b, int x_div, float scale, int epi, int act, void* stream);

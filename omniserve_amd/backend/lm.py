@@ -69,6 +69,7 @@ PROTOTYPES = {
     "lm_gemm_chosen": (_i, [_PP, _PP, _i, _vp, _i, _i, _i, _f, _i, _i, _vp]),
     "lm_gemm_sums": (_i, [_PP, _i, _vp, _vp]),
     "lm_gemm_rows_scratch": (_i64, [_i, _i, _i, _i]),
+    "lm_gemm_sums_room": (_i64, [_i, _i, _i]),
     "lm_gemm_rows_channels": (_i, [_i] * 6 + [_c.POINTER(_i)]),
     "lm_gemm_rows": (_i, [_PP, _PP, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp]),
     "lm_gemm_tiles": (_i, [_PP, _PP, _i, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _vp]),
@@ -223,7 +224,7 @@ class LmOps:
     def sums(self, x, w):
         """x w^T for residual_norm: where few rows are multiplied in K slices, their f32 sums [slices, T, n] (residual_norm adds them up: a launch less), else matmul's rows"""
         T, (n, k) = x.shape[0], w.shape
-        room = self._h.lm_gemm_rows_scratch(n, k, T, EPI_ELEM) if T <= ROWS_MAX and (_p(x) | _p(w)) % 16 == 0 else 0
+        room = self._h.lm_gemm_sums_room(n, k, T) if T <= ROWS_MAX and (_p(x) | _p(w)) % 16 == 0 else 0
         if room == 0:
             return self.matmul(x, w)
         out = torch.empty((room // (T * n), T, n), dtype=torch.float32, device=x.device)

@@ -925,6 +925,25 @@ static RowsPlan plan_rows(int groups, int n, int k, int rows, int epi, bool expe
   return pl;
 }
 
+// ... of a product whose slices the norm behind it adds up (lm_gemm_sums): as lm_gemm_rows has them where those are slices; else slices too where whole K leaves a workgroup few channels, each of
+// which brings x in again, and they pay for what the norm reads: 1.5 us by the model, in one round of workgroups.  (MI355X, bf16, product and norm, whole K | slices, us: 4096 x 4096, 64 rows 18.1 | 15.4,
+// 48 16.8 | 14.9, 24 14.6 | 13.1; 2048 x 2048, 64 rows 11.8 | 10.2, 24 9.6 | 8.6, 16 8.6 | 8.1; 3072 x 3072, 48 rows 14.2 | 12.4; without the launch that adds up, 2048 x 4096, 48 rows 14.7 | 11.7.)
+static RowsPlan plan_sums(int n, int k, int rows) {
+  RowsPlan best = plan_rows(1, n, k, rows, LM_EPI_ELEM, false, true);
+#if LM_ELEM == 0
+  if (best.nw == 0 || best.slices > 1 || n < 2048) return best;
+  const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
+  auto stage = [&](int nw) { return 0.07f * nw + 0.02f * mb + 0.02f; };
+  float time = (float)((((n + 16 * best.nw - 1) / (16 * best.nw)) + 255) / 256) * (float)stages * stage(best.nw) - 1.5f;
+  for (int nw = 4; nw >= 1; nw /= 2)
+    for (int s = 2; s <= 4 && stages >= 8 * s && (n + 16 * nw - 1) / (16 * nw) * s <= 256; s *= 2) {
+      const float t = (float)((stages + s - 1) / s) * stage(nw) + (float)s * rows * n * 8.f / 5e6f;
+      if (t < time) { time = t; best = RowsPlan{nw, s}; }
+    }
+#endif
+  return best;
+}
+
 template <int EPI>
 static int launch_few(const GemmArgs& a, int max_rows, int has_b, float* part, hipStream_t s) {
   const bool one = a.groups == 1 && !a.perm && !has_b && max_rows <= 64 && max_rows == a.rows_a;
@@ -997,7 +1016,7 @@ extern "C" int lm_gemm_chosen(const LmGemmPart* pa, const LmGemmPart* pb, int gr
 extern "C" int lm_gemm_sums(const LmGemmPart* pa, int rows, float* sums, void* stream) {
   GemmArgs a;
   if (fill(a, pa, nullptr, 1, nullptr, nullptr, rows, 0, 1, 1.f, LM_EPI_ELEM, 0) || rows <= 0 || rows > 64 || !sums || ((uintptr_t)a.a.w | (uintptr_t)a.a.x) % 16) return LM_EINVAL;
-  const RowsPlan pl = plan_rows(1, a.a.n, a.a.k, rows, LM_EPI_ELEM, false, true);
+  const RowsPlan pl = plan_sums(a.a.n, a.a.k, rows);
   if (pl.nw == 0 || pl.slices < 2) return LM_EINVAL;
   return launch_stream<LM_EPI_ELEM>(a, 0, pl, sums, (hipStream_t)stream, true);
 }
@@ -1006,6 +1025,12 @@ extern "C" int64_t lm_gemm_rows_scratch(int n, int k, int rows, int epi) {
   if (n <= 0 || k <= 0 || rows <= 0 || rows > 64) return 0;
   const int s = plan_rows(1, n, k, rows, epi, false, true).slices;
   return s > 1 ? (int64_t)s * rows * n : 0;
+}
+
+extern "C" int64_t lm_gemm_sums_room(int n, int k, int rows) {
+  if (n <= 0 || k <= 0 || rows <= 0 || rows > 64) return 0;
+  const RowsPlan pl = plan_sums(n, k, rows);
+  return pl.nw > 0 && pl.slices > 1 ? (int64_t)pl.slices * rows * n : 0;
 }
 
 extern "C" int lm_gemm_rows_channels(int groups, int n, int k, int rows, int epi, int sliced, int* slices) {

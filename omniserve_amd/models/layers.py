@@ -269,6 +269,7 @@ class Norm:
 class Mixer:
     """What a mixer asks of the cache and the batch."""
     segment_workgroups = 0            # workgroups one segment of a prompt gives to the layer (0: it does not use segments)
+    to_norm = False                   # LmOps.residual_norm takes what it returns, and may add up K slices of its last product
 
     def cache_shape(self):
         """(kv heads, key size, value size) of its pages, None without"""
@@ -276,6 +277,9 @@ class Mixer:
 
     def state_shapes(self):
         return []
+
+    def project(self, o):
+        return (self.ops.sums if self.to_norm else self.ops.matmul)(o, self.w_out)
 
 
 class Attention(Mixer):
@@ -324,7 +328,7 @@ class Attention(Mixer):
                 part = torch.empty((b.n_decode * s.heads * nsplit * (self.dv + 2),), dtype=torch.float32, device=h.device)
             ops.attn_decode(x[n:], cut(first, n, None), self.lam, self.freq, b.pos[n:], b.kv_slot[n:], kv[0], kv[1],
                             b.block_table[b.n_entries:], cut(gate, n, None), o[n:], part, nsplit, s.scale, self.window, *heads)
-        return ops.matmul(o, self.w_out), v
+        return self.project(o), v
 
     def splits(self, b) -> int:
         """Parts of the visible keys per (sequence, kv head): enough workgroups for the 256 CUs, at least 128 keys each."""
@@ -368,7 +372,7 @@ class LinearAttention(Mixer):
         if b.n_decode:
             ops.linear_decode(x[n:], o[n:], state, b.state_slot, b.pos[n:], self.log2_decay, *size, s.activation)
         ops.gated_rms(o, o, x[:, self.g0:], self.norm, s.heads * s.vdim, self.eps)
-        return ops.matmul(o, self.w_out)
+        return self.project(o)
 
 
 class LatentAttention(Mixer):
@@ -435,7 +439,7 @@ class LatentAttention(Mixer):
             ops.latent_decode(xd, self.src, self.norm, self.eps, self.freq, b.pos[n:], b.kv_slot[n:], pool, b.block_table[b.n_entries:], qa, lat,
                               part, nsplit, s.scale, self.sizes)
             ops.head_products(lat, self.w_value, o[n:], self.Rp, self.dv, gate=xd[:, self.g0:])
-        return ops.matmul(o, self.w_out)
+        return self.project(o)
 
     def splits(self, b) -> int:
         """Parts of the keys per (sequence, 32 heads, as one workgroup or as two of 16): a workgroup per CU, two if each gets 1024 keys; at least 256 keys each (a part
@@ -484,7 +488,7 @@ class GatedLinearAttention(Mixer):
         if b.n_decode:
             ops.gla_decode(x[n:], o[n:], state, b.state_slot, b.pos[n:], self.low0, self.a2, self.bias, s.tau, scale, self.g0, self.norm,
                            s.vdim, self.eps, *size)
-        return ops.matmul(o, self.w_out)
+        return self.project(o)
 
 
 class DeltaRule(Mixer):
@@ -523,7 +527,7 @@ class DeltaRule(Mixer):
             ops.gated_head_rms(o[:n], o[:n], x[:n, self.g0:], self.norm, s.heads, self.dv, s.vdim, self.eps, "silu")
         if b.n_decode:
             ops.delta_decode(x[n:], o[n:], state, ring, b.state_slot, b.pos[n:], *rule, self.g0, self.norm, s.vdim, self.eps, *size)
-        return ops.matmul(o, self.w_out)
+        return self.project(o)
 
 
 class Dense:
@@ -592,6 +596,7 @@ class Layer:
                       MIXERS[type(spec.mixer)](spec.mixer, m, ops, width, eps))
         self.value_mix = getattr(spec.mixer, "value_mix", False)
         self.ff = FEED_FORWARDS[type(spec.ff)](spec.ff, w.under("mlp."), ops, width) if spec.ff else None
+        self.mixer.to_norm = not isinstance(self.ff, MixtureOfExperts)      # (in front of experts LmOps.norm_choose takes rows)
         # norms before / after the mixer and the feed-forward
         norm = lambda n: Norm(w, n, width, pad64(width), model.norm).pair      # noqa: E731
         names = {"around": ("norm1", "norm1b", "norm2", "norm2b"), "after": (None, "norm1", None, "norm2")}[model.placement]

@@ -33,3 +33,25 @@ def test_same_bits(T, n, k, real, dtype):
             out.append((x, h))
         torch.cuda.synchronize()
         assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), kw.keys()
+
+
+@pytest.mark.parametrize("T", [1, 17, 64])
+@pytest.mark.parametrize("n,k", [(4096, 4096), (2048, 2048), (8192, 8192)])
+def test_slices_that_the_product_alone_does_not_have(T, n, k):
+    """bf16 rows of f32 sums: within a rounding of either (2^-8 of it), and the norm's addition is the slices' one after the other"""
+    ops = lm_ops(torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(T + n)
+    w, a = (k ** -0.5 * torch.randn(n, k, generator=g, device="cuda")).bfloat16(), torch.randn(T, k, generator=g, device="cuda").bfloat16()
+    s = ops.sums(a, w)
+    assert s.dim() == 3 and (n == 8192 or ops._h.lm_gemm_rows_scratch(n, k, T, 0) == 0)
+    rows = s[0].clone()
+    for part in s[1:]:
+        rows += part
+    want = a.double() @ w.double().t()
+    assert (rows - want).norm() < 1e-6 * k ** 0.5 * want.norm()
+    out = []
+    for v in (rows.bfloat16(), s):
+        x, h = torch.ones((T, n), device="cuda"), torch.zeros((T, n), dtype=torch.bfloat16, device="cuda")
+        ops.residual_norm(x, n, "rms", 1e-5, y=v, next=(torch.ones(n, device="cuda"), None), h=h)
+        out.append((x, h))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
