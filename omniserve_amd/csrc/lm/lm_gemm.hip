@@ -794,6 +794,9 @@ static int launch_rows(const GemmArgs& a, int max_rows, int has_b, hipStream_t s
 // or 500 are two (heads and gated units; 28672 x 4096, 64 / 128 channels: 16 rows 42.3 / 37.1 us, 48 rows 48.3 / 39.9, 64 rows 51.8 / 41.5; 32000 x 4096, 80 / 128: 48 rows
 // 52.0 / 43.4; 32000 x 2048, 16 rows 25.4 / 22.9; two and four rounds of few rows and short K lose: 64000 x 2048 at 1 row 45.9 / 48.5, 128256 x 1024 43.1 / 46.7; 96 and
 // 112 channels nowhere the fastest).
+// Gated units (64 or 128 channels) of one round of 128: slices of several rounds cost 3.5 us a round more than that, two rounds of 64 channels have none, and 128 channels take 0.39 - 0.58 us a stage as they fill the chip.  (us, one | 64
+// rows, what the model without these two chose / now: 28672 x 4096, 4 slices, 48.8 / 36.0 at one row; 24576 x 4096, 2 slices, 43.6 / 31.1 | 51.0 / 37.4; 22016 x 4096, 8 slices, 43.3 / 29.3 | 47.5 /
+// 36.5; 10240 x 4096, 8 slices, 23.2 / 18.5; 5120 x 2048, 8 slices, 11.8 / 8.5.)
 struct RowsPlan {
   int nw, slices;      // nw 0: gemm_rows_kernel
 };
@@ -801,17 +804,23 @@ static RowsPlan plan_stream(int groups, int n, int k, int rows, bool glu, bool s
   RowsPlan best{4, 1};
   float time = 1e30f;
   const int stages = (int)((int64_t)k * (int)sizeof(elem_t) / RB), mb = min(4, (rows + 15) / 16);
+  const bool one_round = LM_ELEM == 0 && glu && (int64_t)groups * ((n + 127) / 128) <= 256;
   for (int nw = 5; nw >= 1; --nw) {
     if (glu && nw != 4) continue;                          // (a gate block and its up block share a workgroup)
     const int64_t tiles = (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw));
     for (int s = 1; s <= (sliced ? 8 : 1) && (s == 1 || stages >= 4 * s); s *= 2) {
       float t = (float)((tiles * s + 255) / 256) * (float)((stages + s - 1) / s) * (0.07f * nw + 0.02f * mb + 0.02f);
       if (s > 1) t += 4.5f + (float)s * rows * n * 8.f / 5e6f;
+      if (one_round && s > 1) t += tiles > 256 ? 1e30f : 3.5f * (float)((tiles * s - 1) / 256);
       if (t < time) { time = t; best = RowsPlan{nw, s}; }
     }
   }
-  // 128 channels only in place of workgroups that take K in one chain of stages, as they do: the same order of sums
   auto tiles = [&](int nw) { return (int64_t)groups * ((n + 16 * nw - 1) / (16 * nw)); };
+  // 128 channels only in place of workgroups that take K in one chain of stages, as they do: the same order of sums
+  if (one_round) {
+    if (best.slices == 1 && tiles(best.nw) > 256 && (float)stages * (0.19f + 0.39f * (float)tiles(8) / 256.f + 0.03f * (mb - 1)) + 2.5f < time) best.nw = 8;
+    return best;
+  }
   if (LM_ELEM == 0 && best.slices == 1 && tiles(best.nw) > 256 &&
       (float)((tiles(8) + 255) / 256) * ((float)stages * (0.07f * 8 + 0.02f * mb + 0.02f) + 2.f) + 0.5f < time)
     best.nw = 8;

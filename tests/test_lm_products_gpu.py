@@ -378,3 +378,14 @@ def test_gated_unit_of_many_rows_has_the_bits_of_product_and_unit(m, n, k):
     y, want = ops.matmul(x, w), torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
     ops._call("lm_glu", want.data_ptr(), n, y.data_ptr(), 2 * n, b.data_ptr(), m, n, 1)
     assert torch.equal(ops.glu(x, w, b, "silu"), want)
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(1, 28672, 4096, (128, 1)), (3, 20512, 2048, (128, 1)), (64, 24576, 4096, (128, 1)), (1, 16416, 1024, (128, 1)), (2, 10240, 4096, (64, 1)), (16, 5120, 2048, (64, 2))])
+def test_gated_unit_of_few_rows_in_wide_workgroups(m, n, k, plan):
+    """... of 64 channels in one round, of 128 where those are more; slices where they leave units idle"""
+    ops = _ops(torch.bfloat16)
+    assert _rows_plan(ops, 1, n, k, m, 2) == plan
+    x, w, b = _randn(71, torch.bfloat16, m, k), _randn(72, torch.bfloat16, n, k) * k ** -0.5, _randn(73, torch.float32, n) * 0.1
+    y = (x.double() @ w.double().t() + b.double()).view(m, n // 32, 2, 16)
+    want = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(m, n // 2)
+    assert errors(ops.glu(x, w, b, "silu").float().cpu().numpy(), want.cpu().numpy()).max() < TOL[torch.bfloat16]
