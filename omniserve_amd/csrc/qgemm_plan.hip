@@ -300,7 +300,8 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, 
       time *= 1.f + 0.08f * std::max(0.f, (busy - 0.8f) / 0.2f);
     }
     const bool take = mode == MODE_W8 ? whole < time : g_override_waves == 16 || whole < (mode == MODE_GRP ? 0.98f : 0.985f) * time;      // (per-channel 1501 rows of 28672 x 4096, 0.994 here, 147 / 145 us in a prompt, whose step is no faster for it)
-    const bool share = scratch && shared_time(mode, tiles, stages) < (take ? whole : (mode == MODE_CHN ? 1.f : 0.93f) * time) - 4.f;
+    // (in place of whole W8A8 tiles: by 18 us, which are faster than reckoned where two thirds of the CUs have one: 3000 rows of 4096 x 14336 141.4 / 142.5 shared, a whole prompt 3342 / 3402; 2331 129 / 130, 2100 150 / 123)
+    const bool share = scratch && shared_time(mode, tiles, stages) < (take ? whole - (mode == MODE_W8 ? 18.f : 4.f) : (mode == MODE_CHN ? 1.f : 0.93f) * time - 4.f);
     if ((take || share) && mode == MODE_W8) best = PrefillPlan{16, 1, 1};
     best.w4_tiles = (take || share) && mode != MODE_W8;
     best.share = share;
