@@ -1441,8 +1441,7 @@ static void launch_gemv(const GemmArgs& a, const GemmPlan& pl, hipStream_t st) {
 }
 
 template <int MODE>
-static int launch_gemm(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
-  const TileShare share = take_armed_share();
+static int launch_gemm(GemmArgs a, const TileShare& share, void* ws, size_t ws_bytes, hipStream_t st) {
   if (a.M < 1 || a.N % 64 != 0 || a.K % 64 != 0 || a.K < 64) return OMNI_EINVAL;
   if (MODE == MODE_GRP && a.K % 128 != 0) return OMNI_EINVAL;
   GemmPlan pl = plan_gemm(a.M, a.N, a.K, MODE == MODE_GRP ? 128 : 64, false, MODE == MODE_W8);

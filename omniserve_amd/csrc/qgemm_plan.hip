@@ -385,6 +385,8 @@ extern "C" int omni_gemm_arm_share(void* scratch, size_t bytes) {
   return OMNI_OK;
 }
 
+extern "C" int omni_gemm_share_armed(void) { return omni::g_armed_share.sums != nullptr; }
+
 // Would the row-kernel-free decode forms (omni_*_gemm_silu for gate_up, omni_*_gemm_partial_f16 for o / down) accept a layer
 // with these dimensions?  The same plan conditions launch_gemm_silu / launch_gemm_partial_f16 check at launch (one place to
 // keep in step: qgemm_kernel.h), so that a driver can choose its fusion level BEFORE its first step instead of running into

@@ -6,8 +6,7 @@ using namespace omni;
 
 // out = silu(gate) up fp16 [M, N/2], bit for bit what the product and silu_and_mul leave, in the products' own tiles.
 template <int MODE>
-static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
-  TileShare share = take_armed_share();
+static int launch_gemm_silu_rows(GemmArgs a, TileShare share, hipStream_t st) {
   GemmPlan pl;
   PrefillPlan pp;
   if (!silu_rows_plan(a.M, a.N, a.K, MODE, share.sums != nullptr, &pl, &pp)) return OMNI_EINVAL;
@@ -27,32 +26,35 @@ static int launch_gemm_silu_rows(GemmArgs a, hipStream_t st) {
 
 extern "C" int omni_w4a8_per_chn_gemm_silu_rows(const void* in_feats, const void* qweight, const void* wscales, const void* ascales, const void* w_szs,
                                                 const void* a_ssums, void* act_f16, int M, int N, int K, void* stream) {
+  const TileShare share = take_armed_share();             // (first: an early return must not leave it armed)
   if (!in_feats || !qweight || !wscales || !ascales || !w_szs || !a_ssums || !act_f16) return OMNI_EINVAL;
   GemmArgs a{};
   a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)qweight;
   a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
   a.wsz = (const half_t*)w_szs; a.asum = (const half_t*)a_ssums;
   a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_CHN>(a, (hipStream_t)stream);
+  return launch_gemm_silu_rows<MODE_CHN>(a, share, (hipStream_t)stream);
 }
 
 extern "C" int omni_w4a8_per_group_gemm_silu_rows(const void* in_feats, const void* qweight, const void* zeros, const void* scales_i8, const void* wscales,
                                                   const void* ascales, void* act_f16, int M, int N, int K, void* stream) {
+  const TileShare share = take_armed_share();             // (first: an early return must not leave it armed)
   if (!in_feats || !qweight || !zeros || !scales_i8 || !wscales || !ascales || !act_f16) return OMNI_EINVAL;
   GemmArgs a{};
   a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)qweight;
   a.s2s = (const uint8_t*)scales_i8; a.s2z = (const uint8_t*)zeros;
   a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
   a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_GRP>(a, (hipStream_t)stream);
+  return launch_gemm_silu_rows<MODE_GRP>(a, share, (hipStream_t)stream);
 }
 
 extern "C" int omni_w8a8_gemm_silu_rows(const void* in_feats, const void* weight, const void* wscales, const void* ascales, void* act_f16, int M, int N, int K,
                                         void* stream) {
+  const TileShare share = take_armed_share();             // (first: an early return must not leave it armed)
   if (!in_feats || !weight || !wscales || !ascales || !act_f16) return OMNI_EINVAL;
   GemmArgs a{};
   a.A = (const int8_t*)in_feats; a.W = (const uint8_t*)weight;
   a.wscales = (const half_t*)wscales; a.ascales = (const half_t*)ascales;
   a.out = (half_t*)act_f16; a.M = M; a.N = N; a.K = K; a.out_stride = N / 2;
-  return launch_gemm_silu_rows<MODE_W8>(a, (hipStream_t)stream);
+  return launch_gemm_silu_rows<MODE_W8>(a, share, (hipStream_t)stream);
 }

@@ -49,6 +49,19 @@ def test_invalid_arguments_are_rejected_without_a_gpu():
     assert h.omni_gemm_workspace_bytes(4096, 4096, 4096) == 0
 
 
+def test_refused_products_take_the_arming_of_scratch_back():
+    """... or a caller who frees the scratch after the error would leave its address armed for a later product of this thread"""
+    h = _lib.lib()
+    null = {"omni_w4a8_per_chn_gemm": 7, "omni_w4a8_per_group_gemm": 7, "omni_w8a8_gemm": 5}
+    for name, n in null.items():
+        for call, tail in ((getattr(h, name), (64, None, 0, None)), (getattr(h, name + "_silu_rows"), (None,))):
+            for operands in ((None,) * n, (16,) * (n - 1) + (None,), (None,) + (16,) * (n - 1), (16,) * n):      # (16 of everything: the sizes are refused)
+                assert h.omni_gemm_arm_share(1 << 20, 1 << 30) == 0 and h.omni_gemm_share_armed() == 1
+                assert call(*operands, 300, 100, 512, *tail) == -22
+                assert h.omni_gemm_share_armed() == 0, (name, operands)
+    assert h.omni_gemm_arm_share(1 << 20, 1 << 30) == 0 and h.omni_gemm_arm_share(None, 0) == 0 and h.omni_gemm_share_armed() == 0
+
+
 # reference module -> {function: number of positional parameters}  (kernels/csrc/**.h, SURVEY 2.1)
 REFERENCE_API = {
     "qgemm_w4a8_per_chn": {"gemm_forward_cuda": 7},
