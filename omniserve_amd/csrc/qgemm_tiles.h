@@ -21,7 +21,8 @@
 //    one's, so that the L2 has everything, 983 | 445; no requests at all 934 | 398; no LDS reads 1182 | 498); a line of the tile that is there anyway -> the lines ahead 1067 -> 1056 |
 //    516 -> 500, and of 28672 x 4096 in bands of four 1024 rows 113 -> 105, 2048 213 -> 200, in bands of three 1501 163 -> 157, 2100 217 -> 216; of 4096 x 14336 2100 166 -> 150, 2331 166 -> 131;
 //  * results stored -> streamed 1038 -> 1013 | 470 -> 461, accumulators zeroed -> not 1013 -> 996 | 460 -> 459.
-//  * the next tile requested behind -> before the scaling of the results, 30 sizes of 290 - 7900 rows, 1.009x on average (single rounds with the unit lose 1 %), 12001 rows 1047 -> 1043 | 491 -> 497.
+//  * the next tile requested behind -> before the scaling of the results: 0.99 of the time over 31 sizes without the unit (12001 rows of 6144 x 4096 246 -> 242, 4000 of 4096 x 4096 54.1 -> 52.3, 12001 of 4096 x 14336 482 -> 480;
+//    3700 of 6144 x 4096 92.1 -> 94.4, 7900 of 4096 x 4096 105.6 -> 107.0 are the slower ones); with the unit: launch_tiles.
 // What is left of the 5 POPS nominal is the clock under this load, the ends of a tile, which 4096 of K show, and the L2.
 #pragma once
 #include "lm/mfma_pinned.h"
@@ -48,10 +49,11 @@ __device__ __forceinline__ void tiles_dma16(uint32_t src, const void* base, uint
 // SILU: out = silu(gate) up of a [gate | up] weight, [M][N / 2]: rows 0 - 63 and 128 - 191 of a tile are 128 gate channels, the others the up channels of the same place, so that
 // a wave has both.  Half the stores pay for the exponentials; what it saves is the other half's way
 // through memory: 12001 rows of 28672 x 4096, the quantiser behind the product 156 -> 90 us, both 1.03x of a whole prompt.
-// SHARE: tile_share.h.
-template <int MODE, bool SILU = false, bool SHARE = false>
+// SHARE: tile_share.h.  LATE: the next tile is requested behind the scaling of this one's results, not in front of it (launch_tiles).
+template <int MODE, bool SILU = false, bool SHARE = false, bool LATE = false>
 __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShare share) {
   static_assert(MODE == MODE_W8, "rows of int8 weights");
+  static_assert(!(LATE && SHARE), "parts of a tile are left with the next part requested");
   constexpr int PITCH = 128 * 2 + 16;                       // a row of the write-back buffers: a wave's 128 channels
   // one object: the stages, four write-back buffers of 16 rows, the scales of two tiles
   constexpr int LDS_OUT = 2 * TILES_STAGE, LDS_SC = LDS_OUT + 4 * 16 * PITCH, LDS_SINK = LDS_SC + 2 * 1024;
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
     step(t, BoolTag<false>{}, BoolTag<false>{}, BoolTag<false>{});      // (behind its barrier both stages are free)
     accumulators_settle(acc);
 
-    // The next tile's requests, then the results, which stay in the accumulation registers until they are stored.  The arithmetic of the general kernel: both scales' product, the sum times it, each
+    // The next tile's requests, then the results, which stay in the accumulation registers until they are stored (LATE: the results packed, then the requests, then the stores).  The arithmetic of the general kernel: both scales' product, the sum times it, each
     // rounded to f32, then to fp16 -- opaque in between, or hipcc folds the last two into one rounding.
     const int el = lane_here(), e15 = el & 15, e4 = el >> 4;
     const uint8_t* sc = lds + LDS_SC + 1024 * parity;
@@ -247,8 +249,23 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
         }
       }
     }
-    if (!opened) open = open_tile();
+    if (!LATE && !opened) open = open_tile();
     uint8_t* buf = lds + LDS_OUT + wave * 16 * PITCH;
+    // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
+    auto put = [&](int j, const uint2 (&h)[8]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < (SILU ? 4 : 8); ++i) *(uint2*)(buf + e15 * PITCH + (16 * i + 4 * e4) * 2) = SILU ? silu_mul_h4(h[i], h[i + 4 & 7]) : h[i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < (SILU ? 2 : 4); ++i) {
+        const int r = SILU ? 8 * i + (el >> 3) : 4 * i + e4, q = SILU ? el & 7 : e15;
+        __builtin_nontemporal_store(*(const v4i*)(buf + r * PITCH + q * 16), (v4i*)(out + (size_t)(16 * j + r) * p.out_stride + q * 8));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
     auto store = [&](auto add) __attribute__((always_inline)) {
       constexpr bool ADD = decltype(add)::value;
       accumulators_stay(acc);
@@ -260,8 +277,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
 #pragma unroll
         for (int e = 0; e < 4; ++e) sw[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
       }
-      // through LDS, so that a row leaves in whole 16-byte pieces of neighbouring lanes: 16 rows of the wave's at a time
       v4i x[16];                                            // ADD: of two blocks of rows
+      uint2 packed[LATE ? 8 : 1][8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         if constexpr (ADD) if (j % 2 == 0) {
@@ -269,7 +286,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
           accumulators_stay(acc);
         }
         const float sa = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
-        uint2 h[8];
+        uint2 (&h)[8] = packed[LATE ? j : 0];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           typedef float v2f __attribute__((ext_vector_type(2)));
@@ -282,21 +299,17 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
             v2f r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
             asm volatile("" : "+v"(r));
             hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
+            if constexpr (LATE) asm volatile("" : "+v"(hw[e]));      // (converted here, not where it is stored: half the registers)
           }
           h[i] = make_uint2(hw[0], hw[1]);
         }
+        if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
+        else put(j, h);
+      }
+      if constexpr (LATE) {
+        open = open_tile();
 #pragma unroll
-        for (int i = 0; i < (SILU ? 4 : 8); ++i) *(uint2*)(buf + e15 * PITCH + (16 * i + 4 * e4) * 2) = SILU ? silu_mul_h4(h[i], h[i + 4 & 7]) : h[i];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < (SILU ? 2 : 4); ++i) {
-          const int r = SILU ? 8 * i + (el >> 3) : 4 * i + e4, q = SILU ? el & 7 : e15;
-          __builtin_nontemporal_store(*(const v4i*)(buf + r * PITCH + q * 16), (v4i*)(out + (size_t)(16 * j + r) * p.out_stride + q * 8));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < 8; ++j) put(j, packed[j]);
       }
     };
     if (SHARE && mine.shared()) store(BoolTag<SHARE>{});

@@ -38,7 +38,7 @@ SIZES = [(CHN, 1501, 28672, 4096, 8), (CHN, 1100, 24576, 512, True), (CHN, 700, 
          (CHN, 1024, 57344, 512, True), (CHN, 1500, 57344, 8192, 8), (GRP, 1500, 57344, 8192, "tiles"), (W8, 1500, 57344, 8192, 16),
          (GRP, 2331, 28672, 4096, "tiles"), (GRP, 2049, 14336, 2048, "tiles"), (GRP, 512, 28672, 4096, "tiles"), (GRP, 700, 16384, 256, 6), (GRP, 449, 16384, 256, 8), (GRP, 324, 12288, 256, 5), (GRP, 404, 12288, 256, 7),
          (GRP, 1025, 1024, 512, True),
-         (W8, 12001, 28672, 4096, 16), (W8, 2700, 28672, 1024, 16), (W8, 2305, 32768, 1024, 16), (W8, 1000, 12288, 2048, 16), (W8, 3000, 8192, 768, False), (W8, 300, 512, 768, False), (CHN, 128, 1024, 256, False), (GRP, 600, 768, 640, False)]
+         (W8, 12001, 28672, 4096, 16), (W8, 2700, 28672, 1024, 16), (W8, 2305, 32768, 1024, 16), (W8, 2048, 32768, 1536, 16), (W8, 2049, 32768, 1536, 16), (W8, 1000, 12288, 2048, 16), (W8, 3000, 8192, 768, False), (W8, 300, 512, 768, False), (CHN, 128, 1024, 256, False), (GRP, 600, 768, 640, False)]
 
 
 @pytest.mark.parametrize("mode,M,N,K,tiles", SIZES)
