@@ -74,12 +74,17 @@ inline int with_scratch(const GemmIO& g, const torch::Tensor& like, F call) {
   return rc;
 }
 
-// Scratch for a prompt's product whose last round's tiles share out their K (mode 0: per-channel, 1: per-group, 2: W8A8), from the caching allocator, in the order of the stream it is launched on: the tensor lives until
-// the launch.  Undefined where nothing is shared.
-inline torch::Tensor arm_share(const GemmIO& g, int mode, const torch::Tensor& like) {
+// Scratch for a prompt's product whose last round's tiles share out their K (mode 0: per-channel, 1: per-group, 2: W8A8; unit: with silu_and_mul), from the caching allocator, in the order of the
+// stream it is launched on: the tensor lives until the launch.  Undefined where nothing is shared, and where the device has no room for it: whole tiles need none and leave the same bits.
+inline torch::Tensor arm_share(const GemmIO& g, int mode, const torch::Tensor& like, bool unit = false) {
   const size_t n = omni_gemm_share_bytes(g.M, g.N, g.K, mode);
-  if (n == 0) return torch::Tensor();
-  torch::Tensor t = torch::empty({(int64_t)n}, torch::TensorOptions().dtype(torch::kUInt8).device(like.device()));
+  if (n == 0 || (unit && !omni_gemm_silu_rows_ok(g.M, g.N, g.K, mode))) return torch::Tensor();
+  torch::Tensor t;
+  try {
+    t = torch::empty({(int64_t)n}, torch::TensorOptions().dtype(torch::kUInt8).device(like.device()));
+  } catch (const c10::OutOfMemoryError&) {
+    return t;
+  }
   fail(omni_gemm_arm_share(t.data_ptr(), n), "gemm_forward");
   return t;
 }
@@ -150,7 +155,7 @@ void gate_up_w4a8_per_chn(torch::Tensor out, const torch::Tensor& in, const torc
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows"); need_cuda(w_szs, "gate_up_rows"); need_cuda(a_ssums, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
-            const torch::Tensor share = arm_share(g, 0, in);
+            const torch::Tensor share = arm_share(g, 0, in, true);
             return omni_w4a8_per_chn_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), w_szs.data_ptr(), a_ssums.data_ptr(),
                                                     gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w4a8_per_chn(in, w, wscales, ascales, w_szs, a_ssums, gu); });
@@ -163,7 +168,7 @@ void gate_up_w4a8_per_group(torch::Tensor out, const torch::Tensor& in, const to
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
-            const torch::Tensor share = arm_share(g, 1, in);
+            const torch::Tensor share = arm_share(g, 1, in, true);
             return omni_w4a8_per_group_gemm_silu_rows(in.data_ptr(), w.data_ptr(), zeros.data_ptr(), scales_i8.data_ptr(), wscales.data_ptr(), ascales.data_ptr(),
                                                       gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w4a8_per_group(in, w, zeros, scales_i8, wscales, ascales, gu); });
@@ -175,7 +180,7 @@ void gate_up_w8a8(torch::Tensor out, const torch::Tensor& in, const torch::Tenso
   need_cuda(wscales, "gate_up_rows"); need_cuda(ascales, "gate_up_rows");
   gate_up(g, in, out, gu, sum, scale,
           [&](void* st) {
-            const torch::Tensor share = arm_share(g, 2, in);
+            const torch::Tensor share = arm_share(g, 2, in, true);
             return omni_w8a8_gemm_silu_rows(in.data_ptr(), w.data_ptr(), wscales.data_ptr(), ascales.data_ptr(), gu.data_ptr(), g.M, g.N, g.K, st); },
           [&] { gemm_w8a8(in, w, wscales, ascales, gu); });
 }

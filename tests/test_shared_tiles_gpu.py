@@ -80,6 +80,34 @@ def test_mirror_takes_them_on_two_streams():
     assert all(torch.equal(o, want) for os in got for o in os)
 
 
+@pytest.mark.parametrize("unit", [False, True])
+def test_mirror_without_room_for_scratch(unit):
+    """A device filled up to a few megabytes, as its pages of keys and values may leave it: whole tiles, and no error"""
+    from omniserve_amd import _lib
+    from omniserve_amd.backend import fused_ext, qgemm_w4a8_per_group
+    assert _lib.fast() is not None
+    M, N, K = UNIT[1][1:] if unit else (2331, 4096, 14336)
+    need, call, out, (x, w, ops, ws) = _calls(GRP, M, N, K, False)
+    got, want = out(), call(out())
+    codes, scale = [torch.empty((M, N // 2), dtype=torch.int8, device=DEV) for _ in range(2)], [torch.empty((M,), dtype=torch.half, device=DEV) for _ in range(2)]
+    run = (lambda i: fused_ext.gate_up_rows(codes[i], x, w, ops, got, None, scale[i])) if unit else (lambda i: qgemm_w4a8_per_group.gemm_forward_cuda(x, w, *ops, got))
+    run(0)
+    assert need > 32 << 20
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            torch.empty((need,), dtype=torch.uint8, device=DEV)
+        got.fill_(7)
+        run(1)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    if unit:
+        assert torch.equal(*codes) and torch.equal(*scale) and codes[0].any()
+    else:
+        assert torch.equal(got, want)
+
+
 def test_what_is_refused():
     from omniserve_amd import _lib
     h = _lib.lib()
