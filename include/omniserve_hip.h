@@ -41,7 +41,7 @@ int omni_abi_version(void);
 size_t omni_gemm_workspace_bytes(int M, int N, int K);
 size_t omni_gemm_partial_workspace_bytes(int M, int N, int K);
 /* Prompts' per-channel (mode 0), per-group (1) and W8A8 (2) products, with or without silu_and_mul: scratch with which the last round's tiles share out their K, 0 where that gains nothing.  The
- * same bits with and without.  omni_gemm_arm_share: the next of these products that this thread enqueues may use the scratch (16-byte aligned, any contents), until it has run; any call of
+ * same bits with and without.  omni_gemm_arm_share: the next of these products that this thread enqueues may use the scratch (16-byte aligned, any contents; one of fewer bytes than it asks for is not used), until it has run; any call of
  * them, refused ones included, takes the arming back.  omni_gemm_share_armed: 1 while one is armed. */
 size_t omni_gemm_share_bytes(int M, int N, int K, int mode);
 int omni_gemm_arm_share(void* scratch, size_t bytes);

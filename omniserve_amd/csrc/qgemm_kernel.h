@@ -1293,14 +1293,16 @@ void launch_group_tiles(const GemmArgs& a, const TileShare& share, hipStream_t s
 void launch_chn_tiles(const GemmArgs& a, const TileShare& share, hipStream_t st);
 // qgemm_plan.hip: the scratch that omni_gemm_arm_share left for this thread's next product
 TileShare take_armed_share();
+// ... has it a place for every part of these sizes' last round?  Then it is laid out for them.
+bool share_fits(TileShare* s, int M, int N, int K);
 // qgemm_plan.hip: does omni_*_gemm_silu_rows take these sizes?  pp: its plan
 bool silu_rows_plan(int M, int N, int K, int mode, bool scratch, GemmPlan* pl, PrefillPlan* pp);
 
 // prefill regime (M > 128): chunked LDS staging, weights through L2
 template <int MODE>
-static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, const TileShare& share, hipStream_t st) {
+static void launch_prefill(const GemmArgs& a, const GemmPlan& pl, TileShare share, hipStream_t st) {
   if (exact_shape(a, false)) {
-    const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false, share.sums != nullptr);
+    const PrefillPlan pp = plan_prefill(a.M, a.N, a.K, MODE, pl.sk, false, share_fits(&share, a.M, a.N, a.K));
     if constexpr (MODE == MODE_W8) {
       if (pp.mb == 16) {
         launch_tiles<MODE>(a, pp.share ? share : TileShare{}, st);

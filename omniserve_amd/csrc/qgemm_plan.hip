@@ -41,6 +41,24 @@ TileShare take_armed_share() {
   g_armed_share = TileShare{};
   return s;
 }
+// of the XCDs with a tile more and of those without
+static int share_places_of(int M, int N, int K) {
+  const long long tiles = (long long)((M + TILES_M - 1) / TILES_M) * (N / TILES_N);
+  int places = 0;
+  for (const long long own : {tiles / 8, (tiles + 7) / 8}) {
+    const int left = (int)(own % SHARE_PER);
+    const ShareSplit sp = share_split(left, K / TILES_K);
+    if (left > 0 && sp.head < K / TILES_K) places = std::max(places, share_places(left, sp.used));
+  }
+  return places;
+}
+bool share_fits(TileShare* s, int M, int N, int K) {
+  if (!s->sums || N < TILES_N || K < TILES_K) return false;
+  const int places = share_places_of(M, N, K);
+  if (places == 0 || s->places < places) return false;
+  s->places = places;
+  return true;
+}
 
 GemmPlan plan_gemm(int M, int N, int K, int kalign, bool deferred, bool w8) {
   GemmPlan pl;
@@ -371,17 +389,19 @@ extern "C" size_t omni_gemm_share_bytes(int M, int N, int K, int mode) {
   using namespace omni;
   if (M < TILES_M || N < TILES_N || K < 4 * TILES_K || mode < MODE_CHN || mode > MODE_W8) return 0;
   const GemmPlan pl = plan_gemm(M, N, K, mode == MODE_GRP ? 128 : 64, false, mode == MODE_W8);
-  return !pl.midm && exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, mode, pl.sk, false, true).share ? SHARE_BYTES : 0;
+  return !pl.midm && exact_sizes(M, N, K, pl.kslice) && plan_prefill(M, N, K, mode, pl.sk, false, true).share ? SHARE_MARKS + (size_t)8 * share_places_of(M, N, K) * SHARE_PART : 0;
 }
 
 extern "C" int omni_gemm_arm_share(void* scratch, size_t bytes) {
   using namespace omni;
   g_armed_share = TileShare{};
   if (!scratch) return OMNI_OK;
-  if (bytes < SHARE_BYTES || (reinterpret_cast<uintptr_t>(scratch) & 15) != 0) return OMNI_EINVAL;
+  // (two parts of a tile on every XCD are the least)
+  if (bytes < SHARE_MARKS + (size_t)8 * 2 * SHARE_PART || (reinterpret_cast<uintptr_t>(scratch) & 15) != 0) return OMNI_EINVAL;
   static std::atomic<unsigned long long> launches{(unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count()};
-  g_armed_share = TileShare{static_cast<v4i*>(scratch), reinterpret_cast<unsigned long long*>(static_cast<char*>(scratch) + SHARE_SUMS),
-                            launches.fetch_add(1, std::memory_order_relaxed) << 8};
+  const size_t places = std::min<size_t>((bytes - SHARE_MARKS) / ((size_t)8 * SHARE_PART), 2 * SHARE_PER);
+  g_armed_share = TileShare{static_cast<v4i*>(scratch), reinterpret_cast<unsigned long long*>(static_cast<char*>(scratch) + 8 * places * SHARE_PART), launches.fetch_add(1, std::memory_order_relaxed) << 8,
+                            (int)places};
   return OMNI_OK;
 }
 

@@ -9,7 +9,7 @@ template <int MODE>
 static int launch_gemm_silu_rows(GemmArgs a, TileShare share, hipStream_t st) {
   GemmPlan pl;
   PrefillPlan pp;
-  if (!silu_rows_plan(a.M, a.N, a.K, MODE, share.sums != nullptr, &pl, &pp)) return OMNI_EINVAL;
+  if (!silu_rows_plan(a.M, a.N, a.K, MODE, share_fits(&share, a.M, a.N, a.K), &pl, &pp)) return OMNI_EINVAL;
   a.kslice = pl.kslice;
   if (!pp.share) share = TileShare{};
   if (!exact_shape(a, false)) return OMNI_EINVAL;

@@ -5,7 +5,7 @@
 // stages are as many as make both kinds of workgroups end together, a part beginning and leaving its sums counted as three and a half stages.  (Equal shares of everything from one end to the other, which
 // splits as many tiles: workgroups that work at different k find less of each other's operands in the L2, a stage of the per-group tiles takes 1.9 us instead of 1.65.)
 //
-// Whoever comes to a tile's mark last finishes it: the others leave their int32 sums (256 KB a part, 16 bytes a lane and piece) in a scratch buffer.  Nobody waits for anybody.
+// Whoever comes to a tile's mark last finishes it: the others leave their int32 sums (256 KB a part, 16 bytes a lane and piece) in a scratch buffer of up to 62 parts an XCD (share_places: 10 - 124 MB in all).  Nobody waits for anybody.
 //  * sums and marks are written and read at agent scope (sc1), past the XCDs' L2s and the CUs' L1s: a part's stores are through before its arrival.
 //  * a mark holds the launch's token and the number of arrivals.  Whatever else it holds counts as none, so that nobody clears it; a tile's last arrival leaves 0 in it, for a captured launch
 //    that runs again.
@@ -21,14 +21,15 @@
 namespace omni {
 
 struct TileShare {
-  v4i* sums;                       // [8 XCDs][64][64][256]; null: every tile whole
+  v4i* sums;                       // [8 XCDs][places][64][256]; null: every tile whole
   unsigned long long* marks;       // [8 XCDs][32]
   unsigned long long token;        // << 8
+  int places;                      // of an XCD's parts
 };
 constexpr int SHARE_PER = 32;                               // workgroups of an XCD
 constexpr int SHARE_COST2 = 7;                               // twice the stages that a part's ends are worth
 constexpr int SHARE_MIN = 4;                                // stages that a part has at least: the kernels' loops want them
-constexpr size_t SHARE_SUMS = (size_t)8 * 64 * 64 * 256 * 16, SHARE_BYTES = SHARE_SUMS + 8 * SHARE_PER * 8;
+constexpr int SHARE_PART = 64 * 256 * 16, SHARE_MARKS = 8 * SHARE_PER * 8;      // bytes of a part's sums and of all marks
 
 // How an XCD's last `left` tiles (1 .. 31) of ns stages are dealt: `used` workgroups, the first `left` of which take `head` stages of a tile each; head = ns: not shared.
 struct ShareSplit {
@@ -43,6 +44,9 @@ __host__ __device__ inline ShareSplit share_split(int left, int ns) {
   if (ns - head >= SHARE_MIN && left * (ns - head) >= 7 * (r.used - left)) r.head = head;      // (7: no two borders move to one place)
   return r;
 }
+// Places that the parts of an XCD's last `left` tiles lie in: share and tile number together are below used - 1 (a share and the next have one tile in common at most, so that the sum is another for
+// each part), the first stages' parts behind them.
+__host__ __device__ inline int share_places(int left, int used) { return used - 1 + left; }
 
 __device__ __forceinline__ const uint8_t* wave_uniform(const uint8_t* p) {
   const uint64_t v = (uint64_t)p;
@@ -101,10 +105,11 @@ struct TileParts {
     return true;
   }
   __device__ __forceinline__ bool shared() const { return lo >= 0; }
-  // where the part of the s-th of them lies in the scratch buffer, -1 the first stages' (a share and the next have one tile in common at most: s + rest is another for each part)
-  __device__ __forceinline__ uint32_t place(int s) const {
-    return __builtin_amdgcn_readfirstlane(((blockIdx.x & 7) * 64 + rest + (s < 0 ? 32 : s)) * (64 * 256 * 16));
+  // where the part of the s-th of them lies in the scratch buffer, -1 the first stages'
+  __device__ __forceinline__ uint32_t place(const TileShare& p, int s) const {
+    return __builtin_amdgcn_readfirstlane(((int)(blockIdx.x & 7) * p.places + rest + (s < 0 ? used - 1 : s)) * SHARE_PART);
   }
+  static __device__ __forceinline__ auto buffer(const TileShare& p) { return __builtin_amdgcn_make_buffer_rsrc(p.sums, 0, 8 * p.places * SHARE_PART, 0x00020000); }
   __device__ __forceinline__ int me() const { return k0 == 0 ? -1 : (int)(blockIdx.x >> 3) - left; }
 
   // A part's sums are in c: does this workgroup finish the tile, with what others() adds to them?  If not, or if that was not certain at first, other() has been called, which may request what the
@@ -119,8 +124,8 @@ struct TileParts {
     if (tid == 0) *word = __hip_atomic_load(mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (p.token | rivals);
     __syncthreads();
     if (!__builtin_amdgcn_readfirstlane(*word)) {
-      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(p.sums, 0, (int)SHARE_SUMS, 0x00020000);
-      const uint32_t mine = place(me());
+      const auto rsrc = buffer(p);
+      const uint32_t mine = place(p, me());
       accumulators_stay(c);
 #pragma unroll
       for (int i = 0; i < N; ++i)
@@ -145,16 +150,16 @@ struct TileParts {
   template <int M, class Number>
   __device__ __forceinline__ void others(const TileShare& p, Number number, v4i (&x)[M]) const {
     const int tid = threadIdx.x;
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(p.sums, 0, (int)SHARE_SUMS, 0x00020000);
+    const auto rsrc = buffer(p);
     auto piece = [&](uint32_t at, int q) { return __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, at + number(q) * 4096, 16); };
     // (the first of them is this one or another)
     int s = me() < 0 ? lo : -1;
-    uint32_t at = place(s);
+    uint32_t at = place(p, s);
 #pragma unroll
     for (int q = 0; q < M; ++q) x[q] = piece(at, q);
     for (s = max(s + 1, lo); s <= hi; ++s) {
       if (s == me()) continue;
-      at = place(s);
+      at = place(p, s);
       v4i y[M];
 #pragma unroll
       for (int q = 0; q < M; ++q) y[q] = piece(at, q);

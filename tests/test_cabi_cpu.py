@@ -62,6 +62,13 @@ def test_refused_products_take_the_arming_of_scratch_back():
     assert h.omni_gemm_arm_share(1 << 20, 1 << 30) == 0 and h.omni_gemm_arm_share(None, 0) == 0 and h.omni_gemm_share_armed() == 0
 
 
+def test_scratch_of_shared_rounds_is_sized_by_their_parts():
+    """marks of 2 KB and 256 KB for each of an XCD's parts: of `left` tiles for `used` workgroups, used - 1 + left at most"""
+    h = _lib.lib()
+    for M, N, K, mode, left, used in ((2791, 6144, 8192, 1, 1, 5), (2133, 8192, 28672, 2, 4, 20), (653, 4096, 14336, 2, 6, 30), (2331, 4096, 14336, 1, 20, 32), (1570, 5120, 13824, 1, 18, 32), (3165, 4096, 14336, 1, 26, 32)):
+        assert h.omni_gemm_share_bytes(M, N, K, mode) == 2048 + 8 * (used - 1 + left) * (256 << 10), (M, N, K)
+
+
 # reference module -> {function: number of positional parameters}  (kernels/csrc/**.h, SURVEY 2.1)
 REFERENCE_API = {
     "qgemm_w4a8_per_chn": {"gemm_forward_cuda": 7},

@@ -42,12 +42,16 @@ def test_parts_add_up_to_the_whole(mode, M, N, K, unit):
     assert need > 0
     want = call(out())
     assert torch.isfinite(want).all() and want.abs().sum() > 0
-    scratch = torch.randint(0, 256, (need,), dtype=torch.uint8, device=DEV)
+    room = torch.randint(0, 256, (need + 4096,), dtype=torch.uint8, device=DEV)
+    scratch, behind = room[:need], room[need:].clone()
     for fill in (None, 0, 255, None):      # what was there, and what the launch before left
         if fill is not None:
             scratch.fill_(fill)
         assert torch.equal(call(out(), scratch), want)
     assert torch.equal(call(out()), want)      # one launch an arming
+    assert torch.equal(room[need:], behind)
+    scratch.fill_(7)
+    assert torch.equal(call(out(), scratch[:-16]), want) and (scratch == 7).all()      # too few bytes: whole tiles
 
 
 def test_captured_launches_run_again():
