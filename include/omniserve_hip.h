@@ -42,10 +42,12 @@ size_t omni_gemm_workspace_bytes(int M, int N, int K);
 size_t omni_gemm_partial_workspace_bytes(int M, int N, int K);
 /* Prompts' per-channel (mode 0), per-group (1) and W8A8 (2) products, with or without silu_and_mul: scratch with which the last round's tiles share out their K, 0 where that gains nothing.  The
  * same bits with and without.  omni_gemm_arm_share: the next of these products that this thread enqueues may use the scratch (16-byte aligned, any contents; one of fewer bytes than it asks for is not used), until it has run; any call of
- * them, refused ones included, takes the arming back.  omni_gemm_share_armed: 1 while one is armed. */
+ * them, refused ones included, takes the arming back.  omni_gemm_share_armed: 1 while one is armed.  omni_gemm_share_parts: the parts of one XCD's `own` tiles of `stages` stages of 128, [.][7]:
+ * workgroup, tile, first stage, stages, place in the scratch (-1: a whole tile), and the first and last of the workgroups behind those with a tile of the last round that have parts of it; returns how many. */
 size_t omni_gemm_share_bytes(int M, int N, int K, int mode);
 int omni_gemm_arm_share(void* scratch, size_t bytes);
 int omni_gemm_share_armed(void);
+int omni_gemm_share_parts(int own, int stages, int* parts, int room);
 
 /* Tuning / introspection hooks (tests and bench sweeps; not used by the serving path):
  * override the decode-shape plan (waves per workgroup: 1 or 4; K splits; M > 128: K slices over the grid where the plan may

@@ -27,6 +27,7 @@ PROTOTYPES = {
     "omni_gemm_share_bytes": (_sz, [_i, _i, _i, _i]),
     "omni_gemm_arm_share": (_i, [_vp, _sz]),
     "omni_gemm_share_armed": (_i, []),
+    "omni_gemm_share_parts": (_i, [_i, _i, _vp, _i]),
     "omni_gemm_set_plan_override": (None, [_i, _i]),
     "omni_gemm_set_midm_override": (None, [_i, _i]),
     "omni_prefetch_arm_gemm": (_i, [_vp, _i, _i, _i, _i, _i, _i64, _i]),

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256, 1) void w4a8_tiles_kernel(GemmArgs p, TileShar
   const int own = (tiles >> 3) + (xcd < (tiles & 7)), first = xcd * (tiles >> 3) + min(xcd, tiles & 7);
   int at = blockIdx.x >> 3;
   const int all_stages = p.K / TILES_K;
-  TileParts parts(own, all_stages);                         // (SHARE)
+  TileParts parts(at, own, all_stages);                     // (SHARE)
 
   // a wave's part of a stage: 64 rows of the activations, 8 a piece (lane: row lane / 8, slot lane % 8), and its two tile rows of weights, 2 KB each
   uint32_t src[8], wsrc[4];

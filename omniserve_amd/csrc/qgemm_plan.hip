@@ -405,6 +405,21 @@ extern "C" int omni_gemm_arm_share(void* scratch, size_t bytes) {
   return OMNI_OK;
 }
 
+extern "C" int omni_gemm_share_parts(int own, int stages, int* parts, int room) {
+  using namespace omni;
+  if (own < 0 || stages < SHARE_MIN || stages > 1 << 16 || !parts) return OMNI_EINVAL;
+  int n = 0;
+  for (int wg = 0; wg < SHARE_PER; ++wg) {
+    TileParts p(wg, own, stages);
+    for (int at = wg; p.next(at); at += SHARE_PER, ++n) {
+      if (n == room) return OMNI_EINVAL;
+      const int part[7] = {wg, p.tile, p.k0, p.stages, p.shared() ? p.slot(p.me()) : -1, p.lo, p.hi};
+      std::copy(part, part + 7, parts + 7 * n);
+    }
+  }
+  return n;
+}
+
 extern "C" int omni_gemm_share_armed(void) { return omni::g_armed_share.sums != nullptr; }
 
 // Would the row-kernel-free decode forms (omni_*_gemm_silu for gate_up, omni_*_gemm_partial_f16 for o / down) accept a layer

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
   const int tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x & 7;
   const int own = (tiles >> 3) + (xcd < (tiles & 7)), first = xcd * (tiles >> 3) + min(xcd, tiles & 7);
   int at = blockIdx.x >> 3;
-  TileParts parts(own, p.K / TILES_K);                      // (SHARE)
+  TileParts parts(at, own, p.K / TILES_K);                  // (SHARE)
 
   // a wave's part of a stage: 64 rows of the weights and 64 of the activations, 8 a piece (lane: row lane / 8, slot lane % 8)
   uint32_t src[8];

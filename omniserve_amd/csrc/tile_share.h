@@ -54,28 +54,38 @@ __device__ __forceinline__ const uint8_t* wave_uniform(const uint8_t* p) {
   return (const uint8_t*)((uint64_t)hi << 32 | lo);
 }
 
+// (of a value that all lanes have)
+__host__ __device__ inline int wave_uniform(int v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_readfirstlane(v);
+#else
+  return v;
+#endif
+}
+
+// The parts of an XCD's wg-th workgroup (of SHARE_PER), one after the other.  How they are dealt is host code, too: omni_gemm_share_parts.
 struct TileParts {
-  int own, ns, left, whole, head, used, from, to;           // whole: tiles taken one by one; from, to: this workgroup's share of the last round's stages behind the first ones, tile after tile
+  int wg, own, ns, left, whole, head, used, from, to;       // whole: tiles taken one by one; from, to: this workgroup's share of the last round's stages behind the first ones, tile after tile
   int tile = 0, k0 = 0, stages = 0, rest = 0, lo = 0, hi = 0;      // the part opened last; rest: its tile among the last round's; lo .. hi: the workgroups behind the first `left` that have parts of it
 
-  __device__ __forceinline__ int border(int s) const {      // where the share of the s-th of them begins
+  __host__ __device__ __forceinline__ int border(int s) const {      // where the share of the s-th of them begins
     const int n = ns - head, x = s * left * n / (used - left), in = x % n;
     return in < SHARE_MIN ? x - in : n - in < SHARE_MIN ? x - in + n : x;
   }
-  __device__ __forceinline__ TileParts(int own_, int ns_) : own(own_), ns(ns_), left(own_ % SHARE_PER), whole(own_), head(ns_), used(0), from(0), to(0) {
+  __host__ __device__ __forceinline__ TileParts(int wg_, int own_, int ns_) : wg(wg_), own(own_), ns(ns_), left(own_ % SHARE_PER), whole(own_), head(ns_), used(0), from(0), to(0) {
     if (left == 0) return;
     const ShareSplit sp = share_split(left, ns);
     if (sp.head == ns) return;
     whole = own - left;
     used = sp.used;
     head = sp.head;
-    const int s = (int)(blockIdx.x >> 3) - left;
+    const int s = wg - left;
     if (s >= 0 && s < used - left) {
       from = border(s);
       to = border(s + 1);
     }
   }
-  __device__ __forceinline__ bool next(int at) {
+  __host__ __device__ __forceinline__ bool next(int at) {
     tile = at;
     k0 = 0;
     stages = ns;
@@ -90,7 +100,7 @@ struct TileParts {
       rest = from / n;
       tile = whole + rest;
       k0 = from - rest * n;
-      stages = min(n - k0, to - from);
+      stages = n - k0 < to - from ? n - k0 : to - from;
       k0 += head;
       from += stages;
     }
@@ -101,16 +111,17 @@ struct TileParts {
     while (border(lo + 1) <= rest * n) ++lo;
     hi = lo;
     while (border(hi + 1) < (rest + 1) * n) ++hi;
-    lo = __builtin_amdgcn_readfirstlane(lo), hi = __builtin_amdgcn_readfirstlane(hi), from = __builtin_amdgcn_readfirstlane(from);
+    lo = wave_uniform(lo), hi = wave_uniform(hi), from = wave_uniform(from);
     return true;
   }
-  __device__ __forceinline__ bool shared() const { return lo >= 0; }
+  __host__ __device__ __forceinline__ bool shared() const { return lo >= 0; }
   // where the part of the s-th of them lies in the scratch buffer, -1 the first stages'
+  __host__ __device__ __forceinline__ int slot(int s) const { return rest + (s < 0 ? used - 1 : s); }
   __device__ __forceinline__ uint32_t place(const TileShare& p, int s) const {
-    return __builtin_amdgcn_readfirstlane(((int)(blockIdx.x & 7) * p.places + rest + (s < 0 ? used - 1 : s)) * SHARE_PART);
+    return __builtin_amdgcn_readfirstlane(((int)(blockIdx.x & 7) * p.places + slot(s)) * SHARE_PART);
   }
   static __device__ __forceinline__ auto buffer(const TileShare& p) { return __builtin_amdgcn_make_buffer_rsrc(p.sums, 0, 8 * p.places * SHARE_PART, 0x00020000); }
-  __device__ __forceinline__ int me() const { return k0 == 0 ? -1 : (int)(blockIdx.x >> 3) - left; }
+  __host__ __device__ __forceinline__ int me() const { return k0 == 0 ? -1 : wg - left; }
 
   // A part's sums are in c: does this workgroup finish the tile, with what others() adds to them?  If not, or if that was not certain at first, other() has been called, which may request what the
   // next part needs.

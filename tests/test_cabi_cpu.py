@@ -1,6 +1,7 @@
 """CPU-side checks of the drop-in boundary: the library builds/loads and exports exactly the
 symbols include/omniserve_hip.h declares; the Python mirror has the reference's module and
 function names and arities.  No compute calls (no GPU here)."""
+import ctypes
 import inspect
 import os
 import re
@@ -67,6 +68,39 @@ def test_scratch_of_shared_rounds_is_sized_by_their_parts():
     h = _lib.lib()
     for M, N, K, mode, left, used in ((2791, 6144, 8192, 1, 1, 5), (2133, 8192, 28672, 2, 4, 20), (653, 4096, 14336, 2, 6, 30), (2331, 4096, 14336, 1, 20, 32), (1570, 5120, 13824, 1, 18, 32), (3165, 4096, 14336, 1, 26, 32)):
         assert h.omni_gemm_share_bytes(M, N, K, mode) == 2048 + 8 * (used - 1 + left) * (256 << 10), (M, N, K)
+
+
+def _parts(h, own, stages):
+    room = (ctypes.c_int * (7 * 256))()
+    n = h.omni_gemm_share_parts(own, stages, room, 256)
+    assert n >= 0
+    return [tuple(room[7 * i:7 * i + 7]) for i in range(n)]
+
+
+@pytest.mark.parametrize("left", range(1, 32))
+def test_parts_of_a_shared_round_make_up_its_tiles(left):
+    """Every tile's stages once, in parts of four and more, each with a place of its own, its parts among the workgroups that are counted on: those of `lo .. hi` and the one with its first stages"""
+    h, shared = _lib.lib(), 0
+    for stages in list(range(4, 200)) + [224, 255, 256, 383, 448, 512, 1001]:
+        tiles, slots, used = {}, [], set()
+        for wg, tile, k0, n, slot, lo, hi in _parts(h, 64 + left, stages):
+            tiles.setdefault(tile, []).append((k0, n, wg, lo, hi))
+            if slot >= 0:
+                slots.append(slot)
+                used.add(wg)
+        assert sorted(tiles) == list(range(64 + left))
+        assert len(slots) == len(set(slots)) and all(0 <= s < max(used) + 1 - 1 + left for s in slots)
+        shared += bool(slots)
+        for tile, parts in tiles.items():
+            parts.sort()
+            assert parts[0][0] == 0 and sum(n for _, n, *_ in parts) == stages and all(a[0] + a[1] == b[0] for a, b in zip(parts, parts[1:]))
+            if len(parts) == 1:
+                assert tile < 64 or not slots
+                continue
+            assert tile >= 64 and min(n for _, n, *_ in parts) >= 4
+            assert parts[0][2] == tile - 64 and [left + s for s in range(parts[0][3], parts[0][4] + 1)] == [p[2] for p in parts[1:]]
+            assert len({p[3:] for p in parts}) == 1
+    assert shared
 
 
 # reference module -> {function: number of positional parameters}  (kernels/csrc/**.h, SURVEY 2.1)
