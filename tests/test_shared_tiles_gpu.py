@@ -1,8 +1,10 @@
 """Prompts' products whose last round's tiles share out their K (csrc/tile_share.h): one tile of an XCD and many, two parts of a tile and many, with and without whole
-rounds in front, parts of the fewest stages, row tiles that share rows.  Against the same product with whole tiles: the same bits, whatever the scratch holds, launch after launch."""
+rounds in front, parts of the fewest stages, row tiles that share rows.  Against the same product with whole tiles: the same bits, whatever the scratch holds, launch after launch, and the
+scratch shows which of them it was."""
 import pytest
 import torch
 
+from tests.test_cabi_cpu import _parts
 from tests.test_silu_rows_gpu import CHN, GRP, W8, _case
 
 pytestmark = pytest.mark.gpu
@@ -14,8 +16,24 @@ SIZES = [(GRP, 2331, 4096, 14336), (W8, 2100, 4096, 14336),           # 20, 18, 
          (GRP, 6000, 4096, 14336), (W8, 6000, 4096, 14336),           # 16 behind one: two
          (GRP, 3165, 4096, 14336), (W8, 3000, 4096, 28672),           # 26, 24: one workgroup has the ends of several tiles
          (GRP, 1570, 5120, 13824), (W8, 653, 4096, 14336),            # 18 (some XCDs 17), 6
+         (W8, 513, 4608, 12800), (CHN, 1025, 7680, 16384),            # 7 and 6, 19 and 18; parts of four stages, as in 1570 rows above
          (CHN, 2830, 4096, 28672), (CHN, 2140, 8192, 28672)]          # 24; 4 behind a whole round
-UNIT = [(CHN, 2600, 16384, 16384), (GRP, 2331, 28672, 4096), (GRP, 1500, 16384, 8192), (W8, 2100, 16384, 16384)]
+UNIT = [(CHN, 2600, 16384, 16384), (GRP, 2331, 28672, 4096), (GRP, 1500, 16384, 8192), (W8, 2100, 16384, 16384),
+        (W8, 513, 26624, 8192), (CHN, 1025, 10240, 16384)]           # parts of four stages, as in 2331 rows
+
+
+def _left(M, N, K):
+    """Tiles of each XCD's last round that are shared out"""
+    from omniserve_amd import _lib
+    tiles = (M + 255) // 256 * (N // 256)
+    return [len({p[1] for p in _parts(_lib.lib(), tiles // 8 + (x < tiles % 8), K // 128) if p[4] >= 0}) for x in range(8)]
+
+
+def _shared(scratch, M, N, K):
+    """Has a launch with shared tiles been over these bytes of 255?  Sums lie in them, and every shared tile's mark is 0 again"""
+    marks, left = scratch[-2048:].view(torch.int64).view(8, 32).cpu(), _left(M, N, K)
+    assert any(left)
+    return bool((scratch[:-2048] != 255).any()) and all((marks[x, :n] == 0).all() and (marks[x, n:] == -1).all() for x, n in enumerate(left))
 
 
 def _calls(mode, M, N, K, unit):
@@ -48,9 +66,10 @@ def test_parts_add_up_to_the_whole(mode, M, N, K, unit):
         if fill is not None:
             scratch.fill_(fill)
         assert torch.equal(call(out(), scratch), want)
-    assert torch.equal(call(out()), want)      # one launch an arming
+        assert fill != 255 or _shared(scratch, M, N, K)
     assert torch.equal(room[need:], behind)
     scratch.fill_(7)
+    assert torch.equal(call(out()), want) and (scratch == 7).all()      # one launch an arming
     assert torch.equal(call(out(), scratch[:-16]), want) and (scratch == 7).all()      # too few bytes: whole tiles
 
 
@@ -65,14 +84,17 @@ def test_captured_launches_run_again():
         call(got, scratch)
     for _ in range(4):
         got.fill_(7)
+        scratch.fill_(255)
         g.replay()
-        assert torch.equal(got, want)
+        assert torch.equal(got, want) and _shared(scratch, 2331, 4096, 14336)
         assert torch.equal(call(out(), scratch), want)
 
 
 def test_mirror_takes_them_on_two_streams():
     """The functions that allocate the scratch themselves, side by side"""
+    from omniserve_amd import _lib
     from omniserve_amd.backend import qgemm_w4a8_per_group
+    assert _lib.fast() is not None      # (the functions in Python alone take whole tiles)
     need, call, out, (x, w, ops, ws) = _calls(GRP, 2331, 4096, 14336, False)
     want, streams, got = call(out()), [torch.cuda.Stream(), torch.cuda.Stream()], [[out() for _ in range(6)] for _ in range(2)]
     torch.cuda.synchronize()
@@ -82,6 +104,31 @@ def test_mirror_takes_them_on_two_streams():
                 qgemm_w4a8_per_group.gemm_forward_cuda(x, w, *ops, o[i])
     torch.cuda.synchronize()
     assert all(torch.equal(o, want) for os in got for o in os)
+
+
+@pytest.mark.parametrize("mode,M,N,K,unit", [(GRP, 2331, 4096, 14336, False), (W8, 2100, 4096, 14336, False), (CHN, 1025, 7680, 16384, False),
+                                             (GRP, 2331, 28672, 4096, True), (W8, 513, 26624, 8192, True), (CHN, 1025, 10240, 16384, True)])
+@pytest.mark.parametrize("native", [True, False])
+def test_mirror_arms_its_scratch(mode, M, N, K, unit, native, monkeypatch):
+    """... where the compiled binding is there: the block that the caching allocator gives it is the one freed in front of the call.  The functions in Python alone take whole tiles"""
+    from omniserve_amd import _lib
+    from omniserve_amd.backend import fused_ext, qgemm_w4a8_per_chn, qgemm_w4a8_per_group, qgemm_w8a8
+    assert _lib.fast() is not None
+    if not native:
+        monkeypatch.setattr(_lib, "USE_EXT", False)
+    need, call, out, (x, w, ops, ws) = _calls(mode, M, N, K, False)
+    product = (qgemm_w4a8_per_chn.gemm_forward_cuda, qgemm_w4a8_per_group.gemm_forward_cuda, qgemm_w8a8.w8a8_gemm_forward_cuda)[mode]
+    got, codes, scale, sums = out(), torch.empty((M, N // 2), dtype=torch.int8, device=DEV), torch.empty((M,), dtype=torch.half, device=DEV), torch.empty((M,), dtype=torch.half, device=DEV)
+    run = (lambda: fused_ext.gate_up_rows(codes, x, w, ops, got, sums if mode == CHN else None, scale)) if unit else (lambda: product(x, w, *ops, got))
+    run()
+    torch.cuda.empty_cache()
+    scratch = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    place = scratch.data_ptr()
+    del scratch
+    run()
+    scratch = torch.empty((need,), dtype=torch.uint8, device=DEV)
+    assert scratch.data_ptr() == place
+    assert _shared(scratch, M, N, K) if native else (scratch == 255).all()
 
 
 @pytest.mark.parametrize("unit", [False, True])
