@@ -134,7 +134,7 @@ int lm_delta_decode(const void* x, int64_t ld, void* o, int64_t ldo, float* stat
                     int64_t g_col, const float* w, int n, float eps, int B, int H, int G, int dk, int dv, void* stream);
 
 /* z [tokens][ldz] f32 router logits -> wts [tokens][top], off [experts + 1], perm [tokens * top] (pairs sorted by expert);
- * with tiles: [lm_route_max_tiles][4] (expert, first place, rows, 0) of every row tile, past the last (0, 0, 0, number of tiles). */
+ * with tiles: [lm_route_max_tiles][4] (expert, first place, rows, 0) of every row tile, past the last (0, 0, 0, number of tiles; 0 there: lm_gemm_tiles goes through all). */
 int64_t lm_route_scratch_words(int tokens, int experts, int top);
 int lm_route_max_tiles(int tokens, int experts, int top);
 int lm_route(const float* z, int64_t ldz, const float* bias, int tokens, int experts, int top, float* wts, int* off, int* perm,

@@ -32,7 +32,7 @@ struct GemmArgs {
   const int* off;             // [groups + 1] sorted places of each group; chosen form (perm null): the expert of each of rows_a (token, choice) pairs
   int rows_a, rows_b;
   int x_div;                  // x row = y row / x_div (tokens of (token, choice) pairs)
-  const int* tiles;           // lm_gemm_tiles with perm: (group, first place, rows, 0) of every row tile, rows 0: none
+  const int* tiles;           // lm_gemm_tiles with perm: (group, first place, rows, 0) of every row tile, behind them (0, 0, 0, how many; 0: not said)
   float scale;
   int act;                    // of the gated unit
 };

@@ -248,6 +248,37 @@ def test_experts_in_turn(tokens, E, top, n, k, channels, glu, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("n,k", [(12288, 64), (12288, 192), (4096, 512)])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("empty,says", [(0, 0), (3, 14), (3, 0)])
+def test_tables_of_experts_rows(empty, says, glu, n, k, dtype):
+    """Whole tiles of a table without an entry to spare, with empty ones that say how many tiles there are, and with empty ones that do not; tiles of 1, 128 and 129 rows among them"""
+    ops, counts = _ops(dtype), [256, 129, 1100, 1, 128, 1025]
+    off, tiles = [0], []
+    for e, c in enumerate(counts):
+        tiles += [(e, off[-1] + r, min(256, c - r), 0) for r in range(0, c, 256)]
+        off.append(off[-1] + c)
+    assert len(tiles) == 14
+    tiles += [(0, 0, 0, says)] * empty
+    assert _channels(ops, n, k, len(counts), len(tiles)) == 256
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+    perm = torch.randperm(off[-1], generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).int()
+    x, w = _randn(41, dtype, off[-1], k), _randn(42, dtype, len(counts), n, k) * k ** -0.5
+    y = torch.full((off[-1] + 2, n // 2 if glu else n), 7.0, dtype=dtype, device=DEV)
+    ops.grouped((i32(off), perm, i32(tiles), len(tiles), 1), 0, x, w, y[1:-1], True, glu)
+    assert (y[0] == 7).all() and (y[-1] == 7).all()
+    want = torch.empty(y[1:-1].shape, dtype=torch.float64, device=DEV)
+    for e in range(len(counts)):
+        rows = perm[off[e]:off[e + 1]].long()
+        v = x[rows].double() @ w[e].double().t()
+        if glu:
+            v = v.view(len(rows), n // 32, 2, 16)
+            v = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(len(rows), n // 2)
+        want[rows] = v
+    _rows_close(y[1:-1], want.cpu(), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("m", [1, 20, 64])
 def test_few_rows_between_boundaries(m, dtype):
     """x and w that start between two 16-byte boundaries, which the stream's DMA does not take: plain, gated, per head, experts"""
