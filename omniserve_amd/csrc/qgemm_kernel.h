@@ -1276,7 +1276,7 @@ static void launch_exact_rows(const GemmArgs& a, int mb, int sk, hipStream_t st)
 
 // a workgroup per CU; share.sums: with K of the last round's tiles shared out.  With the unit and more than four rounds of tiles the next one is requested behind
 // the scaling, where that is the faster order.  (MI355X, us, in front / behind, 28672 x 4096: 1000 rows, 1.75 rounds, 103.1 / 104.3; 1501
-// 157.5 / 158.8; 2048, 3.5 rounds, 201.1 / 202.1; 2331, 4.4 rounds, 260.8 / 258.6; 3000 301.6 / 299.9; 4800 458.2 / 456.4; 9000 827.8 / 819.9.)
+// 157.5 / 158.8; 2048, 3.5 rounds, 201.1 / 202.1; 2331, 4.4 rounds, 253.9 / 251.9; 2800 259.3 / 257.1; 4800 445.1 / 443.4; 9000 806 / 802; 12001 1058 / 1054.)
 template <int MODE, bool SILU = false>
 static void launch_tiles(GemmArgs b, const TileShare& share, hipStream_t st) {
   b.tiles_n = b.N / TILES_N;

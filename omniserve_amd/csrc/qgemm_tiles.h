@@ -266,6 +266,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_sched_barrier(0);
     };
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
     auto store = [&](auto add) __attribute__((always_inline)) {
       constexpr bool ADD = decltype(add)::value;
       accumulators_stay(acc);
@@ -278,7 +280,6 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
         for (int e = 0; e < 4; ++e) sw[i][e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
       }
       v4i x[16];                                            // ADD: of two blocks of rows
-      uint2 packed[LATE ? 8 : 1][8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         if constexpr (ADD) if (j % 2 == 0) {
@@ -286,11 +287,9 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
           accumulators_stay(acc);
         }
         const float sa = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
-        uint2 (&h)[8] = packed[LATE ? j : 0];
+        uint2 h[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          typedef float v2f __attribute__((ext_vector_type(2)));
-          typedef _Float16 v2h __attribute__((ext_vector_type(2)));
           uint32_t hw[2];
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
@@ -299,21 +298,46 @@ __global__ __launch_bounds__(256, 1) void w8a8_tiles_kernel(GemmArgs p, TileShar
             v2f r = (v2f){(float)c0 * (sw[i][2 * e] * sa), (float)c1 * (sw[i][2 * e + 1] * sa)};
             asm volatile("" : "+v"(r));
             hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
-            if constexpr (LATE) asm volatile("" : "+v"(hw[e]));      // (converted here, not where it is stored: half the registers)
           }
           h[i] = make_uint2(hw[0], hw[1]);
         }
-        if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
-        else put(j, h);
-      }
-      if constexpr (LATE) {
-        open = open_tile();
-#pragma unroll
-        for (int j = 0; j < 8; ++j) put(j, packed[j]);
+        put(j, h);
       }
     };
-    if (SHARE && mine.shared()) store(BoolTag<SHARE>{});
-    else store(BoolTag<false>{});
+    if constexpr (LATE) {
+      uint2 packed[8][8];                                   // [row block][channel block]
+      float sa[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sa[j] = (float)*(const half_t*)(sc + 512 + 2 * (wm + 16 * j + e15));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint2 w = *(const uint2*)(sc + 2 * (wn + 16 * i + 4 * e4));
+        const uint32_t wv[2] = {w.x, w.y};
+        float sw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sw[e] = (float)__builtin_bit_cast(half_t, (uint16_t)(wv[e >> 1] >> (16 * (e & 1))));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          uint32_t hw[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            v2f r = (v2f){(float)acc[i][j][2 * e] * (sw[2 * e] * sa[j]), (float)acc[i][j][2 * e + 1] * (sw[2 * e + 1] * sa[j])};
+            asm volatile("" : "+v"(r));
+            hw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, v2h));
+            asm volatile("" : "+v"(hw[e]));                 // (converted here, not where it is stored: half the registers)
+          }
+          packed[j][i] = make_uint2(hw[0], hw[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      open = open_tile();
+#pragma unroll
+      for (int j = 0; j < 8; ++j) put(j, packed[j]);
+    } else if (SHARE && mine.shared()) {
+      store(BoolTag<SHARE>{});
+    } else {
+      store(BoolTag<false>{});
+    }
     parity ^= 1;
     if (open) park(parity);
   }
