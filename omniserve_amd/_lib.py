@@ -159,6 +159,7 @@ def lib() -> ctypes.CDLL:
 # library): same checks, same errors, same C-ABI calls, ~1.5 us of host time per call instead of ~7 us of Python + ctypes --
 # what an UNMODIFIED eager reference host is bound by (bench.py `drop_in`).  None when it is not built, when there is no GPU,
 # when a library variant (LIB_PATH changed) or a test harness's fake C ABI is in use, or when USE_EXT is cleared (A/B, tests).
+# It arms prompts' products with scratch for their last round (omni_gemm_arm_share); the functions in Python take whole tiles.
 USE_EXT = True
 _DEFAULT_LIB_PATH = os.path.abspath(LIB_PATH)
 _ext = None

@@ -318,7 +318,10 @@ PrefillPlan plan_prefill(int M, int N, int K, int mode, int sk, bool slab_only, 
       time *= 1.f + 0.08f * std::max(0.f, (busy - 0.8f) / 0.2f);
     }
     const bool take = mode == MODE_W8 ? whole < time : g_override_waves == 16 || whole < (mode == MODE_GRP ? 0.98f : 0.985f) * time;      // (per-channel 1501 rows of 28672 x 4096, 0.994 here, 147 / 145 us in a prompt, whose step is no faster for it)
-    // (in place of whole W8A8 tiles: by 18 us, which are faster than reckoned where two thirds of the CUs have one: 3000 rows of 4096 x 14336 141.4 / 142.5 shared, a whole prompt 3342 / 3402; 2331 129 / 130, 2100 150 / 123)
+    // (in place of whole W8A8 tiles: by 18 us, which are faster than reckoned in a last round of two thirds and more of the CUs.  us, whole / shared, rounds of tiles in brackets.  Shared by this rule: 4096 x 14336, 1501 rows (0.38)
+    // 109 / 92, 2100 (0.56) 153 / 125, 4200 (1.06) 275 / 209, 6000 (1.50) 282 / 258; 10240 x 8192, 2000 (1.25) 167 / 147; 8192 x 28672, 1501 (0.75) 310 / 280.  Left whole: 4096 x 14336, 3000 (0.75) 142 / 143, a whole prompt
+    // 3342 / 3402, 3500 (0.88) 153 / 165, 7000 (1.75) 300 / 304; 6144 x 4096, 4800 (1.78) 98 / 112; 28672 x 4096 with the unit, 3000 (5.25) 291 / 297.  Where the last round has few tiles and K is short the line leaves
+    // some: 6144 x 4096, 2700 - 3400 (1.03 - 1.31) 88 - 105 / 80 - 94; 4096 x 4096, 4800 (1.19) 94 / 84; 4096 x 14336, 2331 (0.62) 131 - 140 / 130; 8192 x 8192, 1000 (0.50) 78 / 66, 2600 (1.38) 175 / 163)
     const bool share = scratch && shared_time(mode, tiles, stages) < (take ? whole - (mode == MODE_W8 ? 18.f : 4.f) : (mode == MODE_CHN ? 1.f : 0.93f) * time - 4.f);
     if ((take || share) && mode == MODE_W8) best = PrefillPlan{16, 1, 1};
     best.w4_tiles = (take || share) && mode != MODE_W8;

@@ -147,8 +147,10 @@ def test_mirror_without_room_for_scratch(unit):
     torch.cuda.empty_cache()
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / torch.cuda.get_device_properties(0).total_memory)
     try:
+        full = []
         with pytest.raises(torch.cuda.OutOfMemoryError):
-            torch.empty((need,), dtype=torch.uint8, device=DEV)
+            while len(full) < 64:      # (what is cached beside tensors of other tests)
+                full.append(torch.empty((need,), dtype=torch.uint8, device=DEV))
         got.fill_(7)
         run(1)
     finally:
